@@ -148,6 +148,21 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
   // mixed prefill + decode steps (16 < M <= 64): the medium-M kernel when the start-up tuner
   // measured it faster (path 2, gemm_mid.hip); it declines shapes / modes it does not take
   if (g.path == 2 && launch_gemm_mid(g, st)) return;
+  // without a plan, 17 .. 64 rows: one block per CU owning whole tiles (wide) where K is short, K slices over narrow
+  // tiles where it is long. us at 32 rows, the K-split / tile kernels below -> now: 17920 x 1536 19 -> 14.5, 6464 x 1536
+  // 14.1 -> 9.0, 1536 x 8960 19.2 -> 13.1, 1024 x 4096 12.1 -> 8.4, 1536 x 1536 8.2 -> 6.6. Above 32 rows the wide form pays
+  // only once its tiles cover the CUs (N >= 4160; at 64 rows 6464 x 1536 17.7 -> 13.0, 1536 x 1536 10.5 -> 7.8 sliced); wide and
+  // long (28672 x 4096: 50 us) stays with the tile kernel.
+  // (both stage rows of x by 16-B LDS-DMA: rows that are not 16-B aligned stay below)
+  const bool rows16 = reinterpret_cast<uintptr_t>(g.x) % 16 == 0 && g.lda % 8 == 0;
+  if (g.path == 0 && rows16 && g.M > 16 && g.M <= 64 && g.waves == 0 && g.splitk == 0 && g.ntb == 0 && g.N >= 512) {
+    GemmArgs h = g;
+    if (g.K > 2048) h.waves = g.N <= 8192 ? 4 : 0;
+    else if (g.M <= 32) h.waves = 8;
+    else if (g.N >= 4160) h.waves = 8;
+    else if (g.K > 512 && g.N <= 2048) h.waves = 4;
+    if (h.waves != 0 && launch_gemm_mid(h, st)) return;
+  }
   // decode rows on the register-stationary kernel (path 4: a decode plan / forced; gemm_kx_bf16.hip)
   if (g.path == 4) {
     GemmArgs h = g;
@@ -167,7 +182,10 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
     launch_dispatch<false>(to_params(h), h, st);
     return;
   }
-  if (g.path == 1 || (g.path == 0 && g.M >= 128 && g.waves == 0 && g.splitk == 0)) {
+  // (65 .. 127 rows: the same forms once the matrix is large enough to be streamed in slices; 1536 x 8960 at 96 rows
+  // 42 -> 19 us, 1024 x 4096 20 -> 13)
+  const bool longer = g.M >= 128 || (g.M > 64 && rows16 && (g.K >= 2560 || (int64_t)g.N * g.K >= 8 * 1024 * 1024));
+  if (g.path == 1 || (g.path == 0 && longer && g.waves == 0 && g.splitk == 0)) {
     GemmArgs h = g;
     if (g.path == 0) h.ntb = 0;
     if (launch_gemm_prefill(h, st)) return;

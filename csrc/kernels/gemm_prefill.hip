@@ -891,16 +891,88 @@ static void launch_prefill_cfg(const GemmParams& p, int nz, hipStream_t st) {
 
 // Split-K partials leave with non-temporal stores: dirty fp32 slabs in L2 are written back at the
 // kernel boundary and held the next launch back 2-4 us (prefill-step timeline, r4).
-// Tile shape: 128 x 128 when that grid covers the chip, else 128 x 64 (narrow N: o_proj,
-// down, 70B/TP shards). A grid still under ~200 blocks is split along K (>= 4 stages of 64 per
-// slice, <= 8 slices, partials within the workspace) and combined by prefill_reduce_kernel.
-// Returns false for shapes the kernel does not take (the caller keeps the N-split tile
-// kernel): K % 64, N % 64, a row gather, the gamma-in-registers RMSNorm mode.
+//
+// The launcher's own choice of tile and K slices: every form below costs about
+//     rounds x (a + b x K / 64) [+ c + d x MB of partials, the combine launch of a K-split grid]
+// with rounds = blocks over the CUs rounded up (one block of these forms fills a CU), so the cheapest by that sum is taken.
+// a, b, c, d in us, fitted to a sweep of 35 shapes (N 128 .. 28672, K 512 .. 14336) x M 128 .. 2048 on cold weights, rms
+// error 5 to 9 % per form. What the forms trade: a large tile has the highest rate (256 x 256: 1.6 PFLOP/s per full
+// round) and the worst last round; splitting K fills the chip for few tiles and costs a pass over the partials.
+// The times of the taken forms are 1.02 of the best of the sweep (geometric mean; the thresholds on block counts used
+// before: 1.31). 2048 rows, us before -> now: 1536 x 8960 154 -> 86, 1536 x 1536 30 -> 22, 1024 x 4096 60 -> 38,
+// 1024 x 1024 19 -> 14; 256 rows: 1536 x 8960 39 -> 27, 1536 x 1536 15 -> 13.
+struct PrefillForm {
+  int code;  // tile code (as the forced ones below); 0: leave it to the tile kernel of gemm_decode.h
+  int nz;    // K slices
+};
+
+static PrefillForm choose_prefill_form(int M, int N, int K, bool slabs, size_t slab_bytes, bool counters) {
+  struct Tile {
+    int code, bm, bn;
+    float a, b, c, d;
+  };
+  // 256 x 256 / 256 x 128 four-phase, 128 x 128 (8 waves) / 128 x 64 on four-deep rings
+  static constexpr Tile tiles[] = {{1024, 256, 256, 10.2f, 1.33f, 1.5f, 0.49f},
+                                   {768, 256, 128, 7.1f, 1.00f, 1.6f, 0.56f},
+                                   {1281, 128, 128, 5.8f, 0.61f, 2.8f, 0.57f},
+                                   {640, 128, 64, 5.0f, 0.50f, 2.9f, 0.68f}};
+  static constexpr int slices[] = {1, 2, 3, 4, 6, 8};
+  const int cus = cu_count() > 0 ? cu_count() : 256, nk = K / 64;
+  auto over = [](int64_t x, int y) { return (int)((x + y - 1) / y); };
+  PrefillForm best{64, 1};
+  float cost = 1e30f;
+  auto take = [&](int code, int nz, float t) {
+    if (t < cost) {
+      cost = t;
+      best = PrefillForm{code, nz};
+    }
+  };
+  // 64 x 64 tiles, weights in registers (gemm_decode.h gemm_tile3_kernel): short K, few rows
+  if (K % 256 == 0 && N / 16 < 1024) take(0, 1, over((int64_t)over(M, 64) * (N / 64), cus) * (4.6f + 0.354f * nk));
+  for (const Tile& t : tiles) {
+    if (N % t.bn != 0) continue;
+    for (int nz : slices) {
+      const int64_t blocks = (int64_t)over(M, t.bm) * (N / t.bn) * nz;
+      const int rounds = over(blocks, cus);
+      if (nz > 1 && (rounds > 1 || nk / nz < 4 || !slabs || ((size_t)nz * M * N + (size_t)nz * M) * 4 > slab_bytes)) continue;
+      const float mb = (float)nz * M * N * 4e-6f;
+      take(t.code, nz, rounds * (t.a + t.b * over(nk, nz)) + (nz > 1 ? t.c + t.d * mb : 0.f));
+    }
+  }
+  // two-deep rings, several blocks per CU: the rate of the small tiles without whole rounds
+  const int n64 = over((int64_t)over(M, 128) * (N / 64), cus), n128 = N % 128 == 0 ? over((int64_t)over(M, 128) * (N / 128), cus) : 0;
+  if (n64 > 1) take(64, 1, 5.0f + 0.54f * nk * n64);
+  if (n128 > 1) take(128, 1, 6.0f + 0.77f * nk * n128);
+  // the persistent four-phase forms: whole rounds, then the rest split along K and met in the launch
+  if (M >= 512 && slabs && counters) {
+    auto persistent = [&](int code, const Tile& t, float e, float f, float g, float h) {
+      if (N % t.bn != 0) return;
+      const int n = over(M, 256) * (N / t.bn), rest = n % cus;
+      if (rest == 0) return;
+      int S = cus / rest > 8 ? 8 : cus / rest;
+      while (S > 1 && nk / S < 4) --S;
+      take(code, 0, (n / cus) * (t.a + t.b * nk) + e + f * nk / S + (S > 1 ? g + h * (S - 1) : 0.f));
+    };
+    persistent(1025, tiles[0], 13.4f, 1.61f, 13.6f, 2.4f);
+    persistent(769, tiles[1], 10.6f, 1.07f, 5.6f, 1.5f);
+  }
+  return best;
+}
+
+// Returns false for shapes the kernels do not take (the caller keeps the N-split tile
+// kernel): K % 64, N % 64, a row gather, the gamma-in-registers RMSNorm mode; and where that tile kernel is the
+// cheapest form.
 template <int EPI, int NORM>
 static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, size_t slab_bytes, int max_counters,
                                hipStream_t st) {
   constexpr int NTB = 1;  // every epilogue works on self-contained 16-column tiles
   if (p.K % 64 != 0 || p.N % 64 != 0 || p.row_idx != nullptr) return false;
+  if (force_bn == 0 && force_sk == 0) {
+    const PrefillForm f = choose_prefill_form(p.M, p.N, p.K, p.slabs != nullptr, slab_bytes, p.counters != nullptr);
+    if (f.code == 0) return false;
+    force_bn = f.code;
+    force_sk = f.nz;
+  }
   const int mb = (p.M + 127) / 128;
   bool wide = p.N % 128 == 0 && mb * (p.N / 128) >= 240;
   if (force_bn == 128) wide = p.N % 128 == 0;
@@ -917,23 +989,6 @@ static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, 
   while (nz > 1 && nk / nz < 4) --nz;
   const size_t need = ((size_t)nz * p.M * p.N + (size_t)nz * p.M) * 4;
   if (nz > 1 && (p.slabs == nullptr || need > slab_bytes)) nz = 1;
-  // 256 x 256 when its grid covers ~3/4 of the chip, else v2 (256 x 128, 3-deep ring)
-  // when its grid still covers the chip without split-K (profiles/r2_prefill_gemm_sched.log: the
-  // 256-square tile +20-35 % at >= 192 blocks, up to -30 % at 128)
-  const int blocks_v3 = ((p.M + 255) / 256) * (p.N % 256 == 0 ? p.N / 256 : 0);
-  const int blocks_v2 = ((p.M + 255) / 256) * (p.N % 128 == 0 ? p.N / 128 : 0);
-  if (force_bn == 0 && force_sk == 0 && blocks_v3 >= 180) {
-    // the 4-phase 256 x 256 kernel (v4: +7-22 % over the same tile with one barrier per K-tile,
-    // profiles/r2_prefill_gemm_v4.log)
-    launch_prefill4_cfg<EPI, NORM, NTB>(p, 1, st);
-    return true;
-  }
-  if (force_bn == 0 && force_sk == 0 && blocks_v2 >= 192) {
-    // the 4-phase kernel on 256 x 128 (+0-8 % over the 3-deep-ring v2 at 192-256 blocks,
-    // profiles/r2_prefill_gemm_v4.log)
-    launch_prefill4_cfg<EPI, NORM, NTB, 128>(p, 1, st);
-    return true;
-  }
   if (force_bn == 256) {  // forced (tests / sweeps), split-K as chosen above
     if (p.N % 128 != 0) return false;
     launch_prefill2_cfg<EPI, NORM, NTB>(p, nz, st);
