@@ -1,0 +1,81 @@
+// What the recurrences that take a portion in chunks of CN tokens share (gated_delta.hip, delta_rule.hip): where a chunk
+// lies, sums over lanes, packed lower triangles and their products with a column kept in registers.
+#pragma once
+#include "common.h"
+
+namespace vgate {
+namespace {
+
+constexpr int CN = 32;   // tokens of a chunk
+
+template <int CTRL>
+__device__ __forceinline__ float row_rot(float v) {  // a rotation inside each row of 16 lanes (DPP), on the VALU
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+// sum over the KG lanes that share lane % (64 / KG)
+template <int KG>
+__device__ __forceinline__ float key_sum(float v) {
+  if (KG >= 32) v += row_rot<0x122>(v);   // lanes 2 apart
+  if (KG >= 16) v += row_rot<0x124>(v);   // 4
+  v += row_rot<0x128>(v);                 // 8
+  v += xor16(v);
+  v += xor32(v);
+  return v;
+}
+
+// chunk `bx` of a step: its sequence and token range (chunks are numbered sequence by sequence; sequences without a slot, or of
+// at most `lim` tokens, have none)
+__device__ __forceinline__ bool locate_chunk(const int32_t* query_start, const int32_t* state_slots, int S, int lim, int bx, int& s,
+                                             int& t0, int& t1) {
+  int base = 0;
+  for (int i = 0; i < S; ++i) {
+    const int a = query_start[i], b = query_start[i + 1];
+    const int nc = (state_slots[i] < 0 || b - a <= lim) ? 0 : (b - a + CN - 1) / CN;
+    if (bx < base + nc) {
+      s = i; t0 = a + (bx - base) * CN; t1 = min(b, t0 + CN);
+      return true;
+    }
+    base += nc;
+  }
+  return false;
+}
+
+// number of the first chunk of sequence s
+__device__ __forceinline__ int first_chunk(const int32_t* query_start, const int32_t* state_slots, int lim, int s) {
+  int base = 0;
+  for (int i = 0; i < s; ++i) {
+    const int a = query_start[i], b = query_start[i + 1];
+    base += (state_slots[i] < 0 || b - a <= lim) ? 0 : (b - a + CN - 1) / CN;
+  }
+  return base;
+}
+
+// sum over j < n (a constant after unrolling) of row[j] x[j]; the row is read in 16-B pieces
+__device__ __forceinline__ float row_dot(const float* row, const float (&x)[CN], int n) {
+  float a = 0.f, b = 0.f;   // (two chains)
+#pragma unroll
+  for (int j0 = 0; j0 < CN; j0 += 4)
+    if (j0 < n) {
+      const float4 v = *reinterpret_cast<const float4*>(row + j0);
+      a = fmaf(v.x, x[j0], a);
+      if (j0 + 1 < n) b = fmaf(v.y, x[j0 + 1], b);
+      if (j0 + 2 < n) a = fmaf(v.z, x[j0 + 2], a);
+      if (j0 + 3 < n) b = fmaf(v.w, x[j0 + 3], b);
+    }
+  return a + b;
+}
+
+// first float of row i of a packed lower triangle whose row i has i entries, padded to whole 16-B pieces (row i of one with
+// the diagonal: tri(i + 1))
+__host__ __device__ constexpr int tri(int i) {
+  const int n = i > 0 ? i - 1 : 0, g = n / 4;
+  return i > 0 ? 4 * (2 * g * (g + 1) + (n - 4 * g) * (g + 1)) : 0;
+}
+
+__device__ __forceinline__ f32x4 ld4(const float* p) {
+  const float4 v = *reinterpret_cast<const float4*>(p);
+  return f32x4{v.x, v.y, v.z, v.w};
+}
+
+}  // namespace
+}  // namespace vgate

@@ -31,7 +31,7 @@
 //          (16x16x4) over the chunks; S stays in registers (C layout) and goes round through LDS as B operand.
 //   chunk finish  as finish, from the scan's [column][token] tiles.
 // Rows past a portion's end are tokens with k = q = v = 0, g = 1, beta = 0.
-#include "common.h"
+#include "chunks.h"
 #include "seq_launchers.h"
 #include "short_conv.h"
 
@@ -41,21 +41,6 @@ namespace {
 __device__ __forceinline__ float sigm(float x) { return 1.f / (1.f + expf(-x)); }
 __device__ __forceinline__ float silu_f(float x) { return x / (1.f + expf(-x)); }
 __device__ __forceinline__ float softplus_f(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
-template <int CTRL>
-__device__ __forceinline__ float row_rot(float v) {  // a rotation inside each row of 16 lanes (DPP), on the VALU
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
-// sum over the KG lanes that share lane % (64 / KG)
-template <int KG>
-__device__ __forceinline__ float key_sum(float v) {
-  if (KG >= 32) v += row_rot<0x122>(v);   // lanes 2 apart
-  if (KG >= 16) v += row_rot<0x124>(v);   // 4
-  v += row_rot<0x128>(v);                 // 8
-  v += xor16(v);
-  v += xor32(v);
-  return v;
-}
-
 // grid (token, q / k head)
 __global__ __launch_bounds__(256) void gated_delta_prep_kernel(GatedDeltaArgs p, float4* __restrict__ vec,
                                                                 float* __restrict__ vals) {
@@ -243,46 +228,9 @@ __global__ __launch_bounds__(256) void gated_delta_finish_kernel(GatedDeltaArgs 
 }
 
 // ------------------------------------------------------------------------------------------ chunks of CN tokens
-constexpr int CN = 32;
 // floats of one (chunk, head) record: [w; q'] [2 CN][DP], the update's keys [DP][CN], gamma_CN [DP], v' [V][CN], and b v', which
 // becomes o [V][CN]
 __host__ __device__ inline int64_t chunk_floats(int DP, int V) { return (int64_t)3 * CN * DP + DP + (int64_t)2 * CN * V; }
-
-__device__ __forceinline__ bool locate_chunk(const GatedDeltaArgs& p, int bx, int& s, int& t0, int& t1) {
-  int base = 0;
-  for (int i = 0; i < p.S; ++i) {
-    const int a = p.query_start[i], b = p.query_start[i + 1];
-    const int nc = (p.state_slots[i] < 0 || b <= a) ? 0 : (b - a + CN - 1) / CN;
-    if (bx < base + nc) {
-      s = i; t0 = a + (bx - base) * CN; t1 = min(b, t0 + CN);
-      return true;
-    }
-    base += nc;
-  }
-  return false;
-}
-
-// sum over j < n (a constant after unrolling) of row[j] x[j]; the row is read in 16-B pieces
-__device__ __forceinline__ float row_dot(const float* row, const float (&x)[CN], int n) {
-  float a = 0.f, b = 0.f;   // (two chains)
-#pragma unroll
-  for (int j0 = 0; j0 < CN; j0 += 4)
-    if (j0 < n) {
-      const float4 v = *reinterpret_cast<const float4*>(row + j0);
-      a = fmaf(v.x, x[j0], a);
-      if (j0 + 1 < n) b = fmaf(v.y, x[j0 + 1], b);
-      if (j0 + 2 < n) a = fmaf(v.z, x[j0 + 2], a);
-      if (j0 + 3 < n) b = fmaf(v.w, x[j0 + 3], b);
-    }
-  return a + b;
-}
-
-// first float of row i of a packed lower triangle whose row i has i entries, padded to whole 16-B pieces (row i of one with
-// the diagonal: tri(i + 1))
-__host__ __device__ constexpr int tri(int i) {
-  const int n = i > 0 ? i - 1 : 0, g = n / 4;
-  return i > 0 ? 4 * (2 * g * (g + 1) + (n - 4 * g) * (g + 1)) : 0;
-}
 
 // grid (chunk, head). At DP = 128 the LDS comes to a third of a CU's.
 template <int DP, bool F32>
@@ -292,7 +240,7 @@ __global__ __launch_bounds__(256, DP > 64 ? 3 : 4) void gated_delta_chunk_kernel
   __shared__ __attribute__((aligned(16))) float As[tri(CN)], Bs[tri(CN + 1)];
   __shared__ float beta[CN];
   int s, t0, t1;
-  if (!locate_chunk(p, blockIdx.x, s, t0, t1)) return;
+  if (!locate_chunk(p.query_start, p.state_slots, p.S, 0, blockIdx.x, s, t0, t1)) return;
   const int h = blockIdx.y, D = p.D, V = p.V, H = p.H, GD = p.G * D;
   const int NC = 2 * GD + H * V, g = h / (H / p.G);
   const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
@@ -435,11 +383,6 @@ __global__ __launch_bounds__(256, DP > 64 ? 3 : 4) void gated_delta_chunk_kernel
   }
 }
 
-__device__ __forceinline__ f32x4 ld4(const float* p) {
-  const float4 v = *reinterpret_cast<const float4*>(p);
-  return f32x4{v.x, v.y, v.z, v.w};
-}
-
 // grid (head, rounded up to the XCDs, 16 columns, sequence): a head's workgroups read the same records on one XCD. NT tiles
 // of 16 channels. MFMA operands: the channel (or token) 16 n + 4 kg + e is element e of lane group kg in both operands, so
 // a lane's four steps are one 16-B piece of a row.
@@ -453,11 +396,7 @@ __global__ __launch_bounds__(256) void gated_delta_chunk_scan_kernel(GatedDeltaA
   const int slot = p.state_slots[s];
   const int t0 = p.query_start[s], t1 = p.query_start[s + 1];
   if (slot < 0 || t1 <= t0) return;
-  int base = 0;
-  for (int i = 0; i < s; ++i) {
-    const int a = p.query_start[i], b = p.query_start[i + 1];
-    base += (p.state_slots[i] < 0 || b <= a) ? 0 : (b - a + CN - 1) / CN;
-  }
+  const int base = first_chunk(p.query_start, p.state_slots, 0, s);
   const int nc = (t1 - t0 + CN - 1) / CN, D = p.D, V = p.V, H = p.H;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, kg = l >> 4;
   const bool con = c0 + lr < V;
@@ -551,7 +490,7 @@ __global__ __launch_bounds__(256) void gated_delta_chunk_finish_kernel(GatedDelt
   __shared__ float lo[CHUNK_MAX_V][CN + 1];
   __shared__ float rn[CN];
   int s, t0, t1;
-  if (!locate_chunk(p, blockIdx.x, s, t0, t1)) return;
+  if (!locate_chunk(p.query_start, p.state_slots, p.S, 0, blockIdx.x, s, t0, t1)) return;
   const int h = blockIdx.y, V = p.V, H = p.H, tid = threadIdx.x;
   const float* o = rec + ((int64_t)blockIdx.x * H + h) * chunk_floats(DP, V) + 3 * CN * DP + DP + CN * V;
   for (int e = tid; e < V * CN; e += 256) lo[e / CN][e % CN] = o[e];

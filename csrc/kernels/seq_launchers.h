@@ -146,8 +146,10 @@ struct DeltaArgs {
   void* out = nullptr; int64_t ldo = 0;
   int S = 0, H = 0, D = 0, f32 = 0;
 };
-// T rows; scratch: T * H * D * 6 floats (the prepared per-channel vectors and the raw outputs)
-void launch_delta_rule(const DeltaArgs& a, int T, float* scratch, hipStream_t st);
+// floats of scratch a step of T rows can use
+size_t delta_rule_scratch_floats(int T, int H, int D);
+// T rows; scratch: `floats` of them, delta_rule_scratch_floats() for portions in chunks
+void launch_delta_rule(const DeltaArgs& a, int T, float* scratch, size_t floats, hipStream_t st);
 
 // Sliding-window attention over paged key / value caches with optional pooled blocks (window_attn.hip).
 struct WindowArgs {

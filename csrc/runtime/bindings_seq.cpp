@@ -267,7 +267,7 @@ void delta_rule(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor&
               scratch.numel() >= 6 * T * HD, "delta_rule: scratch fp32 with T * H * D * 6 elements");
   TORCH_CHECK((reinterpret_cast<uintptr_t>(scratch.data_ptr()) & 15) == 0, "delta_rule: scratch must be 16-B aligned");
   c10::DeviceGuard guard(r.device());
-  vgate::launch_delta_rule(p, (int)T, scratch.data_ptr<float>(), cur_stream());
+  vgate::launch_delta_rule(p, (int)T, scratch.data_ptr<float>(), (size_t)scratch.numel(), cur_stream());
 }
 
 
@@ -927,6 +927,9 @@ void bind_seq(pybind11::module& m) {
     return std::make_pair((int64_t)parts, (int64_t)vgate::latent_attn_part_floats((int)T, (int)S, (int)H, (int)rank, (int)rot, parts));
   }, "workgroups that share a decoded token's key tiles in latent_attn, and the fp32 scratch elements they need");
   m.def("delta_rule", &delta_rule, "generalized delta rule recurrence over state slots + head norm + gate");
+  m.def("delta_rule_scratch", [](int64_t T, int64_t H, int64_t D) {
+    return (int64_t)vgate::delta_rule_scratch_floats((int)T, (int)H, (int)D);
+  }, "floats of scratch delta_rule can use for a step of T tokens (with fewer it takes no chunks)");
   m.def("cast_rows", &cast_rows, "fp32 rows rounded to bf16");
   m.def("glu_rows", &glu_rows, "out = act(gate) * up over a stacked [gate; up] projection", py::arg("gu"), py::arg("out"),
         py::arg("act"), py::arg("limit") = 0.0, py::arg("alpha") = 1.702);
