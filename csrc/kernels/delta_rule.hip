@@ -504,9 +504,13 @@ int delta_chunks(int T, int lim) { return T <= lim ? 0 : T / CN + T / (lim + 1);
 
 template <int DP, bool F32>
 void launch_delta(const DeltaArgs& a, int T, int lim, float* rec, hipStream_t st) {
-  if (a.S > 1 || T <= lim) hipLaunchKernelGGL((delta_short_kernel<DP, F32>), dim3(a.S, a.H), dim3(256), 0, st, a, lim);
-  const int chunks = delta_chunks(T, lim);
+  // T counts padding rows too, so a sequence may be much shorter. A lone one then takes chunks whatever its length (not more
+  // of them than any step of T rows); several are told apart by their lengths on the device.
+  const bool lone = a.S == 1 && T > lim;
+  const int chunks = lone ? (T + CN - 1) / CN : delta_chunks(T, lim);
+  if (!lone) hipLaunchKernelGGL((delta_short_kernel<DP, F32>), dim3(a.S, a.H), dim3(256), 0, st, a, lim);
   if (chunks == 0) return;
+  if (lone) lim = 0;
   const dim3 grid(chunks, a.H), scan((a.H + 7) / 8 * 8, (a.D + 15) / 16, a.S);
   hipLaunchKernelGGL((delta_chunk_kernel<DP, F32>), grid, dim3(256), 0, st, a, lim, rec);
   hipLaunchKernelGGL(delta_chunk_scan_kernel<DP / 16>, scan, dim3(256), 0, st, a, lim, rec);

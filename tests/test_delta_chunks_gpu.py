@@ -8,12 +8,12 @@ from vgate.ops import seq
 pytestmark = pytest.mark.gpu
 
 
-def _inputs(H, D, lens, pos, dt, seed, device):
+def _inputs(H, D, lens, pos, dt, seed, device, pad=3):
     g = torch.Generator().manual_seed(seed)
     T, n, S = sum(lens), H * D, len(lens)
-    P = torch.randn(T + 3, 5 * n + 8, generator=g).to(dt)       # columns of one fused projection; three padding rows
+    P = torch.randn(T + pad, 5 * n + 8, generator=g).to(dt)     # columns of one fused projection, with padding rows
     cols = [P[:, i * n: (i + 1) * n] for i in range(5)]
-    t = dict(r=cols[0], k=cols[1], v=cols[2], g=cols[3], a=cols[4], wl=torch.randn(T + 3, n, generator=g).to(dt),
+    t = dict(r=cols[0], k=cols[1], v=cols[2], g=cols[3], a=cols[4], wl=torch.randn(T + pad, n, generator=g).to(dt),
              w0=torch.randn(n, generator=g), ab=torch.randn(n, generator=g), nw=1 + 0.1 * torch.randn(n, generator=g),
              state=torch.randn(S + 2, H, D, D, generator=g))
     slots = torch.randperm(S + 2, generator=g)[:S].int()
@@ -22,11 +22,11 @@ def _inputs(H, D, lens, pos, dt, seed, device):
     P = P.to(device)
     moved = {k: P[:, i * n: (i + 1) * n] for i, k in enumerate("rkvga")}
     moved.update({k: v.to(device) for k, v in t.items() if k not in moved})
-    return moved, slots.to(device), ctx.to(device), qs.to(device), torch.zeros(T + 3, n, dtype=dt, device=device)
+    return moved, slots.to(device), ctx.to(device), qs.to(device), torch.zeros(T + pad, n, dtype=dt, device=device)
 
 
-def _run(H, D, lens, pos, dt, seed, device):
-    t, slots, ctx, qs, out = _inputs(H, D, lens, pos, dt, seed, device)
+def _run(H, D, lens, pos, dt, seed, device, pad=3):
+    t, slots, ctx, qs, out = _inputs(H, D, lens, pos, dt, seed, device, pad)
     seq.delta_rule(t["r"], t["k"], t["v"], t["g"], t["a"], t["wl"], t["w0"], t["ab"], t["nw"], t["state"], slots, ctx, qs, out,
                    0.6, 1e-6, 1e-6)
     return out[: sum(lens)].float().cpu(), t["state"].cpu()
@@ -44,3 +44,12 @@ def test_matches_cpu_form(H, D, lens, pos, dt):
     rel = lambda a, b: float((a - b).norm() / b.norm())  # noqa: E731
     assert rel(state, state_w) < 2e-5
     assert rel(out, want) < (2e-5 if dt == torch.float32 else 2.0 ** -8)
+
+
+@pytest.mark.parametrize("lens,pos,pad", [([20], [3], 80), ([1], [0], 300), ([48], [1], 17), ([49], [0], 64), ([3, 30], [0, 2], 130)])
+def test_fewer_tokens_than_rows(lens, pos, pad):
+    """A step's rows are padded to a size of their own: few tokens among many rows."""
+    out, state = _run(3, 64, lens, pos, torch.float32, 11, "cuda", pad)
+    want, state_w = _run(3, 64, lens, pos, torch.float32, 11, "cpu", pad)
+    assert float((state - state_w).norm() / state_w.norm()) < 2e-5   # (as above)
+    assert float((out - want).norm() / want.norm()) < 2e-5
