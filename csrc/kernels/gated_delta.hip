@@ -4,7 +4,8 @@
 //   g = exp(-decay[h] softplus(z));  beta = sigmoid(b)
 //   S <- diag(g) S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q
 //   out = o / rms(o) * nw * sigmoid(gate)                               (rms over the head's value channels)
-// Query / key heads may be fewer than value heads (head h reads q / k head h / (H / G)). Three launches:
+// Query / key heads may be fewer than value heads (head h reads q / k head h / (H / G)). Decoding steps run in one
+// launch where a head has its own q / k head and D, V <= 128 (gated_delta_short_kernel). Otherwise three launches:
 //   prep   (token, q / k head) parallel: convolutions, unit norms, decays; per (head, channel) the fp32 vector
 //          {g, beta k, q, g k} (with it the update is S <- g S + (beta k)(v - (g k)^T S_old)) and the values.
 //   scan   the recurrence. Column v of S depends on no other column: a wave owns CL NC columns of one head, lane =
@@ -31,6 +32,8 @@
 //          (16x16x4) over the chunks; S stays in registers (C layout) and goes round through LDS as B operand.
 //   chunk finish  as finish, from the scan's [column][token] tiles.
 // Rows past a portion's end are tokens with k = q = v = 0, g = 1, beta = 0.
+#include <algorithm>
+
 #include "chunks.h"
 #include "seq_launchers.h"
 #include "short_conv.h"
@@ -227,6 +230,194 @@ __global__ __launch_bounds__(256) void gated_delta_finish_kernel(GatedDeltaArgs 
   }
 }
 
+// sum over the 32 lanes of a half wave, in all of them
+__device__ __forceinline__ float half_sum(float v) {
+  v += row_rot<0x128>(v);
+  v += row_rot<0x124>(v);
+  v += row_rot<0x122>(v);
+  v += row_rot<0x121>(v);
+  return v + xor16(v);
+}
+
+constexpr int SHORT_TC = 8;  // tokens staged in LDS at a time
+// grid (sequence, head): sequences of at most `lim` tokens, as many query / key heads as value heads, D and V up to P, at most
+// four taps.
+// One launch for convolutions, norms, the recurrence, the output and the kept inputs; the state is read and written once, whole cache
+// lines, in registers between (lane = four columns of KP keys; the waves' sums over keys meet in LDS, once per token: both sums
+// are of the old state, o = (g q)^T S + (q . k) u). Bound by those bytes once sequences x heads fill the chip: 32 sequences x 12
+// heads of 128 (50 MB) 15.5 us, 43 in three launches of which the scan read the state in pieces of 32 B; one sequence 11.8 (17.6).
+// Further tokens cost 1.9 us each, one workgroup walking them all, against 0.3 where the scan spreads a head's columns over four.
+template <int P, bool F32>
+__global__ __launch_bounds__(256) void gated_delta_short_kernel(GatedDeltaArgs p, int lim) {
+  constexpr int TC = SHORT_TC;
+  constexpr int CG = P / 4, KW = 64 / CG, KG = 4 * KW, KP = P / KG;   // column groups, key groups (of a wave; all), keys of a group
+  __shared__ __attribute__((aligned(16))) float lg[TC][P], lk[TC][P], lgk[TC][P], lgq[TC][P], lv[TC][P], lz[TC][P];
+  __shared__ float beta[TC], qk[TC];
+  __shared__ __attribute__((aligned(16))) float lp[TC][4][P], lo[TC][4][P];   // the waves' parts of (g k)^T S and (g q)^T S
+  const int s = blockIdx.x, h = blockIdx.y;
+  const int slot = p.state_slots[s];
+  const int t0 = p.query_start[s], t1 = p.query_start[s + 1];
+  if (slot < 0 || t1 <= t0 || t1 - t0 > lim) return;
+  const int D = p.D, V = p.V, HD = p.H * D, NC = 2 * HD + p.H * V, pos0 = p.context_lens[s] - (t1 - t0);
+  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+  const int c = 4 * (lane % CG), k0 = KP * (wv * KW + lane / CG);
+  float* sp = p.state + ((int64_t)slot * p.H + h) * D * V;
+  float* kept = p.conv_state + (int64_t)slot * (p.taps - 1) * NC;
+  const bool vec4 = V % 4 == 0 && reinterpret_cast<uintptr_t>(sp) % 16 == 0;
+  f32x4 S[KP];
+#pragma unroll
+  for (int j = 0; j < KP; ++j) {
+    S[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (pos0 <= 0 || k0 + j >= D || c >= V) continue;
+    const float* q = sp + (int64_t)(k0 + j) * V + c;
+    if (vec4) S[j] = ld4(q);
+    else
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[j][e] = c + e < V ? q[e] : 0.f;
+  }
+  const float dec = p.decay[h];
+  auto lraw = [&](int kind) { return kind == 0 ? lgq : (kind == 1 ? lk : lv); };
+  for (int tb = t0; tb < t1; tb += TC) {
+    if (tb > t0) __syncthreads();
+    // the tokens' values; past D, V or the portion's end: q = k = v = 0, g = 1, gate 0
+    const int nt = min(TC, t1 - tb);
+    if (nt == 1) {   // one channel of one kind per thread
+      for (int e = tid; e < 5 * P; e += 256) {
+        const int d = e % P, kind = e / P, w = (kind < 2 || kind == 3) ? D : V, ch = h * w + d;
+        if (kind < 3) {
+          const int col = ch + kind * HD;
+          lraw(kind)[0][d] = d < w ? silu_f(short_conv_at(kind == 0 ? p.q : (kind == 1 ? p.k : p.v), kind == 0 ? p.ldq : (kind == 1 ? p.ldk : p.ldv),
+                                                          F32 ? 1 : 0, ch, p.conv_w, NC, col, 0.f, kept, NC, col, tb, t0, pos0, p.taps))
+                                   : 0.f;
+        } else if (kind == 3) {
+          lg[0][d] = d < w ? expf(-dec * softplus_f(p.z[(int64_t)tb * p.ldz + ch])) : 1.f;
+        } else {
+          lz[0][d] = d < w ? p.nw[d] * sigm(p.gate[(int64_t)tb * p.ldg + ch]) : 0.f;
+        }
+      }
+    } else {
+      for (int e = tid; e < 3 * P; e += 256) {   // one channel of q, k or v per thread
+        const int kind = e / P, d = e % P, w = kind < 2 ? D : V, ch = h * w + d, col = kind * HD + ch;
+        float y[TC];
+#pragma unroll
+        for (int i = 0; i < TC; ++i) y[i] = 0.f;
+        if (d < w)
+          short_conv_run8<F32>(kind == 0 ? p.q : (kind == 1 ? p.k : p.v), kind == 0 ? p.ldq : (kind == 1 ? p.ldk : p.ldv), ch, p.conv_w, NC,
+                               col, kept, NC, col, tb, t0, t1, pos0, p.taps, y);
+#pragma unroll
+        for (int i = 0; i < TC; ++i)
+          if (i < nt) lraw(kind)[i][d] = silu_f(y[i]);
+      }
+#pragma unroll
+      for (int m = 0; m < TC * P / 256; ++m) {
+        const int e = tid + 256 * m, i = e / P, d = e % P;
+        if (i >= nt) break;
+        lg[i][d] = d < D ? expf(-dec * softplus_f(p.z[(int64_t)(tb + i) * p.ldz + h * D + d])) : 1.f;
+        lz[i][d] = d < V ? p.nw[d] * sigm(p.gate[(int64_t)(tb + i) * p.ldg + h * V + d]) : 0.f;
+      }
+    }
+    __syncthreads();
+    if (tid < 32 * nt) {  // 32 lanes per token: unit norms
+      const int i = tid >> 5, l = tid & 31;
+      float q[P / 32], k[P / 32], sq = 0.f, sk = 0.f, x = 0.f;
+#pragma unroll
+      for (int m = 0; m < P / 32; ++m) {
+        q[m] = lgq[i][l + 32 * m];
+        k[m] = lk[i][l + 32 * m];
+        sq = fmaf(q[m], q[m], sq);
+        sk = fmaf(k[m], k[m], sk);
+      }
+      const float fq = p.q_scale / sqrtf(half_sum(sq) + p.unit_eps), fk = 1.f / sqrtf(half_sum(sk) + p.unit_eps);
+#pragma unroll
+      for (int m = 0; m < P / 32; ++m) {
+        const int d = l + 32 * m;
+        const float g = lg[i][d], qn = q[m] * fq, kn = k[m] * fk;
+        x = fmaf(qn, kn, x);
+        lk[i][d] = kn;
+        lgk[i][d] = g * kn;
+        lgq[i][d] = g * qn;
+      }
+      x = half_sum(x);
+      if (l == 0) {
+        qk[i] = x;
+        beta[i] = sigm(conv_ldx(p.b, (int64_t)(tb + i) * p.ldb + h, F32 ? 1 : 0));
+      }
+    }
+    __syncthreads();
+    for (int i = 0; i < nt; ++i) {
+      f32x4 A = {0.f, 0.f, 0.f, 0.f}, O = A;
+#pragma unroll
+      for (int j = 0; j < KP; ++j) {
+        const float gk = lgk[i][k0 + j], gq = lgq[i][k0 + j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          A[e] = fmaf(gk, S[j][e], A[e]);
+          O[e] = fmaf(gq, S[j][e], O[e]);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (KW >= 8) { A[e] += row_rot<0x128>(A[e]); O[e] += row_rot<0x128>(O[e]); }
+        if (KW >= 4) { A[e] += xor16(A[e]); O[e] += xor16(O[e]); }
+        A[e] += xor32(A[e]);
+        O[e] += xor32(O[e]);
+      }
+      if (lane < CG) {
+        *reinterpret_cast<f32x4*>(&lp[i][wv][c]) = A;
+        *reinterpret_cast<f32x4*>(&lo[i][wv][c]) = O;
+      }
+      lds_barrier();
+      A = ld4(&lp[i][0][c]) + ld4(&lp[i][1][c]) + (ld4(&lp[i][2][c]) + ld4(&lp[i][3][c]));
+      const f32x4 u = (ld4(&lv[i][c]) - A) * beta[i];
+#pragma unroll
+      for (int j = 0; j < KP; ++j) {
+        const float g = lg[i][k0 + j], k = lk[i][k0 + j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[j][e] = fmaf(k, u[e], g * S[j][e]);
+      }
+    }
+    __syncthreads();
+    if (tid < 32 * nt) {  // the outputs of the staged tokens: head norm, weight, gate (columns past V are zero)
+      const int i = tid >> 5, l = tid & 31;
+      float o[P / 32], ss = 0.f;
+#pragma unroll
+      for (int m = 0; m < P / 32; ++m) {
+        const int d = l + 32 * m;
+        const float A = lp[i][0][d] + lp[i][1][d] + (lp[i][2][d] + lp[i][3][d]);
+        const float O = lo[i][0][d] + lo[i][1][d] + (lo[i][2][d] + lo[i][3][d]);
+        o[m] = fmaf(qk[i] * beta[i], lv[i][d] - A, O);
+        ss = fmaf(o[m], o[m], ss);
+      }
+      const float inv = 1.f / sqrtf(half_sum(ss) / (float)V + p.eps);
+#pragma unroll
+      for (int m = 0; m < P / 32; ++m) {
+        const int d = l + 32 * m;
+        if (d >= V) continue;
+        const int64_t oi = (int64_t)(tb + i) * p.ldo + h * V + d;
+        const float y = o[m] * inv * lz[i][d];
+        if (F32) reinterpret_cast<float*>(p.out)[oi] = y;
+        else reinterpret_cast<bf16_t*>(p.out)[oi] = f2bf(y);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < KP; ++j) {
+    if (k0 + j >= D || c >= V) continue;
+    float* q = sp + (int64_t)(k0 + j) * V + c;
+    if (vec4) *reinterpret_cast<f32x4*>(q) = S[j];
+    else
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < V) q[e] = S[j][e];
+  }
+  // the slot's rows of this head's channels: no other workgroup reads them, and this one is done with them
+  for (int e = tid; e < 2 * D + V; e += 256) {
+    const int kind = e < D ? 0 : (e < 2 * D ? 1 : 2), ch = kind == 2 ? h * V + e - 2 * D : h * D + e - kind * D;
+    short_conv_keep(kind == 0 ? p.q : (kind == 1 ? p.k : p.v), kind == 0 ? p.ldq : (kind == 1 ? p.ldk : p.ldv), F32 ? 1 : 0, ch, kept, NC,
+                    kind * HD + ch, t0, t1, pos0, p.taps);
+  }
+}
+
 // ------------------------------------------------------------------------------------------ chunks of CN tokens
 // floats of one (chunk, head) record: [w; q'] [2 CN][DP], the update's keys [DP][CN], gamma_CN [DP], v' [V][CN], and b v', which
 // becomes o [V][CN]
@@ -234,13 +425,13 @@ __host__ __device__ inline int64_t chunk_floats(int DP, int V) { return (int64_t
 
 // grid (chunk, head). At DP = 128 the LDS comes to a third of a CU's.
 template <int DP, bool F32>
-__global__ __launch_bounds__(256, DP > 64 ? 3 : 4) void gated_delta_chunk_kernel(GatedDeltaArgs p, float* __restrict__ rec) {
+__global__ __launch_bounds__(256, DP > 64 ? 3 : 4) void gated_delta_chunk_kernel(GatedDeltaArgs p, int lim, float* __restrict__ rec) {
   constexpr int X = DP / 32;   // 16-B pieces of a row a lane of the pair sums holds: channels 32 x + 4 dg ..
   __shared__ __attribute__((aligned(16))) float lk[CN][DP], lq[CN][DP], lg[CN][DP];
   __shared__ __attribute__((aligned(16))) float As[tri(CN)], Bs[tri(CN + 1)];
   __shared__ float beta[CN];
   int s, t0, t1;
-  if (!locate_chunk(p.query_start, p.state_slots, p.S, 0, blockIdx.x, s, t0, t1)) return;
+  if (!locate_chunk(p.query_start, p.state_slots, p.S, lim, blockIdx.x, s, t0, t1)) return;
   const int h = blockIdx.y, D = p.D, V = p.V, H = p.H, GD = p.G * D;
   const int NC = 2 * GD + H * V, g = h / (H / p.G);
   const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
@@ -387,7 +578,7 @@ __global__ __launch_bounds__(256, DP > 64 ? 3 : 4) void gated_delta_chunk_kernel
 // of 16 channels. MFMA operands: the channel (or token) 16 n + 4 kg + e is element e of lane group kg in both operands, so
 // a lane's four steps are one 16-B piece of a row.
 template <int NT>
-__global__ __launch_bounds__(256) void gated_delta_chunk_scan_kernel(GatedDeltaArgs p, float* __restrict__ rec) {
+__global__ __launch_bounds__(256) void gated_delta_chunk_scan_kernel(GatedDeltaArgs p, int lim, float* __restrict__ rec) {
   constexpr int DP = 16 * NT, TW = (NT + 3) / 4;
   __shared__ __attribute__((aligned(16))) float Sl[16][DP + 4];
   __shared__ __attribute__((aligned(16))) float Ul[16][CN + 4];
@@ -395,8 +586,8 @@ __global__ __launch_bounds__(256) void gated_delta_chunk_scan_kernel(GatedDeltaA
   if (h >= p.H) return;
   const int slot = p.state_slots[s];
   const int t0 = p.query_start[s], t1 = p.query_start[s + 1];
-  if (slot < 0 || t1 <= t0) return;
-  const int base = first_chunk(p.query_start, p.state_slots, 0, s);
+  if (slot < 0 || t1 <= t0 || t1 - t0 <= lim) return;
+  const int base = first_chunk(p.query_start, p.state_slots, lim, s);
   const int nc = (t1 - t0 + CN - 1) / CN, D = p.D, V = p.V, H = p.H;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, kg = l >> 4;
   const bool con = c0 + lr < V;
@@ -486,11 +677,11 @@ __global__ __launch_bounds__(256) void gated_delta_chunk_scan_kernel(GatedDeltaA
 
 constexpr int CHUNK_MAX_V = 256;
 // grid (chunk, head)
-__global__ __launch_bounds__(256) void gated_delta_chunk_finish_kernel(GatedDeltaArgs p, int DP, const float* __restrict__ rec) {
+__global__ __launch_bounds__(256) void gated_delta_chunk_finish_kernel(GatedDeltaArgs p, int lim, int DP, const float* __restrict__ rec) {
   __shared__ float lo[CHUNK_MAX_V][CN + 1];
   __shared__ float rn[CN];
   int s, t0, t1;
-  if (!locate_chunk(p.query_start, p.state_slots, p.S, 0, blockIdx.x, s, t0, t1)) return;
+  if (!locate_chunk(p.query_start, p.state_slots, p.S, lim, blockIdx.x, s, t0, t1)) return;
   const int h = blockIdx.y, V = p.V, H = p.H, tid = threadIdx.x;
   const float* o = rec + ((int64_t)blockIdx.x * H + h) * chunk_floats(DP, V) + 3 * CN * DP + DP + CN * V;
   for (int e = tid; e < V * CN; e += 256) lo[e / CN][e % CN] = o[e];
@@ -535,14 +726,33 @@ int chunk_channels(int D) { return D <= 32 ? 32 : (D <= 64 ? 64 : 128); }
 bool takes_chunks(int T, int S, int D, int V) { return T >= 128 && T >= 64 * S && D <= 128 && V <= CHUNK_MAX_V; }
 constexpr int CHUNK_MAX_TAPS = 4;
 
+constexpr int SHORT = 32;   // tokens of a portion that the short form still takes beside chunks
+// Where many sequences share a long step (few chunks for most of them, but a long serial chain for one) each takes the form that
+// suits its own length, decided on the device: 31 decoded tokens beside a portion of 97: 103 us (token scan 246), of 225: 112
+// (510), 64 portions of 16: 113 (169). With 8 or 16 sequences the token scan is ahead for equal portions (8 x 16: 35 us, here 42).
+bool takes_both(int T, int S) { return S >= 32 && T >= 128; }
+int both_chunks(int T, int S) { return T / CN + std::min(S, T / (SHORT + 1)); }   // (each longer portion has at most one that is not whole)
+
 template <int DP>
-void launch_chunks(const GatedDeltaArgs& a, int T, float* rec, hipStream_t st) {
-  const int chunks = T / CN + a.S;
+void launch_chunks(const GatedDeltaArgs& a, int chunks, int lim, float* rec, hipStream_t st) {
   const int hx = (a.H + 7) / 8 * 8;
-  if (a.f32) hipLaunchKernelGGL((gated_delta_chunk_kernel<DP, true>), dim3(chunks, a.H), dim3(256), 0, st, a, rec);
-  else hipLaunchKernelGGL((gated_delta_chunk_kernel<DP, false>), dim3(chunks, a.H), dim3(256), 0, st, a, rec);
-  hipLaunchKernelGGL(gated_delta_chunk_scan_kernel<DP / 16>, dim3(hx, (a.V + 15) / 16, a.S), dim3(256), 0, st, a, rec);
-  hipLaunchKernelGGL(gated_delta_chunk_finish_kernel, dim3(chunks, a.H), dim3(256), 0, st, a, DP, rec);
+  if (a.f32) hipLaunchKernelGGL((gated_delta_chunk_kernel<DP, true>), dim3(chunks, a.H), dim3(256), 0, st, a, lim, rec);
+  else hipLaunchKernelGGL((gated_delta_chunk_kernel<DP, false>), dim3(chunks, a.H), dim3(256), 0, st, a, lim, rec);
+  hipLaunchKernelGGL(gated_delta_chunk_scan_kernel<DP / 16>, dim3(hx, (a.V + 15) / 16, a.S), dim3(256), 0, st, a, lim, rec);
+  hipLaunchKernelGGL(gated_delta_chunk_finish_kernel, dim3(chunks, a.H), dim3(256), 0, st, a, lim, DP, rec);
+}
+
+void launch_chunks_any(const GatedDeltaArgs& a, int chunks, int lim, float* rec, hipStream_t st) {
+  const int DP = chunk_channels(a.D);
+  if (DP == 32) launch_chunks<32>(a, chunks, lim, rec, st);
+  else if (DP == 64) launch_chunks<64>(a, chunks, lim, rec, st);
+  else launch_chunks<128>(a, chunks, lim, rec, st);
+}
+
+template <int P>
+void launch_short(const GatedDeltaArgs& a, int lim, hipStream_t st) {
+  if (a.f32) hipLaunchKernelGGL((gated_delta_short_kernel<P, true>), dim3(a.S, a.H), dim3(256), 0, st, a, lim);
+  else hipLaunchKernelGGL((gated_delta_short_kernel<P, false>), dim3(a.S, a.H), dim3(256), 0, st, a, lim);
 }
 
 template <int KG, int NC, int DQ, int TC>
@@ -555,18 +765,29 @@ void launch_scan(const GatedDeltaArgs& a, const float4* vec, const float* vals, 
 
 size_t gated_delta_scratch_floats(int T, int S, int H, int D, int V) {
   const size_t tokens = (size_t)T * H * (4 * (size_t)D + 2 * (size_t)V);
-  const size_t chunks = takes_chunks(T, S, D, V) ? (size_t)(T / CN + S) * H * chunk_floats(chunk_channels(D), V) : 0;
+  int n = takes_chunks(T, S, D, V) ? T / CN + S : 0;
+  if (takes_both(T, S) && D <= 128 && V <= 128) n = std::max(n, both_chunks(T, S));
+  const size_t chunks = (size_t)n * H * chunk_floats(chunk_channels(D), V);
   return tokens > chunks ? tokens : chunks;
 }
 
 void launch_gated_delta(const GatedDeltaArgs& a, int T, float* scratch, hipStream_t st) {
   if (a.S <= 0 || a.H <= 0 || T <= 0) return;
-  if (a.wide < 0 && a.taps <= CHUNK_MAX_TAPS && takes_chunks(T, a.S, a.D, a.V)) {
-    const int DP = chunk_channels(a.D);
-    if (DP == 32) launch_chunks<32>(a, T, scratch, st);
-    else if (DP == 64) launch_chunks<64>(a, T, scratch, st);
-    else launch_chunks<128>(a, T, scratch, st);
-    return;
+  if (a.wide < 0 && a.taps <= CHUNK_MAX_TAPS) {
+    const bool own = a.G == a.H && a.D <= 128 && a.V <= 128;   // a head's channels are no other head's
+    const bool decode = T <= a.S, both = takes_both(T, a.S);
+    if (takes_chunks(T, a.S, a.D, a.V)) {
+      launch_chunks_any(a, T / CN + a.S, 0, scratch, st);
+      return;
+    }
+    if (own && (decode || both)) {
+      const int lim = decode ? T : SHORT, P = std::max(a.D, a.V);
+      if (P <= 32) launch_short<32>(a, lim, st);
+      else if (P <= 64) launch_short<64>(a, lim, st);
+      else launch_short<128>(a, lim, st);
+      if (!decode) launch_chunks_any(a, both_chunks(T, a.S), lim, scratch, st);
+      return;
+    }
   }
   float4* vec = reinterpret_cast<float4*>(scratch);
   float* vals = scratch + 4 * (int64_t)T * a.H * a.D;
