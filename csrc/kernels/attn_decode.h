@@ -221,7 +221,8 @@ __device__ __forceinline__ void decode_block(const AttnArgs& a, int s, int h, in
   const bool cok = col < G;
   uint4 qf[4];  // (FUSED: from the producer's granules, after the wait)
   if constexpr (!FUSED) {
-    const bf16_t* qp = a.q + (size_t)qbeg * a.q_stride + (size_t)(h * G + (cok ? col : 0)) * D_ + 8 * (lane >> 4);
+    // (a decoded sequence's only row is its last; a padding sequence starts past the step's rows and must not be read there)
+    const bf16_t* qp = a.q + (size_t)max(qend - 1, 0) * a.q_stride + (size_t)(h * G + (cok ? col : 0)) * D_ + 8 * (lane >> 4);
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) qf[kk] = cok ? *reinterpret_cast<const uint4*>(qp + 32 * kk) : make_uint4(0, 0, 0, 0);
   }
