@@ -23,31 +23,50 @@ __device__ __forceinline__ float key_sum(float v) {
   return v;
 }
 
-// chunk `bx` of a step: its sequence and token range (chunks are numbered sequence by sequence; sequences without a slot, or of
-// at most `lim` tokens, have none)
+// chunks of C tokens of sequence i (sequences without a slot, or of at most `lim` tokens, have none)
+template <int C>
+__device__ __forceinline__ int chunks_of(const int32_t* state_slots, int lim, int i, int a, int b) {
+  return (state_slots[i] < 0 || b - a <= lim) ? 0 : (b - a + C - 1) / C;
+}
+
+// chunk `bx` of a step: its sequence and token range (chunks are numbered sequence by sequence). Whole waves: a lane per sequence
+// (one after another they cost 0.5 us each, three times per layer).
+template <int C = CN>
 __device__ __forceinline__ bool locate_chunk(const int32_t* query_start, const int32_t* state_slots, int S, int lim, int bx, int& s,
                                              int& t0, int& t1) {
+  const int lane = threadIdx.x & 63;
   int base = 0;
-  for (int i = 0; i < S; ++i) {
-    const int a = query_start[i], b = query_start[i + 1];
-    const int nc = (state_slots[i] < 0 || b - a <= lim) ? 0 : (b - a + CN - 1) / CN;
-    if (bx < base + nc) {
-      s = i; t0 = a + (bx - base) * CN; t1 = min(b, t0 + CN);
+  for (int s0 = 0; s0 < S; s0 += 64) {
+    const int i = s0 + lane;
+    const int a = i < S ? query_start[i] : 0, b = i < S ? query_start[i + 1] : 0;
+    const int n = i < S ? chunks_of<C>(state_slots, lim, i, a, b) : 0;
+    int end = n;   // inclusive sum over the lanes
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(end, o, 64);
+      if (lane >= o) end += v;
+    }
+    const unsigned long long hit = __ballot(bx >= base + end - n && bx < base + end);
+    if (hit != 0) {
+      const int l = __ffsll(hit) - 1;
+      s = s0 + l;
+      t0 = __builtin_amdgcn_readlane(a, l) + (bx - base - __builtin_amdgcn_readlane(end - n, l)) * C;
+      t1 = min(__builtin_amdgcn_readlane(b, l), t0 + C);
       return true;
     }
-    base += nc;
+    base += __builtin_amdgcn_readlane(end, 63);
   }
   return false;
 }
 
-// number of the first chunk of sequence s
+// number of the first chunk of sequence s (whole waves)
+template <int C = CN>
 __device__ __forceinline__ int first_chunk(const int32_t* query_start, const int32_t* state_slots, int lim, int s) {
-  int base = 0;
-  for (int i = 0; i < s; ++i) {
-    const int a = query_start[i], b = query_start[i + 1];
-    base += (state_slots[i] < 0 || b - a <= lim) ? 0 : (b - a + CN - 1) / CN;
-  }
-  return base;
+  int n = 0;
+  for (int i = threadIdx.x & 63; i < s; i += 64) n += chunks_of<C>(state_slots, lim, i, query_start[i], query_start[i + 1]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
+  return __builtin_amdgcn_readfirstlane(n);
 }
 
 // sum over j < n (a constant after unrolling) of row[j] x[j]; the row is read in 16-B pieces
@@ -75,6 +94,15 @@ __host__ __device__ constexpr int tri(int i) {
 __device__ __forceinline__ f32x4 ld4(const float* p) {
   const float4 v = *reinterpret_cast<const float4*>(p);
   return f32x4{v.x, v.y, v.z, v.w};
+}
+
+// sum over the 32 lanes of a half wave, in all of them
+__device__ __forceinline__ float half_sum(float v) {
+  v += row_rot<0x128>(v);
+  v += row_rot<0x124>(v);
+  v += row_rot<0x122>(v);
+  v += row_rot<0x121>(v);
+  return v + xor16(v);
 }
 
 }  // namespace

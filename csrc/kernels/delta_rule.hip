@@ -38,15 +38,6 @@ __device__ __forceinline__ float ldx(const void* p, int64_t i, int f32) {
 }
 __device__ __forceinline__ float sigm(float x) { return 1.f / (1.f + expf(-x)); }
 
-// sum over the 32 lanes of a half wave, in all of them
-__device__ __forceinline__ float half_sum(float v) {
-  v += row_rot<0x128>(v);
-  v += row_rot<0x124>(v);
-  v += row_rot<0x122>(v);
-  v += row_rot<0x121>(v);
-  return v + xor16(v);
-}
-
 constexpr int TC = 8;  // tokens staged in LDS at a time
 
 // grid (sequence, head): sequences of at most `lim` tokens, head size up to DP. Bound by the state's bytes once sequences x

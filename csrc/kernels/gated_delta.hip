@@ -230,15 +230,6 @@ __global__ __launch_bounds__(256) void gated_delta_finish_kernel(GatedDeltaArgs 
   }
 }
 
-// sum over the 32 lanes of a half wave, in all of them
-__device__ __forceinline__ float half_sum(float v) {
-  v += row_rot<0x128>(v);
-  v += row_rot<0x124>(v);
-  v += row_rot<0x122>(v);
-  v += row_rot<0x121>(v);
-  return v + xor16(v);
-}
-
 constexpr int SHORT_TC = 8;  // tokens staged in LDS at a time
 // grid (sequence, head): sequences of at most `lim` tokens, as many query / key heads as value heads, D and V up to P, at most
 // four taps.
@@ -728,8 +719,8 @@ constexpr int CHUNK_MAX_TAPS = 4;
 
 constexpr int SHORT = 32;   // tokens of a portion that the short form still takes beside chunks
 // Where many sequences share a long step (few chunks for most of them, but a long serial chain for one) each takes the form that
-// suits its own length, decided on the device: 31 decoded tokens beside a portion of 97: 103 us (token scan 246), of 225: 112
-// (510), 64 portions of 16: 113 (169). With 8 or 16 sequences the token scan is ahead for equal portions (8 x 16: 35 us, here 42).
+// suits its own length, decided on the device: 31 decoded tokens beside a portion of 97: 96 us (token scan 246), of 225: 107
+// (510), 64 portions of 16: 94 (169). With 8 or 16 sequences the token scan is ahead for equal portions (8 x 16: 35 us, here 42).
 bool takes_both(int T, int S) { return S >= 32 && T >= 128; }
 int both_chunks(int T, int S) { return T / CN + std::min(S, T / (SHORT + 1)); }   // (each longer portion has at most one that is not whole)
 

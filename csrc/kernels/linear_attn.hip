@@ -26,7 +26,18 @@
 //           recurrence taken CH tokens at a time, all fp32); the slot receives the last one
 //   output  every chunk again from its true initial state I_c, now writing o
 // Twice the arithmetic, but a lone sequence's dependent chain is CH tokens long instead of the whole portion.
-#include "common.h"
+// Decoding steps and long ones of key and value sizes up to 128 take other forms (takes_small() has the line):
+//   short  sequences of few tokens (decoding) in ONE launch, a workgroup per (sequence, head): the vectors in LDS, the whole
+//          state in registers (lane = four columns, key group), read and written once in whole cache lines; the update
+//          does not wait for the outputs, so a token costs no barrier.
+//   chunks of CT = 64 tokens, for longer portions. With g_(j..i) = a_j .. a_i per channel (1 if empty) and I the state a chunk starts from
+//            o_i = (g_(1..i) q_i)^T I + sum_(j<=i) (q_i . g_(j+1..i) k_j) v_j
+//            I' = g_(1..CT) I + sum_j g_(j+1..CT) k_j v_j^T
+//          (with a bonus the products stop at i - 1 and the term j = i is q_i . u k_i). Every product of decays is a product
+//          of factors <= 1 taken in order. local: the second sum, fp32 MFMA (16x16x4); carry as above; output: the
+//          triangle of weighted products (a lane holds k_j g of four D / 32 channels and walks i), then both products
+//          with fp32 MFMA, norm and gate. 2048 tokens, 8 heads of 128: 128 us, by the scan in chunks 162.
+#include "chunks.h"
 #include "seq_launchers.h"
 
 namespace vgate {
@@ -319,6 +330,478 @@ void launch_scan(const LinearAttnArgs& a, int T, const float4* vec, const float*
   else launch_scan_pre<DQ, TC, NC, false>(a, T, vec, vals, oraw, CH, cstate, cdecay, st);
 }
 
+// ------------------------------------------------------------------------------- key and value sizes up to 128
+// the decay, key and query of channel d of head h at token t (x[t][h D + d] of the projections)
+template <bool F32>
+__device__ __forceinline__ void decay_key_query(const LinearAttnArgs& p, int t, int h, int d, float& a, float& k, float& q) {
+  constexpr int f32 = F32 ? 1 : 0;
+  const int e = h * p.D + d;
+  q = ldx(p.q, (int64_t)t * p.ldq + e, f32);
+  k = ldx(p.k, (int64_t)t * p.ldk + e, f32);
+  if (p.in_silu) { q = silu_f(q); k = silu_f(k); }
+  if (d < p.rot_dims) {  // the pair's other entry, then (u, v) -> (u c - v s, v c + u s)
+    const int half = p.rot_dims >> 1;
+    const bool first = p.rot_half ? d < half : !(d & 1);
+    const int eo = p.rot_half ? (first ? e + half : e - half) : (first ? e + 1 : e - 1);
+    float qo = ldx(p.q, (int64_t)t * p.ldq + eo, f32), ko = ldx(p.k, (int64_t)t * p.ldk + eo, f32);
+    if (p.in_silu) { qo = silu_f(qo); ko = silu_f(ko); }
+    const float ang = (float)p.positions[t] * p.inv_freq[p.rot_half ? (first ? d : d - half) : (d >> 1)];
+    const float cs = cosf(ang), sn = sinf(ang);
+    q = first ? q * cs - qo * sn : q * cs + qo * sn;
+    k = first ? k * cs - ko * sn : k * cs + ko * sn;
+  }
+  if (p.z == nullptr) a = p.head_decay[h];
+  else if (p.decay_exp) a = expf(-expf(p.z[(int64_t)t * p.ldz + e]));
+  else a = expf(log_sigmoid(p.z[(int64_t)t * p.ldz + e]) * (1.f / p.tau));
+  k *= p.k_scale;
+  q *= p.q_scale;
+}
+template <bool F32>
+__device__ __forceinline__ float value_at(const LinearAttnArgs& p, int t, int h, int c) {
+  const float v = ldx(p.v, (int64_t)t * p.ldv + h * p.V + c, F32 ? 1 : 0);
+  return p.in_silu ? silu_f(v) : v;
+}
+// weight and gate of output channel c of head h at token t
+template <bool F32>
+__device__ __forceinline__ float weight_gate(const LinearAttnArgs& p, int t, int h, int c) {
+  const float g = ldx(p.g, (int64_t)t * p.ldg + h * p.V + c, F32 ? 1 : 0);
+  return (p.nw == nullptr ? 1.f : p.nw[p.norm_full ? h * p.V + c : c]) * (p.gate_silu ? silu_f(g) : sigm(g));
+}
+
+constexpr int ST = 8;   // tokens the short kernel stages at a time
+
+// grid (sequence, head): sequences of at most `lim` tokens, key and value size up to P. PRE: with a bonus.
+// Bound by the state's bytes once sequences x heads fill the chip: 64 sequences x 8 heads of 128 (67 MB) 17.4 us, three launches
+// 35.2; a further token costs 1.1 us.
+template <int P, bool F32, bool PRE>
+__global__ __launch_bounds__(256) void linear_short_kernel(LinearAttnArgs p, int lim, float* __restrict__ oraw) {
+  constexpr int CG = P / 4, KW = 64 / CG, KG = 4 * KW, KP = P / KG;   // column groups, key groups (of a wave; all), keys of a group
+  __shared__ __attribute__((aligned(16))) float la[ST][P], lk[ST][P], lq[ST][P], lu[PRE ? ST : 1][P], lv[ST][P], lg[ST][P];
+  __shared__ __attribute__((aligned(16))) float lo[ST][4][P];   // the waves' parts of the outputs
+  const int s = blockIdx.x, h = blockIdx.y;
+  const int slot = p.state_slots[s];
+  const int t0 = p.query_start[s], t1 = p.query_start[s + 1];
+  if (slot < 0 || t1 <= t0 || t1 - t0 > lim) return;
+  const int D = p.D, V = p.V, tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+  const int c = 4 * (lane % CG), k0 = KP * (wv * KW + lane / CG);
+  const bool from_zero = p.context_lens[s] - (t1 - t0) <= 0;
+  float* sp = p.state + ((int64_t)slot * p.H + h) * D * V;
+  const bool vec4 = V % 4 == 0 && reinterpret_cast<uintptr_t>(sp) % 16 == 0;
+  f32x4 S[KP];
+#pragma unroll
+  for (int j = 0; j < KP; ++j) {
+    S[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (from_zero || k0 + j >= D || c >= V) continue;
+    const float* x = sp + (int64_t)(k0 + j) * V + c;
+    if (vec4) S[j] = ld4(x);
+    else
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[j][e] = c + e < V ? x[e] : 0.f;
+  }
+  for (int tb = t0; tb < t1; tb += ST) {
+    if (tb > t0) __syncthreads();
+    {  // 32 lanes per token; channels past D: k = q = 0, a = 1 (their state stays zero)
+      const int i = tid >> 5, l = tid & 31, t = tb + i;
+#pragma unroll
+      for (int m = 0; m < P / 32; ++m) {
+        const int d = l + 32 * m;
+        float a = 1.f, k = 0.f, q = 0.f;
+        if (t < t1 && d < D) decay_key_query<F32>(p, t, h, d, a, k, q);
+        la[i][d] = a; lk[i][d] = k; lq[i][d] = q;
+        if (PRE) lu[i][d] = d < D ? p.bonus[h * D + d] * k : 0.f;
+        const bool ok = t < t1 && d < V;
+        lv[i][d] = ok ? value_at<F32>(p, t, h, d) : 0.f;
+        if (!p.norm_all) lg[i][d] = ok ? weight_gate<F32>(p, t, h, d) : 0.f;
+      }
+    }
+    __syncthreads();
+    const int nt = min(ST, t1 - tb);
+    for (int i = 0; i < nt; ++i) {
+      const f32x4 v = ld4(&lv[i][c]);
+      f32x4 O = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < KP; ++j) {
+        const float a = la[i][k0 + j], k = lk[i][k0 + j], q = lq[i][k0 + j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (PRE) O[e] = fmaf(q, fmaf(lu[i][k0 + j], v[e], S[j][e]), O[e]);   // the state before its update
+          S[j][e] = fmaf(k, v[e], a * S[j][e]);
+          if (!PRE) O[e] = fmaf(q, S[j][e], O[e]);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (KW >= 8) O[e] += row_rot<0x128>(O[e]);
+        if (KW >= 4) O[e] += xor16(O[e]);
+        O[e] += xor32(O[e]);
+      }
+      if (lane < CG) *reinterpret_cast<f32x4*>(&lo[i][wv][c]) = O;
+    }
+    __syncthreads();
+    {  // the outputs of the staged tokens: head norm, weight, gate; raw where the norm spans the heads
+      const int i = tid >> 5, l = tid & 31, t = tb + i;
+      float o[P / 32], ss = 0.f;
+#pragma unroll
+      for (int m = 0; m < P / 32; ++m) {
+        const int d = l + 32 * m;
+        o[m] = lo[i][0][d] + lo[i][1][d] + (lo[i][2][d] + lo[i][3][d]);   // (columns past V are zero)
+        ss = fmaf(o[m], o[m], ss);
+      }
+      const float inv = 1.f / sqrtf(half_sum(ss) / (float)V + p.eps);
+#pragma unroll
+      for (int m = 0; m < P / 32; ++m) {
+        const int d = l + 32 * m;
+        if (t >= t1 || d >= V) continue;
+        if (p.norm_all) {
+          oraw[((int64_t)t * p.H + h) * V + d] = o[m];
+          continue;
+        }
+        const float y = o[m] * inv * lg[i][d];
+        const int64_t oi = (int64_t)t * p.ldo + h * V + d;
+        if (F32) reinterpret_cast<float*>(p.out)[oi] = y;
+        else reinterpret_cast<bf16_t*>(p.out)[oi] = f2bf(y);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < KP; ++j) {
+    if (k0 + j >= D || c >= V) continue;
+    float* x = sp + (int64_t)(k0 + j) * V + c;
+    if (vec4) *reinterpret_cast<f32x4*>(x) = S[j];
+    else
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < V) x[e] = S[j][e];
+  }
+}
+
+constexpr int CT = 64;         // tokens of a chunk
+constexpr int CTP = CT + 4;    // padded rows of tokens: 16 lanes' 16-B pieces of 16 rows fall into all 64 banks
+
+// grid (chunk, head): cstate[chunk][h] = sum_j g_(j+1..CT) k_j v_j^T [D][V], cdecay = g_(1..CT). MFMA operands: the token
+// 16 n + 4 kg + e is element e of lane group kg in both operands, so a lane's four steps are one 16-B piece of a row.
+template <int DP, bool F32>
+__global__ __launch_bounds__(256) void linear_local_kernel(LinearAttnArgs p, int lim, float* __restrict__ cstate,
+                                                            float* __restrict__ cdecay) {
+  constexpr int DT = (DP / 16 + 3) / 4;   // channel tiles of a wave
+  __shared__ __attribute__((aligned(16))) float kt[DP][CTP], vt[128][CTP];
+  __shared__ float late[DP];
+  int s, t0, t1;
+  if (!locate_chunk<CT>(p.query_start, p.state_slots, p.S, lim, blockIdx.x, s, t0, t1)) return;
+  const int h = blockIdx.y, D = p.D, V = p.V, tid = threadIdx.x;
+  const int half = tid >> 7, j0 = half * (CT / 2);
+  {
+    const int d = tid & 127;
+    float k[CT / 2], g = 1.f;
+    if (d < DP) {   // from the half's last token to its first: k_j times the decays after it
+      float a[CT / 2];
+#pragma unroll
+      for (int j = 0; j < CT / 2; ++j) {
+        a[j] = 1.f; k[j] = 0.f;
+        float q;
+        if (d < D && t0 + j0 + j < t1) decay_key_query<F32>(p, t0 + j0 + j, h, d, a[j], k[j], q);
+        if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int j = CT / 2 - 1; j >= 0; --j) {
+        k[j] *= g;
+        g *= a[j];
+      }
+      if (half == 1) late[d] = g;
+    }
+#pragma unroll
+    for (int j = 0; j < CT / 2; j += 4) {   // values, a column per thread
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = d < V && t0 + j0 + j + e < t1 ? value_at<F32>(p, t0 + j0 + j + e, h, d) : 0.f;
+      *reinterpret_cast<f32x4*>(&vt[d][j0 + j]) = v;
+    }
+    __syncthreads();
+    if (d < DP) {
+      const float f = half == 0 ? late[d] : 1.f;
+#pragma unroll
+      for (int j = 0; j < CT / 2; j += 4)
+        *reinterpret_cast<f32x4*>(&kt[d][j0 + j]) = f32x4{k[j] * f, k[j + 1] * f, k[j + 2] * f, k[j + 3] * f};
+      if (half == 0 && d < D) cdecay[((int64_t)blockIdx.x * p.H + h) * D + d] = g * f;
+    }
+  }
+  __syncthreads();
+  const int w = tid >> 6, l = tid & 63, lr = l & 15, kg = l >> 4;
+  float* cs = cstate + ((int64_t)blockIdx.x * p.H + h) * D * V;
+  f32x4 acc[DT][8];
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int n = 0; n < CT / 16; ++n) {
+    f32x4 A[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t) A[t] = ld4(&kt[min(16 * (w * DT + t), DP - 16) + lr][16 * n + 4 * kg]);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (16 * u >= V) continue;
+      const f32x4 B = ld4(&vt[16 * u + lr][16 * n + 4 * kg]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < DT; ++t) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[t][e], B[e], acc[t][u], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int d = 16 * (w * DT + t) + 4 * kg + i, c = 16 * u + lr;
+        if (d < D && c < V) cs[(int64_t)d * V + c] = acc[t][u][i];
+      }
+}
+
+// grid (sequence, head, stretches of 256 state entries): as linear_carry_kernel, over the chunks of CT tokens; eight chunks'
+// local states are asked for at a time
+__global__ __launch_bounds__(256) void linear_chunk_carry_kernel(LinearAttnArgs p, int lim, float* __restrict__ cstate,
+                                                                  const float* __restrict__ cdecay) {
+  const int s = blockIdx.x, h = blockIdx.y;
+  const int slot = p.state_slots[s];
+  const int t0 = p.query_start[s], t1 = p.query_start[s + 1];
+  if (slot < 0 || t1 - t0 <= lim) return;
+  const int64_t c0 = first_chunk<CT>(p.query_start, p.state_slots, lim, s);   // (whole waves)
+  const int D = p.D, V = p.V, e = blockIdx.z * 256 + threadIdx.x;
+  if (e >= D * V) return;
+  const int nc = (t1 - t0 + CT - 1) / CT;
+  float* sp = p.state + ((int64_t)slot * p.H + h) * D * V;
+  const int64_t step = (int64_t)p.H * D * V, dstep = (int64_t)p.H * D;
+  float* cs = cstate + (c0 * p.H + h) * D * V + e;
+  const float* cd = cdecay + (c0 * p.H + h) * D + e / V;
+  float cur = p.context_lens[s] - (t1 - t0) <= 0 ? 0.f : sp[e];
+  for (int c = 0; c < nc; c += 8) {
+    float loc[8], dec[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int j = min(c + i, nc - 1);
+      loc[i] = cs[j * step];
+      dec[i] = cd[j * dstep];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (c + i < nc) {
+        cs[(c + i) * step] = cur;
+        cur = fmaf(dec[i], cur, loc[i]);
+      }
+  }
+  sp[e] = cur;
+}
+
+// grid (chunk, head), 512 threads: the outputs of a chunk from the state it starts from. Wave w owns the columns 16 w ..
+template <int DP, bool F32, bool PRE>
+__global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, int lim, const float* __restrict__ cstate,
+                                                             float* __restrict__ oraw) {
+  constexpr int X = DP / 32, NT = DP / 16, DS = DP + 4;   // (padded rows, as CTP)
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* la = lds;                    // [CT][DS] decays
+  float* lk = la + CT * DS;           // keys
+  float* lq = lk + CT * DS;           // queries, then times the decays up to them
+  float* tr = lq + CT * DS;           // [CT][CTP] the triangle
+  float* red = tr + CT * CTP;         // [8][CT] rows' sums of squares; before, [4][DP] decays of 16 tokens
+  int s, t0, t1;
+  if (!locate_chunk<CT>(p.query_start, p.state_slots, p.S, lim, blockIdx.x, s, t0, t1)) return;
+  const int h = blockIdx.y, D = p.D, V = p.V, tid = threadIdx.x;
+  const int w = tid >> 6, l = tid & 63, lr = l & 15, kg = l >> 4;
+  const int col = 16 * w + lr;
+  const bool con = col < V;
+  // B operands straight from memory: the state (channels 16 n + 4 kg + e) and the values (tokens 16 n + 4 kg + e) of the column
+  f32x4 B[NT], vb[CT / 16];
+  const float* cs = cstate + ((int64_t)blockIdx.x * p.H + h) * D * V;
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int d = 16 * n + 4 * kg + e;
+      B[n][e] = con && d < D ? cs[(int64_t)d * V + col] : 0.f;
+    }
+#pragma unroll
+  for (int n = 0; n < CT / 16; ++n)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int t = t0 + 16 * n + 4 * kg + e;
+      vb[n][e] = con && t < t1 ? value_at<F32>(p, t, h, col) : 0.f;
+    }
+#pragma unroll 4
+  for (int e = tid; e < CT * DP; e += 512) {
+    const int i = e / DP, d = e % DP;
+    float a = 1.f, k = 0.f, q = 0.f;
+    if (d < D && t0 + i < t1) decay_key_query<F32>(p, t0 + i, h, d, a, k, q);
+    la[i * DS + d] = a; lk[i * DS + d] = k; lq[i * DS + d] = q;
+  }
+  for (int e = tid; e < CT * CTP; e += 512) tr[e] = 0.f;
+  __syncthreads();
+  {  // the triangle: a wave owns eight columns j, lane = (channel group dg of eight, j). A column has CT - j rows: waves w and
+     // w + 4, which share a SIMD, take stretches that add up alike
+    const int jb = w < 4 ? w : 11 - w;
+    const int dg = l >> 3, j = 8 * jb + (l & 7);
+    float x[4 * X], diag = 0.f;
+#pragma unroll
+    for (int m = 0; m < X; ++m)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int d = 32 * m + 4 * dg + c;
+        x[4 * m + c] = lk[j * DS + d];
+        if (PRE) diag = fmaf(lq[j * DS + d] * (d < D ? p.bonus[h * D + d] : 0.f), x[4 * m + c], diag);
+      }
+    if (PRE) diag = key_sum<8>(diag);
+    for (int i = 8 * jb; i < CT; ++i) {
+      float r = 0.f;
+#pragma unroll
+      for (int m = 0; m < X; ++m) {
+        const f32x4 a = ld4(&la[i * DS + 32 * m + 4 * dg]), q = ld4(&lq[i * DS + 32 * m + 4 * dg]);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          if (PRE) r = fmaf(q[c], x[4 * m + c], r);
+          if (i > j) x[4 * m + c] *= a[c];
+          if (!PRE) r = fmaf(q[c], x[4 * m + c], r);
+        }
+      }
+      r = key_sum<8>(r);
+      if (PRE && i == j) r = diag;
+      if (dg == 0 && i >= j) tr[i * CTP + j] = r;
+    }
+  }
+  __syncthreads();
+  {  // q_i g_(1..i) (with a bonus g_(1..i-1)) in place: a channel and 16 tokens per thread
+    const int d = tid & 127, part = tid >> 7;
+    float g = 1.f;
+    if (d < DP)
+      for (int i = 16 * part; i < 16 * part + 16; ++i) {
+        if (!PRE) g *= la[i * DS + d];
+        lq[i * DS + d] *= g;
+        if (PRE) g *= la[i * DS + d];
+      }
+    if (d < DP) red[part * DP + d] = g;
+    __syncthreads();
+    if (d < DP && part > 0) {
+      float f = 1.f;
+      for (int m = 0; m < part; ++m) f *= red[m * DP + d];
+      for (int i = 16 * part; i < 16 * part + 16; ++i) lq[i * DS + d] *= f;
+    }
+  }
+  __syncthreads();
+  f32x4 acc[CT / 16];
+#pragma unroll
+  for (int r = 0; r < CT / 16; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    f32x4 A[CT / 16];
+#pragma unroll
+    for (int r = 0; r < CT / 16; ++r) A[r] = ld4(&lq[(16 * r + lr) * DS + 16 * n + 4 * kg]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int r = 0; r < CT / 16; ++r) acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[r][e], B[n][e], acc[r], 0, 0, 0);
+  }
+#pragma unroll
+  for (int n = 0; n < CT / 16; ++n) {
+    f32x4 A[CT / 16];
+#pragma unroll
+    for (int r = n; r < CT / 16; ++r) A[r] = ld4(&tr[(16 * r + lr) * CTP + 16 * n + 4 * kg]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int r = n; r < CT / 16; ++r) acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[r][e], vb[n][e], acc[r], 0, 0, 0);
+  }
+  // acc[r][i]: token 16 r + 4 kg + i, column col (columns past V are zero)
+  if (p.norm_all) {
+#pragma unroll
+    for (int r = 0; r < CT / 16; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = t0 + 16 * r + 4 * kg + i;
+        if (con && t < t1) oraw[((int64_t)t * p.H + h) * V + col] = acc[r][i];
+      }
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < CT / 16; ++r)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float ss = acc[r][i] * acc[r][i];
+      ss += row_rot<0x128>(ss);
+      ss += row_rot<0x124>(ss);
+      ss += row_rot<0x122>(ss);
+      ss += row_rot<0x121>(ss);
+      if (lr == 0) red[w * CT + 16 * r + 4 * kg + i] = ss;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < CT / 16; ++r)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 16 * r + 4 * kg + i, t = t0 + row;
+      if (!con || t >= t1) continue;
+      float ss = 0.f;
+#pragma unroll
+      for (int m = 0; m < 8; ++m) ss += red[m * CT + row];
+      const float y = acc[r][i] * (1.f / sqrtf(ss / (float)V + p.eps)) * weight_gate<F32>(p, t, h, col);
+      const int64_t oi = (int64_t)t * p.ldo + h * V + col;
+      if (F32) reinterpret_cast<float*>(p.out)[oi] = y;
+      else reinterpret_cast<bf16_t*>(p.out)[oi] = f2bf(y);
+    }
+}
+
+// Tokens a sequence may have in a step to be run one by one: a chunk of 64 costs what 50 tokens do, and its three launches more.
+int short_limit(int T) { return T <= 96 ? T : 64; }
+// chunks of a step whose sequences longer than lim tokens have T between them: each has at most one that is not whole
+int long_chunks(int T, int lim) { return T <= lim ? 0 : T / CT + T / (lim + 1); }
+// Decoding steps: one launch instead of three (16 sequences x 8 heads of 128: 25.3 -> 11.7 us). Long steps: chunks with fp32 MFMA
+// (2048 tokens 162 -> 128 us, 63 decoded tokens beside a portion of 961 1054 -> 206, 64 portions of 16 62 -> 51). Between them
+// the scan below, which spreads a head's columns over several workgroups, is ahead where sequences are few: one portion of
+// 64 58 us (here 79), of 256 90 (103), 8 of 48 54 (68).
+bool takes_small(int T, int S, int D, int V, int cols_per_lane) {
+  return D <= 128 && V <= 128 && cols_per_lane == 0 &&
+         (T <= 2 * S || T >= (S == 1 ? 1024 : (S < 16 ? 512 : 256)));
+}
+
+template <int DP, bool F32, bool PRE>
+void launch_small(const LinearAttnArgs& a, int T, float* oraw, float* cstate, float* cdecay, hipStream_t st) {
+  // T counts padding rows too, so a sequence may be much shorter. A lone one then takes chunks whatever its length (not more
+  // of them than any step of T rows); several are told apart by their lengths on the device.
+  const int P = max(a.D, a.V);
+  int lim = short_limit(T), chunks = long_chunks(T, lim);
+  if (a.S == 1 && T > lim) {
+    lim = 0;
+    chunks = (T + CT - 1) / CT;
+  }
+  if (lim > 0) {
+    const dim3 grid(a.S, a.H);
+    if (P <= 32) hipLaunchKernelGGL((linear_short_kernel<32, F32, PRE>), grid, dim3(256), 0, st, a, lim, oraw);
+    else if (P <= 64) hipLaunchKernelGGL((linear_short_kernel<64, F32, PRE>), grid, dim3(256), 0, st, a, lim, oraw);
+    else hipLaunchKernelGGL((linear_short_kernel<128, F32, PRE>), grid, dim3(256), 0, st, a, lim, oraw);
+  }
+  if (chunks > 0) {
+    constexpr size_t bytes = ((size_t)3 * CT * (DP + 4) + CT * CTP + 8 * CT) * 4;
+    auto out = linear_output_kernel<DP, F32, PRE>;
+    static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(out), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 (int)bytes) == hipSuccess;
+    (void)attr;
+    hipLaunchKernelGGL((linear_local_kernel<DP, F32>), dim3(chunks, a.H), dim3(256), 0, st, a, lim, cstate, cdecay);
+    hipLaunchKernelGGL(linear_chunk_carry_kernel, dim3(a.S, a.H, (a.D * a.V + 255) / 256), dim3(256), 0, st, a, lim, cstate, cdecay);
+    hipLaunchKernelGGL(out, dim3(chunks, a.H), dim3(512), bytes, st, a, lim, cstate, oraw);
+  }
+  if (a.norm_all) hipLaunchKernelGGL(linear_finish_kernel, dim3(T), dim3(256), 0, st, a, oraw);
+}
+
+template <int DP>
+void launch_small_dp(const LinearAttnArgs& a, int T, float* oraw, float* cstate, float* cdecay, hipStream_t st) {
+  if (a.f32) {
+    if (a.bonus != nullptr) launch_small<DP, true, true>(a, T, oraw, cstate, cdecay, st);
+    else launch_small<DP, true, false>(a, T, oraw, cstate, cdecay, st);
+  } else {
+    if (a.bonus != nullptr) launch_small<DP, false, true>(a, T, oraw, cstate, cdecay, st);
+    else launch_small<DP, false, false>(a, T, oraw, cstate, cdecay, st);
+  }
+}
+
 }  // namespace
 
 int linear_attn_chunk_size(int T, int S) {
@@ -328,7 +811,9 @@ int linear_attn_chunk_size(int T, int S) {
 int linear_attn_chunks(int T, int S, int CH) { return CH > 0 ? T / CH + S : 0; }
 size_t linear_attn_scratch_floats(int T, int S, int H, int D, int V) {
   const int CH = linear_attn_chunk_size(T, S);
-  return (size_t)T * H * (4 * D + 2 * V) + (size_t)linear_attn_chunks(T, S, CH) * H * D * (V + 1);
+  const size_t any = (size_t)T * H * (4 * D + 2 * V) + (size_t)linear_attn_chunks(T, S, CH) * H * D * (V + 1);
+  const size_t small = (size_t)T * H * V + (size_t)long_chunks(T, short_limit(T)) * H * D * (V + 1);
+  return takes_small(T, S, D, V, 0) && small > any ? small : any;
 }
 
 // scratch: linear_attn_scratch_floats(): {a, k, q, -} per key channel, the values, the raw outputs, and for
@@ -336,6 +821,14 @@ size_t linear_attn_scratch_floats(int T, int S, int H, int D, int V) {
 void launch_linear_attn(const LinearAttnArgs& a, int T, float* scratch, hipStream_t st) {
   if (a.S <= 0 || a.H <= 0 || T <= 0) return;
   const int64_t nk = (int64_t)T * a.H * a.D, nv = (int64_t)T * a.H * a.V;
+  if (takes_small(T, a.S, a.D, a.V, a.cols_per_lane)) {   // scratch: raw outputs, the chunks' states, their decays
+    float* states = scratch + nv;
+    float* decays = states + (size_t)long_chunks(T, short_limit(T)) * a.H * a.D * a.V;
+    if (a.D <= 32) launch_small_dp<32>(a, T, scratch, states, decays, st);
+    else if (a.D <= 64) launch_small_dp<64>(a, T, scratch, states, decays, st);
+    else launch_small_dp<128>(a, T, scratch, states, decays, st);
+    return;
+  }
   float4* vec = reinterpret_cast<float4*>(scratch);
   float* vals = scratch + 4 * nk;
   float* oraw = vals + nv;
