@@ -5,7 +5,7 @@
 //   kp [pages][G][NP][D],   vp [pages][G][NP][V]         pooled rows, NP = ceil(page / P): block b's row
 //                                                        lives in the page of its last position e = b P + P - 1,
 //                                                        at index (e mod page) / P
-// window_write  one workgroup per token: query / key RMS norm (per head or over the whole projection,
+// window_write  one wave per (token, head): query / key RMS norm (per head or over the whole projection,
 //               fp32 statistics), interleaved-pair rotation of the leading rot_dims entries of every head
 //               (angle = position * inv_freq in fp32, full-range sin / cos), values optionally turned over
 //               all of V, the paged stores, and the prepared query rows.
@@ -77,90 +77,106 @@ __device__ __forceinline__ int first_key(const WindowArgs& a, int p) {
   return a.chunk > 0 ? max(lo, p - p % a.chunk) : lo;
 }
 
+// One wave per head (queries, keys, values), D <= 128 NP. A lane holds NP pairs of entries and turns each with one angle; nothing goes
+// through LDS and no wave waits for another (a norm over the whole projection is summed by every wave for itself). What bounds it
+// is the way to memory and back, three times (slot and position, row, store), and the angles. 16 tokens of 12 heads of 128: 5.0 us,
+// 2048: 17; a workgroup per token, whose elements went through LDS and took an angle each, 10.5 and 22.
+template <int NP, bool F32>
 __global__ __launch_bounds__(256) void window_write_kernel(WindowArgs a, const void* __restrict__ q, int64_t ldq,
-                                                            const void* __restrict__ k, int64_t ldk,
-                                                            const void* __restrict__ v, int64_t ldv,
-                                                            const float* __restrict__ qw, const float* __restrict__ kw,
-                                                            float eps, int norm_all, void* __restrict__ q_out,
-                                                            bf16_t* __restrict__ vt, const float* __restrict__ q_head_scale,
-                                                            float q_temp_coef, int q_temp_every, int rot_half,
-                                                            const void* __restrict__ v_other, int64_t ldo, float lam) {
-  extern __shared__ float lds[];
+                                                                  const void* __restrict__ k, int64_t ldk,
+                                                                  const void* __restrict__ v, int64_t ldv,
+                                                                  const float* __restrict__ qw, const float* __restrict__ kw, float eps,
+                                                                  int norm_all, void* __restrict__ q_out, bf16_t* __restrict__ vt,
+                                                                  const float* __restrict__ q_head_scale, float q_temp_coef,
+                                                                  int q_temp_every, int rot_half, const void* __restrict__ v_other,
+                                                                  int64_t ldo, float lam) {
+  constexpr int f32 = F32 ? 1 : 0;
   const int H = a.H, G = a.G, D = a.D, V = a.V, GV = a.GV;
-  float* xs = lds;                    // [(H + G) * D] q heads then k heads
-  float* inv = xs + (H + G) * D;      // [H + G]
-  const int t = blockIdx.x;
+  const int t = blockIdx.x, h = 4 * blockIdx.y + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int slot = a.slots[t];
-  if (slot < 0) return;  // padding row (uniform per block)
-  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
-  for (int e = tid; e < H * D; e += 256) xs[e] = ldx(q, (int64_t)t * ldq + e, a.f32);
-  for (int e = tid; e < G * D; e += 256) xs[H * D + e] = ldx(k, (int64_t)t * ldk + e, a.f32);
-  __syncthreads();
-  if (qw != nullptr) {
-    for (int h = wv; h < H + G; h += 4) {  // sum of squares per head
-      float ss = 0.f;
-      for (int d = lane; d < D; d += 64) ss = fmaf(xs[h * D + d], xs[h * D + d], ss);
-      ss = wave_reduce_sum(ss);
-      if (lane == 0) inv[h] = ss;
-    }
-    __syncthreads();
-    float mine = 0.f;
-    if (norm_all) {
-      float sq = 0.f, sk = 0.f;
-      for (int h = 0; h < H; ++h) sq += inv[h];
-      for (int h = 0; h < G; ++h) sk += inv[H + h];
-      if (tid < H + G) mine = 1.f / sqrtf((tid < H ? sq / (float)(H * D) : sk / (float)(G * D)) + eps);
-    } else if (tid < H + G) {
-      mine = 1.f / sqrtf(inv[tid] / (float)D + eps);
-    }
-    __syncthreads();
-    if (tid < H + G) inv[tid] = mine;
-    __syncthreads();
-  }
-  const float pos = (float)a.positions[t];
-  // query temperature of the position: 1 + coef ln(floor((p + 1) / every) + 1)
-  const float qgrow = q_temp_coef != 0.f ? 1.f + q_temp_coef * logf((float)((a.positions[t] + 1) / q_temp_every) + 1.f) : 1.f;
+  if (slot < 0 || h >= H + G + GV) return;  // padding row, no head
+  const int ipos = a.positions[t];
+  const float pos = (float)ipos;
   const int page = a.page;
   const int64_t pg = slot / page, off = slot % page;
-  for (int e = tid; e < (H + G) * D; e += 256) {
-    const int h = e / D, i = e % D;
+  if (h < H + G) {
     const bool isq = h < H;
+    const void* src = isq ? q : k;
+    const int64_t ro = isq ? (int64_t)t * ldq + (int64_t)h * D : (int64_t)t * ldk + (int64_t)(h - H) * D;
     const float* w = isq ? qw : kw;
-    const int wo = norm_all ? (isq ? h : h - H) * D : 0;
-    const float sc = w != nullptr ? inv[h] : 1.f;
-    float o;
-    if (i < a.rot_dims) {  // the pair (i0, i1) = (2j, 2j + 1), or (j, j + rot_dims / 2) with rot_half
-      const int hr = a.rot_dims >> 1;
-      const int j = rot_half ? (i < hr ? i : i - hr) : (i >> 1);
-      const int i0 = rot_half ? j : (i & ~1), i1 = rot_half ? j + hr : (i | 1);
-      const float x0 = xs[h * D + i0] * sc * (w ? w[wo + i0] : 1.f), x1 = xs[h * D + i1] * sc * (w ? w[wo + i1] : 1.f);
-      const float ang = pos * a.inv_freq[j];
-      const float cs = cosf(ang), sn = sinf(ang);
-      o = (i == i1) ? (x1 * cs + x0 * sn) : (x0 * cs - x1 * sn);
-    } else {
-      o = xs[h * D + i] * sc * (w ? w[wo + i] : 1.f);
+    if (w != nullptr && norm_all) w += (isq ? h : h - H) * D;   // (one weight per entry of the projection)
+    const int hr = a.rot_dims >> 1;
+    int i0[NP], i1[NP];
+    float x0[NP], x1[NP], w0[NP], w1[NP], f[NP], ss = 0.f;
+#pragma unroll
+    for (int m = 0; m < NP; ++m) {  // pairs (2j, 2j + 1), or (j, j + rot_dims / 2) with rot_half; past the turned entries neighbours
+      const int j = lane + 64 * m;
+      i0[m] = j < hr && rot_half ? j : 2 * j;
+      i1[m] = j < hr && rot_half ? j + hr : 2 * j + 1;
+      x0[m] = i0[m] < D ? ldx(src, ro + i0[m], f32) : 0.f;
+      x1[m] = i1[m] < D ? ldx(src, ro + i1[m], f32) : 0.f;
+      w0[m] = w != nullptr && i0[m] < D ? w[i0[m]] : 1.f;
+      w1[m] = w != nullptr && i1[m] < D ? w[i1[m]] : 1.f;
+      f[m] = j < hr ? a.inv_freq[j] : 0.f;
+      ss = fmaf(x0[m], x0[m], fmaf(x1[m], x1[m], ss));
     }
-    if (isq) stx(q_out, (int64_t)t * H * D + e, a.f32, o * (q_head_scale != nullptr ? q_head_scale[h] * qgrow : qgrow));
-    else stx(a.kc, ((pg * G + (h - H)) * page + off) * D + i, a.f32, o);
+    float count = (float)D;
+    if (norm_all && w != nullptr) {
+      const int n = (isq ? H : G) * D;
+      const int64_t r0 = isq ? (int64_t)t * ldq : (int64_t)t * ldk;
+      count = (float)n;
+      ss = 0.f;
+      for (int e0 = lane; e0 < n; e0 += 64 * 8) {
+        float x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = ldx(src, r0 + min(e0 + 64 * u, n - 1), f32);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) ss = e0 + 64 * u < n ? fmaf(x[u], x[u], ss) : ss;
+      }
+    }
+    const float sc = w != nullptr ? 1.f / sqrtf(wave_reduce_sum(ss) / count + eps) : 1.f;
+    float grow = 1.f;
+    if (isq) {  // query temperature of the position: 1 + coef ln(floor((p + 1) / every) + 1)
+      if (q_temp_coef != 0.f) grow = 1.f + q_temp_coef * logf((float)((ipos + 1) / q_temp_every) + 1.f);
+      if (q_head_scale != nullptr) grow = q_head_scale[h] * grow;
+    }
+    void* dst = isq ? q_out : a.kc;
+    const int64_t so = isq ? ((int64_t)t * H + h) * D : ((pg * G + (h - H)) * page + off) * D;
+#pragma unroll
+    for (int m = 0; m < NP; ++m) {
+      float y0 = x0[m] * sc * w0[m], y1 = x1[m] * sc * w1[m];
+      if (lane + 64 * m < hr) {
+        float sn, cs;
+        sincosf(pos * f[m], &sn, &cs);
+        const float z0 = y0 * cs - y1 * sn, z1 = y1 * cs + y0 * sn;
+        y0 = z0; y1 = z1;
+      }
+      if (i0[m] < D) stx(dst, so + i0[m], f32, isq ? y0 * grow : y0);
+      if (i1[m] < D) stx(dst, so + i1[m], f32, isq ? y1 * grow : y1);
+    }
+    return;
   }
-  const int vrot = a.v_freq != nullptr ? 2 * (V / 2) : 0;
-  auto val = [&](int e) {  // entry e of the token's values, blended with the other row's
-    const float x = ldx(v, (int64_t)t * ldv + e, a.f32);
-    return v_other != nullptr ? fmaf(lam, ldx(v_other, (int64_t)t * ldo + e, a.f32), (1.f - lam) * x) : x;
+  const int g = h - H - G;
+  const int64_t vo = ((pg * GV + g) * page + off) * V, to = (pg * GV + g) * V;
+  auto val = [&](int i) {  // entry i of the head's values, blended with the other row's
+    const float x = ldx(v, (int64_t)t * ldv + (int64_t)g * V + i, f32);
+    return v_other != nullptr ? fmaf(lam, ldx(v_other, (int64_t)t * ldo + (int64_t)g * V + i, f32), (1.f - lam) * x) : x;
   };
-  for (int e = tid; e < GV * V; e += 256) {
-    const int g = e / V, i = e % V;
-    float o;
-    if (i < vrot) {
-      const float x0 = val(g * V + (i & ~1)), x1 = val(g * V + (i | 1));
-      const float ang = pos * a.v_freq[i >> 1];
-      const float cs = cosf(ang), sn = sinf(ang);
-      o = (i & 1) ? (x1 * cs + x0 * sn) : (x0 * cs - x1 * sn);
-    } else {
-      o = val(e);
+  for (int j = lane; 2 * j < V; j += 64) {
+    const int i = 2 * j;
+    float y0 = val(i), y1 = i + 1 < V ? val(i + 1) : 0.f;
+    if (a.v_freq != nullptr && i + 1 < V) {
+      float sn, cs;
+      sincosf(pos * a.v_freq[j], &sn, &cs);
+      const float z0 = y0 * cs - y1 * sn, z1 = y1 * cs + y0 * sn;
+      y0 = z0; y1 = z1;
     }
-    stx(a.vc, ((pg * GV + g) * page + off) * V + i, a.f32, o);
-    if (vt != nullptr) vt[((pg * GV + g) * V + i) * page + off] = f2bf(o);  // [page][GV][column][key in page]
+    stx(a.vc, vo + i, f32, y0);
+    if (i + 1 < V) stx(a.vc, vo + i + 1, f32, y1);
+    if (vt != nullptr) {  // [page][GV][column][key in page]
+      vt[(to + i) * page + off] = f2bf(y0);
+      if (i + 1 < V) vt[(to + i + 1) * page + off] = f2bf(y1);
+    }
   }
 }
 
@@ -1104,8 +1120,11 @@ void launch_window_write(const WindowArgs& a, const void* q, int64_t ldq, const 
                          const float* q_head_scale, float q_temp_coef, int q_temp_every, int rot_half, const void* v_other,
                          int64_t ldo, float lam, hipStream_t st) {
   if (a.T <= 0) return;
-  const size_t lds = (size_t)((a.H + a.G) * a.D + a.H + a.G) * sizeof(float);
-  hipLaunchKernelGGL(window_write_kernel, dim3(a.T), dim3(256), lds, st, a, q, ldq, k, ldk, v, ldv, qw, kw, eps, norm_all,
+  // (D <= 1024: window_attn_fits())
+  auto kern = a.D <= 128 ? (a.f32 ? window_write_kernel<1, true> : window_write_kernel<1, false>)
+            : a.D <= 256 ? (a.f32 ? window_write_kernel<2, true> : window_write_kernel<2, false>)
+                         : (a.f32 ? window_write_kernel<8, true> : window_write_kernel<8, false>);
+  hipLaunchKernelGGL(kern, dim3(a.T, (a.H + a.G + a.GV + 3) / 4), dim3(256), 0, st, a, q, ldq, k, ldk, v, ldv, qw, kw, eps, norm_all,
                      q_out, reinterpret_cast<bf16_t*>(vt), q_head_scale, q_temp_coef, q_temp_every, rot_half, v_other, ldo, lam);
 }
 
