@@ -1,7 +1,7 @@
 // What the recurrences that take a portion in chunks of CN tokens share (gated_delta.hip, delta_rule.hip): where a chunk
 // lies, sums over lanes, packed lower triangles and their products with a column kept in registers.
 #pragma once
-#include "common.h"
+#include "locate.h"
 
 namespace vgate {
 namespace {
@@ -29,44 +29,22 @@ __device__ __forceinline__ int chunks_of(const int32_t* state_slots, int lim, in
   return (state_slots[i] < 0 || b - a <= lim) ? 0 : (b - a + C - 1) / C;
 }
 
-// chunk `bx` of a step: its sequence and token range (chunks are numbered sequence by sequence). Whole waves: a lane per sequence
-// (one after another they cost 0.5 us each, three times per layer).
+// chunk `bx` of a step: its sequence and token range (chunks are numbered sequence by sequence)
 template <int C = CN>
 __device__ __forceinline__ bool locate_chunk(const int32_t* query_start, const int32_t* state_slots, int S, int lim, int bx, int& s,
                                              int& t0, int& t1) {
-  const int lane = threadIdx.x & 63;
-  int base = 0;
-  for (int s0 = 0; s0 < S; s0 += 64) {
-    const int i = s0 + lane;
-    const int a = i < S ? query_start[i] : 0, b = i < S ? query_start[i + 1] : 0;
-    const int n = i < S ? chunks_of<C>(state_slots, lim, i, a, b) : 0;
-    int end = n;   // inclusive sum over the lanes
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(end, o, 64);
-      if (lane >= o) end += v;
-    }
-    const unsigned long long hit = __ballot(bx >= base + end - n && bx < base + end);
-    if (hit != 0) {
-      const int l = __ffsll(hit) - 1;
-      s = s0 + l;
-      t0 = __builtin_amdgcn_readlane(a, l) + (bx - base - __builtin_amdgcn_readlane(end - n, l)) * C;
-      t1 = min(__builtin_amdgcn_readlane(b, l), t0 + C);
-      return true;
-    }
-    base += __builtin_amdgcn_readlane(end, 63);
-  }
-  return false;
+  int local;
+  s = locate_item(S, bx, local, [&](int i) { return chunks_of<C>(state_slots, lim, i, query_start[i], query_start[i + 1]); });
+  if (s < 0) return false;
+  t0 = query_start[s] + local * C;
+  t1 = min(query_start[s + 1], t0 + C);
+  return true;
 }
 
-// number of the first chunk of sequence s (whole waves)
+// number of the first chunk of sequence s
 template <int C = CN>
 __device__ __forceinline__ int first_chunk(const int32_t* query_start, const int32_t* state_slots, int lim, int s) {
-  int n = 0;
-  for (int i = threadIdx.x & 63; i < s; i += 64) n += chunks_of<C>(state_slots, lim, i, query_start[i], query_start[i + 1]);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
-  return __builtin_amdgcn_readfirstlane(n);
+  return count_items(s, [&](int i) { return chunks_of<C>(state_slots, lim, i, query_start[i], query_start[i + 1]); });
 }
 
 // sum over j < n (a constant after unrolling) of row[j] x[j]; the row is read in 16-B pieces

@@ -15,7 +15,7 @@
 #include <cstdlib>
 #include <type_traits>
 
-#include "common.h"
+#include "locate.h"
 #include "seq_launchers.h"
 
 namespace vgate {
@@ -28,17 +28,12 @@ __device__ __forceinline__ bool locate_tile(const AnyGemmArgs& p, int by, int& g
     grp = 0; r0 = by * bm; rend = p.M;
     return r0 < p.M;
   }
-  int base = 0;
-  for (int g = 0; g < p.groups; ++g) {
-    const int a = p.group_off[g], b = p.group_off[g + 1];
-    const int nt = (b - a + bm - 1) / bm;
-    if (by < base + nt) {
-      grp = g; r0 = a + (by - base) * bm; rend = b;
-      return true;
-    }
-    base += nt;
-  }
-  return false;
+  int local;
+  grp = locate_item(p.groups, by, local, [&](int g) { return (p.group_off[g + 1] - p.group_off[g] + bm - 1) / bm; });
+  if (grp < 0) return false;
+  r0 = p.group_off[grp] + local * bm;
+  rend = p.group_off[grp + 1];
+  return true;
 }
 
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + expf(-x)); }

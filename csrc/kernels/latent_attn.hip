@@ -39,7 +39,7 @@
 // not depend on its neighbours. The workgroups with the most keys start first.
 #include <stdlib.h>
 
-#include "common.h"
+#include "locate.h"
 #include "seq_launchers.h"
 
 namespace vgate {
@@ -285,12 +285,9 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(LatentArgs a, con
   __shared__ float mrg_m[4][16], mrg_l[4][16];
   __shared__ float mrg_o[16][16 * NCT];  // split mode: the merged weighted latent of the 16 rows
   const int E = a.rank + a.rot, KR = a.rank;
-  int s = -1, tile = 0, base = 0;
-  for (int i = 0; i < S; ++i) {  // (sequence, 64-row tile) of this workgroup
-    const int nt = ((query_start[i + 1] - query_start[i]) * H + 63) / 64;
-    if ((int)blockIdx.x < base + nt) { s = i; tile = blockIdx.x - base; break; }
-    base += nt;
-  }
+  int tile;
+  // (sequence, 64-row tile) of this workgroup
+  const int s = locate_item(S, (int)blockIdx.x, tile, [&](int i) { return ((query_start[i + 1] - query_start[i]) * H + 63) / 64; });
   if (s < 0) return;
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, lg = l >> 4;
   const int t0 = query_start[s], ntok = query_start[s + 1] - t0;
@@ -480,13 +477,10 @@ __global__ __launch_bounds__(256) void latent_attn_tiled_kernel(LatentArgs a, co
   __shared__ __attribute__((aligned(16))) bf16_t pl[64][40];      // weights
   __shared__ __attribute__((aligned(16))) float fac[64];          // rescaling factors, at the end 1 / row sums
   const int E = a.rank + a.rot, KR = a.rank;
-  int s = -1, tile = 0, base = 0;
   const int bx = gridDim.x - 1 - blockIdx.x;
-  for (int i = 0; i < S; ++i) {  // (sequence, 64-row tile) of this workgroup
-    const int nt = ((query_start[i + 1] - query_start[i]) * H + 63) / 64;
-    if (bx < base + nt) { s = i; tile = bx - base; break; }
-    base += nt;
-  }
+  int tile;
+  // (sequence, 64-row tile) of this workgroup
+  const int s = locate_item(S, bx, tile, [&](int i) { return ((query_start[i + 1] - query_start[i]) * H + 63) / 64; });
   if (s < 0) return;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, lg = l >> 4;
   const int t0 = query_start[s], ntok = query_start[s + 1] - t0;
@@ -632,12 +626,9 @@ __global__ __launch_bounds__(256) void latent_attn_merge_kernel(int rank, int H,
                                                                  int S, int parts, int vs, const float* __restrict__ part_o,
                                                                  const float* __restrict__ part_ml,
                                                                  bf16_t* __restrict__ ol) {
-  int s = -1, base = 0;
-  for (int i = 0; i < S; ++i) {  // the sequence of this workgroup, numbered as in the attention kernel
-    const int nt = ((query_start[i + 1] - query_start[i]) * H + 63) / 64;
-    if ((int)blockIdx.x < base + nt) { s = i; break; }
-    base += nt;
-  }
+  int tile;
+  // the sequence of this workgroup, numbered as in the attention kernel
+  const int s = locate_item(S, (int)blockIdx.x, tile, [&](int i) { return ((query_start[i + 1] - query_start[i]) * H + 63) / 64; });
   if (s < 0) return;
   const int t0 = query_start[s], nrows = (query_start[s + 1] - t0) * H;
   if (nrows > 16) return;  // (not shared out: the attention kernel has stored its rows)

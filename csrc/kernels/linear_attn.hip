@@ -97,17 +97,15 @@ __global__ __launch_bounds__(256) void linear_prep_kernel(LinearAttnArgs p, floa
 enum { SCAN_WHOLE = 0, SCAN_LOCAL = 1, SCAN_OUTPUT = 2 };
 
 __device__ __forceinline__ bool locate_chunk(const LinearAttnArgs& p, int CH, int bx, int& s, int& t0, int& t1) {
-  int base = 0;
-  for (int i = 0; i < p.S; ++i) {
+  int local;
+  s = locate_item(p.S, bx, local, [&](int i) {
     const int a = p.query_start[i], b = p.query_start[i + 1];
-    const int nc = (p.state_slots[i] < 0 || b <= a) ? 0 : (b - a + CH - 1) / CH;
-    if (bx < base + nc) {
-      s = i; t0 = a + (bx - base) * CH; t1 = min(b, t0 + CH);
-      return true;
-    }
-    base += nc;
-  }
-  return false;
+    return (p.state_slots[i] < 0 || b <= a) ? 0 : (b - a + CH - 1) / CH;
+  });
+  if (s < 0) return false;
+  t0 = p.query_start[s] + local * CH;
+  t1 = min(p.query_start[s + 1], t0 + CH);
+  return true;
 }
 
 template <int DQ, int TC, int NC, int MODE, bool PRE>
@@ -250,11 +248,10 @@ __global__ __launch_bounds__(256) void linear_carry_kernel(LinearAttnArgs p, int
   const int slot = p.state_slots[s];
   const int t0 = p.query_start[s], t1 = p.query_start[s + 1];
   if (slot < 0 || t1 <= t0) return;
-  int base = 0;
-  for (int i = 0; i < s; ++i) {
+  const int base = count_items(s, [&](int i) {
     const int a = p.query_start[i], b = p.query_start[i + 1];
-    base += (p.state_slots[i] < 0 || b <= a) ? 0 : (b - a + CH - 1) / CH;
-  }
+    return (p.state_slots[i] < 0 || b <= a) ? 0 : (b - a + CH - 1) / CH;
+  });
   const int nc = (t1 - t0 + CH - 1) / CH;
   const int D = p.D, V = p.V;
   const bool from_zero = p.context_lens[s] - (t1 - t0) <= 0;

@@ -16,7 +16,7 @@
 //   output  every chunk again from its true initial state, now with outputs
 // The launch that writes the slot's state also rewrites the kept convolution inputs. A portion that starts at position 0
 // starts from zero, so a reused slot needs no clearing.
-#include "common.h"
+#include "locate.h"
 #include "seq_launchers.h"
 #include "short_conv.h"
 
@@ -85,17 +85,15 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ShortConvArgs p) {
 enum { SCAN_WHOLE = 0, SCAN_LOCAL = 1, SCAN_OUTPUT = 2 };
 
 __device__ __forceinline__ bool locate_chunk(const SelectiveScanArgs& p, int CH, int bx, int& s, int& t0, int& t1) {
-  int base = 0;
-  for (int i = 0; i < p.S; ++i) {
+  int local;
+  s = locate_item(p.S, bx, local, [&](int i) {
     const int a = p.query_start[i], b = p.query_start[i + 1];
-    const int nc = (p.state_slots[i] < 0 || b <= a) ? 0 : (b - a + CH - 1) / CH;
-    if (bx < base + nc) {
-      s = i; t0 = a + (bx - base) * CH; t1 = min(b, t0 + CH);
-      return true;
-    }
-    base += nc;
-  }
-  return false;
+    return (p.state_slots[i] < 0 || b <= a) ? 0 : (b - a + CH - 1) / CH;
+  });
+  if (s < 0) return false;
+  t0 = p.query_start[s] + local * CH;
+  t1 = min(p.query_start[s + 1], t0 + CH);
+  return true;
 }
 
 // MODE WHOLE: blockIdx.x a sequence, its whole portion from its slot. LOCAL / OUTPUT: blockIdx.x one chunk of CH tokens
@@ -237,11 +235,10 @@ __global__ __launch_bounds__(256) void selective_carry_kernel(SelectiveScanArgs 
   const int slot = p.state_slots[s];
   const int t0 = p.query_start[s], t1 = p.query_start[s + 1];
   if (slot < 0 || t1 <= t0) return;
-  int base = 0;
-  for (int i = 0; i < s; ++i) {
+  const int base = count_items(s, [&](int i) {
     const int a = p.query_start[i], b = p.query_start[i + 1];
-    base += (p.state_slots[i] < 0 || b <= a) ? 0 : (b - a + CH - 1) / CH;
-  }
+    return (p.state_slots[i] < 0 || b <= a) ? 0 : (b - a + CH - 1) / CH;
+  });
   const int nc = (t1 - t0 + CH - 1) / CH, C = p.C, N = p.N;
   const int pos0 = p.context_lens[s] - (t1 - t0);
   const int64_t CN = (int64_t)C * N;
@@ -250,11 +247,20 @@ __global__ __launch_bounds__(256) void selective_carry_kernel(SelectiveScanArgs 
     const int c = (int)(e / N);
     const float A = p.A[e];
     float cur = pos0 <= 0 ? 0.f : sp[e];
-    for (int k = 0; k < nc; ++k) {
-      float* cs = cstate + (base + k) * CN + e;
-      const float loc = *cs;
-      *cs = cur;
-      cur = fmaf(__builtin_amdgcn_exp2f(cstep[(int64_t)(base + k) * C + c] * A), cur, loc);
+    for (int k0 = 0; k0 < nc; k0 += 8) {   // eight chunks' loads in flight
+      float loc[8], dec[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int64_t k = base + min(k0 + u, nc - 1);
+        loc[u] = cstate[k * CN + e];
+        dec[u] = cstep[k * C + c];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (k0 + u < nc) {
+          cstate[(base + k0 + u) * CN + e] = cur;
+          cur = fmaf(__builtin_amdgcn_exp2f(dec[u] * A), cur, loc[u]);
+        }
     }
     sp[e] = cur;
     if (e % N == 0)

@@ -48,7 +48,7 @@
 // position, so results do not depend on how a prompt is cut or what else is in the batch.
 #include <algorithm>
 
-#include "common.h"
+#include "locate.h"
 #include "seq_launchers.h"
 
 namespace vgate {
@@ -486,12 +486,9 @@ __global__ __launch_bounds__(64 * NW) void window_attn_mfma_kernel(WindowArgs a,
   __shared__ float mrg_o[16][16 * NCT];  // the merged weighted values of the 16 rows
   const int D = a.D, V = a.V, G = a.G, H = a.H, rep = H / G, g = blockIdx.y, P = a.pool;
   const int GV = a.GV, gv = g / (G / GV);  // value heads; the value head of key head g
-  int s = -1, tile = 0, base = 0;
-  for (int i = 0; i < a.S; ++i) {  // (sequence, 16-row tile) of this workgroup
-    const int nt = ((a.query_start[i + 1] - a.query_start[i]) * rep + 15) / 16;
-    if ((int)blockIdx.x < base + nt) { s = i; tile = blockIdx.x - base; break; }
-    base += nt;
-  }
+  int tile;
+  // (sequence, 16-row tile) of this workgroup
+  const int s = locate_item(a.S, (int)blockIdx.x, tile, [&](int i) { return ((a.query_start[i + 1] - a.query_start[i]) * rep + 15) / 16; });
   if (s < 0) return;
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, lg = l >> 4;
   const int t0 = a.query_start[s], ntok = a.query_start[s + 1] - t0;
@@ -739,12 +736,8 @@ __global__ __launch_bounds__(64 * NW) void window_attn_mfma_kernel(WindowArgs a,
 // above (normalise, turn back, gate, store). vs: the row stride of the parts' weighted values.
 __global__ __launch_bounds__(256) void window_attn_merge_kernel(WindowArgs a, int vs, bf16_t* __restrict__ out) {
   const int V = a.V, G = a.G, H = a.H, rep = H / G, g = blockIdx.y;
-  int s = -1, tile = 0, base = 0;
-  for (int i = 0; i < a.S; ++i) {
-    const int nt = ((a.query_start[i + 1] - a.query_start[i]) * rep + 15) / 16;
-    if ((int)blockIdx.x < base + nt) { s = i; tile = blockIdx.x - base; break; }
-    base += nt;
-  }
+  int tile;
+  const int s = locate_item(a.S, (int)blockIdx.x, tile, [&](int i) { return ((a.query_start[i + 1] - a.query_start[i]) * rep + 15) / 16; });
   if (s < 0) return;
   const int t0 = a.query_start[s], ntok = a.query_start[s + 1] - t0;
   const int pos0 = a.context_lens[s] - ntok, nrows = ntok * rep;
@@ -806,12 +799,9 @@ __global__ __launch_bounds__(256) void window_attn_tiled_kernel(WindowArgs a, co
   __shared__ __attribute__((aligned(16))) bf16_t pl[4][16][40];
   const int D = a.D, V = a.V, G = a.G, H = a.H, rep = H / G, g = blockIdx.y, P = a.pool;
   const int GV = a.GV, gv = g / (G / GV);  // value heads; the value head of key head g
-  int s = -1, tile = 0, base = 0;
-  for (int i = 0; i < a.S; ++i) {  // (sequence, 64-row tile) of this workgroup
-    const int nt = ((a.query_start[i + 1] - a.query_start[i]) * rep + 63) / 64;
-    if ((int)blockIdx.x < base + nt) { s = i; tile = blockIdx.x - base; break; }
-    base += nt;
-  }
+  int tile;
+  // (sequence, 64-row tile) of this workgroup
+  const int s = locate_item(a.S, (int)blockIdx.x, tile, [&](int i) { return ((a.query_start[i + 1] - a.query_start[i]) * rep + 63) / 64; });
   if (s < 0) return;
   const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, lr = l & 15, lg = l >> 4;
   const int t0 = a.query_start[s], ntok = a.query_start[s + 1] - t0;
