@@ -70,6 +70,11 @@ __device__ __forceinline__ void with_act(const AnyGemmArgs& p, F&& fn) {
   }
 }
 
+__device__ __forceinline__ void store_value(const AnyGemmArgs& p, int64_t i, float v) {
+  if (p.out_f32) reinterpret_cast<float*>(p.out)[i] = v;
+  else reinterpret_cast<bf16_t*>(p.out)[i] = f2bf(v);
+}
+
 __device__ __forceinline__ void store_out(const AnyGemmArgs& p, int64_t b, int m, int n, float v) {
   if (p.gate != nullptr) {
     const int64_t gi = (int64_t)m * p.ldg + b * p.g_bs + (int64_t)n * p.g_cs;
@@ -77,9 +82,7 @@ __device__ __forceinline__ void store_out(const AnyGemmArgs& p, int64_t b, int m
                                 : bf2f(reinterpret_cast<const bf16_t*>(p.gate)[gi]);
     v *= sigmoidf_(gl);
   }
-  const int64_t oi = (int64_t)m * p.ldo + b * p.o_bs + n;
-  if (p.out_f32) reinterpret_cast<float*>(p.out)[oi] = v;
-  else reinterpret_cast<bf16_t*>(p.out)[oi] = f2bf(v);
+  store_value(p, (int64_t)m * p.ldo + b * p.o_bs + n, v);
 }
 
 __device__ __forceinline__ bf16x8 load_frag(const bf16_t* rowp, int k, int K, bool valid) {
@@ -227,6 +230,25 @@ __global__ __launch_bounds__(256) void gemm_any_mfma_kernel(AnyGemmArgs p) {
         if (DUAL) acc2[i][j] += red[KS ? wn : 0][KS ? 4 + 2 * i + j : 0][KS ? l : 0];
       }
   }
+  float gl[2][NJ][4];   // the gates' logits, asked for together
+  if (p.gate != nullptr) {
+    const bool gf = p.gate_f32 != 0;
+    auto load = [&](auto f32) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int n = min(n0 + wn * 16 * NJ + j * 16 + lr, p.N - 1), m = min(r0 + mrow + i * 16 + 4 * (l >> 4) + e, rend - 1);
+            const int64_t gi = (int64_t)m * p.ldg + b * p.g_bs + (int64_t)n * p.g_cs;
+            gl[i][j][e] = decltype(f32)::value ? reinterpret_cast<const float*>(p.gate)[gi]
+                                               : bf2f(reinterpret_cast<const bf16_t*>(p.gate)[gi]);
+          }
+    };
+    if (gf) load(std::true_type{});
+    else load(std::false_type{});
+  }
   with_act<DUAL>(p, [&](auto act) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -239,10 +261,113 @@ __global__ __launch_bounds__(256) void gemm_any_mfma_kernel(AnyGemmArgs p) {
         for (int e = 0; e < 4; ++e) {
           const int m = r0 + mrow + i * 16 + 4 * (l >> 4) + e;
           if (m >= rend) continue;
-          store_out(p, b, m, n, act_val<decltype(act)::value>(p, acc[i][j][e] + bias, DUAL ? acc2[i][j][e] : 0.f));
+          float v = act_val<decltype(act)::value>(p, acc[i][j][e] + bias, DUAL ? acc2[i][j][e] : 0.f);
+          if (p.gate != nullptr) v *= sigmoidf_(gl[i][j][e]);
+          store_value(p, (int64_t)m * p.ldo + b * p.o_bs + n, v);
         }
       }
   });
+}
+
+// Few rows. Host-checked as AL above. A workgroup owns 16 columns (of both matrices), its four waves take pairs of k-steps (64
+// elements: whole 128-B lines of a weight row) in turn, UB of them in flight at once, and meet in LDS; wave i finishes the i-th
+// 16 rows. A tile's 64 rows go in passes of 32. What bounds it is one trip to memory for the weights, 4 to 6 us a launch; 8 experts
+// of 1024 x 2048 pairs (67 MB, 64 rows): 15 us, as tiles 18.
+template <int DUAL, int UB>
+__global__ __launch_bounds__(256) void gemm_any_rows_kernel(AnyGemmArgs p) {
+  constexpr int NM = 1 + DUAL;
+  __shared__ f32x4 red[4][2 * NM][64];
+  int grp, r0, rend;
+  if (!locate_tile(p, blockIdx.y, grp, r0, rend)) return;
+  const int64_t b = blockIdx.z, wsel = p.group_off != nullptr ? grp : b;
+  const int n0 = blockIdx.x * 16, K = p.K;
+  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = l & 15, lk = 8 * (l >> 4);
+  const int n = n0 + lr;
+  const bf16_t* A = reinterpret_cast<const bf16_t*>(p.a) + b * p.a_bs;
+  const int64_t wo = wsel * p.w_bs + (int64_t)min(n, p.N - 1) * p.ldw;   // (columns past N: the last one's, never stored)
+  const bf16_t* w = reinterpret_cast<const bf16_t*>(p.w) + wo;
+  const bf16_t* w2 = DUAL ? reinterpret_cast<const bf16_t*>(p.w2) + wo : nullptr;
+  rend = min(rend, r0 + BM);
+  for (; r0 < rend; r0 += 32) {
+    const bool two = rend - r0 > 16;   // (workgroup-uniform)
+    const bf16_t* ar[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {      // (rows past the end: the pass's first, never stored)
+      const int m = r0 + 16 * i + lr < rend ? r0 + 16 * i + lr : r0;
+      ar[i] = A + (int64_t)(p.a_rows ? p.a_rows[m] : m) * p.lda;
+    }
+    f32x4 acc[2][NM];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int d = 0; d < NM; ++d) acc[i][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto run = [&](auto mt) {
+      constexpr int MT = decltype(mt)::value;
+      for (int k0 = 64 * wv; k0 < K; k0 += 256 * UB) {
+        uint4 wf[UB][2][NM], af[UB][2][MT];
+#pragma unroll
+        for (int u = 0; u < UB; ++u)
+#pragma unroll
+          for (int st = 0; st < 2; ++st) {
+            const int k = min(k0 + 256 * u + 32 * st + lk, K - 8);   // (past K: a clamped address, A zeroed below)
+            wf[u][st][0] = ld16(w + k);
+            if (DUAL) wf[u][st][NM - 1] = ld16(w2 + k);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) af[u][st][i] = ld16(ar[i] + k);
+          }
+#pragma unroll
+        for (int u = 0; u < UB; ++u)
+#pragma unroll
+          for (int st = 0; st < 2; ++st) {
+            const bool in = k0 + 256 * u + 32 * st + lk < K;
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+              const bf16x8 a = as_bf16x8(in ? af[u][st][i] : make_uint4(0, 0, 0, 0));
+#pragma unroll
+              for (int d = 0; d < NM; ++d) acc[i][d] = mfma16(a, as_bf16x8(wf[u][st][d]), acc[i][d]);
+            }
+          }
+      }
+    };
+    if (two) run(std::integral_constant<int, 2>{});
+    else run(std::integral_constant<int, 1>{});
+    // what the finishing waves need besides is on its way while the others arrive
+    const int mw = r0 + 16 * wv + 4 * (l >> 4);   // first of this lane's four rows, if its wave finishes some
+    const bool last = wv < 2 && (wv == 0 || two);
+    float gl[4] = {0.f, 0.f, 0.f, 0.f}, bias = 0.f;
+    if (last && p.bias != nullptr) bias = p.bias[min(n, p.N - 1)];
+    if (last && p.gate != nullptr) {
+      const int64_t gc = b * p.g_bs + (int64_t)min(n, p.N - 1) * p.g_cs;
+      if (p.gate_f32) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) gl[e] = reinterpret_cast<const float*>(p.gate)[(int64_t)min(mw + e, rend - 1) * p.ldg + gc];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) gl[e] = bf2f(reinterpret_cast<const bf16_t*>(p.gate)[(int64_t)min(mw + e, rend - 1) * p.ldg + gc]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int d = 0; d < NM; ++d)
+        if (i == 0 || two) red[wv][i * NM + d][l] = acc[i][d];
+    __syncthreads();
+    if (last && n < p.N) {
+      f32x4 s[NM];
+#pragma unroll
+      for (int d = 0; d < NM; ++d) s[d] = (red[0][wv * NM + d][l] + red[1][wv * NM + d][l]) + (red[2][wv * NM + d][l] + red[3][wv * NM + d][l]);
+      with_act<DUAL>(p, [&](auto act) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (mw + e >= rend) continue;
+          float v = act_val<decltype(act)::value>(p, s[0][e] + bias, DUAL ? s[NM - 1][e] : 0.f);
+          if (p.gate != nullptr) v *= sigmoidf_(gl[e]);
+          store_value(p, (int64_t)(mw + e) * p.ldo + b * p.o_bs + n, v);
+        }
+      });
+    }
+    __syncthreads();   // (the next pass writes red again)
+  }
 }
 
 // LDS-tiled form. Host-checked: K, the row strides and the batch strides are multiples of 8 elements, the bases
@@ -491,7 +616,20 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st) {
     auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     const bool al = g.K >= 8 && g.K % 8 == 0 && g.lda % 8 == 0 && g.ldw % 8 == 0 && g.a_bs % 8 == 0 &&
                     g.w_bs % 8 == 0 && a16(g.a) && a16(g.w) && (!dual || a16(g.w2));
-    const bool wide = al && g.N >= 512 && g.M >= 256;  // enough 64 x 128 tiles to fill the chip
+    // Few rows, or few 64 x 64 tiles, leave the chip idle behind chains of loads: 16 columns and a quarter of K per wave there. (us,
+    // the tiles' kernels -> now) 64 x 1024 at 32 rows 12.4 -> 6.3, 1024 x 1024 at 512 28.7 -> 16.4, 8 experts of 1024 x 2048 with 8 rows
+    // each 15.6 -> 10.9, with 32 46 -> 16.6. Above the lines the wider tiles read the operands less often: 8192 x 1024 at 128 rows
+    // (256 tiles) 20 against 28, 256 x 512 at 2048 (128 tiles) 12.4 against 16.5, 32 experts with 2 rows each (816 tiles) 20 against 25.
+    const int64_t tiles = (int64_t)grid.x * mt * g.batch;
+    if (al && (g.group_off ? g.M <= 512 && tiles < 768 : g.M <= 64 || tiles <= (g.M <= 512 ? 192 : 64))) {
+      const dim3 gr((g.N + 15) / 16, mt, g.batch);
+      auto kern = g.K > 256 ? (dual ? gemm_any_rows_kernel<1, 2> : gemm_any_rows_kernel<0, 4>)
+                            : (dual ? gemm_any_rows_kernel<1, 1> : gemm_any_rows_kernel<0, 1>);
+      hipLaunchKernelGGL(kern, gr, block, 0, st, g);
+      return;
+    }
+    // enough 64 x 128 tiles to fill the chip (experts with few rows each: tiles whose waves split K)
+    const bool wide = al && g.N >= 512 && g.M >= 256 && (!g.group_off || g.M > 32 * g.groups);
     const dim3 gridw((g.N + 127) / 128, mt, g.batch);
     if (wide && g.M >= 1024 && lds_tiles()) {  // enough 128-row tiles
       const int mt128 = (g.M + LM - 1) / LM + (g.group_off ? g.groups : 0);

@@ -1,0 +1,58 @@
+"""The row-major GEMM's form for few rows or few tiles against fp32 products: rows around its passes and tiles, columns and K
+around its pieces, batches, experts (empty ones and ones of many rows too), gathers, pairs, gates, biases, both result types."""
+import pytest
+import torch
+
+from vgate.ops import seq
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(out, want, K):
+    # fp32 sums of K products of size ~ K^-1/2 in another order, then one rounding to the result's type
+    tol = 4.0 * K * 2.0 ** -24 + (2.0 ** -8 * want.abs() if out.dtype == torch.bfloat16 else 0.0)
+    assert ((out.float() - want).abs() <= 2 * tol + 1e-6).all(), float((out.float() - want).abs().max())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,K", [(8, 1024), (17, 8), (64, 264), (200, 136), (1024, 2048)])
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64, 65, 300, 513])
+def test_plain(M, N, K, dt):
+    g = torch.Generator("cuda").manual_seed(M * N + K)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    a, w, bias = rand(M, K + 8).bfloat16()[:, :K], (rand(N, K) * K ** -0.5).bfloat16(), rand(N)
+    out = torch.full((M, N), float("nan"), device="cuda", dtype=dt)
+    seq.gemm(a, w, out, bias=bias)
+    _close(out, a.float() @ w.float().t() + bias, K)
+
+
+@pytest.mark.parametrize("gate_dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M", [1, 32, 40, 130, 1100])
+def test_batches_with_gates(M, gate_dt):
+    B, N, K = 3, 72, 136
+    g = torch.Generator("cuda").manual_seed(M)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    a, w = rand(M, B, K).bfloat16().transpose(0, 1), (rand(B, N, K) * K ** -0.5).bfloat16()
+    gate = rand(M, B, N).to(gate_dt).transpose(0, 1)
+    out = torch.full((M, B, N), float("nan"), device="cuda", dtype=torch.bfloat16).transpose(0, 1)
+    seq.gemm(a, w, out, gate=gate)
+    _close(out, torch.matmul(a.float(), w.float().transpose(1, 2)) * torch.sigmoid(gate.float()), K)
+
+
+@pytest.mark.parametrize("sizes", [[1, 0, 2, 17], [0, 0, 90], [16, 32, 33, 64, 65], [2] * 64, [5] * 40, [500, 3], [1] * 70])
+@pytest.mark.parametrize("N,K", [(48, 72), (1024, 512)])
+def test_experts(N, K, sizes):
+    E, M = len(sizes), sum(sizes)
+    g = torch.Generator("cuda").manual_seed(M + N)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    x, w, w2 = rand(M, K).bfloat16(), (rand(E, N, K) * K ** -0.5).bfloat16(), (rand(E, N, K) * K ** -0.5).bfloat16()
+    rows = torch.randperm(M, device="cuda", generator=g).int()
+    off = torch.tensor([sum(sizes[:i]) for i in range(E + 1)], dtype=torch.int32, device="cuda")
+    out, pair = (torch.full((M, N), float("nan"), device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    seq.gemm(x, w, out, group_off=off)
+    seq.gemm(x, w, pair, w2=w2, a_rows=rows, group_off=off, act=seq.ACT_SILU_MUL)
+    for e in range(E):
+        a, b = int(off[e]), int(off[e + 1])
+        _close(out[a:b], x[a:b].float() @ w[e].float().t(), K)
+        h = x[rows[a:b].long()].float()
+        _close(pair[a:b], torch.nn.functional.silu(h @ w[e].float().t()) * (h @ w2[e].float().t()), 8 * K)
