@@ -27,7 +27,8 @@ __global__ __launch_bounds__(128) void attn_decode_reduce_kernel(AttnArgs a) {
   const int ctx = a.context_lens[s];
   if (ctx <= 0) return;
   if (a.query_start && a.query_start[s + 1] - a.query_start[s] != 1) return;
-  const int nparts = (ctx + a.part_size - 1) / a.part_size;
+  int plen, nparts;
+  partition(a, ctx, plen, nparts);
   if (nparts <= 1) return;
   const float* pm = a.part_ml + ((size_t)s * a.Hq + hq) * a.num_parts * 2;
   const float* po = a.part_o + ((size_t)s * a.Hq + hq) * a.num_parts * D_;

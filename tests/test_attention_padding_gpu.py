@@ -33,3 +33,35 @@ def test_padding_sequences_behind_full_rows(Hq, Hkv, lens, ctxs):
         ops.attention(q, Hq * D, kc, vc, bt, cl, qs, ts, tq, out, po, pml, Hq, Hkv, 512, D ** -0.5)
         outs.append(out)
     assert torch.isfinite(outs[0].float()).all() and torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("S", [1, 5, 300])
+@pytest.mark.parametrize("part", [64, 512])
+def test_equal_and_whole_partitions(S, part):
+    """Contexts around one, two and three partitions, in launches few enough for equal parts and too many: one partition's result."""
+    Hq, Hkv, D, dev = 12, 2, 128, "cuda"
+    g = torch.Generator(dev).manual_seed(S + part)
+    rand = lambda *s: torch.randn(*s, device=dev, generator=g).bfloat16()  # noqa: E731
+    lens = [part - 1, part, part + 1, 2 * part - 31, 2 * part, 2 * part + 1, 3 * part - 1, 1]
+    ctx = [lens[i % len(lens)] for i in range(S)] if S > 1 else [2 * part + 1]
+    blocks = 3 * part // 16
+    kc, vc = rand(64, Hkv, 16, D), rand(64, Hkv, 16, D)
+    bt = torch.randint(0, 64, (S, blocks), device=dev, generator=g).int()
+    cl, qs = torch.tensor(ctx, dtype=torch.int32, device=dev), torch.arange(S + 1, device=dev).int()
+    q, none = rand(S, Hq * D), torch.empty(0, dtype=torch.int32, device=dev)
+    outs = []
+    for size in (part, 1024 if part == 64 else 512):
+        P = -(-blocks * 16 // size)
+        po, pml = torch.zeros(S, Hq, P, D, device=dev), torch.zeros(S, Hq, P, 2, device=dev)
+        out = torch.zeros(S, Hq * D, device=dev).bfloat16()
+        ops.attention(q, Hq * D, kc, vc, bt, cl, qs, none, none, out, po, pml, Hq, Hkv, size, D ** -0.5)
+        outs.append(out.float())
+    n = [c for c in ctx]
+    k = torch.stack([kc[bt[i].long()].transpose(1, 2).reshape(-1, Hkv, D)[: max(n)] for i in range(S)]).float()
+    v = torch.stack([vc[bt[i].long()].transpose(1, 2).reshape(-1, Hkv, D)[: max(n)] for i in range(S)]).float()
+    qq = q.float().view(S, Hkv, Hq // Hkv, D)
+    sc = torch.matmul(qq, k.permute(0, 2, 3, 1).contiguous()) * D ** -0.5
+    sc = sc.masked_fill(torch.arange(max(n), device=dev) >= cl.view(S, 1, 1, 1), float("-inf"))
+    want = torch.matmul(sc.softmax(-1), v.permute(0, 2, 1, 3).contiguous()).reshape(S, Hq * D)
+    for out in outs:   # weights rounded to bf16 (2^-9 each, of values of size ~ 1 that average out) and a bf16 result
+        assert float((out - want).norm() / want.norm()) < 2.0 ** -7
