@@ -176,9 +176,10 @@ __device__ __forceinline__ void finish_row(const SampleArgs& a, int row, int cho
 // ---- one block per row (NSEG == 1: batches above SAMPLE_MAX_BLOCKS / 2 rows, or no workspace) ----
 // Every pass sweeps the whole row and ends at a block barrier; same passes, noise and acceptance
 // tests as the segmented kernel below.
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_row_kernel(SampleArgs a) {
+template <int NT>
+__global__ __launch_bounds__(NT) void sample_row_kernel(SampleArgs a) {
   TLScope tl_scope(a.tl);
-  __shared__ Acc red[SAMPLE_THREADS / 64];
+  __shared__ Acc red[NT / 64];
   __shared__ Acc merged;
   const int row = blockIdx.y, tid = threadIdx.x;
   const int V4 = a.V >> 2;  // host guarantees V % 4 == 0 and 16-B aligned rows
@@ -352,18 +353,24 @@ int sample_segments(int B, int V) {
   return nseg < 1 ? 1 : nseg;
 }
 
+// More waves where a thread of 256 would have more than 12 pieces of 16 B: the noise of a segment (Philox, two logarithms per logit)
+// then takes longer than the meeting, and four waves cannot keep a CU busy with it. us, top-p 0.95, 256 -> 1024 threads:
+// vocabulary 152064, 32 rows 42.8 -> 37.2, 64 rows 103 -> 78, 256 rows (whole rows) 339 -> 201; 16 rows (9 pieces) 29.7 against 31.2.
+static bool long_rows(int V, int nseg) { return (V >> 2) > 3072 * nseg; }
+
 void launch_sample(const SampleArgs& s, hipStream_t st) {
   if (s.B <= 0) return;
   const int nseg = sample_segments(s.B, s.V);
   SampleArgs a = s;
   if (nseg > 1 && s.gran != nullptr && s.epoch != nullptr && s.B <= SAMPLE_GRAN_ROWS) {
     a.tl = tl_take("sample_gran", nseg * s.B);
-    // 256 threads per block: 512 / 1024 measured no faster / slower (profiles/r4_sampler_single_launch.log)
-    hipLaunchKernelGGL(sample_gran_kernel<256>, dim3(nseg, s.B), dim3(256), 0, st, a);
+    if (long_rows(s.V, nseg)) hipLaunchKernelGGL(sample_gran_kernel<1024>, dim3(nseg, s.B), dim3(1024), 0, st, a);
+    else hipLaunchKernelGGL(sample_gran_kernel<256>, dim3(nseg, s.B), dim3(256), 0, st, a);
     return;
   }
   a.tl = tl_take("sample", s.B);
-  hipLaunchKernelGGL(sample_row_kernel, dim3(1, s.B), dim3(SAMPLE_THREADS), 0, st, a);
+  if (long_rows(s.V, 1)) hipLaunchKernelGGL(sample_row_kernel<1024>, dim3(1, s.B), dim3(1024), 0, st, a);
+  else hipLaunchKernelGGL(sample_row_kernel<SAMPLE_THREADS>, dim3(1, s.B), dim3(SAMPLE_THREADS), 0, st, a);
 }
 
 }  // namespace vgate

@@ -1,0 +1,31 @@
+"""Sampling with few and with many waves per row: the choice of a row does not depend on how many rows share the launch, which
+decides how the row is split and how many waves sweep it."""
+import pytest
+import torch
+
+from vgate import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("V", [4096, 49156, 152064])
+def test_rows_do_not_depend_on_the_batch(V):
+    dev, B = "cuda", 130
+    g = torch.Generator(dev).manual_seed(V)
+    # no two logits closer than a rounding of the sums that a split changes: no candidate on the nucleus' edge at this seed
+    lg = 2.0 * torch.randn(B, V, device=dev, generator=g)
+    t = torch.tensor([0.0, 0.8, 1.0] * B, device=dev)[:B]
+    p = torch.tensor([1.0, 0.95, 0.5, 0.9] * B, device=dev)[:B]
+    k = torch.tensor([-1, -1, -1, 50, -1] * B, dtype=torch.int32, device=dev)[:B]
+    seeds, offs = torch.arange(B, device=dev), torch.arange(B, device=dev) % 7
+
+    def run(rows):
+        out = torch.full((rows.numel(),), -1, dtype=torch.int32, device=dev)
+        ops.sample(lg[rows].contiguous(), t[rows], p[rows], k[rows], seeds[rows], offs[rows], out=out)
+        return out
+
+    whole = run(torch.arange(B, device=dev))                      # one workgroup per row
+    for n in (1, 16, 33, 128):
+        rows = torch.arange(n, device=dev)
+        assert torch.equal(run(rows), whole[:n]), n
+    assert torch.equal(whole[::3], lg[::3].argmax(-1).int())      # temperature 0
