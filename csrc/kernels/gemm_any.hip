@@ -274,7 +274,7 @@ __global__ __launch_bounds__(256) void gemm_any_mfma_kernel(AnyGemmArgs p) {
 // 16 rows. A tile's 64 rows go in passes of 32. What bounds it is one trip to memory for the weights, 4 to 6 us a launch; 8 experts
 // of 1024 x 2048 pairs (67 MB, 64 rows): 15 us, as tiles 18.
 template <int DUAL, int UB>
-__global__ __launch_bounds__(256) void gemm_any_rows_kernel(AnyGemmArgs p) {
+__global__ __launch_bounds__(256, 2) void gemm_any_rows_kernel(AnyGemmArgs p) {
   constexpr int NM = 1 + DUAL;
   __shared__ f32x4 red[4][2 * NM][64];
   int grp, r0, rend;

@@ -787,7 +787,10 @@ __global__ __launch_bounds__(256) void window_attn_merge_kernel(WindowArgs a, in
 // tile t is computed, written after it, one barrier per tile), and every wave takes its fragments from there.
 // Pooled tiles come first and are read straight from the pooled caches by each wave, as in the kernel above.
 template <int NCT, int NQF, int BIAS, bool CAP, bool KEEP>
-__global__ __launch_bounds__(256) void window_attn_tiled_kernel(WindowArgs a, const bf16_t* __restrict__ q,
+// Bound by the vector operations of the softmax, 270 a tile and wave. (two workgroups per CU at least: with more than 256 registers
+// to give, the compiler keeps the sums in accumulation registers and moves them over and back for every rescaling; with the
+// products' tests gone too, 1801 tokens of 8 heads of 128, window 1024: 73 -> 58 us)
+__global__ __launch_bounds__(256, 2) void window_attn_tiled_kernel(WindowArgs a, const bf16_t* __restrict__ q,
                                                                  float scale_log2e, const bf16_t* __restrict__ vt,
                                                                  int num_pages, bf16_t* __restrict__ out) {
   extern __shared__ float btab[];  // BIAS: the distance table of this workgroup's heads (when it is staged)
@@ -877,8 +880,8 @@ __global__ __launch_bounds__(256) void window_attn_tiled_kernel(WindowArgs a, co
       const float v1 = vis1 ? score_log2<CAP>(a, s1[i], scale_log2e, BIAS ? bt1[i] : 0.f) : -INFINITY;
       const float mnew = fmaxf(m[i], group16_max(fmaxf(v0, v1)));
       const float ms = (mnew == -INFINITY) ? 0.f : mnew;
-      al[i] = exp2f(m[i] - ms);
-      const float p0 = exp2f(v0 - ms), p1 = exp2f(v1 - ms);
+      al[i] = __builtin_amdgcn_exp2f(m[i] - ms);   // (below 2^-126: zero)
+      const float p0 = __builtin_amdgcn_exp2f(v0 - ms), p1 = __builtin_amdgcn_exp2f(v1 - ms);
       lsum[i] = lsum[i] * al[i] + p0 + p1;
       m[i] = mnew;
       pl[wv][4 * lg + i][lr] = f2bf(p0);
@@ -979,18 +982,17 @@ __global__ __launch_bounds__(256) void window_attn_tiled_kernel(WindowArgs a, co
     const int kbase = 32 * tile_of(it);
     if (active && (kbase + 31 >= klow || (KEEP && kbase < a.keep)) && kbase <= pmaxw) {  // wave-uniform: some row of the wave may see the tile
       f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = f32x4{0.f, 0.f, 0.f, 0.f};
+      // (no test for the entries past D or V, which are zeros in LDS: a branch per product kept the sums out of its registers,
+      // 100 moves per tile)
 #pragma unroll
-      for (int kk = 0; kk < NQF; ++kk)
-        if (kk < nqf) {
-          s0 = mfma16(qf[kk], as_bf16x8(*reinterpret_cast<const uint4*>(&kl[buf][lr][32 * kk + 8 * lg])), s0);
-          s1 = mfma16(qf[kk], as_bf16x8(*reinterpret_cast<const uint4*>(&kl[buf][16 + lr][32 * kk + 8 * lg])), s1);
-        }
+      for (int kk = 0; kk < NQF; ++kk) {
+        s0 = mfma16(qf[kk], as_bf16x8(*reinterpret_cast<const uint4*>(&kl[buf][lr][32 * kk + 8 * lg])), s0);
+        s1 = mfma16(qf[kk], as_bf16x8(*reinterpret_cast<const uint4*>(&kl[buf][16 + lr][32 * kk + 8 * lg])), s1);
+      }
       softmax_tile(s0, s1, kbase, false);
       const bf16x8 pf = as_bf16x8(*reinterpret_cast<const uint4*>(&pl[wv][lr][8 * lg]));
 #pragma unroll
-      for (int ct = 0; ct < NCT; ++ct)
-        if (ct < nct)
-          O[ct] = mfma16(pf, as_bf16x8(*reinterpret_cast<const uint4*>(&vl[buf][16 * ct + lr][8 * lg])), O[ct]);
+      for (int ct = 0; ct < NCT; ++ct) O[ct] = mfma16(pf, as_bf16x8(*reinterpret_cast<const uint4*>(&vl[buf][16 * ct + lr][8 * lg])), O[ct]);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // P tile read before the next tile overwrites it
     }
     buf ^= 1;
