@@ -485,14 +485,26 @@ __global__ __launch_bounds__(256) void gemm_any_lds_kernel(AnyGemmArgs p) {
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int j = 0; j < (DUAL ? 2 : 4); ++j) {
-        const int n = n0 + (DUAL ? wn * 32 : wn * 64) + j * 16 + lr;
+        const int n = n0 + (DUAL ? wn * 32 : wn * 64) + j * 16 + lr, m = r0 + wm * 64 + i * 16 + 4 * lg;
         if (n >= p.N) continue;
         const float bias = p.bias ? p.bias[n] : 0.f;
+        float gl[4];   // (asked for together)
+        if (p.gate != nullptr) {
+          const int64_t gc = b * p.g_bs + (int64_t)n * p.g_cs;
+          if (p.gate_f32) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) gl[e] = reinterpret_cast<const float*>(p.gate)[(int64_t)min(m + e, rend - 1) * p.ldg + gc];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) gl[e] = bf2f(reinterpret_cast<const bf16_t*>(p.gate)[(int64_t)min(m + e, rend - 1) * p.ldg + gc]);
+          }
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int m = r0 + wm * 64 + i * 16 + 4 * lg + e;
-          if (m >= rend) continue;
-          store_out(p, b, m, n, act_val<decltype(act)::value>(p, acc[i][j][e] + bias, DUAL ? acc[i][j + 2][e] : 0.f));
+          if (m + e >= rend) continue;
+          float v = act_val<decltype(act)::value>(p, acc[i][j][e] + bias, DUAL ? acc[i][j + 2][e] : 0.f);
+          if (p.gate != nullptr) v *= sigmoidf_(gl[e]);
+          store_value(p, (int64_t)(m + e) * p.ldo + b * p.o_bs + n, v);
         }
       }
   });
@@ -631,8 +643,11 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st) {
     // enough 64 x 128 tiles to fill the chip (experts with few rows each: tiles whose waves split K)
     const bool wide = al && g.N >= 512 && g.M >= 256 && (!g.group_off || g.M > 32 * g.groups);
     const dim3 gridw((g.N + 127) / 128, mt, g.batch);
-    if (wide && g.M >= 1024 && lds_tiles()) {  // enough 128-row tiles
-      const int mt128 = (g.M + LM - 1) / LM + (g.group_off ? g.groups : 0);
+    // enough 128-row tiles; also where whole 128-column tiles of many products fill half the chip (us at 2048 rows: 12 of
+    // 128 x 512 27.9 -> 15.8, 8 of 256 x 128 14.1 -> 7.3, 2 of 128 x 256 stay at 9; with a gate per output the small tiles are ahead)
+    const int mt128 = (g.M + LM - 1) / LM + (g.group_off ? g.groups : 0);
+    const bool heads = al && !dual && !g.group_off && g.gate == nullptr && g.N % 128 == 0 && (int64_t)(g.N / 128) * mt128 * g.batch >= 128;
+    if ((wide || heads) && g.M >= 1024 && lds_tiles()) {
       AnyGemmArgs v = g;
       v.vec_out = !g.out_f32 && g.gate == nullptr && g.N % 8 == 0 && g.ldo % 8 == 0 && g.o_bs % 8 == 0 && a16(g.out);
       if (dual) hipLaunchKernelGGL((gemm_any_lds_kernel<1>), dim3((g.N + 63) / 64, mt128, g.batch), block, 0, st, v);

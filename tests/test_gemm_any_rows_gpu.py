@@ -56,3 +56,15 @@ def test_experts(N, K, sizes):
         _close(out[a:b], x[a:b].float() @ w[e].float().t(), K)
         h = x[rows[a:b].long()].float()
         _close(pair[a:b], torch.nn.functional.silu(h @ w[e].float().t()) * (h @ w2[e].float().t()), 8 * K)
+
+
+@pytest.mark.parametrize("M", [1024, 1151, 2049])
+@pytest.mark.parametrize("N,K", [(128, 136), (256, 512)])
+def test_many_products_of_many_rows(M, N, K):
+    B = 16
+    g = torch.Generator("cuda").manual_seed(M + N)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    a, w = rand(M, B, K).bfloat16().transpose(0, 1), (rand(B, N, K) * K ** -0.5).bfloat16()
+    out = torch.full((M, B, N), float("nan"), device="cuda", dtype=torch.bfloat16).transpose(0, 1)
+    seq.gemm(a, w, out)
+    _close(out, torch.matmul(a.float(), w.float().transpose(1, 2)), K)
