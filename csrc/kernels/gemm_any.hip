@@ -10,7 +10,7 @@
 //         fragments straight from global memory (both operands are k-contiguous rows), fp32 accumulate.
 //         Large aligned products (hundreds of rows, wide outputs: the expert GEMMs of a prompt portion):
 //         128 x 128 block tile (a weight pair: 128 x 64 of each matrix), 4 waves of 4 x 4 MFMA tiles, k-steps of
-//         32 staged through two LDS buffers, the next step's loads in flight during the current step's MFMAs.
+//         32 staged through two LDS buffers, the loads of the two steps after the current one in flight.
 //   fp32: 64 x 64 x 16 LDS-tiled FMA kernel, 4 x 4 outputs per thread, k ascending.
 #include <cstdlib>
 #include <type_traits>
@@ -375,10 +375,11 @@ __global__ __launch_bounds__(256, 2) void gemm_any_rows_kernel(AnyGemmArgs p) {
 // same columns of W2, so a lane holds gate and up of one output); wave (wm, wn) owns rows 64 wm .. and 4 x 4 MFMA
 // tiles. A k-step's 128 x 32 A and weight tiles are two 16-B pieces per thread each; rows past the group's end
 // read the tile's first row and columns past N the last one (both dropped at the store), k past K reads a
-// clamped address and zeroes the A piece.
+// clamped address and zeroes the A piece. What bounds it is a k-step's way from memory, so two of them are under way (us, one ->
+// two: 8 experts at 4096 rows, pairs of 1024 x 2048 61 -> 56, 2048 x 1024 41 -> 33; 2048 rows of 1024 x 1024 21.6 -> 16.6).
 constexpr int LM = 128, LKS = 32, LPAD = LKS + 8;
 template <int DUAL>
-__global__ __launch_bounds__(256) void gemm_any_lds_kernel(AnyGemmArgs p) {
+__global__ __launch_bounds__(256, 3) void gemm_any_lds_kernel(AnyGemmArgs p) {
   constexpr int WN = DUAL ? 64 : 128;  // columns of each weight matrix per block
   constexpr int OPAD = WN + 8;         // padded row of the staged outputs
   __shared__ __attribute__((aligned(16))) bf16_t smem[4 * LM * LPAD];  // two A and two weight buffers, then the outputs
@@ -413,32 +414,30 @@ __global__ __launch_bounds__(256) void gemm_any_lds_kernel(AnyGemmArgs p) {
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  uint4 ar[2], wr[2];
-  auto fetch = [&](int k0) {
+  struct Step {
+    uint4 a[2], w[2];
+  };
+  auto fetch = [&](Step& x, int k0) {   // (past K: a clamped address)
     const int k = k0 + kq, kk = min(k, K - 8);
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      ar[u] = ld16(asrc[u] + kk);
-      wr[u] = ld16(wsrc[u] + kk);
-      if (k >= K) ar[u] = make_uint4(0, 0, 0, 0);  // a zero A piece zeroes the product
+      x.a[u] = ld16(asrc[u] + kk);
+      x.w[u] = ld16(wsrc[u] + kk);
     }
   };
-  auto stage = [&](int buf) {
+  auto stage = [&](const Step& x, int buf, int k0) {
+    const bool in = k0 + kq < K;   // a zero A piece zeroes the product
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int row = (tid >> 2) + 64 * u;
-      *reinterpret_cast<uint4*>(&As[buf][row][kq]) = ar[u];
-      *reinterpret_cast<uint4*>(&Ws[buf][row][kq]) = wr[u];
+      *reinterpret_cast<uint4*>(&As[buf][row][kq]) = in ? x.a[u] : make_uint4(0, 0, 0, 0);
+      *reinterpret_cast<uint4*>(&Ws[buf][row][kq]) = x.w[u];
     }
   };
-  fetch(0);
-  stage(0);
-  __syncthreads();
-  int buf = 0;
-  // a buffer is rewritten one step later, after the barrier that every wave reaches only when it has read it
-  for (int k0 = 0; k0 < K; k0 += LKS) {
-    const bool more = k0 + LKS < K;
-    if (more) fetch(k0 + LKS);
+  // k-step k0 from LDS; x: what was asked for step k0 + LKS, two steps ago, goes to the other buffer, then asks for the step
+  // after the next. A buffer is rewritten one step later, after the barrier that every wave reaches only when it has read it
+  // (the barriers wait for LDS traffic only).
+  auto step = [&](Step& x, int buf, int k0) {
     bf16x8 af[4], wf[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) af[i] = as_bf16x8(*reinterpret_cast<const uint4*>(&As[buf][wm * 64 + i * 16 + lr][8 * lg]));
@@ -451,10 +450,22 @@ __global__ __launch_bounds__(256) void gemm_any_lds_kernel(AnyGemmArgs p) {
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[i][j] = mfma16(af[i], wf[j], acc[i][j]);
-    if (more) stage(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
+    stage(x, buf ^ 1, k0 + LKS);
+    fetch(x, k0 + 3 * LKS);
+    lds_barrier();
+  };
+  Step xa, xb;
+  fetch(xa, 0);
+  fetch(xb, LKS);
+  stage(xa, 0, 0);
+  fetch(xa, 2 * LKS);
+  lds_barrier();
+  int k0 = 0;
+  for (; k0 + LKS < K; k0 += 2 * LKS) {
+    step(xb, 0, k0);
+    step(xa, 1, k0 + LKS);
   }
+  if (k0 < K) step(xb, 0, k0);
   if (p.vec_out) {  // bf16 rows of whole 16-B pieces: staged in LDS (the k loop's last barrier has freed it), then stored whole
     with_act<DUAL>(p, [&](auto act) {
 #pragma unroll
