@@ -36,7 +36,7 @@
 //          (with a bonus the products stop at i - 1 and the term j = i is q_i . u k_i). Every product of decays is a product
 //          of factors <= 1 taken in order. local: the second sum, fp32 MFMA (16x16x4); carry as above; output: the
 //          triangle of weighted products (a lane holds k_j g of four D / 32 channels and walks i), then both products
-//          with fp32 MFMA, norm and gate. 2048 tokens, 8 heads of 128: 128 us, by the scan in chunks 162.
+//          with fp32 MFMA, norm and gate. 2048 tokens, 8 heads of 128: 100 us, by the scan in chunks 162.
 #include "chunks.h"
 #include "seq_launchers.h"
 
@@ -328,47 +328,116 @@ void launch_scan(const LinearAttnArgs& a, int T, const float4* vec, const float*
 }
 
 // ------------------------------------------------------------------------------- key and value sizes up to 128
-// the decay, key and query of channel d of head h at token t (x[t][h D + d] of the projections)
-template <bool F32>
-__device__ __forceinline__ void decay_key_query(const LinearAttnArgs& p, int t, int h, int d, float& a, float& k, float& q) {
+// decay, key (scaled) and query (scaled) of N (token, channel) pairs of head h; past t1 or D: 1, 0, 0. Every operand's loads stand
+// together, from clamped addresses: behind a test per pair each would be waited for by itself (2048 tokens of 8 heads of 128: the chunks' local pass 46 -> 26 us, their output
+// 60 -> 49).
+template <bool F32, int N>
+__device__ __forceinline__ void decay_key_query(const LinearAttnArgs& p, int h, int t1, const int (&t)[N], const int (&d)[N], float (&a)[N],
+                                                float (&k)[N], float (&q)[N]) {
   constexpr int f32 = F32 ? 1 : 0;
-  const int e = h * p.D + d;
-  q = ldx(p.q, (int64_t)t * p.ldq + e, f32);
-  k = ldx(p.k, (int64_t)t * p.ldk + e, f32);
-  if (p.in_silu) { q = silu_f(q); k = silu_f(k); }
-  if (d < p.rot_dims) {  // the pair's other entry, then (u, v) -> (u c - v s, v c + u s)
-    const int half = p.rot_dims >> 1;
-    const bool first = p.rot_half ? d < half : !(d & 1);
-    const int eo = p.rot_half ? (first ? e + half : e - half) : (first ? e + 1 : e - 1);
-    float qo = ldx(p.q, (int64_t)t * p.ldq + eo, f32), ko = ldx(p.k, (int64_t)t * p.ldk + eo, f32);
-    if (p.in_silu) { qo = silu_f(qo); ko = silu_f(ko); }
-    const float ang = (float)p.positions[t] * p.inv_freq[p.rot_half ? (first ? d : d - half) : (d >> 1)];
-    const float cs = cosf(ang), sn = sinf(ang);
-    q = first ? q * cs - qo * sn : q * cs + qo * sn;
-    k = first ? k * cs - ko * sn : k * cs + ko * sn;
+  int64_t tt[N];
+  int e[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    tt[i] = min(t[i], t1 - 1);
+    e[i] = h * p.D + min(d[i], p.D - 1);
   }
-  if (p.z == nullptr) a = p.head_decay[h];
-  else if (p.decay_exp) a = expf(-expf(p.z[(int64_t)t * p.ldz + e]));
-  else a = expf(log_sigmoid(p.z[(int64_t)t * p.ldz + e]) * (1.f / p.tau));
-  k *= p.k_scale;
-  q *= p.q_scale;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    q[i] = ldx(p.q, tt[i] * p.ldq + e[i], f32);
+    k[i] = ldx(p.k, tt[i] * p.ldk + e[i], f32);
+  }
+  if (p.z != nullptr) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) a[i] = p.z[tt[i] * p.ldz + e[i]];
+  } else {
+    const float hd = p.head_decay[h];
+#pragma unroll
+    for (int i = 0; i < N; ++i) a[i] = hd;
+  }
+  if (p.in_silu) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) { q[i] = silu_f(q[i]); k[i] = silu_f(k[i]); }
+  }
+  if (p.rot_dims > 0) {  // the pair's other entry, then (u, v) -> (u c - v s, v c + u s)
+    const int half = p.rot_dims >> 1;
+    float qo[N], ko[N], ang[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const bool turn = d[i] < p.rot_dims, first = p.rot_half ? d[i] < half : !(d[i] & 1);
+      const int eo = !turn ? e[i] : (p.rot_half ? (first ? e[i] + half : e[i] - half) : (first ? e[i] + 1 : e[i] - 1));
+      qo[i] = ldx(p.q, tt[i] * p.ldq + eo, f32);
+      ko[i] = ldx(p.k, tt[i] * p.ldk + eo, f32);
+      ang[i] = (float)p.positions[tt[i]] * p.inv_freq[!turn ? 0 : (p.rot_half ? (first ? d[i] : d[i] - half) : (d[i] >> 1))];
+    }
+    if (p.in_silu) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) { qo[i] = silu_f(qo[i]); ko[i] = silu_f(ko[i]); }
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (d[i] < p.rot_dims) {
+        const bool first = p.rot_half ? d[i] < half : !(d[i] & 1);
+        const float cs = cosf(ang[i]), sn = sinf(ang[i]);
+        q[i] = first ? q[i] * cs - qo[i] * sn : q[i] * cs + qo[i] * sn;
+        k[i] = first ? k[i] * cs - ko[i] * sn : k[i] * cs + ko[i] * sn;
+      }
+  }
+  if (p.z != nullptr) {
+    if (p.decay_exp) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) a[i] = expf(-expf(a[i]));
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i) a[i] = expf(log_sigmoid(a[i]) * (1.f / p.tau));
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const bool ok = t[i] < t1 && d[i] < p.D;
+    a[i] = ok ? a[i] : 1.f;
+    k[i] = ok ? k[i] * p.k_scale : 0.f;
+    q[i] = ok ? q[i] * p.q_scale : 0.f;
+  }
 }
-template <bool F32>
-__device__ __forceinline__ float value_at(const LinearAttnArgs& p, int t, int h, int c) {
-  const float v = ldx(p.v, (int64_t)t * p.ldv + h * p.V + c, F32 ? 1 : 0);
-  return p.in_silu ? silu_f(v) : v;
+// values of N (token, channel) pairs of head h; past t1 or V: 0
+template <bool F32, int N>
+__device__ __forceinline__ void values_at(const LinearAttnArgs& p, int h, int t1, const int (&t)[N], const int (&c)[N], float (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = ldx(p.v, (int64_t)min(t[i], t1 - 1) * p.ldv + h * p.V + min(c[i], p.V - 1), F32 ? 1 : 0);
+  if (p.in_silu) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = silu_f(v[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = t[i] < t1 && c[i] < p.V ? v[i] : 0.f;
 }
-// weight and gate of output channel c of head h at token t
-template <bool F32>
-__device__ __forceinline__ float weight_gate(const LinearAttnArgs& p, int t, int h, int c) {
-  const float g = ldx(p.g, (int64_t)t * p.ldg + h * p.V + c, F32 ? 1 : 0);
-  return (p.nw == nullptr ? 1.f : p.nw[p.norm_full ? h * p.V + c : c]) * (p.gate_silu ? silu_f(g) : sigm(g));
+// weight times gate of N (token, output channel) pairs of head h (past t1 or V: some other pair's)
+template <bool F32, int N>
+__device__ __forceinline__ void weights_gates(const LinearAttnArgs& p, int h, int t1, const int (&t)[N], const int (&c)[N], float (&y)[N]) {
+  float w[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    y[i] = ldx(p.g, (int64_t)min(t[i], t1 - 1) * p.ldg + h * p.V + min(c[i], p.V - 1), F32 ? 1 : 0);
+    w[i] = 1.f;
+  }
+  if (p.nw != nullptr) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) w[i] = p.nw[(p.norm_full ? h * p.V : 0) + min(c[i], p.V - 1)];
+  }
+  if (p.gate_silu) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) y[i] = w[i] * silu_f(y[i]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) y[i] = w[i] * sigm(y[i]);
+  }
 }
 
 constexpr int ST = 8;   // tokens the short kernel stages at a time
 
 // grid (sequence, head): sequences of at most `lim` tokens, key and value size up to P. PRE: with a bonus.
-// Bound by the state's bytes once sequences x heads fill the chip: 64 sequences x 8 heads of 128 (67 MB) 17.4 us, three launches
+// Bound by the state's bytes once sequences x heads fill the chip: 64 sequences x 8 heads of 128 (67 MB) 16.0 us, three launches
 // 35.2; a further token costs 1.1 us.
 template <int P, bool F32, bool PRE>
 __global__ __launch_bounds__(256) void linear_short_kernel(LinearAttnArgs p, int lim, float* __restrict__ oraw) {
@@ -398,17 +467,22 @@ __global__ __launch_bounds__(256) void linear_short_kernel(LinearAttnArgs p, int
   for (int tb = t0; tb < t1; tb += ST) {
     if (tb > t0) __syncthreads();
     {  // 32 lanes per token; channels past D: k = q = 0, a = 1 (their state stays zero)
-      const int i = tid >> 5, l = tid & 31, t = tb + i;
+      constexpr int N = P / 32;
+      const int i = tid >> 5, l = tid & 31;
+      int t[N], d[N];
+      float a[N], k[N], q[N], v[N], y[N];
 #pragma unroll
-      for (int m = 0; m < P / 32; ++m) {
-        const int d = l + 32 * m;
-        float a = 1.f, k = 0.f, q = 0.f;
-        if (t < t1 && d < D) decay_key_query<F32>(p, t, h, d, a, k, q);
-        la[i][d] = a; lk[i][d] = k; lq[i][d] = q;
-        if (PRE) lu[i][d] = d < D ? p.bonus[h * D + d] * k : 0.f;
-        const bool ok = t < t1 && d < V;
-        lv[i][d] = ok ? value_at<F32>(p, t, h, d) : 0.f;
-        if (!p.norm_all) lg[i][d] = ok ? weight_gate<F32>(p, t, h, d) : 0.f;
+      for (int m = 0; m < N; ++m) { t[m] = tb + i; d[m] = l + 32 * m; y[m] = 0.f; }
+      if (t[0] < t1) {   // (uniform per half wave)
+        decay_key_query<F32>(p, h, t1, t, d, a, k, q);
+        values_at<F32>(p, h, t1, t, d, v);
+        if (!p.norm_all) weights_gates<F32>(p, h, t1, t, d, y);
+#pragma unroll
+        for (int m = 0; m < N; ++m) {
+          la[i][d[m]] = a[m]; lk[i][d[m]] = k[m]; lq[i][d[m]] = q[m]; lv[i][d[m]] = v[m];
+          if (PRE) lu[i][d[m]] = d[m] < D ? p.bonus[h * D + d[m]] * k[m] : 0.f;
+          if (!p.norm_all) lg[i][d[m]] = t[m] < t1 && d[m] < V ? y[m] : 0.f;
+        }
       }
     }
     __syncthreads();
@@ -493,11 +567,15 @@ __global__ __launch_bounds__(256) void linear_local_kernel(LinearAttnArgs p, int
     if (d < DP) {   // from the half's last token to its first: k_j times the decays after it
       float a[CT / 2];
 #pragma unroll
-      for (int j = 0; j < CT / 2; ++j) {
-        a[j] = 1.f; k[j] = 0.f;
-        float q;
-        if (d < D && t0 + j0 + j < t1) decay_key_query<F32>(p, t0 + j0 + j, h, d, a[j], k[j], q);
-        if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < CT / 2; j += 8) {
+        int t[8], dd[8];
+        float an[8], kn[8], qn[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { t[e] = t0 + j0 + j + e; dd[e] = d; }
+        decay_key_query<F32>(p, h, t1, t, dd, an, kn, qn);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { a[j + e] = an[e]; k[j + e] = kn[e]; }
+        __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
       for (int j = CT / 2 - 1; j >= 0; --j) {
@@ -507,11 +585,14 @@ __global__ __launch_bounds__(256) void linear_local_kernel(LinearAttnArgs p, int
       if (half == 1) late[d] = g;
     }
 #pragma unroll
-    for (int j = 0; j < CT / 2; j += 4) {   // values, a column per thread
-      f32x4 v;
+    for (int j = 0; j < CT / 2; j += 8) {   // values, a column per thread
+      int t[8], c[8];
+      float v[8];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = d < V && t0 + j0 + j + e < t1 ? value_at<F32>(p, t0 + j0 + j + e, h, d) : 0.f;
-      *reinterpret_cast<f32x4*>(&vt[d][j0 + j]) = v;
+      for (int e = 0; e < 8; ++e) { t[e] = t0 + j0 + j + e; c[e] = d; }
+      values_at<F32>(p, h, t1, t, c, v);
+      *reinterpret_cast<f32x4*>(&vt[d][j0 + j]) = f32x4{v[0], v[1], v[2], v[3]};
+      *reinterpret_cast<f32x4*>(&vt[d][j0 + j + 4]) = f32x4{v[4], v[5], v[6], v[7]};
     }
     __syncthreads();
     if (d < DP) {
@@ -618,19 +699,28 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
       const int d = 16 * n + 4 * kg + e;
       B[n][e] = con && d < D ? cs[(int64_t)d * V + col] : 0.f;
     }
+  {
+    int t[CT / 4], c[CT / 4];
+    float v[CT / 4];
 #pragma unroll
-  for (int n = 0; n < CT / 16; ++n)
+    for (int u = 0; u < CT / 4; ++u) { t[u] = t0 + 16 * (u / 4) + 4 * kg + u % 4; c[u] = col; }
+    values_at<F32>(p, h, t1, t, c, v);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int t = t0 + 16 * n + 4 * kg + e;
-      vb[n][e] = con && t < t1 ? value_at<F32>(p, t, h, col) : 0.f;
+    for (int u = 0; u < CT / 4; ++u) vb[u / 4][u % 4] = v[u];
+  }
+  constexpr int PT = CT * DP / 512, PB = PT < 8 ? PT : 8;   // (token, channel) pairs of a thread, and of a batch
+#pragma unroll
+  for (int m = 0; m < PT; m += PB) {
+    int t[PB], dd[PB];
+    float a[PB], k[PB], q[PB];
+#pragma unroll
+    for (int u = 0; u < PB; ++u) { t[u] = t0 + (tid + 512 * (m + u)) / DP; dd[u] = tid % DP; }
+    decay_key_query<F32>(p, h, t1, t, dd, a, k, q);
+#pragma unroll
+    for (int u = 0; u < PB; ++u) {
+      const int at = (t[u] - t0) * DS + dd[u];
+      la[at] = a[u]; lk[at] = k[u]; lq[at] = q[u];
     }
-#pragma unroll 4
-  for (int e = tid; e < CT * DP; e += 512) {
-    const int i = e / DP, d = e % DP;
-    float a = 1.f, k = 0.f, q = 0.f;
-    if (d < D && t0 + i < t1) decay_key_query<F32>(p, t0 + i, h, d, a, k, q);
-    la[i * DS + d] = a; lk[i * DS + d] = k; lq[i * DS + d] = q;
   }
   for (int e = tid; e < CT * CTP; e += 512) tr[e] = 0.f;
   __syncthreads();
@@ -718,6 +808,13 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
       }
     return;
   }
+  float wg[CT / 4];
+  {
+    int t[CT / 4], c[CT / 4];
+#pragma unroll
+    for (int u = 0; u < CT / 4; ++u) { t[u] = t0 + 16 * (u / 4) + 4 * kg + u % 4; c[u] = col; }
+    weights_gates<F32>(p, h, t1, t, c, wg);
+  }
 #pragma unroll
   for (int r = 0; r < CT / 16; ++r)
 #pragma unroll
@@ -739,7 +836,7 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
       float ss = 0.f;
 #pragma unroll
       for (int m = 0; m < 8; ++m) ss += red[m * CT + row];
-      const float y = acc[r][i] * (1.f / sqrtf(ss / (float)V + p.eps)) * weight_gate<F32>(p, t, h, col);
+      const float y = acc[r][i] * (1.f / sqrtf(ss / (float)V + p.eps)) * wg[4 * r + i];
       const int64_t oi = (int64_t)t * p.ldo + h * V + col;
       if (F32) reinterpret_cast<float*>(p.out)[oi] = y;
       else reinterpret_cast<bf16_t*>(p.out)[oi] = f2bf(y);
@@ -750,8 +847,8 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
 int short_limit(int T) { return T <= 96 ? T : 64; }
 // chunks of a step whose sequences longer than lim tokens have T between them: each has at most one that is not whole
 int long_chunks(int T, int lim) { return T <= lim ? 0 : T / CT + T / (lim + 1); }
-// Decoding steps: one launch instead of three (16 sequences x 8 heads of 128: 25.3 -> 11.7 us). Long steps: chunks with fp32 MFMA
-// (2048 tokens 162 -> 128 us, 63 decoded tokens beside a portion of 961 1054 -> 206, 64 portions of 16 62 -> 51). Between them
+// Decoding steps: one launch instead of three (16 sequences x 8 heads of 128: 25.3 -> 12.2 us). Long steps: chunks with fp32 MFMA
+// (2048 tokens 162 -> 100 us, 63 decoded tokens beside a portion of 961 1054 -> 169, 64 portions of 16 62 -> 47). Between them
 // the scan below, which spreads a head's columns over several workgroups, is ahead where sequences are few: one portion of
 // 64 58 us (here 79), of 256 90 (103), 8 of 48 54 (68).
 bool takes_small(int T, int S, int D, int V, int cols_per_lane) {
