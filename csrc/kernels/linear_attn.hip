@@ -850,10 +850,10 @@ int long_chunks(int T, int lim) { return T <= lim ? 0 : T / CT + T / (lim + 1); 
 // Decoding steps: one launch instead of three (16 sequences x 8 heads of 128: 25.3 -> 12.2 us). Long steps: chunks with fp32 MFMA
 // (2048 tokens 162 -> 100 us, 63 decoded tokens beside a portion of 961 1054 -> 169, 64 portions of 16 62 -> 47). Between them
 // the scan below, which spreads a head's columns over several workgroups, is ahead where sequences are few: one portion of
-// 64 58 us (here 79), of 256 90 (103), 8 of 48 54 (68).
+// 96 78 us (here 96; of 128 98 against 84), 8 of 48 54 (59).
 bool takes_small(int T, int S, int D, int V, int cols_per_lane) {
   return D <= 128 && V <= 128 && cols_per_lane == 0 &&
-         (T <= 2 * S || T >= (S == 1 ? 1024 : (S < 16 ? 512 : 256)));
+         (T <= 2 * S || T >= (S == 1 ? 128 : (S < 16 ? 512 : 256)));
 }
 
 template <int DP, bool F32, bool PRE>

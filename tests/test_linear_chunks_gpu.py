@@ -48,7 +48,7 @@ def _run(H, D, V, lens, pos, dt, variant, seed, device, pad=3):
 @pytest.mark.parametrize("variant", list(VARIANTS))
 @pytest.mark.parametrize("H,D,V", [(2, 1, 5), (3, 32, 33), (2, 64, 16), (1, 100, 128), (9, 128, 128), (2, 130, 40)])
 @pytest.mark.parametrize("lens,pos", [([1100], [0]), ([300, 65, 1, 64, 150], [0, 9, 40, 0, 2]), ([1] * 15 + [129, 150], [5] * 17),
-                                      ([1] * 6 + [3, 2], [4] * 8), ([64, 65, 1], [0, 9, 40])])
+                                      ([1] * 6 + [3, 2], [4] * 8), ([64, 65, 1], [0, 9, 40]), ([124], [2]), ([125], [0])])
 def test_matches_cpu_form(H, D, V, lens, pos, variant, dt):
     out, state = _run(H, D, V, lens, pos, dt, variant, 3 * H + D + V, "cuda")
     want, state_w = _run(H, D, V, lens, pos, dt, variant, 3 * H + D + V, "cpu")
