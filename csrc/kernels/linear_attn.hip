@@ -792,10 +792,23 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
     f32x4 A[CT / 16];
 #pragma unroll
     for (int r = n; r < CT / 16; ++r) A[r] = ld4(&tr[(16 * r + lr) * CTP + 16 * n + 4 * kg]);
+    // the zeros above the diagonal would turn an infinity or a NaN into NaN for the tokens before it: such a block goes term by term
+    const f32x4 z = vb[n] * 0.f;
+    const bool finite = __all(z[0] + z[1] + (z[2] + z[3]) == 0.f);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int r = n; r < CT / 16; ++r) acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[r][e], vb[n][e], acc[r], 0, 0, 0);
+      for (int r = n; r < CT / 16; ++r)
+        if (r > n || finite) acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[r][e], vb[n][e], acc[r], 0, 0, 0);
+    if (!finite)
+      for (int j = 0; j < 16; ++j) {
+        const int from = lr + 16 * (j / 4);
+        const float v0 = __shfl(vb[n][0], from, 64), v1 = __shfl(vb[n][1], from, 64), v2 = __shfl(vb[n][2], from, 64), v3 = __shfl(vb[n][3], from, 64);
+        const float v = j % 4 == 0 ? v0 : (j % 4 == 1 ? v1 : (j % 4 == 2 ? v2 : v3));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (j <= 4 * kg + i) acc[n][i] = fmaf(tr[(16 * n + 4 * kg + i) * CTP + 16 * n + j], v, acc[n][i]);
+      }
   }
   // acc[r][i]: token 16 r + 4 kg + i, column col (columns past V are zero)
   if (p.norm_all) {
