@@ -47,6 +47,7 @@
 // Every row of every kernel depends only on its own sequence's cache rows, in an order fixed by the
 // position, so results do not depend on how a prompt is cut or what else is in the batch.
 #include <algorithm>
+#include <type_traits>
 
 #include "locate.h"
 #include "seq_launchers.h"
@@ -77,107 +78,139 @@ __device__ __forceinline__ int first_key(const WindowArgs& a, int p) {
   return a.chunk > 0 ? max(lo, p - p % a.chunk) : lo;
 }
 
-// One wave per head (queries, keys, values), D <= 128 NP. A lane holds NP pairs of entries and turns each with one angle; nothing goes
-// through LDS and no wave waits for another (a norm over the whole projection is summed by every wave for itself). What bounds it
-// is the way to memory and back, three times (slot and position, row, store), and the angles. 16 tokens of 12 heads of 128: 5.0 us,
-// 2048: 17; a workgroup per token, whose elements went through LDS and took an angle each, 10.5 and 22.
-template <int NP, bool F32>
-__global__ __launch_bounds__(256) void window_write_kernel(WindowArgs a, const void* __restrict__ q, int64_t ldq,
+// One wave per head (queries, keys, values), D <= 128 NP. A lane holds NP pairs of entries and turns each with one angle. What bounds
+// it is the way to memory and back, three times (slot and position, row, store), and the angles. 16 tokens of 12 heads of 128: 4.0 us,
+// 2048: 13; a workgroup per token, whose elements went through LDS and took an angle each, 8 and 17.
+// Norm over the whole projections: SUM_WAVE, every wave sums the squares of its projection for itself, and no wave waits for another.
+// SUM_BLOCK, one workgroup per token, whose waves sum together and then take the heads in turn (the queries are read whole before any of
+// them is stored: q_out may be q).
+enum { SUM_HEAD = 0, SUM_WAVE = 1, SUM_BLOCK = 2 };
+constexpr int WRITE_WAVES = 8;   // most waves of a SUM_BLOCK workgroup (us at 2048 tokens of 12 + 12 heads, 4 / 8 / 16: 36, 36, 51)
+template <int NP, bool F32, int SUM>
+__global__ __launch_bounds__(SUM == SUM_BLOCK ? 64 * WRITE_WAVES : 256) void window_write_kernel(WindowArgs a, const void* q, int64_t ldq,
                                                                   const void* __restrict__ k, int64_t ldk,
                                                                   const void* __restrict__ v, int64_t ldv,
                                                                   const float* __restrict__ qw, const float* __restrict__ kw, float eps,
-                                                                  int norm_all, void* __restrict__ q_out, bf16_t* __restrict__ vt,
+                                                                  void* q_out, bf16_t* __restrict__ vt,
                                                                   const float* __restrict__ q_head_scale, float q_temp_coef,
                                                                   int q_temp_every, int rot_half, const void* __restrict__ v_other,
                                                                   int64_t ldo, float lam) {
   constexpr int f32 = F32 ? 1 : 0;
   const int H = a.H, G = a.G, D = a.D, V = a.V, GV = a.GV;
-  const int t = blockIdx.x, h = 4 * blockIdx.y + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int slot = a.slots[t];
-  if (slot < 0 || h >= H + G + GV) return;  // padding row, no head
+  const int t = blockIdx.x, wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int slot = a.slots[t], heads = H + G + GV;
+  const int h0 = SUM == SUM_BLOCK ? wv : 4 * blockIdx.y + wv;
+  if (slot < 0 || (SUM != SUM_BLOCK && h0 >= heads)) return;  // padding row (uniform per workgroup), no head
   const int ipos = a.positions[t];
   const float pos = (float)ipos;
   const int page = a.page;
   const int64_t pg = slot / page, off = slot % page;
-  if (h < H + G) {
-    const bool isq = h < H;
-    const void* src = isq ? q : k;
-    const int64_t ro = isq ? (int64_t)t * ldq + (int64_t)h * D : (int64_t)t * ldk + (int64_t)(h - H) * D;
-    const float* w = isq ? qw : kw;
-    if (w != nullptr && norm_all) w += (isq ? h : h - H) * D;   // (one weight per entry of the projection)
-    const int hr = a.rot_dims >> 1;
-    int i0[NP], i1[NP];
-    float x0[NP], x1[NP], w0[NP], w1[NP], f[NP], ss = 0.f;
+  float all_q = 0.f, all_k = 0.f;   // SUM_BLOCK: sums of squares of the projections
+  if constexpr (SUM == SUM_BLOCK) {
+    __shared__ float part[2][WRITE_WAVES];
+    auto squares = [&](const void* src, int64_t r0, int n) {
+      float ss = 0.f;
+      for (int e0 = threadIdx.x; e0 < n; e0 += 4 * blockDim.x) {
+        float x[4];
 #pragma unroll
-    for (int m = 0; m < NP; ++m) {  // pairs (2j, 2j + 1), or (j, j + rot_dims / 2) with rot_half; past the turned entries neighbours
-      const int j = lane + 64 * m;
-      i0[m] = j < hr && rot_half ? j : 2 * j;
-      i1[m] = j < hr && rot_half ? j + hr : 2 * j + 1;
-      x0[m] = i0[m] < D ? ldx(src, ro + i0[m], f32) : 0.f;
-      x1[m] = i1[m] < D ? ldx(src, ro + i1[m], f32) : 0.f;
-      w0[m] = w != nullptr && i0[m] < D ? w[i0[m]] : 1.f;
-      w1[m] = w != nullptr && i1[m] < D ? w[i1[m]] : 1.f;
-      f[m] = j < hr ? a.inv_freq[j] : 0.f;
-      ss = fmaf(x0[m], x0[m], fmaf(x1[m], x1[m], ss));
-    }
-    float count = (float)D;
-    if (norm_all && w != nullptr) {
-      const int n = (isq ? H : G) * D;
-      const int64_t r0 = isq ? (int64_t)t * ldq : (int64_t)t * ldk;
-      count = (float)n;
-      ss = 0.f;
-      for (int e0 = lane; e0 < n; e0 += 64 * 8) {
-        float x[8];
+        for (int u = 0; u < 4; ++u) x[u] = ldx(src, r0 + min(e0 + u * (int)blockDim.x, n - 1), f32);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = ldx(src, r0 + min(e0 + 64 * u, n - 1), f32);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) ss = e0 + 64 * u < n ? fmaf(x[u], x[u], ss) : ss;
+        for (int u = 0; u < 4; ++u) ss = e0 + u * (int)blockDim.x < n ? fmaf(x[u], x[u], ss) : ss;
       }
-    }
-    const float sc = w != nullptr ? 1.f / sqrtf(wave_reduce_sum(ss) / count + eps) : 1.f;
-    float grow = 1.f;
-    if (isq) {  // query temperature of the position: 1 + coef ln(floor((p + 1) / every) + 1)
-      if (q_temp_coef != 0.f) grow = 1.f + q_temp_coef * logf((float)((ipos + 1) / q_temp_every) + 1.f);
-      if (q_head_scale != nullptr) grow = q_head_scale[h] * grow;
-    }
-    void* dst = isq ? q_out : a.kc;
-    const int64_t so = isq ? ((int64_t)t * H + h) * D : ((pg * G + (h - H)) * page + off) * D;
+      return wave_reduce_sum(ss);
+    };
+    const float sq = squares(q, (int64_t)t * ldq, H * D), sk = squares(k, (int64_t)t * ldk, G * D);
+    if (lane == 0) { part[0][wv] = sq; part[1][wv] = sk; }
+    __syncthreads();
+    for (int i = 0; i < (int)(blockDim.x >> 6); ++i) { all_q += part[0][i]; all_k += part[1][i]; }
+  }
+  auto prepare = [&](int h) {
+    if (h < H + G) {
+      const bool isq = h < H;
+      const void* src = isq ? q : k;
+      const int64_t ro = isq ? (int64_t)t * ldq + (int64_t)h * D : (int64_t)t * ldk + (int64_t)(h - H) * D;
+      const float* w = isq ? qw : kw;
+      if (SUM != SUM_HEAD) w += (isq ? h : h - H) * D;   // (one weight per entry of the projection)
+      const int hr = a.rot_dims >> 1;
+      int i0[NP], i1[NP];
+      float x0[NP], x1[NP], w0[NP], w1[NP], f[NP], ss = 0.f;
 #pragma unroll
-    for (int m = 0; m < NP; ++m) {
-      float y0 = x0[m] * sc * w0[m], y1 = x1[m] * sc * w1[m];
-      if (lane + 64 * m < hr) {
+      for (int m = 0; m < NP; ++m) {  // pairs (2j, 2j + 1), or (j, j + rot_dims / 2) with rot_half; past the turned entries neighbours
+        const int j = lane + 64 * m;
+        i0[m] = j < hr && rot_half ? j : 2 * j;
+        i1[m] = j < hr && rot_half ? j + hr : 2 * j + 1;
+        x0[m] = i0[m] < D ? ldx(src, ro + i0[m], f32) : 0.f;
+        x1[m] = i1[m] < D ? ldx(src, ro + i1[m], f32) : 0.f;
+        w0[m] = w != nullptr && i0[m] < D ? w[i0[m]] : 1.f;
+        w1[m] = w != nullptr && i1[m] < D ? w[i1[m]] : 1.f;
+        f[m] = j < hr ? a.inv_freq[j] : 0.f;
+        ss = fmaf(x0[m], x0[m], fmaf(x1[m], x1[m], ss));
+      }
+      float sc = 1.f;
+      if constexpr (SUM == SUM_BLOCK) {
+        sc = 1.f / sqrtf((isq ? all_q / (float)(H * D) : all_k / (float)(G * D)) + eps);
+      } else if constexpr (SUM == SUM_WAVE) {
+        const int n = (isq ? H : G) * D;
+        const int64_t r0 = isq ? (int64_t)t * ldq : (int64_t)t * ldk;
+        ss = 0.f;
+        for (int e0 = lane; e0 < n; e0 += 64 * 8) {
+          float x[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) x[u] = ldx(src, r0 + min(e0 + 64 * u, n - 1), f32);
+#pragma unroll
+          for (int u = 0; u < 8; ++u) ss = e0 + 64 * u < n ? fmaf(x[u], x[u], ss) : ss;
+        }
+        sc = 1.f / sqrtf(wave_reduce_sum(ss) / (float)n + eps);
+      } else if (w != nullptr) {
+        sc = 1.f / sqrtf(wave_reduce_sum(ss) / (float)D + eps);
+      }
+      float grow = 1.f;
+      if (isq) {  // query temperature of the position: 1 + coef ln(floor((p + 1) / every) + 1)
+        if (q_temp_coef != 0.f) grow = 1.f + q_temp_coef * logf((float)((ipos + 1) / q_temp_every) + 1.f);
+        if (q_head_scale != nullptr) grow = q_head_scale[h] * grow;
+      }
+      void* dst = isq ? q_out : a.kc;
+      const int64_t so = isq ? ((int64_t)t * H + h) * D : ((pg * G + (h - H)) * page + off) * D;
+#pragma unroll
+      for (int m = 0; m < NP; ++m) {
+        float y0 = x0[m] * sc * w0[m], y1 = x1[m] * sc * w1[m];
+        if (lane + 64 * m < hr) {
+          float sn, cs;
+          sincosf(pos * f[m], &sn, &cs);
+          const float z0 = y0 * cs - y1 * sn, z1 = y1 * cs + y0 * sn;
+          y0 = z0; y1 = z1;
+        }
+        if (i0[m] < D) stx(dst, so + i0[m], f32, isq ? y0 * grow : y0);
+        if (i1[m] < D) stx(dst, so + i1[m], f32, isq ? y1 * grow : y1);
+      }
+      return;
+    }
+    const int g = h - H - G;
+    const int64_t vo = ((pg * GV + g) * page + off) * V, to = (pg * GV + g) * V;
+    auto val = [&](int i) {  // entry i of the head's values, blended with the other row's
+      const float x = ldx(v, (int64_t)t * ldv + (int64_t)g * V + i, f32);
+      return v_other != nullptr ? fmaf(lam, ldx(v_other, (int64_t)t * ldo + (int64_t)g * V + i, f32), (1.f - lam) * x) : x;
+    };
+    for (int j = lane; 2 * j < V; j += 64) {
+      const int i = 2 * j;
+      float y0 = val(i), y1 = i + 1 < V ? val(i + 1) : 0.f;
+      if (a.v_freq != nullptr && i + 1 < V) {
         float sn, cs;
-        sincosf(pos * f[m], &sn, &cs);
+        sincosf(pos * a.v_freq[j], &sn, &cs);
         const float z0 = y0 * cs - y1 * sn, z1 = y1 * cs + y0 * sn;
         y0 = z0; y1 = z1;
       }
-      if (i0[m] < D) stx(dst, so + i0[m], f32, isq ? y0 * grow : y0);
-      if (i1[m] < D) stx(dst, so + i1[m], f32, isq ? y1 * grow : y1);
+      stx(a.vc, vo + i, f32, y0);
+      if (i + 1 < V) stx(a.vc, vo + i + 1, f32, y1);
+      if (vt != nullptr) {  // [page][GV][column][key in page]
+        vt[(to + i) * page + off] = f2bf(y0);
+        if (i + 1 < V) vt[(to + i + 1) * page + off] = f2bf(y1);
+      }
     }
-    return;
-  }
-  const int g = h - H - G;
-  const int64_t vo = ((pg * GV + g) * page + off) * V, to = (pg * GV + g) * V;
-  auto val = [&](int i) {  // entry i of the head's values, blended with the other row's
-    const float x = ldx(v, (int64_t)t * ldv + (int64_t)g * V + i, f32);
-    return v_other != nullptr ? fmaf(lam, ldx(v_other, (int64_t)t * ldo + (int64_t)g * V + i, f32), (1.f - lam) * x) : x;
   };
-  for (int j = lane; 2 * j < V; j += 64) {
-    const int i = 2 * j;
-    float y0 = val(i), y1 = i + 1 < V ? val(i + 1) : 0.f;
-    if (a.v_freq != nullptr && i + 1 < V) {
-      float sn, cs;
-      sincosf(pos * a.v_freq[j], &sn, &cs);
-      const float z0 = y0 * cs - y1 * sn, z1 = y1 * cs + y0 * sn;
-      y0 = z0; y1 = z1;
-    }
-    stx(a.vc, vo + i, f32, y0);
-    if (i + 1 < V) stx(a.vc, vo + i + 1, f32, y1);
-    if (vt != nullptr) {  // [page][GV][column][key in page]
-      vt[(to + i) * page + off] = f2bf(y0);
-      if (i + 1 < V) vt[(to + i + 1) * page + off] = f2bf(y1);
-    }
-  }
+  if constexpr (SUM == SUM_BLOCK)
+    for (int h = h0; h < heads; h += blockDim.x >> 6) prepare(h);
+  else prepare(h0);
 }
 
 template <typename T>
@@ -1112,12 +1145,30 @@ void launch_window_write(const WindowArgs& a, const void* q, int64_t ldq, const 
                          const float* q_head_scale, float q_temp_coef, int q_temp_every, int rot_half, const void* v_other,
                          int64_t ldo, float lam, hipStream_t st) {
   if (a.T <= 0) return;
-  // (D <= 1024: window_attn_fits())
-  auto kern = a.D <= 128 ? (a.f32 ? window_write_kernel<1, true> : window_write_kernel<1, false>)
-            : a.D <= 256 ? (a.f32 ? window_write_kernel<2, true> : window_write_kernel<2, false>)
-                         : (a.f32 ? window_write_kernel<8, true> : window_write_kernel<8, false>);
-  hipLaunchKernelGGL(kern, dim3(a.T, (a.H + a.G + a.GV + 3) / 4), dim3(256), 0, st, a, q, ldq, k, ldk, v, ldv, qw, kw, eps, norm_all,
-                     q_out, reinterpret_cast<bf16_t*>(vt), q_head_scale, q_temp_coef, q_temp_every, rot_half, v_other, ldo, lam);
+  // (D <= 1024: window_attn_fits(); norm_all without weights: no norm)
+  const int heads = a.H + a.G + a.GV;
+  const bool all = norm_all && qw != nullptr;
+  // A wave's own sum reads H (or G) times as much in all and waits for nobody: ahead up to some 25 M elements (us, own / workgroup's:
+  // 64 tokens of 64 + 8 heads of 128 12.6, 13.8, of 100 + 10 24.8, 19.1; 256 of 12 + 12 9.3, 10.1, of 32 + 8 14.2, 11.4; 2048 of 8 + 2
+  // 16.1, 17.3, of 12 + 12 47.5, 35.7, of 100 + 10 536, 83). Queries stored over themselves must all have been read.
+  const int64_t es = a.f32 ? 4 : 2, qb = reinterpret_cast<int64_t>(q), ob = reinterpret_cast<int64_t>(q_out);
+  const bool over = ob < qb + ((a.T - 1) * ldq + (int64_t)a.H * a.D) * es && qb < ob + (int64_t)a.T * a.H * a.D * es;
+  const bool block = all && (over || (int64_t)a.T * (a.H * a.H + a.G * a.G) * a.D > 25000000);
+  auto launch = [&](auto np, auto f32) {
+    constexpr int NP = decltype(np)::value;
+    constexpr bool F32 = decltype(f32)::value;
+    auto kern = block ? window_write_kernel<NP, F32, SUM_BLOCK> : (all ? window_write_kernel<NP, F32, SUM_WAVE> : window_write_kernel<NP, F32, SUM_HEAD>);
+    const dim3 grid = block ? dim3(a.T) : dim3(a.T, (heads + 3) / 4);
+    hipLaunchKernelGGL(kern, grid, dim3(block ? 64 * std::min(heads, WRITE_WAVES) : 256), 0, st, a, q, ldq, k, ldk, v, ldv, qw, kw, eps, q_out,
+                       reinterpret_cast<bf16_t*>(vt), q_head_scale, q_temp_coef, q_temp_every, rot_half, v_other, ldo, lam);
+  };
+  auto sized = [&](auto np) {
+    if (a.f32) launch(np, std::true_type{});
+    else launch(np, std::false_type{});
+  };
+  if (a.D <= 128) sized(std::integral_constant<int, 1>{});
+  else if (a.D <= 256) sized(std::integral_constant<int, 2>{});
+  else sized(std::integral_constant<int, 8>{});
 }
 
 void launch_window_pool(const WindowArgs& a, hipStream_t st) {

@@ -45,3 +45,23 @@ def test_matches_cpu_form(H, G, GV, D, V, norm, rot_half, extras, dt):
         assert ((a - b).abs() <= (2e-5 if dt == torch.float32 else 2.0 ** -7 * b.abs() + 2e-5)).all()
     if got[3] is not None:
         assert torch.equal(got[3], got[2].transpose(2, 3))
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("H,G,GV,D", [(1, 1, 1, 8), (12, 2, 2, 128), (14, 2, 2, 128), (100, 10, 5, 128), (8, 4, 4, 300), (250, 5, 1, 24)])
+def test_norm_over_the_whole_projection(H, G, GV, D, in_place, dt):
+    """Heads that fit one workgroup's waves, one more, many: queries prepared beside or in their own rows."""
+    def run(device):
+        g = torch.Generator().manual_seed(H)
+        T, page, pages = 9, 16, 2
+        q, k, v = (torch.randn(T, h * D, generator=g).to(dt).to(device) for h in (H, G, GV))
+        qw, kw = (1 + 0.1 * torch.randn(h * D, generator=g).to(device) for h in (H, G))
+        slots, pos = torch.randperm(page * pages, generator=g)[:T].int().to(device), torch.randint(0, 3000, (T,), generator=g).int().to(device)
+        kc, vc = torch.zeros(pages, G, page, D, dtype=dt, device=device), torch.zeros(pages, GV, page, D, dtype=dt, device=device)
+        out = q if in_place else torch.zeros_like(q)
+        seq.window_write(q, k, v, qw, kw, 1e-6, True, pos, slots, seq.rope_inv_freq(8, 10000.0, device), 8, None, kc, vc, out, H, G)
+        return out.float().cpu(), kc.float().cpu(), vc.float().cpu()
+
+    for a, b in zip(run("cuda"), run("cpu")):   # (bounds as above)
+        assert ((a - b).abs() <= (2e-5 if dt == torch.float32 else 2.0 ** -7 * b.abs() + 2e-5)).all()
