@@ -25,8 +25,17 @@
 //          S stays in registers (C layout) and goes round through LDS as B operand; the part of the update that only
 //          needs v runs before the wait for p.
 //   chunk finish  norm and gate, from the scan's [column][token] tiles.
+// Portions in between, of few sequences (takes_scan() has the lines), take three launches of another kind:
+//   prep   (token, head) parallel: the per-channel fp32 vectors {w, a u, k, r} and u of every token.
+//   scan   the recurrence token by token. Column v of S depends on no other, so a wave owns 8 of a head's value columns: lane =
+//          (key group of eight, column), D / 8 state entries in registers, the sums over keys D / 8 FMAs and three lane
+//          exchanges. The dependent chain of a token is what bounds it. Tokens are staged through LDS eight at a time, the next eight
+//          loaded while the current ones compute.
+//   finish (token, head) parallel: head norm, weight, gate.
 // 2048 tokens, 8 heads of 128: 73 + 154 + 17 us; the tokens one after another (three launches, one wave per 8 columns) took
 // 1060 us, 0.5 us of chain per token. What bounds the chunk scan is its 64 MFMAs per wave and two barriers per 32 tokens.
+#include <algorithm>
+
 #include "chunks.h"
 #include "seq_launchers.h"
 
@@ -173,6 +182,201 @@ __global__ __launch_bounds__(256) void delta_short_kernel(DeltaArgs p, int lim) 
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (c + e < D) q[e] = S[j][e];
+  }
+}
+
+// ------------------------------------------------------------------------------------------ tokens one by one, a head's columns apart
+// token t belongs to a sequence with a slot and at most `lim` tokens (no sequence: a padding row of a graph bucket); whole waves, a lane
+// per sequence
+__device__ __forceinline__ bool token_of_short(const DeltaArgs& p, int t, int lim) {
+  for (int i0 = 0; i0 < p.S; i0 += 64) {
+    const int i = i0 + (threadIdx.x & 63);
+    const int a = i < p.S ? p.query_start[i] : 0, b = i < p.S ? p.query_start[i + 1] : 0;
+    const unsigned long long hit = __ballot(a <= t && t < b), ok = __ballot(i < p.S && p.state_slots[i] >= 0 && b - a <= lim);
+    if (hit != 0) return (hit & ok) != 0;
+  }
+  return false;
+}
+
+// one wave per (token, head): vec[t][h][d] = {w, a u, k, r}, un[t][h][d] = u
+__global__ __launch_bounds__(64) void delta_prep_kernel(DeltaArgs p, int lim, float4* __restrict__ vec,
+                                                         float* __restrict__ un) {
+  const int t = blockIdx.x, h = blockIdx.y;
+  if (!token_of_short(p, t, lim)) return;
+  const int D = p.D, lane = threadIdx.x;
+  float kk[2], rr[2], aa[2], ww[2];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int d = lane + 64 * i;
+    kk[i] = rr[i] = aa[i] = ww[i] = 0.f;
+    if (d < D) {
+      const int ch = h * D + d;
+      const int64_t ix = (int64_t)t * p.ld + ch;
+      kk[i] = ldx(p.k, ix, p.f32);
+      rr[i] = ldx(p.r, ix, p.f32);
+      aa[i] = sigm(ldx(p.a, ix, p.f32) + p.ab[ch]);
+      ww[i] = expf(-p.decay_c * sigm(ldx(p.wl, (int64_t)t * p.ldw + ch, p.f32) + p.w0[ch]));
+      ss = fmaf(kk[i], kk[i], ss);
+    }
+  }
+  ss = wave_reduce_sum(ss);
+  const float inv = 1.f / sqrtf(ss + p.unit_eps);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int d = lane + 64 * i;
+    if (d < D) {
+      const float u = kk[i] * inv;
+      const int64_t o = ((int64_t)t * p.H + h) * D + d;
+      vec[o] = make_float4(ww[i], aa[i] * u, kk[i], rr[i]);
+      un[o] = u;
+    }
+  }
+}
+
+// lane = 8 * q + c: key group q of 8 (keys [q DQ', (q + 1) DQ') with DQ' = ceil(D / 8)), value column c0 + c
+template <int DQ>
+__global__ __launch_bounds__(64) void delta_scan_kernel(DeltaArgs p, int lim, const float4* __restrict__ vec,
+                                                         const float* __restrict__ un, float* __restrict__ oraw) {
+  // quarter strides padded (DQ + 1 float4 / DQ + 4 floats): the four quarters' broadcast reads of one
+  // instruction fall into different LDS banks. Entries of channels past D are zeroed once and never
+  // written, so the token loops run DQ iterations with no bounds test (zeros leave S, u^T S and o alone).
+  constexpr int QV = DQ + 1, QU = DQ + 4;
+  __shared__ float4 lv[2][TC][8 * QV];
+  __shared__ float lu[2][TC][8 * QU];
+  __shared__ float lvv[2][TC][8];  // the slice's value columns of each staged token
+  const int s = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 8;
+  const int slot = p.state_slots[s];
+  const int t0 = p.query_start[s], t1 = p.query_start[s + 1];
+  if (slot < 0 || t1 <= t0 || t1 - t0 > lim) return;
+  const int D = p.D, lane = threadIdx.x;
+  const int q = lane >> 3, c = c0 + (lane & 7);
+  const int dq = (D + 7) >> 3;         // keys per group at run time (<= DQ)
+  const int k0 = q * dq;
+  const bool con = c < D;
+  const int pos0 = p.context_lens[s] - (t1 - t0);
+  float* sp = p.state + ((int64_t)slot * p.H + h) * D * D;
+  float S[DQ];
+#pragma unroll
+  for (int j = 0; j < DQ; ++j)
+    S[j] = (con && j < dq && k0 + j < D && pos0 > 0) ? sp[(int64_t)(k0 + j) * D + c] : 0.f;
+  // staging: a token's D channels are D float4 + D floats; lane l moves channels l, l + 64 of each token
+  float4 pv[TC][2];
+  float pu[TC][2];
+  float pvv;
+  auto fetch = [&](int tb) {
+#pragma unroll
+    for (int i = 0; i < TC; ++i)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int d = lane + 64 * e, t = tb + i;
+        const bool ok = d < D && t < t1;
+        const int64_t o = ((int64_t)(ok ? t : t0) * p.H + h) * D + (ok ? d : 0);
+        pv[i][e] = ok ? vec[o] : make_float4(0.f, 0.f, 0.f, 0.f);
+        pu[i][e] = ok ? un[o] : 0.f;
+      }
+    {  // TC x 8 values, lane -> (token, column)
+      const int t = tb + (lane >> 3), cc = c0 + (lane & 7);
+      pvv = (t < t1 && cc < D) ? ldx(p.v, (int64_t)t * p.ld + h * D + cc, p.f32) : 0.f;
+    }
+  };
+  // LDS index of channel d: quarter-major, padded to DQ per quarter
+  auto put = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < TC; ++i)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int d = lane + 64 * e;
+        if (d < D) {
+          lv[buf][i][(d / dq) * QV + (d % dq)] = pv[i][e];
+          lu[buf][i][(d / dq) * QU + (d % dq)] = pu[i][e];
+        }
+      }
+    lvv[buf][lane >> 3][lane & 7] = pvv;
+  };
+  for (int e = lane; e < 2 * TC * 8 * QV; e += 64) (&lv[0][0][0])[e] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int e = lane; e < 2 * TC * 8 * QU; e += 64) (&lu[0][0][0])[e] = 0.f;
+  __syncthreads();
+  fetch(t0);
+  put(0);
+  __syncthreads();
+  int buf = 0;
+  for (int tb = t0; tb < t1; tb += TC) {
+    const bool more = tb + TC < t1;
+    if (more) fetch(tb + TC);
+    const int nt = min(TC, t1 - tb);
+    // unrolled over the staged tokens, with token i + 1's vectors read from LDS into a second register
+    // set before token i's FMAs and lane exchanges (they do not depend on the state)
+    float4 xv[2][DQ];
+    float xu[2][DQ], xvv[2];
+    auto grab = [&](int i, int r) {
+      const float4* tv = &lv[buf][i][q * QV];
+      const float* tu = &lu[buf][i][q * QU];
+#pragma unroll
+      for (int j = 0; j < DQ; ++j) { xv[r][j] = tv[j]; xu[r][j] = tu[j]; }
+      xvv[r] = lvv[buf][i][lane & 7];
+    };
+    grab(0, 0);
+#pragma unroll
+    for (int i = 0; i < TC; ++i) {
+      if (i >= nt) break;
+      if (i + 1 < TC) grab(i + 1, (i + 1) & 1);  // (past nt: stale but finite LDS, never used)
+      const int r = i & 1;
+      const float vv = xvv[r];
+      float uS = 0.f;
+#pragma unroll
+      for (int j = 0; j < DQ; ++j) uS = fmaf(xu[r][j], S[j], uS);
+      uS += row_rot<0x128>(uS);
+      uS += xor16(uS);
+      uS += xor32(uS);
+      float o = 0.f;
+#pragma unroll
+      for (int j = 0; j < DQ; ++j) {
+        const float4 x = xv[r][j];  // {w, a u, k, r}
+        S[j] = fmaf(x.z, vv, fmaf(-x.y, uS, x.x * S[j]));
+        o = fmaf(x.w, S[j], o);
+      }
+      o += row_rot<0x128>(o);
+      o += xor16(o);
+      o += xor32(o);
+      if (con && q == 0) oraw[(int64_t)(tb + i) * p.H * D + h * D + c] = o;
+    }
+    if (more) {
+      put(buf ^ 1);
+      __syncthreads();
+      buf ^= 1;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < DQ; ++j)
+    if (con && j < dq && k0 + j < D) sp[(int64_t)(k0 + j) * D + c] = S[j];
+}
+
+// one wave per (token, head)
+__global__ __launch_bounds__(64) void delta_finish_kernel(DeltaArgs p, int lim, const float* __restrict__ oraw) {
+  const int t = blockIdx.x, h = blockIdx.y;
+  if (!token_of_short(p, t, lim)) return;
+  const int D = p.D, lane = threadIdx.x;
+  float o[2];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int d = lane + 64 * i;
+    o[i] = d < D ? oraw[((int64_t)t * p.H + h) * D + d] : 0.f;
+    ss = fmaf(o[i], o[i], ss);
+  }
+  ss = wave_reduce_sum(ss);
+  const float inv = 1.f / sqrtf(ss / (float)D + p.eps);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int d = lane + 64 * i;
+    if (d < D) {
+      const int ch = h * D + d;
+      const float y = o[i] * inv * p.nw[ch] * sigm(ldx(p.g, (int64_t)t * p.ld + ch, p.f32));
+      const int64_t oi = (int64_t)t * p.ldo + ch;
+      if (p.f32) reinterpret_cast<float*>(p.out)[oi] = y;
+      else reinterpret_cast<bf16_t*>(p.out)[oi] = f2bf(y);
+    }
   }
 }
 
@@ -486,49 +690,86 @@ __global__ __launch_bounds__(256) void delta_chunk_finish_kernel(DeltaArgs p, in
 }
 
 int delta_channels(int D) { return D <= 32 ? 32 : (D <= 64 ? 64 : 128); }
-// Tokens a sequence may have in a step to be run one by one: 1.35 us each against about 75 us for the shortest portion in
-// chunks (us, 8 heads of 128: 8 x 16 tokens 33, the chunks 71; 8 x 64 127, the chunks 92). A step of at most 64 rows, which may
-// all be decoded tokens, takes one launch.
+// Few sequences, not all of them decoded tokens: the scan is ahead for portions of some 12 to 128 tokens (D <= 64: 20 to 96), 0.4 to
+// 0.5 us a token where all its workgroups run at once (their LDS allows 768 on the chip, 1536 for D <= 64). us, scan / short form / chunks, 8
+// heads of 128: one portion of 8 tokens 17, 16, 69; of 16 22, 27, 69; of 64 47, 91, 79; of 96 63, 134, 80; of 128 80, 176, 84; of 160 96, 219, 86;
+// 4 x 8 18, 17, 22; 4 x 64 49, 92, 82; 8 x 64 (more than run at once) 92, 92, 97. D = 64: 16 tokens 16, 16, 51; 64 34, 55, 51; 96 46, 81,
+// 52; 128 57, 107, 54. The host knows rows and sequences only. In a step of several sequences and more than 128 rows those of more
+// tokens take chunks, told apart on the device: three more launches, 6 us, so not once the sequences are so long on average that the scan
+// has little to give (4 x 64 tokens 56, without the scan 82; 3 + 253 111, 104, by the scan alone 148).
+constexpr int delta_scan_limit(int D) { return D > 64 ? 128 : 96; }
+bool takes_scan(int T, int S, int H, int D) {
+  const int64_t blocks = (int64_t)S * H * ((D + 7) / 8);
+  const int lim = delta_scan_limit(D);
+  return blocks <= (D > 64 ? 768 : (D > 32 ? 1536 : 4096)) && T >= std::max(D > 64 ? 12 : 24, 4 * S) &&
+         (T <= lim || (S > 1 && T <= (lim - 32) * S));
+}
+// Else, tokens a sequence may have in a step to be run one by one in the short form: 1.3 us each against about 75 us for the shortest
+// portion in chunks. A step of at most 64 rows, which may all be decoded tokens, takes one launch.
 int delta_limit(int T) { return T <= 64 ? T : 48; }
 // chunks of a step whose sequences longer than lim tokens have T between them: each has at most one that is not whole
 int delta_chunks(int T, int lim) { return T <= lim ? 0 : T / CN + T / (lim + 1); }
 
+// {w, a u, k, r}, u, the raw outputs; whole 16-B pieces
+size_t scan_floats(int T, int H, int D) { return ((size_t)T * H * D * 6 + 3) / 4 * 4; }
+
+void launch_scan(const DeltaArgs& a, int T, int lim, float* scratch, hipStream_t st) {
+  const int64_t n = (int64_t)T * a.H * a.D;
+  float4* vec = reinterpret_cast<float4*>(scratch);
+  float* un = scratch + 4 * n;
+  float* oraw = scratch + 5 * n;
+  hipLaunchKernelGGL(delta_prep_kernel, dim3(T, a.H), dim3(64), 0, st, a, lim, vec, un);
+  const dim3 grid(a.S, a.H, (a.D + 7) / 8);
+  if (a.D <= 32) hipLaunchKernelGGL(delta_scan_kernel<4>, grid, dim3(64), 0, st, a, lim, vec, un, oraw);
+  else if (a.D <= 64) hipLaunchKernelGGL(delta_scan_kernel<8>, grid, dim3(64), 0, st, a, lim, vec, un, oraw);
+  else hipLaunchKernelGGL(delta_scan_kernel<16>, grid, dim3(64), 0, st, a, lim, vec, un, oraw);
+  hipLaunchKernelGGL(delta_finish_kernel, dim3(T, a.H), dim3(64), 0, st, a, lim, oraw);
+}
+
 template <int DP, bool F32>
-void launch_delta(const DeltaArgs& a, int T, int lim, float* rec, hipStream_t st) {
+void launch_delta(const DeltaArgs& a, int T, const DeltaPlan& plan, float* scratch, hipStream_t st) {
   // T counts padding rows too, so a sequence may be much shorter. A lone one then takes chunks whatever its length (not more
   // of them than any step of T rows); several are told apart by their lengths on the device.
-  const bool lone = a.S == 1 && T > lim;
-  const int chunks = lone ? (T + CN - 1) / CN : delta_chunks(T, lim);
-  if (!lone) hipLaunchKernelGGL((delta_short_kernel<DP, F32>), dim3(a.S, a.H), dim3(256), 0, st, a, lim);
-  if (chunks == 0) return;
-  if (lone) lim = 0;
-  const dim3 grid(chunks, a.H), scan((a.H + 7) / 8 * 8, (a.D + 15) / 16, a.S);
+  const bool lone = a.S == 1 && plan.chunks > 0;
+  if (plan.scan) launch_scan(a, T, plan.lim, scratch, st);
+  else if (!lone) hipLaunchKernelGGL((delta_short_kernel<DP, F32>), dim3(a.S, a.H), dim3(256), 0, st, a, plan.lim);
+  if (plan.chunks == 0) return;
+  const int lim = lone ? 0 : plan.lim;
+  float* rec = scratch + (plan.scan ? scan_floats(T, a.H, a.D) : 0);
+  const dim3 grid(plan.chunks, a.H), scan((a.H + 7) / 8 * 8, (a.D + 15) / 16, a.S);
   hipLaunchKernelGGL((delta_chunk_kernel<DP, F32>), grid, dim3(256), 0, st, a, lim, rec);
   hipLaunchKernelGGL(delta_chunk_scan_kernel<DP / 16>, scan, dim3(256), 0, st, a, lim, rec);
   hipLaunchKernelGGL(delta_chunk_finish_kernel, grid, dim3(256), 0, st, a, lim, DP, rec);
 }
 
 template <int DP>
-void launch_delta_dp(const DeltaArgs& a, int T, int lim, float* rec, hipStream_t st) {
-  if (a.f32) launch_delta<DP, true>(a, T, lim, rec, st);
-  else launch_delta<DP, false>(a, T, lim, rec, st);
+void launch_delta_dp(const DeltaArgs& a, int T, const DeltaPlan& plan, float* scratch, hipStream_t st) {
+  if (a.f32) launch_delta<DP, true>(a, T, plan, scratch, st);
+  else launch_delta<DP, false>(a, T, plan, scratch, st);
 }
 
 }  // namespace
 
-size_t delta_rule_scratch_floats(int T, int H, int D) {
-  const size_t rows = (size_t)T * H * D * 6;
-  const size_t chunks = (size_t)delta_chunks(T, delta_limit(T)) * H * delta_chunk_floats(delta_channels(D), D);
-  return rows > chunks ? rows : chunks;
+DeltaPlan delta_rule_plan(int T, int S, int H, int D) {
+  const bool scan = takes_scan(T, S, H, D);
+  const int lim = scan ? (T <= 128 ? T : delta_scan_limit(D)) : delta_limit(T);
+  return {scan, lim, S == 1 && T > lim ? (T + CN - 1) / CN : delta_chunks(T, lim)};
 }
 
-// scratch: `floats` of them; fewer than delta_rule_scratch_floats(): no chunks, every sequence token by token
+size_t delta_rule_scratch_floats(int T, int S, int H, int D) {
+  const DeltaPlan plan = delta_rule_plan(T, S, H, D);
+  const size_t rows = scan_floats(T, H, D), chunks = (size_t)plan.chunks * H * delta_chunk_floats(delta_channels(D), D);
+  return plan.scan ? rows + chunks : std::max(rows, chunks);
+}
+
+// scratch: `floats` of them, 6 T H D at least; fewer than delta_rule_scratch_floats(): the scan in place of chunks
 void launch_delta_rule(const DeltaArgs& a, int T, float* scratch, size_t floats, hipStream_t st) {
   if (a.S <= 0 || a.H <= 0 || T <= 0) return;
-  const int lim = floats >= delta_rule_scratch_floats(T, a.H, a.D) ? delta_limit(T) : T;
-  if (a.D <= 32) launch_delta_dp<32>(a, T, lim, scratch, st);
-  else if (a.D <= 64) launch_delta_dp<64>(a, T, lim, scratch, st);
-  else launch_delta_dp<128>(a, T, lim, scratch, st);
+  DeltaPlan plan = delta_rule_plan(T, a.S, a.H, a.D);
+  if (plan.chunks > 0 && floats < delta_rule_scratch_floats(T, a.S, a.H, a.D)) plan = DeltaPlan{true, T, 0};
+  if (a.D <= 32) launch_delta_dp<32>(a, T, plan, scratch, st);
+  else if (a.D <= 64) launch_delta_dp<64>(a, T, plan, scratch, st);
+  else launch_delta_dp<128>(a, T, plan, scratch, st);
 }
 
 }  // namespace vgate

@@ -146,9 +146,16 @@ struct DeltaArgs {
   void* out = nullptr; int64_t ldo = 0;
   int S = 0, H = 0, D = 0, f32 = 0;
 };
-// floats of scratch a step of T rows can use
-size_t delta_rule_scratch_floats(int T, int H, int D);
-// T rows; scratch: `floats` of them, delta_rule_scratch_floats() for portions in chunks
+// What a step of T rows (with padding) and S sequences runs as: sequences of up to `lim` tokens token by token, in the scan or the short
+// form, and, if chunks > 0 (workgroups per head), longer ones in chunks (a lone sequence whatever its length)
+struct DeltaPlan {
+  bool scan;
+  int lim, chunks;
+};
+DeltaPlan delta_rule_plan(int T, int S, int H, int D);
+// floats of scratch such a step can use
+size_t delta_rule_scratch_floats(int T, int S, int H, int D);
+// T rows; scratch: `floats` of them, 6 T H D at least, delta_rule_scratch_floats() for portions in chunks
 void launch_delta_rule(const DeltaArgs& a, int T, float* scratch, size_t floats, hipStream_t st);
 
 // Sliding-window attention over paged key / value caches with optional pooled blocks (window_attn.hip).

@@ -264,7 +264,7 @@ void delta_rule(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor&
   p.query_start = i32p(query_start, "query_start", p.S + 1);  // values <= T: set by the step metadata
   p.out = out.data_ptr(); p.ldo = out.stride(0);
   TORCH_CHECK(scratch.is_cuda() && scratch.scalar_type() == torch::kFloat32 && scratch.is_contiguous() &&
-              scratch.numel() >= 6 * T * HD, "delta_rule: scratch fp32 with T * H * D * 6 elements");
+              scratch.numel() >= 6 * T * HD, "delta_rule: scratch fp32 with at least T * H * D * 6 elements (the token scan's)");
   TORCH_CHECK((reinterpret_cast<uintptr_t>(scratch.data_ptr()) & 15) == 0, "delta_rule: scratch must be 16-B aligned");
   c10::DeviceGuard guard(r.device());
   vgate::launch_delta_rule(p, (int)T, scratch.data_ptr<float>(), (size_t)scratch.numel(), cur_stream());
@@ -927,9 +927,14 @@ void bind_seq(pybind11::module& m) {
     return std::make_pair((int64_t)parts, (int64_t)vgate::latent_attn_part_floats((int)T, (int)S, (int)H, (int)rank, (int)rot, parts));
   }, "workgroups that share a decoded token's key tiles in latent_attn, and the fp32 scratch elements they need");
   m.def("delta_rule", &delta_rule, "generalized delta rule recurrence over state slots + head norm + gate");
-  m.def("delta_rule_scratch", [](int64_t T, int64_t H, int64_t D) {
-    return (int64_t)vgate::delta_rule_scratch_floats((int)T, (int)H, (int)D);
-  }, "floats of scratch delta_rule can use for a step of T tokens (with fewer it takes no chunks)");
+  m.def("delta_rule_scratch", [](int64_t T, int64_t H, int64_t D, int64_t S) {
+    return (int64_t)vgate::delta_rule_scratch_floats((int)T, (int)S, (int)H, (int)D);
+  }, "floats of scratch delta_rule can use for a step of T tokens and S sequences (with fewer it takes no chunks)", py::arg("T"),
+        py::arg("H"), py::arg("D"), py::arg("S") = 1);
+  m.def("delta_rule_plan", [](int64_t T, int64_t S, int64_t H, int64_t D) {
+    const auto p = vgate::delta_rule_plan((int)T, (int)S, (int)H, (int)D);
+    return std::make_tuple(p.scan, (int64_t)p.lim, (int64_t)p.chunks);
+  }, "(token scan, most tokens of a sequence that takes it or else the short form, chunks) of a delta_rule step of T rows and S sequences");
   m.def("cast_rows", &cast_rows, "fp32 rows rounded to bf16");
   m.def("glu_rows", &glu_rows, "out = act(gate) * up over a stacked [gate; up] projection", py::arg("gu"), py::arg("out"),
         py::arg("act"), py::arg("limit") = 0.0, py::arg("alpha") = 1.702);

@@ -53,3 +53,31 @@ def test_fewer_tokens_than_rows(lens, pos, pad):
     want, state_w = _run(3, 64, lens, pos, torch.float32, 11, "cpu", pad)
     assert float((state - state_w).norm() / state_w.norm()) < 2e-5   # (as above)
     assert float((out - want).norm() / want.norm()) < 2e-5
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,D", [(1, 1), (2, 5), (3, 33), (3, 64), (1, 100), (5, 128)])
+@pytest.mark.parametrize("lens,pos", [([9], [0]), ([16], [7]), ([92], [3]), ([125], [0]), ([1, 11], [5, 0]), ([17, 30, 1, 9], [0, 3, 40, 1]), ([96, 1, 95], [0, 2, 9]),
+                                      ([1, 129, 3], [4, 0, 9]), ([97, 96, 1], [0, 5, 2]), ([130, 128, 1, 20], [0, 1, 2, 3])])
+def test_token_scan(H, D, lens, pos, dt):
+    """Steps around the lines of the token scan, with staged tokens that fill their eight and do not, and with a longer portion in
+    chunks beside it."""
+    out, state = _run(H, D, lens, pos, dt, H + D, "cuda")
+    want, state_w = _run(H, D, lens, pos, dt, H + D, "cpu")
+    rel = lambda a, b: float((a - b).norm() / b.norm())  # noqa: E731
+    assert rel(state, state_w) < 2e-5   # (as above)
+    assert rel(out, want) < (2e-5 if dt == torch.float32 else 2.0 ** -8)
+
+
+def test_scratch_of_the_scan_alone():
+    """With no more scratch than the token scan's, a step that would take chunks takes the scan."""
+    from vgate import ops
+    lens, pos, H, D = [200], [4], 3, 64
+    t, slots, ctx, qs, out = _inputs(H, D, lens, pos, torch.float32, 1, "cuda")
+    scratch = torch.empty(6 * out.numel(), device="cuda")
+    assert scratch.numel() < ops.native().delta_rule_scratch(out.shape[0], H, D)
+    ops.native().delta_rule(t["r"], t["k"], t["v"], t["g"], t["a"], t["wl"], t["w0"], t["ab"], t["nw"], t["state"], slots, ctx, qs, out,
+                            0.6, 1e-6, 1e-6, scratch)
+    want, state_w = _run(H, D, lens, pos, torch.float32, 1, "cpu")
+    assert float((t["state"].cpu() - state_w).norm() / state_w.norm()) < 2e-5   # (as above)
+    assert float((out[:200].cpu() - want).norm() / want.norm()) < 2e-5

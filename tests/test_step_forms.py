@@ -1,0 +1,40 @@
+"""Which form a step of the recurrent mixers takes, by its rows (with padding) and sequences: host rules, no GPU."""
+import pytest
+
+from vgate import ops
+
+
+def _plan(name, *sizes):
+    return getattr(ops.native(), name)(*sizes)
+
+
+@pytest.mark.parametrize("T", [12, 16, 32, 64, 96, 128])
+def test_delta_rule_lone_middle_portions_take_the_scan(T):
+    assert _plan("delta_rule_plan", T, 1, 8, 128)[0]
+
+
+@pytest.mark.parametrize("T,S,H,D,scan,chunks", [(8, 1, 8, 128, False, False), (192, 1, 8, 128, False, True), (2048, 1, 8, 128, False, True),
+                                                 (128, 2, 8, 128, True, False), (256, 4, 8, 128, True, True), (448, 4, 8, 128, False, True),
+                                                 (64, 8, 8, 128, False, False), (64, 8, 4, 128, True, False), (512, 8, 4, 128, True, True),
+                                                 (96, 1, 8, 64, True, False), (128, 1, 8, 64, False, True), (64, 8, 16, 64, True, False),
+                                                 (64, 16, 16, 64, False, False)])
+def test_delta_rule_lines(T, S, H, D, scan, chunks):
+    one, _, n = _plan("delta_rule_plan", T, S, H, D)
+    assert one == scan and (n > 0) == chunks
+
+
+@pytest.mark.parametrize("name,args", [("delta_rule_plan", (8, 128))])
+def test_chunks_cover_every_way_to_share_the_rows(name, args):
+    """Whole chunks of C tokens and one that is not whole for each sequence of more than `lim` tokens."""
+    C = 32 if name == "delta_rule_plan" else 64
+    for T in (65, 97, 128, 129, 200, 513, 2048):
+        for S in (1, 2, 3, 7, 31, 100):
+            one, lim, chunks = _plan(name, T, S, *args)
+            if T <= lim or (name == "linear_attn_plan" and not one):
+                continue
+            for n in range(1, min(S, T // (lim + 1)) + 1):     # n equal portions, the last one takes the rest
+                lens = [max(lim + 1, T // n // C * C + 1)] * (n - 1)
+                if sum(lens) >= T:
+                    lens = [lim + 1] * (n - 1)
+                lens.append(T - sum(lens))
+                assert sum(-(-m // C) for m in lens if m > lim) <= chunks, (T, S, lens)

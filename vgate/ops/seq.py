@@ -302,7 +302,7 @@ def delta_rule(r, k, v, g, a, wl, w0, ab, nw, state, state_slots, context_lens, 
                decay_c: float, unit_eps: float, eps: float, num_seqs: int | None = None) -> None:
     """Generalized delta rule over state slots (see csrc/kernels/delta_rule.hip); state [slots, H, D, D]."""
     if r.is_cuda:
-        n = _C().delta_rule_scratch(r.shape[0], state.shape[1], state.shape[2])
+        n = _C().delta_rule_scratch(r.shape[0], state.shape[1], state.shape[2], state_slots.numel())
         scratch = torch.empty(n, dtype=torch.float32, device=r.device)
         _C().delta_rule(r, k, v, g, a, wl, w0, ab, nw, state, state_slots, context_lens, query_start, out,
                         decay_c, unit_eps, eps, scratch)
