@@ -705,8 +705,9 @@ bool takes_scan(int T, int S, int H, int D) {
          (T <= lim || (S > 1 && T <= (lim - 32) * S));
 }
 // Else, tokens a sequence may have in a step to be run one by one in the short form: 1.3 us each against about 75 us for the shortest
-// portion in chunks. A step of at most 64 rows, which may all be decoded tokens, takes one launch.
-int delta_limit(int T) { return T <= 64 ? T : 48; }
+// portion in chunks. Decoding steps (T <= S) and others of at most 64 rows, which may be too, take one launch (8 heads of 128, with the
+// chunks' three empty ones: 128 sequences 35 us, 45; 256 65, 82).
+int delta_limit(int T, int S) { return T <= S || T <= 64 ? T : 48; }
 // chunks of a step whose sequences longer than lim tokens have T between them: each has at most one that is not whole
 int delta_chunks(int T, int lim) { return T <= lim ? 0 : T / CN + T / (lim + 1); }
 
@@ -752,7 +753,7 @@ void launch_delta_dp(const DeltaArgs& a, int T, const DeltaPlan& plan, float* sc
 
 DeltaPlan delta_rule_plan(int T, int S, int H, int D) {
   const bool scan = takes_scan(T, S, H, D);
-  const int lim = scan ? (T <= 128 ? T : delta_scan_limit(D)) : delta_limit(T);
+  const int lim = scan ? (T <= 128 ? T : delta_scan_limit(D)) : delta_limit(T, S);
   return {scan, lim, S == 1 && T > lim ? (T + CN - 1) / CN : delta_chunks(T, lim)};
 }
 

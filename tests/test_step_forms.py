@@ -23,6 +23,12 @@ def test_delta_rule_lines(T, S, H, D, scan, chunks):
     assert one == scan and (n > 0) == chunks
 
 
+@pytest.mark.parametrize("T,S", [(1, 1), (64, 64), (96, 128), (128, 128), (256, 256), (512, 512)])
+def test_decoding_steps_take_one_launch(T, S):
+    scan, lim, chunks = _plan("delta_rule_plan", T, S, 8, 128)
+    assert not scan and lim >= T and chunks == 0
+
+
 @pytest.mark.parametrize("name,args", [("delta_rule_plan", (8, 128))])
 def test_chunks_cover_every_way_to_share_the_rows(name, args):
     """Whole chunks of C tokens and one that is not whole for each sequence of more than `lim` tokens."""
