@@ -37,6 +37,8 @@
 //          of factors <= 1 taken in order. local: the second sum, fp32 MFMA (16x16x4); carry as above; output: the
 //          triangle of weighted products (a lane holds k_j g of four D / 32 channels and walks i), then both products
 //          with fp32 MFMA, norm and gate. 2048 tokens, 8 heads of 128: 100 us, by the scan in chunks 162.
+#include <algorithm>
+
 #include "chunks.h"
 #include "seq_launchers.h"
 
@@ -856,29 +858,24 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
     }
 }
 
-// Tokens a sequence may have in a step to be run one by one: a chunk of 64 costs what 50 tokens do, and its three launches more.
-int short_limit(int T) { return T <= 96 ? T : 64; }
+// Tokens a sequence may have in a step to be run one by one: a chunk of 64 costs what 50 tokens do, and its three launches more. Decoding
+// steps (T <= S), and short ones that may nearly be, take one launch (8 heads of 128, in parentheses with empty or few chunks: 128
+// sequences 32 us (53), 256 61 (98); 63 decoded tokens beside a portion of 65 95 (146), 127 beside 65 103 (169), beside 129 183 (170)).
+int short_limit(int T, int S) { return T <= std::max(S, 96) || T <= std::min(2 * S, 256) ? T : 64; }
 // chunks of a step whose sequences longer than lim tokens have T between them: each has at most one that is not whole
 int long_chunks(int T, int lim) { return T <= lim ? 0 : T / CT + T / (lim + 1); }
 // Decoding steps: one launch instead of three (16 sequences x 8 heads of 128: 25.3 -> 12.2 us). Long steps: chunks with fp32 MFMA
 // (2048 tokens 162 -> 100 us, 63 decoded tokens beside a portion of 961 1054 -> 169, 64 portions of 16 62 -> 47). Between them
 // the scan below, which spreads a head's columns over several workgroups, is ahead where sequences are few: one portion of
 // 96 78 us (here 96; of 128 98 against 84), 8 of 48 54 (59).
-bool takes_small(int T, int S, int D, int V, int cols_per_lane) {
-  return D <= 128 && V <= 128 && cols_per_lane == 0 &&
+bool takes_small(int T, int S, int D, int V) {
+  return D <= 128 && V <= 128 &&
          (T <= 2 * S || T >= (S == 1 ? 128 : (S < 16 ? 512 : 256)));
 }
 
 template <int DP, bool F32, bool PRE>
-void launch_small(const LinearAttnArgs& a, int T, float* oraw, float* cstate, float* cdecay, hipStream_t st) {
-  // T counts padding rows too, so a sequence may be much shorter. A lone one then takes chunks whatever its length (not more
-  // of them than any step of T rows); several are told apart by their lengths on the device.
-  const int P = max(a.D, a.V);
-  int lim = short_limit(T), chunks = long_chunks(T, lim);
-  if (a.S == 1 && T > lim) {
-    lim = 0;
-    chunks = (T + CT - 1) / CT;
-  }
+void launch_small(const LinearAttnArgs& a, int T, const LinearPlan& plan, float* oraw, float* cstate, float* cdecay, hipStream_t st) {
+  const int P = max(a.D, a.V), lim = plan.lim, chunks = plan.chunks;
   if (lim > 0) {
     const dim3 grid(a.S, a.H);
     if (P <= 32) hipLaunchKernelGGL((linear_short_kernel<32, F32, PRE>), grid, dim3(256), 0, st, a, lim, oraw);
@@ -899,13 +896,13 @@ void launch_small(const LinearAttnArgs& a, int T, float* oraw, float* cstate, fl
 }
 
 template <int DP>
-void launch_small_dp(const LinearAttnArgs& a, int T, float* oraw, float* cstate, float* cdecay, hipStream_t st) {
+void launch_small_dp(const LinearAttnArgs& a, int T, const LinearPlan& plan, float* oraw, float* cstate, float* cdecay, hipStream_t st) {
   if (a.f32) {
-    if (a.bonus != nullptr) launch_small<DP, true, true>(a, T, oraw, cstate, cdecay, st);
-    else launch_small<DP, true, false>(a, T, oraw, cstate, cdecay, st);
+    if (a.bonus != nullptr) launch_small<DP, true, true>(a, T, plan, oraw, cstate, cdecay, st);
+    else launch_small<DP, true, false>(a, T, plan, oraw, cstate, cdecay, st);
   } else {
-    if (a.bonus != nullptr) launch_small<DP, false, true>(a, T, oraw, cstate, cdecay, st);
-    else launch_small<DP, false, false>(a, T, oraw, cstate, cdecay, st);
+    if (a.bonus != nullptr) launch_small<DP, false, true>(a, T, plan, oraw, cstate, cdecay, st);
+    else launch_small<DP, false, false>(a, T, plan, oraw, cstate, cdecay, st);
   }
 }
 
@@ -916,11 +913,19 @@ int linear_attn_chunk_size(int T, int S) {
   return T >= 256 && T >= 64 * S ? 64 : 0;
 }
 int linear_attn_chunks(int T, int S, int CH) { return CH > 0 ? T / CH + S : 0; }
+LinearPlan linear_attn_plan(int T, int S, int D, int V) {
+  const int lim = short_limit(T, S);
+  // T counts padding rows too, so a sequence may be much shorter. A lone one then takes chunks whatever its length (not more
+  // of them than any step of T rows); several are told apart by their lengths on the device.
+  const bool lone = S == 1 && T > lim;
+  return {takes_small(T, S, D, V), lone ? 0 : lim, lone ? (T + CT - 1) / CT : long_chunks(T, lim)};
+}
 size_t linear_attn_scratch_floats(int T, int S, int H, int D, int V) {
   const int CH = linear_attn_chunk_size(T, S);
   const size_t any = (size_t)T * H * (4 * D + 2 * V) + (size_t)linear_attn_chunks(T, S, CH) * H * D * (V + 1);
-  const size_t small = (size_t)T * H * V + (size_t)long_chunks(T, short_limit(T)) * H * D * (V + 1);
-  return takes_small(T, S, D, V, 0) && small > any ? small : any;
+  const LinearPlan plan = linear_attn_plan(T, S, D, V);
+  const size_t small = (size_t)T * H * V + (size_t)plan.chunks * H * D * (V + 1);
+  return plan.small && small > any ? small : any;
 }
 
 // scratch: linear_attn_scratch_floats(): {a, k, q, -} per key channel, the values, the raw outputs, and for
@@ -928,12 +933,13 @@ size_t linear_attn_scratch_floats(int T, int S, int H, int D, int V) {
 void launch_linear_attn(const LinearAttnArgs& a, int T, float* scratch, hipStream_t st) {
   if (a.S <= 0 || a.H <= 0 || T <= 0) return;
   const int64_t nk = (int64_t)T * a.H * a.D, nv = (int64_t)T * a.H * a.V;
-  if (takes_small(T, a.S, a.D, a.V, a.cols_per_lane)) {   // scratch: raw outputs, the chunks' states, their decays
+  const LinearPlan plan = linear_attn_plan(T, a.S, a.D, a.V);
+  if (plan.small && a.cols_per_lane == 0) {   // scratch: raw outputs, the chunks' states, their decays
     float* states = scratch + nv;
-    float* decays = states + (size_t)long_chunks(T, short_limit(T)) * a.H * a.D * a.V;
-    if (a.D <= 32) launch_small_dp<32>(a, T, scratch, states, decays, st);
-    else if (a.D <= 64) launch_small_dp<64>(a, T, scratch, states, decays, st);
-    else launch_small_dp<128>(a, T, scratch, states, decays, st);
+    float* decays = states + (size_t)plan.chunks * a.H * a.D * a.V;
+    if (a.D <= 32) launch_small_dp<32>(a, T, plan, scratch, states, decays, st);
+    else if (a.D <= 64) launch_small_dp<64>(a, T, plan, scratch, states, decays, st);
+    else launch_small_dp<128>(a, T, plan, scratch, states, decays, st);
     return;
   }
   float4* vec = reinterpret_cast<float4*>(scratch);

@@ -240,6 +240,13 @@ struct LinearAttnArgs {
 // chunks such a step has at most, and the scratch floats it needs
 int linear_attn_chunk_size(int T, int S);
 int linear_attn_chunks(int T, int S, int CH);
+// What a step of T rows (with padding) and S sequences runs as with key and value sizes up to 128: small: sequences of up to `lim` tokens
+// in the short form and, if chunks > 0 (workgroups per head), longer ones in chunks; else the scan
+struct LinearPlan {
+  bool small;
+  int lim, chunks;
+};
+LinearPlan linear_attn_plan(int T, int S, int D, int V);
 size_t linear_attn_scratch_floats(int T, int S, int H, int D, int V);
 // T rows; scratch: linear_attn_scratch_floats() floats, 16-B aligned
 void launch_linear_attn(const LinearAttnArgs& a, int T, float* scratch, hipStream_t st);

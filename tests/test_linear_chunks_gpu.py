@@ -67,3 +67,13 @@ def test_fewer_tokens_than_rows(lens, pos, pad, variant):
     want, state_w = _run(3, 64, 48, lens, pos, torch.float32, variant, 11, "cpu", pad)
     assert float((state - state_w).norm() / state_w.norm()) < 5e-5   # (as above)
     assert float((out - want).norm() / want.norm()) < 5e-5
+
+
+@pytest.mark.parametrize("variant", ["bonus", "constant"])
+@pytest.mark.parametrize("lens,pad", [([1] * 97, 31), ([1] * 128, 0), ([1] * 200, 56), ([1] * 63 + [65], 0), ([1] * 127 + [129], 0), ([1] * 255 + [258], 0)])
+def test_many_decoded_tokens(lens, pad, variant):
+    pos = [3] * len(lens)   # (none at position 0, where a token's output is one product whose rounding the norm can blow up)
+    out, state = _run(2, 64, 48, lens, pos, torch.float32, variant, 7, "cuda", pad)
+    want, state_w = _run(2, 64, 48, lens, pos, torch.float32, variant, 7, "cpu", pad)
+    assert float((state - state_w).norm() / state_w.norm()) < 5e-5   # (as above)
+    assert float((out - want).norm() / want.norm()) < 5e-5
