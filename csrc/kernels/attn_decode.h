@@ -196,16 +196,17 @@ __device__ __forceinline__ bool qa_get8(const QaSync& q, uint32_t pair, uint32_t
   return x.y == tag && x.w == tag && y.y == tag && y.w == tag;
 }
 
-// Tokens of a partition and their number. Where the launch's partitions fit the chip at once, a context longer than part_size goes in
-// equal parts (whole chunks of 32), not in whole ones and a rest: the longest part is what the launch waits for (64 contexts of
-// about 600 tokens, 2 KV heads: 15.8 -> 13.5 us). With more of them whole parts keep the waves evenly loaded (128 such, 8 KV heads:
-// 67.6, equal parts 71.7).
+// Tokens of a partition and their number. Where so many partitions of every sequence and head come to one workgroup per CU at most, a
+// context longer than part_size goes in equal parts (whole chunks of 32), not in whole ones and a rest: the longest part is what the
+// launch waits for (us, whole / equal: 64 contexts of about 600 tokens, 2 KV heads 15.8, 13.7, one such 13.4, 10.8). With more of them
+// whole parts share the CUs better (64 of about 900, three or four parts each, 21.9, 25.1; 32 of 900, 8 KV heads 31.6, 35.3). The context
+// decides, not the room for longer ones (a.num_parts): the same sums whatever the longest context that a model is set up for.
 __device__ __forceinline__ void partition(const AttnArgs& a, int ctx, int& len, int& nparts) {
   len = a.part_size;
   nparts = 1;
   if (ctx <= a.part_size) return;
   nparts = (ctx + a.part_size - 1) / a.part_size;
-  if (a.S * a.num_parts * a.Hkv > 1024) return;
+  if (a.S * nparts * a.Hkv > 256) return;
   len = ((ctx + nparts - 1) / nparts + CHUNK - 1) / CHUNK * CHUNK;
   nparts = (ctx + len - 1) / len;
 }
@@ -231,6 +232,7 @@ __device__ __forceinline__ void decode_block(const AttnArgs& a, int s, int h, in
   int plen = a.part_size, nparts = 1, pstart = 0;
   if (part > 0) {  // (only a later partition waits for the context length before it asks for its pages)
     partition(a, ctx, plen, nparts);
+    if (part >= nparts) return;  // (block-uniform; room for longer contexts: 128 of 600 tokens in a table for 8192 95 -> 87 us)
     pstart = part * plen;
   }
   const int btv = bt[min(pstart / BS_ + lane, a.max_blocks - 1)];

@@ -65,3 +65,26 @@ def test_equal_and_whole_partitions(S, part):
     want = torch.matmul(sc.softmax(-1), v.permute(0, 2, 1, 3).contiguous()).reshape(S, Hq * D)
     for out in outs:   # weights rounded to bf16 (2^-9 each, of values of size ~ 1 that average out) and a bf16 result
         assert float((out - want).norm() / want.norm()) < 2.0 ** -7
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,ctx", [(64, 32, 8, 600), (64, 12, 2, 1300), (16, 32, 8, 600), (64, 12, 2, 600), (300, 12, 2, 600)])
+def test_partitions_do_not_depend_on_the_room_for_longer_contexts(S, Hq, Hkv, ctx):
+    """The same contexts with block tables (and partial results) for 1, 4 and 16 times as many tokens: the same bits."""
+    D, part, dev = 128, 512, "cuda"
+    g = torch.Generator(dev).manual_seed(S)
+    rand = lambda *s: torch.randn(*s, device=dev, generator=g).bfloat16()  # noqa: E731
+    used = -(-ctx // 16)
+    kc, vc = rand(256, Hkv, 16, D), rand(256, Hkv, 16, D)
+    pages = torch.randint(0, 256, (S, used), device=dev, generator=g).int()
+    cl = torch.tensor([ctx - i % 7 for i in range(S)], dtype=torch.int32, device=dev)
+    q, qs, none = rand(S, Hq * D), torch.arange(S + 1, device=dev).int(), torch.empty(0, dtype=torch.int32, device=dev)
+    outs = []
+    for room in (1, 4, 16):
+        bt = torch.zeros(S, used * room, dtype=torch.int32, device=dev)
+        bt[:, :used] = pages
+        P = -(-used * room * 16 // part)
+        po, pml = torch.zeros(S, Hq, P, D, device=dev), torch.zeros(S, Hq, P, 2, device=dev)
+        out = torch.zeros(S, Hq * D, device=dev).bfloat16()
+        ops.attention(q, Hq * D, kc, vc, bt, cl, qs, none, none, out, po, pml, Hq, Hkv, part, D ** -0.5)
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
