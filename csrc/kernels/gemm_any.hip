@@ -270,11 +270,12 @@ __global__ __launch_bounds__(256) void gemm_any_mfma_kernel(AnyGemmArgs p) {
 }
 
 // Few rows. Host-checked as AL above. A workgroup owns 16 columns (of both matrices), its four waves take pairs of k-steps (64
-// elements: whole 128-B lines of a weight row) in turn, UB of them in flight at once, and meet in LDS; wave i finishes the i-th
-// 16 rows. A tile's 64 rows go in passes of 32. What bounds it is one trip to memory for the weights, 4 to 6 us a launch; 8 experts
-// of 1024 x 2048 pairs (67 MB, 64 rows): 15 us, as tiles 18.
+// elements: whole 128-B lines of a weight row) in turn and meet in LDS; wave i finishes the i-th 16 rows. A tile's 64 rows go in passes of
+// 32. What bounds it is one trip to memory for the weights, 4 to 6 us a launch. UB pairs in flight per wave: one, and eight waves per SIMD
+// (with four the registers leave three, and K below 1024 is read in vain: 2048 x 512 with 8 rows each of 8 experts 7.3 us, 12.4); more for
+// up to 8 rows and long K, which are one chain of loads (a row of 2048 x 4096 11.9 -> 9.5 us).
 template <int DUAL, int UB>
-__global__ __launch_bounds__(256, 2) void gemm_any_rows_kernel(AnyGemmArgs p) {
+__global__ __launch_bounds__(256) void gemm_any_rows_kernel(AnyGemmArgs p) {
   constexpr int NM = 1 + DUAL;
   __shared__ f32x4 red[4][2 * NM][64];
   int grp, r0, rend;
@@ -639,20 +640,24 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st) {
     auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     const bool al = g.K >= 8 && g.K % 8 == 0 && g.lda % 8 == 0 && g.ldw % 8 == 0 && g.a_bs % 8 == 0 &&
                     g.w_bs % 8 == 0 && a16(g.a) && a16(g.w) && (!dual || a16(g.w2));
-    // Few rows, or few 64 x 64 tiles, leave the chip idle behind chains of loads: 16 columns and a quarter of K per wave there. (us,
-    // the tiles' kernels -> now) 64 x 1024 at 32 rows 12.4 -> 6.3, 1024 x 1024 at 512 28.7 -> 16.4, 8 experts of 1024 x 2048 with 8 rows
-    // each 15.6 -> 10.9, with 32 46 -> 16.6. Above the lines the wider tiles read the operands less often: 8192 x 1024 at 128 rows
-    // (256 tiles) 20 against 28, 256 x 512 at 2048 (128 tiles) 12.4 against 16.5, 32 experts with 2 rows each (816 tiles) 20 against 25.
+    // Few rows, or few 64 x 64 tiles, leave the chip idle behind chains of loads: 16 columns and a quarter of K per wave there. us, the
+    // tiles' kernels / this form: 64 x 1024 at 32 rows 12.4, 6.1; 128 x 512 of 12 products at 64 rows 12.4, 6.9, at 192 (72 tiles) 12.5, 8.3, at
+    // 384 (144) 12.7, 15; 256 x 1024 at 2048 (128) 19.7, 16.0. Of wide products below 1024 rows, which run as 64 x 128 tiles, up to
+    // 256: 2048 x 1024 at 384 rows (192) 29.7, 20.6, at 512 (256) 29.8, 25.6; from 1024 rows the LDS tiles are ahead of that. Experts: 8 of
+    // 1024 x 2048 pairs with 32 rows each 45, 27; above the line 32 of 1536 x 1024 with 8 (864 tiles) 22, 25.
+    const bool low = g.N >= 512 && g.M >= 256 && g.M < 1024;
     const int64_t tiles = (int64_t)grid.x * mt * g.batch;
-    if (al && (g.group_off ? g.M <= 512 && tiles < 768 : g.M <= 64 || tiles <= (g.M <= 512 ? 192 : 64))) {
+    if (al && (g.group_off ? g.M <= 512 && tiles < 768 : g.M <= 64 || tiles <= (low ? 256 : 128))) {
       const dim3 gr((g.N + 15) / 16, mt, g.batch);
-      auto kern = g.K > 256 ? (dual ? gemm_any_rows_kernel<1, 2> : gemm_any_rows_kernel<0, 4>)
-                            : (dual ? gemm_any_rows_kernel<1, 1> : gemm_any_rows_kernel<0, 1>);
+      const bool deep = g.M <= 8 && g.K > 512;
+      auto kern = dual ? (deep ? gemm_any_rows_kernel<1, 2> : gemm_any_rows_kernel<1, 1>)
+                       : (deep ? gemm_any_rows_kernel<0, 4> : gemm_any_rows_kernel<0, 1>);
       hipLaunchKernelGGL(kern, gr, block, 0, st, g);
       return;
     }
-    // enough 64 x 128 tiles to fill the chip (experts with few rows each: tiles whose waves split K)
-    const bool wide = al && g.N >= 512 && g.M >= 256 && (!g.group_off || g.M > 32 * g.groups);
+    // enough 64 x 128 tiles to fill the chip; experts with few rows each take tiles whose waves split K (32 of 512 x 512 with 24 rows
+    // each 12.5 us, as wide tiles 19.1) until the LDS tiles come in (64 of 1024 x 1024 with 16 each 31.6 us, as LDS tiles 27.1)
+    const bool wide = al && g.N >= 512 && g.M >= 256 && (!g.group_off || g.M > (g.M >= 1024 ? 15 : 32) * g.groups);
     const dim3 gridw((g.N + 127) / 128, mt, g.batch);
     // enough 128-row tiles; also where whole 128-column tiles of many products fill half the chip (us at 2048 rows: 12 of
     // 128 x 512 27.9 -> 15.8, 8 of 256 x 128 14.1 -> 7.3, 2 of 128 x 256 stay at 9; with a gate per output the small tiles are ahead)

@@ -68,3 +68,27 @@ def test_many_products_of_many_rows(M, N, K):
     out = torch.full((M, B, N), float("nan"), device="cuda", dtype=torch.bfloat16).transpose(0, 1)
     seq.gemm(a, w, out)
     _close(out, torch.matmul(a.float(), w.float().transpose(1, 2)), K)
+
+
+@pytest.mark.parametrize("M", [8, 9, 128, 129, 256, 513, 1023, 1024])
+@pytest.mark.parametrize("N,K", [(512, 520), (512, 1032), (2048, 264), (64, 40)])
+def test_lines_between_the_forms(M, N, K):
+    g = torch.Generator("cuda").manual_seed(M * N + K)
+    a, w = torch.randn(M, K, device="cuda", generator=g).bfloat16(), (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).bfloat16()
+    out = torch.full((M, N), float("nan"), device="cuda", dtype=torch.bfloat16)
+    seq.gemm(a, w, out)
+    _close(out, a.float() @ w.float().t(), K)
+
+
+@pytest.mark.parametrize("sizes", [[8, 0], [9, 0], [16] * 63 + [15], [16] * 64, [24] * 32, [33] * 32, [65, 3] * 15])
+@pytest.mark.parametrize("N,K", [(512, 72), (1024, 520)])
+def test_experts_on_the_lines(N, K, sizes):
+    E, M = len(sizes), sum(sizes)
+    g = torch.Generator("cuda").manual_seed(M + N)
+    x, w = torch.randn(M, K, device="cuda", generator=g).bfloat16(), (torch.randn(E, N, K, device="cuda", generator=g) * K ** -0.5).bfloat16()
+    off = torch.tensor([sum(sizes[:i]) for i in range(E + 1)], dtype=torch.int32, device="cuda")
+    out = torch.full((M, N), float("nan"), device="cuda", dtype=torch.bfloat16)
+    seq.gemm(x, w, out, group_off=off)
+    for e in range(E):
+        a, b = int(off[e]), int(off[e + 1])
+        _close(out[a:b], x[a:b].float() @ w[e].float().t(), K)
