@@ -376,10 +376,12 @@ __global__ __launch_bounds__(256) void gemm_any_rows_kernel(AnyGemmArgs p) {
 // same columns of W2, so a lane holds gate and up of one output); wave (wm, wn) owns rows 64 wm .. and 4 x 4 MFMA
 // tiles. A k-step's 128 x 32 A and weight tiles are two 16-B pieces per thread each; rows past the group's end
 // read the tile's first row and columns past N the last one (both dropped at the store), k past K reads a
-// clamped address and zeroes the A piece. What bounds it is a k-step's way from memory, so two of them are under way (us, one ->
-// two: 8 experts at 4096 rows, pairs of 1024 x 2048 61 -> 56, 2048 x 1024 41 -> 33; 2048 rows of 1024 x 1024 21.6 -> 16.6).
+// clamped address and zeroes the A piece. What bounds it is a k-step's way from memory, so two of them are under way (AHEAD; us in an
+// engine step, one -> two: 8 experts at 4096 rows, pairs of 1024 x 2048 69.8 -> 64.3, 2048 x 1024 53.7 -> 47.8; 2048 rows of 1024 x 1024
+// 20.4 -> 20.0, warm 21.8 -> 16.6). Where K is short and workgroups are many, the registers of the second step are better spent on a fourth
+// workgroup per CU: 12 products of 512 x 128 at 2048 rows 14.2 -> 13.6, 16 19.0 -> 16.8 (two workgroups per CU: 10.2 -> 10.6).
 constexpr int LM = 128, LKS = 32, LPAD = LKS + 8;
-template <int DUAL>
+template <int DUAL, int AHEAD>
 __global__ __launch_bounds__(256, 3) void gemm_any_lds_kernel(AnyGemmArgs p) {
   constexpr int WN = DUAL ? 64 : 128;  // columns of each weight matrix per block
   constexpr int OPAD = WN + 8;         // padded row of the staged outputs
@@ -435,10 +437,7 @@ __global__ __launch_bounds__(256, 3) void gemm_any_lds_kernel(AnyGemmArgs p) {
       *reinterpret_cast<uint4*>(&Ws[buf][row][kq]) = x.w[u];
     }
   };
-  // k-step k0 from LDS; x: what was asked for step k0 + LKS, two steps ago, goes to the other buffer, then asks for the step
-  // after the next. A buffer is rewritten one step later, after the barrier that every wave reaches only when it has read it
-  // (the barriers wait for LDS traffic only).
-  auto step = [&](Step& x, int buf, int k0) {
+  auto compute = [&](int buf) {
     bf16x8 af[4], wf[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) af[i] = as_bf16x8(*reinterpret_cast<const uint4*>(&As[buf][wm * 64 + i * 16 + lr][8 * lg]));
@@ -451,22 +450,44 @@ __global__ __launch_bounds__(256, 3) void gemm_any_lds_kernel(AnyGemmArgs p) {
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[i][j] = mfma16(af[i], wf[j], acc[i][j]);
-    stage(x, buf ^ 1, k0 + LKS);
-    fetch(x, k0 + 3 * LKS);
-    lds_barrier();
   };
-  Step xa, xb;
+  // A buffer is rewritten one step later, after the barrier that every wave reaches only when it has read it (the barriers wait for
+  // LDS traffic only).
+  Step xa;
   fetch(xa, 0);
-  fetch(xb, LKS);
-  stage(xa, 0, 0);
-  fetch(xa, 2 * LKS);
-  lds_barrier();
-  int k0 = 0;
-  for (; k0 + LKS < K; k0 += 2 * LKS) {
-    step(xb, 0, k0);
-    step(xa, 1, k0 + LKS);
+  if constexpr (AHEAD == 2) {
+    // k-step k0 from LDS; x: what was asked for step k0 + LKS, two steps ago, goes to the other buffer, then asks for the step
+    // after the next
+    auto step = [&](Step& x, int buf, int k0) {
+      compute(buf);
+      stage(x, buf ^ 1, k0 + LKS);
+      fetch(x, k0 + 3 * LKS);
+      lds_barrier();
+    };
+    Step xb;
+    fetch(xb, LKS);
+    stage(xa, 0, 0);
+    fetch(xa, 2 * LKS);
+    lds_barrier();
+    int k0 = 0;
+    for (; k0 + LKS < K; k0 += 2 * LKS) {
+      step(xb, 0, k0);
+      step(xa, 1, k0 + LKS);
+    }
+    if (k0 < K) step(xb, 0, k0);
+  } else {
+    stage(xa, 0, 0);
+    __syncthreads();
+    int buf = 0;
+    for (int k0 = 0; k0 < K; k0 += LKS) {
+      const bool more = k0 + LKS < K;
+      if (more) fetch(xa, k0 + LKS);
+      compute(buf);
+      if (more) stage(xa, buf ^ 1, k0 + LKS);
+      __syncthreads();
+      buf ^= 1;
+    }
   }
-  if (k0 < K) step(xb, 0, k0);
   if (p.vec_out) {  // bf16 rows of whole 16-B pieces: staged in LDS (the k loop's last barrier has freed it), then stored whole
     with_act<DUAL>(p, [&](auto act) {
 #pragma unroll
@@ -642,12 +663,12 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st) {
                     g.w_bs % 8 == 0 && a16(g.a) && a16(g.w) && (!dual || a16(g.w2));
     // Few rows, or few 64 x 64 tiles, leave the chip idle behind chains of loads: 16 columns and a quarter of K per wave there. us, the
     // tiles' kernels / this form: 64 x 1024 at 32 rows 12.4, 6.1; 128 x 512 of 12 products at 64 rows 12.4, 6.9, at 192 (72 tiles) 12.5, 8.3, at
-    // 384 (144) 12.7, 15; 256 x 1024 at 2048 (128) 19.7, 16.0. Of wide products below 1024 rows, which run as 64 x 128 tiles, up to
+    // 384 (144) 12.7, 15; 256 x 1024 at 2048 (128) 19.7, 16.0. Of broad products below 1024 rows, which run as 64 x 128 tiles, up to
     // 256: 2048 x 1024 at 384 rows (192) 29.7, 20.6, at 512 (256) 29.8, 25.6; from 1024 rows the LDS tiles are ahead of that. Experts: 8 of
     // 1024 x 2048 pairs with 32 rows each 45, 27; above the line 32 of 1536 x 1024 with 8 (864 tiles) 22, 25.
-    const bool low = g.N >= 512 && g.M >= 256 && g.M < 1024;
+    const bool broad = g.N >= 512 && g.M >= 256;
     const int64_t tiles = (int64_t)grid.x * mt * g.batch;
-    if (al && (g.group_off ? g.M <= 512 && tiles < 768 : g.M <= 64 || tiles <= (low ? 256 : 128))) {
+    if (al && (g.group_off ? g.M <= 512 && tiles < 768 : g.M <= 64 || tiles <= (!broad ? 128 : (g.M < 1024 ? 256 : 64)))) {
       const dim3 gr((g.N + 15) / 16, mt, g.batch);
       const bool deep = g.M <= 8 && g.K > 512;
       auto kern = dual ? (deep ? gemm_any_rows_kernel<1, 2> : gemm_any_rows_kernel<1, 1>)
@@ -657,7 +678,7 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st) {
     }
     // enough 64 x 128 tiles to fill the chip; experts with few rows each take tiles whose waves split K (32 of 512 x 512 with 24 rows
     // each 12.5 us, as wide tiles 19.1) until the LDS tiles come in (64 of 1024 x 1024 with 16 each 31.6 us, as LDS tiles 27.1)
-    const bool wide = al && g.N >= 512 && g.M >= 256 && (!g.group_off || g.M > (g.M >= 1024 ? 15 : 32) * g.groups);
+    const bool wide = al && broad && (!g.group_off || g.M > (g.M >= 1024 ? 15 : 32) * g.groups);
     const dim3 gridw((g.N + 127) / 128, mt, g.batch);
     // enough 128-row tiles; also where whole 128-column tiles of many products fill half the chip (us at 2048 rows: 12 of
     // 128 x 512 27.9 -> 15.8, 8 of 256 x 128 14.1 -> 7.3, 2 of 128 x 256 stay at 9; with a gate per output the small tiles are ahead)
@@ -666,8 +687,10 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st) {
     if ((wide || heads) && g.M >= 1024 && lds_tiles()) {
       AnyGemmArgs v = g;
       v.vec_out = !g.out_f32 && g.gate == nullptr && g.N % 8 == 0 && g.ldo % 8 == 0 && g.o_bs % 8 == 0 && a16(g.out);
-      if (dual) hipLaunchKernelGGL((gemm_any_lds_kernel<1>), dim3((g.N + 63) / 64, mt128, g.batch), block, 0, st, v);
-      else hipLaunchKernelGGL((gemm_any_lds_kernel<0>), dim3((g.N + 127) / 128, mt128, g.batch), block, 0, st, v);
+      const dim3 grid2((g.N + (dual ? 63 : 127)) / (dual ? 64 : 128), mt128, g.batch);
+      const bool one = !dual && g.K <= 256 && (int64_t)grid2.x * grid2.y * grid2.z > 512;
+      auto kern = dual ? gemm_any_lds_kernel<1, 2> : (one ? gemm_any_lds_kernel<0, 1> : gemm_any_lds_kernel<0, 2>);
+      hipLaunchKernelGGL(kern, grid2, block, 0, st, v);
     } else if (dual && wide) hipLaunchKernelGGL((gemm_any_mfma_kernel<1, true, 4>), gridw, block, 0, st, g);
     else if (wide) hipLaunchKernelGGL((gemm_any_mfma_kernel<0, true, 4>), gridw, block, 0, st, g);
     else if (dual && al) hipLaunchKernelGGL((gemm_any_mfma_kernel<1, true, 2>), grid, block, 0, st, g);

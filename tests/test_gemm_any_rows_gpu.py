@@ -92,3 +92,15 @@ def test_experts_on_the_lines(N, K, sizes):
     for e in range(E):
         a, b = int(off[e]), int(off[e + 1])
         _close(out[a:b], x[a:b].float() @ w[e].float().t(), K)
+
+
+@pytest.mark.parametrize("M", [1024, 1153])
+@pytest.mark.parametrize("K", [8, 32, 40, 136, 256, 264])
+def test_many_workgroups_and_short_k(M, K):
+    B, N = 16, 640
+    g = torch.Generator("cuda").manual_seed(M + K)
+    a = torch.randn(M, B, K, device="cuda", generator=g).bfloat16().transpose(0, 1)
+    w = (torch.randn(B, N, K, device="cuda", generator=g) * K ** -0.5).bfloat16()
+    out = torch.full((M, B, N), float("nan"), device="cuda", dtype=torch.bfloat16).transpose(0, 1)
+    seq.gemm(a, w, out)
+    _close(out, torch.matmul(a.float(), w.float().transpose(1, 2).contiguous()), K)
