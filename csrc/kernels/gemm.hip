@@ -154,13 +154,17 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
   // without a plan, 17 .. 64 rows: one block per CU owning whole tiles (wide) where K is short, K slices over narrow
   // tiles where it is long. us at 32 rows, the K-split / tile kernels below -> now: 17920 x 1536 19 -> 14.5, 6464 x 1536
   // 14.1 -> 9.0, 1536 x 8960 19.2 -> 13.1, 1024 x 4096 12.1 -> 8.4, 1536 x 1536 8.2 -> 6.6. Above 32 rows the wide form pays
-  // only once its tiles cover the CUs (N >= 4160; at 64 rows 6464 x 1536 17.7 -> 13.0, 1536 x 1536 10.5 -> 7.8 sliced); wide and
-  // long (28672 x 4096: 50 us) stays with the tile kernel.
+  // only once its tiles cover the CUs (N >= 4160; at 64 rows 6464 x 1536 17.7 -> 13.0, 1536 x 1536 10.5 -> 7.8 sliced). Long and wide stays
+  // with the kernels below (8192 x 3072 at 64 rows 23.6, sliced 29.3; 28672 x 4096 50), and so do few rows of 3072 to 4096 columns, which
+  // fill the chip without slices (4096 x 4096 at 24 rows 12.8, sliced 14.4; at 48 as fast or faster sliced).
   // (both stage rows of x by 16-B LDS-DMA: rows that are not 16-B aligned stay below)
   const bool rows16 = reinterpret_cast<uintptr_t>(g.x) % 16 == 0 && g.lda % 8 == 0;
   if (g.path == 0 && rows16 && g.M > 16 && g.M <= 64 && g.waves == 0 && g.splitk == 0 && g.ntb == 0 && g.N >= 512) {
     GemmArgs h = g;
-    if (g.K > 2048) h.waves = g.N <= 8192 ? 4 : 0;
+    if (g.K > 2048) {
+      const bool filled = g.N >= 3072 && g.N <= 4096 && g.M <= 24 && g.K <= 5120;
+      h.waves = (g.N < 8192 || (g.N == 8192 && g.M <= 32)) && !filled ? 4 : 0;
+    }
     else if (g.M <= 32) h.waves = 8;
     else if (g.N >= 4160) h.waves = 8;
     else if (g.K > 512 && g.N <= 2048) h.waves = 4;

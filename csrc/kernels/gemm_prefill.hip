@@ -902,7 +902,7 @@ static void launch_prefill_cfg(const GemmParams& p, int nz, hipStream_t st) {
 // before: 1.31). 2048 rows, us before -> now: 1536 x 8960 154 -> 86, 1536 x 1536 30 -> 22, 1024 x 4096 60 -> 38,
 // 1024 x 1024 19 -> 14; 256 rows: 1536 x 8960 39 -> 27, 1536 x 1536 15 -> 13.
 struct PrefillForm {
-  int code;  // tile code (as the forced ones below); 0: leave it to the tile kernel of gemm_decode.h
+  int code;  // tile code (as the forced ones below); 0: leave it to the kernels of gemm_decode.h
   int nz;    // K slices
 };
 
@@ -927,7 +927,9 @@ static PrefillForm choose_prefill_form(int M, int N, int K, bool slabs, size_t s
       best = PrefillForm{code, nz};
     }
   };
-  // 64 x 64 tiles, weights in registers (gemm_decode.h gemm_tile3_kernel): short K, few rows
+  // 64 x 64 tiles, weights in registers (gemm_decode.h): short K, few rows. The cost is gemm_tile3_kernel's. launch_m() runs that from
+  // K = 768 on and from 128 rows or 128 tiles on, and where it runs another kernel, that one is ahead (us, gemm_tile3_kernel / its choice:
+  // 512 x 512 at 2048 rows 8.3, 7.5; 1536 x 8960 at 96 rows without a workspace 53.6, 43.0)
   if (K % 256 == 0 && N / 16 < 1024) take(0, 1, over((int64_t)over(M, 64) * (N / 64), cus) * (4.6f + 0.354f * nk));
   for (const Tile& t : tiles) {
     if (N % t.bn != 0) continue;
@@ -960,8 +962,7 @@ static PrefillForm choose_prefill_form(int M, int N, int K, bool slabs, size_t s
 }
 
 // Returns false for shapes the kernels do not take (the caller keeps the N-split tile
-// kernel): K % 64, N % 64, a row gather, the gamma-in-registers RMSNorm mode; and where that tile kernel is the
-// cheapest form.
+// kernels): K % 64, N % 64, a row gather, the gamma-in-registers RMSNorm mode; and where those are the cheapest form.
 template <int EPI, int NORM>
 static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, size_t slab_bytes, int max_counters,
                                hipStream_t st) {

@@ -46,3 +46,16 @@ def test_default_form_matches_float32(N, K, epi):
             bound = bound + tol * 8.0   # (the product of the pair carries both errors, each times the other's size)
         bad = (out.float() - y).abs() > bound
         assert not bad.any(), (M, N, K, float((out.float() - y).abs().max()))
+
+
+@pytest.mark.parametrize("N,K", [(3008, 2304), (3072, 2304), (4096, 4096), (4160, 2304), (8128, 2304), (8192, 2304), (8256, 2304)])
+def test_lines_of_the_medium_forms(N, K):
+    C, dev = ops.native(), "cuda"
+    g = torch.Generator(dev).manual_seed(N + K)
+    w = (torch.randn(N, K, device=dev, generator=g) * K ** -0.5).bfloat16()
+    wp = ops.pack_weight(w)
+    for M in (17, 24, 25, 32, 33, 64):
+        x, out = torch.randn(M, K, device=dev, generator=g).bfloat16(), torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+        C.gemm(x, wp, N, K, out, 0, ws=ops.workspace(torch.device(dev)), fault=ops.fault_word(dev))
+        y = x.float() @ w.float().t()
+        assert ((out.float() - y).abs() <= 4.0 * K * 2.0 ** -24 + 2.0 ** -8 * y.abs()).all(), (M, N, K)   # (bound as above)
