@@ -7,6 +7,9 @@
 // routing (sigmoid or softmax scores with an optional selection-only correction, top-k, counting sort by
 // expert, weighted combine with an optional shared-expert row). Every kernel reads its sizes from arguments and its per-step metadata from device
 // memory, so the launches are graph-capturable.
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 #include "seq_launchers.h"
 
@@ -771,11 +774,27 @@ void launch_map_pair_combine(const void* a, int f32, float lam, float scale, flo
                      out, H, G, V, T);
 }
 
+// fn(NI) with NI columns of a row per thread, `ni` or the next form, MOST at most
+template <int MOST, typename F>
+static void row_columns(int ni, F&& fn) {
+  if (ni <= 1) fn(std::integral_constant<int, 1>{});
+  else if (ni == 2) fn(std::integral_constant<int, 2>{});
+  else if (ni == 3) fn(std::integral_constant<int, 3>{});
+  else if (ni == 4 || MOST == 4) fn(std::integral_constant<int, 4>{});
+  else if (ni <= 6) fn(std::integral_constant<int, MOST == 4 ? 4 : 6>{});
+  else fn(std::integral_constant<int, MOST>{});
+}
+
 void launch_post_norm_add(const PostNormArgs& a, hipStream_t st) {
   if (a.T <= 0 || a.W <= 0) return;
-  auto kern = a.W <= 1024 ? (a.y_f32 ? post_norm_add_kernel<4, true> : post_norm_add_kernel<4, false>)
-                          : (a.y_f32 ? post_norm_add_kernel<8, true> : post_norm_add_kernel<8, false>);
-  hipLaunchKernelGGL(kern, dim3(a.T), dim3(256), 0, st, a);
+  // A column past the row costs what any other does, and registers keep waves off a CU that reads planes of a history: at 2048 rows with
+  // three of them, us with four columns per thread / eight, 1536 wide 16.1, 23.1 (a thread per column and pass 20.0), 4096 wide 39, 55 (46).
+  const int most = a.hist != nullptr ? 4 : (a.W > 2048 && a.T >= 1024 ? 6 : 8);
+  row_columns<8>(std::min(most, (a.W + 255) / 256), [&](auto ni) {
+    constexpr int NI = decltype(ni)::value;
+    auto kern = a.y_f32 ? post_norm_add_kernel<NI, true> : post_norm_add_kernel<NI, false>;
+    hipLaunchKernelGGL(kern, dim3(a.T), dim3(256), 0, st, a);
+  });
 }
 
 void launch_norm_rows(const void* x, int64_t ldx_, int x_f32, const int32_t* rows, const float* w, int w_scalar,
@@ -794,8 +813,14 @@ void launch_embed_rows(const int32_t* ids, const int32_t* prev, const void* tabl
 void launch_gated_residual(float* x, const void* y1, const void* g1, int64_t ldg1, const float* b1, const void* y2,
                            const void* g2, int64_t ldg2, const float* b2, int f32, int T, int W, hipStream_t st) {
   if (T <= 0) return;
-  auto kern = f32 ? gated_residual_kernel<4, true> : gated_residual_kernel<4, false>;
-  hipLaunchKernelGGL(kern, dim3(T), dim3(256), 0, st, x, y1, g1, ldg1, b1, y2, g2, ldg2, b2, W);
+  // the fewest columns per thread that take no more passes than four do (2048 rows, us with four / the fewest: 256 wide 6.5, 4.3, 1536
+  // wide 13.2, 11.5)
+  const int passes = (W + 1023) / 1024;
+  row_columns<4>((W + 256 * passes - 1) / (256 * passes), [&](auto ni) {
+    constexpr int NI = decltype(ni)::value;
+    auto kern = f32 ? gated_residual_kernel<NI, true> : gated_residual_kernel<NI, false>;
+    hipLaunchKernelGGL(kern, dim3(T), dim3(256), 0, st, x, y1, g1, ldg1, b1, y2, g2, ldg2, b2, W);
+  });
 }
 
 void launch_moe_route(const float* z, const float* corr, int T, int E, int top, float norm_eps, int score, float scale,
