@@ -1,7 +1,11 @@
 """Which form a step of the recurrent mixers takes, by its rows (with padding) and sequences: host rules, no GPU."""
+from types import SimpleNamespace
+
 import pytest
+import torch
 
 from vgate import ops
+from vgate.models import hybrid
 
 
 def _plan(name, *sizes):
@@ -51,3 +55,12 @@ def test_chunks_cover_every_way_to_share_the_rows(name, args):
                     lens = [lim + 1] * (n - 1)
                 lens.append(T - sum(lens))
                 assert sum(-(-m // C) for m in lens if m > lim) <= chunks, (T, S, lens)
+
+
+@pytest.mark.parametrize("rows", [1000, 1024, 1088, 1360])
+@pytest.mark.parametrize("f32", [False, True])
+def test_row_major_projections_are_not_padded_past_whole_tiles_of_64(rows, f32):
+    w = torch.randn(rows, 64).to(torch.float32 if f32 else torch.bfloat16)
+    proj, col = hybrid._fuse_inputs(SimpleNamespace(in_rows=[("a", w)]), [], 64, "cpu", f32)
+    assert proj.N == -(-rows // 64) * 64 and col == {"a": (0, rows)}
+    assert torch.equal(proj.w[:rows], w) and not proj.w[rows:].any()

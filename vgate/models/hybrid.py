@@ -51,7 +51,7 @@ from vgate.parallel.comm import TPGroup
 
 def _fuse_inputs(mixer, extra: list, width: int, device, f32: bool):
     """Stack every matrix that multiplies the layer's input into ONE GEMM (segments padded to 8 rows,
-    the total to 64 columns, or 256 where it is wide). Returns (Proj, {name: (first column, columns)})."""
+    the total to 64 columns, or 256 where it is wide and packed). Returns (Proj, {name: (first column, columns)})."""
     rows = list(mixer.in_rows) + extra
     if not rows:   # a mixer whose projections all read inputs of their own
         del mixer.in_rows
@@ -66,9 +66,10 @@ def _fuse_inputs(mixer, extra: list, width: int, device, f32: bool):
         parts.append(w)
         bparts.append(torch.cat([b, torch.zeros(w.shape[0] - b.shape[0], dtype=b.dtype)]))
         off += w.shape[0]
-    # whole 64-column tiles: what the packed GEMMs ask for; from 1024 columns on whole 256-column tiles, which the fast
-    # prompt kernels need (2048 rows x 6464 columns of 1536: 99 us, 6656 columns 44 us)
-    tile = 256 if off >= 1024 else 64
+    # whole 64-column tiles: what the packed GEMMs ask for; from 1024 columns on whole 256-column tiles, which their fast
+    # prompt kernels need (2048 rows x 6464 columns of 1536: 99 us, 6656 columns 44 us). The row-major GEMMs (fp32, CPU,
+    # narrow inputs) would only multiply more zeros.
+    tile = 256 if off >= 1024 and Proj.packs(width, device, f32) else 64
     if off % tile:
         parts.append(torch.zeros(tile - off % tile, width, dtype=parts[0].dtype))
         bparts.append(torch.zeros(tile - off % tile, dtype=bparts[0].dtype))

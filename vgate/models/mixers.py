@@ -61,8 +61,7 @@ class Proj:
         self.pair_act, self.limit, self.alpha = pair_act, limit, alpha
         dev = torch.device(device)
         n_ok = (N // 2) % 64 == 0 if silu_pair else N % 64 == 0
-        self.packed = (USE_PACKED and allow_packed and not f32 and dev.type == "cuda" and n_ok and K % 64 == 0
-                       and K >= PACKED_MIN_K)
+        self.packed = allow_packed and n_ok and self.packs(K, device, f32)
         # the packed kernels' pair epilogue is SiLU: another pair activation runs the stacked [gate; up]
         # matrix as a plain packed GEMM and applies act(gate) * up in a row kernel
         self.split_act = self.packed and silu_pair and pair_act != seq.ACT_SILU_MUL
@@ -76,6 +75,11 @@ class Proj:
             self.w = w.to(dev, torch.float32 if f32 else torch.bfloat16).contiguous()
             self.bias = None if bias is None else bias.to(dev, torch.float32).contiguous()
         self.out_features = N // 2 if silu_pair else N
+
+    @staticmethod
+    def packs(K: int, device, f32: bool) -> bool:
+        """Whether a matrix of whole 64-row tiles and K columns goes to the packed GEMMs."""
+        return USE_PACKED and not f32 and torch.device(device).type == "cuda" and K % 64 == 0 and K >= PACKED_MIN_K
 
     def nbytes(self) -> int:
         return self.lin.nbytes() if self.packed else self.w.numel() * self.w.element_size()
