@@ -5,7 +5,7 @@ back-to-back launches (weights warm in the Infinity Cache / L2). Inside a prefil
 reads its weights cold. This times every candidate both ways, plus hipBLASLt (torch.mm, oracle)
 cold, and prints the best of each per (shape, M).
 
-    python benchmarks/probes/prefill_cold_sweep.py [--ms 320,448,640] [--model llama8b] [--only 1024,1025]
+    python benchmarks/probes/prefill_cold_sweep.py [--ms 320,448,640] [--model llama8b | --shapes 1024x1024,1536x8960] [--only 1024,1025]
 """
 from __future__ import annotations
 
@@ -30,6 +30,7 @@ def main():
     ap.add_argument("--ms", default="320,448,640")
     ap.add_argument("--iters", type=int, default=4)
     ap.add_argument("--model", default="qwen", choices=sorted(SHAPES))
+    ap.add_argument("--shapes", default="", help="comma list of NxK in place of the model's")
     ap.add_argument("--only", default="", help="comma list of tile codes to time (default: every candidate)")
     ap.add_argument("--norm", action="store_true", help="with the folded RMSNorm row scale (qkv / gate_up in a step)")
     a = ap.parse_args()
@@ -63,7 +64,8 @@ def main():
     cands = ops.PREFILL_CANDIDATES + ops.PREFILL_RING_CANDIDATES
     cands += [(t, s) for t in (1025, 769) for s in range(9) if (t, s) not in cands]  # persistent: tail slices
     only = {int(c) for c in a.only.split(",") if c}
-    for name, N, K in SHAPES[a.model]:
+    shapes = [(s, *map(int, s.split("x"))) for s in a.shapes.split(",") if s] or SHAPES[a.model]
+    for name, N, K in shapes:
         w = (torch.randn(N, K, device=dev) / math.sqrt(K)).bfloat16()
         wp = ops.pack_weight(w)
         for M in [int(m) for m in a.ms.split(",")]:

@@ -898,8 +898,9 @@ static void launch_prefill_cfg(const GemmParams& p, int nz, hipStream_t st) {
 // a, b, c, d in us, fitted to a sweep of 35 shapes (N 128 .. 28672, K 512 .. 14336) x M 128 .. 2048 on cold weights, rms
 // error 5 to 9 % per form. What the forms trade: a large tile has the highest rate (256 x 256: 1.6 PFLOP/s per full
 // round) and the worst last round; splitting K fills the chip for few tiles and costs a pass over the partials.
-// The times of the taken forms are 1.02 of the best of the sweep (geometric mean; the thresholds on block counts used
-// before: 1.31). 2048 rows, us before -> now: 1536 x 8960 154 -> 86, 1536 x 1536 30 -> 22, 1024 x 4096 60 -> 38,
+// The times of the taken forms are 0.95 to 1.03 of the best of these forms by the number of rows (geometric means;
+// profiles/prefill_gemm_forms_sweep.txt; the thresholds on block counts used before: 1.31). 64 x 512 and 128 x 320 tiles, which
+// start-up plans may take, would gain 0.2 % at most. 2048 rows, us before -> now: 1536 x 8960 154 -> 86, 1536 x 1536 30 -> 22, 1024 x 4096 60 -> 38,
 // 1024 x 1024 19 -> 14; 256 rows: 1536 x 8960 39 -> 27, 1536 x 1536 15 -> 13.
 struct PrefillForm {
   int code;  // tile code (as the forced ones below); 0: leave it to the kernels of gemm_decode.h
