@@ -357,6 +357,10 @@ int sample_segments(int B, int V) {
 // then takes longer than the meeting, and four waves cannot keep a CU busy with it. us, top-p 0.95, 256 -> 1024 threads:
 // vocabulary 152064, 32 rows 42.8 -> 37.2, 64 rows 103 -> 78, 256 rows (whole rows) 339 -> 201; 16 rows (9 pieces) 29.7 against 31.2.
 static bool long_rows(int V, int nseg) { return (V >> 2) > 3072 * nseg; }
+// More whole rows than CUs: two workgroups of 1024 threads share a CU, of 256 eight, and only a long row makes up for that (us, 256 ->
+// 1024 threads, greedy and top-p: 512 rows of 32000 27, 104 -> 35, 114, of 65536 44, 179 -> 48, 180, of 128256 76, 347 -> 71, 295; 768 rows of
+// 128256 93, 493 -> 108, 512).
+static bool long_whole_rows(int V, int B) { return B <= SAMPLE_MAX_BLOCKS ? long_rows(V, 1) : B <= 2 * SAMPLE_MAX_BLOCKS && V > 65536; }
 
 void launch_sample(const SampleArgs& s, hipStream_t st) {
   if (s.B <= 0) return;
@@ -369,7 +373,7 @@ void launch_sample(const SampleArgs& s, hipStream_t st) {
     return;
   }
   a.tl = tl_take("sample", s.B);
-  if (long_rows(s.V, 1)) hipLaunchKernelGGL(sample_row_kernel<1024>, dim3(1, s.B), dim3(1024), 0, st, a);
+  if (long_whole_rows(s.V, s.B)) hipLaunchKernelGGL(sample_row_kernel<1024>, dim3(1, s.B), dim3(1024), 0, st, a);
   else hipLaunchKernelGGL(sample_row_kernel<SAMPLE_THREADS>, dim3(1, s.B), dim3(SAMPLE_THREADS), 0, st, a);
 }
 

@@ -29,3 +29,21 @@ def test_rows_do_not_depend_on_the_batch(V):
         rows = torch.arange(n, device=dev)
         assert torch.equal(run(rows), whole[:n]), n
     assert torch.equal(whole[::3], lg[::3].argmax(-1).int())      # temperature 0
+
+
+@pytest.mark.parametrize("V,B", [(16384, 257), (49152, 300), (70000, 513), (70000, 512)])
+def test_more_rows_than_workgroups(V, B):
+    dev = "cuda"
+    g = torch.Generator(dev).manual_seed(V + B)
+    lg = 2.0 * torch.randn(B, V, device=dev, generator=g)
+    t, p = torch.tensor([0.0, 0.8, 1.0] * B, device=dev)[:B], torch.tensor([1.0, 0.95, 0.5, 0.9] * B, device=dev)[:B]
+    k = torch.tensor([-1, -1, -1, 50, -1] * B, dtype=torch.int32, device=dev)[:B]
+    seeds, offs = torch.arange(B, device=dev), torch.arange(B, device=dev) % 7
+
+    def run(n):
+        out = torch.full((n,), -1, dtype=torch.int32, device=dev)
+        ops.sample(lg[:n].contiguous(), t[:n], p[:n], k[:n], seeds[:n], offs[:n], out=out)
+        return out
+
+    whole = run(B)
+    assert torch.equal(run(64), whole[:64]) and torch.equal(whole[::3], lg[::3].argmax(-1).int())
