@@ -907,7 +907,7 @@ struct PrefillForm {
   int nz;    // K slices
 };
 
-static PrefillForm choose_prefill_form(int M, int N, int K, bool slabs, size_t slab_bytes, bool counters) {
+static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool slabs, size_t slab_bytes, bool counters) {
   struct Tile {
     int code, bm, bn;
     float a, b, c, d;
@@ -931,7 +931,13 @@ static PrefillForm choose_prefill_form(int M, int N, int K, bool slabs, size_t s
   // 64 x 64 tiles, weights in registers (gemm_decode.h): short K, few rows. The cost is gemm_tile3_kernel's. launch_m() runs that from
   // K = 768 on and from 128 rows or 128 tiles on, and where it runs another kernel, that one is ahead (us, gemm_tile3_kernel / its choice:
   // 512 x 512 at 2048 rows 8.3, 7.5; 1536 x 8960 at 96 rows without a workspace 53.6, 43.0)
-  if (K % 256 == 0 && N / 16 < 1024) take(0, 1, over((int64_t)over(M, 64) * (N / 64), cus) * (4.6f + 0.354f * nk));
+  // With a folded norm every wave sums the squares of its 64 rows on the way: half as much again (2048 x 1536 at 256 rows 23.3 us, plain 16.7,
+  // where 128 x 64 tiles take 17.5; 1024 x 4096 at 1024 rows 48.7, K-split 128 x 128 tiles 31.6); not the
+  // kernel below K = 768 (1024 x 512 at 384 rows 13.0).
+  if (K % 256 == 0 && N / 16 < 1024) {
+    const int rounds = over((int64_t)over(M, 64) * (N / 64), cus);
+    take(0, 1, norm && K >= 768 ? 9.7f + rounds * (1.25f + 0.532f * nk) : rounds * (4.6f + 0.354f * nk));
+  }
   for (const Tile& t : tiles) {
     if (N % t.bn != 0) continue;
     for (int nz : slices) {
@@ -970,7 +976,7 @@ static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, 
   constexpr int NTB = 1;  // every epilogue works on self-contained 16-column tiles
   if (p.K % 64 != 0 || p.N % 64 != 0 || p.row_idx != nullptr) return false;
   if (force_bn == 0 && force_sk == 0) {
-    const PrefillForm f = choose_prefill_form(p.M, p.N, p.K, p.slabs != nullptr, slab_bytes, p.counters != nullptr);
+    const PrefillForm f = choose_prefill_form(p.M, p.N, p.K, NORM == 2, p.slabs != nullptr, slab_bytes, p.counters != nullptr);
     if (f.code == 0) return false;
     force_bn = f.code;
     force_sk = f.nz;

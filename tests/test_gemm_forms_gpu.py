@@ -59,3 +59,18 @@ def test_lines_of_the_medium_forms(N, K):
         C.gemm(x, wp, N, K, out, 0, ws=ops.workspace(torch.device(dev)), fault=ops.fault_word(dev))
         y = x.float() @ w.float().t()
         assert ((out.float() - y).abs() <= 4.0 * K * 2.0 ** -24 + 2.0 ** -8 * y.abs()).all(), (M, N, K)   # (bound as above)
+
+
+@pytest.mark.parametrize("N,K", [(512, 512), (1024, 1024), (1536, 1536), (1600, 2048), (2048, 1792), (4096, 1024), (4160, 2048), (1024, 4096)])
+def test_folded_norm_on_the_lines(N, K):
+    C, dev = ops.native(), "cuda"
+    g = torch.Generator(dev).manual_seed(N + K)
+    w = (torch.randn(N, K, device=dev, generator=g) * K ** -0.5).bfloat16()
+    wp = ops.pack_weight(w)
+    for M in (17, 20, 21, 32, 33, 64, 96, 128, 257, 512, 1024):
+        x, out = (3 * torch.randn(M, K, device=dev, generator=g)).bfloat16(), torch.empty(M, N, dtype=torch.float32, device=dev)
+        C.gemm(x, wp, N, K, out, 1, rownorm=True, eps=1e-6, ws=ops.workspace(torch.device(dev)), fault=ops.fault_word(dev))
+        f = x.double()
+        y = f @ w.double().t() * torch.rsqrt(f.pow(2).mean(1, keepdim=True) + 1e-6)
+        # K fp32 products with |x| |w| sums < 4 after the norm, and a sum of K squares: each off by K 2^-24 of itself at most
+        assert ((out.double() - y).abs() <= 8.0 * K * 2.0 ** -24 + K * 2.0 ** -24 * y.abs()).all(), (M, N, K)
