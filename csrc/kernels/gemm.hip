@@ -155,19 +155,28 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
   // tiles where it is long. us at 32 rows, the K-split / tile kernels below -> now: 17920 x 1536 19 -> 14.5, 6464 x 1536
   // 14.1 -> 9.0, 1536 x 8960 19.2 -> 13.1, 1024 x 4096 12.1 -> 8.4, 1536 x 1536 8.2 -> 6.6. Above 32 rows the wide form pays
   // only once its tiles cover the CUs (N >= 4160; at 64 rows 6464 x 1536 17.7 -> 13.0, 1536 x 1536 10.5 -> 7.8 sliced). Long and wide stays
-  // with the kernels below (8192 x 3072 at 64 rows 23.6, sliced 29.3; 28672 x 4096 50), and so do few rows of 3072 to 4096 columns, which
-  // fill the chip without slices (4096 x 4096 at 24 rows 12.8, sliced 14.4; at 48 as fast or faster sliced).
+  // with the kernels below (8192 x 3072 at 64 rows 23.6, sliced 29.3; 28672 x 4096 50), and so do up to 32 rows of 3072 to 4096 columns, which
+  // fill the chip without slices (4096 x 4096 at 24 rows 14.1, sliced 17.2, at 32 15.4, 17.3, at 48 21.0, 19.4; with longer K sooner:
+  // 3072 x 5120 at 32 18.8, 16.3), slices that come to little more than a workgroup per CU (2048 x 8960, 288 of them, at 24 rows 19.7, 20.9, at 64
+  // 29.3, 31.2; 6144 x 3072 at 17 17.2, 19.0) and the very shortest (1536 x 3072 at 17 rows 11.0, 12.1, at 32 13.1, 12.5; 1024 x 1024 at 48 9.5, 10.3).
+  // A folded norm costs the wide form more than the K-split kernels, which have more waves to sum squares: few columns of K up to 1024 and of
+  // 2048 stay with them (4096 x 1024 at 17 rows 8.4, wide 10.3, at 32 9.2, 10.5; 1024 x 2048 at 24 10.3, 11.4; 1024 x 1536 at 24 11.0, 10.2;
+  // 6144 x 4096 at 17 19.9, sliced 21.9, at 24 23.0, 22.2).
   // (both stage rows of x by 16-B LDS-DMA: rows that are not 16-B aligned stay below)
   const bool rows16 = reinterpret_cast<uintptr_t>(g.x) % 16 == 0 && g.lda % 8 == 0;
   if (g.path == 0 && rows16 && g.M > 16 && g.M <= 64 && g.waves == 0 && g.splitk == 0 && g.ntb == 0 && g.N >= 512) {
     GemmArgs h = g;
     if (g.K > 2048) {
-      const bool filled = g.N >= 3072 && g.N <= 4096 && g.M <= 24 && g.K <= 5120;
-      h.waves = (g.N < 8192 || (g.N == 8192 && g.M <= 32)) && !filled ? 4 : 0;
+      const int64_t groups = g.N / 64;   // (workgroups per slice; slices of 32 k-steps at most, as launch_gemm_mid() cuts them)
+      const int64_t blocks = groups * ((g.K + 1023) / 1024);
+      const bool filled = g.N >= 3072 && g.N <= 4096 && g.M <= 32 && g.K <= (g.N > 3584 ? (g.M <= 24 ? 14336 : 5120) : 4096);
+      const bool over = blocks > 256 && blocks <= 320 && (g.M <= 24 || g.N <= 4096);
+      const bool shortest = g.M <= 20 && ((g.K <= 3072 && g.N <= 2048) || (g.rownorm && g.K <= 4096 && g.N > 4096 && g.N < 8192));
+      h.waves = (g.N < 8192 || (g.N == 8192 && g.M <= 32)) && !filled && !over && !shortest ? 4 : 0;
     }
-    else if (g.M <= 32) h.waves = 8;
+    else if (g.M <= 32) h.waves = g.rownorm && g.N <= 4096 && (g.K <= 1024 || g.K > 1792) ? 0 : 8;
     else if (g.N >= 4160) h.waves = 8;
-    else if (g.K > 512 && g.N <= 2048) h.waves = 4;
+    else if (g.K > 1024 && g.N <= 2048) h.waves = 4;
     if (h.waves != 0 && launch_gemm_mid(h, st)) return;
   }
   // decode rows on the register-stationary kernel (path 4: a decode plan / forced; gemm_kx_bf16.hip)
