@@ -709,7 +709,7 @@ bool takes_scan(int T, int S, int H, int D) {
 // chunks' three empty ones: 128 sequences 35 us, 45; 256 65, 82).
 int delta_limit(int T, int S) { return T <= S || T <= 64 ? T : 48; }
 // chunks of a step whose sequences longer than lim tokens have T between them: each has at most one that is not whole
-int delta_chunks(int T, int lim) { return T <= lim ? 0 : T / CN + T / (lim + 1); }
+int delta_chunks(int T, int S, int lim) { return T <= lim ? 0 : (T + std::min(S, T / (lim + 1)) * (CN - 1)) / CN; }
 
 // {w, a u, k, r}, u, the raw outputs; whole 16-B pieces
 size_t scan_floats(int T, int H, int D) { return ((size_t)T * H * D * 6 + 3) / 4 * 4; }
@@ -754,7 +754,7 @@ void launch_delta_dp(const DeltaArgs& a, int T, const DeltaPlan& plan, float* sc
 DeltaPlan delta_rule_plan(int T, int S, int H, int D) {
   const bool scan = takes_scan(T, S, H, D);
   const int lim = scan ? (T <= 128 ? T : delta_scan_limit(D)) : delta_limit(T, S);
-  return {scan, lim, S == 1 && T > lim ? (T + CN - 1) / CN : delta_chunks(T, lim)};
+  return {scan, lim, S == 1 && T > lim ? (T + CN - 1) / CN : delta_chunks(T, S, lim)};
 }
 
 size_t delta_rule_scratch_floats(int T, int S, int H, int D) {

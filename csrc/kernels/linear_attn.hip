@@ -862,8 +862,9 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
 // steps (T <= S), and short ones that may nearly be, take one launch (8 heads of 128, in parentheses with empty or few chunks: 128
 // sequences 32 us (53), 256 61 (98); 63 decoded tokens beside a portion of 65 95 (146), 127 beside 65 103 (169), beside 129 183 (170)).
 int short_limit(int T, int S) { return T <= std::max(S, 96) || T <= std::min(2 * S, 256) ? T : 64; }
-// chunks of a step whose sequences longer than lim tokens have T between them: each has at most one that is not whole
-int long_chunks(int T, int lim) { return T <= lim ? 0 : T / CT + T / (lim + 1); }
+// chunks of a step whose sequences longer than lim tokens have T between them: each has at most one that is not whole. (Workgroups past
+// the last chunk leave at once, but push real ones together on fewer CUs.)
+int long_chunks(int T, int S, int lim) { return T <= lim ? 0 : (T + std::min(S, T / (lim + 1)) * (CT - 1)) / CT; }
 // Decoding steps: one launch instead of three (16 sequences x 8 heads of 128: 25.3 -> 12.2 us). Long steps: chunks with fp32 MFMA
 // (2048 tokens 162 -> 100 us, 63 decoded tokens beside a portion of 961 1054 -> 169, 64 portions of 16 62 -> 47). Between them
 // the scan below, which spreads a head's columns over several workgroups, is ahead where sequences are few: one portion of
@@ -918,7 +919,7 @@ LinearPlan linear_attn_plan(int T, int S, int D, int V) {
   // T counts padding rows too, so a sequence may be much shorter. A lone one then takes chunks whatever its length (not more
   // of them than any step of T rows); several are told apart by their lengths on the device.
   const bool lone = S == 1 && T > lim;
-  return {takes_small(T, S, D, V), lone ? 0 : lim, lone ? (T + CT - 1) / CT : long_chunks(T, lim)};
+  return {takes_small(T, S, D, V), lone ? 0 : lim, lone ? (T + CT - 1) / CT : long_chunks(T, S, lim)};
 }
 size_t linear_attn_scratch_floats(int T, int S, int H, int D, int V) {
   const int CH = linear_attn_chunk_size(T, S);
