@@ -868,10 +868,22 @@ int long_chunks(int T, int S, int lim) { return T <= lim ? 0 : (T + std::min(S, 
 // Decoding steps: one launch instead of three (16 sequences x 8 heads of 128: 25.3 -> 12.2 us). Long steps: chunks with fp32 MFMA
 // (2048 tokens 162 -> 100 us, 63 decoded tokens beside a portion of 961 1054 -> 169, 64 portions of 16 62 -> 47). Between them
 // the scan below, which spreads a head's columns over several workgroups, is ahead where sequences are few: one portion of
-// 96 78 us (here 96; of 128 98 against 84), 8 of 48 54 (59).
-bool takes_small(int T, int S, int D, int V) {
-  return D <= 128 && V <= 128 &&
-         (T <= 2 * S || T >= (S == 1 ? 128 : (S < 16 ? 512 : 256)));
+// 96 78 us (here 96; of 128 98 against 84), 8 of 48 54 (59), and where sequences x heads are few besides (16 of 48, 4 heads: 50, here 54).
+// With key sizes up to 64 a token of the scan costs half as much, and a long step's own chunks there spread better than the MFMA ones:
+// those are ahead where portions are long on average only while their workgroups fill the chip about once (us, scan / MFMA chunks, heads of
+// 64: 2048 tokens, 8 heads 98, 68; 16 heads 115, 123; 32 heads 144, 229; 512 tokens, 8 heads 54, 60; 4 x 400, 4 heads 80, 63, 16 heads 103, 123,
+// 32 heads 134, 229; 20 + 700, 8 heads 58, 75).
+bool takes_small(int T, int S, int H, int D, int V) {
+  if (D > 128 || V > 128) return false;
+  if (T <= 2 * S) return true;
+  if (T < (S == 1 ? 128 : (S < 16 ? 512 : 256)) || (T < 64 * S && S * H < 128)) return false;
+  if (D > 64 || T < 96 * S) return true;
+  if (S == 1 && T < 256) return T >= 160;   // (the scan has no chunks below 256 tokens)
+  const bool tiny = D <= 32 && V <= 32;
+  const int64_t work = (int64_t)T * H;      // (a workgroup per 64)
+  if (S == 1) return work >= (tiny ? 12288 : 8192) && work <= 16384;
+  if (S == 2) return !tiny && work >= 8192 && work <= 16000;
+  return work >= (tiny ? 8000 : 4000) && work <= 16000;
 }
 
 template <int DP, bool F32, bool PRE>
@@ -914,17 +926,17 @@ int linear_attn_chunk_size(int T, int S) {
   return T >= 256 && T >= 64 * S ? 64 : 0;
 }
 int linear_attn_chunks(int T, int S, int CH) { return CH > 0 ? T / CH + S : 0; }
-LinearPlan linear_attn_plan(int T, int S, int D, int V) {
+LinearPlan linear_attn_plan(int T, int S, int H, int D, int V) {
   const int lim = short_limit(T, S);
   // T counts padding rows too, so a sequence may be much shorter. A lone one then takes chunks whatever its length (not more
   // of them than any step of T rows); several are told apart by their lengths on the device.
   const bool lone = S == 1 && T > lim;
-  return {takes_small(T, S, D, V), lone ? 0 : lim, lone ? (T + CT - 1) / CT : long_chunks(T, S, lim)};
+  return {takes_small(T, S, H, D, V), lone ? 0 : lim, lone ? (T + CT - 1) / CT : long_chunks(T, S, lim)};
 }
 size_t linear_attn_scratch_floats(int T, int S, int H, int D, int V) {
   const int CH = linear_attn_chunk_size(T, S);
   const size_t any = (size_t)T * H * (4 * D + 2 * V) + (size_t)linear_attn_chunks(T, S, CH) * H * D * (V + 1);
-  const LinearPlan plan = linear_attn_plan(T, S, D, V);
+  const LinearPlan plan = linear_attn_plan(T, S, H, D, V);
   const size_t small = (size_t)T * H * V + (size_t)plan.chunks * H * D * (V + 1);
   return plan.small && small > any ? small : any;
 }
@@ -934,7 +946,7 @@ size_t linear_attn_scratch_floats(int T, int S, int H, int D, int V) {
 void launch_linear_attn(const LinearAttnArgs& a, int T, float* scratch, hipStream_t st) {
   if (a.S <= 0 || a.H <= 0 || T <= 0) return;
   const int64_t nk = (int64_t)T * a.H * a.D, nv = (int64_t)T * a.H * a.V;
-  const LinearPlan plan = linear_attn_plan(T, a.S, a.D, a.V);
+  const LinearPlan plan = linear_attn_plan(T, a.S, a.H, a.D, a.V);
   if (plan.small && a.cols_per_lane == 0) {   // scratch: raw outputs, the chunks' states, their decays
     float* states = scratch + nv;
     float* decays = states + (size_t)plan.chunks * a.H * a.D * a.V;

@@ -246,7 +246,7 @@ struct LinearPlan {
   bool small;
   int lim, chunks;
 };
-LinearPlan linear_attn_plan(int T, int S, int D, int V);
+LinearPlan linear_attn_plan(int T, int S, int H, int D, int V);
 size_t linear_attn_scratch_floats(int T, int S, int H, int D, int V);
 // T rows; scratch: linear_attn_scratch_floats() floats, 16-B aligned
 void launch_linear_attn(const LinearAttnArgs& a, int T, float* scratch, hipStream_t st);

@@ -931,8 +931,8 @@ void bind_seq(pybind11::module& m) {
     return (int64_t)vgate::delta_rule_scratch_floats((int)T, (int)S, (int)H, (int)D);
   }, "floats of scratch delta_rule can use for a step of T tokens and S sequences (with fewer it takes no chunks)", py::arg("T"),
         py::arg("H"), py::arg("D"), py::arg("S") = 1);
-  m.def("linear_attn_plan", [](int64_t T, int64_t S, int64_t D, int64_t V) {
-    const auto p = vgate::linear_attn_plan((int)T, (int)S, (int)D, (int)V);
+  m.def("linear_attn_plan", [](int64_t T, int64_t S, int64_t H, int64_t D, int64_t V) {
+    const auto p = vgate::linear_attn_plan((int)T, (int)S, (int)H, (int)D, (int)V);
     return std::make_tuple(p.small, (int64_t)p.lim, (int64_t)p.chunks);
   }, "(not the scan, most tokens of a sequence in the short form, chunks) of a linear_attn step of T rows and S sequences");
   m.def("delta_rule_plan", [](int64_t T, int64_t S, int64_t H, int64_t D) {

@@ -31,16 +31,25 @@ def test_delta_rule_lines(T, S, H, D, scan, chunks):
 def test_decoding_steps_take_one_launch(T, S):
     scan, lim, chunks = _plan("delta_rule_plan", T, S, 8, 128)
     assert not scan and lim >= T and chunks == 0
-    small, lim, chunks = _plan("linear_attn_plan", T, S, 128, 128)
+    small, lim, chunks = _plan("linear_attn_plan", T, S, 8, 128, 128)
     assert small and lim >= T and chunks == 0
 
 
 @pytest.mark.parametrize("T,S", [(128, 64), (192, 128), (256, 128)])
 def test_linear_attention_nearly_decoding_steps_take_one_launch(T, S):
-    assert _plan("linear_attn_plan", T, S, 128, 128)[2] == 0
+    assert _plan("linear_attn_plan", T, S, 8, 128, 128)[2] == 0
 
 
-@pytest.mark.parametrize("name,args", [("delta_rule_plan", (8, 128)), ("linear_attn_plan", (128, 128))])
+@pytest.mark.parametrize("T,S,H,D,V,small", [(2048, 1, 8, 64, 64, True), (2048, 1, 16, 64, 64, False), (2048, 1, 32, 64, 64, False),
+                                             (512, 1, 8, 64, 64, False), (160, 1, 8, 64, 64, True), (128, 1, 8, 64, 64, False),
+                                             (128, 1, 8, 128, 128, True), (2048, 1, 16, 128, 128, True), (1600, 4, 4, 64, 64, True),
+                                             (1600, 4, 16, 64, 64, False), (720, 2, 8, 64, 64, False), (1024, 2, 8, 32, 32, False),
+                                             (1024, 16, 32, 64, 64, True), (768, 16, 4, 128, 128, False), (256, 256, 1, 32, 32, True)])
+def test_linear_attention_lines(T, S, H, D, V, small):
+    assert _plan("linear_attn_plan", T, S, H, D, V)[0] == small
+
+
+@pytest.mark.parametrize("name,args", [("delta_rule_plan", (8, 128)), ("linear_attn_plan", (8, 128, 128))])
 def test_chunks_cover_every_way_to_share_the_rows(name, args):
     """Whole chunks of C tokens and one that is not whole for each sequence of more than `lim` tokens."""
     C = 32 if name == "delta_rule_plan" else 64
