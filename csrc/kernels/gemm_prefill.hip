@@ -912,11 +912,25 @@ static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool slab
     int code, bm, bn;
     float a, b, c, d;
   };
-  // 256 x 256 / 256 x 128 four-phase, 128 x 128 (8 waves) / 128 x 64 on four-deep rings
-  static constexpr Tile tiles[] = {{1024, 256, 256, 10.2f, 1.33f, 1.5f, 0.49f},
-                                   {768, 256, 128, 7.1f, 1.00f, 1.6f, 0.56f},
-                                   {1281, 128, 128, 5.8f, 0.61f, 2.8f, 0.57f},
-                                   {640, 128, 64, 5.0f, 0.50f, 2.9f, 0.68f}};
+  struct Costs {
+    Tile tiles[4];        // 256 x 256 / 256 x 128 four-phase, 128 x 128 (8 waves) / 128 x 64 on four-deep rings
+    float n64[2], n128[2];   // two-deep rings: whole, per K-tile and block of a CU
+    float p256[4], p128[4];  // persistent: the last round whole, per K-tile, and of its K slices
+  };
+  // With the row scale of a folded norm (second set, fitted by itself to 16 shapes at 96 .. 2048 rows) every form sums the squares of its
+  // rows on the way, the more often the narrower its tiles: by the plain costs its choice is 1.06 of the best form (geometric mean at 512
+  // rows), by its own 1.006 (2048 x 1536 at 128 rows 22.6 -> 15.9 us, 1024 x 4096 at 1024 48.4 -> 31.4).
+  static constexpr Costs sets[2] = {{{{1024, 256, 256, 10.2f, 1.33f, 1.5f, 0.49f},
+                                      {768, 256, 128, 7.1f, 1.00f, 1.6f, 0.56f},
+                                      {1281, 128, 128, 5.8f, 0.61f, 2.8f, 0.57f},
+                                      {640, 128, 64, 5.0f, 0.50f, 2.9f, 0.68f}},
+                                     {5.0f, 0.54f}, {6.0f, 0.77f}, {13.4f, 1.61f, 13.6f, 2.4f}, {10.6f, 1.07f, 5.6f, 1.5f}},
+                                    {{{1024, 256, 256, 16.2f, 1.52f, -3.1f, 0.485f},
+                                      {768, 256, 128, 11.7f, 1.13f, -0.8f, 0.506f},
+                                      {1281, 128, 128, 9.0f, 0.705f, 2.4f, 0.395f},
+                                      {640, 128, 64, 7.6f, 0.585f, 3.0f, 0.412f}},
+                                     {10.5f, 0.548f}, {12.0f, 0.78f}, {22.0f, 1.59f, 13.7f, 4.2f}, {15.3f, 1.175f, 6.3f, 2.4f}}};
+  const Costs& cs = sets[norm ? 1 : 0];
   static constexpr int slices[] = {1, 2, 3, 4, 6, 8};
   const int cus = cu_count() > 0 ? cu_count() : 256, nk = K / 64;
   auto over = [](int64_t x, int y) { return (int)((x + y - 1) / y); };
@@ -931,14 +945,11 @@ static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool slab
   // 64 x 64 tiles, weights in registers (gemm_decode.h): short K, few rows. The cost is gemm_tile3_kernel's. launch_m() runs that from
   // K = 768 on and from 128 rows or 128 tiles on, and where it runs another kernel, that one is ahead (us, gemm_tile3_kernel / its choice:
   // 512 x 512 at 2048 rows 8.3, 7.5; 1536 x 8960 at 96 rows without a workspace 53.6, 43.0)
-  // With a folded norm every wave sums the squares of its 64 rows on the way: half as much again (2048 x 1536 at 256 rows 23.3 us, plain 16.7,
-  // where 128 x 64 tiles take 17.5; 1024 x 4096 at 1024 rows 48.7, K-split 128 x 128 tiles 31.6); not the
-  // kernel below K = 768 (1024 x 512 at 384 rows 13.0).
   if (K % 256 == 0 && N / 16 < 1024) {
     const int rounds = over((int64_t)over(M, 64) * (N / 64), cus);
-    take(0, 1, norm && K >= 768 ? 9.7f + rounds * (1.25f + 0.532f * nk) : rounds * (4.6f + 0.354f * nk));
+    take(0, 1, norm && K >= 768 ? 5.2f + rounds * (3.58f + 0.591f * nk) : rounds * (4.6f + 0.354f * nk));
   }
-  for (const Tile& t : tiles) {
+  for (const Tile& t : cs.tiles) {
     if (N % t.bn != 0) continue;
     for (int nz : slices) {
       const int64_t blocks = (int64_t)over(M, t.bm) * (N / t.bn) * nz;
@@ -950,20 +961,20 @@ static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool slab
   }
   // two-deep rings, several blocks per CU: the rate of the small tiles without whole rounds
   const int n64 = over((int64_t)over(M, 128) * (N / 64), cus), n128 = N % 128 == 0 ? over((int64_t)over(M, 128) * (N / 128), cus) : 0;
-  if (n64 > 1) take(64, 1, 5.0f + 0.54f * nk * n64);
-  if (n128 > 1) take(128, 1, 6.0f + 0.77f * nk * n128);
+  if (n64 > 1) take(64, 1, cs.n64[0] + cs.n64[1] * nk * n64);
+  if (n128 > 1) take(128, 1, cs.n128[0] + cs.n128[1] * nk * n128);
   // the persistent four-phase forms: whole rounds, then the rest split along K and met in the launch
   if (M >= 512 && slabs && counters) {
-    auto persistent = [&](int code, const Tile& t, float e, float f, float g, float h) {
+    auto persistent = [&](int code, const Tile& t, const float (&x)[4]) {
       if (N % t.bn != 0) return;
       const int n = over(M, 256) * (N / t.bn), rest = n % cus;
       if (rest == 0) return;
       int S = cus / rest > 8 ? 8 : cus / rest;
       while (S > 1 && nk / S < 4) --S;
-      take(code, 0, (n / cus) * (t.a + t.b * nk) + e + f * nk / S + (S > 1 ? g + h * (S - 1) : 0.f));
+      take(code, 0, (n / cus) * (t.a + t.b * nk) + x[0] + x[1] * nk / S + (S > 1 ? x[2] + x[3] * (S - 1) : 0.f));
     };
-    persistent(1025, tiles[0], 13.4f, 1.61f, 13.6f, 2.4f);
-    persistent(769, tiles[1], 10.6f, 1.07f, 5.6f, 1.5f);
+    persistent(1025, cs.tiles[0], cs.p256);
+    persistent(769, cs.tiles[1], cs.p128);
   }
   return best;
 }
