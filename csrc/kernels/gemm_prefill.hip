@@ -9,8 +9,7 @@
 //   * W: the packed layout Wp[nt][kt][lane][8] IS the MFMA A-fragment order, so one 1 KiB
 //     piece (one 16-column tile x one k-step) lands lane-linear and every wave reads its
 //     fragments back with conflict-free ds_read_b128 (lane l at +16 l) — no swizzle needed;
-//   * x: each 1 KiB piece gathers the B fragments of 16 rows x 32 k (per-lane source address =
-//     row m0 + (l & 15), column 8 (l >> 4)), so the LDS image is fragment-major too.
+//   * x: each 1 KiB piece is 8 rows x 64 k, eight consecutive lanes to a 128-B line (x_piece_row).
 // Pipeline (cdna_hip_programming.md §5 'glds vs register staging', first row): the stage t+1
 // DMA is issued before stage t's ds_reads + MFMAs, one vmcnt(0) + barrier per stage.
 // Block tile BM x BN over 4 waves (2 x 2), wave tile (BM/2) x (BN/2) in 16x16x32 bf16 MFMAs,
@@ -34,6 +33,23 @@ __device__ __forceinline__ float sumsq8(uint4 v, float acc) {
   acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.y), __builtin_bit_cast(p4_bf2, v.y), acc, false);
   acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.z), __builtin_bit_cast(p4_bf2, v.z), acc, false);
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.w), __builtin_bit_cast(p4_bf2, v.w), acc, false);
+}
+
+// ---- x in LDS: a 16-row x 64-k tile is two 1 KiB pieces of 8 rows ----
+// Eight consecutive lanes of the DMA fetch one row's whole 128-B line. (Gathering MFMA fragments directly, 64 lanes on 16 rows of
+// 64 B each, kept the CU's address path busy four times as long and bounded every tile shape at 20 to 22 B per clock and CU: 1536 x
+// 8960 at 2048 rows as 128 x 128 tiles 115 -> 88 us, 4096 x 4096 as 256 x 128 92 -> 73, 28672 x 4096 as 256 x 128 545 -> 476.) LDS-DMA
+// writes lane-linear, so the 16-B chunks of a row are permuted at the source: chunk c of row r lies at c ^ x_swz(r), which spreads the
+// 16 rows of a fragment read over all banks (SQ_LDS_BANK_CONFLICT 0).
+__device__ __forceinline__ int x_swz(int r) { return (r >> 1) & 7; }
+__device__ __forceinline__ int x_piece_row(int tile_row0, int half, int lane, int M) {
+  const int row = tile_row0 + 8 * half + (lane >> 3);
+  return row < M ? row : M - 1;  // rows past M repeat row M - 1 (never stored)
+}
+__device__ __forceinline__ int x_piece_col(int half, int lane) { return ((lane & 7) ^ x_swz(8 * half + (lane >> 3))) * 8; }
+__device__ __forceinline__ int x_frag_off(int ks, int lane) {
+  const int r = lane & 15;
+  return r * 128 + (((4 * ks + (lane >> 4)) ^ x_swz(r)) << 4);
 }
 
 template <int BM, int BN, int EPI, int NORM, int NTB>
@@ -76,14 +92,13 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill_kernel(GemmParams p) {
       step[i] = KS * 1024;
     } else {
       const int g = f - WTN * KS;
-      const int mt = g / KS, ks = g % KS;
-      int row = m0 + mt * 16 + (lane & 15);
-      row = row < p.M ? row : p.M - 1;  // rows past M repeat row M-1 (never stored)
-      src[i] = reinterpret_cast<const char*>(p.x + (size_t)row * p.lda + kst0 * 64 + ks * 32 + 8 * (lane >> 4));
+      const int row = x_piece_row(m0 + (g >> 1) * 16, g & 1, lane, p.M);
+      src[i] = reinterpret_cast<const char*>(p.x + (size_t)row * p.lda + kst0 * 64 + x_piece_col(g & 1, lane));
       step[i] = 64 * 2;
     }
   }
   const uint32_t lds0 = lds_addr_of(smem);
+  const int xo[2] = {x_frag_off(0, lane), x_frag_off(1, lane)};
   auto issue = [&](int stage, int buf) {
 #pragma unroll
     for (int i = 0; i < PPW; ++i) {
@@ -115,7 +130,7 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill_kernel(GemmParams p) {
         wa[a] = *reinterpret_cast<const uint4*>(sb + ((wn * NT + a) * KS + ks) * 1024 + lane * 16);
 #pragma unroll
       for (int b = 0; b < MT; ++b)
-        xb[b] = *reinterpret_cast<const uint4*>(sb + (WTN * KS + (wm * MT + b) * KS + ks) * 1024 + lane * 16);
+        xb[b] = *reinterpret_cast<const uint4*>(sb + (WTN + wm * MT + b) * 2048 + xo[ks]);
       if constexpr (NORM == 2) {
 #pragma unroll
         for (int b = 0; b < MT; ++b) {
@@ -193,7 +208,7 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill_kernel(GemmParams p) {
 template <int BM, int BN, int WM, int WN, int NS, int EPI, int NORM, int NTB, int SCHED = 0, int KS = 2>
 __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_prefill2_kernel(GemmParams p) {
   constexpr int NW = WM * WN;
-  // KS: 32-deep k-steps per stage (BK = 32 KS)
+  static_assert(KS == 2, "stages of 64 k: an x tile's two pieces are its row halves");
   constexpr int WTN = BN / 16, XTM = BM / 16;  // 16-wide tiles per block
   constexpr int NT = WTN / WN, MT = XTM / WM;  // per wave
   constexpr int PIECES = (WTN + XTM) * KS;     // 1 KiB pieces per stage
@@ -226,14 +241,13 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_prefill2_kernel(GemmPara
       step[i] = KS * 1024;
     } else {
       const int g = f - WTN * KS;
-      const int mt = g / KS, ks = g % KS;
-      int row = m0 + mt * 16 + (lane & 15);
-      row = row < p.M ? row : p.M - 1;
-      src[i] = reinterpret_cast<const char*>(p.x + (size_t)row * p.lda + kst0 * 32 * KS + ks * 32 + 8 * (lane >> 4));
-      step[i] = 32 * KS * 2;
+      const int row = x_piece_row(m0 + (g >> 1) * 16, g & 1, lane, p.M);
+      src[i] = reinterpret_cast<const char*>(p.x + (size_t)row * p.lda + kst0 * 64 + x_piece_col(g & 1, lane));
+      step[i] = 64 * 2;
     }
   }
   const uint32_t lds0 = lds_addr_of(smem);
+  const int xo[2] = {x_frag_off(0, lane), x_frag_off(1, lane)};
   auto issue_part = [&](int stage, int buf, int i0, int i1) {
     const int st = stage < nk ? stage : nk - 1;  // past the end: a clamped duplicate, never read
 #pragma unroll
@@ -274,7 +288,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_prefill2_kernel(GemmPara
         wall[ks][a] = *reinterpret_cast<const uint4*>(sb + ((wn * NT + a) * KS + ks) * 1024 + lane * 16);
 #pragma unroll
       for (int b = 0; b < MT; ++b)
-        xall[ks][b] = *reinterpret_cast<const uint4*>(sb + (WTN * KS + (wm * MT + b) * KS + ks) * 1024 + lane * 16);
+        xall[ks][b] = *reinterpret_cast<const uint4*>(sb + (WTN + wm * MT + b) * 2048 + xo[ks]);
     }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
@@ -385,6 +399,7 @@ __device__ __forceinline__ void p4_kloop(const GemmParams& p, char* smem, int wi
   int step[PPW];
   uint32_t dst[PPW];
   const uint32_t lds0 = lds_addr_of(smem);
+  const int xo[2] = {x_frag_off(0, lane), x_frag_off(1, lane)};
 #pragma unroll
   for (int i = 0; i < PPW; ++i) {
     int e, isw, t;
@@ -416,9 +431,8 @@ __device__ __forceinline__ void p4_kloop(const GemmParams& p, char* smem, int wi
       step[i] = KS * 1024;
       dst[i] = (uint32_t)((t * KS + ks) * 1024);
     } else {
-      int row = m0 + t * 16 + (lane & 15);
-      row = row < p.M ? row : p.M - 1;
-      src[i] = reinterpret_cast<const char*>(p.x + (size_t)row * p.lda + kst0 * 64 + ks * 32 + 8 * (lane >> 4));
+      const int row = x_piece_row(m0 + t * 16, ks, lane, p.M);  // (an x tile's two pieces are its row halves, see x_piece_row)
+      src[i] = reinterpret_cast<const char*>(p.x + (size_t)row * p.lda + kst0 * 64 + x_piece_col(ks, lane));
       step[i] = 64 * 2;
       dst[i] = (uint32_t)((WTN * KS + t * KS + ks) * 1024);
     }
@@ -445,7 +459,7 @@ __device__ __forceinline__ void p4_kloop(const GemmParams& p, char* smem, int wi
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
       for (int b = 0; b < 2; ++b)
-        xf[ks][b] = *reinterpret_cast<const uint4*>(sb + (WTN * KS + (wc * 4 + half * 2 + b) * KS + ks) * 1024 + lane * 16);
+        xf[ks][b] = *reinterpret_cast<const uint4*>(sb + (WTN + wc * 4 + half * 2 + b) * 2048 + xo[ks]);
     // folded RMSNorm: x^2 of the rows in packed bf16 dot products (v_dot2_f32_bf16: one op per 2
     // elements, no unpack), and only in wave row 0 — wave row 1 reads the same x tiles; the row
     // sums reach it through LDS in p4_finish. (The unpack + FMA form in both wave rows cost the
