@@ -198,9 +198,9 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
     launch_dispatch<false>(to_params(h), h, st);
     return;
   }
-  // (65 .. 127 rows: the same forms once the matrix is large enough to be streamed in slices; 1536 x 8960 at 96 rows
-  // 42 -> 19 us, 1024 x 4096 20 -> 13)
-  const bool longer = g.M >= 128 || (g.M > 64 && rows16 && (g.K >= 2560 || (int64_t)g.N * g.K >= 8 * 1024 * 1024));
+  // (65 .. 127 rows: the same forms unless K is short, where the kernels below are ahead: 512 x 512 at 80 rows 8.2, 9.2 us, 1024 x 512 8.4,
+  // 9.0; from there on the forms: 1024 x 1024 at 96 rows 12.1 -> 10.6, 1536 x 1536 at 96 14.7 -> 12.3, 1536 x 8960 at 96 42 -> 19)
+  const bool longer = g.M >= 128 || (g.M > 64 && rows16 && g.K >= 1024);
   if (g.path == 1 || (g.path == 0 && longer && g.waves == 0 && g.splitk == 0)) {
     GemmArgs h = g;
     if (g.path == 0) h.ntb = 0;

@@ -21,36 +21,9 @@
 // column panel run back to back on one XCD (one HBM read of the panel per XCD L2).
 #include <cstdlib>
 
-#include "gemm_epilogue.h"
+#include "gemm_prompt.h"
 
 namespace vgate {
-
-// x^2 of 8 bf16 (one B fragment) into acc: 4 packed dot products (v_dot2_f32_bf16), no unpack — the
-// folded RMSNorm's row sums ride along the MFMA loop at a quarter of the unpack + FMA VALU cost
-typedef __bf16 p4_bf2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float sumsq8(uint4 v, float acc) {
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.x), __builtin_bit_cast(p4_bf2, v.x), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.y), __builtin_bit_cast(p4_bf2, v.y), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.z), __builtin_bit_cast(p4_bf2, v.z), acc, false);
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.w), __builtin_bit_cast(p4_bf2, v.w), acc, false);
-}
-
-// ---- x in LDS: a 16-row x 64-k tile is two 1 KiB pieces of 8 rows ----
-// Eight consecutive lanes of the DMA fetch one row's whole 128-B line. (Gathering MFMA fragments directly, 64 lanes on 16 rows of
-// 64 B each, kept the CU's address path busy four times as long and bounded every tile shape at 20 to 22 B per clock and CU: 1536 x
-// 8960 at 2048 rows as 128 x 128 tiles 115 -> 88 us, 4096 x 4096 as 256 x 128 92 -> 73, 28672 x 4096 as 256 x 128 545 -> 476.) LDS-DMA
-// writes lane-linear, so the 16-B chunks of a row are permuted at the source: chunk c of row r lies at c ^ x_swz(r), which spreads the
-// 16 rows of a fragment read over all banks (SQ_LDS_BANK_CONFLICT 0).
-__device__ __forceinline__ int x_swz(int r) { return (r >> 1) & 7; }
-__device__ __forceinline__ int x_piece_row(int tile_row0, int half, int lane, int M) {
-  const int row = tile_row0 + 8 * half + (lane >> 3);
-  return row < M ? row : M - 1;  // rows past M repeat row M - 1 (never stored)
-}
-__device__ __forceinline__ int x_piece_col(int half, int lane) { return ((lane & 7) ^ x_swz(8 * half + (lane >> 3))) * 8; }
-__device__ __forceinline__ int x_frag_off(int ks, int lane) {
-  const int r = lane & 15;
-  return r * 128 + (((4 * ks + (lane >> 4)) ^ x_swz(r)) << 4);
-}
 
 template <int BM, int BN, int EPI, int NORM, int NTB>
 __global__ __launch_bounds__(256, 2) void gemm_prefill_kernel(GemmParams p) {
@@ -906,92 +879,88 @@ static void launch_prefill_cfg(const GemmParams& p, int nz, hipStream_t st) {
 // Split-K partials leave with non-temporal stores: dirty fp32 slabs in L2 are written back at the
 // kernel boundary and held the next launch back 2-4 us (prefill-step timeline, r4).
 //
-// The launcher's own choice of tile and K slices: every form below costs about
-//     rounds x (a + b x K / 64) [+ c + d x MB of partials, the combine launch of a K-split grid]
-// with rounds = blocks over the CUs rounded up (one block of these forms fills a CU), so the cheapest by that sum is taken.
-// a, b, c, d in us, fitted to a sweep of 35 shapes (N 128 .. 28672, K 512 .. 14336) x M 128 .. 2048 on cold weights, rms
-// error 5 to 9 % per form. What the forms trade: a large tile has the highest rate (256 x 256: 1.6 PFLOP/s per full
-// round) and the worst last round; splitting K fills the chip for few tiles and costs a pass over the partials.
-// The times of the taken forms are 0.95 to 1.03 of the best of these forms by the number of rows (geometric means;
-// profiles/prefill_gemm_forms_sweep.txt; the thresholds on block counts used before: 1.31). 64 x 512 and 128 x 320 tiles, which
-// start-up plans may take, would gain 0.2 % at most. 2048 rows, us before -> now: 1536 x 8960 154 -> 86, 1536 x 1536 30 -> 22, 1024 x 4096 60 -> 38,
-// 1024 x 1024 19 -> 14; 256 rows: 1536 x 8960 39 -> 27, 1536 x 1536 15 -> 13.
+// The launcher's own choice of tile and K slices: the cheapest form by a fitted cost (us),
+//     e + a x rounds + b x K-tiles of the busiest CU + w x MB of weights + o x MB of output
+//     [+ c + d x MB of partials: a K-split grid and its combine launch]
+// with rounds = blocks over what the CUs hold, rounded up. A large tile has the highest rate and the worst last round, the small ones
+// the shortest chain; splitting K fills the chip for few tiles and costs a pass over the partials. Fitted (non-negative least squares
+// on relative errors) to 26 shapes (N 512 .. 28672, K 512 .. 14336) x 15 row counts 65 .. 2048 on cold weights, apart with the row
+// scale of a folded norm; rms error 3 to 6 % per form (the persistent ones 11). The choice takes 1.008 of the time of the best form there
+// (geometric mean) and 0.92 of hipBLASLt's; without 64 x 64 1.054, without 128 x 64 1.021, without 128 x 128 1.016, without any other one of
+// them 1.009 to 1.011. us before the four-wave forms (gemm_prompt.h) -> now: 1536 x 1536 at 256 rows 16.6 -> 12.5, 2048 x 1536 at 448
+// 17.1 -> 12.6, 17920 x 1536 at 448 46.8 -> 38.8, 4352 x 1024 at 2048 36.6 -> 30.3, 1024 x 4096 at 1024 32.2 -> 24.0.
 struct PrefillForm {
-  int code;  // tile code (as the forced ones below); 0: leave it to the kernels of gemm_decode.h
+  int code;  // tile code (as the forced ones below)
   int nz;    // K slices
 };
 
-static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool slabs, size_t slab_bytes, bool counters) {
+static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool rows16, bool slabs, size_t slab_bytes, bool counters) {
+  struct Cost {
+    float e, a, b, c, d, w, o;
+  };
   struct Tile {
-    int code, bm, bn;
-    float a, b, c, d;
+    int code, bm, bn, per_cu;
+    Cost cost[2];  // plain, with a folded norm
   };
-  struct Costs {
-    Tile tiles[4];        // 256 x 256 / 256 x 128 four-phase, 128 x 128 (8 waves) / 128 x 64 on four-deep rings
-    float n64[2], n128[2];   // two-deep rings: whole, per K-tile and block of a CU
-    float p256[4], p128[4];  // persistent: the last round whole, per K-tile, and of its K slices
+  static constexpr Tile tiles[] = {
+      {5220, 64, 64, 2, {{6.58f, 0.615f, 0.232f, 2.7f, 0.566f, 0.034f, 0.063f}, {6.96f, 0.657f, 0.238f, 2.73f, 0.514f, 0.035f, 0.105f}}},
+      {5340, 96, 128, 1, {{6.19f, 2.54f, 0.473f, 2.84f, 0.432f, 0.031f, 0.187f}, {7.24f, 2.94f, 0.49f, 1.8f, 0.422f, 0.024f, 0.224f}}},
+      {5380, 96, 256, 1, {{9.21f, 2.5f, 0.737f, 0.f, 0.f, 0.034f, 0.f}, {11.5f, 2.48f, 0.757f, 0.f, 0.f, 0.02f, 0.f}}},
+      {5580, 160, 256, 1, {{9.64f, 6.38f, 0.948f, 0.f, 0.f, 0.018f, 0.f}, {15.4f, 5.08f, 0.986f, 0.f, 0.f, 0.005f, 0.f}}},
+      {5640, 192, 128, 1, {{8.36f, 3.99f, 0.624f, 0.f, 0.f, 0.012f, 0.139f}, {9.96f, 5.92f, 0.67f, 0.f, 0.f, 0.f, 0.f}}},
+      {5680, 192, 256, 1, {{14.5f, 1.91f, 1.25f, 0.f, 0.f, 0.007f, 0.f}, {19.4f, 1.41f, 1.25f, 0.f, 0.f, 0.f, 0.f}}},
+      {641, 128, 64, 1, {{5.18f, 1.15f, 0.374f, 3.25f, 0.492f, 0.003f, 0.402f}, {5.11f, 1.5f, 0.408f, 3.32f, 0.454f, 0.017f, 0.445f}}},
+      {1281, 128, 128, 1, {{5.48f, 2.17f, 0.52f, 3.05f, 0.42f, 0.012f, 0.362f}, {5.8f, 2.3f, 0.641f, 2.74f, 0.414f, 0.01f, 0.367f}}},
+      {768, 256, 128, 1, {{7.23f, 1.58f, 0.811f, 1.76f, 0.461f, 0.f, 0.408f}, {7.75f, 2.09f, 0.916f, 1.16f, 0.444f, 0.f, 0.414f}}},
+      {1024, 256, 256, 1, {{8.56f, 4.43f, 1.26f, 0.f, 0.458f, 0.f, 0.39f}, {8.52f, 4.65f, 1.39f, 0.f, 0.445f, 0.f, 0.427f}}}};
+  // the persistent four-phase forms: e + b x K-tiles in whole rounds, then r x K-tiles of the rest [+ c + d x (slices - 1): their meeting]
+  struct Persistent {
+    int code, bn;
+    struct {
+      float e, b, r, c, d, w, o;
+    } cost[2];
   };
-  // With the row scale of a folded norm (second set, fitted by itself to 16 shapes at 96 .. 2048 rows) every form sums the squares of its
-  // rows on the way, the more often the narrower its tiles: by the plain costs its choice is 1.06 of the best form (geometric mean at 512
-  // rows), by its own 1.006 (2048 x 1536 at 128 rows 22.6 -> 15.9 us, 1024 x 4096 at 1024 48.4 -> 31.4).
-  static constexpr Costs sets[2] = {{{{1024, 256, 256, 10.2f, 1.33f, 1.5f, 0.49f},
-                                      {768, 256, 128, 7.1f, 1.00f, 1.6f, 0.56f},
-                                      {1281, 128, 128, 5.8f, 0.61f, 2.8f, 0.57f},
-                                      {640, 128, 64, 5.0f, 0.50f, 2.9f, 0.68f}},
-                                     {5.0f, 0.54f}, {6.0f, 0.77f}, {13.4f, 1.61f, 13.6f, 2.4f}, {10.6f, 1.07f, 5.6f, 1.5f}},
-                                    {{{1024, 256, 256, 16.2f, 1.52f, -3.1f, 0.485f},
-                                      {768, 256, 128, 11.7f, 1.13f, -0.8f, 0.506f},
-                                      {1281, 128, 128, 9.0f, 0.705f, 2.4f, 0.395f},
-                                      {640, 128, 64, 7.6f, 0.585f, 3.0f, 0.412f}},
-                                     {10.5f, 0.548f}, {12.0f, 0.78f}, {22.0f, 1.59f, 13.7f, 4.2f}, {15.3f, 1.175f, 6.3f, 2.4f}}};
-  const Costs& cs = sets[norm ? 1 : 0];
+  static constexpr Persistent persistent[] = {
+      {1025, 256, {{0.f, 0.638f, 1.15f, 18.8f, 4.42f, 0.231f, 0.819f}, {0.f, 0.75f, 1.27f, 19.9f, 4.63f, 0.217f, 0.824f}}},
+      {769, 128, {{6.94f, 0.703f, 0.815f, 7.04f, 2.78f, 0.051f, 0.538f}, {7.24f, 0.71f, 0.841f, 7.87f, 2.85f, 0.11f, 0.631f}}}};
   static constexpr int slices[] = {1, 2, 3, 4, 6, 8};
   const int cus = cu_count() > 0 ? cu_count() : 256, nk = K / 64;
-  auto over = [](int64_t x, int y) { return (int)((x + y - 1) / y); };
-  PrefillForm best{64, 1};
-  float cost = 1e30f;
+  const float wmb = 2e-6f * (float)N * (float)K, omb = 2e-6f * (float)M * (float)N;
+  auto over = [](int64_t x, int64_t y) { return (int)((x + y - 1) / y); };
+  PrefillForm best{641, 1};
+  float least = 1e30f;
   auto take = [&](int code, int nz, float t) {
-    if (t < cost) {
-      cost = t;
+    if (t < least) {
+      least = t;
       best = PrefillForm{code, nz};
     }
   };
-  // 64 x 64 tiles, weights in registers (gemm_decode.h): short K, few rows. The cost is gemm_tile3_kernel's. launch_m() runs that from
-  // K = 768 on and from 128 rows or 128 tiles on, and where it runs another kernel, that one is ahead (us, gemm_tile3_kernel / its choice:
-  // 512 x 512 at 2048 rows 8.3, 7.5; 1536 x 8960 at 96 rows without a workspace 53.6, 43.0)
-  if (K % 256 == 0 && N / 16 < 1024) {
-    const int rounds = over((int64_t)over(M, 64) * (N / 64), cus);
-    take(0, 1, norm && K >= 768 ? 5.2f + rounds * (3.58f + 0.591f * nk) : rounds * (4.6f + 0.354f * nk));
-  }
-  for (const Tile& t : cs.tiles) {
-    if (N % t.bn != 0) continue;
+  for (const Tile& t : tiles) {
+    if (N % t.bn != 0 || (t.code >= 5000 && !rows16)) continue;
+    const Cost& x = t.cost[norm ? 1 : 0];
+    const bool sliced = x.d > 0.f && !(t.bm == 256 && M >= 512);  // (the four-phase tiles of long steps are split by the persistent forms)
     for (int nz : slices) {
       const int64_t blocks = (int64_t)over(M, t.bm) * (N / t.bn) * nz;
-      const int rounds = over(blocks, cus);
-      if (nz > 1 && (rounds > 1 || nk / nz < 4 || !slabs || ((size_t)nz * M * N + (size_t)nz * M) * 4 > slab_bytes)) continue;
-      const float mb = (float)nz * M * N * 4e-6f;
-      take(t.code, nz, rounds * (t.a + t.b * over(nk, nz)) + (nz > 1 ? t.c + t.d * mb : 0.f));
+      if (nz > 1 && (!sliced || blocks > 600 || nk / nz < 4 || !slabs || ((size_t)nz * M * N + (size_t)nz * M) * 4 > slab_bytes)) continue;
+      take(t.code, nz, x.e + x.a * over(blocks, (int64_t)cus * t.per_cu) + x.b * over(blocks, cus) * over(nk, nz) + x.w * wmb + x.o * omb +
+                           (nz > 1 ? x.c + x.d * 2.f * nz * omb : 0.f));
     }
   }
-  // two-deep rings, several blocks per CU: the rate of the small tiles without whole rounds
-  const int n64 = over((int64_t)over(M, 128) * (N / 64), cus), n128 = N % 128 == 0 ? over((int64_t)over(M, 128) * (N / 128), cus) : 0;
-  if (n64 > 1) take(64, 1, cs.n64[0] + cs.n64[1] * nk * n64);
-  if (n128 > 1) take(128, 1, cs.n128[0] + cs.n128[1] * nk * n128);
-  // the persistent four-phase forms: whole rounds, then the rest split along K and met in the launch
   if (M >= 512 && slabs && counters) {
-    auto persistent = [&](int code, const Tile& t, const float (&x)[4]) {
-      if (N % t.bn != 0) return;
-      const int n = over(M, 256) * (N / t.bn), rest = n % cus;
-      if (rest == 0) return;
+    for (const Persistent& t : persistent) {
+      const auto& x = t.cost[norm ? 1 : 0];
+      const int n = N % t.bn == 0 ? over(M, 256) * (N / t.bn) : 0, rest = n % cus;
+      if (rest == 0) continue;
       int S = cus / rest > 8 ? 8 : cus / rest;
       while (S > 1 && nk / S < 4) --S;
-      take(code, 0, (n / cus) * (t.a + t.b * nk) + x[0] + x[1] * nk / S + (S > 1 ? x[2] + x[3] * (S - 1) : 0.f));
-    };
-    persistent(1025, cs.tiles[0], cs.p256);
-    persistent(769, cs.tiles[1], cs.p128);
+      take(t.code, 0, x.e + x.b * (n / cus) * nk + x.r * nk / S + (S > 1 ? x.c + x.d * (S - 1) : 0.f) + x.w * wmb + x.o * omb);
+    }
   }
   return best;
 }
+
+template <int EPI, int NORM>
+bool launch_gemm_w4(const GemmParams& p, int code, int nz, hipStream_t st);
 
 // Returns false for shapes the kernels do not take (the caller keeps the N-split tile
 // kernels): K % 64, N % 64, a row gather, the gamma-in-registers RMSNorm mode; and where those are the cheapest form.
@@ -1000,9 +969,10 @@ static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, 
                                hipStream_t st) {
   constexpr int NTB = 1;  // every epilogue works on self-contained 16-column tiles
   if (p.K % 64 != 0 || p.N % 64 != 0 || p.row_idx != nullptr) return false;
+  // the four-wave forms address a block's rows of x by 32-bit offsets and fetch them in 16-B pieces
+  const bool rows16 = reinterpret_cast<uintptr_t>(p.x) % 16 == 0 && p.lda % 8 == 0 && p.lda < (1 << 20) && p.K < (1 << 20);
   if (force_bn == 0 && force_sk == 0) {
-    const PrefillForm f = choose_prefill_form(p.M, p.N, p.K, NORM == 2, p.slabs != nullptr, slab_bytes, p.counters != nullptr);
-    if (f.code == 0) return false;
+    const PrefillForm f = choose_prefill_form(p.M, p.N, p.K, NORM == 2, rows16, p.slabs != nullptr, slab_bytes, p.counters != nullptr);
     force_bn = f.code;
     force_sk = f.nz;
   }
@@ -1022,6 +992,13 @@ static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, 
   while (nz > 1 && nk / nz < 4) --nz;
   const size_t need = ((size_t)nz * p.M * p.N + (size_t)nz * p.M) * 4;
   if (nz > 1 && (p.slabs == nullptr || need > slab_bytes)) nz = 1;
+  if (force_bn >= 5000) {
+    if (!rows16) return false;
+    if (force_sk <= 0) nz = 1;
+    if (!launch_gemm_w4<EPI, NORM>(p, force_bn, nz, st)) return false;
+    if (nz > 1) launch_prefill_reduce<EPI, NORM, 1>(p, nz, st);
+    return true;
+  }
   if (force_bn == 256) {  // forced (tests / sweeps), split-K as chosen above
     if (p.N % 128 != 0) return false;
     launch_prefill2_cfg<EPI, NORM, NTB>(p, nz, st);

@@ -1,0 +1,211 @@
+// Prompt GEMM on four waves, one per SIMD: each computes a quarter (2 x 2) of the block tile, MT x NT MFMA tiles of 16 x 16, so a block
+// is 32 MT rows x 32 NT columns and the sizes between the powers of two come for the asking.
+//
+// What bounds it. A K-tile of 64 asks a CU for (BM + BN) x 128 B from L2 (25 to 30 B per clock and CU with all of them at it: 64 x 64
+// tiles 0.25 us a K-tile for the loads alone, 0.31 in all), for (MT + NT) x 16 KiB of fragment reads (108 B per clock) and for BM x BN / 32
+// matrix cycles; from 160 x 256 on the matrix cores bound it, at the clock that their power leaves (1.5 to 2.1 GHz on random data: a K-tile
+// of 256 x 256 1.1 to 1.4 us at best, 1.6 here as in the four-phase kernel of gemm_prefill.hip). So:
+//   * a wave reads its fragments once per k-step into registers, 32 B of LDS per MFMA where eight waves of half the size read 48;
+//   * the reads of a k-step are under way during the MFMAs of the one before (two register sets), the DMA of a K-tile during the NS - 1
+//     before it, and one barrier per K-tile stands between its two k-steps, where every operand of the second is in registers already;
+//   * accumulators stay in AGPRs (mfma_acc), addresses in SGPRs (blds16): the loop is MFMA, ds_read and DMA only.
+// us, eight-wave forms -> these (MI355X, cold weights): 64 x 64 tiles 2048 x 1536 at 448 rows 17.1 -> 12.6, 1536 x 1536 at 256 16.6 -> 12.5,
+// 1024 x 4096 at 1024 32.2 -> 24.0; 160 x 256 17920 x 1536 at 448 46.8 -> 38.8, 4352 x 1024 at 2048 36.6 -> 30.3; 192 x 128 17920 x 1536 at
+// 1024 87 -> 80. As 256 x 256 tiles it is no faster than the four-phase kernel (28672 x 4096 at 2048 rows 445, 449), which keeps those.
+#pragma once
+#include <type_traits>
+
+#include "gemm_epilogue.h"
+
+namespace vgate {
+
+// x^2 of 8 bf16 (one B fragment) into acc: 4 packed dot products (v_dot2_f32_bf16), no unpack — the
+// folded RMSNorm's row sums ride along the MFMA loop at a quarter of the unpack + FMA VALU cost
+typedef __bf16 p4_bf2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float sumsq8(uint4 v, float acc) {
+  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.x), __builtin_bit_cast(p4_bf2, v.x), acc, false);
+  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.y), __builtin_bit_cast(p4_bf2, v.y), acc, false);
+  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.z), __builtin_bit_cast(p4_bf2, v.z), acc, false);
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.w), __builtin_bit_cast(p4_bf2, v.w), acc, false);
+}
+
+// ---- x in LDS: a 16-row x 64-k tile is two 1 KiB pieces of 8 rows ----
+// Eight consecutive lanes of the DMA fetch one row's whole 128-B line. (Gathering MFMA fragments directly, 64 lanes on 16 rows of
+// 64 B each, kept the CU's address path busy four times as long and bounded every tile shape at 20 to 22 B per clock and CU: 1536 x
+// 8960 at 2048 rows as 128 x 128 tiles 115 -> 88 us, 4096 x 4096 as 256 x 128 92 -> 73, 28672 x 4096 as 256 x 128 545 -> 476.) LDS-DMA
+// writes lane-linear, so the 16-B chunks of a row are permuted at the source: chunk c of row r lies at c ^ x_swz(r), which spreads the
+// 16 rows of a fragment read over all banks (SQ_LDS_BANK_CONFLICT 0).
+__device__ __forceinline__ int x_swz(int r) { return (r >> 1) & 7; }
+__device__ __forceinline__ int x_piece_row(int tile_row0, int half, int lane, int M) {
+  const int row = tile_row0 + 8 * half + (lane >> 3);
+  return row < M ? row : M - 1;  // rows past M repeat row M - 1 (never stored)
+}
+__device__ __forceinline__ int x_piece_col(int half, int lane) { return ((lane & 7) ^ x_swz(8 * half + (lane >> 3))) * 8; }
+__device__ __forceinline__ int x_frag_off(int ks, int lane) {
+  const int r = lane & 15;
+  return r * 128 + (((4 * ks + (lane >> 4)) ^ x_swz(r)) << 4);
+}
+
+// LDS-DMA through a buffer descriptor: 16 B per lane from base + voff + soff to lds + 16 lane (inline asm and vmcnt by the caller, as
+// glds16; no 64-bit address per piece: a wave that issues alone on its SIMD has no slots for those)
+__device__ __forceinline__ void blds16(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
+  unsigned keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory");
+}
+__device__ __forceinline__ u32x4 rsrc_words(const void* base) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xffffu)), 0x7fffffffu, 0x00020000u};
+}
+
+// acc += W(A) . X(B) on an accumulator that stays in its AGPRs: up to 256 of them are the whole file, and with the builtin (whose result is
+// another register than its addend) the allocator shuffles them through VGPRs all the way. The operands come from LDS (waited for by
+// the compiler, as any asm input); what follows the last one and reads the accumulators calls mfma_settle() first.
+__device__ __forceinline__ void mfma_acc(f32x4& acc, const uint4& w, const uint4& x) {
+  asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(as_bf16x8(w)), "v"(as_bf16x8(x)));
+}
+
+template <int MT, int NT>
+struct W4 {  // geometry: block (32 MT) rows x (32 NT) columns, stages of 64 k
+  static constexpr int BM = 32 * MT, BN = 32 * NT;
+  static constexpr int PPW = MT + NT;             // 1 KiB pieces per wave and stage
+  static constexpr int STAGE = 4 * PPW * 1024;
+};
+
+// NS: stages in LDS. K-split (grid.y), epilogues and the order of the blocks as in gemm_prefill.hip.
+template <int MT, int NT, int NS, int EPI, int NORM>
+__global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmParams p) {
+  using G = W4<MT, NT>;
+  constexpr int PPW = G::PPW, STAGE = G::STAGE, WPC = NT;  // W pieces of a wave: NT (NT / 2 tiles x 2 k-steps)
+  constexpr int XB = 4 * NT * 1024;                        // x tiles of a stage lie behind its W tiles
+  static_assert(NT % 2 == 0 && (MT * NT) % 4 == 0 && NS >= 2 && (NS - 1) * PPW < 64, "pieces per wave, groups of four MFMAs, vmcnt");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  TLScope tl_scope(p.dbg_ts);
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wid >> 1, wn = wid & 1;
+  const int KT = p.K >> 5, nk_all = p.K >> 6;
+  const int z = blockIdx.y, nz = gridDim.y;
+  const int kst0 = (nk_all * z) / nz, nk = (nk_all * (z + 1)) / nz - kst0;
+  const int mblocks = (p.M + G::BM - 1) / G::BM;
+  const int nwg = gridDim.x, orig = blockIdx.x, xcd = orig & 7, q = nwg >> 3, r = nwg & 7;
+  const int wgid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (orig >> 3);
+  // groups of up to 8 row blocks, inside a group rows fastest: the blocks that run together on an XCD share few panels of both operands
+  // (rows fastest over all of them, 64 x 64 tiles: 1024 x 4096 at 2048 rows 44.5 -> 36.2 us; a group of 2, 4 or 8 is the same)
+  const int per = 8 * (p.N / G::BN), grp = wgid / per, in = wgid - grp * per, gm = min(8, mblocks - 8 * grp);
+  const int m0 = (8 * grp + in % gm) * G::BM;
+  const int nt_blk = (in / gm) * (2 * NT);
+  const u32x4 wrs = rsrc_words(p.wp + ((size_t)nt_blk * KT + 2 * kst0) * 64);
+  const u32x4 xrs = rsrc_words(p.x + (size_t)m0 * p.lda + kst0 * 64);
+  const uint32_t wvo = lane * 16;
+  uint32_t xvo[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int g = wid * MT + i;
+    xvo[i] = (uint32_t)(x_piece_row(m0 + (g >> 1) * 16, g & 1, lane, p.M) - m0) * (uint32_t)p.lda * 2u + (uint32_t)x_piece_col(g & 1, lane) * 2u;
+  }
+  const uint32_t lds0 = lds_addr_of(smem);
+  const uint32_t wrow = (uint32_t)KT * 1024u, wso0 = (uint32_t)wid * (NT / 2) * wrow;
+  // piece i of this wave's share of `stage` into `buf`
+  auto issue_piece = [&](int i, int st, int buf) {
+    if (i < WPC) blds16(wrs, wvo, wso0 + (uint32_t)(i >> 1) * wrow + (uint32_t)(2 * st + (i & 1)) * 1024u,
+                        lds0 + buf * STAGE + (uint32_t)(wid * NT + i) * 1024u);
+    else blds16(xrs, xvo[i - WPC], (uint32_t)st * 128u, lds0 + buf * STAGE + XB + (uint32_t)(wid * MT + i - WPC) * 1024u);
+  };
+  f32x4 acc[NT][MT];
+#pragma unroll
+  for (int a = 0; a < NT; ++a)
+#pragma unroll
+    for (int b = 0; b < MT; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float ss[MT];
+#pragma unroll
+  for (int b = 0; b < MT; ++b) ss[b] = 0.f;
+  uint4 wf[2][NT], xf[2][MT];
+  const int wlo = lane * 16 + wn * NT * 2048, xlo[2] = {XB + wm * MT * 2048 + x_frag_off(0, lane), XB + wm * MT * 2048 + x_frag_off(1, lane)};
+  // fragment read rd (0: W tile 0, 1 .. MT: x, then the other W tiles: the order in which a phase needs them)
+  auto read_frag = [&](int rd, int ks, const char* sb) {
+    if (rd == 0) wf[ks][0] = *reinterpret_cast<const uint4*>(sb + wlo + ks * 1024);
+    else if (rd <= MT) xf[ks][rd - 1] = *reinterpret_cast<const uint4*>(sb + xlo[ks] + (rd - 1) * 2048);
+    else wf[ks][rd - MT] = *reinterpret_cast<const uint4*>(sb + wlo + (rd - MT) * 2048 + ks * 1024);
+  };
+  constexpr int GR = MT * NT / 4, RD = MT + NT;
+  constexpr int HG = GR > 1 ? GR / 2 : 1, RPG = (RD + HG - 1) / HG;  // reads per group: done by the middle of the phase
+  // one phase: the MFMAs of k-step ks in groups of four, between them the reads of the other k-step (from sb) and, if `dma`, the next
+  // stage's pieces
+  auto phase = [&](auto ksc, const char* sb, auto dmac, int st, int buf) {
+    constexpr int ks = decltype(ksc)::value, dma = decltype(dmac)::value;
+#pragma unroll
+    for (int g = 0; g < GR; ++g) {
+#pragma unroll
+      for (int u = 0; u < RPG; ++u)
+        if (g * RPG + u < RD) read_frag(g * RPG + u, ks ^ 1, sb);
+      if constexpr (dma) {
+#pragma unroll
+        for (int i = (g * PPW) / GR; i < ((g + 1) * PPW) / GR; ++i) issue_piece(i, st, buf);
+      }
+#pragma unroll
+      for (int e = 4 * g; e < 4 * g + 4; ++e) {
+        const int a = e / MT, b = e % MT;
+        if constexpr (NORM == 2)
+          if (a == NT / 2) ss[b] = sumsq8(xf[ks][b], ss[b]);
+        mfma_acc(acc[a][b], wf[ks][a], xf[ks][b]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  using C0 = std::integral_constant<int, 0>;
+  using C1 = std::integral_constant<int, 1>;
+#pragma unroll
+  for (int s0 = 0; s0 < NS; ++s0)
+#pragma unroll
+    for (int i = 0; i < PPW; ++i) issue_piece(i, s0 < nk ? s0 : nk - 1, s0);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * PPW) : "memory");
+#pragma unroll
+  for (int rd = 0; rd < RD; ++rd) read_frag(rd, 0, smem);
+  int buf = 0;
+  for (int t = 0; t < nk; ++t) {
+    const char* sb = smem + buf * STAGE;
+    const int nb = buf + 1 == NS ? 0 : buf + 1;
+    phase(C0{}, sb, C0{}, 0, 0);
+    // this stage is read (its second k-step is in registers), the next one has landed: both for every wave
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * PPW) : "memory");
+    const int st = t + NS < nk ? t + NS : nk - 1;  // past the end: clamped duplicates, never used
+    phase(C1{}, smem + nb * STAGE, C1{}, st, buf);
+    buf = nb;
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");  // the trailing duplicates
+#pragma unroll
+  for (int a = 0; a < NT; ++a)
+#pragma unroll
+    for (int b = 0; b < MT; ++b) asm volatile("" : "+a"(acc[a][b]));
+  float* part = p.slabs + (size_t)z * p.M * p.N;
+  float* ssq = p.slabs + (size_t)nz * p.M * p.N + (size_t)z * p.M;
+#pragma unroll
+  for (int b = 0; b < MT; ++b) {
+    const int m = m0 + (wm * MT + b) * 16 + (lane & 15);
+    float sc = 1.f, s2 = 0.f;
+    if constexpr (NORM == 2) {
+      s2 = ss[b];
+      s2 += xor16(s2);
+      s2 += xor32(s2);
+      sc = rsqrtf(s2 / (float)p.K + p.eps);
+    }
+    if (nz > 1) {  // fp32 partial of this K slice, as the other forms leave it for prefill_reduce_kernel
+      if (m < p.M) {
+        if (NORM == 2 && wn == 0 && nt_blk == 0 && lane < 16) ssq[m] = s2;
+#pragma unroll
+        for (int a = 0; a < NT; ++a)
+          __builtin_nontemporal_store(acc[a][b], reinterpret_cast<f32x4*>(part + (size_t)m * p.N + (nt_blk + wn * NT + a) * 16 + 4 * (lane >> 4)));
+      }
+    } else {
+#pragma unroll
+      for (int a = 0; a < NT; ++a) {
+        f32x4 v[1] = {acc[a][b] * sc};
+        epilogue<1, EPI, false>(p, v, m, nt_blk + wn * NT + a, 4 * (lane >> 4), EpiPre<1>{}, m < p.M);
+      }
+    }
+  }
+}
+
+}  // namespace vgate

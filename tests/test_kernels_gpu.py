@@ -1196,6 +1196,28 @@ def test_prefill_lds_gemm_all_epilogues(M, bn, sk):
     assert _rel_err(kc, kc2) < 2e-2 and _rel_err(vc, vc2) < 2e-2
 
 
+@pytest.mark.parametrize("M,bn,sk", [(M, bn, sk) for bn in (5220, 5340, 5380, 5580, 5640, 5680) for M, sk in
+                                     ((1, 1), (65, 3), (97, 1), (577, 1), (2049, 1))])
+def test_prefill_four_wave_tiles(M, bn, sk):
+    """The four-wave tiles (gemm_prompt.h) through every epilogue, one row, a row past a tile and past a group of eight row blocks,
+    K in slices: the references and bounds of the other tiles."""
+    test_prefill_lds_gemm_all_epilogues(M, bn, sk)
+
+
+@pytest.mark.parametrize("bn", [5220, 5340, 5380, 5580, 5640, 5680])
+@pytest.mark.parametrize("K", [64, 128, 448])
+def test_prefill_four_wave_tiles_short_k(bn, K):
+    """Fewer K-tiles than the ring has stages (the rest are duplicates that nothing reads), rows of a wider matrix, fp32 output."""
+    torch.manual_seed(K + bn)
+    M, N = 130, 256
+    x = torch.randn(M, K + 72, device=DEV).bfloat16()[:, :K]
+    w = (torch.randn(N, K, device=DEV) / math.sqrt(K)).bfloat16()
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops.native().gemm(x, ops.Linear(w).wp, N, K, out, 1, ws=ops.workspace(DEV), path=1, ntb=bn, splitk=1)
+    # fp32 sums of bf16 products: K roundings of 2^-24 at most, against 64 bits
+    assert _rel_err(out, x.double() @ w.double().t()) < K * 2.0 ** -24
+
+
 @pytest.mark.parametrize("M", [200, 448, 640])
 @pytest.mark.parametrize("bn,sk", [(2560, 0), (2561, 0), (2560, 2), (2561, 3)])
 def test_prefill_wide_tiles(M, bn, sk):

@@ -658,19 +658,14 @@ def _plan_bucket(plan: dict, M: int):
 
 
 # (tile code, K slices) candidates of the prefill kernels (csrc/kernels/gemm_prefill.hip
-# launch_prefill_epi): 0 = the launcher's heuristic, 64 / 128 = 128 x 64 / 128 x 128 tiles,
-# 256 = 256 x 128 3-deep ring, 768 / 1024 = the 4-phase 256 x 128 / 256 x 256 kernels
-PREFILL_CANDIDATES = [(0, 0), (64, 0), (128, 0), (128, 2), (128, 4), (256, 0), (256, 4), (256, 6), (768, 0),
-                      (768, 2), (768, 3), (768, 4), (768, 6), (1024, 0), (1024, 2), (1024, 3), (1024, 4),
+# launch_prefill_epi): 0 = the launcher's own choice, 5000 + 100 MT + 10 NT = the four-wave tiles of 32 MT rows x
+# 32 NT columns (gemm_prompt.h), 768 / 1024 = the 4-phase 256 x 128 / 256 x 256 kernels, 1025 / 769 = their
+# persistent forms (one block per CU, whole rounds of tiles + the last round K-split and met in-launch)
+PREFILL_CANDIDATES = [(0, 0), (5220, 1), (5220, 2), (5220, 3), (5340, 1), (5340, 2), (5340, 4), (5580, 1), (5640, 1),
+                      (768, 1), (768, 2), (768, 3), (768, 4), (768, 6), (1024, 1), (1024, 2), (1024, 3), (1024, 4),
                       (1024, 6), (1025, 0), (769, 0)]
-# (1025 / 769: the persistent forms of the 4-phase 256 x 256 / 256 x 128 kernel — one block per CU,
-# whole rounds of tiles + the last round K-split and met in-launch; gemm_prefill.hip
-# gemm_prefill4sk_kernel)
-# 128-row tiles on a 4-deep ring, one block per CU (128 x 128 / 128 x 64, 4 or 8 waves): timed for
-# 64 < M <= 1024 only, where the grid of the 2-deep-ring tile is one or two partial rounds
-# + the wide-N tiles 64 x 512 / 128 x 320 (gate_up at 320 / 448 rows: 245 / 224 blocks, 35 vs 44-64 us)
-PREFILL_RING_CANDIDATES = ([(t, s) for t in (1280, 1281, 640, 641) for s in (0, 2, 3)]
-                           + [(2560, 0), (2561, 0)])
+# smaller tiles, timed for 64 < M <= 1024 only: 128 x 128 / 128 x 64 on 4-deep rings, one block per CU
+PREFILL_RING_CANDIDATES = [(t, s) for t in (1281, 641) for s in (1, 2, 3)] + [(5220, 4), (5380, 1)]
 # medium-M kernel (csrc/kernels/gemm_mid.hip, 16 < M <= 64) candidates, encoded as tile code
 # MID_BASE - W (W tiles = waves per block) and K slices (0 = its heuristic)
 MID_BASE = -10
@@ -721,7 +716,7 @@ MEDIUM_DEFAULT = (-1, -1)  # medium-M plan entry: keep the default (decode / til
 
 # bump whenever the MEANING of a stored plan changes on the Python side (the _plan_kw encoding of a
 # (tile, K slices) code, MID_BASE, the tuner margin): a cached plan set is keyed on this too
-PLAN_FORMAT = 3  # 3: candidates timed with the layer's folded-norm row scale
+PLAN_FORMAT = 4  # 4: the four-wave tiles
 TUNE_MARGIN = 0.05
 LONG_M, LONG_MARGIN = 1024, 0.02  # the margin for M >= LONG_M buckets
 
