@@ -222,6 +222,7 @@ void launch_awq_gemm(const GemmArgs& g, hipStream_t st) {
   if (g.path == 0 && ((g.ntb == 0 && g.waves == 0) || (g.ntb <= -12 && g.ntb >= -14)) && launch_awq_kx(g, st)) return;
   // mixed prefill + decode steps (16 < M <= 64) on the int4 medium kernel (path 2)
   if (g.path == 2 && launch_awq_mid(g, st)) return;
+  if (g.path == 5 && launch_q4_prompt(g, st)) return;
   launch_dispatch<true>(to_params(g), g, st);
 }
 

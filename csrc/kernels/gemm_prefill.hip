@@ -892,6 +892,7 @@ static void launch_prefill_cfg(const GemmParams& p, int nz, hipStream_t st) {
 struct PrefillForm {
   int code;  // tile code (as the forced ones below)
   int nz;    // K slices
+  float us;  // its cost
 };
 
 static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool rows16, bool slabs, size_t slab_bytes, bool counters) {
@@ -927,13 +928,9 @@ static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool rows
   const int cus = cu_count() > 0 ? cu_count() : 256, nk = K / 64;
   const float wmb = 2e-6f * (float)N * (float)K, omb = 2e-6f * (float)M * (float)N;
   auto over = [](int64_t x, int64_t y) { return (int)((x + y - 1) / y); };
-  PrefillForm best{641, 1};
-  float least = 1e30f;
+  PrefillForm best{641, 1, 1e30f};
   auto take = [&](int code, int nz, float t) {
-    if (t < least) {
-      least = t;
-      best = PrefillForm{code, nz};
-    }
+    if (t < best.us) best = PrefillForm{code, nz, t};
   };
   for (const Tile& t : tiles) {
     if (N % t.bn != 0 || (t.code >= 5000 && !rows16)) continue;
@@ -957,6 +954,10 @@ static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool rows
     }
   }
   return best;
+}
+
+float prefill_cost_us(int M, int N, int K, bool norm, size_t slab_bytes) {
+  return N % 64 == 0 && K % 64 == 0 ? choose_prefill_form(M, N, K, norm, true, slab_bytes > 0, slab_bytes, slab_bytes > 0).us : 1e30f;
 }
 
 template <int EPI, int NORM>

@@ -60,8 +60,9 @@ __device__ __forceinline__ u32x4 rsrc_words(const void* base) {
 }
 
 // acc += W(A) . X(B) on an accumulator that stays in its AGPRs: up to 256 of them are the whole file, and with the builtin (whose result is
-// another register than its addend) the allocator shuffles them through VGPRs all the way. The operands come from LDS (waited for by
-// the compiler, as any asm input); what follows the last one and reads the accumulators calls mfma_settle() first.
+// another register than its addend) the allocator shuffles them through VGPRs all the way. The compiler does not see an MFMA here, so the
+// waits that it would put around one are the caller's: operands come from LDS (waited for as any asm input) or, written by the VALU, with
+// two wait states between; before the accumulators are read, the last MFMA is given its 16 cycles and more.
 __device__ __forceinline__ void mfma_acc(f32x4& acc, const uint4& w, const uint4& x) {
   asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(as_bf16x8(w)), "v"(as_bf16x8(x)));
 }
@@ -117,7 +118,10 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmParams p) {
 #pragma unroll
   for (int a = 0; a < NT; ++a)
 #pragma unroll
-    for (int b = 0; b < MT; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < MT; ++b) {
+      acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+      asm volatile("" : "+a"(acc[a][b]));  // (written here, well before the first mfma_acc)
+    }
   float ss[MT];
 #pragma unroll
   for (int b = 0; b < MT; ++b) ss[b] = 0.f;

@@ -1,0 +1,329 @@
+// Prompt GEMM on int4 weights (AWQ, groups of 128): the weights are unpacked between LDS and the matrix cores, so a step reads them at
+// 4 bits and no bf16 copy is written and read back. Every fragment holds the very bf16 values of that copy ((v s - s z) gamma, rounded once).
+//
+// As gemm_w4_kernel (gemm_prompt.h): four waves, one per SIMD, operands of a k-step read (here: and unpacked) during the MFMAs of the one
+// before, stages by LDS-DMA. The waves stand side by side over the columns, so that each fragment of W is unpacked by one wave of the block
+// only: unpacking is what bounds it (per fragment 23 VALU operations, 31 with gamma, against MT MFMAs of four cycles' issue and 16 cycles each),
+// hence the tiles of many rows and few columns. us, a bf16 copy and the bf16 kernels -> here (MI355X, cold weights): 256 rows, 17920 x 1536
+// with a norm 50.4 -> 39.0, 1536 x 8960 35.3 -> 27.3, 1536 x 1536 18.4 -> 14.7; 96 rows, 28672 x 4096 117 -> 52, 1536 x 8960 28.2 -> 17.8.
+#include "gemm_prompt.h"
+
+namespace vgate {
+
+template <int MT, int NT>
+struct Q4 {  // geometry: four waves side by side, each 16 MT rows x 16 NT columns; stages of 128 k (one group)
+  static constexpr int BM = 16 * MT, BN = 64 * NT;
+  static constexpr int XB = BN * 64, SB = XB + BM * 256;  // W | x (two 64-k halves) | scales, zeros, gamma: 1 KiB each
+  static constexpr int STAGE = SB + 3072;
+  static constexpr int PPW = MT + NT + 1;  // DMA of a wave and stage
+};
+
+template <int MT, int NT, int NS, int EPI, bool NORM>
+__global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
+  using G = Q4<MT, NT>;
+  constexpr int PPW = G::PPW, STAGE = G::STAGE;
+  static_assert(NS * STAGE <= 160 * 1024, "LDS");
+  static_assert(NS >= 2 && (NS - 1) * PPW < 64 && (NT & (NT - 1)) == 0 && NT <= 8, "vmcnt; the block's scales repeat in 1 KiB");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  TLScope tl_scope(p.dbg_ts);
+  const int lane = threadIdx.x & 63, quad = lane >> 4;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int KQ = p.K >> 7;
+  const int z = blockIdx.y, nz = gridDim.y;
+  const int q0 = (KQ * z) / nz, nk = (KQ * (z + 1)) / nz - q0;
+  const int mblocks = (p.M + G::BM - 1) / G::BM;
+  const int nwg = gridDim.x, orig = blockIdx.x, xcd = orig & 7, q = nwg >> 3, r = nwg & 7;
+  const int wgid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (orig >> 3);
+  const int per = 8 * (p.N / G::BN), grp = wgid / per, in = wgid - grp * per, gm = min(8, mblocks - 8 * grp);
+  const int m0 = (8 * grp + in % gm) * G::BM;
+  const int n0 = (in / gm) * G::BN, nt0 = n0 / 16 + wid * NT;  // the wave's first column tile
+  const u32x4 wrs = rsrc_words(p.wp + ((size_t)(n0 / 16) * KQ + q0) * 64);
+  const u32x4 xrs = rsrc_words(p.x + (size_t)m0 * p.lda + q0 * 128);
+  // the wave's small piece: the group's scales, zeros (of the block's columns, asked for again until the 1 KiB is full) or gamma
+  const int kind = NORM ? min(wid, 2) : wid & 1;
+  const bf16_t* small = kind == 0 ? p.scales : kind == 1 ? p.zeros : p.norm_w;
+  const u32x4 srs = rsrc_words(small + (kind < 2 ? (size_t)q0 * p.N + n0 : (size_t)q0 * 128));
+  const uint32_t sstep = kind < 2 ? (uint32_t)p.N * 2u : 256u;
+  const uint32_t wvo = lane * 16, svo = (uint32_t)(lane * 16) & (kind < 2 ? 2u * G::BN - 1u : 255u);
+  uint32_t xvo[MT];  // pieces of 8 rows x 64 k: tile (piece >> 2), k half (piece >> 1) & 1, row half piece & 1
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int g = wid * MT + i;
+    xvo[i] = (uint32_t)(x_piece_row(m0 + (g >> 2) * 16, g & 1, lane, p.M) - m0) * (uint32_t)p.lda * 2u + (uint32_t)x_piece_col(g & 1, lane) * 2u +
+             (uint32_t)((g >> 1) & 1) * 128u;
+  }
+  const uint32_t lds0 = lds_addr_of(smem);
+  const uint32_t wrow = (uint32_t)KQ * 1024u;
+  auto issue_piece = [&](int i, int st, int buf) {
+    const uint32_t base = lds0 + buf * STAGE;
+    if (i < NT) blds16(wrs, wvo, (uint32_t)(wid * NT + i) * wrow + (uint32_t)st * 1024u, base + (uint32_t)(wid * NT + i) * 1024u);
+    else if (i < NT + MT) blds16(xrs, xvo[i - NT], (uint32_t)st * 256u, base + G::XB + (uint32_t)(wid * MT + i - NT) * 1024u);
+    else blds16(srs, svo, (uint32_t)st * sstep, base + G::SB + kind * 1024u);
+  };
+  f32x4 acc[NT][MT];
+#pragma unroll
+  for (int a = 0; a < NT; ++a)
+#pragma unroll
+    for (int b = 0; b < MT; ++b) {
+      acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+      asm volatile("" : "+a"(acc[a][b]));  // (written here, well before the first mfma_acc)
+    }
+  float ss[MT];
+#pragma unroll
+  for (int b = 0; b < MT; ++b) ss[b] = 0.f;
+  uint4 wf[2][NT], xf[2][MT], wq[NT];
+  float sc[NT], zs[NT], gam[8];
+  const int xlo[2] = {G::XB + x_frag_off(0, lane), G::XB + x_frag_off(1, lane)};
+  auto read_stage = [&](const char* sb) {  // the group's packed weights and scales
+#pragma unroll
+    for (int a = 0; a < NT; ++a) {
+      wq[a] = *reinterpret_cast<const uint4*>(sb + (wid * NT + a) * 1024 + lane * 16);
+      sc[a] = bf2f(*reinterpret_cast<const bf16_t*>(sb + G::SB + ((wid * NT + a) * 16 + (lane & 15)) * 2));
+      zs[a] = bf2f(*reinterpret_cast<const bf16_t*>(sb + G::SB + 1024 + ((wid * NT + a) * 16 + (lane & 15)) * 2));
+    }
+  };
+  auto read_gamma = [&](int u, const char* sb) {
+    if constexpr (NORM) unpack8(*reinterpret_cast<const uint4*>(sb + G::SB + 2048 + u * 64 + quad * 16), gam);
+  };
+  // half h of the wave's fragment of tile a at k-step u: the bf16 that the unpacked copy of the matrix would hold. (The low nibbles of a
+  // word's bytes are elements 0 4 1 5, the high ones 2 6 3 7; opaque once masked, so that each is one v_cvt_f32_ubyte away.)
+  auto unpack = [&](int a, int h, int u) {
+    const uint32_t w = u == 0 ? wq[a].x : u == 1 ? wq[a].y : u == 2 ? wq[a].z : wq[a].w;
+    uint32_t m = (h ? w >> 4 : w) & 0x0F0F0F0Fu;
+    asm("" : "+v"(m));
+    float f[4] = {(float)(m & 0xFFu) * sc[a] - zs[a], (float)((m >> 16) & 0xFFu) * sc[a] - zs[a], (float)((m >> 8) & 0xFFu) * sc[a] - zs[a],
+                  (float)(m >> 24) * sc[a] - zs[a]};
+    if constexpr (NORM) {
+      f[0] *= gam[2 * h];
+      f[1] *= gam[2 * h + 1];
+      f[2] *= gam[2 * h + 4];
+      f[3] *= gam[2 * h + 5];
+    }
+    uint4& o = wf[u & 1][a];
+    (h ? o.y : o.x) = pack_bf2(f[0], f[1]);
+    (h ? o.w : o.z) = pack_bf2(f[2], f[3]);
+  };
+  auto read_x = [&](int b, int u, const char* sb) {
+    xf[u & 1][b] = *reinterpret_cast<const uint4*>(sb + xlo[u & 1] + b * 4096 + (u >> 1) * 2048);
+  };
+  constexpr int U = 2 * NT;  // halves of fragments of a k-step to unpack
+  // the MFMAs of k-step u, a row tile at a time; between them the next k-step is read and unpacked and, at the last, the next stage asked for
+  auto phase = [&](auto uc, const char* sb, int st, int buf) {
+    constexpr int u = decltype(uc)::value, v = (u + 1) & 3;
+    // (an MFMA reads what the VALU wrote two wait states before at the soonest, and the compiler does not see that mfma_acc() is one)
+#pragma unroll
+    for (int a = 0; a < NT; ++a) {
+      u32x4 f = __builtin_bit_cast(u32x4, wf[u & 1][a]);
+      asm volatile("s_nop 1" : "+v"(f));
+      wf[u & 1][a] = __builtin_bit_cast(uint4, f);
+    }
+    if constexpr (u == 3) read_stage(sb);
+    read_gamma(v, sb);
+    if constexpr (NORM) {
+      if (wid == u) {
+#pragma unroll
+        for (int b = 0; b < MT; ++b) ss[b] = sumsq8(xf[u & 1][b], ss[b]);
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < MT; ++b) {
+      read_x(b, v, sb);
+      if constexpr (u == 3) {
+#pragma unroll
+        for (int i = (b * PPW) / MT; i < ((b + 1) * PPW) / MT; ++i) issue_piece(i, st, buf);
+      }
+#pragma unroll
+      for (int e = (b * U) / MT; e < ((b + 1) * U) / MT; ++e) unpack(e >> 1, e & 1, v);
+#pragma unroll
+      for (int a = 0; a < NT; ++a) mfma_acc(acc[a][b], wf[u & 1][a], xf[u & 1][b]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  using C0 = std::integral_constant<int, 0>;
+  using C1 = std::integral_constant<int, 1>;
+  using C2 = std::integral_constant<int, 2>;
+  using C3 = std::integral_constant<int, 3>;
+#pragma unroll
+  for (int s0 = 0; s0 < NS; ++s0)
+#pragma unroll
+    for (int i = 0; i < PPW; ++i) issue_piece(i, s0 < nk ? s0 : nk - 1, s0);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * PPW) : "memory");
+  read_stage(smem);
+  read_gamma(0, smem);
+#pragma unroll
+  for (int b = 0; b < MT; ++b) read_x(b, 0, smem);
+#pragma unroll
+  for (int e = 0; e < U; ++e) unpack(e >> 1, e & 1, 0);
+  int buf = 0;
+  for (int t = 0; t < nk; ++t) {
+    const char* sb = smem + buf * STAGE;
+    const int nb = buf + 1 == NS ? 0 : buf + 1;
+    phase(C0{}, sb, 0, 0);
+    phase(C1{}, sb, 0, 0);
+    phase(C2{}, sb, 0, 0);
+    // this stage is read (its last k-step is in registers), the next one has landed: both for every wave
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * PPW) : "memory");
+    phase(C3{}, smem + nb * STAGE, t + NS < nk ? t + NS : nk - 1, buf);  // past the end: clamped duplicates, never used
+    buf = nb;
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");  // the trailing duplicates
+#pragma unroll
+  for (int a = 0; a < NT; ++a)
+#pragma unroll
+    for (int b = 0; b < MT; ++b) asm volatile("" : "+a"(acc[a][b]));
+  float* rows = reinterpret_cast<float*>(smem);  // [wave][row] sums of squares
+  if constexpr (NORM) {
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < MT; ++b) {
+      float s2 = ss[b];
+      s2 += xor16(s2);
+      s2 += xor32(s2);
+      if (lane < 16) rows[wid * G::BM + b * 16 + lane] = s2;
+    }
+    __syncthreads();
+  }
+  float* part = p.slabs + (size_t)z * p.M * p.N;
+  float* ssq = p.slabs + (size_t)nz * p.M * p.N + (size_t)z * p.M;
+#pragma unroll
+  for (int b = 0; b < MT; ++b) {
+    const int rl = b * 16 + (lane & 15), m = m0 + rl;
+    float scale = 1.f, s2 = 0.f;
+    if constexpr (NORM) {
+      s2 = (rows[rl] + rows[G::BM + rl]) + (rows[2 * G::BM + rl] + rows[3 * G::BM + rl]);
+      scale = rsqrtf(s2 / (float)p.K + p.eps);
+    }
+    if (nz > 1) {
+      if (m < p.M) {
+        if (NORM && wid == 0 && n0 == 0 && lane < 16) ssq[m] = s2;
+#pragma unroll
+        for (int a = 0; a < NT; ++a)
+          __builtin_nontemporal_store(acc[a][b], reinterpret_cast<f32x4*>(part + (size_t)m * p.N + (nt0 + a) * 16 + 4 * quad));
+      }
+    } else {
+#pragma unroll
+      for (int a = 0; a < NT; ++a) {
+        f32x4 v[1] = {acc[a][b] * scale};
+        epilogue<1, EPI, false>(p, v, m, nt0 + a, 4 * quad, EpiPre<1>{}, m < p.M);
+      }
+    }
+  }
+}
+
+template <int EPI, int NORM, int NTB>
+void launch_prefill_reduce(const GemmParams& p, int nz, hipStream_t st);
+
+template <int MT, int NT, int NS, int EPI, bool NORM>
+static bool launch_q4_one(const GemmParams& p, int nz, hipStream_t st) {
+  using G = Q4<MT, NT>;
+  if (p.N % G::BN != 0) return false;
+  const int blocks = ((p.M + G::BM - 1) / G::BM) * (p.N / G::BN);
+  GemmParams q = p;
+  if (q.dbg_ts == nullptr) q.dbg_ts = tl_take("gemm_q4_prompt", blocks * nz);
+  auto kern = gemm_q4_prompt_kernel<MT, NT, NS, EPI, NORM>;
+  static bool attr = [&] {
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, NS * G::STAGE) == hipSuccess;
+  }();
+  (void)attr;
+  hipLaunchKernelGGL(kern, dim3(blocks, nz), dim3(256), NS * G::STAGE, st, q);
+  if (nz > 1) launch_prefill_reduce<EPI, NORM ? 2 : 0, 1>(p, nz, st);
+  return true;
+}
+
+template <int EPI, bool NORM>
+static bool launch_q4_epi(const GemmParams& p, int code, int nz, hipStream_t st) {
+  switch (code) {
+#define VG_Q4(MT, NT, NS) case 100 * MT + 10 * NT: return launch_q4_one<MT, NT, NS, EPI, NORM>(p, nz, st)
+    VG_Q4(4, 1, 3);  // two blocks to a CU
+    VG_Q4(6, 1, 3);
+    VG_Q4(6, 2, 4);
+    VG_Q4(8, 2, 3);
+    VG_Q4(10, 2, 3);
+    VG_Q4(16, 2, 2);
+    VG_Q4(6, 4, 3);
+#undef VG_Q4
+  }
+  return false;
+}
+
+// Costs (us) as in choose_prefill_form() of gemm_prefill.hip, fitted to 15 shapes (N 512 .. 28672, K 1024 .. 14336) x 10 row counts 65 ..
+// 2048 on cold weights; K-tiles of 128. Unpacking is repeated by every row of blocks, so from some row count on a bf16 copy (2.2 us + 0.56
+// a million weights) and the bf16 kernels are ahead: 17920 x 1536 at 448 rows 60 against 64 us, at 1024 114 against 89; 1536 x 1536 at 1024 17
+// against 22. The choice between all forms and that takes 1.019 of the best one's time, and 1 / 1.26 of the copy's (geometric means).
+bool q4_prompt_form(int M, int N, int K, bool norm, size_t slab_bytes, int* code, int* slices) {
+  struct Tile {
+    int code, bm, bn, per_cu;
+    struct {
+      float e, a, b, c, d, w, o;
+    } cost[2];  // plain, with a norm in front
+  };
+  static constexpr Tile tiles[] = {
+      {410, 64, 64, 2, {{8.3f, 0.907f, 0.415f, 1.87f, 0.328f, 0.009f, 0.f}, {9.35f, 0.883f, 0.547f, 1.75f, 0.232f, 0.006f, 0.f}}},
+      {610, 96, 64, 1, {{5.99f, 2.07f, 0.594f, 2.46f, 0.434f, 0.f, 0.405f}, {6.74f, 2.86f, 0.81f, 2.26f, 0.299f, 0.f, 0.341f}}},
+      {620, 96, 128, 1, {{7.29f, 3.86f, 0.989f, 1.5f, 0.339f, 0.f, 0.087f}, {7.68f, 4.57f, 1.25f, 1.4f, 0.293f, 0.f, 0.113f}}},
+      {820, 128, 128, 1, {{7.92f, 3.83f, 1.15f, 1.06f, 0.358f, 0.f, 0.217f}, {8.51f, 5.2f, 1.41f, 0.477f, 0.298f, 0.f, 0.144f}}},
+      {1020, 160, 128, 1, {{8.98f, 4.86f, 1.31f, 0.152f, 0.336f, 0.f, 0.151f}, {9.24f, 6.01f, 1.59f, 0.f, 0.29f, 0.f, 0.154f}}},
+      {1620, 256, 128, 1, {{10.5f, 4.19f, 1.84f, 0.f, 0.347f, 0.f, 0.339f}, {10.9f, 5.22f, 2.17f, 0.f, 0.325f, 0.f, 0.426f}}},
+      {640, 96, 256, 1, {{8.39f, 5.55f, 1.74f, 0.353f, 0.343f, 0.f, 0.082f}, {8.99f, 6.65f, 2.09f, 0.f, 0.287f, 0.f, 0.079f}}}};
+  static constexpr int cuts[] = {1, 2, 3, 4, 6, 8};
+  if (M <= 64 || N % 64 != 0 || K % 128 != 0) return false;
+  static const int cus = [] {
+    int v = 0, dev = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev);
+    return v > 0 ? v : 256;
+  }();
+  const float weights = 1e-6f * (float)N * (float)K, omb = 2e-6f * (float)M * (float)N;
+  float least = 2.2f + 0.56f * weights + prefill_cost_us(M, N, K, norm, slab_bytes);
+  auto over = [](int64_t x, int64_t y) { return (int)((x + y - 1) / y); };
+  *code = 0;
+  for (const Tile& t : tiles) {
+    if (N % t.bn != 0) continue;
+    const auto& x = t.cost[norm ? 1 : 0];
+    for (int nz : cuts) {
+      const int64_t blocks = (int64_t)over(M, t.bm) * (N / t.bn) * nz;
+      if (nz > 1 && (blocks > 600 || K / 128 / nz < 2 || ((size_t)nz * M * N + (size_t)nz * M) * 4 > slab_bytes)) continue;
+      const float us = x.e + x.a * over(blocks, (int64_t)cus * t.per_cu) + x.b * over(blocks, cus) * over(K / 128, nz) + x.w * 2.f * weights +
+                       x.o * omb + (nz > 1 ? x.c + x.d * 2.f * nz * omb : 0.f);
+      if (us < least) {
+        least = us;
+        *code = t.code;
+        *slices = nz;
+      }
+    }
+  }
+  return *code != 0;
+}
+
+bool launch_q4_prompt(const GemmArgs& g, hipStream_t st) {
+  if (g.M <= 0 || g.group != 128 || g.N % 64 != 0 || g.K % 128 != 0 || g.rownorm || g.ssp_in != nullptr || g.hg != nullptr ||
+      g.ssp_out != nullptr || g.row_idx != nullptr || reinterpret_cast<uintptr_t>(g.x) % 16 != 0 || g.lda % 8 != 0 || g.lda >= (1 << 20) ||
+      g.K >= (1 << 20) || g.scales == nullptr || g.zeros == nullptr ||
+      ((reinterpret_cast<uintptr_t>(g.scales) | reinterpret_cast<uintptr_t>(g.zeros) | reinterpret_cast<uintptr_t>(g.norm_w)) & 15) != 0)
+    return false;
+  GemmParams p{};
+  p.x = g.x; p.lda = g.lda; p.M = g.M;
+  p.wp = reinterpret_cast<const uint4*>(g.wp); p.N = g.N; p.K = g.K;
+  p.norm_w = g.norm_w; p.eps = g.eps;
+  p.bias = g.bias; p.res = g.res; p.ldr = g.ldr;
+  p.out = g.out; p.ldo = g.ldo;
+  p.splitk = 1;
+  p.slabs = g.slabs;
+  p.positions = g.positions; p.slots = g.slots; p.cos_sin = g.cos_sin;
+  p.k_cache = g.k_cache; p.v_cache = g.v_cache; p.hq = g.hq; p.hkv = g.hkv; p.bs = g.bs;
+  p.scales = g.scales; p.zeros = g.zeros; p.group = g.group;
+  p.dbg_ts = g.dbg_ts;
+  int nz = g.splitk > 0 ? g.splitk : 1;
+  while (nz > 1 && p.K / 128 / nz < 2) --nz;
+  if (nz > 1 && (p.slabs == nullptr || ((size_t)nz * p.M * p.N + (size_t)nz * p.M) * 4 > g.slab_bytes)) nz = 1;
+#define VG_Q4E(E) return g.norm_w != nullptr ? launch_q4_epi<E, true>(p, g.ntb, nz, st) : launch_q4_epi<E, false>(p, g.ntb, nz, st)
+  switch (g.epi) {
+    case EPI_SILU: VG_Q4E(EPI_SILU);
+    case EPI_QKV: VG_Q4E(EPI_QKV);
+    case EPI_F32: VG_Q4E(EPI_F32);
+    default: VG_Q4E(EPI_BF16);
+  }
+#undef VG_Q4E
+}
+
+}  // namespace vgate

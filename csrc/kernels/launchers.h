@@ -95,6 +95,11 @@ bool launch_dense_kx(const GemmArgs& g, hipStream_t st);
 // AWQ W4A16 medium-M kernel (gemm_awq_mid.hip, 16 < M <= 64): g.waves tiles per block (8: one block
 // per CU owning whole tiles), g.splitk K slices; false for a shape / mode it does not take
 bool launch_awq_mid(const GemmArgs& g, hipStream_t st);
+// AWQ W4A16 prompt kernel (gemm_prompt_q4.hip, M > 64): g.ntb = a tile code, g.splitk = K slices, as q4_prompt_form() gives them; false
+// for a shape / mode it does not take. q4_prompt_form(): false where a bf16 copy of the matrix and the bf16 kernels are faster.
+bool launch_q4_prompt(const GemmArgs& g, hipStream_t st);
+bool q4_prompt_form(int M, int N, int K, bool norm, size_t slab_bytes, int* code, int* slices);
+float prefill_cost_us(int M, int N, int K, bool norm, size_t slab_bytes);  // the bf16 kernels' cost of a product (gemm_prefill.hip)
 // AWQ int4 fragments -> bf16 fragment-packed copy (optionally gamma-folded) for the prefill kernel
 void launch_awq_dequant(const void* wq, const uint16_t* scales, const uint16_t* sz, const uint16_t* gamma,
                         void* out, int N, int K, int group, hipStream_t st);

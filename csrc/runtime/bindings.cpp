@@ -653,6 +653,13 @@ PYBIND11_MODULE(_C, m) {
   m.def("awq_dequant", &awq_dequant, "AWQ int4 packed -> bf16 fragment-packed (prefill operand; optional gamma fold)",
         py::arg("wq"), py::arg("scales"), py::arg("sz"), py::arg("N"), py::arg("K"), py::arg("group"), py::arg("out"),
         py::arg("gamma") = py::none());
+  m.def("q4_prompt_form", [](int64_t M, int64_t N, int64_t K, bool norm, const Tensor& ws) {
+    int code = 0, slices = 1;
+    const size_t slab_bytes = ws.numel() > 65536 ? (size_t)(ws.numel() - 65536) * 4 : 0;
+    if (!vgate::q4_prompt_form((int)M, (int)N, (int)K, norm, slab_bytes, &code, &slices)) code = 0;
+    return std::make_pair(code, slices);
+  }, "(tile code, K slices) of the int4 prompt GEMM (gemm path 5), or (0, 1): dequantise and take the bf16 kernels",
+        py::arg("M"), py::arg("N"), py::arg("K"), py::arg("norm"), py::arg("ws"));
   m.def("silu_mul", &silu_mul, "out = silu(y[:, :I]) * y[:, I:] (library gate_up epilogue)");
   m.def("attn_decode", &attn_decode, "paged split-K decode attention");
   m.def("attn_prefill", &attn_prefill, "paged varlen causal prefill attention",

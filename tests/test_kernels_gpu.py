@@ -1218,6 +1218,60 @@ def test_prefill_four_wave_tiles_short_k(bn, K):
     assert _rel_err(out, x.double() @ w.double().t()) < K * 2.0 ** -24
 
 
+def _awq(N, K, layout, seed, **kw):
+    g = torch.Generator().manual_seed(seed)
+    scales = (torch.rand(K // 128, N, generator=g) * 0.02 + 0.01).bfloat16()
+    zeros = torch.randint(0, 16, (K // 128, N), generator=g).float()
+    q = torch.randint(0, 16, (N, K), generator=g, dtype=torch.int32)
+    return ops.Linear(None, layout=layout, awq=dict(qint=q, scales=scales.to(DEV), zeros=zeros.to(DEV), group=128), **kw)
+
+
+@pytest.mark.parametrize("code", [410, 610, 620, 820, 1020, 1620, 640])
+@pytest.mark.parametrize("M,K,sk", [(1, 128, 1), (65, 256, 1), (97, 640, 2), (577, 1536, 3)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_awq_prompt_tiles(code, M, K, sk, norm):
+    """Every tile of the int4 prompt kernel (gemm_prompt_q4.hip) against 64-bit sums over the bf16 values that awq_dequant() writes: fewer
+    groups than the ring has stages, one row, rows past a tile and past eight row blocks, K slices, rows of a wider matrix."""
+    C, N = ops.native(), 256
+    lin = _awq(N, K, "plain", M + K)
+    x = torch.randn(M, K + 8, device=DEV, generator=torch.Generator(DEV).manual_seed(K)).bfloat16()[:, :K]
+    gamma = (torch.rand(K, device=DEV) + 0.5).bfloat16() if norm else None
+    copy = torch.empty(N * K, dtype=torch.bfloat16, device=DEV)
+    C.awq_dequant(lin.wp, lin.scales, lin.zeros, N, K, 128, copy, gamma)
+    want = x.double() @ ops.unpack_weight(copy, N, K).double().t()
+    if norm:
+        want *= torch.rsqrt((x.double() ** 2).mean(1, keepdim=True) + 1e-6)
+    out = torch.full((M, N), float("nan"), device=DEV)
+    C.gemm(x, lin.wp, N, K, out, 1, ws=ops.workspace(DEV), ntb=code, splitk=sk, path=5, awq_scales=lin.scales, awq_zeros=lin.zeros,
+           group=128, norm_w=gamma, eps=1e-6)
+    # fp32 sums of exact bf16 products: K roundings of 2^-24 at most, a few more for the row scale
+    assert ((out.double() - want).norm() / want.norm()).item() < (K + 8) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("M", [65, 130, 256])
+def test_awq_prompt_epilogues_match_the_copied_matrix(M):
+    """Residual, SiLU * mul, QKV + RoPE + cache write of the int4 prompt kernel against the bf16 kernels on the dequantised matrix."""
+    torch.manual_seed(M)
+    K, hq, hkv, BS = 1536, 12, 2, 16
+    x = torch.randn(M, K, device=DEV).bfloat16()
+    norm = ((torch.rand(K, device=DEV) + 0.5).bfloat16(), 1e-6)
+    lin, res = _awq(1536, K, "plain", 1), torch.randn(M, 1536, device=DEV).bfloat16()
+    pairs = []
+    for fn in (ops._linear_awq_prompt, ops._linear_awq_dequant):
+        got = [res.clone(), torch.empty(M, 4480, dtype=torch.bfloat16, device=DEV), torch.empty(M, hq * 128, dtype=torch.bfloat16, device=DEV)]
+        assert fn(x, lin, got[0], got[0], None, None, 0, M) is not False
+        assert fn(x, _awq(8960, K, "silu", 2), got[1], None, norm, None, 2, M) is not False
+        nblk = (M + BS - 1) // BS + 2
+        kc = torch.zeros(nblk, hkv, BS, 128, device=DEV).bfloat16()
+        qkv = dict(positions=torch.arange(M, dtype=torch.int32, device=DEV), slots=torch.arange(M, device=DEV).flip(0).int(),
+                   cos_sin=ref.rope_cos_sin(4096, 128, 1e6, device=DEV), k_cache=kc, v_cache=torch.zeros_like(kc), hq=hq, hkv=hkv)
+        bias = (torch.randn(2048, device=DEV, generator=torch.Generator(DEV).manual_seed(5)) * 0.1).bfloat16()
+        assert fn(x, _awq(2048, K, "qkv", 3, bias=bias), got[2], None, norm, qkv, 3, M) is not False
+        pairs.append(got + [qkv["k_cache"], qkv["v_cache"]])
+    for a, b in zip(*pairs):  # the same bf16 operands: fp32 sums in another order, rounded to bf16
+        assert _rel_err(a, b) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("M", [200, 448, 640])
 @pytest.mark.parametrize("bn,sk", [(2560, 0), (2561, 0), (2560, 2), (2561, 3)])
 def test_prefill_wide_tiles(M, bn, sk):

@@ -339,6 +339,8 @@ def linear(x: torch.Tensor, lin: Linear, out: torch.Tensor | None = None,
     if awq_mid:
         path = 2  # int4 medium kernel (csrc/kernels/gemm_awq_mid.hip awq_mid_kernel): no bf16 scratch
     elif lin.kind == "awq" and M >= AWQ_DEQUANT_MIN_M and row_idx is None and waves == 0 and splitk == 0:
+        if path == 0 and M > 64 and _linear_awq_prompt(x, lin, out, residual, norm, qkv, epi, M):
+            return out
         return _linear_awq_dequant(x, lin, out, residual, norm, qkv, epi, M)
     ntb = 0
     sk = False
@@ -427,8 +429,8 @@ def _attn_after(q, qkv, attn):
               int(attn["part_size"]), float(attn["scale"]))
 
 
-# AWQ steps of 16 < M <= 64 rows (mixed prefill + decode) run the int4 medium kernel; longer ones
-# (M >= AWQ_DEQUANT_MIN_M not taken by it) dequantise to scratch + the bf16 prefill / tile kernels
+# AWQ steps of 16 < M <= 64 rows (mixed prefill + decode) run the int4 medium kernel, longer ones the int4 prompt
+# kernel; what neither takes (M >= AWQ_DEQUANT_MIN_M) dequantises to scratch + the bf16 prefill / tile kernels
 AWQ_DEQUANT_MIN_M = 32
 _AWQ_SCRATCH: dict = {}
 
@@ -440,6 +442,28 @@ def reserve_awq_scratch(device, numel: int) -> torch.Tensor:
     if t is None or t.numel() < numel:
         t = _AWQ_SCRATCH[key] = torch.empty(numel, dtype=torch.bfloat16, device=device)
     return t
+
+
+def _linear_awq_prompt(x, lin: "Linear", out, residual, norm, qkv, epi, M) -> bool:
+    """Long AWQ step on the int4 prompt kernel (csrc/kernels/gemm_prompt_q4.hip), which unpacks the weights on their way to the
+    matrix cores. False: a group size, an alignment or a size that stays with :func:`_linear_awq_dequant`."""
+    gamma = norm[0] if norm is not None else None
+    if lin.group != 128 or x.stride(0) % 8 or x.stride(0) >= 1 << 20 or x.data_ptr() % 16 or (gamma is not None and gamma.data_ptr() % 16):
+        return False
+    C = native()
+    ws = workspace(x.device)
+    code, slices = C.q4_prompt_form(M, lin.N, lin.K, gamma is not None, ws)
+    if code == 0:
+        return False
+    kw = dict(bias=lin.bias, res=residual, ws=ws, ntb=code, splitk=slices, path=5, awq_scales=lin.scales, awq_zeros=lin.zeros,
+              group=lin.group)
+    if gamma is not None:
+        kw.update(norm_w=gamma, eps=float(norm[1]))
+    if qkv is not None:
+        kw.update(positions=qkv["positions"], slots=qkv["slots"], cos_sin=qkv["cos_sin"], k_cache=qkv["k_cache"],
+                  v_cache=qkv["v_cache"], hq=qkv["hq"], hkv=qkv["hkv"])
+    C.gemm(x, lin.wp, lin.N, lin.K, out, epi, **kw)
+    return True
 
 
 def _linear_awq_dequant(x, lin: "Linear", out, residual, norm, qkv, epi, M):
