@@ -53,6 +53,7 @@ VG_EXTERN_EPI(EPI_F32)
 VG_EXTERN_EPI(EPI_SILU)
 VG_EXTERN_EPI(EPI_QKV)
 VG_EXTERN_EPI(EPI_BF16_AR)
+extern template void dispatch_epi<EPI_GLU, false>(GemmParams, const GemmArgs&, hipStream_t);
 
 // ---- AWQ prefill operand: int4 fragments -> bf16 fragments (same fragment order) ----
 // Long AWQ steps run the LDS-tiled bf16 prefill kernel (gemm_prefill.hip) on a per-call scratch
@@ -108,6 +109,9 @@ void launch_awq_dequant(const void* wq, const uint16_t* scales, const uint16_t* 
 
 template <bool AWQ>
 static void launch_dispatch(GemmParams p, const GemmArgs& g, hipStream_t st) {
+  if constexpr (!AWQ) {
+    if (g.act != 0) return dispatch_epi<EPI_GLU, false>(p, g, st);
+  }
   switch (g.epi) {
     case EPI_SILU: dispatch_epi<EPI_SILU, AWQ>(p, g, st); break;
     case EPI_QKV: dispatch_epi<EPI_QKV, AWQ>(p, g, st); break;
@@ -123,6 +127,7 @@ static GemmParams to_params(const GemmArgs& g) {
   p.norm_w = g.norm_w; p.eps = g.eps;
   p.bias = g.bias; p.res = g.res; p.ldr = g.ldr;
   p.out = g.out; p.ldo = g.ldo;
+  p.act = g.act; p.limit = g.limit; p.alpha = g.alpha;
   p.slabs = g.slabs; p.counters = g.counters;
   p.gran = nullptr; p.fault = g.fault;  // (granule split-K: set by the decode launchers when it fits)
   p.positions = g.positions; p.slots = g.slots; p.cos_sin = g.cos_sin;

@@ -803,7 +803,9 @@ void dispatch_epi(GemmParams p, const GemmArgs& g, hipStream_t st) {
     else if (norm == 3) launch_m<NTB_, EPI, 3, AWQ>(p, g, st);                  \
     else launch_m<NTB_, EPI, 0, AWQ>(p, g, st);                                 \
   } while (0)
-  if constexpr (EPI == EPI_SILU) {  // self-contained 16-column tiles (8 gate + 8 up); g.ntb 2 / 4: tiles per block (sweeps)
+  if constexpr (EPI == EPI_GLU) {
+    launch_m<1, EPI, 0, AWQ>(p, g, st);  // (no norm in front: the binding checks it)
+  } else if constexpr (EPI == EPI_SILU) {  // self-contained 16-column tiles (8 gate + 8 up); g.ntb 2 / 4: tiles per block (sweeps)
     if constexpr (!AWQ) {
       if (g.ntb == 4 && ntiles % 4 == 0 && g.M <= 16) { VG_NORM(4); return; }
       if (g.ntb == 2 && ntiles % 2 == 0 && g.M <= 16) { VG_NORM(2); return; }

@@ -11,7 +11,8 @@ namespace vgate {
 
 // EPI_BF16_AR: EPI_BF16 with the TP all-reduce in the epilogue (epilogue_ar); its own instantiations
 // (gemm_epi_bf16ar.hip), so the TP = 1 kernels carry none of its code or registers
-enum GemmEpi : int { EPI_BF16 = 0, EPI_F32 = 1, EPI_SILU = 2, EPI_QKV = 3, EPI_BF16_AR = 4 };
+enum GemmEpi : int { EPI_BF16 = 0, EPI_F32 = 1, EPI_SILU = 2, EPI_QKV = 3, EPI_BF16_AR = 4,
+                    EPI_GLU = 5 };  // EPI_GLU: EPI_SILU's layout with another pair activation (GemmParams::act), apart so that the SiLU kernels stay short
 constexpr int SK_MAX = 8;  // split-K slices per tile (the combine issues all slices' loads at once)
 
 // TP row-parallel decode GEMM: the all-reduce runs in the epilogue (epilogue_ar) when world >= 1
@@ -46,6 +47,7 @@ struct GemmParams {
   unsigned long long* dbg_ts;  // per-block [start, end] realtime stamps (profiling), or null
   ArFused ar;                  // world 0: no fused all-reduce
   uint4* qa_gran;              // EPI_QKV: also write q / K / V as tagged granules (qkv_attn.hip), or null
+  int act; float limit, alpha;  // EPI_GLU: 2 the clamped pair with its limit and alpha, 4 gelu_tanh(gate) * up
   int vgx;                     // > 0: a 1-D launch carries the (vgx, 1, slices) grid z-major (qkv_attn.hip)
 };
 
@@ -421,28 +423,35 @@ __device__ __forceinline__ void epilogue(const GemmParams& p, const f32x4 (&v)[N
       return;
     }
   }
-  if constexpr (EPI != EPI_QKV && EPI != EPI_SILU) {
+  if constexpr (EPI != EPI_QKV && EPI != EPI_SILU && EPI != EPI_GLU) {
     if (!valid) return;
   }
-  if constexpr (EPI == EPI_SILU) {
+  if constexpr (EPI == EPI_SILU || EPI == EPI_GLU) {
     // SiLU tile layout (ops.row_permutation "silu"): tile t holds gate columns 8t..8t+7 (lane
     // groups 0, 1) and their up partners (groups 2, 3), so a pair sits on lanes l and l ^ 32 of
     // ONE tile: every tile is self-contained and a decode block can own a single tile.
+    // Of a pair of lanes' four gates and ups each computes two: one half-wave swap puts (gate, up) of columns 0 / 1 on the gate's
+    // lane and of columns 2 / 3 on the up's. (All four on the gate's lane, the other one computing waste, made the epilogue of a
+    // 256 x 256 tile twice as long.)
     const bool gate = nsub < 8;
 #pragma unroll
     for (int j = 0; j < NTB; ++j) {
-      float o[4];
+      float o[2];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float up = xor32(v[j][i]);  // all 64 lanes active
-        o[i] = silu(v[j][i]) * up;
+      for (int i = 0; i < 2; ++i) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[j][i]), __float_as_uint(v[j][i + 2]), false, false);
+        const float g = __uint_as_float(r[0]), up = __uint_as_float(r[1]);
+        if constexpr (EPI == EPI_SILU) {
+          o[i] = silu(g) * up;
+        } else {  // x sigmoid(y) up': 2: x = min(g, L), y = alpha x, up' = clamp(u, -L, L) + 1; 4 (tanh GELU): (1 + tanh z) / 2 = sigmoid(2 z)
+          const float x = p.act == 2 ? fminf(g, p.limit) : g;
+          const float y = p.act == 2 ? p.alpha * x : 1.5957691216057308f * (x + 0.044715f * x * x * x);
+          o[i] = x / (1.f + expf(-y)) * (p.act == 2 ? fminf(fmaxf(up, -p.limit), p.limit) + 1.f : up);
+        }
       }
-      if (valid && gate) {
-        uint2 pk;
-        pk.x = pack_bf2(o[0], o[1]);
-        pk.y = pack_bf2(o[2], o[3]);
-        *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(p.out) + (size_t)m * p.ldo + (nt0 + j) * 8 + nsub) = pk;
-      }
+      if (valid)
+        *reinterpret_cast<uint32_t*>(reinterpret_cast<bf16_t*>(p.out) + (size_t)m * p.ldo + (nt0 + j) * 8 + (gate ? nsub : nsub - 6)) =
+            pack_bf2(o[0], o[1]);
     }
   } else if constexpr (EPI == EPI_QKV) {
     static_assert(NTB == 1, "QKV tiles carry their rotation partners (see qkv_col)");

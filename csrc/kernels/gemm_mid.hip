@@ -347,6 +347,7 @@ bool launch_gemm_mid(const GemmArgs& g, hipStream_t st) {
   p.norm_w = nullptr; p.eps = g.eps;
   p.bias = g.bias; p.res = g.res; p.ldr = g.ldr;
   p.out = g.out; p.ldo = g.ldo;
+  p.act = g.act; p.limit = g.limit; p.alpha = g.alpha;
   p.splitk = 1;
   p.slabs = g.slabs;
   p.positions = g.positions; p.slots = g.slots; p.cos_sin = g.cos_sin;
@@ -357,6 +358,7 @@ bool launch_gemm_mid(const GemmArgs& g, hipStream_t st) {
   if (g.waves == 8) return norm == 2 ? launch_midw_epi<E, 2>(p, st) : launch_midw_epi<E, 0>(p, st); \
   return norm == 2 ? launch_mid_epi<E, 2>(p, g.waves, g.splitk, g.slab_bytes, st)           \
                    : launch_mid_epi<E, 0>(p, g.waves, g.splitk, g.slab_bytes, st)
+  if (g.act != 0) return g.waves == 8 ? launch_midw_epi<EPI_GLU, 0>(p, st) : launch_mid_epi<EPI_GLU, 0>(p, g.waves, g.splitk, g.slab_bytes, st);
   switch (g.epi) {
     case EPI_SILU: VG_MD(EPI_SILU);
     case EPI_QKV: VG_MD(EPI_QKV);

@@ -766,6 +766,7 @@ VG_RED_INST(EPI_BF16)
 VG_RED_INST(EPI_F32)
 VG_RED_INST(EPI_SILU)
 VG_RED_INST(EPI_QKV)
+template void launch_prefill_reduce<EPI_GLU, 0, 1>(const GemmParams&, int, hipStream_t);
 #undef VG_RED_INST
 
 template <int EPI, int NORM, int NTB, int BM = 256, int BN = 128, int WM = 4, int WN = 2, int NS = 3, int SCHED = 0,
@@ -1077,6 +1078,7 @@ bool launch_gemm_prefill(const GemmArgs& g, hipStream_t st) {
   p.norm_w = nullptr; p.eps = g.eps;
   p.bias = g.bias; p.res = g.res; p.ldr = g.ldr;
   p.out = g.out; p.ldo = g.ldo;
+  p.act = g.act; p.limit = g.limit; p.alpha = g.alpha;
   p.splitk = 1;
   p.slabs = g.slabs;
   p.counters = g.counters; p.fault = g.fault;
@@ -1088,6 +1090,7 @@ bool launch_gemm_prefill(const GemmArgs& g, hipStream_t st) {
 #define VG_PF(E)                                                                                         \
   return norm == 2 ? launch_prefill_epi<E, 2>(p, fb, fs, g.slab_bytes, g.max_counters, st)               \
                    : launch_prefill_epi<E, 0>(p, fb, fs, g.slab_bytes, g.max_counters, st)
+  if (g.act != 0) return launch_prefill_epi<EPI_GLU, 0>(p, fb, fs, g.slab_bytes, g.max_counters, st);
   switch (g.epi) {
     case EPI_SILU: VG_PF(EPI_SILU);
     case EPI_QKV: VG_PF(EPI_QKV);

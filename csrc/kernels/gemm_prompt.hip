@@ -40,6 +40,7 @@ VG_W4_INST(EPI_BF16)
 VG_W4_INST(EPI_F32)
 VG_W4_INST(EPI_SILU)
 VG_W4_INST(EPI_QKV)
+template bool launch_gemm_w4<EPI_GLU, 0>(const GemmParams&, int, int, hipStream_t);
 #undef VG_W4_INST
 
 }  // namespace vgate

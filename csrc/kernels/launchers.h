@@ -26,6 +26,8 @@ struct GemmArgs {
   void* out;          // bf16 [M, N] (silu: [M, N/2]; f32 for EPI_F32; qkv: q [M, hq*128])
   int ldo;
   int epi;            // 0 bf16, 1 f32, 2 silu*mul (gate/up tiles interleaved), 3 qkv+rope+kv-write
+  int act = 0;        // epi 2: 0 silu*mul; 2 the clamped pair (min(g, L) sigmoid(alpha min(g, L)) (clamp(u, -L, L) + 1)); 4 gelu_tanh*mul
+  float limit = 0.f, alpha = 0.f;
   int waves;          // 0 = heuristic
   int splitk;         // 0 = heuristic
   int ntb;            // 16-column tiles per block for plain / f32 epilogues (0 = heuristic; 1, 2, 4)

@@ -69,7 +69,7 @@ void gemm(const Tensor& x, const Tensor& wp, int64_t N, int64_t K, Tensor& out, 
           const c10::optional<Tensor>& fa_out, const c10::optional<Tensor>& fa_part_o,
           const c10::optional<Tensor>& fa_part_ml, const c10::optional<Tensor>& fa_tickets,
           const c10::optional<Tensor>& fa_sync, int64_t fa_part_size, double fa_scale,
-          const c10::optional<Tensor>& fa_dbg_ts) {
+          const c10::optional<Tensor>& fa_dbg_ts, int64_t act, double limit, double alpha) {
   CHECK_DEV(x); CHECK_DEV(wp); CHECK_DEV(out);
   CHECK_DT(x, torch::kBFloat16);
   CHECK_LASTDIM(x); CHECK_LASTDIM(out);
@@ -114,6 +114,9 @@ void gemm(const Tensor& x, const Tensor& wp, int64_t N, int64_t K, Tensor& out, 
   g.ldr = g.res ? (int)res->stride(0) : 0;
   if (g.res) TORCH_CHECK(res->size(0) >= M && res->size(1) >= N, "gemm: residual shape");
   g.out = out.data_ptr(); g.ldo = (int)out.stride(0);
+  TORCH_CHECK(act == 0 || ((act == 2 || act == 4) && epi == 2 && !awq && !g.norm_w && !rownorm && !(ssp_in.has_value() && ssp_in->defined())),
+              "gemm: act 2 (clamped) and 4 (tanh GELU) belong to the silu epilogue of bf16 weights without a norm");
+  g.act = (int)act; g.limit = (float)limit; g.alpha = (float)alpha;
   g.epi = (int)epi; g.waves = (int)waves; g.splitk = (int)splitk; g.ntb = (int)ntb; g.path = (int)path;
   if (ws.has_value() && ws->defined()) {
     CHECK_DEV(*ws); CHECK_DT(*ws, torch::kInt32);
@@ -637,7 +640,8 @@ PYBIND11_MODULE(_C, m) {
         py::arg("ar_fused_off") = 0, py::arg("fa_block_tables") = py::none(), py::arg("fa_context_lens") = py::none(),
         py::arg("fa_query_start") = py::none(), py::arg("fa_out") = py::none(), py::arg("fa_part_o") = py::none(),
         py::arg("fa_part_ml") = py::none(), py::arg("fa_tickets") = py::none(), py::arg("fa_sync") = py::none(),
-        py::arg("fa_part_size") = 512, py::arg("fa_scale") = 1.0, py::arg("fa_dbg_ts") = py::none());
+        py::arg("fa_part_size") = 512, py::arg("fa_scale") = 1.0, py::arg("fa_dbg_ts") = py::none(),
+        py::arg("act") = 0, py::arg("limit") = 0.0, py::arg("alpha") = 0.0);
   m.def("attention", &attention, "unified paged attention: decode (partitions merged in-launch) + varlen prefill tiles",
         py::arg("q"), py::arg("q_stride"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("context_lens"), py::arg("query_start"), py::arg("tile_seq"), py::arg("tile_q0"), py::arg("out"),

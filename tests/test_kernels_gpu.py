@@ -1218,6 +1218,26 @@ def test_prefill_four_wave_tiles_short_k(bn, K):
     assert _rel_err(out, x.double() @ w.double().t()) < K * 2.0 ** -24
 
 
+@pytest.mark.parametrize("act", ["clamped", "gelu_tanh"])
+@pytest.mark.parametrize("M", [1, 16, 17, 48, 64, 65, 300, 1100])
+def test_gemm_pair_activations(act, M):
+    """The pair epilogue's other activations in every form that takes a step's rows (decode, medium, tile, prompt) against 64 bits:
+    fp32 sums and activation, one rounding to bf16."""
+    from vgate.ops import seq
+    torch.manual_seed(M)
+    K, I = 1024, 1280
+    x = torch.randn(M, K, device=DEV).bfloat16()
+    w = (torch.randn(2 * I, K, device=DEV) * (4.0 / math.sqrt(K))).bfloat16()
+    lin = ops.Linear(w, layout="silu")
+    code = seq.ACT_CLAMPED_GLU if act == "clamped" else seq.ACT_GELU_TANH_MUL
+    lin.glu = (code, 3.0, 1.702)
+    got = ops.linear(x, lin)
+    g, u = (x.double() @ w.double().t()).split(I, 1)
+    want = seq._act(g, u, code, 3.0, 1.702)
+    assert ((got.double() - want).norm() / want.norm()).item() < 2.0 ** -8
+    assert torch.isfinite(got).all()
+
+
 def _awq(N, K, layout, seed, **kw):
     g = torch.Generator().manual_seed(seed)
     scales = (torch.rand(K // 128, N, generator=g) * 0.02 + 0.01).bfloat16()

@@ -62,13 +62,12 @@ class Proj:
         dev = torch.device(device)
         n_ok = (N // 2) % 64 == 0 if silu_pair else N % 64 == 0
         self.packed = allow_packed and n_ok and self.packs(K, device, f32)
-        # the packed kernels' pair epilogue is SiLU: another pair activation runs the stacked [gate; up]
-        # matrix as a plain packed GEMM and applies act(gate) * up in a row kernel
-        self.split_act = self.packed and silu_pair and pair_act != seq.ACT_SILU_MUL
         self.bias = None
         if self.packed:
-            self.lin = ops.Linear(w.to(dev, torch.bfloat16), kind="silu" if silu_pair and not self.split_act else "plain",
+            self.lin = ops.Linear(w.to(dev, torch.bfloat16), kind="silu" if silu_pair else "plain",
                                   bias=None if bias is None else bias.to(dev, torch.bfloat16).contiguous())
+            if silu_pair and pair_act != seq.ACT_SILU_MUL:
+                self.lin.glu = (pair_act, limit, alpha)
             self.w = None
         else:
             self.lin = None
@@ -86,10 +85,6 @@ class Proj:
 
     def __call__(self, x: torch.Tensor, out_f32: bool = False, act: int = 0, out: torch.Tensor | None = None) -> torch.Tensor:
         M = x.shape[0]
-        if self.split_act:
-            if out is None:
-                out = torch.empty(M, self.out_features, dtype=torch.bfloat16, device=x.device)
-            return seq.glu_rows(ops.linear(x, self.lin), out, self.pair_act, limit=self.limit, alpha=self.alpha)
         if self.packed:   # (a single matrix's activation is a row kernel behind the packed GEMM)
             y = ops.linear(x, self.lin, out=out, out_f32=out_f32)
             return seq.act_rows(y, act) if act else y

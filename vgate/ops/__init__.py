@@ -170,6 +170,7 @@ class Linear:
             self.layout = "silu"
         self.kind = "awq" if awq is not None else "dense"
         self.bias = bias
+        self.glu = None  # "silu" layout: (act, limit, alpha) of another pair activation (vgate.ops.seq.ACT_CLAMPED_GLU)
         self.norm_gamma = None  # RMSNorm weight folded into the packed copy (see fold_norm)
         # decode-GEMM decomposition for M <= 16 steps (0 = the launcher's heuristic): set by the
         # model from the measured per-shape table (vgate/models/decode_plans.py)
@@ -372,6 +373,8 @@ def linear(x: torch.Tensor, lin: Linear, out: torch.Tensor | None = None,
     if qkv is not None:
         kw.update(positions=qkv["positions"], slots=qkv["slots"], cos_sin=qkv["cos_sin"],
                   k_cache=qkv["k_cache"], v_cache=qkv["v_cache"], hq=qkv["hq"], hkv=qkv["hkv"])
+    if lin.glu is not None:
+        kw.update(act=lin.glu[0], limit=lin.glu[1], alpha=lin.glu[2])
     if lin.kind == "awq":
         kw.update(awq_scales=lin.scales, awq_zeros=lin.zeros, group=lin.group)
         if getattr(lin, "szp", None) is not None:
