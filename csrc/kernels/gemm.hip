@@ -127,11 +127,11 @@ static GemmParams to_params(const GemmArgs& g) {
   p.norm_w = g.norm_w; p.eps = g.eps;
   p.bias = g.bias; p.res = g.res; p.ldr = g.ldr;
   p.out = g.out; p.ldo = g.ldo;
-  p.act = g.act; p.limit = g.limit; p.alpha = g.alpha;
   p.slabs = g.slabs; p.counters = g.counters;
   p.gran = nullptr; p.fault = g.fault;  // (granule split-K: set by the decode launchers when it fits)
   p.positions = g.positions; p.slots = g.slots; p.cos_sin = g.cos_sin;
   p.k_cache = g.k_cache; p.v_cache = g.v_cache; p.hq = g.hq; p.hkv = g.hkv; p.bs = g.bs;
+  if (g.act != 0) set_glu(p, GluAct{g.act, g.limit, g.alpha});
   p.scales = g.scales; p.zeros = g.zeros; p.group = g.group; p.szp = g.awq_szp;
   p.dbg_ts = g.dbg_ts;
   p.hg = g.hg; p.hg_gamma = g.hg_gamma; p.ssp_out = g.ssp_out; p.ssp_in = g.ssp_in; p.ssn = g.ssn;

@@ -12,7 +12,7 @@ namespace vgate {
 // EPI_BF16_AR: EPI_BF16 with the TP all-reduce in the epilogue (epilogue_ar); its own instantiations
 // (gemm_epi_bf16ar.hip), so the TP = 1 kernels carry none of its code or registers
 enum GemmEpi : int { EPI_BF16 = 0, EPI_F32 = 1, EPI_SILU = 2, EPI_QKV = 3, EPI_BF16_AR = 4,
-                    EPI_GLU = 5 };  // EPI_GLU: EPI_SILU's layout with another pair activation (GemmParams::act), apart so that the SiLU kernels stay short
+                    EPI_GLU = 5 };  // EPI_GLU: EPI_SILU's layout with another pair activation (glu_of), apart so that the SiLU kernels stay short
 constexpr int SK_MAX = 8;  // split-K slices per tile (the combine issues all slices' loads at once)
 
 // TP row-parallel decode GEMM: the all-reduce runs in the epilogue (epilogue_ar) when world >= 1
@@ -23,7 +23,7 @@ struct ArFused {
   uint32_t spin;   // polls before a wait gives up
 };
 
-struct GemmParams {
+struct GemmParams {  // (no longer than need be: with 12 bytes more a step's short kernels took 0.4 us longer)
   const bf16_t* x; int lda; int M; const int32_t* row_idx;
   const uint4* wp; int N; int K;
   const bf16_t* norm_w; float eps;  // norm_w null under NORM = gamma folded into W (row scale only)
@@ -47,9 +47,20 @@ struct GemmParams {
   unsigned long long* dbg_ts;  // per-block [start, end] realtime stamps (profiling), or null
   ArFused ar;                  // world 0: no fused all-reduce
   uint4* qa_gran;              // EPI_QKV: also write q / K / V as tagged granules (qkv_attn.hip), or null
-  int act; float limit, alpha;  // EPI_GLU: 2 the clamped pair with its limit and alpha, 4 gelu_tanh(gate) * up
   int vgx;                     // > 0: a 1-D launch carries the (vgx, 1, slices) grid z-major (qkv_attn.hip)
 };
+
+// EPI_GLU's activation, in fields that only other epilogues use: 2 the clamped pair with its limit and alpha, 4 gelu_tanh(gate) * up
+struct GluAct {
+  int act;
+  float limit, alpha;
+};
+__host__ __device__ __forceinline__ void set_glu(GemmParams& p, GluAct a) {
+  p.hq = a.act;
+  p.eps = a.limit;
+  p.hkv = __builtin_bit_cast(int, a.alpha);
+}
+__device__ __forceinline__ GluAct glu_of(const GemmParams& p) { return GluAct{p.hq, p.eps, __builtin_bit_cast(float, p.hkv)}; }
 
 // (column-tile block, K slice, slices) of this block: the grid decomposition of gemm_finish's hand-off
 struct SplitPos {
@@ -444,9 +455,10 @@ __device__ __forceinline__ void epilogue(const GemmParams& p, const f32x4 (&v)[N
         if constexpr (EPI == EPI_SILU) {
           o[i] = silu(g) * up;
         } else {  // x sigmoid(y) up': 2: x = min(g, L), y = alpha x, up' = clamp(u, -L, L) + 1; 4 (tanh GELU): (1 + tanh z) / 2 = sigmoid(2 z)
-          const float x = p.act == 2 ? fminf(g, p.limit) : g;
-          const float y = p.act == 2 ? p.alpha * x : 1.5957691216057308f * (x + 0.044715f * x * x * x);
-          o[i] = x / (1.f + expf(-y)) * (p.act == 2 ? fminf(fmaxf(up, -p.limit), p.limit) + 1.f : up);
+          const GluAct a = glu_of(p);
+          const float x = a.act == 2 ? fminf(g, a.limit) : g;
+          const float y = a.act == 2 ? a.alpha * x : 1.5957691216057308f * (x + 0.044715f * x * x * x);
+          o[i] = x / (1.f + expf(-y)) * (a.act == 2 ? fminf(fmaxf(up, -a.limit), a.limit) + 1.f : up);
         }
       }
       if (valid)

@@ -347,11 +347,11 @@ bool launch_gemm_mid(const GemmArgs& g, hipStream_t st) {
   p.norm_w = nullptr; p.eps = g.eps;
   p.bias = g.bias; p.res = g.res; p.ldr = g.ldr;
   p.out = g.out; p.ldo = g.ldo;
-  p.act = g.act; p.limit = g.limit; p.alpha = g.alpha;
   p.splitk = 1;
   p.slabs = g.slabs;
   p.positions = g.positions; p.slots = g.slots; p.cos_sin = g.cos_sin;
   p.k_cache = g.k_cache; p.v_cache = g.v_cache; p.hq = g.hq; p.hkv = g.hkv; p.bs = g.bs;
+  if (g.act != 0) set_glu(p, GluAct{g.act, g.limit, g.alpha});
   p.dbg_ts = g.dbg_ts;
   const int norm = g.rownorm ? 2 : 0;
 #define VG_MD(E)                                                                             \

@@ -1078,12 +1078,12 @@ bool launch_gemm_prefill(const GemmArgs& g, hipStream_t st) {
   p.norm_w = nullptr; p.eps = g.eps;
   p.bias = g.bias; p.res = g.res; p.ldr = g.ldr;
   p.out = g.out; p.ldo = g.ldo;
-  p.act = g.act; p.limit = g.limit; p.alpha = g.alpha;
   p.splitk = 1;
   p.slabs = g.slabs;
   p.counters = g.counters; p.fault = g.fault;
   p.positions = g.positions; p.slots = g.slots; p.cos_sin = g.cos_sin;
   p.k_cache = g.k_cache; p.v_cache = g.v_cache; p.hq = g.hq; p.hkv = g.hkv; p.bs = g.bs;
+  if (g.act != 0) set_glu(p, GluAct{g.act, g.limit, g.alpha});
   p.dbg_ts = g.dbg_ts;
   const int fb = g.ntb;      // reused as the forced tile width (0 = heuristic, 64 / 128)
   const int fs = g.splitk;   // forced K slices (0 = heuristic)
