@@ -308,24 +308,18 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_prefill2_kernel(GemmPara
     }
     return;
   }
+  float sc[MT];
 #pragma unroll
   for (int b = 0; b < MT; ++b) {
-    const int m = m0 + wm * (BM / WM) + b * 16 + (lane & 15);
-    float sc = 1.f;
+    sc[b] = 1.f;
     if constexpr (NORM == 2) {
       float s2 = ss[b];
       s2 += xor16(s2);
       s2 += xor32(s2);
-      sc = rsqrtf(s2 / (float)p.K + p.eps);
-    }
-#pragma unroll
-    for (int a = 0; a < NT; a += NTB) {
-      f32x4 v[NTB];
-#pragma unroll
-      for (int j = 0; j < NTB; ++j) v[j] = acc[a + j][b] * sc;
-      epilogue<NTB, EPI, false>(p, v, m, nt_blk + wn * NT + a, 4 * (lane >> 4), EpiPre<NTB>{}, m < p.M);
+      sc[b] = rsqrtf(s2 / (float)p.K + p.eps);
     }
   }
+  prompt_epilogue<NT, MT, EPI>(p, m0 + wm * (BM / WM), nt_blk + wn * NT, lane, [&](int a, int b) { return acc[a][b] * sc[b]; });
 }
 
 // ---- v4: 256 x 256 tile in four phases per K-tile ----
@@ -515,18 +509,8 @@ __device__ __forceinline__ void p4_finish(const GemmParams& p, char* smem, int w
     }
   }
 #pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    const int m = m0 + wc * 64 + b * 16 + (lane & 15);
-    float sc = 1.f;
-    if constexpr (NORM == 2) sc = rsqrtf(rs[b] / (float)p.K + p.eps);
-#pragma unroll
-    for (int a = 0; a < NWN; a += NTB) {
-      f32x4 v[NTB];
-#pragma unroll
-      for (int j = 0; j < NTB; ++j) v[j] = acc[a + j][b] * sc;
-      epilogue<NTB, EPI, false>(p, v, m, nt_blk + wr * NWN + a, 4 * (lane >> 4), EpiPre<NTB>{}, m < p.M);
-    }
-  }
+  for (int b = 0; b < 4; ++b) rs[b] = NORM == 2 ? rsqrtf(rs[b] / (float)p.K + p.eps) : 1.f;
+  prompt_epilogue<NWN, 4, EPI>(p, m0 + wc * 64, nt_blk + wr * NWN, lane, [&](int a, int b) { return acc[a][b] * rs[b]; });
 }
 
 template <int BN, int EPI, int NORM, int NTB>

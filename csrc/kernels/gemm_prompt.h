@@ -46,6 +46,105 @@ __device__ __forceinline__ int x_frag_off(int ks, int lane) {
   return r * 128 + (((4 * ks + (lane >> 4)) ^ x_swz(r)) << 4);
 }
 
+// The epilogue of a wave's MT x NT tiles of a prompt GEMM (rows m0 + 16 b, tiles nt0 + a; value(a, b): the tile's accumulator, row scale
+// applied): epilogue()'s results, with what does not depend on the tile loaded, and divided, once per row. Tile by tile the loads of
+// positions, rotations, slots and residuals cannot pass the stores before them (they may alias), and every tile waits for memory:
+// Llama-3-8B prompt of 2048 tokens, step 3538 -> 3491 us.
+template <int NT, int MT, int EPI, typename V>
+__device__ __forceinline__ void prompt_epilogue(const GemmParams& p, int m0, int nt0, int lane, V value) {
+  const int nsub = 4 * (lane >> 4);
+  if constexpr (EPI == EPI_QKV && 8 % NT == 0) {  // the wave's tiles lie in one head
+    const int head = __builtin_amdgcn_readfirstlane(nt0 >> 3);
+    const bool rotated = head < p.hq + p.hkv, upper = nsub >= 8;
+    const int d0 = qkv_rot(nt0, nsub), dcol = (upper ? 64 : 0) + d0;
+    uint2 bias[NT];
+    int pos[MT], slot[MT];
+#pragma unroll
+    for (int a = 0; a < NT; ++a)
+      bias[a] = p.bias ? *reinterpret_cast<const uint2*>(p.bias + qkv_col(nt0 + a, nsub)) : make_uint2(0, 0);
+#pragma unroll
+    for (int b = 0; b < MT; ++b) {
+      const int mm = min(m0 + b * 16 + (lane & 15), p.M - 1);
+      pos[b] = rotated ? p.positions[mm] : 0;
+      slot[b] = p.slots[mm];
+    }
+#pragma unroll
+    for (int b = 0; b < MT; ++b) {
+      const int m = m0 + b * 16 + (lane & 15);
+      float4 cs[NT], sn[NT];
+      if (rotated) {
+        const float* cp = p.cos_sin + (size_t)pos[b] * 128 + d0;
+#pragma unroll
+        for (int a = 0; a < NT; ++a) {
+          cs[a] = *reinterpret_cast<const float4*>(cp + 8 * a);
+          sn[a] = *reinterpret_cast<const float4*>(cp + 64 + 8 * a);
+        }
+      }
+      bf16_t* dst;
+      if (head < p.hq) {
+        dst = reinterpret_cast<bf16_t*>(p.out) + (size_t)m * p.ldo + head * 128 + dcol;
+      } else {
+        const int blk = slot[b] / p.bs, kh = rotated ? head - p.hq : head - p.hq - p.hkv;
+        dst = (rotated ? p.k_cache : p.v_cache) + (((size_t)blk * p.hkv + kh) * p.bs + (slot[b] - blk * p.bs)) * 128 + dcol;
+      }
+      const bool store = m < p.M && (head < p.hq || slot[b] >= 0);
+#pragma unroll
+      for (int a = 0; a < NT; ++a) {
+        const f32x4 v = value(a, b);
+        const float bb[4] = {bf_lo(bias[a].x), bf_hi(bias[a].x), bf_lo(bias[a].y), bf_hi(bias[a].y)};
+        float x[4], xp[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = bf2f(f2bf(v[i] + bb[i]));  // qkv is bf16 in the reference: round before rotating
+        if (rotated) {
+          const float cc[4] = {cs[a].x, cs[a].y, cs[a].z, cs[a].w}, sc[4] = {sn[a].x, sn[a].y, sn[a].z, sn[a].w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) xp[i] = xor32(x[i]);  // the partner column's value (all 64 lanes active)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[i] = upper ? x[i] * cc[i] + xp[i] * sc[i] : x[i] * cc[i] - xp[i] * sc[i];
+        }
+        if (store) *reinterpret_cast<uint2*>(dst + 8 * a) = make_uint2(pack_bf2(x[0], x[1]), pack_bf2(x[2], x[3]));
+      }
+    }
+  } else if constexpr (EPI == EPI_BF16 || EPI == EPI_F32) {
+    uint2 bias[NT], res[2][NT];
+    auto load_res = [&](int b) {
+      const bf16_t* r = p.res + (size_t)min(m0 + b * 16 + (lane & 15), p.M - 1) * p.ldr + nt0 * 16 + nsub;
+#pragma unroll
+      for (int a = 0; a < NT; ++a) res[b & 1][a] = *reinterpret_cast<const uint2*>(r + 16 * a);
+    };
+    if (p.bias) {
+#pragma unroll
+      for (int a = 0; a < NT; ++a) bias[a] = *reinterpret_cast<const uint2*>(p.bias + (nt0 + a) * 16 + nsub);
+    }
+    if (EPI == EPI_BF16 && p.res) load_res(0);
+#pragma unroll
+    for (int b = 0; b < MT; ++b) {
+      if (EPI == EPI_BF16 && b + 1 < MT && p.res) load_res(b + 1);  // (rows of its own: out may be the residual)
+      const int m = m0 + b * 16 + (lane & 15);
+      if (m < p.M) {
+#pragma unroll
+        for (int a = 0; a < NT; ++a) {
+          const f32x4 v[1] = {value(a, b)};
+          EpiPre<1> e;
+          e.b0 = bias[a];
+          e.r0 = res[b & 1][a];
+          epilogue<1, EPI, true>(p, v, m, nt0 + a, nsub, e, true);
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int b = 0; b < MT; ++b) {
+      const int m = m0 + b * 16 + (lane & 15);
+#pragma unroll
+      for (int a = 0; a < NT; ++a) {
+        const f32x4 v[1] = {value(a, b)};
+        epilogue<1, EPI, false>(p, v, m, nt0 + a, nsub, EpiPre<1>{}, m < p.M);
+      }
+    }
+  }
+}
+
 // LDS-DMA through a buffer descriptor: 16 B per lane from base + voff + soff to lds + 16 lane (inline asm and vmcnt by the caller, as
 // glds16; no 64-bit address per piece: a wave that issues alone on its SIMD has no slots for those)
 __device__ __forceinline__ void blds16(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
@@ -183,33 +282,39 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmParams p) {
   for (int a = 0; a < NT; ++a)
 #pragma unroll
     for (int b = 0; b < MT; ++b) asm volatile("" : "+a"(acc[a][b]));
-  float* part = p.slabs + (size_t)z * p.M * p.N;
-  float* ssq = p.slabs + (size_t)nz * p.M * p.N + (size_t)z * p.M;
+  if (nz > 1) {  // fp32 partial of this K slice, as the other forms leave it for prefill_reduce_kernel
+    float* part = p.slabs + (size_t)z * p.M * p.N;
+    float* ssq = p.slabs + (size_t)nz * p.M * p.N + (size_t)z * p.M;
 #pragma unroll
-  for (int b = 0; b < MT; ++b) {
-    const int m = m0 + (wm * MT + b) * 16 + (lane & 15);
-    float sc = 1.f, s2 = 0.f;
-    if constexpr (NORM == 2) {
-      s2 = ss[b];
-      s2 += xor16(s2);
-      s2 += xor32(s2);
-      sc = rsqrtf(s2 / (float)p.K + p.eps);
-    }
-    if (nz > 1) {  // fp32 partial of this K slice, as the other forms leave it for prefill_reduce_kernel
+    for (int b = 0; b < MT; ++b) {
+      const int m = m0 + (wm * MT + b) * 16 + (lane & 15);
+      float s2 = 0.f;
+      if constexpr (NORM == 2) {
+        s2 = ss[b];
+        s2 += xor16(s2);
+        s2 += xor32(s2);
+      }
       if (m < p.M) {
         if (NORM == 2 && wn == 0 && nt_blk == 0 && lane < 16) ssq[m] = s2;
 #pragma unroll
         for (int a = 0; a < NT; ++a)
           __builtin_nontemporal_store(acc[a][b], reinterpret_cast<f32x4*>(part + (size_t)m * p.N + (nt_blk + wn * NT + a) * 16 + 4 * (lane >> 4)));
       }
-    } else {
+    }
+    return;
+  }
+  float sc[MT];
 #pragma unroll
-      for (int a = 0; a < NT; ++a) {
-        f32x4 v[1] = {acc[a][b] * sc};
-        epilogue<1, EPI, false>(p, v, m, nt_blk + wn * NT + a, 4 * (lane >> 4), EpiPre<1>{}, m < p.M);
-      }
+  for (int b = 0; b < MT; ++b) {
+    sc[b] = 1.f;
+    if constexpr (NORM == 2) {
+      float s2 = ss[b];
+      s2 += xor16(s2);
+      s2 += xor32(s2);
+      sc[b] = rsqrtf(s2 / (float)p.K + p.eps);
     }
   }
+  prompt_epilogue<NT, MT, EPI>(p, m0 + wm * MT * 16, nt_blk + wn * NT, lane, [&](int a, int b) { return NORM == 2 ? acc[a][b] * sc[b] : acc[a][b]; });
 }
 
 }  // namespace vgate

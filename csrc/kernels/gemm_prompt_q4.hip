@@ -183,31 +183,33 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
     }
     __syncthreads();
   }
-  float* part = p.slabs + (size_t)z * p.M * p.N;
-  float* ssq = p.slabs + (size_t)nz * p.M * p.N + (size_t)z * p.M;
+  float scale[MT], s2[MT];
 #pragma unroll
   for (int b = 0; b < MT; ++b) {
-    const int rl = b * 16 + (lane & 15), m = m0 + rl;
-    float scale = 1.f, s2 = 0.f;
+    scale[b] = 1.f;
+    s2[b] = 0.f;
     if constexpr (NORM) {
-      s2 = (rows[rl] + rows[G::BM + rl]) + (rows[2 * G::BM + rl] + rows[3 * G::BM + rl]);
-      scale = rsqrtf(s2 / (float)p.K + p.eps);
+      const int rl = b * 16 + (lane & 15);
+      s2[b] = (rows[rl] + rows[G::BM + rl]) + (rows[2 * G::BM + rl] + rows[3 * G::BM + rl]);
+      scale[b] = rsqrtf(s2[b] / (float)p.K + p.eps);
     }
-    if (nz > 1) {
+  }
+  if (nz > 1) {
+    float* part = p.slabs + (size_t)z * p.M * p.N;
+    float* ssq = p.slabs + (size_t)nz * p.M * p.N + (size_t)z * p.M;
+#pragma unroll
+    for (int b = 0; b < MT; ++b) {
+      const int m = m0 + b * 16 + (lane & 15);
       if (m < p.M) {
-        if (NORM && wid == 0 && n0 == 0 && lane < 16) ssq[m] = s2;
+        if (NORM && wid == 0 && n0 == 0 && lane < 16) ssq[m] = s2[b];
 #pragma unroll
         for (int a = 0; a < NT; ++a)
           __builtin_nontemporal_store(acc[a][b], reinterpret_cast<f32x4*>(part + (size_t)m * p.N + (nt0 + a) * 16 + 4 * quad));
       }
-    } else {
-#pragma unroll
-      for (int a = 0; a < NT; ++a) {
-        f32x4 v[1] = {acc[a][b] * scale};
-        epilogue<1, EPI, false>(p, v, m, nt0 + a, 4 * quad, EpiPre<1>{}, m < p.M);
-      }
     }
+    return;
   }
+  prompt_epilogue<NT, MT, EPI>(p, m0, nt0, lane, [&](int a, int b) { return NORM ? acc[a][b] * scale[b] : acc[a][b]; });
 }
 
 template <int EPI, int NORM, int NTB>
