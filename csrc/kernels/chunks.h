@@ -74,6 +74,25 @@ __device__ __forceinline__ f32x4 ld4(const float* p) {
   return f32x4{v.x, v.y, v.z, v.w};
 }
 
+// Where element (row, k) of an MFMA operand lies in a record: [16-row tile][16-k tile of kt][lane = (k quad, row)][4 k], so that a wave's
+// load of a 16-B piece per lane is one KiB in a row. (With rows in a row, 64 lanes touched 16 lines of which they took 64 B: the address
+// path bound the chunk scans. 2048 tokens, 8 heads of 128, delta rule 154 -> 112 us, gated 82 -> 60.)
+__device__ __forceinline__ int frag(int row, int k, int kt) {
+  return (((row >> 4) * kt + (k >> 4)) * 64 + ((k >> 2) & 3) * 16 + (row & 15)) * 4 + (k & 3);
+}
+__host__ __device__ constexpr int whole16(int n) { return (n + 15) / 16 * 16; }
+
+// Rows row0 .. row0 + 3 of column c, one column per lane of whole quads (c % 4 = lane % 4), into a record: turned so that a lane stores four
+// columns of one row, a 16-B piece.
+__device__ __forceinline__ void put_rows4(float* base, int row0, int c, int kt, f32x4 v) {
+  const bool odd = c & 1, high = c & 2;
+  const float x0 = row_rot<0xB1>(odd ? v[0] : v[1]), x1 = row_rot<0xB1>(odd ? v[2] : v[3]);   // (quad_perm [1, 0, 3, 2])
+  v = odd ? f32x4{x0, v[1], x1, v[3]} : f32x4{v[0], x0, v[2], x1};
+  const float y0 = row_rot<0x4E>(high ? v[0] : v[2]), y1 = row_rot<0x4E>(high ? v[1] : v[3]);   // ([2, 3, 0, 1])
+  v = high ? f32x4{y0, y1, v[2], v[3]} : f32x4{v[0], v[1], y0, y1};
+  *reinterpret_cast<f32x4*>(base + frag(row0 + (c & 3), c & ~3, kt)) = v;
+}
+
 // sum over the 32 lanes of a half wave, in all of them
 __device__ __forceinline__ float half_sum(float v) {
   v += row_rot<0x128>(v);

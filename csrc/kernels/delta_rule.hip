@@ -32,7 +32,7 @@
 //          exchanges. The dependent chain of a token is what bounds it. Tokens are staged through LDS eight at a time, the next eight
 //          loaded while the current ones compute.
 //   finish (token, head) parallel: head norm, weight, gate.
-// 2048 tokens, 8 heads of 128: 73 + 154 + 17 us; the tokens one after another (three launches, one wave per 8 columns) took
+// 2048 tokens, 8 heads of 128: 69 + 112 + 13 us; the tokens one after another (three launches, one wave per 8 columns) took
 // 1060 us, 0.5 us of chain per token. What bounds the chunk scan is its 64 MFMAs per wave and two barriers per 32 tokens.
 #include <algorithm>
 
@@ -381,9 +381,9 @@ __global__ __launch_bounds__(64) void delta_finish_kernel(DeltaArgs p, int lim, 
 }
 
 // ------------------------------------------------------------------------------------------ chunks of CN tokens
-// floats of one (chunk, head) record: [W; Q] [2 CN][DP], the update's b and k [DP][CN] each, g_(1..CN) [DP], then per
-// column [CN] each: y, the outputs, v
-__host__ __device__ inline int64_t delta_chunk_floats(int DP, int D) { return (int64_t)4 * CN * DP + DP + (int64_t)3 * CN * D; }
+// floats of one (chunk, head) record: [W; Q] (rows, channels), the update's b and k (channels, tokens) each, g_(1..CN) [DP], then y, the
+// outputs and v (columns, tokens) each; all but g in the order of frag()
+__host__ __device__ inline int64_t delta_chunk_floats(int DP, int D) { return (int64_t)4 * CN * DP + DP + (int64_t)3 * CN * whole16(D); }
 
 // grid (chunk, head). At DP = 128 the LDS comes to half of a CU's.
 template <int DP, bool F32>
@@ -401,8 +401,10 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(DeltaArgs p, int li
   float* kk = kb + CN * DP;
   float* gam = kk + CN * DP;
   float* yy = gam + DP;
-  float* oo = yy + CN * D;
-  float* vo = oo + CN * D;
+  float* oo = yy + CN * whole16(D);
+  float* vo = oo + CN * whole16(D);
+  constexpr int KT = DP / 16;
+  const int DQ4 = (D + 3) & ~3;   // channels in whole quads of lanes (u = b = r = 0, w = 1 in those past D)
   constexpr int f32 = F32 ? 1 : 0;
 #pragma unroll 4
   for (int e = tid; e < CN * DP; e += 256) {   // rows past the end: u = b = r = 0, w = 1
@@ -480,9 +482,9 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(DeltaArgs p, int li
     }
   }
   __syncthreads();
-  for (int c = tid; c < 2 * D; c += 256) {   // one column of [W | y] per thread
+  for (int c = tid; c < DQ4 + D; c += 256) {   // one column of [W | y] per thread
     float x[CN];
-    if (c < D) {
+    if (c < DQ4) {
       float gm = 1.f;
 #pragma unroll
       for (int i = 0; i < CN; ++i) {
@@ -501,20 +503,26 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(DeltaArgs p, int li
           vk[j] = lu[j0 + j][c] * len[j0 + j] * gb;
           gb *= lw[j0 + j][c];
         }
-        *reinterpret_cast<f32x4*>(kb + c * CN + j0) = vb;
-        *reinterpret_cast<f32x4*>(kk + c * CN + j0) = vk;
+        *reinterpret_cast<f32x4*>(kb + frag(c, j0, 2)) = vb;
+        *reinterpret_cast<f32x4*>(kk + frag(c, j0, 2)) = vk;
         __builtin_amdgcn_sched_barrier(0);
       }
       gm = 1.f;
 #pragma unroll
-      for (int i = 0; i < CN; ++i) {
-        gm *= lw[i][c];
-        r0[i * DP + c] = x[i];
-        r0[(CN + i) * DP + c] = gm * lr[i][c] - row_dot(Rb + tri(i + 1), x, i + 1);
-        if (i % 2) __builtin_amdgcn_sched_barrier(0);
+      for (int i0 = 0; i0 < CN; i0 += 4) {
+        f32x4 q;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          gm *= lw[i0 + i][c];
+          q[i] = gm * lr[i0 + i][c] - row_dot(Rb + tri(i0 + i + 1), x, i0 + i + 1);
+          if (i % 2) __builtin_amdgcn_sched_barrier(0);
+        }
+        put_rows4(r0, i0, c, KT, f32x4{x[i0], x[i0 + 1], x[i0 + 2], x[i0 + 3]});
+        put_rows4(r0, CN + i0, c, KT, q);
+        __builtin_amdgcn_sched_barrier(0);
       }
     } else {
-      const int vc = c - D;
+      const int vc = c - DQ4;
       float v[CN];
 #pragma unroll
       for (int i = 0; i < CN; ++i) v[i] = t0 + i < t1 ? ldx(p.v, (int64_t)(t0 + i) * p.ld + h * D + vc, f32) : 0.f;
@@ -528,20 +536,24 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(DeltaArgs p, int li
         f32x4 o;
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = row_dot(Rk + tri(i0 + i + 1), v, i0 + i + 1) - row_dot(Rb + tri(i0 + i + 1), x, i0 + i + 1);
-        *reinterpret_cast<f32x4*>(yy + vc * CN + i0) = f32x4{x[i0], x[i0 + 1], x[i0 + 2], x[i0 + 3]};
-        *reinterpret_cast<f32x4*>(oo + vc * CN + i0) = o;
-        *reinterpret_cast<f32x4*>(vo + vc * CN + i0) = f32x4{v[i0], v[i0 + 1], v[i0 + 2], v[i0 + 3]};
+        *reinterpret_cast<f32x4*>(yy + frag(vc, i0, 2)) = f32x4{x[i0], x[i0 + 1], x[i0 + 2], x[i0 + 3]};
+        *reinterpret_cast<f32x4*>(oo + frag(vc, i0, 2)) = o;
+        *reinterpret_cast<f32x4*>(vo + frag(vc, i0, 2)) = f32x4{v[i0], v[i0 + 1], v[i0 + 2], v[i0 + 3]};
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
-  for (int e = tid; e < (DP - D) * CN; e += 256) {   // channels past D: zero
-    const int d = D + e / CN, i = e % CN;
-    r0[i * DP + d] = 0.f;
-    r0[(CN + i) * DP + d] = 0.f;
-    kb[d * CN + i] = 0.f;
-    kk[d * CN + i] = 0.f;
+  for (int e = tid; e < (DP - DQ4) * CN; e += 256) {   // channels past them: zero
+    const int d = DQ4 + e / CN, i = e % CN;
+    r0[frag(i, d, KT)] = 0.f;
+    r0[frag(CN + i, d, KT)] = 0.f;
+    kb[frag(d, i, 2)] = 0.f;
+    kk[frag(d, i, 2)] = 0.f;
     if (i == 0) gam[d] = 0.f;
+  }
+  for (int e = tid; e < (whole16(D) - D) * CN; e += 256) {   // columns of a last tile that is not whole: zero
+    const int at = frag(D + e / CN, e % CN, 2);
+    yy[at] = oo[at] = vo[at] = 0.f;
   }
 }
 
@@ -561,7 +573,6 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaArgs p, int 
   const int nc = (t1 - t0 + CN - 1) / CN, D = p.D, H = p.H;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, kg = l >> 4;
   const bool con = c0 + lr < D;
-  const int col = con ? c0 + lr : D - 1;   // (a column past the last: computed on the last one's inputs, never stored)
   const bool from_zero = p.context_lens[s] - (t1 - t0) <= 0;
   float* sp = p.state + ((int64_t)slot * H + h) * D * D;
   f32x4 S[TW];
@@ -587,20 +598,21 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaArgs p, int 
     const float* kk = kb + CN * DP;
     float* gam = r + 4 * CN * DP;
     float* yy = gam + DP;
-    x.out = yy + (w < 2 ? 0 : CN * D) + (int64_t)col * CN + 16 * (w & 1) + 4 * kg;   // y of waves 0, 1; the outputs of 2, 3
+    yy += blockIdx.y * 512 + 4 * l;   // (the workgroup's columns: two pieces)
+    x.out = yy + (w < 2 ? 0 : CN * whole16(D)) + 256 * (w & 1);   // y of waves 0, 1; the outputs of 2, 3
 #pragma unroll
-    for (int n = 0; n < NT; ++n) x.A[n] = ld4(r + (16 * w + lr) * DP + 16 * n + 4 * kg);
+    for (int n = 0; n < NT; ++n) x.A[n] = ld4(r + (w * NT + n) * 256 + 4 * l);
     x.add = ld4(x.out);
 #pragma unroll
-    for (int m = 0; m < 2; ++m) x.v[m] = ld4(yy + 2 * CN * D + (int64_t)col * CN + 16 * m + 4 * kg);
+    for (int m = 0; m < 2; ++m) x.v[m] = ld4(yy + 2 * CN * whole16(D) + 256 * m);
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
       const int tile = min(w + 4 * t, NT - 1);
       x.gm[t] = ld4(gam + 16 * tile + 4 * kg);
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
-        x.K[t][m] = ld4(kk + (16 * tile + lr) * CN + 16 * m + 4 * kg);
-        x.B[t][m] = ld4(kb + (16 * tile + lr) * CN + 16 * m + 4 * kg);
+        x.K[t][m] = ld4(kk + (2 * tile + m) * 256 + 4 * l);
+        x.B[t][m] = ld4(kb + (2 * tile + m) * 256 + 4 * l);
       }
     }
   };
@@ -666,8 +678,13 @@ __global__ __launch_bounds__(256) void delta_chunk_finish_kernel(DeltaArgs p, in
   int s, t0, t1;
   if (!locate_chunk(p.query_start, p.state_slots, p.S, lim, blockIdx.x, s, t0, t1)) return;
   const int h = blockIdx.y, D = p.D, H = p.H, tid = threadIdx.x;
-  const float* o = rec + ((int64_t)blockIdx.x * H + h) * delta_chunk_floats(DP, D) + 4 * CN * DP + DP + CN * D;
-  for (int e = tid; e < D * CN; e += 256) lo[e / CN][e % CN] = o[e];
+  const float* o = rec + ((int64_t)blockIdx.x * H + h) * delta_chunk_floats(DP, D) + 4 * CN * DP + DP + CN * whole16(D);
+  for (int e = tid; e < whole16(D) * CN / 4; e += 256) {   // (frag(): column, then token)
+    const int c = (e >> 7) * 16 + (e & 15), i = ((e >> 6) & 1) * 16 + ((e >> 4) & 3) * 4;
+    const f32x4 v = ld4(o + 4 * e);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) lo[c][i + j] = v[j];
+  }
   __syncthreads();
   {  // eight threads per token
     const int i = tid >> 3, part = tid & 7;

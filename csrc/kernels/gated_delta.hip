@@ -410,9 +410,9 @@ __global__ __launch_bounds__(256) void gated_delta_short_kernel(GatedDeltaArgs p
 }
 
 // ------------------------------------------------------------------------------------------ chunks of CN tokens
-// floats of one (chunk, head) record: [w; q'] [2 CN][DP], the update's keys [DP][CN], gamma_CN [DP], v' [V][CN], and b v', which
-// becomes o [V][CN]
-__host__ __device__ inline int64_t chunk_floats(int DP, int V) { return (int64_t)3 * CN * DP + DP + (int64_t)2 * CN * V; }
+// floats of one (chunk, head) record: [w; q'] (rows, channels), the update's keys (channels, tokens), gamma_CN [DP], v' (columns, tokens),
+// and b v', which becomes o; all but gamma in the order of frag()
+__host__ __device__ inline int64_t chunk_floats(int DP, int V) { return (int64_t)3 * CN * DP + DP + (int64_t)2 * CN * whole16(V); }
 
 // grid (chunk, head). At DP = 128 the LDS comes to a third of a CU's.
 template <int DP, bool F32>
@@ -432,7 +432,9 @@ __global__ __launch_bounds__(256, DP > 64 ? 3 : 4) void gated_delta_chunk_kernel
   float* kt = r0 + 2 * CN * DP;
   float* gam = kt + CN * DP;
   float* vh = gam + DP;
-  float* cc = vh + CN * V;
+  float* cc = vh + CN * whole16(V);
+  constexpr int KT = DP / 16;
+  const int DQ4 = (D + 3) & ~3;   // channels in whole quads of lanes (k = q = 0, g = 1 in those past D)
   for (int e = tid; e < 2 * DP; e += 256) {
     const bool isq = e < DP;
     const int d = isq ? e : e - DP, c = g * D + d, col = isq ? c : GD + c;
@@ -498,9 +500,9 @@ __global__ __launch_bounds__(256, DP > 64 ? 3 : 4) void gated_delta_chunk_kernel
     }
   }
   __syncthreads();
-  for (int c = tid; c < D + V; c += 256) {   // one column of [w | v'] per thread
+  for (int c = tid; c < DQ4 + V; c += 256) {   // one column of [w | v'] per thread
     float x[CN];
-    if (c < D) {
+    if (c < DQ4) {
       float gm = 1.f;
 #pragma unroll
       for (int i = 0; i < CN; ++i) {
@@ -508,7 +510,7 @@ __global__ __launch_bounds__(256, DP > 64 ? 3 : 4) void gated_delta_chunk_kernel
         x[i] = gm * lk[i][c];
       }
     } else {
-      const int vc = h * V + c - D, col = 2 * GD + vc;
+      const int vc = h * V + c - DQ4, col = 2 * GD + vc;
 #pragma unroll
       for (int i0 = 0; i0 < CN; i0 += 8) {
         float y[8];
@@ -522,7 +524,7 @@ __global__ __launch_bounds__(256, DP > 64 ? 3 : 4) void gated_delta_chunk_kernel
       x[i] = beta[i] * (x[i] - row_dot(As + tri(i), x, i));
       if (i % 2) __builtin_amdgcn_sched_barrier(0);   // (rows ahead of time would take hundreds of registers)
     }
-    if (c < D) {
+    if (c < DQ4) {
       float gb = 1.f;
 #pragma unroll
       for (int j0 = CN - 4; j0 >= 0; j0 -= 4) {
@@ -532,17 +534,23 @@ __global__ __launch_bounds__(256, DP > 64 ? 3 : 4) void gated_delta_chunk_kernel
           v[j] = lk[j0 + j][c] * gb;
           gb *= lg[j0 + j][c];
         }
-        *reinterpret_cast<f32x4*>(kt + c * CN + j0) = v;
+        *reinterpret_cast<f32x4*>(kt + frag(c, j0, 2)) = v;
         __builtin_amdgcn_sched_barrier(0);
       }
       gam[c] = gb;
       float gm = 1.f;
 #pragma unroll
-      for (int i = 0; i < CN; ++i) {
-        gm *= lg[i][c];
-        r0[i * DP + c] = x[i];
-        r0[(CN + i) * DP + c] = gm * lq[i][c] - row_dot(Bs + tri(i + 1), x, i + 1);
-        if (i % 2) __builtin_amdgcn_sched_barrier(0);
+      for (int i0 = 0; i0 < CN; i0 += 4) {
+        f32x4 q;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          gm *= lg[i0 + i][c];
+          q[i] = gm * lq[i0 + i][c] - row_dot(Bs + tri(i0 + i + 1), x, i0 + i + 1);
+          if (i % 2) __builtin_amdgcn_sched_barrier(0);
+        }
+        put_rows4(r0, i0, c, KT, f32x4{x[i0], x[i0 + 1], x[i0 + 2], x[i0 + 3]});
+        put_rows4(r0, CN + i0, c, KT, q);
+        __builtin_amdgcn_sched_barrier(0);
       }
     } else {
 #pragma unroll
@@ -550,18 +558,22 @@ __global__ __launch_bounds__(256, DP > 64 ? 3 : 4) void gated_delta_chunk_kernel
         f32x4 v;
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = row_dot(Bs + tri(i0 + i + 1), x, i0 + i + 1);
-        *reinterpret_cast<f32x4*>(vh + (c - D) * CN + i0) = f32x4{x[i0], x[i0 + 1], x[i0 + 2], x[i0 + 3]};
-        *reinterpret_cast<f32x4*>(cc + (c - D) * CN + i0) = v;
+        *reinterpret_cast<f32x4*>(vh + frag(c - DQ4, i0, 2)) = f32x4{x[i0], x[i0 + 1], x[i0 + 2], x[i0 + 3]};
+        *reinterpret_cast<f32x4*>(cc + frag(c - DQ4, i0, 2)) = v;
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
-  for (int e = tid; e < (DP - D) * CN; e += 256) {   // channels past D: zero
-    const int d = D + e / CN, i = e % CN;
-    r0[i * DP + d] = 0.f;
-    r0[(CN + i) * DP + d] = 0.f;
-    kt[d * CN + i] = 0.f;
+  for (int e = tid; e < (DP - DQ4) * CN; e += 256) {   // channels past them: zero
+    const int d = DQ4 + e / CN, i = e % CN;
+    r0[frag(i, d, KT)] = 0.f;
+    r0[frag(CN + i, d, KT)] = 0.f;
+    kt[frag(d, i, 2)] = 0.f;
     if (i == 0) gam[d] = 0.f;
+  }
+  for (int e = tid; e < (whole16(V) - V) * CN; e += 256) {   // columns of a last tile that is not whole: zero
+    const int at = frag(V + e / CN, e % CN, 2);
+    vh[at] = cc[at] = 0.f;
   }
 }
 
@@ -582,7 +594,6 @@ __global__ __launch_bounds__(256) void gated_delta_chunk_scan_kernel(GatedDeltaA
   const int nc = (t1 - t0 + CN - 1) / CN, D = p.D, V = p.V, H = p.H;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, kg = l >> 4;
   const bool con = c0 + lr < V;
-  const int col = con ? c0 + lr : V - 1;   // (a column past the last: computed on the last one's inputs, never stored)
   const bool from_zero = p.context_lens[s] - (t1 - t0) <= 0;
   float* sp = p.state + ((int64_t)slot * H + h) * D * V;
   f32x4 S[TW];
@@ -606,16 +617,16 @@ __global__ __launch_bounds__(256) void gated_delta_chunk_scan_kernel(GatedDeltaA
     float* r = r0 + (int64_t)ch * H * per;
     const float* kt = r + 2 * CN * DP;
     float* gam = r + 3 * CN * DP;
-    x.vc = gam + DP + (w < 2 ? 0 : CN * V) + (int64_t)col * CN + 16 * (w & 1) + 4 * kg;   // v' of waves 0, 1; b v' / o of 2, 3
+    x.vc = gam + DP + (w < 2 ? 0 : CN * whole16(V)) + blockIdx.y * 512 + 256 * (w & 1) + 4 * l;   // v' of waves 0, 1; b v' / o of 2, 3
 #pragma unroll
-    for (int n = 0; n < NT; ++n) x.A[n] = ld4(r + (16 * w + lr) * DP + 16 * n + 4 * kg);
+    for (int n = 0; n < NT; ++n) x.A[n] = ld4(r + (w * NT + n) * 256 + 4 * l);
     x.add = ld4(x.vc);
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
       const int tile = min(w + 4 * t, NT - 1);
       x.gm[t] = ld4(gam + 16 * tile + 4 * kg);
-      x.K[t][0] = ld4(kt + (16 * tile + lr) * CN + 4 * kg);
-      x.K[t][1] = ld4(kt + (16 * tile + lr) * CN + 16 + 4 * kg);
+      x.K[t][0] = ld4(kt + 2 * tile * 256 + 4 * l);
+      x.K[t][1] = ld4(kt + (2 * tile + 1) * 256 + 4 * l);
     }
   };
   // chunk ch from `x`, while chunk ch + 1 is on its way into `y` (the barriers wait for LDS traffic only)
@@ -674,8 +685,13 @@ __global__ __launch_bounds__(256) void gated_delta_chunk_finish_kernel(GatedDelt
   int s, t0, t1;
   if (!locate_chunk(p.query_start, p.state_slots, p.S, lim, blockIdx.x, s, t0, t1)) return;
   const int h = blockIdx.y, V = p.V, H = p.H, tid = threadIdx.x;
-  const float* o = rec + ((int64_t)blockIdx.x * H + h) * chunk_floats(DP, V) + 3 * CN * DP + DP + CN * V;
-  for (int e = tid; e < V * CN; e += 256) lo[e / CN][e % CN] = o[e];
+  const float* o = rec + ((int64_t)blockIdx.x * H + h) * chunk_floats(DP, V) + 3 * CN * DP + DP + CN * whole16(V);
+  for (int e = tid; e < whole16(V) * CN / 4; e += 256) {   // (frag(): column, then token)
+    const int c = (e >> 7) * 16 + (e & 15), i = ((e >> 6) & 1) * 16 + ((e >> 4) & 3) * 4;
+    const f32x4 v = ld4(o + 4 * e);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) lo[c][i + j] = v[j];
+  }
   __syncthreads();
   {  // eight threads per token
     const int i = tid >> 3, part = tid & 7;

@@ -498,6 +498,32 @@ def test_delta_rule_state_carry_and_slots(device, D):
 
 
 @pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("D", [5, 18, 33, 126])
+def test_delta_rule_chunks_of_odd_sizes(device, D):
+    """Portions in chunks (operand records whose last tiles of rows, channels and columns are not whole; a last chunk of nine tokens)
+    against the same tokens in steps of eight, which another form takes."""
+    from vgate.ops import seq
+    g = torch.Generator().manual_seed(D)
+    H, n, d = 2, 201, _dev(device)
+    hd = H * D
+    P, wl = torch.randn(n, 5 * hd, generator=g).to(d), torch.randn(n, hd, generator=g).to(d)
+    w0, ab, nw = (torch.randn(hd, generator=g).to(d) for _ in range(3))
+
+    def run(step, state):
+        out = torch.zeros(n, hd, device=d)
+        for at in range(0, n, step):
+            sl = slice(at, min(at + step, n))
+            m = sl.stop - at
+            seq.delta_rule(*(P[sl, i * hd:(i + 1) * hd] for i in range(5)), wl[sl], w0, ab, nw, state, torch.tensor([1], dtype=torch.int32, device=d),
+                           torch.tensor([at + m], dtype=torch.int32, device=d), torch.tensor([0, m], dtype=torch.int32, device=d), out[sl],
+                           0.55, 1e-6, 1e-5, num_seqs=1)
+        return out.cpu(), state[1].cpu()
+
+    (a, sa), (b, sb) = (run(step, torch.zeros(2, H, D, D, device=d)) for step in (n, 8))
+    assert rel(a, b) < 2e-5 and rel(sa, sb) < 2e-5   # 201 steps of fp32 sums in another order, as above
+
+
+@pytest.mark.parametrize("device", DEVICES)
 def test_moe_choice_uses_correction_weights_do_not(device):
     from vgate.ops import seq
     d = _dev(device)
