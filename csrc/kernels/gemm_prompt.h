@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "gemm_epilogue.h"
+#include "lds_rows.h"
 
 namespace vgate {
 
@@ -27,23 +28,6 @@ __device__ __forceinline__ float sumsq8(uint4 v, float acc) {
   acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.y), __builtin_bit_cast(p4_bf2, v.y), acc, false);
   acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.z), __builtin_bit_cast(p4_bf2, v.z), acc, false);
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.w), __builtin_bit_cast(p4_bf2, v.w), acc, false);
-}
-
-// ---- x in LDS: a 16-row x 64-k tile is two 1 KiB pieces of 8 rows ----
-// Eight consecutive lanes of the DMA fetch one row's whole 128-B line. (Gathering MFMA fragments directly, 64 lanes on 16 rows of
-// 64 B each, kept the CU's address path busy four times as long and bounded every tile shape at 20 to 22 B per clock and CU: 1536 x
-// 8960 at 2048 rows as 128 x 128 tiles 115 -> 88 us, 4096 x 4096 as 256 x 128 92 -> 73, 28672 x 4096 as 256 x 128 545 -> 476.) LDS-DMA
-// writes lane-linear, so the 16-B chunks of a row are permuted at the source: chunk c of row r lies at c ^ x_swz(r), which spreads the
-// 16 rows of a fragment read over all banks (SQ_LDS_BANK_CONFLICT 0).
-__device__ __forceinline__ int x_swz(int r) { return (r >> 1) & 7; }
-__device__ __forceinline__ int x_piece_row(int tile_row0, int half, int lane, int M) {
-  const int row = tile_row0 + 8 * half + (lane >> 3);
-  return row < M ? row : M - 1;  // rows past M repeat row M - 1 (never stored)
-}
-__device__ __forceinline__ int x_piece_col(int half, int lane) { return ((lane & 7) ^ x_swz(8 * half + (lane >> 3))) * 8; }
-__device__ __forceinline__ int x_frag_off(int ks, int lane) {
-  const int r = lane & 15;
-  return r * 128 + (((4 * ks + (lane >> 4)) ^ x_swz(r)) << 4);
 }
 
 // The epilogue of a wave's MT x NT tiles of a prompt GEMM (rows m0 + 16 b, tiles nt0 + a; value(a, b): the tile's accumulator, row scale
@@ -143,27 +127,6 @@ __device__ __forceinline__ void prompt_epilogue(const GemmParams& p, int m0, int
       }
     }
   }
-}
-
-// LDS-DMA through a buffer descriptor: 16 B per lane from base + voff + soff to lds + 16 lane (inline asm and vmcnt by the caller, as
-// glds16; no 64-bit address per piece: a wave that issues alone on its SIMD has no slots for those)
-__device__ __forceinline__ void blds16(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
-  unsigned keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep) : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory");
-}
-__device__ __forceinline__ u32x4 rsrc_words(const void* base) {
-  const uint64_t a = reinterpret_cast<uint64_t>(base);
-  return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xffffu)), 0x7fffffffu, 0x00020000u};
-}
-
-// acc += W(A) . X(B) on an accumulator that stays in its AGPRs: up to 256 of them are the whole file, and with the builtin (whose result is
-// another register than its addend) the allocator shuffles them through VGPRs all the way. The compiler does not see an MFMA here, so the
-// waits that it would put around one are the caller's: operands come from LDS (waited for as any asm input) or, written by the VALU, with
-// two wait states between; before the accumulators are read, the last MFMA is given its 16 cycles and more.
-__device__ __forceinline__ void mfma_acc(f32x4& acc, const uint4& w, const uint4& x) {
-  asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(as_bf16x8(w)), "v"(as_bf16x8(x)));
 }
 
 template <int MT, int NT>

@@ -37,8 +37,11 @@
 // (two per tile) wait for LDS traffic only. A row's running max moves only when a tile exceeds it by more than 2^8 (the
 // weights stay below 2^8 then, and the accumulators are rarely rescaled); that is decided per row, so a row's result does
 // not depend on its neighbours. The workgroups with the most keys start first.
+// latent_attn, bf16 caches, prompt portions, latents of 128, 256 or 512 with a rotated part of 64: staged kernel. Pages come into LDS by
+// DMA a step ahead and each wave carries 16 or 32 rows from scores to weighted latents in registers (latent_attn_staged_kernel).
 #include <stdlib.h>
 
+#include "lds_rows.h"
 #include "locate.h"
 #include "seq_launchers.h"
 
@@ -619,6 +622,250 @@ __global__ __launch_bounds__(256) void latent_attn_tiled_kernel(LatentArgs a, co
     }
 }
 
+// Prompt portions, rows of whole 128-B lines (E = 64 NE, rank = 16 NCT): a workgroup owns 64 (token, head) rows, KW of its waves share 16 KW of
+// them and take every KW-th tile of 32 keys (absolute positions, so that a row's sums keep their order). The pages of a step are staged
+// by LDS-DMA, keys as rows of lines (lds_rows.h) and the transposed latents as they lie, one step ahead. A wave computes K Q^T, so that a
+// lane holds eight keys of one row: the row's maximum takes two exchanges, and the weights are the B operand of C^T P as they are, once
+// the latents are read in the same order of keys: nothing but the stages goes through LDS until the KW waves' results are added.
+// What bounds it is the chain of a lone wave per SIMD (products, softmax, products: some 400 instructions between two barriers for 72
+// products) and LDS, per wave and tile of 32 keys 2 NE + NCT KiB of fragments for KW row tiles. The sums stay in AGPRs (mfma_acc, and a
+// read only inside the rare rescaling: hoisted before its branch it was 128 moves per step), latents are asked for before the softmax,
+// masks are a branch (most tiles have none hidden).
+// (latent_attn_tiled_kernel, which this one replaces there: keys straight into registers, 64 lanes on 16 lines for 64 B each, scores and
+// weights through LDS between barriers. 1999 tokens of 8 heads, rank 256: 131 -> 66 us; 3 x 601 tokens of 12 heads among 5 decoded,
+// rank 512: 94 -> 55. On the way: with the builtin products 102 / 90, in AGPRs 83 / 57.)
+template <int NE, int NCT, int KW>
+__global__ __launch_bounds__(256, 1) void latent_attn_staged_kernel(LatentArgs a, const bf16_t* __restrict__ qa, int H,
+                                                                    float scale_log2e, const int32_t* __restrict__ block_tables,
+                                                                    int max_blocks, int num_pages,
+                                                                    const int32_t* __restrict__ context_lens,
+                                                                    const int32_t* __restrict__ query_start, int S,
+                                                                    const bf16_t* __restrict__ cache_t, bf16_t* __restrict__ ol,
+                                                                    int window, const float* __restrict__ sink) {
+  constexpr int E = 64 * NE, KR = 16 * NCT, PP = 2 * NE + NCT / 2;   // 1 KiB pieces of a page: keys, transposed latents
+  constexpr int PPW = KW == 2 ? PP : (2 * NE > NCT / 2 ? 2 * NE : NCT / 2), STAGE = 2 * KW * PP * 1024, STEP = 32 * KW;
+  static_assert(NCT % 8 == 0 && PPW % 2 == 0 && (KW == 1 || KW == 2) && 2 * PPW < 64, "whole pieces, vmcnt");
+  extern __shared__ __attribute__((aligned(16))) char smem[];   // two stages; at the end the KW waves' results
+  int tile;
+  const int s = __builtin_amdgcn_readfirstlane(
+      locate_item(S, (int)(gridDim.x - 1 - blockIdx.x), tile, [&](int i) { return ((query_start[i + 1] - query_start[i]) * H + 63) / 64; }));
+  if (s < 0) return;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, lr = l & 15, lg = l >> 4;
+  const int kw = KW == 2 ? wid & 1 : 0, rw = KW == 2 ? wid >> 1 : wid;
+  const int t0 = query_start[s], ntok = query_start[s + 1] - t0;
+  const int pos0 = context_lens[s] - ntok;
+  const int nrows = ntok * H, row0 = __builtin_amdgcn_readfirstlane(tile) * 64, wrow = row0 + 16 * KW * rw;
+  bf16x8 qf[KW][2 * NE];   // B operands: lane holds Q[row wrow + 16 r + lr][32 i + 8 lg ..]
+  int limit[KW], lowest[KW];   // the row's visible keys: [lowest, limit)
+  float m[KW], lsum[KW];
+#pragma unroll
+  for (int r = 0; r < KW; ++r) {
+    const int row = wrow + 16 * r + lr;
+    const bool ok = row < nrows;
+    const bf16_t* qrow = qa + ((int64_t)(t0 + (ok ? row / H : 0)) * H + (ok ? row % H : 0)) * E;
+#pragma unroll
+    for (int i = 0; i < 2 * NE; ++i) qf[r][i] = as_bf16x8(ld16(qrow + 32 * i + 8 * lg));
+    limit[r] = ok ? pos0 + row / H + 1 : 0;
+    lowest[r] = max(0, limit[r] - window);
+    const bool sk = ok && sink != nullptr && kw == 0;
+    m[r] = sk ? sink[row % H] * 1.4426950408889634f : -INFINITY;
+    lsum[r] = (sk && lg == 0) ? 1.f : 0.f;
+  }
+  const int kmax = __builtin_amdgcn_readfirstlane(pos0 + min(row0 + 63, nrows - 1) / H + 1);
+  const int first = __builtin_amdgcn_readfirstlane(max(0, pos0 + row0 / H + 1 - window)), kmin = first & ~(STEP - 1);
+  const int open = pos0 + row0 / H + 1;   // below: every row's limit is further on
+  const int nsteps = (kmax - kmin + STEP - 1) / STEP;
+  const int32_t* bt = block_tables + (int64_t)s * max_blocks;
+  // this wave's share of a step's pages: page pgw, or (KW = 1) its keys or its latents, the fewer of them some twice
+  const int pgw = KW == 2 ? wid : wid >> 1;
+  auto page_of = [&](int t) {
+    const int j = kmin + STEP * t + 16 * pgw;
+    return min(max(bt[min(j, kmax - 1) >> 4], 0), num_pages - 1);
+  };
+  const uint32_t lds0 = lds_addr_of(smem), cvo = l * 16;
+  uint32_t kvo[2];   // (x_piece_col(), the second page of a tile turned by two chunks: a fragment has rows of both)
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = 8 * i + (l >> 3);
+    kvo[i] = (uint32_t)r * (2u * E) - 1024u * i + (uint32_t)(((l & 7) ^ x_swz(r) ^ ((pgw & 1) << 1)) << 4);
+  }
+  auto issue = [&](int page, int buf) {
+    const u32x4 krs = rsrc_words(reinterpret_cast<const bf16_t*>(a.cache) + (int64_t)page * 16 * E);
+    const u32x4 crs = rsrc_words(cache_t + (int64_t)page * 16 * KR);
+    const uint32_t dst = lds0 + buf * STAGE + (uint32_t)(pgw * PP) * 1024u;
+    constexpr int NK = KW == 2 ? 2 * NE : PPW, NC = KW == 2 ? NCT / 2 : PPW;
+    if (KW == 2 || (wid & 1) == 0) {
+#pragma unroll
+      for (int q = 0; q < NK; q += 2) {
+        const int x = q % (2 * NE);
+        blds16_run<2>(krs, kvo, (uint32_t)(x >> 1) * 128u, dst + x * 1024u);
+      }
+    }
+    if (KW == 2 || (wid & 1) == 1) {
+#pragma unroll
+      for (int q = 0; q < NC; q += q + 4 <= NC ? 4 : 2) {
+        const int x = q % (NCT / 2);
+        if (q + 4 <= NC) blds16_run<4>(crs, {cvo, cvo, cvo, cvo}, (uint32_t)x * 1024u, dst + (2 * NE + x) * 1024u);
+        else blds16_run<2>(crs, {cvo, cvo}, (uint32_t)x * 1024u, dst + (2 * NE + x) * 1024u);
+      }
+    }
+  };
+  f32x4 O[KW][NCT];
+#pragma unroll
+  for (int r = 0; r < KW; ++r)
+#pragma unroll
+    for (int c = 0; c < NCT; ++c) {
+      O[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      asm volatile("" : "+a"(O[r][c]));
+    }
+  // row lr of key fragment k is the tile's key 8 (lr / 4) + 4 k + lr % 4: a lane's scores are then those of keys 8 lg .. 8 lg + 7, which it
+  // meets again as 16 B of a transposed latent
+  int ko[2][2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int pg = lr >> 3, r = ((8 * (lr >> 2)) & 15) + 4 * k + (lr & 3);
+      ko[k][i] = pg * PP * 1024 + r * 128 + (((4 * i + lg) ^ x_swz(r) ^ (pg << 1)) << 4);
+    }
+  const int co = (2 * NE + (lg >> 1) * PP) * 1024 + lr * 32 + (lg & 1) * 16;
+  // (the loads above are waited for here: from now on the counter holds DMA alone)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  issue(page_of(0), 0);
+  issue(page_of(1), 1);
+  int next = page_of(2);
+  for (int t = 0; t < nsteps; ++t) {
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PPW) : "memory");   // the step's pages are there, for every wave
+    const int j0 = kmin + STEP * t + 32 * kw;
+    const char* sb = smem + (t & 1) * STAGE + 2 * kw * PP * 1024;
+    if (j0 < kmax && j0 + 32 > first) {
+      f32x4 sc[KW][2];
+#pragma unroll
+      for (int r = 0; r < KW; ++r) sc[r][0] = sc[r][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 2 * NE; ++i)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const bf16x8 kf = as_bf16x8(*reinterpret_cast<const uint4*>(sb + (i >> 1) * 2048 + ko[k][i & 1]));
+#pragma unroll
+          for (int r = 0; r < KW; ++r) sc[r][k] = mfma16(kf, qf[r][i], sc[r][k]);
+        }
+      constexpr int CA = 16 < NCT ? 16 : NCT;   // latents asked for before the softmax
+      uint4 cf[CA];
+#pragma unroll
+      for (int c = 0; c < CA; ++c) cf[c] = *reinterpret_cast<const uint4*>(sb + co + c * 512);
+      __builtin_amdgcn_sched_barrier(0xf);   // (arithmetic may pass)
+      float v[KW][8], al[KW];
+#pragma unroll
+      for (int r = 0; r < KW; ++r)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[r][e] = sc[r][e >> 2][e & 3] * scale_log2e;
+      if (j0 + 32 > open || j0 < kmax - window) {   // a key that one of the rows doesn't see
+        asm volatile("");   // (a branch)
+#pragma unroll
+        for (int r = 0; r < KW; ++r)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int j = j0 + 8 * lg + e;
+            v[r][e] = (j < limit[r] && j >= lowest[r]) ? v[r][e] : -INFINITY;
+          }
+      }
+      uint4 pf[KW];
+      bool moved = false;
+#pragma unroll
+      for (int r = 0; r < KW; ++r) {
+        float top = v[r][0];
+#pragma unroll
+        for (int e = 1; e < 8; ++e) top = fmaxf(top, v[r][e]);
+        top = fmaxf(top, xor16(top));
+        top = fmaxf(top, xor32(top));
+        const bool move = top > m[r] + LAZY_MAX;   // (m = -inf: the first visible keys; the same in the row's four lanes)
+        moved |= move;
+        al[r] = move ? __builtin_amdgcn_exp2f(m[r] - top) : 1.f;
+        m[r] = move ? top : m[r];
+        const float ms = (m[r] == -INFINITY) ? 0.f : m[r];   // a row that has seen no key yet
+        float w[8], sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          w[e] = __builtin_amdgcn_exp2f(v[r][e] - ms);
+          sum += w[e];
+        }
+        lsum[r] = lsum[r] * al[r] + sum;
+        pf[r] = pack8(w);
+      }
+      if (__any(moved)) {
+#pragma unroll
+        for (int r = 0; r < KW; ++r)
+#pragma unroll
+          for (int c = 0; c < NCT; ++c) {
+            asm volatile("" : "+a"(O[r][c]));   // (read here, not before the branch)
+            O[r][c] *= al[r];
+            asm volatile("" : "+a"(O[r][c]));
+          }
+      }
+#pragma unroll
+      for (int r = 0; r < KW; ++r) {
+        u32x4 pk = __builtin_bit_cast(u32x4, pf[r]);
+        asm volatile("s_nop 1" : "+v"(pk));   // (the wait states that mfma_acc asks for)
+        pf[r] = __builtin_bit_cast(uint4, pk);
+      }
+#pragma unroll
+      for (int c = 0; c < NCT; ++c) {
+        const uint4 f = c < CA ? cf[c < CA ? c : 0] : *reinterpret_cast<const uint4*>(sb + co + c * 512);
+#pragma unroll
+        for (int r = 0; r < KW; ++r) mfma_acc(O[r][c], f, pf[r]);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // every wave is done with the buffer
+    issue(next, t & 1);   // (past the last step: pages that are there, never used)
+    next = page_of(t + 3);
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int r = 0; r < KW; ++r)
+#pragma unroll
+    for (int c = 0; c < NCT; ++c) asm volatile("" : "+a"(O[r][c]));
+  if constexpr (KW == 2) {   // the odd key tiles' results onto the even ones'
+    f32x4* po = reinterpret_cast<f32x4*>(smem) + (rw * 64 + l) ;
+    float* pm = reinterpret_cast<float*>(smem + 2 * KW * NCT * 1024);
+    if (kw == 1) {
+#pragma unroll
+      for (int r = 0; r < KW; ++r) {
+#pragma unroll
+        for (int c = 0; c < NCT; ++c) po[(r * NCT + c) * 128] = O[r][c];
+        pm[(r * 2 + rw) * 128 + l] = m[r];
+        pm[(r * 2 + rw) * 128 + 64 + l] = lsum[r];
+      }
+    }
+    __syncthreads();
+    if (kw == 1) return;
+#pragma unroll
+    for (int r = 0; r < KW; ++r) {
+      const float mo = pm[(r * 2 + rw) * 128 + l], lo = pm[(r * 2 + rw) * 128 + 64 + l];
+      const float M = fmaxf(m[r], mo);
+      const float f0 = exp2f(m[r] - M), f1 = exp2f(mo - M);   // a half that saw no key: max -inf, factor 0
+      lsum[r] = lsum[r] * f0 + lo * f1;
+#pragma unroll
+      for (int c = 0; c < NCT; ++c) O[r][c] = O[r][c] * f0 + po[(r * NCT + c) * 128] * f1;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < KW; ++r) {
+    float tot = lsum[r];
+    tot += xor16(tot);
+    tot += xor32(tot);
+    const float inv = 1.f / tot;
+    const int row = wrow + 16 * r + lr;
+    if (row < nrows) {
+      bf16_t* orow = ol + ((int64_t)(t0 + row / H) * H + row % H) * KR + 4 * lg;
+#pragma unroll
+      for (int c = 0; c < NCT; ++c)
+        *reinterpret_cast<uint2*>(orow + 16 * c) =
+            make_uint2(pack_bf2(O[r][c][0] * inv, O[r][c][1] * inv), pack_bf2(O[r][c][2] * inv, O[r][c][3] * inv));
+    }
+  }
+}
+
 // The rows of a split sequence from the partial results of `parts` workgroups: M = max of the parts' maxima (log2
 // units), sums and weighted latents rescaled by 2^(M_p - M) and added in part order, then normalised and stored.
 // vs: the row stride of the parts' weighted latents.
@@ -666,11 +913,30 @@ bool tiled_prefill() {
   return on;
 }
 
+// Latents of 128, 256 or 512 with a rotated part of 64: rows of whole lines, 16-B aligned (else the tiled kernel)
+template <int NCT>
+bool staged_takes(const LatentArgs& a, const void* qa, const void* cache_t, const void* ol) {
+  const uintptr_t at = reinterpret_cast<uintptr_t>(a.cache) | reinterpret_cast<uintptr_t>(qa) | reinterpret_cast<uintptr_t>(cache_t) |
+                       reinterpret_cast<uintptr_t>(ol);
+  return a.rank == 16 * NCT && a.rot == 64 && at % 16 == 0;
+}
+
 template <int NCT, int NQF>
 void launch_mfma(const LatentArgs& a, const void* qa, int H, float scale, const int32_t* block_tables, int max_blocks,
                  int num_pages, const int32_t* context_lens, const int32_t* query_start, int S, const void* cache_t,
                  void* ol, int window, const float* sink, int parts, float* scratch, hipStream_t st) {
   const int blocks = (a.T * H + 63) / 64 + S;
+  if ((int64_t)a.T * H > 16 * (int64_t)S && tiled_prefill() && staged_takes<NCT>(a, qa, cache_t, ol)) {
+    constexpr int NE = NCT / 4 + 1, KW = NCT <= 16 ? 2 : 1;
+    constexpr int LDS = 2 * 2 * KW * (2 * NE + NCT / 2) * 1024;
+    auto kern = latent_attn_staged_kernel<NE, NCT, KW>;
+    static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS) == hipSuccess;
+    (void)attr;
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), LDS, st, a, reinterpret_cast<const bf16_t*>(qa), H, scale * 1.4426950408889634f,
+                       block_tables, max_blocks, num_pages, context_lens, query_start, S, reinterpret_cast<const bf16_t*>(cache_t),
+                       reinterpret_cast<bf16_t*>(ol), window, sink);
+    return;
+  }
   if ((int64_t)a.T * H > 16 * (int64_t)S && tiled_prefill()) {  // (prompt portions among the step's sequences)
     hipLaunchKernelGGL((latent_attn_tiled_kernel<NCT / 4, (NQF + 3) / 4>), dim3(blocks), dim3(256), 0, st, a,
                        reinterpret_cast<const bf16_t*>(qa), H, scale * 1.4426950408889634f, block_tables, max_blocks, num_pages,

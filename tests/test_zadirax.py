@@ -410,6 +410,55 @@ def test_latent_attention_far_keys_and_edges(device, f32):
     assert rel(oracle_attend(qa.float(), rows.float(), rank, 0.7, ctx - nq + 1), want) > 0.05
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("window", [1 << 30, 50])
+@pytest.mark.parametrize("rank,H", [(128, 8), (256, 8), (256, 3), (512, 12), (512, 1)])
+def test_latent_attention_of_prompts_at_tile_edges(rank, H, window):
+    """Prompt portions whose rows are whole 128-B lines, against 64-bit sums: portions of one token up to several tiles of 64 rows, contexts
+    that end before, at and after a step of 32 or 64 keys, a finite sink, and rows larger after the context. Bound: weights and results are
+    each rounded to bf16, whose unit is 2^-8 (8 bits of precision): 2 * 2^-8 sum p |c|; scores and sums are fp32."""
+    from vgate.ops import seq
+    g = torch.Generator().manual_seed(rank + H)
+    rot, E, scale = 64, rank + 64, 0.05
+    new = [70, 1, 33, 64, 5, 17]
+    ctx = [70, 97, 64, 129, 5, 32]
+    pages = [(c + 15) // 16 for c in ctx]
+    perm = torch.randperm(sum(pages) + 3, generator=g)
+    cache = torch.full((len(perm), 16, E), 30.0, dtype=torch.bfloat16)
+    bt = torch.zeros(len(ctx), max(pages), dtype=torch.int32)
+    rows, at = [], 0
+    for s, c in enumerate(ctx):
+        r = (torch.randn(c, E, generator=g) * (1 + 4 * (torch.rand(c, 1, generator=g) < 0.1))).bfloat16()
+        bt[s, :pages[s]] = perm[at: at + pages[s]].int()
+        for j in range(c):
+            cache[bt[s, j // 16], j % 16] = r[j]
+        rows.append(r.double())
+        at += pages[s]
+    T = sum(new)
+    qa = torch.randn(T, H, E, generator=g).bfloat16()
+    sink = torch.randn(H, generator=g)
+    qs = [0]
+    for n in new:
+        qs.append(qs[-1] + n)
+    assert T * H > 16 * len(new)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    ol = torch.full((T, H, rank), 9.0, dtype=torch.bfloat16, device="cuda")
+    seq.latent_attn(qa.cuda(), cache.cuda(), bt.cuda(), i32(ctx), i32(qs), ol, scale, H, rank, rot,
+                    cache_t=cache[:, :, :rank].transpose(1, 2).contiguous().cuda(), window=window, sink=sink.cuda())
+    ol = ol.double().cpu()
+    for s, c in enumerate(ctx):
+        pos = torch.arange(c - new[s], c)[:, None]
+        key = torch.arange(c)[None]
+        hidden = (key > pos) | (pos - key >= window)
+        sc = torch.einsum("thd,jd->htj", qa[qs[s]: qs[s + 1]].double(), rows[s]) * scale
+        sc = torch.cat([sc.masked_fill(hidden, -math.inf), sink.double()[:, None, None].expand(H, new[s], 1)], -1)
+        p = torch.softmax(sc, -1)[..., :-1]
+        want = (p @ rows[s][:, :rank]).transpose(0, 1)
+        size = (p @ rows[s][:, :rank].abs()).transpose(0, 1)
+        err = (ol[qs[s]: qs[s + 1]] - want).abs()
+        assert bool((err <= 2 * 2.0 ** -8 * size + 1e-4).all()), (s, float((err / (size + 1e-2)).max()))
+
+
 def oracle_attend(qa, rows, rank, scale, first_pos):
     out = torch.zeros(qa.shape[0], qa.shape[1], rank)
     for i in range(qa.shape[0]):
