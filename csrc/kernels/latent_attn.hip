@@ -729,7 +729,14 @@ __global__ __launch_bounds__(256, 1) void latent_attn_staged_kernel(LatentArgs a
       ko[k][i] = pg * PP * 1024 + r * 128 + (((4 * i + lg) ^ x_swz(r) ^ (pg << 1)) << 4);
     }
   const int co = (2 * NE + (lg >> 1) * PP) * 1024 + lr * 32 + (lg & 1) * 16;
-  // (the loads above are waited for here: from now on the counter holds DMA alone)
+  // the loads above are waited for here, and the compiler sees that: from now on the counter holds DMA alone (a wait for the queries inside
+  // the loop waits for the next step's pages too)
+#pragma unroll
+  for (int r = 0; r < KW; ++r) {
+#pragma unroll
+    for (int i = 0; i < 2 * NE; ++i) asm volatile("" : "+v"(qf[r][i]));
+    asm volatile("" : "+v"(m[r]));
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   issue(page_of(0), 0);
   issue(page_of(1), 1);
@@ -781,17 +788,11 @@ __global__ __launch_bounds__(256, 1) void latent_attn_staged_kernel(LatentArgs a
         top = fmaxf(top, xor32(top));
         const bool move = top > m[r] + LAZY_MAX;   // (m = -inf: the first visible keys; the same in the row's four lanes)
         moved |= move;
-        al[r] = move ? __builtin_amdgcn_exp2f(m[r] - top) : 1.f;
+        al[r] = move ? exp2f(m[r] - top) : 1.f;   // (not the bare instruction, for which results below 2^-126 are zero)
         m[r] = move ? top : m[r];
         const float ms = (m[r] == -INFINITY) ? 0.f : m[r];   // a row that has seen no key yet
-        float w[8], sum = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          w[e] = __builtin_amdgcn_exp2f(v[r][e] - ms);
-          sum += w[e];
-        }
-        lsum[r] = lsum[r] * al[r] + sum;
-        pf[r] = pack8(w);
+        lsum[r] = lsum[r] * al[r] + weights8(v[r], ms);
+        pf[r] = pack8(v[r]);
       }
       if (__any(moved)) {
 #pragma unroll

@@ -58,4 +58,23 @@ __device__ __forceinline__ void mfma_acc(f32x4& acc, const uint4& w, const uint4
   asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(as_bf16x8(w)), "v"(as_bf16x8(x)));
 }
 
+// eight scores in log2 units become softmax weights 2^(v - ms), and their sum. (The bare instruction gives zero below 2^-126, where a
+// large value may still count: a wave that meets such a weight takes exp2f(), five instructions more each.)
+__device__ __forceinline__ float weights8(float (&v)[8], float ms) {
+  float least = v[0];
+#pragma unroll
+  for (int e = 1; e < 8; ++e) least = fminf(least, v[e]);
+  float sum = 0.f;
+  if (__any(least - ms < -126.f)) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = exp2f(v[e] - ms);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = __builtin_amdgcn_exp2f(v[e] - ms);
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sum += v[e];
+  return sum;
+}
+
 }  // namespace vgate
