@@ -222,7 +222,7 @@ __device__ __forceinline__ float ld_as_float<bf16_t>(const bf16_t* p, int64_t i)
 
 template <typename T>
 __global__ __launch_bounds__(256) void window_pool_kernel(WindowArgs a) {
-  __shared__ int32_t pages[64];  // the pages of the block's rows, a stretch of up to 64 at a time
+  __shared__ int64_t rows[64];  // where a stretch of the block's rows lies, in rows of one head
   const int t = blockIdx.x;
   if (t >= a.query_start[a.S]) return;
   const int e = a.positions[t], P = a.pool;
@@ -232,11 +232,13 @@ __global__ __launch_bounds__(256) void window_pool_kernel(WindowArgs a) {
   const int G = a.G, D = a.D, V = a.V, page = a.page;
   const int64_t dpg = bt[e / page];
   const int drow = (e % page) / P;
-  const int j0 = e + 1 - P, pg_first = j0 / page, npg = e / page - pg_first + 1;
+  const int j0 = e + 1 - P;
   const int nx = G * (D + V);
-  // every thread sums one element over the block's rows in position order; the page ids come from LDS, so a
-  // row's loads do not wait for a block-table load and sixteen rows are in flight (the rows were written by
-  // the launch before, mostly on other XCDs: each batch costs a trip past the L2)
+  // every thread sums one element over the block's rows in position order; where the rows lie comes from LDS, so a row's load waits for
+  // no block-table load and no division, and 32 rows are in flight (the rows were written by the launch before, mostly on other XCDs:
+  // each batch costs a trip past the L2).
+  // What bounds it is that chain: 28 blocks of 64 tokens among 1801, 2 heads of 128 + 128, 28.7 us with 16 rows in flight and two
+  // divisions per row, 13.6 now
   {  // blockIdx.y: which 256 elements
     const int x = blockIdx.y * blockDim.x + threadIdx.x;
     const bool on = x < nx;
@@ -244,24 +246,21 @@ __global__ __launch_bounds__(256) void window_pool_kernel(WindowArgs a) {
     const int y = isk ? x : x - G * D;
     const int w = isk ? D : V;
     const int g = on ? y / w : 0, i = on ? y % w : 0;
-    const T* src = reinterpret_cast<const T*>(isk ? a.kc : a.vc);
+    const T* src = reinterpret_cast<const T*>(isk ? a.kc : a.vc) + (int64_t)g * page * w + i;
     float sum = 0.f;
-    for (int pb = 0; pb < npg; pb += 64) {
+    for (int jb = j0; jb <= e; jb += 64) {
+      const int n = min(64, e + 1 - jb);
       __syncthreads();
-      if ((int)threadIdx.x < min(64, npg - pb)) pages[threadIdx.x] = bt[pg_first + pb + threadIdx.x];
+      if ((int)threadIdx.x < n) rows[threadIdx.x] = (int64_t)bt[(jb + (int)threadIdx.x) / page] * G * page + (jb + (int)threadIdx.x) % page;
       __syncthreads();
-      const int ja = max(j0, (pg_first + pb) * page), jb = min(e, (pg_first + min(npg, pb + 64)) * page - 1);
       if (on) {
-        for (int j = ja; j <= jb; j += 16) {  // sixteen rows' loads in flight, added in position order
-          float v[16];
+        for (int j = 0; j < n; j += 32) {  // 32 rows' loads in flight, added in position order
+          float v[32];
 #pragma unroll
-          for (int u = 0; u < 16; ++u) {
-            const int jj = min(j + u, jb);
-            v[u] = ld_as_float<T>(src, (((int64_t)pages[jj / page - pg_first - pb] * G + g) * page + jj % page) * w + i);
-          }
+          for (int u = 0; u < 32; ++u) v[u] = ld_as_float<T>(src, rows[min(j + u, n - 1)] * w);
 #pragma unroll
-          for (int u = 0; u < 16; ++u)
-            if (j + u <= jb) sum += v[u];
+          for (int u = 0; u < 32; ++u)
+            if (j + u < n) sum += v[u];
         }
       }
     }
