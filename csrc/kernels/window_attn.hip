@@ -44,11 +44,13 @@
 //               are seen beside the window. Their key tiles (those before the window's first tile) come first (KEEP
 //               instantiations of the MFMA kernels); a tile that holds both kinds is one of the window's.
 // Value mixing: window_write can blend a token's values with another row of values of the same token (fp32).
+// window_attn, prompt portions with keys and values of 128, no distance term, no softcap: staged kernel (window_attn_staged_kernel).
 // Every row of every kernel depends only on its own sequence's cache rows, in an order fixed by the
 // position, so results do not depend on how a prompt is cut or what else is in the batch.
 #include <algorithm>
 #include <type_traits>
 
+#include "lds_rows.h"
 #include "locate.h"
 #include "seq_launchers.h"
 
@@ -1057,6 +1059,237 @@ __global__ __launch_bounds__(256, 2) void window_attn_tiled_kernel(WindowArgs a,
   }
 }
 
+// A row's reference moves only when a tile exceeds it by more than 2^8: weights and sums stay below 2^8 times what the largest would give
+// (as 256 equal keys do), and the sums are rarely rescaled. That is decided per row.
+constexpr float LAZY_MAX = 8.f;
+// Prompt portions, keys and values of 128 (whole 128-B lines), neither distance term nor softcap: 64 rows per workgroup, 16 per wave, over
+// steps of 64 keys at absolute positions, whose pages come into LDS by DMA one step ahead: keys as rows of lines (lds_rows.h), transposed
+// values as they lie. A wave computes K Q^T, so that a lane holds 16 scores of one row: the row's maximum takes two exchanges where it took
+// sixteen, and the weights are the B operand of V^T P as they are, once the values are read in the same order of keys. Pooled rows are
+// brought into the same places by the threads, 64 at a time, and come first.
+// What bounds it is the chain of the wave (scores, softmax, values), then LDS, 16 KiB of fragments per wave and 32 keys.
+// (window_attn_tiled_kernel, which this one replaces there, 300 vector operations a tile and wave: 1801 tokens of 8 heads, window 1024,
+// 55 -> 20.5 us, and 67 -> 28 with pooled blocks and turned values; 3 x 601 tokens of 12 heads with kept first ones among decoded tokens
+// 43 -> 22.5. Four waves with both tiles each 36; two stages and two barriers a step 34; the page table by vector loads, whose waits
+// drain the DMA, 29.)
+__global__ __launch_bounds__(512, 4) void window_attn_staged_kernel(WindowArgs a, const int32_t* __restrict__ tables,
+                                                                    const bf16_t* __restrict__ q, float scale_log2e,
+                                                                    const bf16_t* __restrict__ vt, int num_pages, bf16_t* __restrict__ out) {
+  constexpr int D = 128, PP = 8, STAGE = 4 * PP * 1024;   // 1 KiB pieces of a page: four of keys, four of values
+  __shared__ __attribute__((aligned(16))) char smem[3 * STAGE];
+  const int G = a.G, H = a.H, rep = H / G, g = blockIdx.y, P = a.pool, GV = a.GV, gv = g / (G / GV);
+  int tile;
+  const int s = __builtin_amdgcn_readfirstlane(locate_item(
+      a.S, (int)(gridDim.x - 1 - blockIdx.x), tile, [&](int i) { return ((a.query_start[i + 1] - a.query_start[i]) * rep + 63) / 64; }));
+  if (s < 0) return;
+  const int tid = threadIdx.x, wid = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, lr = l & 15, lg = l >> 4;
+  const int t0 = a.query_start[s], ntok = a.query_start[s + 1] - t0, pos0 = a.context_lens[s] - ntok, nrows = ntok * rep;
+  const int rw = wid & 3, kw = wid >> 2;   // the wave's rows, and which of a step's two tiles of 32 keys it takes
+  const int rowb = __builtin_amdgcn_readfirstlane(tile) * 64, row0 = rowb + 16 * rw;
+  if (rowb >= nrows) return;
+  const bool active = row0 < nrows;   // an idle wave still brings its pages and meets the barriers
+  const int row = row0 + lr;          // this lane's row
+  const bool ok = row < nrows;
+  const int p = pos0 + (ok ? row / rep : 0), h = g * rep + (ok ? row % rep : 0);
+  const int64_t t = t0 + (ok ? row / rep : 0);
+  bf16x8 qf[4];   // B operands: lane holds Q[row][32 i + 8 lg ..]
+#pragma unroll
+  for (int i = 0; i < 4; ++i) qf[i] = as_bf16x8(ld16(q + (t * H + h) * D + 32 * i + 8 * lg));
+  const int hi = ok ? p : -1, lo = first_key(a, p), nb = (ok && P > 0) ? max(0, lo) / P : 0;
+  const bool sk = ok && a.sink != nullptr && kw == 0;
+  float m = sk ? a.sink[h] * 1.4426950408889634f : -INFINITY;
+  float lsum = (sk && lg == 0) ? 1.f : 0.f;
+  f32x4 O[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) O[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // the workgroup's positions, and the wave's
+  const int pminb = pos0 + rowb / rep, pmaxb = pos0 + min(rowb + 63, nrows - 1) / rep;
+  const int pminw = pos0 + row0 / rep, pmaxw = pos0 + min(row0 + 15, nrows - 1) / rep;
+  const int klow = max(0, first_key(a, pminw)), lomax = first_key(a, pmaxw);
+  const int32_t* bt = tables + (int64_t)s * a.max_blocks;   // (a.block_tables, as a scalar load: a vector load's wait is one for the DMA too)
+  // row lr of key fragment k is the tile's key 8 (lr / 4) + 4 k + lr % 4: a lane's scores are then those of keys 8 lg .. 8 lg + 7, which it
+  // meets again as 16 B of a transposed value; the second page of a tile is turned by two chunks, a fragment has rows of both
+  int ko[2][2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int pg = lr >> 3, r = ((8 * (lr >> 2)) & 15) + 4 * k + (lr & 3);
+      ko[k][i] = pg * PP * 1024 + r * 128 + (((4 * i + lg) ^ x_swz(r) ^ (pg << 1)) << 4);
+    }
+  const int co = (4 + (lg >> 1) * PP) * 1024 + lr * 32 + (lg & 1) * 16;
+
+  // the 32 keys from `kbase` on; pooled: below nbw they are seen by some row of the wave
+  auto keys = [&](auto pooled, const char* sb, int kbase, int nbw) {
+    constexpr bool POOLED = decltype(pooled)::value;
+    f32x4 sc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) sc[k] = mfma16(as_bf16x8(*reinterpret_cast<const uint4*>(sb + (i >> 1) * 2048 + ko[k][i & 1])), qf[i], sc[k]);
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = sc[e >> 2][e & 3] * scale_log2e;
+    if (POOLED || kbase < lomax || kbase + 31 > pminw) {   // a key that one of the rows doesn't see
+      asm volatile("");   // (a branch)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int j = kbase + 8 * lg + e;
+        const bool vis = POOLED ? j < nb : ((j >= lo || j < a.keep) && j <= hi);
+        v[e] = vis ? v[e] : -INFINITY;
+      }
+    }
+    float top = v[0];
+#pragma unroll
+    for (int e = 1; e < 8; ++e) top = fmaxf(top, v[e]);
+    top = fmaxf(top, xor16(top));
+    top = fmaxf(top, xor32(top));
+    const bool move = top > m + LAZY_MAX;   // (m = -inf: the first visible keys; the same in the row's four lanes)
+    if (__any(move)) {
+      const float al = move ? exp2f(m - top) : 1.f;   // (not the bare instruction, for which results below 2^-126 are zero)
+      m = move ? top : m;
+      lsum *= al;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) O[c] *= al;
+    }
+    const float ms = (m == -INFINITY) ? 0.f : m;   // a row that has seen no key yet
+    lsum += weights8(v, ms);
+    const bf16x8 pf = as_bf16x8(pack8(v));
+    uint32_t on[4];
+    if (POOLED) {   // what no row of the wave sees has weights of zero, and may be no number
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int k = kbase + 8 * lg + 2 * j;
+        on[j] = (k < nbw ? 0xffffu : 0u) | (k + 1 < nbw ? 0xffff0000u : 0u);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      uint4 f = *reinterpret_cast<const uint4*>(sb + co + c * 512);
+      if (POOLED) f = make_uint4(f.x & on[0], f.y & on[1], f.z & on[2], f.w & on[3]);
+      O[c] = mfma16(as_bf16x8(f), pf, O[c]);
+    }
+  };
+
+  const int nbb = P > 0 ? max(0, first_key(a, pmaxb)) / P : 0, nbw = (active && P > 0) ? max(0, lomax) / P : 0;   // pooled rows seen
+  for (int b0 = 0; b0 < nbb; b0 += 64) {
+    const bf16_t* kp = reinterpret_cast<const bf16_t*>(a.kp);
+    const bf16_t* vp = reinterpret_cast<const bf16_t*>(a.vp);
+    uint4 kr[2], vr[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int key = (tid + 512 * u) >> 4, ch = tid & 15, e = min(b0 + key, nbb - 1) * P + P - 1;
+      const int64_t r = ((int64_t)min(max(bt[e >> 4], 0), num_pages - 1) * G + g) * a.npool + (e & 15) / P;
+      kr[u] = ld16(kp + r * D + 8 * ch);
+      vr[u] = ld16(vp + r * D + 8 * ch);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int key = (tid + 512 * u) >> 4, ch = tid & 15, pg = key >> 4, r = key & 15;
+      char* to = smem + pg * PP * 1024;
+      *reinterpret_cast<uint4*>(to + (ch >> 3) * 2048 + r * 128 + (((ch & 7) ^ x_swz(r) ^ ((pg & 1) << 1)) << 4)) = kr[u];
+      const uint32_t w[4] = {vr[u].x, vr[u].y, vr[u].z, vr[u].w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) *reinterpret_cast<bf16_t*>(to + 4096 + (8 * ch + e) * 32 + r * 2) = (bf16_t)(w[e >> 1] >> (16 * (e & 1)));
+    }
+    __syncthreads();
+    if (b0 + 32 * kw < nbw) keys(std::true_type{}, smem + kw * 2 * PP * 1024, b0 + 32 * kw, nbw);
+    __syncthreads();
+  }
+
+  // steps of kept first tokens, then the window's
+  const int js0 = max(0, first_key(a, pminb)) >> 6, js1 = pmaxb >> 6, nkept = min((a.keep + 63) >> 6, js0);
+  const int nsteps = nkept + js1 - js0 + 1;
+  auto first_of = [&](int i) { return 64 * (i < nkept ? i : js0 + i - nkept); };
+  auto page_of = [&](int i) { return min(max(bt[min(first_of(min(i, nsteps - 1)) + 16 * rw, pmaxb) >> 4], 0), num_pages - 1); };
+  const uint32_t lds0 = lds_addr_of(smem) + (uint32_t)(rw * PP + 4 * kw) * 1024u;   // a wave brings the keys or the values of a step's page rw
+  uint32_t vo[4] = {l * 16u, l * 16u, l * 16u, l * 16u};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = 8 * i + (l >> 3);
+    if (kw == 0) vo[i] = (uint32_t)r * (2u * D) - 1024u * i + (uint32_t)(((l & 7) ^ x_swz(r) ^ ((rw & 1) << 1)) << 4);
+  }
+  auto issue = [&](int page, int buf) {
+    const uint32_t dst = lds0 + buf * STAGE;
+    if (kw == 0) {
+      const u32x4 rs = rsrc_words(reinterpret_cast<const bf16_t*>(a.kc) + ((int64_t)page * G + g) * 16 * D);
+      blds16_run<2>(rs, {vo[0], vo[1]}, 0u, dst);
+      blds16_run<2>(rs, {vo[0], vo[1]}, 128u, dst + 2048u);
+    } else {
+      blds16_run<4>(rsrc_words(vt + ((int64_t)page * GV + gv) * 16 * D), vo, 0u, dst);
+    }
+  };
+  auto sees = [&](int kbase) { return active && (kbase + 31 >= klow || kbase < a.keep) && kbase <= pmaxw; };
+  // the loads above are waited for here, and the compiler sees that: from now on the counter holds DMA alone (a wait for the queries inside
+  // the loop waits for the next step's pages too)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(qf[i]));
+  asm volatile("" : "+v"(m));
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  issue(page_of(0), 0);
+  issue(page_of(1), 1);
+  int next = page_of(2), buf = 0;
+  for (int i = 0; i < nsteps; ++i) {
+    // the step's pages are there, for every wave, and every wave is done with the step before, whose buffer is the next to be filled
+    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    issue(next, buf == 0 ? 2 : buf - 1);   // (past the last step: pages that are there, never used)
+    next = page_of(i + 3);
+    const int kbase = first_of(i) + 32 * kw;
+    if (sees(kbase)) keys(std::false_type{}, smem + buf * STAGE + kw * 2 * PP * 1024, kbase, 0);
+    buf = buf == 2 ? 0 : buf + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");   // (the last DMA has landed)
+  lsum += xor16(lsum);
+  lsum += xor32(lsum);
+  // the odd tiles' results onto the even ones'
+  f32x4* po = reinterpret_cast<f32x4*>(smem) + rw * 64 + l;
+  float* pm = reinterpret_cast<float*>(smem + STAGE) + rw * 64 + l;
+  if (kw == 1) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) po[c * 256] = O[c];
+    pm[0] = m;
+    pm[256] = lsum;
+  }
+  __syncthreads();
+  if (kw == 1) return;
+  {
+    const float mo = pm[0], M = fmaxf(m, mo), Ms = (M == -INFINITY) ? 0.f : M;   // (rows past the sequence's last)
+    const float f0 = exp2f(m - Ms), f1 = exp2f(mo - Ms);   // a half that saw no key: max -inf, factor 0
+    lsum = lsum * f0 + pm[256] * f1;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) O[c] = O[c] * f0 + po[c * 256] * f1;
+  }
+  if (!ok) return;
+  const float inv = 1.f / lsum, fp = -(float)p;
+  bf16_t* orow = out + (t * H + h) * D;
+  const bf16_t* grow = a.gate == nullptr ? nullptr : reinterpret_cast<const bf16_t*>(a.gate) + t * a.ldg + (int64_t)h * D;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {   // columns 16 c + 4 lg ..
+    const int col = 16 * c + 4 * lg;
+    f32x4 y = O[c] * inv;
+    if (a.v_freq != nullptr) {
+#pragma unroll
+      for (int j = 0; j < 4; j += 2) {
+        const float ang = fp * a.v_freq[(col + j) >> 1], cs = cosf(ang), sn = sinf(ang), y0 = y[j], y1 = y[j + 1];
+        y[j] = y0 * cs - y1 * sn;
+        y[j + 1] = y1 * cs + y0 * sn;
+      }
+    }
+    if (grow != nullptr) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] *= gate_of(grow, col + j);
+    }
+    *reinterpret_cast<uint2*>(orow + col) = make_uint2(pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3]));
+  }
+}
+
+// (whole lines of keys and values, 16-B aligned; else the tiled kernel)
+bool staged_takes(const WindowArgs& a, const void* q, const void* vt, const void* out) {
+  const uintptr_t at = reinterpret_cast<uintptr_t>(a.kc) | reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(vt) |
+                       reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(a.kp) | reinterpret_cast<uintptr_t>(a.vp);
+  return a.D == 128 && a.V == 128 && at % 16 == 0;
+}
+
 template <int NCT, int NQF, int BIAS, bool CAP, bool KEEP>
 void launch_window_mfma(const WindowArgs& a, const void* q, float scale, const void* vt, int num_pages, void* out,
                         hipStream_t st) {
@@ -1078,6 +1311,9 @@ void launch_window_mfma(const WindowArgs& a, const void* q, float scale, const v
   }
   else if (a.prefill_kernel == 1 || NCT > 8)
     hipLaunchKernelGGL((window_attn_mfma_kernel<NCT, NQF, 4, BIAS, CAP, KEEP>), dim3(blocks, a.G), dim3(256), dyn, st, a, qp, sl, vp, num_pages, op);
+  else if (BIAS == 0 && !CAP && NCT == 8 && staged_takes(a, q, vt, out))
+    hipLaunchKernelGGL(window_attn_staged_kernel, dim3((a.T * rep + 63) / 64 + a.S, a.G), dim3(512), 0, st, a, a.block_tables, qp, sl, vp,
+                       num_pages, op);
   else
     hipLaunchKernelGGL((window_attn_tiled_kernel<NCT, NQF, BIAS, CAP, KEEP>), dim3((a.T * rep + 63) / 64 + a.S, a.G), dim3(256), dyn, st, a, qp, sl,
                        vp, num_pages, op);

@@ -679,3 +679,49 @@ def test_linear_attention_long_portions(device, D, V):
         o3 = step([(A, 650, 50)], [2], [700], state, cols)                      # short step: one pass from the slot
         assert rel(torch.cat([o1, o2[:200], o3]), wa) < 5e-5, cols
         assert rel(o2[200:], wb) < 5e-5, cols
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,size,pool,keep,chunk,turn", [
+    (8, 2, 100, 0, 0, 0, False), (8, 2, 20, 4, 0, 0, True), (3, 3, 64, 48, 0, 0, False), (12, 2, 50, 0, 40, 0, False),
+    (4, 1, 33, 0, 1, 0, True), (8, 2, 1 << 20, 0, 0, 70, False), (5, 1, 1, 0, 65, 0, False)])
+def test_window_attention_of_prompts_at_tile_edges(H, G, size, pool, keep, chunk, turn):
+    """Prompt portions with keys and values of whole lines, against the reference in fp32 on the same (bf16) numbers: portions of one token
+    up to several tiles of 64 rows, contexts that end before, at and after a step of 64 keys, more than 64 pooled rows, kept first tokens
+    over a step's edge, a sink and a gate. Bound: weights and results are each rounded to bf16 (2^-8): 2 * 2^-8 sum p |v|, of a turned
+    pair's both entries; the gate's own exponential and the fp32 sums are within the constant."""
+    from vgate.ops import seq
+    g = torch.Generator().manual_seed(H + size)
+    D, new, ctx = 128, [70, 1, 33, 64, 5, 200], [70, 97, 64, 129, 5, 330]
+    pages = [(c + 15) // 16 for c in ctx]
+    perm = torch.randperm(sum(pages) + 2, generator=g).int()
+    npool = (16 + pool - 1) // pool if pool else 0
+    r = lambda *shape: torch.randn(*shape, generator=g).bfloat16()  # noqa: E731
+    kc, vc = r(len(perm), G, 16, D), r(len(perm), G, 16, D)
+    kp, vp = (r(len(perm), G, npool, D), r(len(perm), G, npool, D)) if pool else (None, None)
+    kc[::3] *= 3                                             # some keys well ahead of the others
+    bt = torch.zeros(len(ctx), max(pages), dtype=torch.int32)
+    for s, n in enumerate(pages):
+        bt[s, :n] = perm[sum(pages[:s]): sum(pages[:s]) + n]
+    T, qs = sum(new), [0]
+    for n in new:
+        qs.append(qs[-1] + n)
+    assert T * (H // G) > 16 * len(new)
+    q, gate, sink = r(T, H * D), r(T, H * D), torch.randn(H, generator=g)
+
+    def run(device, dt, values, pooled, with_gate=True, turned=turn):
+        to = lambda x: None if x is None else x.to(device, dt)  # noqa: E731
+        i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=device)  # noqa: E731
+        vf = seq.rope_inv_freq(D, 30.0, torch.device(device)) if turned else None
+        out = torch.full((T, H * D), 9.0, device=device, dtype=dt)
+        vt = to(values).transpose(2, 3).contiguous() if device == "cuda" else None
+        seq.window_attn(to(q), to(kc), to(values), to(kp), to(pooled), bt.to(device), i32(ctx), i32(qs), out, 0.1, H, size, pool,
+                        sink.to(device), vf, vt=vt, gate=to(gate) if with_gate else None, keep=keep, chunk=chunk)
+        return out.float().cpu()
+
+    got, want = run("cuda", torch.bfloat16, vc, vp), run("cpu", torch.float32, vc, vp)
+    most = run("cpu", torch.float32, vc.abs(), None if vp is None else vp.abs(), False, False)
+    if turn:
+        most = most.view(T, -1, 2).sum(-1, keepdim=True).expand(-1, -1, 2).reshape(T, -1)
+    err = (got - want).abs()
+    assert bool((err <= 2 * 2.0 ** -8 * most + 2e-4).all()), float((err / (most + 1e-2)).max())
