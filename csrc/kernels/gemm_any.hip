@@ -381,7 +381,9 @@ __global__ __launch_bounds__(256) void gemm_any_rows_kernel(AnyGemmArgs p) {
 // 20.4 -> 20.0, warm 21.8 -> 16.6). Where K is short and workgroups are many, the registers of the second step are better spent on a fourth
 // workgroup per CU: 12 products of 512 x 128 at 2048 rows 14.2 -> 13.6, 16 19.0 -> 16.8 (two workgroups per CU: 10.2 -> 10.6).
 constexpr int LM = 128, LKS = 32, LPAD = LKS + 8;
-template <int DUAL, int AHEAD>
+// GATED: whole pieces with a gate, whose work in every store would slow the forms without one (12 products of 512 x 128 at 2048 rows
+// 13.4 -> 17.9 us).
+template <int DUAL, int AHEAD, bool GATED>
 __global__ __launch_bounds__(256, 3) void gemm_any_lds_kernel(AnyGemmArgs p) {
   constexpr int WN = DUAL ? 64 : 128;  // columns of each weight matrix per block
   constexpr int OPAD = WN + 8;         // padded row of the staged outputs
@@ -488,7 +490,27 @@ __global__ __launch_bounds__(256, 3) void gemm_any_lds_kernel(AnyGemmArgs p) {
       buf ^= 1;
     }
   }
-  if (p.vec_out) {  // bf16 rows of whole 16-B pieces: staged in LDS (the k loop's last barrier has freed it), then stored whole
+  if (GATED || p.vec_out) {  // bf16 rows of whole 16-B pieces: staged in LDS (the k loop's last barrier has freed it), then stored whole
+    // a gate: one logit per row, or its tile brought in whole pieces to where the outputs will lie, each lane's to its own
+    const bool tiled = GATED && p.g_cs != 0, rowed = GATED && p.g_cs == 0;
+    float rg[4][4];
+    if (rowed) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int64_t at = (int64_t)min(r0 + wm * 64 + i * 16 + 4 * lg + e, rend - 1) * p.ldg + b * p.g_bs;
+          rg[i][e] = sigmoidf_(p.gate_f32 ? reinterpret_cast<const float*>(p.gate)[at] : bf2f(reinterpret_cast<const bf16_t*>(p.gate)[at]));
+        }
+    } else if (tiled) {
+      const bf16_t* gate = reinterpret_cast<const bf16_t*>(p.gate) + b * p.g_bs;
+#pragma unroll
+      for (int u = 0; u < LM * WN / 8 / 256; ++u) {
+        const int x = tid + 256 * u, row = x / (WN / 8), col = (x % (WN / 8)) * 8;
+        if (n0 + col < p.N) *reinterpret_cast<uint4*>(&smem[row * OPAD + col]) = ld16(gate + (int64_t)min(r0 + row, rend - 1) * p.ldg + n0 + col);
+      }
+      __syncthreads();
+    }
     with_act<DUAL>(p, [&](auto act) {
 #pragma unroll
       for (int j = 0; j < (DUAL ? 2 : 4); ++j) {
@@ -497,9 +519,13 @@ __global__ __launch_bounds__(256, 3) void gemm_any_lds_kernel(AnyGemmArgs p) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            smem[(wm * 64 + i * 16 + 4 * lg + e) * OPAD + col] =
-                f2bf(act_val<decltype(act)::value>(p, acc[i][j][e] + bias, DUAL ? acc[i][j + 2][e] : 0.f));
+          for (int e = 0; e < 4; ++e) {
+            bf16_t* at = &smem[(wm * 64 + i * 16 + 4 * lg + e) * OPAD + col];
+            float v = act_val<decltype(act)::value>(p, acc[i][j][e] + bias, DUAL ? acc[i][j + 2][e] : 0.f);
+            if (rowed) v *= rg[i][e];
+            if (tiled) v *= sigmoidf_(bf2f(*at));
+            *at = f2bf(v);
+          }
       }
     });
     __syncthreads();
@@ -681,15 +707,21 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st) {
     const bool wide = al && broad && (!g.group_off || g.M > (g.M >= 1024 ? 15 : 32) * g.groups);
     const dim3 gridw((g.N + 127) / 128, mt, g.batch);
     // enough 128-row tiles; also where whole 128-column tiles of many products fill half the chip (us at 2048 rows: 12 of
-    // 128 x 512 27.9 -> 15.8, 8 of 256 x 128 14.1 -> 7.3, 2 of 128 x 256 stay at 9; with a gate per output the small tiles are ahead)
+    // 128 x 512 27.9 -> 15.8, 8 of 256 x 128 14.1 -> 7.3, 2 of 128 x 256 stay at 9; with gates, which come
+    // through LDS in whole pieces, from 192 tiles on: 12 of 128 x 512 30.8 -> 23.7, 8 of 128 x 256 15.3, as wide tiles 18.3)
     const int mt128 = (g.M + LM - 1) / LM + (g.group_off ? g.groups : 0);
-    const bool heads = al && !dual && !g.group_off && g.gate == nullptr && g.N % 128 == 0 && (int64_t)(g.N / 128) * mt128 * g.batch >= 128;
+    const bool gates = g.gate == nullptr || g.g_cs == 0 || (g.g_cs == 1 && !g.gate_f32 && g.ldg % 8 == 0 && g.g_bs % 8 == 0 && a16(g.gate));
+    const bool vec = !g.out_f32 && gates && !(dual && g.gate != nullptr) && g.N % 8 == 0 && g.ldo % 8 == 0 && g.o_bs % 8 == 0 && a16(g.out);
+    const bool heads = al && !dual && !g.group_off && (g.gate == nullptr || vec) && g.N % 128 == 0 &&
+                       (int64_t)(g.N / 128) * mt128 * g.batch >= (g.gate != nullptr ? 192 : 128);
     if ((wide || heads) && g.M >= 1024 && lds_tiles()) {
       AnyGemmArgs v = g;
-      v.vec_out = !g.out_f32 && g.gate == nullptr && g.N % 8 == 0 && g.ldo % 8 == 0 && g.o_bs % 8 == 0 && a16(g.out);
+      v.vec_out = vec;
       const dim3 grid2((g.N + (dual ? 63 : 127)) / (dual ? 64 : 128), mt128, g.batch);
       const bool one = !dual && g.K <= 256 && (int64_t)grid2.x * grid2.y * grid2.z > 512;
-      auto kern = dual ? gemm_any_lds_kernel<1, 2> : (one ? gemm_any_lds_kernel<0, 1> : gemm_any_lds_kernel<0, 2>);
+      const bool gated = v.vec_out && g.gate != nullptr;
+      auto kern = dual ? gemm_any_lds_kernel<1, 2, false>
+                       : (gated ? gemm_any_lds_kernel<0, 2, true> : (one ? gemm_any_lds_kernel<0, 1, false> : gemm_any_lds_kernel<0, 2, false>));
       hipLaunchKernelGGL(kern, grid2, block, 0, st, v);
     } else if (dual && wide) hipLaunchKernelGGL((gemm_any_mfma_kernel<1, true, 4>), gridw, block, 0, st, g);
     else if (wide) hipLaunchKernelGGL((gemm_any_mfma_kernel<0, true, 4>), gridw, block, 0, st, g);

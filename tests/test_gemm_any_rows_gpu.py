@@ -39,6 +39,25 @@ def test_batches_with_gates(M, gate_dt):
     _close(out, torch.matmul(a.float(), w.float().transpose(1, 2)) * torch.sigmoid(gate.float()), K)
 
 
+@pytest.mark.parametrize("kind", ["outputs", "rows", "rows fp32", "outputs fp32", "outputs off 16 B"])
+@pytest.mark.parametrize("M,B,N,K", [(1412, 16, 128, 72), (1025, 11, 256, 512), (2047, 12, 128, 8)])
+def test_long_batches_with_gates(M, B, N, K, kind):
+    """Products of whole 128-column tiles that fill the chip: a gate per output (its tile through LDS), one per row, and the gates that
+    the 64-row tiles keep; rows past the last whole tile, K below and past a step."""
+    g = torch.Generator("cuda").manual_seed(M + K)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    a, w = rand(M, B, K).bfloat16().transpose(0, 1), (rand(B, N, K) * K ** -0.5).bfloat16()
+    dt = torch.float32 if "fp32" in kind else torch.bfloat16
+    if kind.startswith("rows"):
+        gate = rand(M, B).to(dt).unsqueeze(-1).expand(-1, -1, N).transpose(0, 1)
+    else:
+        off = 1 if "off" in kind else 0
+        gate = rand(M * B * N + 1).to(dt)[off: off + M * B * N].view(M, B, N).transpose(0, 1)
+    out = torch.full((M, B, N), float("nan"), device="cuda", dtype=torch.bfloat16).transpose(0, 1)
+    seq.gemm(a, w, out, gate=gate)
+    _close(out, torch.matmul(a.float(), w.float().transpose(1, 2)) * torch.sigmoid(gate.float()), K)
+
+
 @pytest.mark.parametrize("sizes", [[1, 0, 2, 17], [0, 0, 90], [16, 32, 33, 64, 65], [2] * 64, [5] * 40, [500, 3], [1] * 70])
 @pytest.mark.parametrize("N,K", [(48, 72), (1024, 512)])
 def test_experts(N, K, sizes):
