@@ -381,9 +381,11 @@ __global__ __launch_bounds__(256) void gemm_any_rows_kernel(AnyGemmArgs p) {
 // 20.4 -> 20.0, warm 21.8 -> 16.6). Where K is short and workgroups are many, the registers of the second step are better spent on a fourth
 // workgroup per CU: 12 products of 512 x 128 at 2048 rows 14.2 -> 13.6, 16 19.0 -> 16.8 (two workgroups per CU: 10.2 -> 10.6).
 constexpr int LM = 128, LKS = 32, LPAD = LKS + 8;
-// GATED: whole pieces with a gate, whose work in every store would slow the forms without one (12 products of 512 x 128 at 2048 rows
-// 13.4 -> 17.9 us).
-template <int DUAL, int AHEAD, bool GATED>
+// OUT: how the outputs are stored, apart so that one way's work does not slow the others (gates in the plain form: 12 products of 512 x 128
+// at 2048 rows 13.4 -> 17.9 us). OUT_GATED: bf16 in whole pieces, times a gate. OUT_F32: fp32, 64 rows at a time through LDS, in whole lines
+// (1808 rows of 3072 x 96 19.5 -> 9.7 us, 1801 of 1024 x 128 16.7 -> 6.8 against a store per value).
+enum { OUT_PLAIN = 0, OUT_GATED = 1, OUT_F32 = 2 };
+template <int DUAL, int AHEAD, int OUT>
 __global__ __launch_bounds__(256, 3) void gemm_any_lds_kernel(AnyGemmArgs p) {
   constexpr int WN = DUAL ? 64 : 128;  // columns of each weight matrix per block
   constexpr int OPAD = WN + 8;         // padded row of the staged outputs
@@ -490,9 +492,38 @@ __global__ __launch_bounds__(256, 3) void gemm_any_lds_kernel(AnyGemmArgs p) {
       buf ^= 1;
     }
   }
-  if (GATED || p.vec_out) {  // bf16 rows of whole 16-B pieces: staged in LDS (the k loop's last barrier has freed it), then stored whole
+  if constexpr (OUT == OUT_F32) {   // (the k loop's last barrier has freed the buffers)
+    constexpr int FP = 128 + 4;
+    static_assert(!DUAL && 64 * FP * 4 <= (int)sizeof(smem), "64 rows fit the operand buffers");
+    float* fs = reinterpret_cast<float*>(smem);
+    float* out = reinterpret_cast<float*>(p.out) + b * p.o_bs;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      if (wm == half)
+        with_act<DUAL>(p, [&](auto act) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int col = wn * 64 + j * 16 + lr;
+            const float bias = p.bias ? p.bias[min(n0 + col, p.N - 1)] : 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) fs[(i * 16 + 4 * lg + e) * FP + col] = act_val<decltype(act)::value>(p, acc[i][j][e] + bias, 0.f);
+          }
+        });
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < 64 * 32 / 256; ++u) {
+        const int x = tid + 256 * u, row = x >> 5, col = (x & 31) * 4, m = r0 + 64 * half + row;
+        if (m < rend && n0 + col < p.N) *reinterpret_cast<f32x4*>(out + (int64_t)m * p.ldo + n0 + col) = *reinterpret_cast<const f32x4*>(&fs[row * FP + col]);
+      }
+      if (half == 0) __syncthreads();
+    }
+    return;
+  }
+  if (OUT == OUT_GATED || p.vec_out) {  // bf16 rows of whole 16-B pieces: staged in LDS (the k loop's last barrier has freed it), then stored whole
     // a gate: one logit per row, or its tile brought in whole pieces to where the outputs will lie, each lane's to its own
-    const bool tiled = GATED && p.g_cs != 0, rowed = GATED && p.g_cs == 0;
+    const bool tiled = OUT == OUT_GATED && p.g_cs != 0, rowed = OUT == OUT_GATED && p.g_cs == 0;
     float rg[4][4];
     if (rowed) {
 #pragma unroll
@@ -719,9 +750,12 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st) {
       v.vec_out = vec;
       const dim3 grid2((g.N + (dual ? 63 : 127)) / (dual ? 64 : 128), mt128, g.batch);
       const bool one = !dual && g.K <= 256 && (int64_t)grid2.x * grid2.y * grid2.z > 512;
-      const bool gated = v.vec_out && g.gate != nullptr;
-      auto kern = dual ? gemm_any_lds_kernel<1, 2, false>
-                       : (gated ? gemm_any_lds_kernel<0, 2, true> : (one ? gemm_any_lds_kernel<0, 1, false> : gemm_any_lds_kernel<0, 2, false>));
+      const bool gated = vec && g.gate != nullptr;
+      const bool f32 = g.out_f32 && !dual && g.gate == nullptr && g.N % 4 == 0 && g.ldo % 4 == 0 && g.o_bs % 4 == 0 && a16(g.out);
+      auto kern = dual ? gemm_any_lds_kernel<1, 2, OUT_PLAIN>
+                       : (gated ? gemm_any_lds_kernel<0, 2, OUT_GATED>
+                                : (f32 ? gemm_any_lds_kernel<0, 2, OUT_F32>
+                                       : (one ? gemm_any_lds_kernel<0, 1, OUT_PLAIN> : gemm_any_lds_kernel<0, 2, OUT_PLAIN>)));
       hipLaunchKernelGGL(kern, grid2, block, 0, st, v);
     } else if (dual && wide) hipLaunchKernelGGL((gemm_any_mfma_kernel<1, true, 4>), gridw, block, 0, st, g);
     else if (wide) hipLaunchKernelGGL((gemm_any_mfma_kernel<0, true, 4>), gridw, block, 0, st, g);

@@ -58,6 +58,21 @@ def test_long_batches_with_gates(M, B, N, K, kind):
     _close(out, torch.matmul(a.float(), w.float().transpose(1, 2)) * torch.sigmoid(gate.float()), K)
 
 
+@pytest.mark.parametrize("off", [0, 1, 4])
+@pytest.mark.parametrize("M,N,K", [(1024, 512, 64), (1153, 516, 96), (1090, 640, 8), (1025, 518, 136), (1024, 1020, 40)])
+def test_long_products_in_fp32(M, N, K, off):
+    """fp32 outputs of the 128-row tiles, stored in whole pieces where rows lie on 16 B and by the value where they don't: rows and columns
+    past the last whole tile, K below and past a step; what lies beside the outputs stays."""
+    g = torch.Generator("cuda").manual_seed(M + N)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    a, w, bias = rand(M, K).bfloat16(), (rand(N, K) * K ** -0.5).bfloat16(), rand(N)
+    whole = torch.full((M + 1, N + 8), 7.0, device="cuda")
+    out = whole[:M, off: off + N]
+    seq.gemm(a, w, out, bias=bias)
+    _close(out, a.float() @ w.float().t() + bias, K)
+    assert bool((whole[M] == 7).all() and (whole[:, :off] == 7).all() and (whole[:, off + N:] == 7).all())
+
+
 @pytest.mark.parametrize("sizes", [[1, 0, 2, 17], [0, 0, 90], [16, 32, 33, 64, 65], [2] * 64, [5] * 40, [500, 3], [1] * 70])
 @pytest.mark.parametrize("N,K", [(48, 72), (1024, 512)])
 def test_experts(N, K, sizes):
