@@ -675,6 +675,8 @@ __global__ __launch_bounds__(256) void linear_chunk_carry_kernel(LinearAttnArgs 
 }
 
 // grid (chunk, head), 512 threads: the outputs of a chunk from the state it starts from. Wave w owns the columns 16 w ..
+// Bound by chains through LDS with two waves per SIMD, the triangle's rows first: a row's operands are asked for a row ahead, and the decays'
+// products read their 16 tokens together (29 chunks of 8 heads of 128: 43.5 -> 37.0 us).
 template <int DP, bool F32, bool PRE>
 __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, int lim, const float* __restrict__ cstate,
                                                              float* __restrict__ oraw) {
@@ -740,18 +742,29 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
         if (PRE) diag = fmaf(lq[j * DS + d] * (d < D ? p.bonus[h * D + d] : 0.f), x[4 * m + c], diag);
       }
     if (PRE) diag = key_sum<8>(diag);
-    for (int i = 8 * jb; i < CT; ++i) {
-      float r = 0.f;
+    f32x4 na[X], nq[X];   // the next row's, asked for a row ahead (past the last: the last)
+    auto row = [&](int i) {
 #pragma unroll
       for (int m = 0; m < X; ++m) {
-        const f32x4 a = ld4(&la[i * DS + 32 * m + 4 * dg]), q = ld4(&lq[i * DS + 32 * m + 4 * dg]);
+        na[m] = ld4(&la[i * DS + 32 * m + 4 * dg]);
+        nq[m] = ld4(&lq[i * DS + 32 * m + 4 * dg]);
+      }
+    };
+    row(8 * jb);
+    for (int i = 8 * jb; i < CT; ++i) {
+      float r = 0.f;
+      f32x4 a[X], q[X];
+#pragma unroll
+      for (int m = 0; m < X; ++m) { a[m] = na[m]; q[m] = nq[m]; }
+      row(min(i + 1, CT - 1));
+#pragma unroll
+      for (int m = 0; m < X; ++m)
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          if (PRE) r = fmaf(q[c], x[4 * m + c], r);
-          if (i > j) x[4 * m + c] *= a[c];
-          if (!PRE) r = fmaf(q[c], x[4 * m + c], r);
+          if (PRE) r = fmaf(q[m][c], x[4 * m + c], r);
+          if (i > j) x[4 * m + c] *= a[m][c];
+          if (!PRE) r = fmaf(q[m][c], x[4 * m + c], r);
         }
-      }
       r = key_sum<8>(r);
       if (PRE && i == j) r = diag;
       if (dg == 0 && i >= j) tr[i * CTP + j] = r;
@@ -760,19 +773,31 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
   __syncthreads();
   {  // q_i g_(1..i) (with a bonus g_(1..i-1)) in place: a channel and 16 tokens per thread
     const int d = tid & 127, part = tid >> 7;
-    float g = 1.f;
-    if (d < DP)
-      for (int i = 16 * part; i < 16 * part + 16; ++i) {
-        if (!PRE) g *= la[i * DS + d];
-        lq[i * DS + d] *= g;
-        if (PRE) g *= la[i * DS + d];
+    float g = 1.f, a[16], q[16];   // (read together: a store between them would order the reads)
+    if (d < DP) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        a[i] = la[(16 * part + i) * DS + d];
+        q[i] = lq[(16 * part + i) * DS + d];
       }
-    if (d < DP) red[part * DP + d] = g;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if (!PRE) g *= a[i];
+        q[i] *= g;
+        if (PRE) g *= a[i];
+      }
+      red[part * DP + d] = g;
+    }
     __syncthreads();
-    if (d < DP && part > 0) {
-      float f = 1.f;
-      for (int m = 0; m < part; ++m) f *= red[m * DP + d];
-      for (int i = 16 * part; i < 16 * part + 16; ++i) lq[i * DS + d] *= f;
+    if (d < DP) {
+      if (part > 0) {
+        float f = 1.f;
+        for (int m = 0; m < part; ++m) f *= red[m * DP + d];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) q[i] *= f;
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) lq[(16 * part + i) * DS + d] = q[i];
     }
   }
   __syncthreads();
