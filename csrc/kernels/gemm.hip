@@ -156,6 +156,7 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
   // mixed prefill + decode steps (16 < M <= 64): the medium-M kernel when the start-up tuner
   // measured it faster (path 2, gemm_mid.hip); it declines shapes / modes it does not take
   if (g.path == 2 && launch_gemm_mid(g, st)) return;
+  if (g.path == 6) return launch_dispatch<false>(to_params(g), g, st);  // the kernels of gemm_decode.h (q4_prompt_form)
   // without a plan, 17 .. 64 rows: one block per CU owning whole tiles (wide) where K is short, K slices over narrow
   // tiles where it is long. us at 32 rows, the K-split / tile kernels below -> now: 17920 x 1536 19 -> 14.5, 6464 x 1536
   // 14.1 -> 9.0, 1536 x 8960 19.2 -> 13.1, 1024 x 4096 12.1 -> 8.4, 1536 x 1536 8.2 -> 6.6. Above 32 rows the wide form pays

@@ -874,13 +874,8 @@ static void launch_prefill_cfg(const GemmParams& p, int nz, hipStream_t st) {
 // (geometric mean) and 0.92 of hipBLASLt's; without 64 x 64 1.054, without 128 x 64 1.021, without 128 x 128 1.016, without any other one of
 // them 1.009 to 1.011. us before the four-wave forms (gemm_prompt.h) -> now: 1536 x 1536 at 256 rows 16.6 -> 12.5, 2048 x 1536 at 448
 // 17.1 -> 12.6, 17920 x 1536 at 448 46.8 -> 38.8, 4352 x 1024 at 2048 36.6 -> 30.3, 1024 x 4096 at 1024 32.2 -> 24.0.
-struct PrefillForm {
-  int code;  // tile code (as the forced ones below)
-  int nz;    // K slices
-  float us;  // its cost
-};
-
-static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool rows16, bool slabs, size_t slab_bytes, bool counters) {
+// cut > 0: that many K slices and none of the persistent forms
+static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool rows16, bool slabs, size_t slab_bytes, bool counters, int cut = 0) {
   struct Cost {
     float e, a, b, c, d, w, o;
   };
@@ -921,14 +916,20 @@ static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool rows
     if (N % t.bn != 0 || (t.code >= 5000 && !rows16)) continue;
     const Cost& x = t.cost[norm ? 1 : 0];
     const bool sliced = x.d > 0.f && !(t.bm == 256 && M >= 512);  // (the four-phase tiles of long steps are split by the persistent forms)
-    for (int nz : slices) {
+    auto consider = [&](int nz) {
       const int64_t blocks = (int64_t)over(M, t.bm) * (N / t.bn) * nz;
-      if (nz > 1 && (!sliced || blocks > 600 || nk / nz < 4 || !slabs || ((size_t)nz * M * N + (size_t)nz * M) * 4 > slab_bytes)) continue;
+      if (nz > 1 && (nk / nz < 4 || !slabs || ((size_t)nz * M * N + (size_t)nz * M) * 4 > slab_bytes)) return;
       take(t.code, nz, x.e + x.a * over(blocks, (int64_t)cus * t.per_cu) + x.b * over(blocks, cus) * over(nk, nz) + x.w * wmb + x.o * omb +
                            (nz > 1 ? x.c + x.d * 2.f * nz * omb : 0.f));
+    };
+    if (cut > 0) {
+      if (cut == 1 || x.d > 0.f) consider(cut);
+      continue;
     }
+    for (int nz : slices)
+      if (nz == 1 || (sliced && (int64_t)over(M, t.bm) * (N / t.bn) * nz <= 600)) consider(nz);
   }
-  if (M >= 512 && slabs && counters) {
+  if (M >= 512 && slabs && counters && cut == 0) {
     for (const Persistent& t : persistent) {
       const auto& x = t.cost[norm ? 1 : 0];
       const int n = N % t.bn == 0 ? over(M, 256) * (N / t.bn) : 0, rest = n % cus;
@@ -941,8 +942,97 @@ static PrefillForm choose_prefill_form(int M, int N, int K, bool norm, bool rows
   return best;
 }
 
-float prefill_cost_us(int M, int N, int K, bool norm, size_t slab_bytes) {
-  return N % 64 == 0 && K % 64 == 0 ? choose_prefill_form(M, N, K, norm, true, slab_bytes > 0, slab_bytes, slab_bytes > 0).us : 1e30f;
+// Products with int4 weights: how each sum over K is cut. An output is the sum of `nz` chains over equal stretches of 64-k tiles, whichever
+// tile computes it, on a bf16 copy (here) or on the int4 weights themselves (gemm_prompt_q4.hip), so the cut alone decides the last bits of
+// the result. It has costs of its own, which stay as they are when those above are fitted anew: with random int4 weights, whose values have
+// a mean, nearly all of a token's last hidden state lies along one direction, and on which side of zero it comes to lie there can rest on
+// the rounding of a sum (a cut chosen by the costs above: in 8 of 400 steps some token's cached keys and values had the opposite sign).
+// code 641 .. 1281: chains of a tile; 769 / 1025: of the persistent forms' slices, or (nz 0: more tiles than CUs) the persistent form
+// itself; 0: the tile kernels of gemm_decode.h, one chain; -1: the K-split kernels there. tiles_only: not those because the rows are few.
+PrefillForm q4_cut(int M, int N, int K, bool norm, bool rows16, bool tiles_only, size_t slab_bytes) {
+  struct Tile {
+    int code, bm, bn;
+    float a, b, c, d;  // rounds x (a + b x K-tiles) [+ c + d x MB of partials]
+  };
+  struct Costs {
+    Tile tiles[4];
+    float n64[2], n128[2];   // whole, per K-tile and block of a CU
+    float p256[4], p128[4];  // persistent: the last round whole, per K-tile, and of its K slices
+  };
+  static constexpr Costs sets[2] = {{{{1024, 256, 256, 10.2f, 1.33f, 1.5f, 0.49f},
+                                      {768, 256, 128, 7.1f, 1.00f, 1.6f, 0.56f},
+                                      {1281, 128, 128, 5.8f, 0.61f, 2.8f, 0.57f},
+                                      {641, 128, 64, 5.0f, 0.50f, 2.9f, 0.62f}},
+                                     {5.0f, 0.54f}, {6.0f, 0.77f}, {13.4f, 1.61f, 13.6f, 2.4f}, {10.6f, 1.07f, 5.6f, 1.5f}},
+                                    {{{1024, 256, 256, 16.2f, 1.52f, -3.1f, 0.485f},
+                                      {768, 256, 128, 11.7f, 1.13f, -0.8f, 0.506f},
+                                      {1281, 128, 128, 9.0f, 0.705f, 2.4f, 0.395f},
+                                      {641, 128, 64, 7.6f, 0.585f, 3.0f, 0.412f}},
+                                     {10.5f, 0.548f}, {12.0f, 0.78f}, {22.0f, 1.59f, 13.7f, 4.2f}, {15.3f, 1.175f, 6.3f, 2.4f}}};
+  const bool longer = M >= 128 || tiles_only || (rows16 && (K >= 2560 || (int64_t)N * K >= 8 * 1024 * 1024));
+  if (!longer || N % 64 != 0 || K % 64 != 0) return PrefillForm{-1, 0, 0.f};
+  const Costs& cs = sets[norm ? 1 : 0];
+  static constexpr int slices[] = {1, 2, 3, 4, 6, 8};
+  const int cus = cu_count() > 0 ? cu_count() : 256, nk = K / 64;
+  auto over = [](int64_t x, int y) { return (int)((x + y - 1) / y); };
+  PrefillForm best{641, 1, 1e30f};
+  auto take = [&](int code, int nz, float t) {
+    if (t < best.us) best = PrefillForm{code, nz, t};
+  };
+  if (K % 256 == 0 && N / 16 < 1024) {  // 64 x 64 tiles, weights in registers
+    const int rounds = over((int64_t)over(M, 64) * (N / 64), cus);
+    const bool tiles = M >= 128 || (int64_t)(N / 64) * over(M, 64) >= 128;
+    take(tiles ? 0 : -1, 1, norm && K >= 768 ? 5.2f + rounds * (3.58f + 0.591f * nk) : rounds * (4.6f + 0.354f * nk));
+  }
+  for (const Tile& t : cs.tiles) {
+    if (N % t.bn != 0) continue;
+    for (int nz : slices) {
+      const int64_t blocks = (int64_t)over(M, t.bm) * (N / t.bn) * nz;
+      const int rounds = over(blocks, cus);
+      if (nz > 1 && (rounds > 1 || nk / nz < 4 || ((size_t)nz * M * N + (size_t)nz * M) * 4 > slab_bytes)) continue;
+      const float mb = (float)nz * M * N * 4e-6f;
+      take(t.code, nz, rounds * (t.a + t.b * over(nk, nz)) + (nz > 1 ? t.c + t.d * mb : 0.f));
+    }
+  }
+  const int n64 = over((int64_t)over(M, 128) * (N / 64), cus), n128 = N % 128 == 0 ? over((int64_t)over(M, 128) * (N / 128), cus) : 0;
+  if (n64 > 1) take(641, 1, cs.n64[0] + cs.n64[1] * nk * n64);
+  if (n128 > 1) take(1281, 1, cs.n128[0] + cs.n128[1] * nk * n128);
+  if (M >= 512 && slab_bytes > 0) {
+    auto persistent = [&](int code, const Tile& t, const float (&x)[4]) {
+      if (N % t.bn != 0) return;
+      const int n = over(M, 256) * (N / t.bn), rest = n % cus;
+      if (rest == 0) return;
+      int S = cus / rest > 8 ? 8 : cus / rest;
+      while (S > 1 && nk / S < 4) --S;
+      take(code, n < cus ? S : 0, (n / cus) * (t.a + t.b * nk) + x[0] + x[1] * nk / S + (S > 1 ? x[2] + x[3] * (S - 1) : 0.f));
+    };
+    persistent(1025, cs.tiles[0], cs.p256);
+    persistent(769, cs.tiles[1], cs.p128);
+  }
+  return best;
+}
+
+// 128-column tiles of the two-deep ring (else 64): forced, or where they fill the chip
+static bool two_deep_wide(int M, int N, int code) {
+  if (code == 64 || N % 128 != 0) return false;
+  return code == 128 || (M + 127) / 128 * (N / 128) >= 240;
+}
+
+// K slices of a forced tile: `sk` of them, or (0) enough for about a block per CU in tiles of the two-deep ring; at least four K-tiles
+// each, and no more than the workspace holds
+int prefill_slices(int M, int N, int K, int code, int sk, size_t slab_bytes) {
+  int nz = sk > 0 ? sk : 1;
+  if (sk <= 0 && code < 5000) {
+    const int blocks = (M + 127) / 128 * (N / (two_deep_wide(M, N, code) ? 128 : 64));
+    if (blocks < 200) nz = min(8, (256 + blocks - 1) / blocks);
+  }
+  while (nz > 1 && K / 64 / nz < 4) --nz;
+  return nz > 1 && ((size_t)nz * M * N + (size_t)nz * M) * 4 > slab_bytes ? 1 : nz;
+}
+
+// The cheapest form with `cut` K slices (gemm_prompt_q4.hip compares it)
+PrefillForm prefill_form_cut(int M, int N, int K, bool norm, bool rows16, size_t slab_bytes, int cut) {
+  return choose_prefill_form(M, N, K, norm, rows16, slab_bytes > 0, slab_bytes, slab_bytes > 0, cut);
 }
 
 template <int EPI, int NORM>
@@ -962,25 +1052,10 @@ static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, 
     force_bn = f.code;
     force_sk = f.nz;
   }
-  const int mb = (p.M + 127) / 128;
-  bool wide = p.N % 128 == 0 && mb * (p.N / 128) >= 240;
-  if (force_bn == 128) wide = p.N % 128 == 0;
-  if (force_bn == 64) wide = false;
-  const int blocks = mb * (p.N / (wide ? 128 : 64));
-  int nz = 1;
-  if (force_sk > 0) {
-    nz = force_sk;
-  } else if (blocks < 200) {
-    nz = (256 + blocks - 1) / blocks;
-    nz = nz > 8 ? 8 : nz;
-  }
-  const int nk = p.K / 64;
-  while (nz > 1 && nk / nz < 4) --nz;
-  const size_t need = ((size_t)nz * p.M * p.N + (size_t)nz * p.M) * 4;
-  if (nz > 1 && (p.slabs == nullptr || need > slab_bytes)) nz = 1;
+  const bool wide = two_deep_wide(p.M, p.N, force_bn);
+  const int nz = prefill_slices(p.M, p.N, p.K, force_bn, force_sk, p.slabs != nullptr ? slab_bytes : 0);
   if (force_bn >= 5000) {
     if (!rows16) return false;
-    if (force_sk <= 0) nz = 1;
     if (!launch_gemm_w4<EPI, NORM>(p, force_bn, nz, st)) return false;
     if (nz > 1) launch_prefill_reduce<EPI, NORM, 1>(p, nz, st);
     return true;

@@ -1,5 +1,6 @@
 // Prompt GEMM on int4 weights (AWQ, groups of 128): the weights are unpacked between LDS and the matrix cores, so a step reads them at
-// 4 bits and no bf16 copy is written and read back. Every fragment holds the very bf16 values of that copy ((v s - s z) gamma, rounded once).
+// 4 bits and no bf16 copy is written and read back. Every fragment holds the very bf16 values of that copy ((v s - s z) gamma, rounded once),
+// and products and squares are summed in the order of the bf16 forms: the bits are theirs.
 //
 // As gemm_w4_kernel (gemm_prompt.h): four waves, one per SIMD, operands of a k-step read (here: and unpacked) during the MFMAs of the one
 // before, stages by LDS-DMA. The waves stand side by side over the columns, so that each fragment of W is unpacked by one wave of the block
@@ -29,8 +30,9 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
   const int lane = threadIdx.x & 63, quad = lane >> 4;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int KQ = p.K >> 7;
-  const int z = blockIdx.y, nz = gridDim.y;
-  const int q0 = (KQ * z) / nz, nk = (KQ * (z + 1)) / nz - q0;
+  // K slices in tiles of 64 k, as the bf16 forms cut them: a slice can begin or end inside a group, whose other half then counts as zeros
+  const int z = blockIdx.y, nz = gridDim.y, kt0 = (2 * KQ * z) / nz, kt1 = (2 * KQ * (z + 1)) / nz;
+  const int q0 = kt0 >> 1, nk = ((kt1 + 1) >> 1) - q0;
   const int mblocks = (p.M + G::BM - 1) / G::BM;
   const int nwg = gridDim.x, orig = blockIdx.x, xcd = orig & 7, q = nwg >> 3, r = nwg & 7;
   const int wgid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (orig >> 3);
@@ -68,9 +70,9 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
       acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
       asm volatile("" : "+a"(acc[a][b]));  // (written here, well before the first mfma_acc)
     }
-  float ss[MT];
+  float ss[(MT + 3) / 4];  // wave w sums the squares of the row tiles w, w + 4, ...: a row in the order of K, as the bf16 forms do
 #pragma unroll
-  for (int b = 0; b < MT; ++b) ss[b] = 0.f;
+  for (int i = 0; i < (MT + 3) / 4; ++i) ss[i] = 0.f;
   uint4 wf[2][NT], xf[2][MT], wq[NT];
   float sc[NT], zs[NT], gam[8];
   const int xlo[2] = {G::XB + x_frag_off(0, lane), G::XB + x_frag_off(1, lane)};
@@ -108,8 +110,16 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
   };
   constexpr int U = 2 * NT;  // halves of fragments of a k-step to unpack
   // the MFMAs of k-step u, a row tile at a time; between them the next k-step is read and unpacked and, at the last, the next stage asked for
-  auto phase = [&](auto uc, const char* sb, int st, int buf) {
+  auto phase = [&](auto uc, bool off, const char* sb, int st, int buf) {
     constexpr int u = decltype(uc)::value, v = (u + 1) & 3;
+    if (off) {  // (uniform) a k-step of the slice before or after
+#pragma unroll
+      for (int b = 0; b < MT; ++b) {
+        u32x4 none = {0, 0, 0, 0};
+        asm volatile("s_nop 1" : "+v"(none));
+        xf[u & 1][b] = __builtin_bit_cast(uint4, none);
+      }
+    }
     // (an MFMA reads what the VALU wrote two wait states before at the soonest, and the compiler does not see that mfma_acc() is one)
 #pragma unroll
     for (int a = 0; a < NT; ++a) {
@@ -120,10 +130,12 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
     if constexpr (u == 3) read_stage(sb);
     read_gamma(v, sb);
     if constexpr (NORM) {
-      if (wid == u) {
 #pragma unroll
-        for (int b = 0; b < MT; ++b) ss[b] = sumsq8(xf[u & 1][b], ss[b]);
-      }
+      for (int w = 0; w < 4; ++w)
+        if (wid == w) {
+#pragma unroll
+          for (int b = w; b < MT; b += 4) ss[b >> 2] = sumsq8(xf[u & 1][b], ss[b >> 2]);
+        }
     }
 #pragma unroll
     for (int b = 0; b < MT; ++b) {
@@ -158,12 +170,13 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
   for (int t = 0; t < nk; ++t) {
     const char* sb = smem + buf * STAGE;
     const int nb = buf + 1 == NS ? 0 : buf + 1;
-    phase(C0{}, sb, 0, 0);
-    phase(C1{}, sb, 0, 0);
-    phase(C2{}, sb, 0, 0);
+    const bool before = t == 0 && (kt0 & 1) != 0, after = t == nk - 1 && (kt1 & 1) != 0;
+    phase(C0{}, before, sb, 0, 0);
+    phase(C1{}, before, sb, 0, 0);
+    phase(C2{}, after, sb, 0, 0);
     // this stage is read (its last k-step is in registers), the next one has landed: both for every wave
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * PPW) : "memory");
-    phase(C3{}, smem + nb * STAGE, t + NS < nk ? t + NS : nk - 1, buf);  // past the end: clamped duplicates, never used
+    phase(C3{}, after, smem + nb * STAGE, t + NS < nk ? t + NS : nk - 1, buf);  // past the end: clamped duplicates, never used
     buf = nb;
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");  // the trailing duplicates
@@ -171,15 +184,15 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
   for (int a = 0; a < NT; ++a)
 #pragma unroll
     for (int b = 0; b < MT; ++b) asm volatile("" : "+a"(acc[a][b]));
-  float* rows = reinterpret_cast<float*>(smem);  // [wave][row] sums of squares
+  float* rows = reinterpret_cast<float*>(smem);  // sums of squares
   if constexpr (NORM) {
     __syncthreads();
 #pragma unroll
     for (int b = 0; b < MT; ++b) {
-      float s2 = ss[b];
+      float s2 = ss[b >> 2];
       s2 += xor16(s2);
       s2 += xor32(s2);
-      if (lane < 16) rows[wid * G::BM + b * 16 + lane] = s2;
+      if (wid == (b & 3) && lane < 16) rows[b * 16 + lane] = s2;
     }
     __syncthreads();
   }
@@ -189,8 +202,7 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
     scale[b] = 1.f;
     s2[b] = 0.f;
     if constexpr (NORM) {
-      const int rl = b * 16 + (lane & 15);
-      s2[b] = (rows[rl] + rows[G::BM + rl]) + (rows[2 * G::BM + rl] + rows[3 * G::BM + rl]);
+      s2[b] = rows[b * 16 + (lane & 15)];
       scale[b] = rsqrtf(s2[b] / (float)p.K + p.eps);
     }
   }
@@ -251,8 +263,9 @@ static bool launch_q4_epi(const GemmParams& p, int code, int nz, hipStream_t st)
 // Costs (us) as in choose_prefill_form() of gemm_prefill.hip, fitted to 15 shapes (N 512 .. 28672, K 1024 .. 14336) x 10 row counts 65 ..
 // 2048 on cold weights; K-tiles of 128. Unpacking is repeated by every row of blocks, so from some row count on a bf16 copy (2.2 us + 0.56
 // a million weights) and the bf16 kernels are ahead: 17920 x 1536 at 448 rows 60 against 64 us, at 1024 114 against 89; 1536 x 1536 at 1024 17
-// against 22. The choice between all forms and that takes 1.019 of the best one's time, and 1 / 1.26 of the copy's (geometric means).
-bool q4_prompt_form(int M, int N, int K, bool norm, size_t slab_bytes, int* code, int* slices) {
+// against 22. Free in its slices the choice took 1.019 of the best form's time, and 1 / 1.26 of the copy's (geometric means); with the cut of K
+// given, a step of 256 rows through six layers of 1536 / 8960 takes 751 us instead of 730 (945 with copies).
+Q4Form q4_prompt_form(int M, int N, int K, bool norm, bool rows16, bool group128, size_t slab_bytes, int code, int sk) {
   struct Tile {
     int code, bm, bn, per_cu;
     struct {
@@ -267,8 +280,13 @@ bool q4_prompt_form(int M, int N, int K, bool norm, size_t slab_bytes, int* code
       {1020, 160, 128, 1, {{8.98f, 4.86f, 1.31f, 0.152f, 0.336f, 0.f, 0.151f}, {9.24f, 6.01f, 1.59f, 0.f, 0.29f, 0.f, 0.154f}}},
       {1620, 256, 128, 1, {{10.5f, 4.19f, 1.84f, 0.f, 0.347f, 0.f, 0.339f}, {10.9f, 5.22f, 2.17f, 0.f, 0.325f, 0.f, 0.426f}}},
       {640, 96, 256, 1, {{8.39f, 5.55f, 1.74f, 0.353f, 0.343f, 0.f, 0.082f}, {8.99f, 6.65f, 2.09f, 0.f, 0.287f, 0.f, 0.079f}}}};
-  static constexpr int cuts[] = {1, 2, 3, 4, 6, 8};
-  if (M <= 64 || N % 64 != 0 || K % 128 != 0) return false;
+  // columns of the form's tiles; a width that N is no multiple of: launch_gemm() goes on to the kernels of gemm_decode.h
+  const int width = code >= 5000 ? code / 10 % 10 * 32 : code == 1024 || code == 1025 || code == 512 ? 256 : code == 2560 ? 512 :
+                    code == 2561 ? 320 : code == 256 || code == 768 || code == 769 || code == 1280 || code == 1281 ? 128 : 64;
+  if (code < 0 || N % 64 != 0 || K % 64 != 0 || N % width != 0) return Q4Form{6, max(code, 0), sk};
+  if (code == 0 && norm) return Q4Form{6, 0, 0};   // (the tile kernels there sum the squares of a row in an order of their own)
+  const int nz = code == 0 ? 1 : prefill_slices(M, N, K, code, sk, slab_bytes);
+  if ((code == 1025 || code == 769) && (sk == 0 || nz != sk)) return Q4Form{1, code, sk};   // (whole rounds, or partials only it has room for)
   static const int cus = [] {
     int v = 0, dev = 0;
     (void)hipGetDevice(&dev);
@@ -276,25 +294,23 @@ bool q4_prompt_form(int M, int N, int K, bool norm, size_t slab_bytes, int* code
     return v > 0 ? v : 256;
   }();
   const float weights = 1e-6f * (float)N * (float)K, omb = 2e-6f * (float)M * (float)N;
-  float least = 2.2f + 0.56f * weights + prefill_cost_us(M, N, K, norm, slab_bytes);
+  const PrefillForm copy = prefill_form_cut(M, N, K, norm, rows16, slab_bytes, nz);
+  Q4Form best = copy.us < 1e30f ? Q4Form{1, copy.code, nz} : Q4Form{code == 0 ? 6 : 1, code, sk};
+  if (!group128 || !rows16 || K % 128 != 0) return best;
+  float least = 2.2f + 0.56f * weights + copy.us;
   auto over = [](int64_t x, int64_t y) { return (int)((x + y - 1) / y); };
-  *code = 0;
   for (const Tile& t : tiles) {
+    const int64_t blocks = (int64_t)over(M, t.bm) * (N / t.bn) * nz;
     if (N % t.bn != 0) continue;
     const auto& x = t.cost[norm ? 1 : 0];
-    for (int nz : cuts) {
-      const int64_t blocks = (int64_t)over(M, t.bm) * (N / t.bn) * nz;
-      if (nz > 1 && (blocks > 600 || K / 128 / nz < 2 || ((size_t)nz * M * N + (size_t)nz * M) * 4 > slab_bytes)) continue;
-      const float us = x.e + x.a * over(blocks, (int64_t)cus * t.per_cu) + x.b * over(blocks, cus) * over(K / 128, nz) + x.w * 2.f * weights +
-                       x.o * omb + (nz > 1 ? x.c + x.d * 2.f * nz * omb : 0.f);
-      if (us < least) {
-        least = us;
-        *code = t.code;
-        *slices = nz;
-      }
+    const float us = x.e + x.a * over(blocks, (int64_t)cus * t.per_cu) + x.b * over(blocks, cus) * over(K / 128, nz) + x.w * 2.f * weights +
+                     x.o * omb + (nz > 1 ? x.c + x.d * 2.f * nz * omb : 0.f);
+    if (us < least) {
+      least = us;
+      best = Q4Form{5, t.code, nz};
     }
   }
-  return *code != 0;
+  return best;
 }
 
 bool launch_q4_prompt(const GemmArgs& g, hipStream_t st) {
@@ -316,7 +332,7 @@ bool launch_q4_prompt(const GemmArgs& g, hipStream_t st) {
   p.scales = g.scales; p.zeros = g.zeros; p.group = g.group;
   p.dbg_ts = g.dbg_ts;
   int nz = g.splitk > 0 ? g.splitk : 1;
-  while (nz > 1 && p.K / 128 / nz < 2) --nz;
+  while (nz > 1 && p.K / 64 / nz < 4) --nz;
   if (nz > 1 && (p.slabs == nullptr || ((size_t)nz * p.M * p.N + (size_t)nz * p.M) * 4 > g.slab_bytes)) nz = 1;
 #define VG_Q4E(E) return g.norm_w != nullptr ? launch_q4_epi<E, true>(p, g.ntb, nz, st) : launch_q4_epi<E, false>(p, g.ntb, nz, st)
   switch (g.epi) {

@@ -98,10 +98,22 @@ bool launch_dense_kx(const GemmArgs& g, hipStream_t st);
 // per CU owning whole tiles), g.splitk K slices; false for a shape / mode it does not take
 bool launch_awq_mid(const GemmArgs& g, hipStream_t st);
 // AWQ W4A16 prompt kernel (gemm_prompt_q4.hip, M > 64): g.ntb = a tile code, g.splitk = K slices, as q4_prompt_form() gives them; false
-// for a shape / mode it does not take. q4_prompt_form(): false where a bf16 copy of the matrix and the bf16 kernels are faster.
+// for a shape / mode it does not take.
 bool launch_q4_prompt(const GemmArgs& g, hipStream_t st);
-bool q4_prompt_form(int M, int N, int K, bool norm, size_t slab_bytes, int* code, int* slices);
-float prefill_cost_us(int M, int N, int K, bool norm, size_t slab_bytes);  // the bf16 kernels' cost of a product (gemm_prefill.hip)
+// How a step of more than 64 rows multiplies by int4 weights: path 5 that kernel; 1 a bf16 copy and a form of gemm_prefill.hip; 6 a bf16
+// copy and the kernels of gemm_decode.h. K is cut as form (code, sk), of q4_cut() or of a plan, cuts it: all of them give that form's bits.
+struct Q4Form {
+  int path, code, slices;
+};
+Q4Form q4_prompt_form(int M, int N, int K, bool norm, bool rows16, bool group128, size_t slab_bytes, int code, int sk);
+struct PrefillForm {
+  int code;  // tile code (gemm_prefill.hip launch_prefill_epi)
+  int nz;    // K slices
+  float us;  // its cost
+};
+PrefillForm q4_cut(int M, int N, int K, bool norm, bool rows16, bool tiles_only, size_t slab_bytes);   // (gemm_prefill.hip)
+PrefillForm prefill_form_cut(int M, int N, int K, bool norm, bool rows16, size_t slab_bytes, int cut);
+int prefill_slices(int M, int N, int K, int code, int sk, size_t slab_bytes);
 // AWQ int4 fragments -> bf16 fragment-packed copy (optionally gamma-folded) for the prefill kernel
 void launch_awq_dequant(const void* wq, const uint16_t* scales, const uint16_t* sz, const uint16_t* gamma,
                         void* out, int N, int K, int group, hipStream_t st);

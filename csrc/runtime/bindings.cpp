@@ -51,6 +51,9 @@ vgate::AttnArgs attn_common(const Tensor& q, int64_t q_stride, const Tensor& k_c
 // out = epilogue(prologue(x) @ W^T); W fragment-packed [N/16, K/32, 64, 8] bf16, or AWQ
 // int4 [N/16, K/128, 64, 4] int32 with scales/zeros. ws = int32 workspace: [0, 65536)
 // split-K tickets (zeroed once, self-resetting), the rest fp32 slabs.
+// bytes of the fp32 slabs behind the counters of a workspace
+size_t slab_bytes_of(const Tensor& ws) { return ws.numel() > 65536 ? (size_t)(ws.numel() - 65536) * 4 : 0; }
+
 void gemm(const Tensor& x, const Tensor& wp, int64_t N, int64_t K, Tensor& out, int64_t epi,
           const c10::optional<Tensor>& bias, const c10::optional<Tensor>& res,
           const c10::optional<Tensor>& norm_w, double eps, const c10::optional<Tensor>& row_idx,
@@ -657,13 +660,18 @@ PYBIND11_MODULE(_C, m) {
   m.def("awq_dequant", &awq_dequant, "AWQ int4 packed -> bf16 fragment-packed (prefill operand; optional gamma fold)",
         py::arg("wq"), py::arg("scales"), py::arg("sz"), py::arg("N"), py::arg("K"), py::arg("group"), py::arg("out"),
         py::arg("gamma") = py::none());
-  m.def("q4_prompt_form", [](int64_t M, int64_t N, int64_t K, bool norm, const Tensor& ws) {
-    int code = 0, slices = 1;
-    const size_t slab_bytes = ws.numel() > 65536 ? (size_t)(ws.numel() - 65536) * 4 : 0;
-    if (!vgate::q4_prompt_form((int)M, (int)N, (int)K, norm, slab_bytes, &code, &slices)) code = 0;
-    return std::make_pair(code, slices);
-  }, "(tile code, K slices) of the int4 prompt GEMM (gemm path 5), or (0, 1): dequantise and take the bf16 kernels",
-        py::arg("M"), py::arg("N"), py::arg("K"), py::arg("norm"), py::arg("ws"));
+  m.def("q4_prompt_form", [](int64_t M, int64_t N, int64_t K, bool norm, bool rows16, bool group128, const Tensor& ws, int64_t code, int64_t sk) {
+    const vgate::Q4Form f = vgate::q4_prompt_form((int)M, (int)N, (int)K, norm, rows16, group128, slab_bytes_of(ws), (int)code, (int)sk);
+    return std::make_tuple(f.path, f.code, f.slices);
+  }, "(path, tile code, K slices) of a step of more than 64 rows on int4 weights whose sums are cut as form (code, sk) cuts them: path 5 the "
+     "int4 prompt GEMM, 1 a bf16 copy and the prefill kernels, 6 a bf16 copy and the decode / tile kernels",
+        py::arg("M"), py::arg("N"), py::arg("K"), py::arg("norm"), py::arg("rows16"), py::arg("group128"), py::arg("ws"), py::arg("code"),
+        py::arg("sk"));
+  m.def("q4_cut", [](int64_t M, int64_t N, int64_t K, bool norm, bool rows16, bool tiles_only, const Tensor& ws) {
+    const vgate::PrefillForm f = vgate::q4_cut((int)M, (int)N, (int)K, norm, rows16, tiles_only, slab_bytes_of(ws));
+    return std::make_pair(f.code, f.nz);
+  }, "(tile code, K slices) that cuts the sums of a step of more than 64 rows on int4 weights", py::arg("M"), py::arg("N"), py::arg("K"),
+        py::arg("norm"), py::arg("rows16"), py::arg("tiles_only"), py::arg("ws"));
   m.def("silu_mul", &silu_mul, "out = silu(y[:, :I]) * y[:, I:] (library gate_up epilogue)");
   m.def("attn_decode", &attn_decode, "paged split-K decode attention");
   m.def("attn_prefill", &attn_prefill, "paged varlen causal prefill attention",

@@ -1268,6 +1268,61 @@ def test_awq_prompt_tiles(code, M, K, sk, norm):
     assert ((out.double() - want).norm() / want.norm()).item() < (K + 8) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("M,K,sk", [(65, 256, 1), (97, 640, 2), (130, 1152, 4), (300, 1536, 3), (577, 1664, 6)])
+def test_awq_prompt_tiles_give_the_bits_of_the_copied_matrix(M, K, sk, norm):
+    """Every int4 tile against every bf16 form on the dequantised copy, K in as many slices, some of which begin or end inside a group of
+    128: the same chains of the same products, so the same bits."""
+    C, N = ops.native(), 512
+    lin = _awq(N, K, "plain", M + K)
+    x = torch.randn(M, K, device=DEV, generator=torch.Generator(DEV).manual_seed(K)).bfloat16()
+    gamma = (torch.rand(K, device=DEV, generator=torch.Generator(DEV).manual_seed(M)) + 0.5).bfloat16() if norm else None
+    copy = torch.empty(N * K, dtype=torch.bfloat16, device=DEV)
+    C.awq_dequant(lin.wp, lin.scales, lin.zeros, N, K, 128, copy, gamma)
+    want = None
+    for code in (641, 1281, 768, 1024, 5220, 5340, 5380, 5580, 5640, 5680):
+        out = torch.full((M, N), float("nan"), device=DEV)
+        C.gemm(x, copy, N, K, out, 1, ws=ops.workspace(DEV), path=1, ntb=code, splitk=sk, rownorm=norm, eps=1e-6)
+        want = out if want is None else want
+        assert torch.equal(out, want), code
+    for code in (410, 610, 620, 820, 1020, 1620, 640):
+        out = torch.full((M, N), float("nan"), device=DEV)
+        C.gemm(x, lin.wp, N, K, out, 1, ws=ops.workspace(DEV), ntb=code, splitk=sk, path=5, awq_scales=lin.scales, awq_zeros=lin.zeros,
+               group=128, norm_w=gamma, eps=1e-6)
+        assert torch.equal(out, want), code
+
+
+@pytest.mark.parametrize("M", [65, 128, 200, 256, 448, 1024])
+def test_awq_steps_give_the_bits_of_their_cut(M):
+    """A step's int4 products through linear(), every epilogue, against the form that cuts K, on the dequantised copy."""
+    torch.manual_seed(M)
+    K, F, hq, hkv, ws = 1536, 8960, 12, 2, ops.workspace(DEV)
+    gamma = (torch.rand(K, device=DEV) + 0.5).bfloat16()
+    x, a, res = torch.randn(M, K, device=DEV).bfloat16(), torch.randn(M, F, device=DEV).bfloat16(), torch.randn(M, K, device=DEV).bfloat16()
+    shape = (M // 16 + 2, hkv, 16, 128)
+    bias = torch.randn(2048, device=DEV).bfloat16()
+    for lin, rows, norm in ((_awq(2048, K, "qkv", 1, bias=bias), x, True), (_awq(K, K, "plain", 2), x, False),
+                            (_awq(2 * F, K, "silu", 3), x, True), (_awq(K, F, "plain", 4), a, False)):
+        code, sk = ops._awq_cut(None, M, lin.N, lin.K, norm, True, ws)
+        pairs = []
+        for copy in (False, True):
+            kw = dict(norm=(gamma, 1e-6)) if norm else dict(residual=res.clone())
+            if lin.layout == "qkv":
+                kw["qkv"] = dict(positions=torch.arange(M, dtype=torch.int32, device=DEV), slots=torch.arange(M, device=DEV).flip(0).int(),
+                                 cos_sin=ref.rope_cos_sin(4096, 128, 1e6, device=DEV), k_cache=torch.zeros(shape, device=DEV).bfloat16(),
+                                 v_cache=torch.zeros(shape, device=DEV).bfloat16(), hq=hq, hkv=hkv)
+            if copy:
+                out = torch.empty(M, {"qkv": K, "silu": F, "plain": K}[lin.layout], dtype=torch.bfloat16, device=DEV)
+                form = dict(path=1, ntb=code, splitk=sk) if code > 0 else dict(path=6)
+                ops._linear_awq_dequant(rows, lin, out, kw.get("residual"), kw.get("norm"), kw.get("qkv"),
+                                        {"qkv": 3, "silu": 2, "plain": 0}[lin.layout], M, form)
+            else:
+                out = ops.linear(rows, lin, **kw)
+            pairs.append([out] + ([kw["qkv"]["k_cache"], kw["qkv"]["v_cache"]] if "qkv" in kw else []))
+        for got, want in zip(*pairs):
+            assert torch.equal(got, want), (lin.N, lin.K, code, sk)
+
+
 @pytest.mark.parametrize("M", [65, 130, 256])
 def test_awq_prompt_epilogues_match_the_copied_matrix(M):
     """Residual, SiLU * mul, QKV + RoPE + cache write of the int4 prompt kernel against the bf16 kernels on the dequantised matrix."""

@@ -73,3 +73,35 @@ def test_row_major_projections_are_not_padded_past_whole_tiles_of_64(rows, f32):
     proj, col = hybrid._fuse_inputs(SimpleNamespace(in_rows=[("a", w)]), [], 64, "cpu", f32)
     assert proj.N == -(-rows // 64) * 64 and col == {"a": (0, rows)}
     assert torch.equal(proj.w[:rows], w) and not proj.w[rows:].any()
+
+
+@pytest.mark.parametrize("N,K,norm,slices", [
+    (2048, 1536, True, {128: 6, 192: 4, 256: 4, 320: 4, 384: 2, 448: 2, 640: 1, 1024: 1, 2048: 1}),
+    (1536, 1536, False, {128: 6, 192: 1, 256: 1, 512: 1, 768: 1, 2048: 1}),
+    (17920, 1536, True, {96: 1, 128: 1, 256: 1, 448: 1, 1024: 1, 2048: 1}),
+    (1536, 8960, False, {65: 8, 96: 8, 256: 8, 320: 6, 384: 6, 448: 4, 640: 4, 768: 3, 1024: 4, 1536: 3, 2048: 4})])
+def test_int4_steps_keep_their_cut_of_k(N, K, norm, slices):
+    """The stretches into which K is cut decide the last bits of a product, and in a model with random int4 weights those can decide a
+    token: the cut of every size stays as it is, whichever kernels are added or fitted anew."""
+    C, ws = ops.native(), torch.empty(65536 + (64 << 20), dtype=torch.int32)
+    lin = SimpleNamespace(N=N, K=K, layout="qkv" if norm else "plain")
+    plan = ops._awq_plan(lin, sorted(slices), ws)
+    for M, nz in slices.items():
+        code, sk = ops._awq_cut(plan[M], M, N, K, norm, True, ws)
+        for group128 in (False, True):
+            path, code2, sk2 = C.q4_prompt_form(M, N, K, norm, True, group128, ws, code, sk)
+            # (path 6: the tile kernels of short K, a single chain; K-tiles of 64 cut into sk2 slices otherwise)
+            assert (path == 6 and sk2 == 0 and nz == 1) or (path in (1, 5) and sk2 == nz), (M, path, code2, sk2)
+
+
+def test_int4_forms_that_only_one_kernel_sums_alike():
+    """Persistent forms of more tiles than CUs, tile kernels that sum the squares of a norm their own way, few rows of short K."""
+    C, ws = ops.native(), torch.empty(65536 + (64 << 20), dtype=torch.int32)
+    form = lambda *a, code, sk: C.q4_prompt_form(*a, True, ws, code, sk)  # noqa: E731
+    assert C.q4_cut(2048, 28672, 4096, False, True, False, ws) == (1025, 0)
+    assert form(2048, 28672, 4096, False, True, code=1025, sk=0) == (1, 1025, 0)
+    assert form(300, 1536, 1536, True, True, code=0, sk=1)[0] == 6 and form(300, 1536, 1536, False, True, code=0, sk=1)[2] <= 1
+    assert C.q4_cut(96, 1536, 1536, False, True, False, ws)[0] == -1 and form(96, 1536, 1536, False, True, code=-1, sk=0) == (6, 0, 0)
+    assert C.q4_prompt_form(300, 1536, 1536, False, False, True, ws, 641, 2)[0] == 1   # (rows off 16 B)
+    small = torch.empty(65536 + 4096, dtype=torch.int32)                                # no room for partials: one chain
+    assert C.q4_prompt_form(300, 1536, 8960, False, True, True, small, *C.q4_cut(300, 1536, 8960, False, True, False, small))[2] == 1

@@ -340,8 +340,8 @@ def linear(x: torch.Tensor, lin: Linear, out: torch.Tensor | None = None,
     if awq_mid:
         path = 2  # int4 medium kernel (csrc/kernels/gemm_awq_mid.hip awq_mid_kernel): no bf16 scratch
     elif lin.kind == "awq" and M >= AWQ_DEQUANT_MIN_M and row_idx is None and waves == 0 and splitk == 0:
-        if path == 0 and M > 64 and _linear_awq_prompt(x, lin, out, residual, norm, qkv, epi, M):
-            return out
+        if path == 0 and M > 64:
+            return _linear_awq_prompt(x, lin, out, residual, norm, qkv, epi, M)
         return _linear_awq_dequant(x, lin, out, residual, norm, qkv, epi, M)
     ntb = 0
     sk = False
@@ -433,7 +433,8 @@ def _attn_after(q, qkv, attn):
 
 
 # AWQ steps of 16 < M <= 64 rows (mixed prefill + decode) run the int4 medium kernel, longer ones the int4 prompt
-# kernel; what neither takes (M >= AWQ_DEQUANT_MIN_M) dequantises to scratch + the bf16 prefill / tile kernels
+# kernel or a dequantised copy + the bf16 prefill / tile kernels, which give the same bits; what the medium kernel
+# does not take (M >= AWQ_DEQUANT_MIN_M) the dequantised copy
 AWQ_DEQUANT_MIN_M = 32
 _AWQ_SCRATCH: dict = {}
 
@@ -447,18 +448,21 @@ def reserve_awq_scratch(device, numel: int) -> torch.Tensor:
     return t
 
 
-def _linear_awq_prompt(x, lin: "Linear", out, residual, norm, qkv, epi, M) -> bool:
-    """Long AWQ step on the int4 prompt kernel (csrc/kernels/gemm_prompt_q4.hip), which unpacks the weights on their way to the
-    matrix cores. False: a group size, an alignment or a size that stays with :func:`_linear_awq_dequant`."""
-    gamma = norm[0] if norm is not None else None
-    if lin.group != 128 or x.stride(0) % 8 or x.stride(0) >= 1 << 20 or x.data_ptr() % 16 or (gamma is not None and gamma.data_ptr() % 16):
-        return False
+def _linear_awq_prompt(x, lin: "Linear", out, residual, norm, qkv, epi, M):
+    """Long AWQ step: on the int4 prompt kernel (csrc/kernels/gemm_prompt_q4.hip), which unpacks the weights on their way to the
+    matrix cores, or on a dequantised copy, whichever its size makes the faster. K is cut alike on both, as the plan or
+    :func:`_awq_cut` says: the bits of the result do not depend on the choice."""
     C = native()
+    gamma = norm[0] if norm is not None else None
     ws = workspace(x.device)
-    code, slices = C.q4_prompt_form(M, lin.N, lin.K, gamma is not None, ws)
-    if code == 0:
-        return False
-    kw = dict(bias=lin.bias, res=residual, ws=ws, ntb=code, splitk=slices, path=5, awq_scales=lin.scales, awq_zeros=lin.zeros,
+    rows16 = x.stride(0) % 8 == 0 and x.stride(0) < 1 << 20 and x.data_ptr() % 16 == 0 and lin.K < 1 << 20
+    aligned = not any(t is not None and t.data_ptr() % 16 for t in (gamma, lin.scales, lin.zeros))
+    plan = lin.prefill_plan.get(_plan_bucket(lin.prefill_plan, M)) if lin.prefill_plan else None
+    code, sk = _awq_cut(plan, M, lin.N, lin.K, gamma is not None, rows16, ws)
+    path, code, sk = C.q4_prompt_form(M, lin.N, lin.K, gamma is not None, rows16, lin.group == 128 and aligned, ws, code, sk)
+    if path != 5:
+        return _linear_awq_dequant(x, lin, out, residual, norm, qkv, epi, M, dict(path=path, ntb=code, splitk=sk))
+    kw = dict(bias=lin.bias, res=residual, ws=ws, ntb=code, splitk=sk, path=5, awq_scales=lin.scales, awq_zeros=lin.zeros,
               group=lin.group)
     if gamma is not None:
         kw.update(norm_w=gamma, eps=float(norm[1]))
@@ -466,12 +470,20 @@ def _linear_awq_prompt(x, lin: "Linear", out, residual, norm, qkv, epi, M) -> bo
         kw.update(positions=qkv["positions"], slots=qkv["slots"], cos_sin=qkv["cos_sin"], k_cache=qkv["k_cache"],
                   v_cache=qkv["v_cache"], hq=qkv["hq"], hkv=qkv["hkv"])
     C.gemm(x, lin.wp, lin.N, lin.K, out, epi, **kw)
-    return True
+    return out
 
 
-def _linear_awq_dequant(x, lin: "Linear", out, residual, norm, qkv, epi, M):
+def _awq_cut(plan, M, N, K, norm: bool, rows16: bool, ws) -> tuple[int, int]:
+    """(tile code, K slices) of the bf16 form that cuts the sums of a long AWQ step: the plan's, else the launcher's rule."""
+    if plan is not None and plan != MEDIUM_DEFAULT and plan != (0, 0):
+        return plan
+    return native().q4_cut(M, N, K, norm, rows16, plan == (0, 0), ws)
+
+
+def _linear_awq_dequant(x, lin: "Linear", out, residual, norm, qkv, epi, M, form: dict | None = None):
     """Long AWQ step: int4 -> bf16 fragment-packed scratch (RMSNorm gamma folded in), then the
-    bf16 kernels with the row-scale-only RMSNorm mode — same epilogues, no resident bf16 copy."""
+    bf16 kernels with the row-scale-only RMSNorm mode — same epilogues, no resident bf16 copy.
+    form: C.gemm's path, ntb and splitk (default: the plan's)."""
     C = native()
     scratch = reserve_awq_scratch(x.device, lin.N * lin.K)[: lin.N * lin.K]
     gamma = norm[0] if norm is not None else None
@@ -482,7 +494,9 @@ def _linear_awq_dequant(x, lin: "Linear", out, residual, norm, qkv, epi, M):
     if qkv is not None:
         kw.update(positions=qkv["positions"], slots=qkv["slots"], cos_sin=qkv["cos_sin"],
                   k_cache=qkv["k_cache"], v_cache=qkv["v_cache"], hq=qkv["hq"], hkv=qkv["hkv"])
-    if M > 16 and lin.prefill_plan:
+    if form is not None:
+        kw.update(form)
+    elif M > 16 and lin.prefill_plan:
         kw.update(_plan_kw(lin.prefill_plan.get(_plan_bucket(lin.prefill_plan, M)), M))
     C.gemm(x, scratch, lin.N, lin.K, out, epi, **kw)
     return out
@@ -743,9 +757,20 @@ MEDIUM_DEFAULT = (-1, -1)  # medium-M plan entry: keep the default (decode / til
 
 # bump whenever the MEANING of a stored plan changes on the Python side (the _plan_kw encoding of a
 # (tile, K slices) code, MID_BASE, the tuner margin): a cached plan set is keyed on this too
-PLAN_FORMAT = 4  # 4: the four-wave tiles
+PLAN_FORMAT = 5  # 4: the four-wave tiles; 5: a plan of an int4 layer is the cut of K
 TUNE_MARGIN = 0.05
 LONG_M, LONG_MARGIN = 1024, 0.02  # the margin for M >= LONG_M buckets
+
+
+def _awq_plan(lin: "Linear", ms: list[int], ws) -> dict:
+    """Plan of an int4 layer (group 128), whose entries say how a step's sums are cut and not which kernel computes them: the
+    launcher's rule, but four slices where it has more of the persistent form (1536 x 8960 at 1024 and 2048 rows: five).
+    Nothing is timed, so a step's bits do not depend on what start-up measured."""
+    plan = {}
+    for M in ms:
+        code, nz = native().q4_cut(M, lin.N, lin.K, lin.layout in ("qkv", "silu"), True, False, ws) if M > 64 else (-1, 0)
+        plan[M] = (code - 1, 4) if code in (1025, 769) and nz > 4 else MEDIUM_DEFAULT if M < 128 else (0, 0)
+    return plan
 
 
 def tune_prefill(lins: list, ms: list[int], iters: int = 5, margin: float = TUNE_MARGIN) -> dict:
@@ -757,7 +782,8 @@ def tune_prefill(lins: list, ms: list[int], iters: int = 5, margin: float = TUNE
     40 us, profiles/r2_prefill_tile_sweep.log). Every candidate is timed on random operands of
     the layer's shape (plain epilogue, all candidates are exact kernels of the same product);
     the heuristic is kept unless a candidate beats it by more than ``margin``. The plan is
-    shared by every Linear of the same shape (AWQ layers: the plan of their bf16 dequant scratch).
+    shared by every Linear of the same shape. AWQ layers of group 128 are not timed: their plan is a cut of K
+    (:func:`_awq_plan`), of other groups it is that of their bf16 dequant scratch.
 
     Medium buckets (16 < M < 128: the mixed steps of a serving load, one prompt chunk beside the
     decode rows) are timed against the DEFAULT path at that M too (the K-split decode kernels /
@@ -778,10 +804,13 @@ def tune_prefill(lins: list, ms: list[int], iters: int = 5, margin: float = TUNE
         if key in plans:
             lin.prefill_plan = plans[key]
             continue
+        if lin.kind == "awq" and lin.group == 128:
+            plans[key] = lin.prefill_plan = _awq_plan(lin, ms, ws)
+            continue
         plan = {}
         g = torch.Generator(device=dev)
         g.manual_seed(lin.N + lin.K)
-        # AWQ layers run their long steps on a bf16 fragment-packed dequant scratch of the same
+        # AWQ layers of other groups: steps on a bf16 fragment-packed dequant scratch of the same
         # shape (_linear_awq_dequant): time a random bf16 matrix in that layout
         wp = lin.wp if lin.kind == "dense" else pack_weight(
             (torch.rand(lin.N, lin.K, device=dev, generator=g) * 2 - 1).bfloat16())
