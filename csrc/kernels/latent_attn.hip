@@ -844,7 +844,8 @@ __global__ __launch_bounds__(256, 1) void latent_attn_staged_kernel(LatentArgs a
     for (int r = 0; r < KW; ++r) {
       const float mo = pm[(r * 2 + rw) * 128 + l], lo = pm[(r * 2 + rw) * 128 + 64 + l];
       const float M = fmaxf(m[r], mo);
-      const float f0 = exp2f(m[r] - M), f1 = exp2f(mo - M);   // a half that saw no key: max -inf, factor 0
+      // a half that saw no key: max -inf, factor 0; a sink of +inf, in the even half's maximum: factor 1, the row's weights are zero
+      const float f0 = m[r] == M ? 1.f : exp2f(m[r] - M), f1 = mo == M ? 1.f : exp2f(mo - M);
       lsum[r] = lsum[r] * f0 + lo * f1;
 #pragma unroll
       for (int c = 0; c < NCT; ++c) O[r][c] = O[r][c] * f0 + po[(r * NCT + c) * 128] * f1;

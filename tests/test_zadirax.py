@@ -459,6 +459,32 @@ def test_latent_attention_of_prompts_at_tile_edges(rank, H, window):
         assert bool((err <= 2 * 2.0 ** -8 * size + 1e-4).all()), (s, float((err / (size + 1e-2)).max()))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rank", [128, 256, 512])
+def test_latent_attention_of_prompts_with_sinks_beyond_any_key(rank):
+    """Sinks of +inf, and of a size that overflows on its way to base 2, take all of a row's weight and leave zeros; one of -inf takes none."""
+    from vgate.ops import seq
+    g = torch.Generator().manual_seed(rank)
+    H, T, rot, scale = 4, 75, 64, 0.05
+    rows = torch.randn(T, rank + rot, generator=g).bfloat16()
+    qa = torch.randn(T, H, rank + rot, generator=g).bfloat16()
+    cache = torch.zeros(5, 16, rank + rot, dtype=torch.bfloat16)
+    cache.view(80, -1)[:T] = rows
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    ol = torch.full((T, H, rank), 9.0, dtype=torch.bfloat16, device="cuda")
+    seq.latent_attn(qa.cuda(), cache.cuda(), i32([list(range(5))]), i32([T]), i32([0, T]), ol, scale, H, rank, rot,
+                    cache_t=cache[:, :, :rank].transpose(1, 2).contiguous().cuda(),
+                    sink=torch.tensor([math.inf, 3e38, -math.inf, 0.0], device="cuda"))
+    ol = ol.double().cpu()
+    assert bool((ol[:, :2] == 0).all())
+    sc = torch.einsum("thd,jd->htj", qa[:, 2:].double(), rows.double()) * scale
+    sc = sc.masked_fill(torch.ones(T, T, dtype=torch.bool).triu(1), -math.inf)
+    extra = torch.tensor([-math.inf, 0.0], dtype=torch.float64)[:, None, None].expand(2, T, 1)
+    p = torch.softmax(torch.cat([sc, extra], -1), -1)[..., :-1]
+    c = rows[:, :rank].double()
+    assert bool(((ol[:, 2:].transpose(0, 1) - p @ c).abs() <= 2 * 2.0 ** -8 * (p @ c.abs()) + 1e-4).all())   # (as above)
+
+
 def oracle_attend(qa, rows, rank, scale, first_pos):
     out = torch.zeros(qa.shape[0], qa.shape[1], rank)
     for i in range(qa.shape[0]):
