@@ -629,6 +629,25 @@ def test_glu_rows(device, act):
 
 
 @pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("K,N,f32", [(512, 256, False), (40, 48, False), (40, 48, True)])
+def test_pair_projection_with_a_bias(device, act, K, N, f32):
+    """A gated pair with a bias on gate and up (packed, row-major, fp32): the bias is part of what is activated."""
+    from vgate.models.mixers import Proj
+    from vgate.ops import seq
+    g = torch.Generator().manual_seed(K)
+    dt = torch.float32 if f32 else torch.bfloat16
+    x, w = torch.randn(9, K, generator=g).to(dt), (torch.randn(N, K, generator=g) * K ** -0.5).to(dt)
+    bias = (3 * torch.randn(N, generator=g)).to(dt)
+    code = seq.ACT_GELU_TANH_MUL if act == "gelu_tanh" else seq.ACT_SILU_MUL
+    out = Proj(w, device, f32, silu_pair=True, bias=bias, pair_act=code)(x.to(device))
+    gate, up = (x.float() @ w.float().t() + bias.float()).split(N // 2, 1)
+    want = (oracle.gelu_tanh(gate) if act == "gelu_tanh" else oracle.silu(gate)) * up
+    # bf16: gate and up are rounded, then their result, 2^-9 of each at most
+    assert out.dtype == dt and rel(out, want) < (1e-5 if f32 else 3 * 2.0 ** -9)
+
+
+@pytest.mark.parametrize("device", DEVICES)
 @pytest.mark.parametrize("D,V", [(16, 24), (72, 40)])
 def test_linear_attention_long_portions(device, D, V):
     """Portions of hundreds of tokens (on the GPU scanned in parallel chunks with a carry between them): a

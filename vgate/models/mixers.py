@@ -62,11 +62,13 @@ class Proj:
         dev = torch.device(device)
         n_ok = (N // 2) % 64 == 0 if silu_pair else N % 64 == 0
         self.packed = allow_packed and n_ok and self.packs(K, device, f32)
+        # the pair epilogues take no bias: a pair with one is the plain product of [gate; up], then the activation
+        self.split_act = silu_pair and bias is not None
         self.bias = None
         if self.packed:
-            self.lin = ops.Linear(w.to(dev, torch.bfloat16), kind="silu" if silu_pair else "plain",
+            self.lin = ops.Linear(w.to(dev, torch.bfloat16), kind="silu" if silu_pair and not self.split_act else "plain",
                                   bias=None if bias is None else bias.to(dev, torch.bfloat16).contiguous())
-            if silu_pair and pair_act != seq.ACT_SILU_MUL:
+            if silu_pair and not self.split_act and pair_act != seq.ACT_SILU_MUL:
                 self.lin.glu = (pair_act, limit, alpha)
             self.w = None
         else:
@@ -85,6 +87,8 @@ class Proj:
 
     def __call__(self, x: torch.Tensor, out_f32: bool = False, act: int = 0, out: torch.Tensor | None = None) -> torch.Tensor:
         M = x.shape[0]
+        if self.split_act:
+            return self._split_pair(x, out_f32, out)
         if self.packed:   # (a single matrix's activation is a row kernel behind the packed GEMM)
             y = ops.linear(x, self.lin, out=out, out_f32=out_f32)
             return seq.act_rows(y, act) if act else y
@@ -95,6 +99,17 @@ class Proj:
             I = self.N // 2
             return seq.gemm(x, self.w[:I], out, w2=self.w[I:], act=self.pair_act, limit=self.limit, alpha=self.alpha)
         return seq.gemm(x, self.w, out, act=act, bias=self.bias)
+
+    def _split_pair(self, x: torch.Tensor, out_f32: bool, out: torch.Tensor | None) -> torch.Tensor:
+        M, I = x.shape[0], self.N // 2
+        dt = torch.float32 if not self.packed and (out_f32 or self.f32) else torch.bfloat16
+        if out is None:
+            out = torch.empty(M, I, dtype=dt, device=x.device)
+        if self.packed:
+            return seq.glu_rows(ops.linear(x, self.lin), out, self.pair_act, limit=self.limit, alpha=self.alpha)
+        gu = seq.gemm(x, self.w, torch.empty(M, self.N, dtype=dt, device=x.device), bias=self.bias).float()
+        out.copy_(seq._act(gu[:, :I], gu[:, I:], self.pair_act, self.limit, self.alpha))
+        return out
 
 
 def _f32(t: torch.Tensor, device) -> torch.Tensor:
