@@ -1,6 +1,7 @@
 """CPU checks of the op layer: weight packing layouts and the reference paths."""
 import math
 
+import pytest
 import torch
 
 from vgate import ops
@@ -26,6 +27,30 @@ def test_interleave_gate_up_roundtrip():
     assert torch.equal(lin.dense_weight(), torch.cat([wg, wu]))
     x = torch.randn(3, K).bfloat16()
     assert torch.allclose(ops.linear(x, lin).float(), ref.silu_mul_linear_ref(x, wg, wu).float())
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("M", [3, 70])
+def test_other_pair_activations_are_applied_or_refused(device, M):
+    """A pair's activation is the Linear's on every device; where no kernel has it (int4 weights, a norm in front, a layout without
+    pairs) the call raises, whatever its rows: never SiLU in its place."""
+    from vgate.ops import seq
+    I, K = 64, 128
+    w, x = torch.randn(2 * I, K).bfloat16() * 0.3, torch.randn(M, K).bfloat16()
+    glu = (seq.ACT_CLAMPED_GLU, 1.0, 1.702)
+    lin = ops.Linear(w.to(device), kind="silu")
+    lin.glu = glu
+    want = seq._act(x.float() @ w[:I].float().t(), x.float() @ w[I:].float().t(), *glu)
+    got = ops.linear(x.to(device), lin).float().cpu()
+    assert ((got - want).norm() / want.norm()).item() < 2.0 ** -8   # (fp32 sums, one rounding to bf16)
+    with pytest.raises(ValueError, match="pair activation"):
+        ops.linear(x.to(device), lin, norm=(torch.ones(K).bfloat16().to(device), 1e-6))
+    awq = dict(qint=torch.randint(0, 16, (2 * I, K), dtype=torch.int32), scales=torch.full((1, 2 * I), 0.02).bfloat16().to(device),
+               zeros=torch.full((1, 2 * I), 8.0).to(device), group=128)
+    for other in (ops.Linear(None, layout="silu", awq=awq), ops.Linear(w.to(device))):
+        other.glu = glu
+        with pytest.raises(ValueError, match="pair activation"):
+            ops.linear(x.to(device), other)
 
 
 def test_pack_awq_layout():

@@ -309,6 +309,8 @@ def linear(x: torch.Tensor, lin: Linear, out: torch.Tensor | None = None,
     """
     M = row_idx.numel() if row_idx is not None else x.shape[0]
     silu = lin.layout == "silu"
+    if lin.glu is not None and (not silu or lin.kind == "awq" or norm is not None or prenorm is not None):
+        raise ValueError("a pair activation other than SiLU: [gate; up] in bf16, without a norm in front")
     if qkv is not None:
         ncols = qkv["hq"] * 128
     else:
@@ -322,7 +324,11 @@ def linear(x: torch.Tensor, lin: Linear, out: torch.Tensor | None = None,
         wd = lin.dense_weight()
         if silu:
             I = lin.N // 2
-            out.copy_(ref.silu_mul_linear_ref(xx, wd[:I], wd[I:]))
+            if lin.glu is not None:
+                from vgate.ops import seq
+                out.copy_(seq._act(xx.float() @ wd[:I].float().t(), xx.float() @ wd[I:].float().t(), *lin.glu))
+            else:
+                out.copy_(ref.silu_mul_linear_ref(xx, wd[:I], wd[I:]))
         elif qkv is not None:
             y = ref.linear_ref(xx, wd, lin.bias)
             ref.rope_kv_ref(y, qkv["positions"], qkv["slots"], qkv["cos_sin"], qkv["k_cache"], qkv["v_cache"],
