@@ -41,6 +41,8 @@
 // (scale, scale*zero) applied in registers before the bf16 MFMA.
 // The kernel templates and their launch logic live in gemm_decode.h; each epilogue's
 // instantiations are compiled in gemm_epi_{bf16,f32,silu,qkv}.hip.
+#include <stdexcept>
+
 #include "gemm_decode.h"
 
 namespace vgate {
@@ -211,6 +213,10 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
     GemmArgs h = g;
     if (g.path == 0) h.ntb = 0;
     if (launch_gemm_prefill(h, st)) return;
+    if (h.ntb >= 5000) {  // rows off 16 B, a norm in registers or a row gather: the launcher's choice, a plan's numbers mean nothing below
+      h.path = 0; h.ntb = 0; h.splitk = 0;
+      return launch_gemm(h, st);
+    }
   }
   launch_dispatch<false>(to_params(g), g, st);
 }
@@ -228,7 +234,10 @@ void launch_awq_gemm(const GemmArgs& g, hipStream_t st) {
   if (g.path == 0 && ((g.ntb == 0 && g.waves == 0) || (g.ntb <= -12 && g.ntb >= -14)) && launch_awq_kx(g, st)) return;
   // mixed prefill + decode steps (16 < M <= 64) on the int4 medium kernel (path 2)
   if (g.path == 2 && launch_awq_mid(g, st)) return;
-  if (g.path == 5 && launch_q4_prompt(g, st)) return;
+  if (g.path == 5) {
+    if (launch_q4_prompt(g, st)) return;
+    throw std::runtime_error("gemm: the int4 prompt kernel does not take this tile, shape or alignment");
+  }
   launch_dispatch<true>(to_params(g), g, st);
 }
 

@@ -20,6 +20,7 @@
 // Grid: 1-D, XCD-aware bijective remap, m-blocks fastest so the blocks that share a weight
 // column panel run back to back on one XCD (one HBM read of the panel per XCD L2).
 #include <cstdlib>
+#include <stdexcept>
 
 #include "gemm_prompt.h"
 
@@ -1056,7 +1057,7 @@ static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, 
   const int nz = prefill_slices(p.M, p.N, p.K, force_bn, force_sk, p.slabs != nullptr ? slab_bytes : 0);
   if (force_bn >= 5000) {
     if (!rows16) return false;
-    if (!launch_gemm_w4<EPI, NORM>(p, force_bn, nz, st)) return false;
+    if (!launch_gemm_w4<EPI, NORM>(p, force_bn, nz, st)) throw std::runtime_error("gemm: no such four-wave tile, or none of N");
     if (nz > 1) launch_prefill_reduce<EPI, NORM, 1>(p, nz, st);
     return true;
   }

@@ -1218,6 +1218,46 @@ def test_prefill_four_wave_tiles_short_k(bn, K):
     assert _rel_err(out, x.double() @ w.double().t()) < K * 2.0 ** -24
 
 
+def test_forced_tiles_that_do_not_fit_raise():
+    """A forced four-wave or int4 tile that is none, or none of N, is an error: results of another kernel would pass for its own."""
+    C, M, N, K = ops.native(), 130, 320, 256
+    x, lin, q4 = torch.randn(M, K, device=DEV).bfloat16(), ops.Linear(torch.randn(N, K, device=DEV).bfloat16()), _awq(N, K, "plain", 1)
+    out = torch.empty(M, N, device=DEV)
+    dense = lambda code: C.gemm(x, lin.wp, N, K, out, 1, ws=ops.workspace(DEV), path=1, ntb=code, splitk=1)  # noqa: E731
+
+    def int4(code, scales=q4.scales):
+        C.gemm(x, q4.wp, N, K, out, 1, ws=ops.workspace(DEV), ntb=code, splitk=1, path=5, awq_scales=scales, awq_zeros=q4.zeros, group=128)
+    for code in (5340, 5380, 5999):
+        with pytest.raises(RuntimeError, match="four-wave tile"):
+            dense(code)
+    off = torch.zeros(q4.scales.numel() + 1, dtype=torch.bfloat16, device=DEV)[1:].view_as(q4.scales)
+    for code, scales in ((820, q4.scales), (99, q4.scales), (410, off)):
+        with pytest.raises(RuntimeError, match="int4 prompt kernel"):
+            int4(code, scales)
+    dense(5220)
+    assert _rel_err(out, x.float() @ lin.dense_weight().float().t()) < 1e-4
+    int4(410)
+    assert _rel_err(out, x.float() @ q4.dense_weight().float().t()) < 1e-4
+
+
+@pytest.mark.parametrize("M", [20, 70, 300])
+def test_plans_and_scales_that_a_step_cannot_use(M):
+    """A plan's four-wave tile for rows off 16 B, and int4 scales off 16 B: other kernels take the step, with the same products."""
+    N, K = 512, 512
+    lin = ops.Linear((torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16())
+    lin.prefill_plan = {32: (5220, 2), 96: (5220, 2), 512: (5340, 2)}
+    wide = torch.randn(M, K + 9, device=DEV).bfloat16()
+    for x in (wide[:, :K], wide[:, 1: K + 1]):
+        assert _rel_err(ops.linear(x, lin), x.float() @ lin.dense_weight().float().t()) < 2.0 ** -8
+    q4, x = _awq(N, K, "plain", M), wide[:, :K].contiguous()
+    want = ops.linear(x, q4, out_f32=True)
+    for name in ("scales", "zeros"):
+        t = getattr(q4, name)
+        off = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)[1:].view_as(t).copy_(t)
+        setattr(q4, name, off)
+        assert torch.equal(ops.linear(x, q4, out_f32=True), want), name
+
+
 @pytest.mark.parametrize("act", ["clamped", "gelu_tanh"])
 @pytest.mark.parametrize("M", [1, 16, 17, 48, 64, 65, 300, 1100])
 def test_gemm_pair_activations(act, M):
