@@ -1040,7 +1040,8 @@ template <int EPI, int NORM>
 bool launch_gemm_w4(const GemmParams& p, int code, int nz, hipStream_t st);
 
 // Returns false for shapes the kernels do not take (the caller keeps the N-split tile
-// kernels): K % 64, N % 64, a row gather, the gamma-in-registers RMSNorm mode; and where those are the cheapest form.
+// kernels): K % 64, N % 64, a row gather, the gamma-in-registers RMSNorm mode. A forced form that N is no multiple of: false too, but an
+// error for the four-wave tiles.
 template <int EPI, int NORM>
 static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, size_t slab_bytes, int max_counters,
                                hipStream_t st) {
@@ -1053,7 +1054,6 @@ static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, 
     force_bn = f.code;
     force_sk = f.nz;
   }
-  const bool wide = two_deep_wide(p.M, p.N, force_bn);
   const int nz = prefill_slices(p.M, p.N, p.K, force_bn, force_sk, p.slabs != nullptr ? slab_bytes : 0);
   if (force_bn >= 5000) {
     if (!rows16) return false;
@@ -1061,23 +1061,17 @@ static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, 
     if (nz > 1) launch_prefill_reduce<EPI, NORM, 1>(p, nz, st);
     return true;
   }
-  if (force_bn == 256) {  // forced (tests / sweeps), split-K as chosen above
-    if (p.N % 128 != 0) return false;
-    launch_prefill2_cfg<EPI, NORM, NTB>(p, nz, st);
-    return true;
-  }
-  if (force_bn == 512) {  // 256 x 256 block tile, 8 waves of 64 (m) x 128 (n), 2-deep ring (sweeps)
-    if (p.N % 256 != 0) return false;
-    launch_prefill2_cfg<EPI, NORM, NTB, 256, 256, 4, 2, 2>(p, nz, st);
-    return true;
-  }
-  if (force_bn == 1024) {  // v4: the 4-phase 256 x 256 kernel (sweeps / tests)
+  if (force_bn == 1024) {  // the 4-phase 256 x 256 kernel
     if (p.N % 256 != 0) return false;
     launch_prefill4_cfg<EPI, NORM, NTB>(p, nz, st);
     return true;
   }
-  // persistent forms of the 4-phase kernel, K-split tail (start-up tuner candidates; force_sk = the
-  // tail's K slices); declined -> the tile grid
+  if (force_bn == 768) {  // on a 256 x 128 tile
+    if (p.N % 128 != 0) return false;
+    launch_prefill4_cfg<EPI, NORM, NTB, 128>(p, nz, st);
+    return true;
+  }
+  // persistent forms of the 4-phase kernel, K-split tail (force_sk = the tail's K slices); declined -> the tile grid
   if (force_bn == 1025) {
     if (p.N % 256 != 0) return false;
     if (!launch_prefill4sk_cfg<EPI, NORM, NTB, 256>(p, force_sk, max_counters, slab_bytes, st))
@@ -1090,42 +1084,33 @@ static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, 
       launch_prefill4_cfg<EPI, NORM, NTB, 128>(p, 1, st);
     return true;
   }
-  if (force_bn == 768) {  // v4 on a 256 x 128 tile (sweeps / tests)
+  // 128-row tiles over 8 waves on a 4-deep ring, one block per CU
+  if (force_bn == 1281) {
     if (p.N % 128 != 0) return false;
-    launch_prefill4_cfg<EPI, NORM, NTB, 128>(p, nz, st);
+    launch_prefill2_cfg<EPI, NORM, NTB, 128, 128, 2, 4, 4>(p, nz, st);
     return true;
   }
-  // mid-M (128 < M <= 512) tuner candidates: the 128-row tiles on a 4-deep ring, one block per CU
-  // (the 2-deep ring above waits vmcnt(0) per K-tile and relies on a second resident block)
-  if (force_bn == 1280 || force_bn == 1281) {
-    if (p.N % 128 != 0) return false;
-    if (force_bn == 1280) launch_prefill2_cfg<EPI, NORM, NTB, 128, 128, 2, 2, 4>(p, nz, st);
-    else launch_prefill2_cfg<EPI, NORM, NTB, 128, 128, 2, 4, 4>(p, nz, st);
+  if (force_bn == 641) {
+    launch_prefill2_cfg<EPI, NORM, NTB, 128, 64, 4, 2, 4>(p, nz, st);
     return true;
   }
-  // wide-N mid-M tiles that fill the chip where the 256- / 128-row tiles leave CUs idle or waste rows
-  // (gate_up at 448 rows: 256 x 256 covers 140 of 256 CUs, 128-row tiles make 280 blocks): 64 x 512
-  // over 8 waves (448 rows: 7 x 35 = 245 blocks, no padded rows) and 128 x 320 over 8 waves (224)
-  if (force_bn == 2560) {
-    if (p.N % 512 != 0) return false;
-    launch_prefill2_cfg<EPI, NORM, NTB, 64, 512, 1, 8, 2>(p, nz, st);
+  // Sweeps and tests only: 256 x 128 on a 3-deep ring, 256 x 256 on a 2-deep one, the 128-row tiles above over 4 waves, 64 x 512 and
+  // 128 x 320 (with 32-deep stages on 4-deep rings those took 15-30 % longer, warm and cold: profiles/r5_prefill_wide_tiles_sweep.log), and,
+  // for any other code, 128 x 128 or 128 x 64 on a 2-deep ring, which waits for the stage it has just asked for and relies on a second block.
+  if constexpr (EPI != EPI_GLU) {
+    const int width = force_bn == 512 ? 256 : force_bn == 2560 ? 512 : force_bn == 2561 ? 320 : force_bn == 256 || force_bn == 1280 ? 128 : 64;
+    if (p.N % width != 0) return false;
+    if (force_bn == 256) launch_prefill2_cfg<EPI, NORM, NTB>(p, nz, st);
+    else if (force_bn == 512) launch_prefill2_cfg<EPI, NORM, NTB, 256, 256, 4, 2, 2>(p, nz, st);
+    else if (force_bn == 1280) launch_prefill2_cfg<EPI, NORM, NTB, 128, 128, 2, 2, 4>(p, nz, st);
+    else if (force_bn == 640) launch_prefill2_cfg<EPI, NORM, NTB, 128, 64, 2, 2, 4>(p, nz, st);
+    else if (force_bn == 2560) launch_prefill2_cfg<EPI, NORM, NTB, 64, 512, 1, 8, 2>(p, nz, st);
+    else if (force_bn == 2561) launch_prefill2_cfg<EPI, NORM, NTB, 128, 320, 2, 4, 2>(p, nz, st);
+    else if (two_deep_wide(p.M, p.N, force_bn)) launch_prefill_cfg<128, 128, EPI, NORM, NTB>(p, nz, st);
+    else launch_prefill_cfg<128, 64, EPI, NORM, NTB>(p, nz, st);
     return true;
   }
-  if (force_bn == 2561) {
-    if (p.N % 320 != 0) return false;
-    launch_prefill2_cfg<EPI, NORM, NTB, 128, 320, 2, 4, 2>(p, nz, st);
-    return true;
-  }
-  // (the same tiles with 32-deep stages on 4-deep rings measured 15-30 % slower warm and cold:
-  // profiles/r5_prefill_wide_tiles_sweep.log)
-  if (force_bn == 640 || force_bn == 641) {
-    if (force_bn == 640) launch_prefill2_cfg<EPI, NORM, NTB, 128, 64, 2, 2, 4>(p, nz, st);
-    else launch_prefill2_cfg<EPI, NORM, NTB, 128, 64, 4, 2, 4>(p, nz, st);
-    return true;
-  }
-  if (wide) launch_prefill_cfg<128, 128, EPI, NORM, NTB>(p, nz, st);
-  else launch_prefill_cfg<128, 64, EPI, NORM, NTB>(p, nz, st);
-  return true;
+  return false;
 }
 
 bool launch_gemm_prefill(const GemmArgs& g, hipStream_t st) {
