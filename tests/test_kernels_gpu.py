@@ -1218,6 +1218,27 @@ def test_prefill_four_wave_tiles_short_k(bn, K):
     assert _rel_err(out, x.double() @ w.double().t()) < K * 2.0 ** -24
 
 
+@pytest.mark.parametrize("act", [2, 4])
+@pytest.mark.parametrize("path,code,sk", [(1, c, sk) for c in (5220, 5340, 5380, 5580, 5640, 5680, 641, 1281, 768, 1024) for sk in (1, 3)] +
+                         [(1, 769, 0), (1, 1025, 0), (2, 2, 0), (2, 4, 0), (2, 4, 3), (2, 8, 0)])
+def test_pair_activations_in_every_form(path, code, sk, act):
+    """The clamped pair and the tanh GELU in each form that a step or a plan can take (prompt tiles, K slices and their combine, the
+    persistent forms' split tail, the medium kernel with its waves), rows past a tile, against 64 bits; their limit and alpha count."""
+    from vgate.ops import seq
+    C, K, I = ops.native(), 1024, 1280
+    for M in (300, 577) if path == 1 else (17, 50):
+        g = torch.Generator(DEV).manual_seed(M)
+        x = torch.randn(M, K, device=DEV, generator=g).bfloat16()
+        w = (torch.randn(2 * I, K, device=DEV, generator=g) * (4.0 / math.sqrt(K))).bfloat16()
+        lin, out = ops.Linear(w, layout="silu"), torch.full((M, I), float("nan"), dtype=torch.bfloat16, device=DEV)
+        kw = dict(ntb=code, splitk=sk) if path == 1 else dict(waves=code, splitk=sk)
+        C.gemm(x, lin.wp, 2 * I, K, out, 2, ws=ops.workspace(DEV), fault=ops.fault_word(DEV), path=path, act=act, limit=2.5, alpha=1.3, **kw)
+        gate, up = (x.double() @ w.double().t()).split(I, 1)
+        want = seq._act(gate, up, act, 2.5, 1.3)
+        assert ((out.double() - want).norm() / want.norm()).item() < 2.0 ** -8   # one rounding to bf16
+        assert torch.isfinite(out).all()
+
+
 def test_forced_tiles_that_do_not_fit_raise():
     """A forced four-wave or int4 tile that is none, or none of N, is an error: results of another kernel would pass for its own."""
     C, M, N, K = ops.native(), 130, 320, 256
@@ -1385,6 +1406,43 @@ def test_awq_prompt_epilogues_match_the_copied_matrix(M):
         pairs.append(got + [qkv["k_cache"], qkv["v_cache"]])
     for a, b in zip(*pairs):  # the same bf16 operands: fp32 sums in another order, rounded to bf16
         assert _rel_err(a, b) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("code", [410, 610, 620, 820, 1020, 1620, 640])
+@pytest.mark.parametrize("M,sk", [(65, 1), (300, 3)])
+def test_awq_prompt_epilogues_against_64_bits(M, sk, code):
+    """SiLU * mul and bias + QKV + RoPE + cache write of every int4 tile, with a norm, over the bf16 values that awq_dequant() writes."""
+    C, K, hq, hkv = ops.native(), 1024, 4, 2
+    g = torch.Generator(DEV).manual_seed(M)
+    x = torch.randn(M, K, device=DEV, generator=g).bfloat16()
+    gamma = (torch.rand(K, device=DEV, generator=g) + 0.5).bfloat16()
+    bias = torch.randn((hq + 2 * hkv) * 128, device=DEV, generator=g).bfloat16()
+    kw = dict(ws=ops.workspace(DEV), ntb=code, splitk=sk, path=5, group=128, norm_w=gamma, eps=1e-6)
+
+    def product(lin):
+        copy, w = torch.empty(lin.N * K, dtype=torch.bfloat16, device=DEV), torch.empty(lin.N, K, dtype=torch.float64, device=DEV)
+        C.awq_dequant(lin.wp, lin.scales, lin.zeros, lin.N, K, 128, copy, gamma)
+        w[ops.row_permutation(lin.N, lin.layout).to(DEV)] = ops.unpack_weight(copy, lin.N, K).double()
+        return x.double() @ w.t() * torch.rsqrt((x.double() ** 2).mean(1, keepdim=True) + 1e-6)
+
+    gu, h = _awq(1024, K, "silu", M), torch.full((M, 512), float("nan"), dtype=torch.bfloat16, device=DEV)
+    C.gemm(x, gu.wp, 1024, K, h, 2, awq_scales=gu.scales, awq_zeros=gu.zeros, **kw)
+    gate, up = product(gu).split(512, 1)
+    want = torch.nn.functional.silu(gate) * up
+    assert ((h.double() - want).norm() / want.norm()).item() < 2.0 ** -8   # one rounding to bf16
+
+    lin, q = _awq(1024, K, "qkv", M + 1, bias=bias), torch.full((M, hq * 128), float("nan"), dtype=torch.bfloat16, device=DEV)
+    kc = torch.zeros(M // 16 + 2, hkv, 16, 128, device=DEV).bfloat16()
+    vc, pos, slots = torch.zeros_like(kc), torch.arange(M, dtype=torch.int32, device=DEV) * 3, torch.arange(M, device=DEV).flip(0).int()
+    cs = ref.rope_cos_sin(4096, 128, 1e6, device=DEV)
+    C.gemm(x, lin.wp, 1024, K, q, 3, awq_scales=lin.scales, awq_zeros=lin.zeros, bias=bias, positions=pos, slots=slots, cos_sin=cs,
+           k_cache=kc, v_cache=vc, hq=hq, hkv=hkv, **kw)
+    y = (product(lin) + bias.double()).bfloat16().cpu()   # (rounded before it is rotated)
+    kc2, vc2 = torch.zeros_like(kc).cpu(), torch.zeros_like(vc).cpu()
+    ref.rope_kv_ref(y, pos.cpu(), slots.cpu(), cs.cpu(), kc2, vc2, hq, hkv, 128)
+    for got, want in ((q.cpu(), y[:, :hq * 128]), (kc.cpu(), kc2), (vc.cpu(), vc2)):
+        # bf16 twice, and values between two of them that the two sums round apart
+        assert _rel_err(got, want) < 2.0 ** -7
 
 
 @pytest.mark.parametrize("M", [200, 448, 640])
