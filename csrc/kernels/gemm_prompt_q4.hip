@@ -70,10 +70,17 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
       acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
       asm volatile("" : "+a"(acc[a][b]));  // (written here, well before the first mfma_acc)
     }
-  float ss[(MT + 3) / 4];  // wave w sums the squares of the row tiles w, w + 4, ...: a row in the order of K, as the bf16 forms do
+  // wave w sums the squares of the row tiles w, w + 4, ...: a row in the order of K, as the bf16 forms do. It reads them again: which of the
+  // fragments in registers are its own would be a branch per k-step, around which the accumulators lose their place (5 to 7 times as long)
+  constexpr int SQ = NORM ? (MT + 3) / 4 : 1;
+  float ss[SQ];
+  int so[SQ];
 #pragma unroll
-  for (int i = 0; i < (MT + 3) / 4; ++i) ss[i] = 0.f;
-  uint4 wf[2][NT], xf[2][MT], wq[NT];
+  for (int i = 0; i < SQ; ++i) {
+    ss[i] = 0.f;
+    so[i] = min(wid + 4 * i, MT - 1) * 4096;
+  }
+  uint4 wf[2][NT], xf[2][MT], wq[NT], sq[2][SQ];
   float sc[NT], zs[NT], gam[8];
   const int xlo[2] = {G::XB + x_frag_off(0, lane), G::XB + x_frag_off(1, lane)};
   auto read_stage = [&](const char* sb) {  // the group's packed weights and scales
@@ -107,19 +114,19 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
   };
   auto read_x = [&](int b, int u, const char* sb) {
     xf[u & 1][b] = *reinterpret_cast<const uint4*>(sb + xlo[u & 1] + b * 4096 + (u >> 1) * 2048);
+    if constexpr (NORM)
+      if (b < SQ) sq[u & 1][b] = *reinterpret_cast<const uint4*>(sb + xlo[u & 1] + so[b] + (u >> 1) * 2048);
+  };
+  // zeros in place of a stage's k half that belongs to the slice before or after (once in a slice at either end; no wave is reading it)
+  auto clear = [&](char* sb, int half) {
+    for (int e = threadIdx.x; e < MT * 128; e += 256)
+      *reinterpret_cast<uint4*>(sb + G::XB + (e >> 7) * 4096 + half * 2048 + (e & 127) * 16) = make_uint4(0, 0, 0, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   };
   constexpr int U = 2 * NT;  // halves of fragments of a k-step to unpack
   // the MFMAs of k-step u, a row tile at a time; between them the next k-step is read and unpacked and, at the last, the next stage asked for
-  auto phase = [&](auto uc, bool off, const char* sb, int st, int buf) {
+  auto phase = [&](auto uc, const char* sb, int st, int buf) {
     constexpr int u = decltype(uc)::value, v = (u + 1) & 3;
-    if (off) {  // (uniform) a k-step of the slice before or after
-#pragma unroll
-      for (int b = 0; b < MT; ++b) {
-        u32x4 none = {0, 0, 0, 0};
-        asm volatile("s_nop 1" : "+v"(none));
-        xf[u & 1][b] = __builtin_bit_cast(uint4, none);
-      }
-    }
     // (an MFMA reads what the VALU wrote two wait states before at the soonest, and the compiler does not see that mfma_acc() is one)
 #pragma unroll
     for (int a = 0; a < NT; ++a) {
@@ -129,16 +136,10 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
     }
     if constexpr (u == 3) read_stage(sb);
     read_gamma(v, sb);
-    if constexpr (NORM) {
-#pragma unroll
-      for (int w = 0; w < 4; ++w)
-        if (wid == w) {
-#pragma unroll
-          for (int b = w; b < MT; b += 4) ss[b >> 2] = sumsq8(xf[u & 1][b], ss[b >> 2]);
-        }
-    }
 #pragma unroll
     for (int b = 0; b < MT; ++b) {
+      if constexpr (NORM)
+        if (b < SQ) ss[b] = sumsq8(sq[u & 1][b], ss[b]);
       read_x(b, v, sb);
       if constexpr (u == 3) {
 #pragma unroll
@@ -160,6 +161,7 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
 #pragma unroll
     for (int i = 0; i < PPW; ++i) issue_piece(i, s0 < nk ? s0 : nk - 1, s0);
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * PPW) : "memory");
+  if (kt0 & 1) clear(smem, 0);
   read_stage(smem);
   read_gamma(0, smem);
 #pragma unroll
@@ -168,15 +170,15 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
   for (int e = 0; e < U; ++e) unpack(e >> 1, e & 1, 0);
   int buf = 0;
   for (int t = 0; t < nk; ++t) {
-    const char* sb = smem + buf * STAGE;
+    char* sb = smem + buf * STAGE;
     const int nb = buf + 1 == NS ? 0 : buf + 1;
-    const bool before = t == 0 && (kt0 & 1) != 0, after = t == nk - 1 && (kt1 & 1) != 0;
-    phase(C0{}, before, sb, 0, 0);
-    phase(C1{}, before, sb, 0, 0);
-    phase(C2{}, after, sb, 0, 0);
+    if (t == nk - 1 && (kt1 & 1) != 0) clear(sb, 1);
+    phase(C0{}, sb, 0, 0);
+    phase(C1{}, sb, 0, 0);
+    phase(C2{}, sb, 0, 0);
     // this stage is read (its last k-step is in registers), the next one has landed: both for every wave
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * PPW) : "memory");
-    phase(C3{}, after, smem + nb * STAGE, t + NS < nk ? t + NS : nk - 1, buf);  // past the end: clamped duplicates, never used
+    phase(C3{}, smem + nb * STAGE, t + NS < nk ? t + NS : nk - 1, buf);  // past the end: clamped duplicates, never used
     buf = nb;
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");  // the trailing duplicates
