@@ -266,7 +266,7 @@ static bool launch_q4_epi(const GemmParams& p, int code, int nz, hipStream_t st)
 // 2048 on cold weights; K-tiles of 128. Unpacking is repeated by every row of blocks, so from some row count on a bf16 copy (2.2 us + 0.56
 // a million weights) and the bf16 kernels are ahead: 17920 x 1536 at 448 rows 60 against 64 us, at 1024 114 against 89; 1536 x 1536 at 1024 17
 // against 22. Free in its slices the choice took 1.019 of the best form's time, and 1 / 1.26 of the copy's (geometric means); with the cut of K
-// given, a step of 256 rows through six layers of 1536 / 8960 takes 751 us instead of 730 (945 with copies).
+// given, a step of 256 rows through six layers of 1536 / 8960 takes 737 us instead of 734 (947 with copies), one of 320 rows 795 instead of 745.
 Q4Form q4_prompt_form(int M, int N, int K, bool norm, bool rows16, bool group128, size_t slab_bytes, int code, int sk) {
   struct Tile {
     int code, bm, bn, per_cu;
