@@ -290,7 +290,7 @@ int64_t ar_error_offset() { return (int64_t)offsetof(ArSignal, error); }
 uint32_t ar_spin() { return ar_spin_limit(); }
 int64_t ar_blocks_used() { return ar_blocks(); }
 static_assert(offsetof(ArSignal, ticks) == offsetof(ArSignal, error) + 4 && offsetof(ArSignal, calls) == offsetof(ArSignal, error) + 8,
-              "ids_to_host copies {error, ticks, calls} as consecutive words");
+              "the sampler copies {error, ticks, calls} as consecutive words");
 
 void launch_custom_allgather(const void* in, void* out, int64_t nbytes, char* const* bases, int rank, int world,
                              int64_t max_bytes, hipStream_t st) {

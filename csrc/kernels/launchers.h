@@ -165,12 +165,6 @@ void launch_prefetch(const void* p, size_t bytes, int blocks, hipStream_t st);
 void set_dec_u(int u);  // decode GEMM register group: -100 the launcher's rule, 6 / 8 / 10 / 12 forced (tests)
 void set_flash_prefill(int on);  // prefill tiles on the flash kernel: 1 on, 0 off (16-query tiles), -1 env
 void launch_copy16(const void* src, void* dst, size_t bytes, bool to_host, hipStream_t st);
-// ids[0, n) -> ring[*slot * stride + i] (ring: device-mapped pinned host memory); with `ar` (the
-// own custom all-reduce signal area's error word, or null) also its {error, ticks, calls} words ->
-// ring[*slot * stride + stride - 4 + {0, 1, 2}] (the TP collective health / time, no host sync); with
-// `fault` (ops.fault_word: the sticky give-up word of the in-launch hand-offs) also -> stride - 1
-void launch_ids_to_host(const int32_t* ids, int32_t* ring, const int32_t* slot, int stride, int n, hipStream_t st,
-                        const uint32_t* ar = nullptr, const uint32_t* fault = nullptr);
 
 // NeoX RoPE on q,k inside the fused qkv buffer + paged KV-cache write.
 // qkv: [T, (Hq + 2*Hkv) * D]; cos_sin: [max_pos, D] f32 (cos | sin halves)
@@ -220,7 +214,7 @@ struct AttnArgs {
   size_t fl_ws_bytes = 0;
   uint32_t* fl_tickets = nullptr;
   // sticky kernel-fault word (bit 1: a flash K-split waiter gave up), copied to the host each step by
-  // launch_ids_to_host; null = none
+  // launch_sample; null = none
   uint32_t* fault = nullptr;
 };
 // In-launch hand-off of the fused QKV projection + decode attention (qkv_attn.hip): the nprod GEMM
@@ -259,6 +253,13 @@ struct SampleArgs {
   void* gran = nullptr;
   uint32_t* epoch = nullptr;
   uint32_t* fault = nullptr;
+  // the step's results for the host (device-mapped pinned memory), or null: out[0, B) -> ring[*ring_slot * ring_stride + i], the fault word
+  // if it is set -> ring_stride - 1 and, with `ar` (the own custom all-reduce signal area's error word), its {error, ticks, calls} words ->
+  // ring_stride - 4 + {0, 1, 2}: the health and time of the collectives without a sync
+  int32_t* ring = nullptr;
+  const int32_t* ring_slot = nullptr;
+  int ring_stride = 0;
+  const uint32_t* ar = nullptr;
 };
 // sampler workspace (int32 words): [0, SAMPLE_WS_GRAN) per-row epochs, then the granule regions
 constexpr int SAMPLE_GRAN_SEGS = 64;                        // max segments per row

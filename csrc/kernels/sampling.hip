@@ -23,6 +23,7 @@
 // Merges read the segments' partials in a fixed order: bit-reproducible.
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #include "launchers.h"
 #include "sampling_common.h"
@@ -46,43 +47,66 @@ __device__ __forceinline__ uint32_t lane_x(uint32_t v) {
     return (threadIdx.x & 32) ? r[0] : r[1];
   }
 }
-template <int K>
-__device__ __forceinline__ void acc_step(Acc& a, float c) {
-  const float om = __uint_as_float(lane_x<K>(__float_as_uint(a.mx)));
-  const float oz = __uint_as_float(lane_x<K>(__float_as_uint(a.z)));
-  const int oi = (int)lane_x<K>((uint32_t)a.amx);
-  const float ok = __uint_as_float(lane_x<K>(__float_as_uint(a.gk)));
-  const int ogi = (int)lane_x<K>((uint32_t)a.gi);
-  const float ocnt = __uint_as_float(lane_x<K>(__float_as_uint(a.cnt)));
-  const float oq = __uint_as_float(lane_x<K>(__float_as_uint(a.q)));
-  merge_mz(a.mx, a.z, a.amx, om, oz, oi, c);
-  merge_g(a.gk, a.gi, ok, ogi);
-  a.cnt += ocnt;
-  a.q += oq;
+// a wave's values under a commutative operation, the same in every lane
+template <typename T, typename F>
+__device__ __forceinline__ T wave_all(T v, F f) {
+  auto other = [](T x, auto k) { return __builtin_bit_cast(T, lane_x<decltype(k)::value>(__builtin_bit_cast(uint32_t, x))); };
+  v = f(v, other(v, std::integral_constant<int, 1>{}));
+  v = f(v, other(v, std::integral_constant<int, 2>{}));
+  v = f(v, other(v, std::integral_constant<int, 4>{}));
+  v = f(v, other(v, std::integral_constant<int, 8>{}));
+  v = f(v, other(v, std::integral_constant<int, 16>{}));
+  v = f(v, other(v, std::integral_constant<int, 32>{}));
+  return __builtin_bit_cast(T, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ float wave_max(float v) { return wave_all(v, [](float a, float b) { return fmaxf(a, b); }); }
+__device__ __forceinline__ float wave_sum(float v) { return wave_all(v, [](float a, float b) { return a + b; }); }
+__device__ __forceinline__ int wave_min(int v) { return wave_all(v, [](int a, int b) { return a < b ? a : b; }); }
+
+using Mode0 = std::integral_constant<int, 0>;
+using Mode1 = std::integral_constant<int, 1>;
+
+// The merge of a wave's partials, in every lane. Maxima first, then one rescaling per lane and plain sums: merged pairwise, each of the six
+// steps waits for two exponentials (1.2 us a merge and three merges a pass).
+template <typename Mode>
+__device__ __forceinline__ Acc wave_merge(const Acc& a, float c, Mode) {
+  Acc r = acc_init();
+  r.gk = wave_max(a.gk);
+  r.gi = wave_min(a.gi >= 0 && a.gk == r.gk ? a.gi : 0x7fffffff);  // (equal keys: the lower index)
+  const uint64_t at = __ballot(a.gi == r.gi);
+  if (at == 0) {
+    r.gi = -1;
+  } else {
+    r.gx = __uint_as_float(__builtin_amdgcn_readlane((int)__float_as_uint(a.gx), __builtin_ctzll(at)));
+  }
+  if constexpr (Mode::value == 0) {
+    r.mx = wave_max(a.mx);
+    r.amx = wave_min(a.mx == r.mx ? a.amx : 0x7fffffff);
+    r.z = wave_sum(a.mx == r.mx ? a.z : a.z * __builtin_amdgcn_exp2f((a.mx - r.mx) * c));  // (z = 0 where mx = -inf)
+  } else {
+    r.cnt = wave_sum(a.cnt);
+    r.q = wave_sum(a.q);
+  }
+  return r;
 }
 
-// Block-wide reduction of an Acc into LDS slot `out` (thread 0 holds the result).
-__device__ __forceinline__ void block_reduce_acc(Acc& a, float c, Acc* red) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  __syncthreads();  // `red` may still be read by thread 0 from a previous reduction
-  acc_step<1>(a, c);
-  acc_step<2>(a, c);
-  acc_step<4>(a, c);
-  acc_step<8>(a, c);
-  acc_step<16>(a, c);
-  acc_step<32>(a, c);
-  if (lane == 0) red[wid] = a;
+// The merge of the waves' results that `red` holds, in every lane of the calling wave
+template <typename Mode>
+__device__ __forceinline__ Acc merge_waves(const Acc* red, int nw, float c, Mode mode) {
+  const int lane = threadIdx.x & 63;
+  Acc a = red[lane < nw ? lane : 0];
+  if (lane >= nw) a = acc_init();
+  return wave_merge(a, c, mode);
+}
+
+// Block-wide reduction (the first wave holds the result).
+template <typename Mode>
+__device__ __forceinline__ Acc block_reduce_acc(const Acc& a, float c, Acc* red, Mode mode) {
+  __syncthreads();  // `red` may still be read by the first wave from a previous reduction
+  const Acc w = wave_merge(a, c, mode);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = w;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    Acc r = red[0];
-    for (int w = 1; w < nw; ++w) {
-      merge_mz(r.mx, r.z, r.amx, red[w].mx, red[w].z, red[w].amx, c);
-      merge_g(r.gk, r.gi, red[w].gk, red[w].gi);
-      r.cnt += red[w].cnt;
-      r.q += red[w].q;
-    }
-    a = r;
-  }
+  return threadIdx.x < 64 ? merge_waves(red, blockDim.x >> 6, c, mode) : w;
 }
 
 // Per-row sampling parameters (row-uniform).
@@ -108,27 +132,36 @@ __device__ __forceinline__ RowParams row_params(const SampleArgs& a, int row) {
   return r;
 }
 
-// One element's contribution to a pass (shared by the memory sweep and the register-resident
-// rounds below, so both produce the same bits): mode 0 (max / Z / argmax + Gumbel key), mode 1
+// Four logits' contribution to a pass (shared by the memory sweep and the register-resident
+// segments, so both produce the same bits): mode 0 (max / Z / argmax + Gumbel key), mode 1
 // (count and mass above xj + the key restricted to x > xj). L = logf(fmaxf(-logf(u), 1e-30f)) of
-// this element's uniform for the pass's round (key = v / T - L: a Gumbel draw).
-__device__ __forceinline__ void accum_elem(int mode, float v, int i, float L, float xj, float rmx, const RowParams& rp,
-                                           Acc& acc) {
-  if (mode == 0) {
-    if (v > acc.mx) {
-      acc.z = (acc.mx == -INFINITY ? 0.f : acc.z * exp2f((acc.mx - v) * rp.c)) + 1.f;
-      acc.mx = v;
-      acc.amx = i;
-    } else if (v > -INFINITY) {
-      acc.z += exp2f((v - acc.mx) * rp.c);
+// each logit's uniform for the pass's round (key = v / T - L: a Gumbel draw). The maximum of the four comes first, so that the sum over them
+// waits for one rescaling and not for four (the exponents are those of the maximum so far; v == mx counts 1 also where both are infinite).
+// (Modes are known when this is compiled: with one that is not, stores into either mode's fields are merged into one through a pointer,
+// and the accumulator moves to memory.)
+template <int mode>
+__device__ __forceinline__ void accum4(const float (&v)[4], int i, const float (&L)[4], float xj, float rmx, const RowParams& rp, Acc& acc) {
+  if constexpr (mode == 0) {
+    const float m = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
+    if (m > acc.mx) {
+      acc.z = acc.z * __builtin_amdgcn_exp2f((acc.mx - m) * rp.c);  // (0 while mx = -inf)
+      acc.mx = m;
+      acc.amx = i + (v[0] == m ? 0 : v[1] == m ? 1 : v[2] == m ? 2 : 3);
     }
-  } else if (v > xj) {
-    acc.cnt += 1.f;
-    acc.q += exp2f((v - rmx) * rp.c);
   }
-  if (!rp.greedy && (mode == 0 || v > xj) && v > -INFINITY) {
-    const float g = v * rp.cn - L;
-    if (g > acc.gk) { acc.gk = g; acc.gi = i; }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if constexpr (mode == 0) {
+      acc.z += v[j] > -INFINITY ? (v[j] == acc.mx ? 1.f : __builtin_amdgcn_exp2f((v[j] - acc.mx) * rp.c)) : 0.f;
+    } else {
+      acc.cnt += v[j] > xj ? 1.f : 0.f;
+      acc.q += v[j] > xj ? __builtin_amdgcn_exp2f((v[j] - rmx) * rp.c) : 0.f;
+    }
+    const float g = v[j] * rp.cn - L[j];
+    const bool take = !rp.greedy && (mode == 0 || v[j] > xj) && v[j] > -INFINITY && g > acc.gk;
+    acc.gk = take ? g : acc.gk;
+    acc.gi = take ? i + j : acc.gi;
+    acc.gx = take ? v[j] : acc.gx;
   }
 }
 
@@ -139,7 +172,8 @@ __device__ __forceinline__ float gumbel_log(float u) { return logf(fmaxf(-logf(u
 // thread). mode 0: max / Z / argmax + Gumbel keys; mode 1: acceptance statistics of candidate
 // value xj (count and mass of x > xj, mass relative to the row max rmx) + Gumbel keys restricted
 // to x > xj with the noise of `round`.
-__device__ __forceinline__ void sweep_range(const float4* x4, int v_lo, int v_hi, int mode, float xj, float rmx,
+template <int mode>
+__device__ __forceinline__ void sweep_range(const float4* x4, int v_lo, int v_hi, float xj, float rmx,
                                             uint32_t round, const RowParams& rp, Acc& acc) {
   const int tid = threadIdx.x, nt = blockDim.x;
   for (int v0 = v_lo + tid; v0 < v_hi; v0 += nt * 8) {
@@ -158,18 +192,40 @@ __device__ __forceinline__ void sweep_range(const float4* x4, int v_lo, int v_hi
       const float e[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
       float uu[4] = {0.5f, 0.5f, 0.5f, 0.5f};
       if (!rp.greedy) philox4(rp.seed, rp.off, (uint32_t)vi, round, uu);
+float L[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float v = e[j];
-        const float L = (!rp.greedy && (mode == 0 || v > xj) && v > -INFINITY) ? gumbel_log(uu[j]) : 0.f;
-        accum_elem(mode, v, 4 * vi + j, L, xj, rmx, rp, acc);
-      }
+      for (int j = 0; j < 4; ++j)
+        L[j] = (!rp.greedy && (mode == 0 || e[j] > xj) && e[j] > -INFINITY) ? gumbel_log(uu[j]) : 0.f;
+      accum4<mode>(e, 4 * vi, L, xj, rmx, rp, acc);
     }
   }
 }
 
+// The host ring's words past the sampled ids: the sticky fault word, if it is set (the host clears its copies after a recovery), and the
+// custom all-reduce's {error, ticks, calls}. What earlier launches of the step raised is final here; a wait of this launch that gives up
+// hands its own bit over (fault_to_host).
+__device__ __forceinline__ void ring_store(const SampleArgs& a, int at, uint32_t v) {
+  __hip_atomic_store(reinterpret_cast<uint32_t*>(a.ring) + (size_t)*a.ring_slot * a.ring_stride + at, v, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void fault_to_host(const SampleArgs& a, uint32_t more) {
+  if (a.fault == nullptr || a.ring == nullptr) return;
+  const uint32_t f = __hip_atomic_load(a.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) | more;
+  if (f != 0) ring_store(a, a.ring_stride - 1, f);
+}
+
 __device__ __forceinline__ void finish_row(const SampleArgs& a, int row, int chosen, float mx, float z, float c) {
   a.out[row] = chosen;
+  if (a.ring != nullptr) {
+    ring_store(a, row, (uint32_t)chosen);
+    fault_to_host(a, 0u);
+    if (a.ar != nullptr && row == 0) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        ring_store(a, a.ring_stride - 4 + i, __hip_atomic_load(a.ar + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
+    }
+    drain_stores();
+  }
   if (a.out_logprob) a.out_logprob[row] = ((a.logits[(size_t)row * a.ldl + chosen] - mx) * c - log2f(z)) / LOG2E_S;
 }
 
@@ -187,21 +243,21 @@ __global__ __launch_bounds__(NT) void sample_row_kernel(SampleArgs a) {
   const float4* x4 = reinterpret_cast<const float4*>(x);
   const RowParams rp = row_params(a, row);
   const float c = rp.c;
-  auto pass = [&](int mode, float xj, float rmx, uint32_t round) {
+  auto pass = [&](auto mode, float xj, float rmx, uint32_t round) {
     Acc acc = acc_init();
-    sweep_range(x4, 0, V4, mode, xj, rmx, round, rp, acc);
-    block_reduce_acc(acc, c, red);
+    sweep_range<decltype(mode)::value>(x4, 0, V4, xj, rmx, round, rp, acc);
+    acc = block_reduce_acc(acc, c, red, mode);
     if (tid == 0) merged = acc;
     __syncthreads();
   };
-  pass(0, 0.f, 0.f, 0u);
+  pass(Mode0{}, 0.f, 0.f, 0u);
   const float mx = merged.mx, z = merged.z;
   int chosen = merged.amx, j = merged.gi;
   if (!rp.greedy) {
     if (rp.use_k || rp.use_p) {
       const float pmass = rp.topp * z;
       for (uint32_t round = 1; round <= SAMPLE_MAX_ROUNDS && j >= 0; ++round) {
-        pass(1, x[j], mx, round);
+        pass(Mode1{}, merged.gx, mx, round);
         const bool ok_k = !rp.use_k || merged.cnt < (float)rp.topk;
         const bool ok_p = !rp.use_p || merged.q < pmass;
         if (ok_k && ok_p) break;
@@ -214,6 +270,8 @@ __global__ __launch_bounds__(NT) void sample_row_kernel(SampleArgs a) {
 }
 
 // ---- single launch: tagged granules instead of tickets / counters ----
+// What a pass takes: the noise, and the merges and meetings, 3 us of them (6.5 before the merges of wave_merge; us, top-p 0.95, rows half
+// greedy, before -> now: 8 rows of 32000 21.7 -> 13.2, 32 rows 23.5 -> 15.3, 64 rows 33.8 -> 21.3; greedy, one row 9.7 -> 6.9).
 // The pass kernels' meetings cost a launch boundary per pass, the in-launch ones a serialised
 // atomic per arriving block (~0.5 us each, 32 per row). Here every block of a row publishes its
 // pass partial as two 16-B granules {.., tag} (device-coherent sc1 stores, one transaction each),
@@ -227,23 +285,24 @@ __global__ __launch_bounds__(NT) void sample_row_kernel(SampleArgs a) {
 // Each row owns a FIXED granule region of SAMPLE_GRAN_SEGS segments whatever the launch's (B, nseg):
 // a slot is only ever written by its own row, under that row's monotonic epoch. (A layout that moved
 // with nseg let row r read row r' < r's leftovers from a launch of another batch size whose tag
-// happened to equal r's current one — round-4 ADVICE.)
+// happened to equal r's current one.)
 // Every wait is bounded: a give-up sets fault bit 16 (the engine fails the step) and the row
 // falls back to its argmax. B x nseg <= 256 blocks: all co-resident.
-__device__ __forceinline__ void gran_publish(uint4* g, const Acc& a, int mode, uint32_t tag) {
-  // mode 0 (pass 0): {mx, z, amx} + {gk, gi}; mode 1 (rounds): {cnt, q, gk} + {gi}
-  const f32x4 g0 = mode == 0 ? f32x4{a.mx, a.z, __int_as_float(a.amx), __uint_as_float(tag)}
-                             : f32x4{a.cnt, a.q, a.gk, __uint_as_float(tag)};
-  const f32x4 g1 = mode == 0 ? f32x4{a.gk, __int_as_float(a.gi), 0.f, __uint_as_float(tag)}
-                             : f32x4{__int_as_float(a.gi), 0.f, 0.f, __uint_as_float(tag)};
-  st_sc1_x4(reinterpret_cast<float*>(g), 0u, g0);
-  st_sc1_x4(reinterpret_cast<float*>(g), 16u, g1);
+template <typename Mode>
+__device__ __forceinline__ void gran_publish(uint4* g, const Acc& a, Mode, uint32_t tag) {
+  // mode 0 (pass 0): {mx, z, amx}, mode 1 (rounds): {cnt, q}; then {gk, gi, gx}. (Word by word out of the struct: put together as one vector
+  // from it, the struct is read as a vector and lives in memory.)
+  float p0 = Mode::value == 0 ? +a.mx : +a.cnt, p1 = Mode::value == 0 ? +a.z : +a.q, p2 = __int_as_float(a.amx);
+  float k0 = a.gk, k1 = __int_as_float(a.gi), k2 = a.gx;
+  asm volatile("" : "+v"(p0), "+v"(p1), "+v"(p2), "+v"(k0), "+v"(k1), "+v"(k2));
+  st_sc1_x4(reinterpret_cast<float*>(g), 0u, f32x4{p0, p1, p2, __uint_as_float(tag)});
+  st_sc1_x4(reinterpret_cast<float*>(g), 16u, f32x4{k0, k1, k2, __uint_as_float(tag)});
 }
 
-// wave 0: gather the nseg granule pairs of (row, parity) and merge them in lane order; lane 0 ends
-// with the merge. Returns false if a wait gave up.
-__device__ __forceinline__ bool gran_gather(const uint4* gbase, int nseg, int mode, uint32_t tag, float c, Acc& out,
-                                            uint32_t* fault) {
+// one wave: gather the nseg granule pairs of (row, parity) and merge them, in every lane. Returns false if a wait gave up.
+template <typename Mode>
+__device__ __forceinline__ bool gran_gather(const SampleArgs& args, const uint4* gbase, int nseg, Mode mode, uint32_t tag, float c,
+                                            Acc& out) {
   const int lane = threadIdx.x & 63;
   Acc a = acc_init();
   bool ok = true;
@@ -259,22 +318,23 @@ __device__ __forceinline__ bool gran_gather(const uint4* gbase, int nseg, int mo
       __builtin_amdgcn_s_sleep(1);
     }
     if (ok) {
-      if (mode == 0) {
-        a.mx = g0[0]; a.z = g0[1]; a.amx = __float_as_int(g0[2]); a.gk = g1[0]; a.gi = __float_as_int(g1[1]);
+      if constexpr (Mode::value == 0) {
+        a.mx = g0[0];
+        a.z = g0[1];
+        a.amx = __float_as_int(g0[2]);
       } else {
-        a.cnt = g0[0]; a.q = g0[1]; a.gk = g0[2]; a.gi = __float_as_int(g1[0]);
+        a.cnt = g0[0];
+        a.q = g0[1];
       }
+      a.gk = g1[0]; a.gi = __float_as_int(g1[1]); a.gx = g1[2];
     }
   }
   const bool all_ok = __all(ok);
-  if (!all_ok && lane == 0 && fault != nullptr) atomicOr(fault, 16u);
-  acc_step<1>(a, c);
-  acc_step<2>(a, c);
-  acc_step<4>(a, c);
-  acc_step<8>(a, c);
-  acc_step<16>(a, c);
-  acc_step<32>(a, c);
-  out = a;
+  if (!all_ok && lane == 0 && args.fault != nullptr) {
+    atomicOr(args.fault, 16u);
+    fault_to_host(args, 16u);
+  }
+  out = wave_merge(a, c, mode);
   return all_ok;
 }
 
@@ -294,10 +354,10 @@ __global__ __launch_bounds__(NT) void sample_gran_kernel(SampleArgs a) {
   const uint32_t ep = __builtin_amdgcn_readfirstlane(__float_as_uint(ld_sc1(reinterpret_cast<const float*>(a.epoch + row))));
   uint4* rowg = reinterpret_cast<uint4*>(a.gran) + (size_t)row * SAMPLE_GRAN_ROW;  // [parity][SEGS][2]
   // one pass: sweep, block merge, publish, gather every segment's granules, share the row merge
-  auto pass = [&](int mode, float xj, float rmx, uint32_t round, uint32_t gen) -> bool {
+  auto pass = [&](auto mode, float xj, float rmx, uint32_t round, uint32_t gen) -> bool {
     Acc acc = acc_init();
-    sweep_range(x4, v_lo, v_hi, mode, xj, rmx, round, rp, acc);
-    block_reduce_acc(acc, c, red);
+    sweep_range<decltype(mode)::value>(x4, v_lo, v_hi, xj, rmx, round, rp, acc);
+    acc = block_reduce_acc(acc, c, red, mode);
     const uint32_t tag = (ep << 6) | gen;
     uint4* pg = rowg + (size_t)(gen & 1) * SAMPLE_GRAN_SEGS * 2;
     if (tid == 0) {
@@ -305,7 +365,7 @@ __global__ __launch_bounds__(NT) void sample_gran_kernel(SampleArgs a) {
     }
     if (tid < 64) {
       Acc r;
-      const bool ok = gran_gather(pg, nseg, mode, tag, c, r, a.fault);
+      const bool ok = gran_gather(a, pg, nseg, mode, tag, c, r);
       if (tid == 0) {
         merged = r;
         s_ok = ok;
@@ -315,19 +375,21 @@ __global__ __launch_bounds__(NT) void sample_gran_kernel(SampleArgs a) {
     return s_ok != 0;
   };
   uint32_t gen = 1;
-  bool ok = pass(0, 0.f, 0.f, 0u, gen);
+  bool ok = pass(Mode0{}, 0.f, 0.f, 0u, gen);
   const float mx = merged.mx, z = merged.z;
   int chosen = merged.amx, j = merged.gi;
+  float xj = merged.gx;
   if (ok && !rp.greedy) {
     if (rp.use_k || rp.use_p) {
       const float pmass = rp.topp * z;
       for (uint32_t round = 1; round <= SAMPLE_MAX_ROUNDS && j >= 0; ++round) {
-        ok = pass(1, x[j], mx, round, ++gen);
+        ok = pass(Mode1{}, xj, mx, round, ++gen);
         if (!ok) { j = -1; break; }
         const bool ok_k = !rp.use_k || merged.cnt < (float)rp.topk;
         const bool ok_p = !rp.use_p || merged.q < pmass;
         if (ok_k && ok_p) break;
         j = merged.gi;  // next candidate, drawn from {x > x_j}
+        xj = merged.gx;
       }
     }
     if (j >= 0) chosen = j;
@@ -344,18 +406,20 @@ __global__ __launch_bounds__(NT) void sample_gran_kernel(SampleArgs a) {
 int g_sample_nseg = SAMPLE_GRAN_SEGS;  // segments per row cap (set_sample_nseg; benchmarks/sampler_stress.py)
 void set_sample_nseg(int n) { g_sample_nseg = n < 1 ? 1 : (n > SAMPLE_GRAN_SEGS ? SAMPLE_GRAN_SEGS : n); }
 
+// At least 1024 logits in a segment, and no more than 8 to 24 segments of 2048: each block of a row polls all of the row's partials, which
+// takes 1 us with 8 of them and 2.8 with 31 (us, top-p 0.95, 8 rows of 32000: 31 segments 19.4, 16 14.7, 8 15.3; of 151936: 31 25, 24 19.6,
+// 16 21.5, 8 29.3).
 int sample_segments(int B, int V) {
   const int V4 = V >> 2;
   int nseg = SAMPLE_MAX_BLOCKS / (B > 0 ? B : 1);
   if (nseg > g_sample_nseg) nseg = g_sample_nseg;
-  const int cap = V4 / 256;  // >= 1024 logits per segment
-  if (nseg > cap) nseg = cap;
+  nseg = std::min(nseg, std::min(V4 / 256, std::max(8, std::min(24, V4 / 512))));
   return nseg < 1 ? 1 : nseg;
 }
 
 // More waves where a thread of 256 would have more than 12 pieces of 16 B: the noise of a segment (Philox, two logarithms per logit)
-// then takes longer than the meeting, and four waves cannot keep a CU busy with it. us, top-p 0.95, 256 -> 1024 threads:
-// vocabulary 152064, 32 rows 42.8 -> 37.2, 64 rows 103 -> 78, 256 rows (whole rows) 339 -> 201; 16 rows (9 pieces) 29.7 against 31.2.
+// then takes longer than the meeting (us, top-p 0.95, 512 -> 1024 threads: vocabulary 151936, 32 rows 29.4 -> 27.6, 64 rows 68.6 -> 62.9, 16 rows
+// 24.0, 23.7; 32000, 64 rows 21.3, 21.6, 128 rows 34.5 -> 33.0, 8 rows 14.7, 15.5. 256 threads: 15.2 and 24.4 at 8 and 64 rows of 32000).
 static bool long_rows(int V, int nseg) { return (V >> 2) > 3072 * nseg; }
 // More whole rows than CUs: two workgroups of 1024 threads share a CU, of 256 eight, and only a long row makes up for that (us, 256 ->
 // 1024 threads, greedy and top-p: 512 rows of 32000 27, 104 -> 35, 114, of 65536 44, 179 -> 48, 180, of 128256 76, 347 -> 71, 295; 768 rows of
@@ -369,7 +433,7 @@ void launch_sample(const SampleArgs& s, hipStream_t st) {
   if (nseg > 1 && s.gran != nullptr && s.epoch != nullptr && s.B <= SAMPLE_GRAN_ROWS) {
     a.tl = tl_take("sample_gran", nseg * s.B);
     if (long_rows(s.V, nseg)) hipLaunchKernelGGL(sample_gran_kernel<1024>, dim3(nseg, s.B), dim3(1024), 0, st, a);
-    else hipLaunchKernelGGL(sample_gran_kernel<256>, dim3(nseg, s.B), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(sample_gran_kernel<512>, dim3(nseg, s.B), dim3(512), 0, st, a);
     return;
   }
   a.tl = tl_take("sample", s.B);

@@ -1,5 +1,5 @@
 // Sampling math of the sampler (sampling.hip): Philox4x32-10 uniforms, the (max, Z, argmax,
-// Gumbel key) accumulator and its merges.
+// Gumbel key) accumulator.
 #pragma once
 #include "common.h"
 
@@ -44,24 +44,10 @@ struct Acc {  // POD (lives in LDS too); start from acc_init()
   int amx;
   float gk;
   int gi;
+  float gx;  // the logit at gi
   float cnt, q;
 };
 
-__device__ __forceinline__ Acc acc_init() { return Acc{-INFINITY, 0.f, 0x7fffffff, -INFINITY, -1, 0.f, 0.f}; }
-
-__device__ __forceinline__ void merge_mz(float& mx, float& z, int& amx, float om, float oz, int oi, float c) {
-  const float nm = fmaxf(mx, om);
-  const float zz = (mx == -INFINITY ? 0.f : z * exp2f((mx - nm) * c)) + (om == -INFINITY ? 0.f : oz * exp2f((om - nm) * c));
-  if (om > mx || (om == mx && oi < amx)) amx = oi;
-  mx = nm;
-  z = zz;
-}
-
-__device__ __forceinline__ void merge_g(float& gk, int& gi, float ok, int oi) {
-  if (oi >= 0 && (ok > gk || (ok == gk && (gi < 0 || oi < gi)))) {
-    gk = ok;
-    gi = oi;
-  }
-}
+__device__ __forceinline__ Acc acc_init() { return Acc{-INFINITY, 0.f, 0x7fffffff, -INFINITY, -1, 0.f, 0.f, 0.f}; }
 
 }  // namespace vgate

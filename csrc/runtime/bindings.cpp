@@ -442,11 +442,21 @@ void attention(const Tensor& q, int64_t q_stride, const Tensor& k_cache, const T
   vgate::launch_attention(a, a.S, cur_stream());
 }
 
+static void* device_view(const Tensor& t) {
+  if (t.is_cuda()) return t.data_ptr();
+  TORCH_CHECK(t.is_pinned(), "kernel_copy: host tensor must be pinned");
+  void* d = nullptr;
+  TORCH_CHECK(hipHostGetDevicePointer(&d, t.data_ptr(), 0) == hipSuccess && d != nullptr,
+              "kernel_copy: pinned host memory is not device-mapped");
+  return d;
+}
+
 void sample(const Tensor& logits, const c10::optional<Tensor>& temperature,
             const c10::optional<Tensor>& top_p, const c10::optional<Tensor>& top_k,
             const c10::optional<Tensor>& seeds, const c10::optional<Tensor>& offsets, Tensor& out,
             const c10::optional<Tensor>& out_logprob, const c10::optional<Tensor>& ws,
-            const c10::optional<Tensor>& fault) {
+            const c10::optional<Tensor>& fault, const c10::optional<Tensor>& ring, const c10::optional<Tensor>& ring_slot,
+            int64_t ar_base) {
   CHECK_DEV(logits); CHECK_DEV(out);
   CHECK_DT(logits, torch::kFloat32); CHECK_DT(out, torch::kInt32);
   CHECK_LASTDIM(logits);
@@ -481,21 +491,22 @@ void sample(const Tensor& logits, const c10::optional<Tensor>& temperature,
   }
   s.fault = reinterpret_cast<uint32_t*>(opt_ptr<int32_t>(fault, torch::kInt32, "fault"));
   c10::DeviceGuard guard(logits.device());
+  if (ring.has_value() && ring->defined()) {
+    CHECK_DT((*ring), torch::kInt32);
+    TORCH_CHECK(ring->dim() == 2 && ring->is_contiguous() && !ring->is_cuda(), "sample: ring = pinned int32 [slots, stride]");
+    TORCH_CHECK(s.B <= ring->size(1) - 4, "sample: a ring slot holds the ids and four words");
+    TORCH_CHECK(ring_slot.has_value() && ring_slot->defined() && ring_slot->numel() >= 1, "sample: the ring needs its slot");
+    s.ring = static_cast<int32_t*>(device_view(*ring));
+    s.ring_slot = static_cast<const int32_t*>(fp(ring_slot, torch::kInt32));
+    s.ring_stride = (int)ring->size(1);
+    if (ar_base) s.ar = reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(ar_base) + vgate::ar_error_offset());
+  }
   vgate::launch_sample(s, cur_stream());
 }
 
 // Warm the memory-side cache with a tensor's bytes (default-policy read sweep, nothing written).
 // Copy the first `nbytes` (rounded up to 16, within both tensors) between a pinned host tensor and
 // a device tensor with a kernel on the current stream (no SDMA engine hand-off, see elementwise.hip).
-static void* device_view(const Tensor& t) {
-  if (t.is_cuda()) return t.data_ptr();
-  TORCH_CHECK(t.is_pinned(), "kernel_copy: host tensor must be pinned");
-  void* d = nullptr;
-  TORCH_CHECK(hipHostGetDevicePointer(&d, t.data_ptr(), 0) == hipSuccess && d != nullptr,
-              "kernel_copy: pinned host memory is not device-mapped");
-  return d;
-}
-
 void kernel_copy(Tensor& dst, const Tensor& src, int64_t nbytes) {
   TORCH_CHECK(dst.is_contiguous() && src.is_contiguous(), "kernel_copy: contiguous tensors");
   TORCH_CHECK(dst.is_cuda() != src.is_cuda(), "kernel_copy: one host (pinned) and one device tensor");
@@ -507,23 +518,6 @@ void kernel_copy(Tensor& dst, const Tensor& src, int64_t nbytes) {
               "kernel_copy: 16-B aligned tensors");
   c10::DeviceGuard guard(dev.device());
   vgate::launch_copy16(device_view(src), device_view(dst), (size_t)n, !dst.is_cuda(), cur_stream());
-}
-
-void ids_to_host(const Tensor& ids, Tensor& ring, const Tensor& slot, int64_t n, int64_t ar_base,
-                 const c10::optional<Tensor>& fault) {
-  CHECK_DEV(ids); CHECK_DEV(slot);
-  CHECK_DT(ids, torch::kInt32); CHECK_DT(ring, torch::kInt32); CHECK_DT(slot, torch::kInt32);
-  TORCH_CHECK(ring.dim() == 2 && ring.is_contiguous() && !ring.is_cuda(), "ids_to_host: ring = pinned int32 [slots, stride]");
-  TORCH_CHECK(n >= 0 && n <= ids.numel() && n <= ring.size(1), "ids_to_host: n exceeds ids or a ring slot");
-  const uint32_t* fw = reinterpret_cast<const uint32_t*>(opt_ptr<int32_t>(fault, torch::kInt32, "fault"));
-  TORCH_CHECK((ar_base == 0 && fw == nullptr) || n <= ring.size(1) - 4,
-              "ids_to_host: the all-reduce / fault words need the slot's last 4 ints");
-  const uint32_t* ar = ar_base ? reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(ar_base) + vgate::ar_error_offset())
-                               : nullptr;
-  c10::DeviceGuard guard(ids.device());
-  vgate::launch_ids_to_host(reinterpret_cast<const int32_t*>(ids.data_ptr()), reinterpret_cast<int32_t*>(device_view(ring)),
-                            reinterpret_cast<const int32_t*>(slot.data_ptr()), (int)ring.size(1), (int)n, cur_stream(), ar,
-                            fw);
 }
 
 void prefetch(const Tensor& t, int64_t blocks) {
@@ -682,7 +676,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("sample", &sample, "temperature/top-k/top-p sampling (segmented Gumbel-max + exact rejection)",
         py::arg("logits"), py::arg("temperature"), py::arg("top_p"), py::arg("top_k"), py::arg("seeds"),
         py::arg("offsets"), py::arg("out"), py::arg("out_logprob") = py::none(), py::arg("ws") = py::none(),
-        py::arg("fault") = py::none());
+        py::arg("fault") = py::none(), py::arg("ring") = py::none(), py::arg("ring_slot") = py::none(), py::arg("ar_base") = 0);
   m.def("sample_segments", &vgate::sample_segments, "blocks per row the sampler uses for (B, V)");
   m.def("set_sample_nseg", &vgate::set_sample_nseg, "cap the sampler's segments per row (1 = one block per row)");
   m.attr("SAMPLE_WS_WORDS") = vgate::SAMPLE_WS_WORDS;
@@ -690,9 +684,6 @@ PYBIND11_MODULE(_C, m) {
         py::arg("dst"), py::arg("src"), py::arg("nbytes"));
   m.def("set_flash_prefill", &vgate::set_flash_prefill, "flash prefill attention: 1 on, 0 off, -1 environment");
   m.def("set_dec_u", &vgate::set_dec_u, "decode GEMM register group: 0 auto, -1 round-2 rule, 6/8/10/12 forced, -100 environment");
-  m.def("ids_to_host", &ids_to_host, "sampled ids -> slot *slot of a pinned host ring (graph-capturable, device-read slot)",
-        py::arg("ids"), py::arg("ring"), py::arg("slot"), py::arg("n"), py::arg("ar_base") = 0,
-        py::arg("fault") = py::none());
   m.def("prefetch", &prefetch, "read a tensor once with the default cache policy (MALL warm-up)",
         py::arg("t"), py::arg("blocks") = 256);
   m.def("ar_alloc", &ar_alloc, "uncached device allocation for the custom all-reduce (zeroed)");

@@ -47,3 +47,39 @@ def test_more_rows_than_workgroups(V, B):
 
     whole = run(B)
     assert torch.equal(run(64), whole[:64]) and torch.equal(whole[::3], lg[::3].argmax(-1).int())
+
+
+@pytest.mark.parametrize("B,V", [(1, 4096), (8, 32000), (40, 8192), (300, 4096)])
+def test_extreme_logits_and_the_ring(B, V):
+    """Masked logits (-inf, the type's lowest value), one of +inf and NaN beside finite ones: the token is one of the few that count. The
+    ids also go to the ring's slot, with the fault word behind them only where it is set."""
+    dev = "cuda"
+    g = torch.Generator().manual_seed(B * V)
+    lg = torch.empty(B, V)
+    few = torch.randint(0, V, (B, 3), generator=g)
+    for b in range(B):
+        lg[b] = (-torch.inf, torch.finfo(torch.float32).min, torch.nan)[b % 3]
+        lg[b, few[b]] = torch.tensor([1.0, 1.5, 0.5])
+        if b % 4 == 3:
+            lg[b, few[b, 0]] = torch.inf
+    t = torch.tensor([0.8, 0.0, 1.0, 0.7, 0.9] * B)[:B]
+    p = torch.tensor([0.9, 1.0, 0.95] * B)[:B]
+    ring = torch.full((2, B + 4), -7, dtype=torch.int32, pin_memory=True)
+    slot = torch.tensor([1], dtype=torch.int32, device=dev)
+    fault = ops.fault_word(torch.device(dev))
+    seen = []
+    for word in (0, 4):
+        fault.fill_(word)
+        out = ops.sample(lg.to(dev), t.to(dev), p.to(dev), None, torch.arange(B, device=dev), torch.full((B,), 3, device=dev), ring=(ring, slot, 0))
+        torch.cuda.synchronize()
+        seen.append((out.cpu(), ring.clone()))
+    fault.zero_()
+    for (ids, r), tail in zip(seen, (-7, 4)):
+        assert torch.equal(r[1, :B], ids) and torch.all(r[0] == -7) and r[1, B:].tolist() == [-7, -7, -7, tail]
+        assert torch.equal(ids, seen[0][0])
+        for b in range(B):
+            assert ids[b] in few[b], (b, int(ids[b]))
+            if b % 4 == 3:
+                assert ids[b] == few[b, 0], b
+            elif t[b] == 0.0:
+                assert ids[b] == few[b][lg[b, few[b]].argmax()], b

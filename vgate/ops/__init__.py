@@ -683,8 +683,11 @@ def attention_prefill(q, q_stride, k_cache, v_cache, block_tables, context_lens,
 
 
 def sample(logits, temperature=None, top_p=None, top_k=None, seeds=None, offsets=None,
-           out=None, out_logprob=None, generators=None):
-    """Temperature / top-k / top-p sampling per row (csrc/kernels/sampling.hip)."""
+           out=None, out_logprob=None, generators=None, ring: tuple | None = None):
+    """Temperature / top-k / top-p sampling per row (csrc/kernels/sampling.hip).
+
+    ring (GPU): (pinned int32 [slots, >= B + 4], device int32 [1], address of the own custom all-reduce or 0): the ids also go to that
+    slot of the ring, with the fault and collective words behind them (launchers.h SampleArgs)."""
     B = logits.shape[0]
     if out is None:
         out = torch.empty(B, dtype=torch.int32, device=logits.device)
@@ -692,7 +695,7 @@ def sample(logits, temperature=None, top_p=None, top_k=None, seeds=None, offsets
         out.copy_(ref.sample_ref(logits, temperature, top_p, top_k, generators))
         return out
     native().sample(logits, temperature, top_p, top_k, seeds, offsets, out, out_logprob, sample_workspace(logits.device),
-                    fault_word(logits.device))
+                    fault_word(logits.device), *(ring or ()))
     return out
 
 

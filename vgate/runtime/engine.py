@@ -809,7 +809,7 @@ class LLMEngine:
         ar = self.tp.custom_ar
         if ar is None:
             return
-        # the step graph's ids_to_host node copies the all-reduce's words into the ring slot; a CPU
+        # the step graph's last node copies the all-reduce's words into the ring slot; a CPU
         # group (gloo, no ring words) reads the error word through ar.check() below
         if self.runner.gpu and self.runner.ar_base:
             err, secs, calls = self.runner.collective_words()

@@ -236,11 +236,9 @@ class ModelRunner:
     # ----------------------------------------------------------------- forward
     def _forward_sample(self, view):
         logits = self.model.forward(view, self.kv, self.part_size)
+        # last node of the step graph: the sampled ids, also (with fault / collective words) to the pinned ring slot
         ops.sample(logits, view.temperature, view.top_p, view.top_k, view.seeds, view.offsets,
-                   out=self.out_tokens[: view.S])
-        if self.gpu:  # last node of the step graph: sampled ids (+ fault / collective words) -> pinned ring slot
-            ops.native().ids_to_host(self.out_tokens, self.out_ring, view.ring_slot, view.S, self.ar_base,
-                                     fault=self.fault)
+                   out=self.out_tokens[: view.S], ring=(self.out_ring, view.ring_slot, self.ar_base) if self.gpu else None)
         return logits
 
     def _capture(self, T: int, S: int):
