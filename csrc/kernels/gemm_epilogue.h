@@ -118,6 +118,16 @@ __device__ __forceinline__ uint4 norm_frag(uint4 a, const bf16_t* w, int k0, flo
   }
 }
 
+// x^2 of 8 bf16 (one B fragment) into acc: 4 packed dot products (v_dot2_f32_bf16), no unpack — the
+// folded RMSNorm's row sums ride along the MFMA loop at a quarter of the unpack + FMA VALU cost
+typedef __bf16 p4_bf2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float sumsq8(uint4 v, float acc) {
+  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.x), __builtin_bit_cast(p4_bf2, v.x), acc, false);
+  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.y), __builtin_bit_cast(p4_bf2, v.y), acc, false);
+  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.z), __builtin_bit_cast(p4_bf2, v.z), acc, false);
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.w), __builtin_bit_cast(p4_bf2, v.w), acc, false);
+}
+
 // ---- epilogue operands that do not depend on the GEMM result ----
 // The decode kernel loads them at launch (phase A: row / bias / residual words, phase B:
 // the RoPE cos/sin row of the position, issued once the first weight group is in flight),

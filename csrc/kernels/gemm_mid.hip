@@ -11,8 +11,8 @@
 //
 // Here a block is W waves = W adjacent 16-column tiles (one per wave) over one K slice of at most
 // KS k-steps:
-//   1. the slice of x (MT m-tiles x KS k-steps, 1 KiB fragment-major pieces, rows past M repeat
-//      row M - 1) is DMA'd into LDS (global_load_lds_dwordx4), spread over the W waves;
+//   1. the slice of x (MT m-tiles x KS k-steps, in 64-k tiles of two 1 KiB pieces of whole 128-B lines, lds_rows.h; rows past M
+//      repeat row M - 1) is DMA'd into LDS (global_load_lds_dwordx4), spread over the W waves;
 //   2. every wave then issues ALL KS weight fragments of its tile (non-temporal 16-B loads into
 //      registers): the whole launch's weights are requested in the first microsecond;
 //   3. one counted vmcnt (the x pieces only) + barrier, then per k-step MT conflict-free
@@ -25,6 +25,7 @@
 #include <cstdlib>
 
 #include "gemm_epilogue.h"
+#include "lds_rows.h"
 
 namespace vgate {
 
@@ -38,27 +39,45 @@ static int cu_count_mid() {
   return n;
 }
 
+// Pieces of x for the 64-k tiles t0, t0 + dt, .. < nt of an image whose first k is the descriptor's: 8 rows each, the c-th of the 2 R in a
+// tile (16-row tile c / 2, half c & 1), at lds + (t 2 R + c) KiB. A wave keeps to one c, so that a piece is an addition to a scalar:
+// addresses worked out piece by piece took the small forms as long as their loads (1024 x 1024 at 24 rows 5.9 against 5.3 us).
+template <int R>
+__device__ __forceinline__ void stage_x(const GemmParams& p, u32x4 xrs, int row0, int kleft, int c, int t0, int dt, int nt, int lane,
+                                        uint32_t lds) {
+  const int col = x_piece_col(c & 1, lane);
+  const uint32_t vo = (uint32_t)x_piece_row(row0 + 16 * (c >> 1), c & 1, lane, p.M) * (uint32_t)p.lda * 2u + (uint32_t)col * 2u;
+  for (int t = t0; t < nt; t += dt) {
+    uint32_t v = vo;
+    if (64 * t + 64 > kleft && col >= 32) v -= 64;  // (K % 64 = 32: the second half of the last tile repeats the first and is not read)
+    blds16(xrs, v, (uint32_t)t * 128u, __builtin_amdgcn_readfirstlane(lds + (uint32_t)(t * 2 * R + c) * 1024u));
+  }
+}
+// the whole image by a block of nw waves
+template <int R>
+__device__ __forceinline__ void stage_x_all(const GemmParams& p, u32x4 xrs, int row0, int kleft, int nt, int wid, int nw, int lane, uint32_t lds) {
+  if (nw >= 2 * R) {
+    const int c = wid % (2 * R);
+    stage_x<R>(p, xrs, row0, kleft, c, wid / (2 * R), (nw - c + 2 * R - 1) / (2 * R), nt, lane, lds);
+  } else {
+    for (int c = wid; c < 2 * R; c += nw) stage_x<R>(p, xrs, row0, kleft, c, 0, 1, nt, lane, lds);
+  }
+}
+
 template <int MT, int KS, int EPI, int NORM>
 __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmParams p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];  // [KS][MT][64][16 B]
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // [KS / 2][MT][2 KiB]
   TLScope tl_scope(p.dbg_ts);
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int W = blockDim.x >> 6;
   const int KT = p.K >> 5;
   const int z = blockIdx.y, S = gridDim.y;
-  const int k0 = (KT * z) / S, nks = (KT * (z + 1)) / S - k0;  // nks <= KS (host-checked)
+  const int KT2 = (KT + 1) >> 1, kt0 = (KT2 * z) / S, kt1 = (KT2 * (z + 1)) / S;  // slices of whole 64-k tiles
+  const int k0 = 2 * kt0, nks = min(2 * kt1, KT) - k0;  // nks <= KS (host-checked)
   const int nt = blockIdx.x * W + wid;
-  // 1) x slice -> LDS: piece f = (k-step f / MT, m-tile f % MT); wave w takes f = w, w + W, ...
-  const uint32_t lds0 = lds_addr_of(smem);
-  const int npc = nks * MT;
-  for (int f = wid; f < npc; f += W) {
-    const int ks = f / MT, mt = f % MT;
-    int row = mt * 16 + (lane & 15);
-    row = row < p.M ? row : p.M - 1;
-    const bf16_t* src = p.x + (size_t)row * p.lda + (size_t)(k0 + ks) * 32 + 8 * (lane >> 4);
-    glds16(src, __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)f * 1024u));
-  }
+  // 1) x slice -> LDS
+  stage_x_all<MT>(p, rsrc_words(p.x + (size_t)kt0 * 64), 0, p.K - kt0 * 64, kt1 - kt0, wid, W, lane, lds_addr_of(smem));
   // 2) every weight fragment of this wave's tile slice (clamped past the slice: never consumed)
   uint4 w[KS];
   const uint4* wb = p.wp + ((size_t)nt * KT + k0) * 64 + lane;
@@ -74,20 +93,18 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmParams p) {
   float ss[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) ss[mt] = 0.f;
-  const uint4* xs = reinterpret_cast<const uint4*>(smem);
+  const int xo[2] = {x_frag_off(0, lane), x_frag_off(1, lane)};
+  const bool sums = S == 1 || (blockIdx.x == 0 && wid == 0);  // wave-uniform: who needs the rows' squares
 #pragma unroll
   for (int u = 0; u < KS; ++u) {
     if (u < nks) {  // wave-uniform
       uint4 xb[MT];
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) xb[mt] = xs[(u * MT + mt) * 64 + lane];
+      for (int mt = 0; mt < MT; ++mt) xb[mt] = *reinterpret_cast<const uint4*>(smem + ((u >> 1) * MT + mt) * 2048 + xo[u & 1]);
       if constexpr (NORM == 2) {
+        if (sums) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          float f[8];
-          unpack8(xb[mt], f);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) ss[mt] += f[j] * f[j];
+          for (int mt = 0; mt < MT; ++mt) ss[mt] = sumsq8(xb[mt], ss[mt]);
         }
       }
 #pragma unroll
@@ -131,13 +148,15 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmParams p) {
 // enough every CU can own WHOLE tiles instead: block b owns tiles [N b / B, N (b + 1) / B) (4-5 of
 // Qwen2.5-1.5B's 1120 gate_up tiles on 256 CUs: one round, no tail of late blocks), each tile's K
 // is cut into KP parts of <= 16 k-steps, one wave per (tile, part) holding all of its weight
-// fragments in registers (64 VGPRs, issued at launch: ~200 KB per CU in flight). x is shared
+// fragments in registers (64 VGPRs, issued at launch: ~200 KB per CU in flight). us, cold weights, x staged by fragments and squared by
+// every wave -> by whole lines and once: 17920 x 1536 at 32 rows 14.1 -> 13.0, with a norm 17.7 -> 14.9, at 64 rows 19.1 -> 16.2 and 24.6 ->
+// 19.1 (96 x 128 four-wave tiles 20.9); sliced form 6144 x 4096 with a norm at 48 31.0 -> 26.0, at 64 36.0 -> 30.6. x is shared
 // through LDS, a PAIR of m-tiles (32 rows x full K, 2 KB per k-step) at a time: the weights stay
 // in registers while the second pair is DMA'd in. The parts of a tile meet in LDS (fixed part
 // order: bit-reproducible) and the part-0 wave runs the epilogue.
 template <int MT, int EPI, int NORM>
 __global__ __launch_bounds__(1024) void gemm_midw_kernel(GemmParams p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];  // x [KT][PH][64][16 B] | red, ssq
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // x [(KT + 1) / 2][PH][2 KiB] | red, ssq
   TLScope tl_scope(p.dbg_ts);
   constexpr int PH = MT == 1 ? 1 : 2;  // m-tiles per x phase
   constexpr int NPH = (MT + PH - 1) / PH;
@@ -151,9 +170,13 @@ __global__ __launch_bounds__(1024) void gemm_midw_kernel(GemmParams p) {
   const bool active = my < ntb;  // wave-uniform
   const int nt = t0 + (active ? my : 0);
   const int kb = part * 16, nks = min(16, KT - kb);
+  // wave-uniform: the rows' squares are summed once, by the first tile's waves (shared out over all of them, a test per k-step: 64 rows,
+  // 17920 x 1536 19.8 us against 19.1)
+  const bool sums = my == 0 || KP == 1;
   uint4 w[16];
   const uint32_t lds0 = lds_addr_of(smem);
-  const uint4* xs = reinterpret_cast<const uint4*>(smem);
+  const u32x4 xrs = rsrc_words(p.x);
+  const int xo[2] = {x_frag_off(0, lane), x_frag_off(1, lane)};
   f32x4 acc[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -163,13 +186,7 @@ __global__ __launch_bounds__(1024) void gemm_midw_kernel(GemmParams p) {
 #pragma unroll
   for (int ph = 0; ph < NPH; ++ph) {
     if (ph > 0) __builtin_amdgcn_s_barrier();  // every wave is done reading the previous phase's x
-    // x pieces of m-tiles (PH ph ..): piece f = (k-step f / PH, m-tile PH ph + f % PH)
-    for (int f = wid; f < PH * KT; f += nw) {
-      int row = (PH * ph + f % PH) * 16 + (lane & 15);
-      row = row < p.M ? row : p.M - 1;
-      glds16(p.x + (size_t)row * p.lda + (size_t)(f / PH) * 32 + 8 * (lane >> 4),
-             __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)f * 1024u));
-    }
+    stage_x_all<PH>(p, xrs, PH * ph * 16, p.K, (KT + 1) >> 1, wid, nw, lane, lds0);
     if (ph == 0) {
       if (active) {
         const uint4* wb = p.wp + ((size_t)nt * KT + kb) * 64 + lane;
@@ -191,12 +208,9 @@ __global__ __launch_bounds__(1024) void gemm_midw_kernel(GemmParams p) {
 #pragma unroll
           for (int i = 0; i < PH; ++i) {
             if (PH * ph + i < MT) {
-              const uint4 xv = xs[((kb + u) * PH + i) * 64 + lane];
+              const uint4 xv = *reinterpret_cast<const uint4*>(smem + (((kb + u) >> 1) * PH + i) * 2048 + xo[u & 1]);  // (kb is even)
               if constexpr (NORM == 2) {
-                float f[8];
-                unpack8(xv, f);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) ss[PH * ph + i] += f[j] * f[j];
+                if (sums) ss[PH * ph + i] = sumsq8(xv, ss[PH * ph + i]);
               }
               acc[PH * ph + i] = mfma16(as_bf16x8(w[u]), as_bf16x8(xv), acc[PH * ph + i]);
             }
@@ -234,7 +248,7 @@ __global__ __launch_bounds__(1024) void gemm_midw_kernel(GemmParams p) {
         float s2 = ss[mt];
         s2 += xor16(s2);
         s2 += xor32(s2);
-        if (lane < 16) ssq[(wid * MT + mt) * 16 + lane] = s2;
+        if (sums && lane < 16) ssq[(wid * MT + mt) * 16 + lane] = s2;
       }
     }
   }
@@ -244,12 +258,12 @@ __global__ __launch_bounds__(1024) void gemm_midw_kernel(GemmParams p) {
   for (int mt = 0; mt < MT; ++mt) {
     const int m = mt * 16 + (lane & 15);
     f32x4 v[1] = {red[(wid * MT + mt) * 64 + lane]};
-    float s2 = NORM == 2 ? ssq[(wid * MT + mt) * 16 + (lane & 15)] : 0.f;
-    for (int q = 1; q < KP; ++q) {
-      v[0] += red[((wid + q) * MT + mt) * 64 + lane];
-      if constexpr (NORM == 2) s2 += ssq[((wid + q) * MT + mt) * 16 + (lane & 15)];
+    for (int q = 1; q < KP; ++q) v[0] += red[((wid + q) * MT + mt) * 64 + lane];
+    if constexpr (NORM == 2) {
+      float s2 = 0.f;
+      for (int q = 0; q < KP; ++q) s2 += ssq[(q * MT + mt) * 16 + (lane & 15)];
+      v[0] *= rsqrtf(s2 / (float)p.K + p.eps);
     }
-    if constexpr (NORM == 2) v[0] *= rsqrtf(s2 / (float)p.K + p.eps);
     epilogue<1, EPI, false>(p, v, m, nt, nsub, EpiPre<1>{}, m < p.M);
   }
 }
@@ -294,11 +308,11 @@ static bool launch_mid_epi(const GemmParams& p, int force_w, int force_s, size_t
   const int groups = ntiles / W;
   int S = force_s > 0 ? force_s : 1;
   if (force_s <= 0) {
-    while ((KT + S - 1) / S > 32) ++S;
+    while (2 * (((KT + 1) / 2 + S - 1) / S) > 32) ++S;
     while (groups * S < 192 && (KT + 2 * S - 1) / (2 * S) >= 4) S *= 2;
   }
-  const int ks = (KT + S - 1) / S;
-  if (S < 1 || S > KT || ks > 32) return false;
+  const int ks = 2 * (((KT + 1) / 2 + S - 1) / S);  // (slices of whole 64-k tiles)
+  if (S < 1 || S > (KT + 1) / 2 || ks > 32) return false;
   if (S > 1 && (p.slabs == nullptr || ((size_t)S * p.M * p.N + (size_t)S * p.M) * 4 > slab_bytes)) return false;
   if (MT <= 2) launch_mid_mt<2, EPI, NORM>(p, W, S, ks, st);
   else if (MT == 3) launch_mid_mt<3, EPI, NORM>(p, W, S, ks, st);
@@ -316,7 +330,7 @@ static bool launch_midw_epi(const GemmParams& p, hipStream_t st) {
   if (KT > 64 || KP * tmax > 16 || ntiles < nb) return false;
   const int MT = (p.M + 15) / 16;
   const dim3 grid(nb), block(64 * KP * tmax);
-  const size_t lds = std::max<size_t>((size_t)KT * (MT == 1 ? 1 : 2) * 1024, (size_t)KP * tmax * MT * (1024 + 64));
+  const size_t lds = std::max<size_t>((size_t)(KT + 1) / 2 * (MT == 1 ? 1 : 2) * 2048, (size_t)KP * tmax * MT * (1024 + 64));
   GemmParams q = p;
   if (q.dbg_ts == nullptr) q.dbg_ts = tl_take("gemm_midw", nb);
 #define VG_MW(P_)                                                                                      \

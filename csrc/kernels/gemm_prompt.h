@@ -20,16 +20,6 @@
 
 namespace vgate {
 
-// x^2 of 8 bf16 (one B fragment) into acc: 4 packed dot products (v_dot2_f32_bf16), no unpack — the
-// folded RMSNorm's row sums ride along the MFMA loop at a quarter of the unpack + FMA VALU cost
-typedef __bf16 p4_bf2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float sumsq8(uint4 v, float acc) {
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.x), __builtin_bit_cast(p4_bf2, v.x), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.y), __builtin_bit_cast(p4_bf2, v.y), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.z), __builtin_bit_cast(p4_bf2, v.z), acc, false);
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(p4_bf2, v.w), __builtin_bit_cast(p4_bf2, v.w), acc, false);
-}
-
 // The epilogue of a wave's MT x NT tiles of a prompt GEMM (rows m0 + 16 b, tiles nt0 + a; value(a, b): the tile's accumulator, row scale
 // applied): epilogue()'s results, with what does not depend on the tile loaded, and divided, once per row. Tile by tile the loads of
 // positions, rotations, slots and residuals cannot pass the stores before them (they may alias), and every tile waits for memory:

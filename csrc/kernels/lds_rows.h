@@ -1,5 +1,5 @@
 // Rows of a bf16 matrix staged in LDS by DMA so that both sides are fast: whole 128-B lines from memory, MFMA fragments free of bank
-// conflicts out of LDS (gemm_prefill.hip, gemm_prompt.h, gemm_prompt_q4.hip, latent_attn.hip).
+// conflicts out of LDS (gemm_prefill.hip, gemm_prompt.h, gemm_prompt_q4.hip, gemm_mid.hip, latent_attn.hip).
 #pragma once
 #include "common.h"
 
