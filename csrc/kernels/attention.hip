@@ -171,11 +171,13 @@ __device__ __forceinline__ constexpr int vm_imm(int n) {  // s_waitcnt vmcnt(n),
   return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8);
 }
 
-// dec_seqs > 0: the step's decode rows ride in the same launch — grid rows y >= num_tiles are
-// (sequence, partition) decode blocks (part z == 0 of each KV head), so a prefill or mixed step has
-// ONE attention launch (in a prefill-only step those blocks see no single-token sequence and exit)
+// dec_seqs > 0: the step's decode rows ride in the same launch — the last dec_seqs x partitions x KV heads blocks of the 1-D grid — so a
+// prefill or mixed step has ONE attention launch (in a prefill-only step those blocks see no single-token sequence and exit). A CU holds
+// one block at a time (215 VGPRs): with a block per (decode row, KV head, part of a tile) in a 2-D grid, three quarters of which only
+// exited, the rows waited for those (23 contexts of about 300 beside a prompt of 210 tokens 17.3 -> 12.7 us; the rows alone 9.7, the prompt
+// alone 12.5).
 template <int CT, int NW, int FL_NST, bool SWP>
-__global__ __launch_bounds__(64 * NW) void attn_flash_kernel(AttnArgs a, int lazy, int dec_seqs) {
+__global__ __launch_bounds__(64 * NW) void attn_flash_kernel(AttnArgs a, int lazy, int dec_seqs, int zs) {
   constexpr int P = (32 + NW - 1) / NW;  // DMA pieces per wave per chunk
   constexpr int FL_LDS = FL_NST * FL_STAGE;
   static_assert((FL_NST - 2) * P < 64, "vmcnt immediate");
@@ -185,16 +187,17 @@ __global__ __launch_bounds__(64 * NW) void attn_flash_kernel(AttnArgs a, int laz
   const int G = a.Hq / a.Hkv;
   const int QG = NW / G;
   const int QPB = 16 * CT * QG;
-  // grid (Hkv x halves, tiles): the KV heads (and a split range's two halves) of one tile are
+  // tiles x (Hkv x parts): the KV heads (and a split range's parts) of one tile are
   // adjacent in dispatch order, so the tile list's longest-first order holds across every head
-  const int zs = gridDim.x / a.Hkv;
-  const int h = blockIdx.x / zs;
-  const int tile = blockIdx.y;
-  if (tile >= a.num_tiles) {  // block-uniform: a decode block
-    const int r = tile - a.num_tiles;
-    if (blockIdx.x % zs == 0 && dec_seqs > 0) decode_block(a, r % dec_seqs, h, r / dec_seqs, smem);
+  const int per = a.Hkv * zs, tile_blocks = a.num_tiles * per;
+  if ((int)blockIdx.x >= tile_blocks) {  // block-uniform: a decode block (sequence fastest, partition slowest)
+    const int r = (int)blockIdx.x - tile_blocks;
+    decode_block(a, r % dec_seqs, (r / dec_seqs) % a.Hkv, r / (dec_seqs * a.Hkv), smem);
     return;
   }
+  const int tile = __builtin_amdgcn_readfirstlane((int)blockIdx.x / per);  // (a division is VALU work: its result is made scalar again)
+  const int x = (int)blockIdx.x - tile * per;
+  const int h = __builtin_amdgcn_readfirstlane(x / zs);
   const int s = a.tile_seq[tile];
   if (s < 0) return;
   const int q0 = a.tile_q0[tile];
@@ -215,7 +218,7 @@ __global__ __launch_bounds__(64 * NW) void attn_flash_kernel(AttnArgs a, int laz
   // min(zs, nch / 2) parts of whole chunks (>= 2 each), part z on [nch z / nsp, nch (z+1) / nsp),
   // met in the epilogue; the causal triangle's long tail then costs 1 / nsp of a range per block.
   // Parts past nsp exit at once. Block-uniform, before any barrier.
-  const int z = blockIdx.x % zs;
+  const int z = x - h * zs;
   const int nsp = SWP ? 1 : min(zs, nch / 2);
   const bool split = nsp > 1;
   if (z >= max(nsp, 1)) return;
@@ -642,16 +645,17 @@ void launch_attention(const AttnArgs& a, int dec_seqs, hipStream_t st) {
       const int qpb = 16 * fc.ct * (fc.nw / (a.Hq / a.Hkv));
       const size_t leaders = (size_t)tiles * 16 / qpb + (size_t)a.S + 1;
       const size_t slots = leaders * a.Hkv * fc.nw;
-      const size_t blocks = (size_t)tiles * 16 / qpb * a.Hkv;
+      const size_t work = (size_t)tiles * 16 / qpb * a.Hkv;
       const size_t cap = (size_t)cu_count() * (fc.ct == 2 ? 1 : 2);
-      if (blocks < 2 * cap) zs = 2;
-      if (blocks * 4 <= cap) zs = 4;
+      if (work < 2 * cap) zs = 2;
+      if (work * 4 <= cap) zs = 4;
       if (slots > 32768 || slots * zs * (fc.ct * 4 + 1) * 1024 > f.fl_ws_bytes) zs = 1;
     }
-    const dim3 grid(a.Hkv * zs, tiles + dec_rows, 1), block(64 * fc.nw);
-    f.tl = tl_take("attn_flash", (tiles + dec_rows) * a.Hkv * zs);
+    const int blocks = (dec_rows + tiles * zs) * a.Hkv;
+    const dim3 grid(blocks, 1, 1), block(64 * fc.nw);
+    f.tl = tl_take("attn_flash", blocks);
     const size_t lds_all = std::max(lds, (size_t)attn_lds_bytes(fc.nw));
-#define VG_FL(CT_, NW_) hipLaunchKernelGGL((attn_flash_kernel<CT_, NW_, 2, false>), grid, block, lds_all, st, f, lazy, dec_seqs)
+#define VG_FL(CT_, NW_) hipLaunchKernelGGL((attn_flash_kernel<CT_, NW_, 2, false>), grid, block, lds_all, st, f, lazy, dec_seqs, zs)
     if (fc.nw == 8) {
       if (fc.ct == 2) VG_FL(2, 8); else VG_FL(1, 8);
     } else {

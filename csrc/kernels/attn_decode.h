@@ -518,11 +518,12 @@ __device__ __forceinline__ void decode_block(const AttnArgs& a, int s, int h, in
     ATTN_STAMP(3);
     return;
   }
-  // partial (normalised o, running max M, sum L) by device-coherent stores
+  // partial (normalised o, running max M, sum L) by device-coherent stores, 16 B each (dword by dword, 8 of 1500 tokens 15.7 -> 14.5 us)
+  float* const heads_o = a.part_o + ((size_t)s * a.Hq + h * G) * a.num_parts * D_;  // (block-uniform)
   if (it < items) {
-    float* po = a.part_o + (((size_t)s * a.Hq + hq) * a.num_parts + part) * D_ + d0;
-    st_sc1_f4(po, acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
-    st_sc1_f4(po + 4, acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv);
+    const uint32_t po = (uint32_t)((icol * a.num_parts + part) * D_ + d0) * 4u;
+    st_sc1_x4(heads_o, po, f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
+    st_sc1_x4(heads_o, po + 16u, f32x4{acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv});
     if ((it & 15) == 0) {
       float* pm = a.part_ml + (((size_t)s * a.Hq + hq) * a.num_parts + part) * 2;
       st_sc1(pm, M);
@@ -546,20 +547,38 @@ __device__ __forceinline__ void decode_block(const AttnArgs& a, int s, int h, in
     for (int i = threadIdx.x; i < G * 32; i += blockDim.x)
       st_sc1_x4(reinterpret_cast<float*>(qs->gran), (row0 + (uint32_t)(h * G * D_ / 2) + 2u * (uint32_t)i) * 8u, z);
   }
-  // last arriver: merge the nparts partials of the G heads (one thread per (head, 4 d))
+  // last arriver: merge the nparts partials of the G heads (one thread per (head, 4 d)), four partitions' loads under way at a time
   for (int idx = threadIdx.x; idx < G * (D_ / 4); idx += blockDim.x) {
     const int hh = h * G + idx / (D_ / 4);
     const int dd = (idx % (D_ / 4)) * 4;
     const float* pm = a.part_ml + ((size_t)s * a.Hq + hh) * a.num_parts * 2;
-    const float* po = a.part_o + ((size_t)s * a.Hq + hh) * a.num_parts * D_ + dd;
-    float MM = -INFINITY;
-    for (int p = 0; p < nparts; ++p) MM = fmaxf(MM, ld_sc1(pm + 2 * p));
-    float LL = 0.f, r[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int p = 0; p < nparts; ++p) {
-      const float w = ld_sc1(pm + 2 * p + 1) * exp2f(ld_sc1(pm + 2 * p) - MM);
-      const f32x4 v = ld_sc1_f4(po + (size_t)p * D_);
-      LL += w;
-      r[0] += w * v[0]; r[1] += w * v[1]; r[2] += w * v[2]; r[3] += w * v[3];
+    const uint32_t po = (uint32_t)((idx / (D_ / 4)) * a.num_parts * D_ + dd) * 4u;
+    float MM = -INFINITY, LL = 0.f, r[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int p0 = 0; p0 < nparts; p0 += 4) {
+      f32x4 v[4];
+      float pmv[4], plv[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int p = min(p0 + u, nparts - 1);
+        v[u] = ld_sc1_x4(heads_o, po + (uint32_t)p * (D_ * 4u));
+        pmv[u] = ld_sc1(pm + 2 * p);
+        plv[u] = ld_sc1(pm + 2 * p + 1);
+      }
+      float mx = MM;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) mx = fmaxf(mx, pmv[u]);
+      const float mref = mx == -INFINITY ? 0.f : mx, keep = exp2f(MM - mref);
+      LL *= keep;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r[j] *= keep;
+      MM = mx;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float w = p0 + u < nparts ? plv[u] * exp2f(pmv[u] - mref) : 0.f;
+        LL += w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r[j] += w * v[u][j];
+      }
     }
     const float iv = LL > 0.f ? 1.f / LL : 0.f;
     uint2 pk;

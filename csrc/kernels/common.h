@@ -143,12 +143,6 @@ __device__ __forceinline__ void st_sc1(float* p, float v) {
 __device__ __forceinline__ float ld_sc1(const float* p) {
   return __uint_as_float(__hip_atomic_load(reinterpret_cast<const uint32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
-__device__ __forceinline__ void st_sc1_f4(float* p, float a, float b, float c, float d) {
-  st_sc1(p, a); st_sc1(p + 1, b); st_sc1(p + 2, c); st_sc1(p + 3, d);
-}
-__device__ __forceinline__ f32x4 ld_sc1_f4(const float* p) {
-  return f32x4{ld_sc1(p), ld_sc1(p + 1), ld_sc1(p + 2), ld_sc1(p + 3)};
-}
 // Bulk hand-off payloads: ONE 16-B write-through (sc1) vector store / sc1 load per lane through a
 // buffer descriptor (four dword sc1 stores of the same bytes are 3-20x slower to publish:
 // cdna_hip_programming.md Guideline 16, Pitfall 7). `base` must be wave-uniform (a kernel
