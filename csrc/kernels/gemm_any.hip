@@ -15,6 +15,7 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "lds_rows.h"
 #include "locate.h"
 #include "seq_launchers.h"
 
@@ -385,12 +386,127 @@ constexpr int LM = 128, LKS = 32, LPAD = LKS + 8;
 // at 2048 rows 13.4 -> 17.9 us). OUT_GATED: bf16 in whole pieces, times a gate. OUT_F32: fp32, 64 rows at a time through LDS, in whole lines
 // (1808 rows of 3072 x 96 19.5 -> 9.7 us, 1801 of 1024 x 128 16.7 -> 6.8 against a store per value).
 enum { OUT_PLAIN = 0, OUT_GATED = 1, OUT_F32 = 2 };
+constexpr int LDS_TILE_BYTES = 4 * LM * LPAD * 2;   // operand buffers of gemm_any_lds_kernel, the least that lds_store() may use
+// The outputs of a 128-row block tile from the waves' accumulators, by way of LDS that nobody reads or writes any more
+template <int DUAL, int OUT>
+__device__ __forceinline__ void lds_store(const AnyGemmArgs& p, const f32x4 (&acc)[4][4], bf16_t* smem, int64_t b, int r0, int rend, int n0) {
+  constexpr int WN = DUAL ? 64 : 128;  // columns of each weight matrix per block
+  constexpr int OPAD = WN + 8;         // padded row of the staged outputs
+  static_assert(LM * OPAD * 2 <= LDS_TILE_BYTES, "the staged outputs fit the operand buffers");
+  const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6;
+  const int wm = wv & 1, wn = wv >> 1, lr = l & 15, lg = l >> 4;
+  if constexpr (OUT == OUT_F32) {
+    constexpr int FP = 128 + 4;
+    static_assert(!DUAL && 64 * FP * 4 <= LDS_TILE_BYTES, "64 rows fit the operand buffers");
+    float* fs = reinterpret_cast<float*>(smem);
+    float* out = reinterpret_cast<float*>(p.out) + b * p.o_bs;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      if (wm == half)
+        with_act<DUAL>(p, [&](auto act) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int col = wn * 64 + j * 16 + lr;
+            const float bias = p.bias ? p.bias[min(n0 + col, p.N - 1)] : 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) fs[(i * 16 + 4 * lg + e) * FP + col] = act_val<decltype(act)::value>(p, acc[i][j][e] + bias, 0.f);
+          }
+        });
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < 64 * 32 / 256; ++u) {
+        const int x = tid + 256 * u, row = x >> 5, col = (x & 31) * 4, m = r0 + 64 * half + row;
+        if (m < rend && n0 + col < p.N) *reinterpret_cast<f32x4*>(out + (int64_t)m * p.ldo + n0 + col) = *reinterpret_cast<const f32x4*>(&fs[row * FP + col]);
+      }
+      if (half == 0) __syncthreads();
+    }
+    return;
+  }
+  if (OUT == OUT_GATED || p.vec_out) {  // bf16 rows of whole 16-B pieces: staged in LDS, then stored whole
+    // a gate: one logit per row, or its tile brought in whole pieces to where the outputs will lie, each lane's to its own
+    const bool tiled = OUT == OUT_GATED && p.g_cs != 0, rowed = OUT == OUT_GATED && p.g_cs == 0;
+    float rg[4][4];
+    if (rowed) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int64_t at = (int64_t)min(r0 + wm * 64 + i * 16 + 4 * lg + e, rend - 1) * p.ldg + b * p.g_bs;
+          rg[i][e] = sigmoidf_(p.gate_f32 ? reinterpret_cast<const float*>(p.gate)[at] : bf2f(reinterpret_cast<const bf16_t*>(p.gate)[at]));
+        }
+    } else if (tiled) {
+      const bf16_t* gate = reinterpret_cast<const bf16_t*>(p.gate) + b * p.g_bs;
+#pragma unroll
+      for (int u = 0; u < LM * WN / 8 / 256; ++u) {
+        const int x = tid + 256 * u, row = x / (WN / 8), col = (x % (WN / 8)) * 8;
+        if (n0 + col < p.N) *reinterpret_cast<uint4*>(&smem[row * OPAD + col]) = ld16(gate + (int64_t)min(r0 + row, rend - 1) * p.ldg + n0 + col);
+      }
+      __syncthreads();
+    }
+    with_act<DUAL>(p, [&](auto act) {
+#pragma unroll
+      for (int j = 0; j < (DUAL ? 2 : 4); ++j) {
+        const int col = (DUAL ? wn * 32 : wn * 64) + j * 16 + lr;
+        const float bias = p.bias ? p.bias[min(n0 + col, p.N - 1)] : 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            bf16_t* at = &smem[(wm * 64 + i * 16 + 4 * lg + e) * OPAD + col];
+            float v = act_val<decltype(act)::value>(p, acc[i][j][e] + bias, DUAL ? acc[i][j + 2][e] : 0.f);
+            if (rowed) v *= rg[i][e];
+            if (tiled) v *= sigmoidf_(bf2f(*at));
+            *at = f2bf(v);
+          }
+      }
+    });
+    __syncthreads();
+    bf16_t* out = reinterpret_cast<bf16_t*>(p.out) + b * p.o_bs;
+#pragma unroll
+    for (int u = 0; u < LM * WN / 8 / 256; ++u) {
+      const int x = tid + 256 * u, row = x / (WN / 8), col = (x % (WN / 8)) * 8;
+      if (r0 + row < rend && n0 + col < p.N)
+        *reinterpret_cast<uint4*>(out + (int64_t)(r0 + row) * p.ldo + n0 + col) =
+            *reinterpret_cast<const uint4*>(&smem[row * OPAD + col]);
+    }
+    return;
+  }
+  with_act<DUAL>(p, [&](auto act) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < (DUAL ? 2 : 4); ++j) {
+        const int n = n0 + (DUAL ? wn * 32 : wn * 64) + j * 16 + lr, m = r0 + wm * 64 + i * 16 + 4 * lg;
+        if (n >= p.N) continue;
+        const float bias = p.bias ? p.bias[n] : 0.f;
+        float gl[4];   // (asked for together)
+        if (p.gate != nullptr) {
+          const int64_t gc = b * p.g_bs + (int64_t)n * p.g_cs;
+          if (p.gate_f32) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) gl[e] = reinterpret_cast<const float*>(p.gate)[(int64_t)min(m + e, rend - 1) * p.ldg + gc];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) gl[e] = bf2f(reinterpret_cast<const bf16_t*>(p.gate)[(int64_t)min(m + e, rend - 1) * p.ldg + gc]);
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (m + e >= rend) continue;
+          float v = act_val<decltype(act)::value>(p, acc[i][j][e] + bias, DUAL ? acc[i][j + 2][e] : 0.f);
+          if (p.gate != nullptr) v *= sigmoidf_(gl[e]);
+          store_value(p, (int64_t)(m + e) * p.ldo + b * p.o_bs + n, v);
+        }
+      }
+  });
+}
+
 template <int DUAL, int AHEAD, int OUT>
 __global__ __launch_bounds__(256, 3) void gemm_any_lds_kernel(AnyGemmArgs p) {
   constexpr int WN = DUAL ? 64 : 128;  // columns of each weight matrix per block
-  constexpr int OPAD = WN + 8;         // padded row of the staged outputs
   __shared__ __attribute__((aligned(16))) bf16_t smem[4 * LM * LPAD];  // two A and two weight buffers, then the outputs
-  static_assert(LM * OPAD <= 4 * LM * LPAD, "the staged outputs fit the operand buffers");
   typedef bf16_t Tile[LM][LPAD];
   Tile* As = reinterpret_cast<Tile*>(smem);
   Tile* Ws = As + 2;
@@ -492,112 +608,112 @@ __global__ __launch_bounds__(256, 3) void gemm_any_lds_kernel(AnyGemmArgs p) {
       buf ^= 1;
     }
   }
-  if constexpr (OUT == OUT_F32) {   // (the k loop's last barrier has freed the buffers)
-    constexpr int FP = 128 + 4;
-    static_assert(!DUAL && 64 * FP * 4 <= (int)sizeof(smem), "64 rows fit the operand buffers");
-    float* fs = reinterpret_cast<float*>(smem);
-    float* out = reinterpret_cast<float*>(p.out) + b * p.o_bs;
+  lds_store<DUAL, OUT>(p, acc, smem, b, r0, rend, n0);
+}
+
+// The same block tile from operands brought by LDS-DMA, for K of whole 64-k stages: both matrices are rows of k, so both lie in LDS as x does
+// in the prompt GEMMs (lds_rows.h), and the loop is theirs (gemm_prompt.h): fragments of a k-step read during the MFMAs of the one before,
+// one barrier per stage between its two k-steps, accumulators in AGPRs. By way of registers a thread brought 64 B of a row at a time, which
+// keeps the CU's address path busy four times as long as whole 128-B lines.
+template <int DUAL, int NS, int OUT>
+__global__ __launch_bounds__(256, NS == 2 ? 2 : 1) void gemm_any_dma_kernel(AnyGemmArgs p) {
+  constexpr int WN = DUAL ? 64 : 128, STAGE = 32 * 1024, PPW = 8, AB = 16 * 1024;  // W tiles, then A tiles (16 rows x 64 k: 2 KiB each)
+  extern __shared__ __attribute__((aligned(16))) char dsm[];
+  int grp, r0, rend;
+  if (!locate_tile(p, blockIdx.y, grp, r0, rend, LM)) return;
+  const int64_t b = blockIdx.z;
+  const int64_t wsel = (p.group_off != nullptr) ? grp : b;
+  const int n0 = blockIdx.x * WN;
+  const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wv & 1, wn = wv >> 1;
+  const bf16_t* A = reinterpret_cast<const bf16_t*>(p.a) + b * p.a_bs;
+  const bf16_t* W = reinterpret_cast<const bf16_t*>(p.w) + wsel * p.w_bs;
+  const bf16_t* W2 = DUAL ? reinterpret_cast<const bf16_t*>(p.w2) + wsel * p.w_bs : nullptr;
+  const int nk = p.K >> 6;
+  const bf16_t* src[PPW];   // pieces of this wave: two tiles of W, two of A, two halves each
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      if (wm == half)
-        with_act<DUAL>(p, [&](auto act) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int col = wn * 64 + j * 16 + lr;
-            const float bias = p.bias ? p.bias[min(n0 + col, p.N - 1)] : 0.f;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) fs[(i * 16 + 4 * lg + e) * FP + col] = act_val<decltype(act)::value>(p, acc[i][j][e] + bias, 0.f);
-          }
-        });
-      __syncthreads();
-#pragma unroll
-      for (int u = 0; u < 64 * 32 / 256; ++u) {
-        const int x = tid + 256 * u, row = x >> 5, col = (x & 31) * 4, m = r0 + 64 * half + row;
-        if (m < rend && n0 + col < p.N) *reinterpret_cast<f32x4*>(out + (int64_t)m * p.ldo + n0 + col) = *reinterpret_cast<const f32x4*>(&fs[row * FP + col]);
-      }
-      if (half == 0) __syncthreads();
-    }
-    return;
+  for (int i = 0; i < 4; ++i) {
+    const int tile = 2 * wv + (i >> 1), row = tile * 16 + 8 * (i & 1) + (l >> 3), col = x_piece_col(i & 1, l);
+    const int n = min(n0 + (DUAL ? (row & 63) : row), p.N - 1);
+    src[i] = ((DUAL && row >= 64) ? W2 : W) + (int64_t)n * p.ldw + col;
+    const int m = r0 + row < rend ? r0 + row : r0;
+    src[4 + i] = A + (int64_t)(p.a_rows ? p.a_rows[m] : m) * p.lda + col;
   }
-  if (OUT == OUT_GATED || p.vec_out) {  // bf16 rows of whole 16-B pieces: staged in LDS (the k loop's last barrier has freed it), then stored whole
-    // a gate: one logit per row, or its tile brought in whole pieces to where the outputs will lie, each lane's to its own
-    const bool tiled = OUT == OUT_GATED && p.g_cs != 0, rowed = OUT == OUT_GATED && p.g_cs == 0;
-    float rg[4][4];
-    if (rowed) {
+  const uint32_t lds0 = lds_addr_of(dsm) + (uint32_t)wv * 4096u;
+  auto issue = [&](int i, int st, int buf) {
+    glds16(src[i] + (size_t)st * 64, lds0 + (uint32_t)(buf * STAGE + (i >> 2) * AB + (i & 3) * 1024));
+  };
+  f32x4 acc[4][4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int64_t at = (int64_t)min(r0 + wm * 64 + i * 16 + 4 * lg + e, rend - 1) * p.ldg + b * p.g_bs;
-          rg[i][e] = sigmoidf_(p.gate_f32 ? reinterpret_cast<const float*>(p.gate)[at] : bf2f(reinterpret_cast<const bf16_t*>(p.gate)[at]));
-        }
-    } else if (tiled) {
-      const bf16_t* gate = reinterpret_cast<const bf16_t*>(p.gate) + b * p.g_bs;
-#pragma unroll
-      for (int u = 0; u < LM * WN / 8 / 256; ++u) {
-        const int x = tid + 256 * u, row = x / (WN / 8), col = (x % (WN / 8)) * 8;
-        if (n0 + col < p.N) *reinterpret_cast<uint4*>(&smem[row * OPAD + col]) = ld16(gate + (int64_t)min(r0 + row, rend - 1) * p.ldg + n0 + col);
-      }
-      __syncthreads();
+    for (int j = 0; j < 4; ++j) {
+      acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      asm volatile("" : "+a"(acc[i][j]));  // (written here, well before the first mfma_acc)
     }
-    with_act<DUAL>(p, [&](auto act) {
-#pragma unroll
-      for (int j = 0; j < (DUAL ? 2 : 4); ++j) {
-        const int col = (DUAL ? wn * 32 : wn * 64) + j * 16 + lr;
-        const float bias = p.bias ? p.bias[min(n0 + col, p.N - 1)] : 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            bf16_t* at = &smem[(wm * 64 + i * 16 + 4 * lg + e) * OPAD + col];
-            float v = act_val<decltype(act)::value>(p, acc[i][j][e] + bias, DUAL ? acc[i][j + 2][e] : 0.f);
-            if (rowed) v *= rg[i][e];
-            if (tiled) v *= sigmoidf_(bf2f(*at));
-            *at = f2bf(v);
-          }
-      }
-    });
-    __syncthreads();
-    bf16_t* out = reinterpret_cast<bf16_t*>(p.out) + b * p.o_bs;
-#pragma unroll
-    for (int u = 0; u < LM * WN / 8 / 256; ++u) {
-      const int x = tid + 256 * u, row = x / (WN / 8), col = (x % (WN / 8)) * 8;
-      if (r0 + row < rend && n0 + col < p.N)
-        *reinterpret_cast<uint4*>(out + (int64_t)(r0 + row) * p.ldo + n0 + col) =
-            *reinterpret_cast<const uint4*>(&smem[row * OPAD + col]);
+  uint4 af[2][4], wf[2][4];
+  const int xo[2] = {x_frag_off(0, l), x_frag_off(1, l)};
+  // fragment read rd, in the order in which a phase needs them: A tile 0, W tiles, the other A tiles
+  auto read_frag = [&](int rd, int ks, const char* sb) {
+    if (rd == 0 || rd > 4) {
+      const int i = rd == 0 ? 0 : rd - 4;
+      af[ks][i] = *reinterpret_cast<const uint4*>(sb + AB + (wm * 4 + i) * 2048 + xo[ks]);
+    } else {
+      const int j = rd - 1;
+      wf[ks][j] = *reinterpret_cast<const uint4*>(sb + (DUAL ? (j >> 1) * 4 + wn * 2 + (j & 1) : wn * 4 + j) * 2048 + xo[ks]);
     }
-    return;
+  };
+  // the MFMAs of k-step ks, between them the reads of the other k-step (from sb) and, if `dma`, the pieces of stage st
+  auto phase = [&](auto ksc, const char* sb, auto dmac, int st, int buf) {
+    constexpr int ks = decltype(ksc)::value, dma = decltype(dmac)::value;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (i < 2) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) read_frag(4 * i + u, ks ^ 1, sb);
+      }
+      if constexpr (dma) {
+        issue(2 * i, st, buf);
+        issue(2 * i + 1, st, buf);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) mfma_acc(acc[i][j], af[ks][i], wf[ks][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  using C0 = std::integral_constant<int, 0>;
+  using C1 = std::integral_constant<int, 1>;
+#pragma unroll
+  for (int s0 = 0; s0 < NS; ++s0)
+#pragma unroll
+    for (int i = 0; i < PPW; ++i) issue(i, s0 < nk ? s0 : nk - 1, s0);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * PPW) : "memory");
+#pragma unroll
+  for (int rd = 0; rd < 8; ++rd) read_frag(rd, 0, dsm);
+  int buf = 0;
+  for (int t = 0; t < nk; ++t) {
+    const char* sb = dsm + buf * STAGE;
+    const int nb = buf + 1 == NS ? 0 : buf + 1;
+    phase(C0{}, sb, C0{}, 0, 0);
+    // this stage is read (its second k-step is in registers), the next one has landed: both for every wave
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * PPW) : "memory");
+    phase(C1{}, dsm + nb * STAGE, C1{}, t + NS < nk ? t + NS : nk - 1, buf);   // past the end: clamped duplicates, never used
+    buf = nb;
   }
-  with_act<DUAL>(p, [&](auto act) {
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15\n\ts_barrier" ::: "memory");  // the trailing duplicates, of every wave
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < (DUAL ? 2 : 4); ++j) {
-        const int n = n0 + (DUAL ? wn * 32 : wn * 64) + j * 16 + lr, m = r0 + wm * 64 + i * 16 + 4 * lg;
-        if (n >= p.N) continue;
-        const float bias = p.bias ? p.bias[n] : 0.f;
-        float gl[4];   // (asked for together)
-        if (p.gate != nullptr) {
-          const int64_t gc = b * p.g_bs + (int64_t)n * p.g_cs;
-          if (p.gate_f32) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) gl[e] = reinterpret_cast<const float*>(p.gate)[(int64_t)min(m + e, rend - 1) * p.ldg + gc];
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) gl[e] = bf2f(reinterpret_cast<const bf16_t*>(p.gate)[(int64_t)min(m + e, rend - 1) * p.ldg + gc]);
-          }
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (m + e >= rend) continue;
-          float v = act_val<decltype(act)::value>(p, acc[i][j][e] + bias, DUAL ? acc[i][j + 2][e] : 0.f);
-          if (p.gate != nullptr) v *= sigmoidf_(gl[e]);
-          store_value(p, (int64_t)(m + e) * p.ldo + b * p.o_bs + n, v);
-        }
-      }
-  });
+    for (int j = 0; j < 4; ++j) asm volatile("" : "+a"(acc[i][j]));
+  lds_store<DUAL, OUT>(p, acc, reinterpret_cast<bf16_t*>(dsm), b, r0, rend, n0);
+}
+
+template <int DUAL, int NS, int OUT>
+void launch_any_dma(const AnyGemmArgs& p, dim3 grid, hipStream_t st) {
+  auto kern = gemm_any_dma_kernel<DUAL, NS, OUT>;
+  static bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, NS * 32 * 1024) == hipSuccess;
+  (void)attr;
+  hipLaunchKernelGGL(kern, grid, dim3(256), NS * 32 * 1024, st, p);
 }
 
 template <typename T>
@@ -752,6 +868,26 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st) {
       const bool one = !dual && g.K <= 256 && (int64_t)grid2.x * grid2.y * grid2.z > 512;
       const bool gated = vec && g.gate != nullptr;
       const bool f32 = g.out_f32 && !dual && g.gate == nullptr && g.N % 4 == 0 && g.ldo % 4 == 0 && g.o_bs % 4 == 0 && a16(g.out);
+      // By LDS-DMA from four stages of k on (us, through registers -> by DMA: K = 64 of 3072 columns 9.5, 9.6; 12 products of 512 x 128 at 2048 rows
+      // 12.9, 15.2, 16 of them 15.4, 18.8; 4096 x 256 at 1024 8.6 -> 8.3, 12 of 128 x 512 11.2, 11.3; 8 of 512 x 512 at 4096 33.0 -> 30.9): two stages
+      // in LDS and two workgroups to a CU, or four stages where there is one at most (two / four: 1024 x 4096 at 2048 rows, 128 workgroups, 47.6
+      // -> 43.3 / 33.6; 8 experts of 1024 x 2048 with 150 rows each, 144, 28.5 -> 25.7 / 21.6, with 500, 320, 45.8 -> 33.2 / 42.2; pairs of 2048 x
+      // 1024 with 500, 64.8 -> 61.6 / 73.6). What bounds the many then is the operands' way through L2, 25 B a clock and CU.
+      if (g.K % 64 == 0 && g.K >= 256) {
+        const bool few = (int64_t)grid2.x * grid2.y * grid2.z <= 256;
+        auto by_dma = [&](auto du, auto out) {
+          constexpr int DU = decltype(du)::value, O = decltype(out)::value;
+          if (few) launch_any_dma<DU, 4, O>(v, grid2, st);
+          else launch_any_dma<DU, 2, O>(v, grid2, st);
+        };
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        if (dual) by_dma(I1{}, std::integral_constant<int, OUT_PLAIN>{});
+        else if (gated) by_dma(I0{}, std::integral_constant<int, OUT_GATED>{});
+        else if (f32) by_dma(I0{}, std::integral_constant<int, OUT_F32>{});
+        else by_dma(I0{}, std::integral_constant<int, OUT_PLAIN>{});
+        return;
+      }
       auto kern = dual ? gemm_any_lds_kernel<1, 2, OUT_PLAIN>
                        : (gated ? gemm_any_lds_kernel<0, 2, OUT_GATED>
                                 : (f32 ? gemm_any_lds_kernel<0, 2, OUT_F32>

@@ -138,3 +138,26 @@ def test_many_workgroups_and_short_k(M, K):
     out = torch.full((M, B, N), float("nan"), device="cuda", dtype=torch.bfloat16).transpose(0, 1)
     seq.gemm(a, w, out)
     _close(out, torch.matmul(a.float(), w.float().transpose(1, 2).contiguous()), K)
+
+
+@pytest.mark.parametrize("out", ["bf16", "odd", "gate", "row", "fp32"])
+@pytest.mark.parametrize("M,N,K", [(1025, 640, 256), (1153, 520, 320), (4100, 1160, 256), (4224, 1032, 576)])
+def test_stages_by_dma(M, N, K, out):
+    """128-row tiles whose operands come by LDS-DMA, four stages (few tiles) and two (many): rows and columns past the last whole tile,
+    strided operands, as few k stages as there are buffers and more, every way to store; what lies beside the outputs stays."""
+    g = torch.Generator("cuda").manual_seed(M + N)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    N -= 3 if out == "odd" else 0
+    a, w, bias = rand(M, K + 8).bfloat16()[:, :K], (rand(N, K) * K ** -0.5).bfloat16(), rand(N)
+    gate = rand(M, N).bfloat16() if out == "gate" else (rand(M, 1).bfloat16().expand(M, N) if out == "row" else None)
+    whole = torch.full((M + 1, N + 8), 7.0, device="cuda", dtype=torch.float32 if out == "fp32" else torch.bfloat16)
+    seq.gemm(a, w, whole[:M, :N], bias=bias, gate=gate)
+    want = a.float() @ w.float().t() + bias
+    _close(whole[:M, :N], want if gate is None else want * torch.sigmoid(gate.float()), K)
+    assert bool((whole[M] == 7).all() and (whole[:, N:] == 7).all())
+
+
+@pytest.mark.parametrize("sizes", [[300, 0, 129, 1, 600], [128] * 9 + [127, 0, 2], [700] * 6])
+@pytest.mark.parametrize("N,K", [(520, 256), (1024, 320)])
+def test_experts_by_dma(N, K, sizes):
+    test_experts(N, K, sizes)
