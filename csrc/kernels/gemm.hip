@@ -136,7 +136,7 @@ static GemmParams to_params(const GemmArgs& g) {
   if (g.act != 0) set_glu(p, GluAct{g.act, g.limit, g.alpha});
   p.scales = g.scales; p.zeros = g.zeros; p.group = g.group; p.szp = g.awq_szp;
   p.dbg_ts = g.dbg_ts;
-  p.hg = g.hg; p.hg_gamma = g.hg_gamma; p.ssp_out = g.ssp_out; p.ssp_in = g.ssp_in; p.ssn = g.ssn;
+  p.hg = g.hg; p.hg_gamma = g.hg_gamma; p.ssp_out = g.ssp_out; p.ssp_in = g.ssp_in; p.ssn = g.ssn; p.ss8 = g.ss8;
   p.ar = ArFused{};
   if (g.ar_world > 0) {
     for (int r = 0; r < 8; ++r) p.ar.base[r] = g.ar_fused[r];
@@ -188,6 +188,7 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
     if (h.waves != 0 && launch_gemm_mid(h, st)) return;
   }
   // decode rows on the register-stationary kernel (path 4: a decode plan / forced; gemm_kx_bf16.hip)
+  if (g.path == 0 && g.waves == 0 && g.splitk == 0 && g.ntb == 0 && launch_kx_half(g, st)) return;
   if (g.path == 4) {
     GemmArgs h = g;
     if (h.ntb > -12 || h.ntb < -14) h.ntb = 0;

@@ -271,7 +271,7 @@ bool launch_awq_mid(const GemmArgs& g, hipStream_t st) {
   p.k_cache = g.k_cache; p.v_cache = g.v_cache; p.hq = g.hq; p.hkv = g.hkv; p.bs = g.bs;
   p.szp = g.awq_szp; p.group = g.group;
   p.dbg_ts = g.dbg_ts;
-  p.hg = g.hg; p.hg_gamma = g.hg_gamma; p.ssp_out = g.ssp_out; p.ssp_in = g.ssp_in; p.ssn = g.ssn;
+  p.hg = g.hg; p.hg_gamma = g.hg_gamma; p.ssp_out = g.ssp_out; p.ssp_in = g.ssp_in; p.ssn = g.ssn; p.ss8 = g.ss8;
   const bool gam = g.norm_w != nullptr, pre = g.ssp_in != nullptr;
 #define VG_AMD(E)                                                                  \
   return gam ? launch_awq_mid_epi<E, 1>(p, g.waves, g.splitk, g.slab_bytes, st)    \

@@ -44,6 +44,7 @@ struct GemmParams {  // (no longer than need be: with 12 bytes more a step's sho
   // applied; int4) or x = h with gamma folded into the bf16 weights (hg null), row scale
   // rsqrt(sum of ssp_in[m][0..ssn) / K + eps) — no gamma loads, no x^2 pass.
   bf16_t* hg; const bf16_t* hg_gamma; float* ssp_out; const float* ssp_in; int ssn;
+  int ss8;  // M <= 8: ssp_out / ssp_in hold sums of 8 columns, [M][N / 8], [M][ssn = K / 8] (the half tiles of gemm_kx.h own 8 columns each)
   unsigned long long* dbg_ts;  // per-block [start, end] realtime stamps (profiling), or null
   ArFused ar;                  // world 0: no fused all-reduce
   uint4* qa_gran;              // EPI_QKV: also write q / K / V as tagged granules (qkv_attn.hip), or null
@@ -243,8 +244,12 @@ __device__ __forceinline__ void epilogue_norm_out(const GemmParams& p, const f32
       for (int i = 0; i < 4; ++i) s2 += h4[i] * h4[i];
     }
     s2 += xor16(s2);
-    s2 += xor32(s2);
-    if (valid && nsub == 0) p.ssp_out[(size_t)m * (p.N >> 4) + nt0 + j] = s2;
+    if (p.ss8) {
+      if (valid && (nsub & 4) == 0) p.ssp_out[(size_t)m * (p.N >> 3) + 2 * (nt0 + j) + (nsub >> 3)] = s2;
+    } else {
+      s2 += xor32(s2);
+      if (valid && nsub == 0) p.ssp_out[(size_t)m * (p.N >> 4) + nt0 + j] = s2;
+    }
   }
 }
 
@@ -296,10 +301,13 @@ struct SsPre {
   int n4;  // 0: prenorm_ss after the stream (ssn not in the prefetch form)
 };
 __device__ __forceinline__ int ss_pre_n4(const GemmParams& p) {
+  if (p.ss8) return (p.ssn & 31) == 0 && p.ssn <= 32 * SS_PRE ? p.ssn >> 5 : 0;
   return (p.ssn & 15) == 0 && p.ssn <= 16 * SS_PRE ? p.ssn >> 4 : 0;
 }
+// (sums of 8 columns: the lanes of rows 8 .. 15, which M <= 8 has no use for, read the second half of a quarter of rows 0 .. 7)
 __device__ __forceinline__ void ss_pre_issue(const GemmParams& p, SsPre& s, int m, int quarter) {
-  const f32x4* src = reinterpret_cast<const f32x4*>(p.ssp_in + (size_t)min(m, p.M - 1) * p.ssn + quarter * (p.ssn >> 2));
+  const int row = p.ss8 ? m & 7 : m, part = p.ss8 ? 2 * quarter + (m >> 3) : quarter;
+  const f32x4* src = reinterpret_cast<const f32x4*>(p.ssp_in + (size_t)min(row, p.M - 1) * p.ssn + part * (4 * s.n4));
 #pragma unroll
   for (int u = 0; u < SS_PRE; ++u) s.r[u] = src[min(u, s.n4 - 1)];
 }
@@ -315,6 +323,7 @@ __device__ __forceinline__ float ss_pre_sum(const GemmParams& p, const SsPre& s,
     asm volatile("" : "+v"(r));
     if (u < s.n4) acc += (r[0] + r[1]) + (r[2] + r[3]);
   }
+  if (p.ss8) acc += __shfl_xor(acc, 8, 64);
   return acc;
 }
 

@@ -22,7 +22,7 @@
 //   X = the k-quad's activation sum per row (v_dot2 with (1, 1) over the B fragments).
 //   bf16(128 + v) = (nibbles & 0x000F000F) | 0x43004300: one v_and_or_b32 per 2 values (+ a shift).
 //
-// Two grid forms:
+// Grid forms (and, for up to 8 rows, half tiles: kx_half_kernel):
 //   WIDE  (N >= one tile per CU, gate_up): one block per CU owning whole tiles [t0, t0 + ntb),
 //         ntb <= TMAX; the waves' partials meet in LDS and wave j finishes tile t0 + j.
 //   GROUP (narrow N: qkv, o_proj, down_proj): TMAX = 1, 2 or 4 adjacent tiles per block, gridDim.z
@@ -303,6 +303,60 @@ __global__ __launch_bounds__((kx_max_threads<Q4, XP, KQW, TMAX, NORM>())) void k
   kx_block<Q4, XP, KQW, TMAX, EPI, NORM, WIDE>(p);
 }
 
+// Half tiles for up to 8 rows: a 16 x 16 x 32 MFMA then has room for two k-steps of 8 columns side by side. Lanes r16 < 8 bring column r16 of
+// the block's half of the tile and row r16 of x, both of the even k-step, lanes r16 >= 8 the same of the odd one: the two products stand on the
+// diagonal of D, and lanes folded across it (l ^ 40) hold the sum. Rows of x come as an XP = 2 load has them, 128 B of each.
+// A block owns 8 columns over all of K: N / 16 tiles spread over twice as many CUs with no K slices that meet through memory, which
+// is what a short decode launch waits for (us, tile blocks -> half tiles: 1536 x 8960 at 1 row 9.1 -> 7.2, 1536 x 1536 4.5 -> 3.4).
+template <int KQW>
+__global__ __launch_bounds__(1024) void kx_half_kernel(GemmParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  TLScope tl_scope(p.dbg_ts);
+  const int lane = threadIdx.x & 63, r16 = lane & 15, grp = lane >> 4;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+  const int KQ = p.K >> 7, t0 = (int)blockIdx.x >> 1, h = (int)blockIdx.x & 1;
+  const int q0 = (KQ * wid) / nw, nq = (KQ * (wid + 1)) / nw - q0;  // 1 .. KQW (host)
+  EpiPre<1> pre;
+  if (wid == 0) epi_pre_a<1, EPI_BF16>(p, pre, r16, t0, 4 * grp);
+  const int r8 = r16 & 7, odd = r16 >> 3;
+  const bf16_t* xrow = p.x + (size_t)min(r8, p.M - 1) * p.lda + odd * 32 + 8 * grp;
+  const uint4* wrow = p.wp + ((size_t)t0 * KQ * 4 + odd) * 64 + grp * 16 + h * 8 + r8;
+  uint4 xa[KQW][2], w[KQW][2];
+#pragma unroll
+  for (int q = 0; q < KQW; ++q) {
+    const int kq = q0 + min(q, nq - 1);
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      xa[q][v] = *reinterpret_cast<const uint4*>(xrow + (size_t)(kq * 4 + 2 * v) * 32);
+      w[q][v] = ld_nt16(wrow + (size_t)(kq * 4 + 2 * v) * 64);
+    }
+  }
+  asm volatile("" ::: "memory");  // every load of the wave is in flight before the first MFMA
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < KQW; ++q) {
+    if (q >= nq) break;  // wave-uniform
+#pragma unroll
+    for (int v = 0; v < 2; ++v) acc = mfma16(as_bf16x8(w[q][v]), as_bf16x8(xa[q][v]), acc);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] += __shfl_xor(acc[i], 40, 64);
+  // 16 items per wave: row r8, 4 columns of the half
+  f32x4* red = reinterpret_cast<f32x4*>(smem);
+  if (r16 < 8 && grp < 2) red[wid * 16 + grp * 8 + r8] = acc;
+  __syncthreads();
+  if (wid != 0) return;
+  // the four lanes of an item sum every fourth wave's, then each other's: all of them hold it
+  f32x4 v[1] = {{0.f, 0.f, 0.f, 0.f}};
+  for (int w2 = 2 * (grp >> 1) + odd; w2 < nw; w2 += 4) v[0] += red[w2 * 16 + (grp & 1) * 8 + r8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[0][i] += __shfl_xor(v[0][i], 8, 64);
+    v[0][i] += __shfl_xor(v[0][i], 32, 64);
+  }
+  epilogue<1, EPI_BF16, true>(p, v, r16, t0, 4 * grp, pre, r16 < p.M && (grp >> 1) == h);
+}
+
 // The fused QKV projection + decode attention launch on this kernel (design: qkv_attn.hip): GROUP
 // one-tile blocks of <= 8 waves (z-major in the 1-D grid), then the attention blocks
 template <bool Q4, int XP, int KQW, int NORM>
@@ -466,7 +520,7 @@ static GemmParams kx_params(const GemmArgs& g) {
   p.k_cache = g.k_cache; p.v_cache = g.v_cache; p.hq = g.hq; p.hkv = g.hkv; p.bs = g.bs;
   p.szp = g.awq_szp; p.group = g.group;
   p.dbg_ts = g.dbg_ts;
-  p.hg = g.hg; p.hg_gamma = g.hg_gamma; p.ssp_out = g.ssp_out; p.ssp_in = g.ssp_in; p.ssn = g.ssn;
+  p.hg = g.hg; p.hg_gamma = g.hg_gamma; p.ssp_out = g.ssp_out; p.ssp_in = g.ssp_in; p.ssn = g.ssn; p.ss8 = g.ss8;
   return p;
 }
 

@@ -61,6 +61,7 @@ struct GemmArgs {
   float* ssp_out = nullptr;
   const float* ssp_in = nullptr;
   int ssn = 0;
+  int ss8 = 0;  // sums of 8 columns in ssp_out / ssp_in ([M][N / 8], [M][K / 8]; M <= 8)
   // stream-K decode kernel (path 3, gemm_streamk.hip): zeroed publisher-slot workspace and the
   // sticky fault word (bit 2: a partial poll gave up)
   void* sk_pub = nullptr;
@@ -93,6 +94,7 @@ bool launch_gemm_mid(const GemmArgs& g, hipStream_t st);
 // 1-4 tiles per block + K slices): AWQ W4A16 (group 128, packed scales) and bf16. False: shape / mode
 // not taken (the caller falls back on the other decode kernels).
 bool launch_awq_kx(const GemmArgs& g, hipStream_t st);
+bool launch_kx_half(const GemmArgs& g, hipStream_t st);  // half tiles, M <= 8 (gemm_kx_bf16.hip)
 bool launch_dense_kx(const GemmArgs& g, hipStream_t st);
 // AWQ W4A16 medium-M kernel (gemm_awq_mid.hip, 16 < M <= 64): g.waves tiles per block (8: one block
 // per CU owning whole tiles), g.splitk K slices; false for a shape / mode it does not take

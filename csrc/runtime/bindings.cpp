@@ -54,6 +54,11 @@ vgate::AttnArgs attn_common(const Tensor& q, int64_t q_stride, const Tensor& k_c
 // bytes of the fp32 slabs behind the counters of a workspace
 size_t slab_bytes_of(const Tensor& ws) { return ws.numel() > 65536 ? (size_t)(ws.numel() - 65536) * 4 : 0; }
 
+// sums of squares of 8 columns (steps of up to 8 rows) by their shape, of 16 otherwise
+static bool sums_of_8(const Tensor& t, int64_t M, int64_t N) {
+  return M <= 8 && N % 8 == 0 && t.dim() == 2 && t.size(1) == N / 8 && t.size(0) >= M && t.is_contiguous();
+}
+
 void gemm(const Tensor& x, const Tensor& wp, int64_t N, int64_t K, Tensor& out, int64_t epi,
           const c10::optional<Tensor>& bias, const c10::optional<Tensor>& res,
           const c10::optional<Tensor>& norm_w, double eps, const c10::optional<Tensor>& row_idx,
@@ -147,6 +152,7 @@ void gemm(const Tensor& x, const Tensor& wp, int64_t N, int64_t K, Tensor& out, 
     TORCH_CHECK(epi == 0 && M <= 16, "ssp_out: epi 0, M <= 16");
     CHECK_DEV(*ssp_out); CHECK_DT(*ssp_out, torch::kFloat32);
     TORCH_CHECK(ssp_out->numel() >= M * (N / 16), "ssp_out: [M][N/16]");
+    if (sums_of_8(*ssp_out, M, N)) g.ss8 = 1;
     g.ssp_out = reinterpret_cast<float*>(ssp_out->data_ptr());
     if (hg_out.has_value() && hg_out->defined()) {
       CHECK_DEV(*hg_out); CHECK_DT(*hg_out, torch::kBFloat16); CHECK_LASTDIM(*hg_out);
@@ -166,6 +172,11 @@ void gemm(const Tensor& x, const Tensor& wp, int64_t N, int64_t K, Tensor& out, 
                 "ssp_in: [M][K/16], 16-B aligned");
     g.ssp_in = reinterpret_cast<const float*>(ssp_in->data_ptr());
     g.ssn = (int)(K / 16);
+    if (sums_of_8(*ssp_in, M, K)) {
+      TORCH_CHECK(!g.ssp_out, "gemm: one of ssp_in, ssp_out");
+      g.ss8 = 1;
+      g.ssn = (int)(K / 8);
+    }
   }
   if (sk_ws.has_value() && sk_ws->defined()) {
     CHECK_DEV(*sk_ws); CHECK_DT(*sk_ws, torch::kInt32);

@@ -1,0 +1,57 @@
+"""Half tiles of the decode GEMMs (8 columns over all of K per workgroup, up to 8 rows) against fp32 products: rows, waves with fewer k-quads than
+others, strides, bias and residual, and the sums of squares of 8 columns that they hand to the next projection's norm."""
+import pytest
+import torch
+
+from vgate import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _rand(*s):
+    return torch.randn(*s, device="cuda")
+
+
+def _close(out, want, K):
+    # fp32 sums of K products of size ~ K^-1/2 in another order, rounded to bf16 before and after the residual
+    assert ((out.float() - want).abs() <= 2.0 ** -7 * want.abs() + 8.0 * K * 2.0 ** -24 + 2.0 ** -7).all()
+
+
+@pytest.mark.parametrize("M", [1, 2, 4, 5, 8])
+@pytest.mark.parametrize("N,K", [(16, 128), (48, 384), (512, 2176), (1536, 1536), (2048, 6144), (1024, 6272), (256, 10240), (2048, 8960)])
+def test_half_tiles(M, N, K):
+    torch.manual_seed(M + N + K)
+    w, bias = (_rand(N, K) * K ** -0.5).bfloat16(), _rand(N).bfloat16()
+    lin, lb = ops.Linear(w), ops.Linear(w, bias=bias)
+    x, res = _rand(M, K + 64).bfloat16()[:, 32:K + 32], _rand(M, N + 8).bfloat16()[:, :N]
+    want = x.float() @ w.float().t()
+    whole = torch.full((M + 1, N + 8), 7.0, device="cuda", dtype=torch.bfloat16)
+    ops.linear(x, lin, out=whole[:M, :N], residual=res)
+    _close(whole[:M, :N], want + res.float(), K)
+    assert bool((whole[M] == 7).all() and (whole[:, N:] == 7).all())
+    _close(ops.linear(x, lb), want + bias.float(), K)
+
+
+@pytest.mark.parametrize("M", [1, 3, 8])
+@pytest.mark.parametrize("N,K", [(256, 256), (1536, 1536), (1536, 8960), (2048, 10240)])
+def test_sums_of_8_columns(M, N, K):
+    """The residual projection stores the sums, three kinds of consumers take their row scale from them: the same as from the rows."""
+    torch.manual_seed(M + N + K)
+    assert ops.half_tiles(M, N)
+    lin = ops.Linear((_rand(N, K) * K ** -0.5).bfloat16())
+    x, h = _rand(M, K).bfloat16(), _rand(M, N).bfloat16()
+    plain, ssp = h.clone(), torch.full((M, N // 8), float("nan"), device="cuda")
+    ops.linear(x, lin, out=h, residual=h, norm_out=(None, ssp, None))
+    ops.linear(x, lin, out=plain, residual=plain)
+    assert torch.equal(h, plain) or not bool(((h.float() - plain.float()).abs() > 2.0 ** -6 * plain.float().abs() + 2.0 ** -7).any())
+    torch.testing.assert_close(ssp, h.float().pow(2).reshape(M, N // 8, 8).sum(-1), rtol=1e-5, atol=1e-4)
+    for rows, path in ((512, 0), (8192, 0), (8192, 4)):   # few tiles, many, whole tiles per CU
+        w, gamma = (_rand(rows, N) * N ** -0.5).bfloat16(), (torch.rand(N, device="cuda") + 0.5).bfloat16()
+        nx = ops.Linear(w.clone(), kind="silu")
+        assert nx.fold_norm(gamma)
+        nx.dec_path = path
+        got, want = ops.linear(h, nx, prenorm=(ssp, 1e-6)), ops.linear(h, nx, norm=(gamma, 1e-6))
+        assert ((got.float() - want.float()).abs() <= 2.0 ** -7 * want.float().abs() + 2.0 ** -9).all()
+        sums16 = ssp.reshape(M, N // 16, 2).sum(-1).contiguous()
+        old = ops.linear(h, nx, prenorm=(sums16, 1e-6))
+        assert ((got.float() - old.float()).abs() <= 2.0 ** -7 * old.float().abs() + 2.0 ** -9).all()

@@ -225,7 +225,8 @@ class DecoderModel:
         awq = self.quant == "awq"
         if hand:
             hg = torch.empty(T, a.hidden_size, dtype=torch.bfloat16, device=dev) if awq else None
-            ssp = torch.empty(T, a.hidden_size // 16, dtype=torch.float32, device=dev)
+            # (sums of 8 columns where the projections onto the hidden size run as half tiles: ops.half_tiles)
+            ssp = torch.empty(T, a.hidden_size // (8 if not awq and ops.half_tiles(T, a.hidden_size) else 16), dtype=torch.float32, device=dev)
         nl = len(self.layers)
 
         def takes(lin) -> bool:  # a consumer of the hand-off

@@ -282,6 +282,11 @@ def workspace(device) -> torch.Tensor:
     return ws
 
 
+def half_tiles(M: int, N: int) -> bool:
+    """Whether a bf16 projection of M rows onto N columns may run as half tiles, whose sums of squares (``norm_out``) cover 8 columns each."""
+    return M <= 8 and N % 256 == 0 and N <= 2048
+
+
 def linear(x: torch.Tensor, lin: Linear, out: torch.Tensor | None = None,
            residual: torch.Tensor | None = None, out_f32: bool = False, waves: int = 0, splitk: int = 0,
            norm: tuple | None = None, row_idx: torch.Tensor | None = None, qkv: dict | None = None,
