@@ -188,7 +188,7 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
     if (h.waves != 0 && launch_gemm_mid(h, st)) return;
   }
   // decode rows on the register-stationary kernel (path 4: a decode plan / forced; gemm_kx_bf16.hip)
-  if (g.path == 0 && g.waves == 0 && g.splitk == 0 && g.ntb == 0 && launch_kx_half(g, st)) return;
+  if (g.path == 0 && g.waves == 0 && g.splitk == 0 && g.ntb == 0 && (launch_kx_half(g, st) || (dense_kx_fits(g) && launch_dense_kx(g, st)))) return;
   if (g.path == 4) {
     GemmArgs h = g;
     if (h.ntb > -12 || h.ntb < -14) h.ntb = 0;

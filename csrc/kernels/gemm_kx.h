@@ -308,7 +308,7 @@ __global__ __launch_bounds__((kx_max_threads<Q4, XP, KQW, TMAX, NORM>())) void k
 // diagonal of D, and lanes folded across it (l ^ 40) hold the sum. Rows of x come as an XP = 2 load has them, 128 B of each.
 // A block owns 8 columns over all of K: N / 16 tiles spread over twice as many CUs with no K slices that meet through memory, which
 // is what a short decode launch waits for (us, tile blocks -> half tiles: 1536 x 8960 at 1 row 9.1 -> 7.2, 1536 x 1536 4.5 -> 3.4).
-template <int KQW>
+template <int KQW, int EPI>
 __global__ __launch_bounds__(1024) void kx_half_kernel(GemmParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   TLScope tl_scope(p.dbg_ts);
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(1024) void kx_half_kernel(GemmParams p) {
   const int KQ = p.K >> 7, t0 = (int)blockIdx.x >> 1, h = (int)blockIdx.x & 1;
   const int q0 = (KQ * wid) / nw, nq = (KQ * (wid + 1)) / nw - q0;  // 1 .. KQW (host)
   EpiPre<1> pre;
-  if (wid == 0) epi_pre_a<1, EPI_BF16>(p, pre, r16, t0, 4 * grp);
+  if (wid == 0) epi_pre_a<1, EPI>(p, pre, r16, t0, 4 * grp);
   const int r8 = r16 & 7, odd = r16 >> 3;
   const bf16_t* xrow = p.x + (size_t)min(r8, p.M - 1) * p.lda + odd * 32 + 8 * grp;
   const uint4* wrow = p.wp + ((size_t)t0 * KQ * 4 + odd) * 64 + grp * 16 + h * 8 + r8;
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(1024) void kx_half_kernel(GemmParams p) {
     v[0][i] += __shfl_xor(v[0][i], 8, 64);
     v[0][i] += __shfl_xor(v[0][i], 32, 64);
   }
-  epilogue<1, EPI_BF16, true>(p, v, r16, t0, 4 * grp, pre, r16 < p.M && (grp >> 1) == h);
+  epilogue<1, EPI, true>(p, v, r16, t0, 4 * grp, pre, r16 < p.M && (grp >> 1) == h);
 }
 
 // The fused QKV projection + decode attention launch on this kernel (design: qkv_attn.hip): GROUP
@@ -483,11 +483,16 @@ static bool kx_launch_xp(GemmParams p, const GemmArgs& g, hipStream_t st) {
     if (ntiles >= ncu && g.splitk <= 1 && g.ntb != -13 && g.ntb != -14) {
       const int nb = ncu, tneed = (ntiles + nb - 1) / nb;
       const int nw = g.waves > 0 ? g.waves : std::min(16, KQ);
-      if (nw > 16) return false;
+      if (nw > 16 || tneed > nw) return false;  // (wave j finishes tile t0 + j)
       const int kqw = (KQ + nw - 1) / nw;
       if (p.dbg_ts == nullptr) p.dbg_ts = tl_take(Q4 ? "awq_kx_wide" : "kx_wide", nb);
       p.splitk = 1;
       const dim3 grid(nb);
+      if constexpr (!Q4) {
+        if (tneed == 1 && kqw == 1) return kx_go<Q4, XP, 1, 1, EPI, NORM, true>(p, grid, nw, st);
+        if (tneed == 3 && kqw == 1) return kx_go<Q4, XP, 1, 3, EPI, NORM, true>(p, grid, nw, st);
+        if (tneed == 4 && kqw == 1) return kx_go<Q4, XP, 1, 4, EPI, NORM, true>(p, grid, nw, st);
+      }
       if (tneed <= 2 && kqw == 1) return kx_go<Q4, XP, 1, 2, EPI, NORM, true>(p, grid, nw, st);
       if (tneed <= 5 && kqw == 1) return kx_go<Q4, XP, 1, 5, EPI, NORM, true>(p, grid, nw, st);
       if (tneed <= 5 && kqw == 2) return kx_go<Q4, XP, 2, 5, EPI, NORM, true>(p, grid, nw, st);
@@ -518,6 +523,7 @@ static GemmParams kx_params(const GemmArgs& g) {
   p.gran = nullptr; p.fault = g.fault;
   p.positions = g.positions; p.slots = g.slots; p.cos_sin = g.cos_sin;
   p.k_cache = g.k_cache; p.v_cache = g.v_cache; p.hq = g.hq; p.hkv = g.hkv; p.bs = g.bs;
+  if (g.act != 0) set_glu(p, GluAct{g.act, g.limit, g.alpha});   // (in fields set above)
   p.szp = g.awq_szp; p.group = g.group;
   p.dbg_ts = g.dbg_ts;
   p.hg = g.hg; p.hg_gamma = g.hg_gamma; p.ssp_out = g.ssp_out; p.ssp_in = g.ssp_in; p.ssn = g.ssn; p.ss8 = g.ss8;

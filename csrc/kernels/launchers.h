@@ -96,6 +96,8 @@ bool launch_gemm_mid(const GemmArgs& g, hipStream_t st);
 bool launch_awq_kx(const GemmArgs& g, hipStream_t st);
 bool launch_kx_half(const GemmArgs& g, hipStream_t st);  // half tiles, M <= 8 (gemm_kx_bf16.hip)
 bool launch_dense_kx(const GemmArgs& g, hipStream_t st);
+bool dense_kx_fits(const GemmArgs& g);  // (the launcher's choice without a plan)
+bool launch_dense_kx_out(const GemmArgs& g, hipStream_t st);  // fp32 outputs and pair activations, no norm (gemm_kx_out.hip)
 // AWQ W4A16 medium-M kernel (gemm_awq_mid.hip, 16 < M <= 64): g.waves tiles per block (8: one block
 // per CU owning whole tiles), g.splitk K slices; false for a shape / mode it does not take
 bool launch_awq_mid(const GemmArgs& g, hipStream_t st);

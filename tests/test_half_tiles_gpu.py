@@ -55,3 +55,31 @@ def test_sums_of_8_columns(M, N, K):
         sums16 = ssp.reshape(M, N // 16, 2).sum(-1).contiguous()
         old = ops.linear(h, nx, prenorm=(sums16, 1e-6))
         assert ((got.float() - old.float()).abs() <= 2.0 ** -7 * old.float().abs() + 2.0 ** -9).all()
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(48, 128), (1024, 1280), (2064, 1024), (3072, 1536), (4096, 512), (4112, 1536), (8208, 2048), (12304, 512), (20480, 1408),
+                                 (1024, 4096), (512, 10240), (20496, 512), (28672, 512), (28672, 1024), (32784, 1024)])
+def test_register_stationary_choice(M, N, K):
+    """Shapes on the lines of the launcher's choice of the register-stationary kernel: one to eight whole tiles per CU, more tiles than waves to
+    finish them, one-tile blocks, K slices; both result types, pairs of either activation, a folded norm."""
+    torch.manual_seed(M + N + K)
+    w, x = (_rand(N, K) * K ** -0.5).bfloat16(), _rand(M, K).bfloat16()
+    lin, want = ops.Linear(w), x.float() @ w.float().t()
+    res = _rand(M, N).bfloat16()
+    _close(ops.linear(x, lin, residual=res), want + res.float(), K)
+    f32 = ops.linear(x, lin, out_f32=True)
+    assert ((f32 - want).abs() <= 8.0 * K * 2.0 ** -24 + 1e-6).all()
+    g, u = want[:, : N // 2], want[:, N // 2:]
+    _close(ops.linear(x, ops.Linear(w, kind="silu")), torch.nn.functional.silu(g) * u, 8 * K)
+    gelu = ops.Linear(w, kind="silu")
+    gelu.glu = (4, 0.0, 0.0)
+    _close(ops.linear(x, gelu), torch.nn.functional.gelu(g, approximate="tanh") * u, 8 * K)
+    gelu.glu = (2, 0.7, 1.702)
+    gc, uc = g.clamp(max=0.7), u.clamp(-0.7, 0.7)
+    _close(ops.linear(x, gelu), gc * torch.sigmoid(1.702 * gc) * (uc + 1), 8 * K)
+    nl, gamma = ops.Linear(w.clone(), kind="silu"), (torch.rand(K, device="cuda") + 0.5).bfloat16()
+    assert nl.fold_norm(gamma)
+    xn = x.float() * torch.rsqrt((x.float() ** 2).mean(-1, keepdim=True) + 1e-6)
+    y = xn @ (w.float() * gamma.float()).bfloat16().float().t()
+    _close(ops.linear(x, nl, norm=(gamma, 1e-6)), torch.nn.functional.silu(y[:, : N // 2]) * y[:, N // 2:], 8 * K)
