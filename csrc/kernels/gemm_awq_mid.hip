@@ -183,7 +183,7 @@ __global__ __launch_bounds__(512) void awq_mid_kernel(GemmParams p, int wide) { 
     const int m = mt * 16 + r16;
     f32x4 v[1] = {acc[mt]};
     if constexpr (NORM == 1) v[0] *= rsqrtf(ssr[mt] / (float)p.K + p.eps);
-    epilogue<1, EPI, false>(p, v, m, nt, nsub, EpiPre<1>{}, m < p.M);
+    epilogue<1, EPI, false, true>(p, v, m, nt, nsub, EpiPre<1>{}, m < p.M);
   }
 }
 

@@ -439,15 +439,16 @@ __device__ __forceinline__ void epilogue_ar(const GemmParams& p, const f32x4 (&v
 // `have` is a compile-time choice: a runtime select between a prefetched register value
 // and a load becomes a select of ADDRESSES that puts the prefetch struct in scratch.
 // `valid`: row m < M. Every lane of the wave calls in (the QKV pair exchange is a cross-lane
-// op); only valid rows store.
-template <int NTB, int EPI, bool have>
+// op); only valid rows store. HAND: the kernel may be given p.ssp_out (decode rows). Where it can't, as in the prompt kernels with one
+// epilogue per accumulator tile, that path was three quarters of a 64 KiB kernel.
+template <int NTB, int EPI, bool have, bool HAND = false>
 __device__ __forceinline__ void epilogue(const GemmParams& p, const f32x4 (&v)[NTB], int m, int nt0, int nsub,
                                          const EpiPre<NTB> e, bool valid) {
   if constexpr (EPI == EPI_BF16_AR) {  // every lane calls in: wave-wide arrival poll
     epilogue_ar<NTB, have>(p, v, m, nt0, nsub, e, valid);
     return;
   }
-  if constexpr (EPI == EPI_BF16) {
+  if constexpr (EPI == EPI_BF16 && HAND) {
     if (p.ssp_out != nullptr) {  // every lane calls in: the tile's sum of squares is a cross-lane fold
       epilogue_norm_out<NTB, have>(p, v, m, nt0, nsub, e, valid);
       return;
@@ -691,7 +692,7 @@ __device__ __forceinline__ void gemm_finish(const GemmParams& p, f32x4 (&acc)[MB
 #pragma unroll
         for (int j = 0; j < NTB; ++j) v[j] *= sc;
       }
-      epilogue<NTB, EPI, PRE>(p, v, m_base + (l & 15), nt0, 4 * (l >> 4), pre, m_base + (l & 15) < p.M);
+      epilogue<NTB, EPI, PRE, MB == 1>(p, v, m_base + (l & 15), nt0, 4 * (l >> 4), pre, m_base + (l & 15) < p.M);
       return;
     }
   }
@@ -768,7 +769,7 @@ __device__ __forceinline__ void gemm_finish(const GemmParams& p, f32x4 (&acc)[MB
 #pragma unroll
         for (int j = 0; j < NTB; ++j) v[j] *= sc;
       }
-      epilogue<NTB, EPI, PRE>(p, v, m, nt0, 4 * (l >> 4), pre, m < p.M);
+      epilogue<NTB, EPI, PRE, MB == 1>(p, v, m, nt0, 4 * (l >> 4), pre, m < p.M);
     }
     return;
   }
@@ -795,7 +796,7 @@ __device__ __forceinline__ void gemm_finish(const GemmParams& p, f32x4 (&acc)[MB
 #pragma unroll
       for (int j = 0; j < NTB; ++j) v[j] *= sc;
     }
-    epilogue<NTB, EPI, PRE>(p, v, m, nt0, 4 * (l >> 4), pre, m < p.M);
+    epilogue<NTB, EPI, PRE, MB == 1>(p, v, m, nt0, 4 * (l >> 4), pre, m < p.M);
   }
 }
 

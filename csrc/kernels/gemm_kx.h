@@ -294,7 +294,7 @@ __device__ __forceinline__ void kx_block(const GemmParams& p) {
       ss += xor32(ss);
       v[0] *= rsqrtf(ss / (float)p.K + p.eps);
     }
-    epilogue<1, EPI, false>(p, v, r16, t0 + wid, 4 * grp, EpiPre<1>{}, row_ok);
+    epilogue<1, EPI, false, true>(p, v, r16, t0 + wid, 4 * grp, EpiPre<1>{}, row_ok);
   }
 }
 
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(1024) void kx_half_kernel(GemmParams p) {
     v[0][i] += __shfl_xor(v[0][i], 8, 64);
     v[0][i] += __shfl_xor(v[0][i], 32, 64);
   }
-  epilogue<1, EPI, true>(p, v, r16, t0, 4 * grp, pre, r16 < p.M && (grp >> 1) == h);
+  epilogue<1, EPI, true, true>(p, v, r16, t0, 4 * grp, pre, r16 < p.M && (grp >> 1) == h);
 }
 
 // The fused QKV projection + decode attention launch on this kernel (design: qkv_attn.hip): GROUP
