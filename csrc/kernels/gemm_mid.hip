@@ -154,11 +154,12 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmParams p) {
 // through LDS, a PAIR of m-tiles (32 rows x full K, 2 KB per k-step) at a time: the weights stay
 // in registers while the second pair is DMA'd in. The parts of a tile meet in LDS (fixed part
 // order: bit-reproducible) and the part-0 wave runs the epilogue.
-template <int MT, int EPI, int NORM>
+// PH: m-tiles of an image, two, or all three of 33 .. 48 rows where they fit (17920 x 1536 at 40 rows 15.5 -> 15.0, 6464 x 1536 9.3 -> 8.8. Of
+// four, the last one staged over the first during the MFMAs of the third: no faster, 17.4, 17.5, and slower with fewer tiles, 10.0 -> 10.6).
+template <int MT, int PH, int EPI, int NORM>
 __global__ __launch_bounds__(1024) void gemm_midw_kernel(GemmParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // x [(KT + 1) / 2][PH][2 KiB] | red, ssq
   TLScope tl_scope(p.dbg_ts);
-  constexpr int PH = MT == 1 ? 1 : 2;  // m-tiles per x phase
   constexpr int NPH = (MT + PH - 1) / PH;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -330,22 +331,24 @@ static bool launch_midw_epi(const GemmParams& p, hipStream_t st) {
   if (KT > 64 || KP * tmax > 16 || ntiles < nb) return false;
   const int MT = (p.M + 15) / 16;
   const dim3 grid(nb), block(64 * KP * tmax);
-  const size_t lds = std::max<size_t>((size_t)(KT + 1) / 2 * (MT == 1 ? 1 : 2) * 2048, (size_t)KP * tmax * MT * (1024 + 64));
+  const int PH = MT == 3 && (size_t)(KT + 1) / 2 * 6144 <= 160 * 1024 ? 3 : std::min(MT, 2);
+  const size_t lds = std::max<size_t>((size_t)(KT + 1) / 2 * PH * 2048, (size_t)KP * tmax * MT * (1024 + 64));
   GemmParams q = p;
   if (q.dbg_ts == nullptr) q.dbg_ts = tl_take("gemm_midw", nb);
-#define VG_MW(P_)                                                                                      \
+#define VG_MW(P_, PH_)                                                                                      \
   do {                                                                                                 \
-    auto kern = gemm_midw_kernel<P_, EPI, NORM>;                                                       \
+    auto kern = gemm_midw_kernel<P_, PH_, EPI, NORM>;                                                       \
     static bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                        \
                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) ==  \
                        hipSuccess;                                                                     \
     (void)attr;                                                                                        \
     hipLaunchKernelGGL(kern, grid, block, lds, st, q);                                                 \
   } while (0)
-  if (MT == 1) VG_MW(1);
-  else if (MT == 2) VG_MW(2);
-  else if (MT == 3) VG_MW(3);
-  else VG_MW(4);
+  if (MT == 1) VG_MW(1, 1);
+  else if (MT == 2) VG_MW(2, 2);
+  else if (MT == 3 && PH == 3) VG_MW(3, 3);
+  else if (MT == 3) VG_MW(3, 2);
+  else VG_MW(4, 2);
 #undef VG_MW
   return true;
 }
