@@ -186,6 +186,20 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
     else if (g.N >= 4160) h.waves = 8;
     else if (g.K > 1024 && g.N <= 2048) h.waves = 4;
     if (h.waves != 0 && launch_gemm_mid(h, st)) return;
+    // What the mid kernel leaves, long K of many columns and LM heads with a row gather, went to the K-split kernels and the N-split tiles, which
+    // hold one stage of weights ahead and stage x anew for each block's k-range. The four-wave tiles keep three to five stages in flight:
+    // 64 x 64, two blocks to a CU, or 64 x 128 where those come to one block per CU. us with a norm folded in, before -> now, at 17 / 64 rows:
+    // 8256 x 2560 24.4 -> 17.2 / 28.7 -> 18.4, 12288 x 4096 37.1 -> 26.2 / 41.0 -> 29.9, 28672 x 4096 76.5 -> 38.2 / 80.8 -> 38.8, heads of 32000 x 1536
+    // 26.1 -> 22.3 / 29.8 -> 24.4, 8192 x 1024 11.9 -> 8.5 / 14.1 -> 9.0 (4096 x 1024 5.2, 8.1 / 8.9, 8.4: stays). Without one the old
+    // kernels hold up to 24 rows (10240 x 4096 24.5, 25.7 / 31.6 -> 28.7; 14336 x 6144 35.9 -> 28.8 / 48.3 -> 29.7) and short K of the widest (32000 x
+    // 512 10.1, 11.7 / 12.4, 14.2, 20480 x 1024 12.8, 12.7 / 15.6, 15.3). 64 x 64 / 64 x 128: 32000 x 1536 at 64 rows 25.6, 24.4, at 32 22.9, 23.3; 32000 x
+    // 4096 47.7, 44.0 / 43.5, 43.7; 32000 x 2048 30.8, 31.6 / 27.5, 29.7; 16384 x 4096 (128 blocks) 29.9, 45.2.
+    if (g.norm_w == nullptr && g.N >= 8192 && (g.rownorm || (g.N <= 12288 ? g.M > 24 : g.K > 2048))) {
+      const int wide = g.N % 128 == 0 ? g.N / 128 : 0;
+      h = g;
+      h.ntb = wide > 192 && wide <= 256 && (g.K > 2048 || (g.K >= 1536 && g.K < 2048 && g.M > 32)) ? 5240 : 5220;
+      if (launch_gemm_prefill(h, st)) return;
+    }
   }
   // decode rows on the register-stationary kernel (path 4: a decode plan / forced; gemm_kx_bf16.hip)
   if (g.path == 0 && g.waves == 0 && g.splitk == 0 && g.ntb == 0 && (launch_kx_half(g, st) || (dense_kx_fits(g) && launch_dense_kx(g, st)))) return;

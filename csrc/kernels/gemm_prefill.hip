@@ -1043,10 +1043,11 @@ bool launch_gemm_w4(const GemmParams& p, int code, int nz, hipStream_t st);
 // kernels): K % 64, N % 64, a row gather, the gamma-in-registers RMSNorm mode. A forced form that N is no multiple of: false too, but an
 // error for the four-wave tiles.
 template <int EPI, int NORM>
-static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, size_t slab_bytes, int max_counters,
+static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, size_t slab_bytes, int max_counters, int64_t span,
                                hipStream_t st) {
   constexpr int NTB = 1;  // every epilogue works on self-contained 16-column tiles
-  if (p.K % 64 != 0 || p.N % 64 != 0 || p.row_idx != nullptr) return false;
+  if (p.K % 64 != 0 || p.N % 64 != 0) return false;
+  if (p.row_idx != nullptr && (EPI != EPI_F32 || force_bn < 5000 || span >= (1ll << 31))) return false;
   // the four-wave forms address a block's rows of x by 32-bit offsets and fetch them in 16-B pieces
   const bool rows16 = reinterpret_cast<uintptr_t>(p.x) % 16 == 0 && p.lda % 8 == 0 && p.lda < (1 << 20) && p.K < (1 << 20);
   if (force_bn == 0 && force_sk == 0) {
@@ -1133,9 +1134,9 @@ bool launch_gemm_prefill(const GemmArgs& g, hipStream_t st) {
   const int fb = g.ntb;      // reused as the forced tile width (0 = heuristic, 64 / 128)
   const int fs = g.splitk;   // forced K slices (0 = heuristic)
 #define VG_PF(E)                                                                                         \
-  return norm == 2 ? launch_prefill_epi<E, 2>(p, fb, fs, g.slab_bytes, g.max_counters, st)               \
-                   : launch_prefill_epi<E, 0>(p, fb, fs, g.slab_bytes, g.max_counters, st)
-  if (g.act != 0) return launch_prefill_epi<EPI_GLU, 0>(p, fb, fs, g.slab_bytes, g.max_counters, st);
+  return norm == 2 ? launch_prefill_epi<E, 2>(p, fb, fs, g.slab_bytes, g.max_counters, g.x_span, st)               \
+                   : launch_prefill_epi<E, 0>(p, fb, fs, g.slab_bytes, g.max_counters, g.x_span, st)
+  if (g.act != 0) return launch_prefill_epi<EPI_GLU, 0>(p, fb, fs, g.slab_bytes, g.max_counters, g.x_span, st);
   switch (g.epi) {
     case EPI_SILU: VG_PF(EPI_SILU);
     case EPI_QKV: VG_PF(EPI_QKV);

@@ -150,13 +150,15 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmParams p) {
   const int m0 = (8 * grp + in % gm) * G::BM;
   const int nt_blk = (in / gm) * (2 * NT);
   const u32x4 wrs = rsrc_words(p.wp + ((size_t)nt_blk * KT + 2 * kst0) * 64);
-  const u32x4 xrs = rsrc_words(p.x + (size_t)m0 * p.lda + kst0 * 64);
+  const bool gather = EPI == EPI_F32 && p.row_idx != nullptr;   // (LM heads; every row within 2 GiB of the first: the launcher)
+  const u32x4 xrs = rsrc_words(p.x + (gather ? 0 : (size_t)m0 * p.lda) + kst0 * 64);
   const uint32_t wvo = lane * 16;
   uint32_t xvo[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int g = wid * MT + i;
-    xvo[i] = (uint32_t)(x_piece_row(m0 + (g >> 1) * 16, g & 1, lane, p.M) - m0) * (uint32_t)p.lda * 2u + (uint32_t)x_piece_col(g & 1, lane) * 2u;
+    const int row = x_piece_row(m0 + (g >> 1) * 16, g & 1, lane, p.M);
+    xvo[i] = (uint32_t)(gather ? p.row_idx[row] : row - m0) * (uint32_t)p.lda * 2u + (uint32_t)x_piece_col(g & 1, lane) * 2u;
   }
   const uint32_t lds0 = lds_addr_of(smem);
   const uint32_t wrow = (uint32_t)KT * 1024u, wso0 = (uint32_t)wid * (NT / 2) * wrow;

@@ -24,6 +24,7 @@ bool launch_gemm_w4(const GemmParams& p, int code, int nz, hipStream_t st) {
   switch (code) {
 #define VG_W4(MT, NT, NS) case 5000 + MT * 100 + NT * 10: return launch_w4_one<MT, NT, NS, EPI, NORM>(p, nz, st)
     VG_W4(2, 2, 4);  // two blocks to a CU
+    VG_W4(2, 4, 6);
     VG_W4(3, 4, 5);
     VG_W4(3, 8, 3);
     VG_W4(5, 8, 3);

@@ -76,6 +76,7 @@ struct GemmArgs {
   // decode-only step, EPI_QKV: the step's decode attention rides in the same launch when the decode
   // tile kernel takes the shape (qkv_attn.hip; fa_done set), else the caller launches it after
   const AttnArgs* fa = nullptr;
+  int64_t x_span = 0;           // bytes from the first row of x to the end of its last
   void* fa_gran = nullptr;      // zeroed granule buffer (QaSync::gran), fa_gran_bytes long
   size_t fa_gran_bytes = 0;
   bool* fa_done = nullptr;

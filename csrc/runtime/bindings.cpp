@@ -113,6 +113,7 @@ void gemm(const Tensor& x, const Tensor& wp, int64_t N, int64_t K, Tensor& out, 
   TORCH_CHECK(out.size(0) >= M, "gemm: out rows");
   vgate::GemmArgs g{};
   g.x = bf16p(x); g.lda = (int)x.stride(0); g.M = (int)M; g.row_idx = ridx;
+  g.x_span = x.size(0) * x.stride(0) * 2;
   g.wp = wp.data_ptr(); g.N = (int)N; g.K = (int)K;
   g.norm_w = opt_bf16(norm_w); g.eps = (float)eps; g.rownorm = rownorm ? 1 : 0;
   g.dbg_ts = reinterpret_cast<unsigned long long*>(opt_ptr<int64_t>(dbg_ts, torch::kInt64, "dbg_ts"));

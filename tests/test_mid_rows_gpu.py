@@ -28,3 +28,31 @@ def test_rows_of_a_mixed_step(M, N, K):
     for forced in (None, dict(path=2, waves=8), dict(path=2, waves=4)):
         got = ops.linear(x, nl, norm=(gamma, 1e-6), **(forced or {}))
         assert close(got, torch.nn.functional.silu(y[:, : N // 2]) * y[:, N // 2:])
+
+
+@pytest.mark.parametrize("M", [17, 25, 33, 64])
+@pytest.mark.parametrize("N,K", [(8192, 1024), (8256, 2560), (12352, 2112), (32000, 1536), (28672, 2176), (25600, 576)])
+def test_many_columns_of_a_mixed_step(M, N, K):
+    """Four-wave tiles of 64 and 128 columns: LM heads whose rows come from anywhere in x, and pairs with a norm folded in."""
+    torch.manual_seed(M + N + K)
+    w, gamma = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16(), (torch.rand(K, device="cuda") + 0.5).bfloat16()
+    x = torch.randn(300, K + 8, device="cuda").bfloat16()[:, :K]
+    rows = torch.randint(0, 300, (M,), device="cuda", dtype=torch.int32)
+    rows[0], rows[-1] = 299, 0
+    y = x[rows.long()].float()
+    yn = y * torch.rsqrt((y ** 2).mean(-1, keepdim=True) + 1e-6)
+    head = ops.Linear(w.clone())
+    out = torch.full((M + 1, N + 8), 7.0, device="cuda")
+    ops.linear(x, head, out=out[:M, :N], out_f32=True, row_idx=rows)
+    assert ((out[:M, :N] - y @ w.float().t()).abs() <= 8.0 * K * 2.0 ** -24 + 1e-6).all()
+    assert bool((out[M] == 7).all() and (out[:, N:] == 7).all())
+    assert head.fold_norm(gamma)
+    wg = (w.float() * gamma.float()).bfloat16().float()
+    got = ops.linear(x, head, out_f32=True, row_idx=rows, norm=(gamma, 1e-6))
+    assert ((got - yn @ wg.t()).abs() <= 32.0 * K * 2.0 ** -24 + 1e-5).all()
+    pair = ops.Linear(w.clone(), kind="silu")
+    assert pair.fold_norm(gamma)
+    got, want = ops.linear(x[:M], pair, norm=(gamma, 1e-6)), x[:M].float()
+    want = (want * torch.rsqrt((want ** 2).mean(-1, keepdim=True) + 1e-6)) @ wg.t()
+    want = torch.nn.functional.silu(want[:, : N // 2]) * want[:, N // 2:]
+    assert ((got.float() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -7).all()
