@@ -35,7 +35,8 @@ PLANS: dict[tuple[int, int, str, str], tuple] = {
     # Qwen2.5-1.5B bf16 gate_up on the register-stationary kernel (one block per CU owning 4-5 whole
     # tiles, every weight fragment requested at once; csrc/kernels/gemm_kx.h): 10.5 vs 11.9 us per
     # launch as the hand-off consumer, cold weights (benchmarks/probes/dense_kx_sweep.py,
-    # profiles/r5_dense_kx_sweep.log). qkv / o_proj / down_proj stay on the tile kernels there.
+    # profiles/r5_dense_kx_sweep.log). qkv stays on the tile kernels there; o_proj (to 8 rows) and down_proj (to 4) run as half tiles
+    # by the launcher's own rule (csrc/kernels/gemm_kx_bf16.hip).
     (17920, 1536, "silu", "dense"): ("kx", 0, 0, 0),
     # Qwen2.5-1.5B AWQ int4: no entries — every int4 decode GEMM runs the register-stationary kernel
     # (csrc/kernels/gemm_awq_kx.hip) on its own grid rule (round 3's awq_stream / wide plans:

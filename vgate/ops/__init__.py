@@ -305,7 +305,7 @@ def linear(x: torch.Tensor, lin: Linear, out: torch.Tensor | None = None,
 
     RMSNorm hand-off to the int4 decode kernels (GPU, <= 16 rows, TP = 1; gemm_epilogue.h):
     norm_out=(hg, ssp, gamma) on a residual GEMM also writes hg = out * gamma and per-16-column
-    sums of out^2 into ssp; prenorm=(ssp, eps) on an AWQ consumer whose x IS that hg applies the
+    sums of out^2 into ssp (per 8 columns where ssp is [M][N / 8], see half_tiles); prenorm=(ssp, eps) on an AWQ consumer whose x IS that hg applies the
     row scale from ssp (no gamma loads or x^2 pass in the int4 kernel).
 
     norm=(w, eps): fused RMSNorm of x rows (deferred row scale, see gemm.hip); row_idx: gather rows of x first;
