@@ -83,3 +83,18 @@ def test_register_stationary_choice(M, N, K):
     xn = x.float() * torch.rsqrt((x.float() ** 2).mean(-1, keepdim=True) + 1e-6)
     y = xn @ (w.float() * gamma.float()).bfloat16().float().t()
     _close(ops.linear(x, nl, norm=(gamma, 1e-6)), torch.nn.functional.silu(y[:, : N // 2]) * y[:, N // 2:], 8 * K)
+
+
+@pytest.mark.parametrize("M", [1, 16])
+@pytest.mark.parametrize("N,K", [(20480, 512), (28672, 512), (16384, 384)])
+def test_int4_blocks_with_fewer_waves_than_tiles(M, N, K):
+    from vgate.ops import reference as ref
+    torch.manual_seed(M + N + K)
+    q = torch.randint(0, 16, (N, K), dtype=torch.int32)
+    scales, zeros = (torch.rand(K // 128, N) * 0.02 + 0.005).bfloat16(), torch.randint(0, 16, (K // 128, N)).float().bfloat16()
+    w = ref.awq_dequant_ref(q, scales, zeros, 128).cuda()
+    lin = ops.Linear(None, awq={"qint": q, "scales": scales.cuda(), "zeros": zeros.cuda(), "group": 128})
+    x = _rand(M, K).bfloat16()
+    got, want = ops.linear(x, lin).float(), ref.linear_ref(x, w).float()
+    assert (got - want).norm() / want.norm() < 2e-2   # (as every int4 product here: bf16 scales times zero points)
+    assert bool(((got - want).abs().amax(0) < 0.1 * want.abs().max()).all())
