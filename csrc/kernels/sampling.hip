@@ -82,7 +82,7 @@ __device__ __forceinline__ Acc wave_merge(const Acc& a, float c, Mode) {
   if constexpr (Mode::value == 0) {
     r.mx = wave_max(a.mx);
     r.amx = wave_min(a.mx == r.mx ? a.amx : 0x7fffffff);
-    r.z = wave_sum(a.mx == r.mx ? a.z : a.z * __builtin_amdgcn_exp2f((a.mx - r.mx) * c));  // (z = 0 where mx = -inf)
+    r.z = wave_sum(a.mx == r.mx ? a.z : a.mx == -INFINITY ? 0.f : a.z * __builtin_amdgcn_exp2f((a.mx - r.mx) * c));
   } else {
     r.cnt = wave_sum(a.cnt);
     r.q = wave_sum(a.q);
@@ -144,7 +144,8 @@ __device__ __forceinline__ void accum4(const float (&v)[4], int i, const float (
   if constexpr (mode == 0) {
     const float m = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
     if (m > acc.mx) {
-      acc.z = acc.z * __builtin_amdgcn_exp2f((acc.mx - m) * rp.c);  // (0 while mx = -inf)
+      // (nothing yet: the exponent may be no number, -inf times the scale 0 of an infinite temperature)
+      acc.z = acc.mx == -INFINITY ? 0.f : acc.z * __builtin_amdgcn_exp2f((acc.mx - m) * rp.c);
       acc.mx = m;
       acc.amx = i + (v[0] == m ? 0 : v[1] == m ? 1 : v[2] == m ? 2 : 3);
     }
@@ -192,7 +193,7 @@ __device__ __forceinline__ void sweep_range(const float4* x4, int v_lo, int v_hi
       const float e[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
       float uu[4] = {0.5f, 0.5f, 0.5f, 0.5f};
       if (!rp.greedy) philox4(rp.seed, rp.off, (uint32_t)vi, round, uu);
-float L[4];
+      float L[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         L[j] = (!rp.greedy && (mode == 0 || e[j] > xj) && e[j] > -INFINITY) ? gumbel_log(uu[j]) : 0.f;

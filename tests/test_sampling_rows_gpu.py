@@ -83,3 +83,30 @@ def test_extreme_logits_and_the_ring(B, V):
                 assert ids[b] == few[b, 0], b
             elif t[b] == 0.0:
                 assert ids[b] == few[b][lg[b, few[b]].argmax()], b
+
+
+@pytest.mark.parametrize("T", [3.0e38, float("inf")])
+@pytest.mark.parametrize("B,V", [(1, 4096), (8, 32000), (300, 4096)])
+def test_infinite_temperature(B, V, T):
+    """Every logit that counts weighs the same: draws come from all of the nucleus (those with fewer than top_p n, or top_k, above them),
+    and the log-probability is that of one in n. Some rows have most of their logits masked."""
+    dev, draws = "cuda", 24
+    g = torch.Generator().manual_seed(B + V)
+    lg = torch.randn(B, V, generator=g)
+    lg[::3, V // 4:] = -torch.inf
+    n = torch.isfinite(lg).sum(1)
+    p, k = torch.tensor([0.5, 1.0, 0.9, 1.0] * B)[:B], torch.tensor([-1, -1, -1, 300] * B, dtype=torch.int32)[:B]
+    most = torch.where(p < 1.0, p.double() * n, torch.where(k > 0, k, n).double())
+    above = lg.argsort(dim=1, descending=True, stable=True).argsort(dim=1)
+    seen = []
+    for d in range(draws):
+        lp = torch.empty(B, device=dev)
+        ids = ops.sample(lg.to(dev), torch.full((B,), T, device=dev), p.to(dev), k.to(dev), torch.arange(B, device=dev),
+                         torch.full((B,), d, device=dev), out_logprob=lp).cpu()
+        assert torch.isfinite(lg[torch.arange(B), ids.long()]).all()
+        torch.testing.assert_close(lp.cpu(), -n.float().log(), rtol=1e-5, atol=0.0)
+        seen.append(above[torch.arange(B), ids.long()])
+    seen = torch.stack(seen).double() / most   # ranks as shares of the nucleus, uniform on [0, 1)
+    assert (seen < 1.0).all()
+    # mean 1/2 with a deviation of (12 draws)^-1/2 = 0.06; 6 of them
+    assert ((seen.mean(0) - 0.5).abs() < 6 * (12 * draws) ** -0.5).all()
