@@ -763,7 +763,9 @@ static void launch_m(GemmParams p, const GemmArgs& g, hipStream_t st) {
       // two-deep stage pipeline (gemm_tile3_kernel) once K has >= 3 stages; waves -1 / -2 force
       // the one-deep / two-deep form (sweeps, tests)
       // (one column tile per wave only: with 2 / 4 the three weight groups spill to scratch)
-      const bool deep = NTW == 1 && g.K % (32 * TG_KS) == 0 &&
+      // (its offsets into x and the weights have 32 bits, within descriptors of 2 GiB)
+      const bool near = g.x_span < (1ll << 31) && (int64_t)g.N * g.K * 2 < (1ll << 31);
+      const bool deep = NTW == 1 && near && g.K % (32 * TG_KS) == 0 &&
                         (g.waves == -2 || (g.waves != -1 && (g.K / 32) >= 3 * TG_KS));
       if (p.dbg_ts == nullptr) p.dbg_ts = tl_take(deep ? "gemm_tile3" : "gemm_tile", tblocks);
       if constexpr (NTW == 1) {

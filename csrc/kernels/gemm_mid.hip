@@ -358,6 +358,7 @@ bool launch_gemm_mid(const GemmArgs& g, hipStream_t st) {
   if ((g.M <= 16 && g.waves != 8) || g.M > 64 || g.row_idx != nullptr || g.norm_w != nullptr || g.N % 16 != 0 ||
       g.K % 32 != 0)
     return false;
+  if (g.x_span >= (1ll << 31)) return false;  // (stage_x: 32-bit offsets within a descriptor of 2 GiB)
   GemmParams p{};
   p.x = g.x; p.lda = g.lda; p.M = g.M; p.row_idx = nullptr;
   p.wp = reinterpret_cast<const uint4*>(g.wp); p.N = g.N; p.K = g.K;

@@ -56,3 +56,41 @@ def test_many_columns_of_a_mixed_step(M, N, K):
     want = (want * torch.rsqrt((want ** 2).mean(-1, keepdim=True) + 1e-6)) @ wg.t()
     want = torch.nn.functional.silu(want[:, : N // 2]) * want[:, N // 2:]
     assert ((got.float() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -7).all()
+
+
+@pytest.mark.parametrize("stride", [17_300_000, (1 << 25) + 8])
+@pytest.mark.parametrize("M", [17, 64])
+def test_rows_far_apart(M, stride):
+    """Rows of x that span more than 2 GiB, of which 32-bit offsets (the larger stride) and buffer descriptors (both) see only a part."""
+    gap = stride if M == 64 else 4 * stride
+    K = 4128
+    x = torch.empty((M - 1) * gap + K, device="cuda", dtype=torch.bfloat16).as_strided((M, K), (gap, 1))
+    x.copy_(torch.randn(M, K, device="cuda"))
+    assert x.stride(0) * (M - 1) * 2 > 1 << 31
+    rows = torch.randperm(M, device="cuda").int()
+    for N, k in ((1536, 1536), (4608, 992), (512, 4128), (8192, 1024)):
+        torch.manual_seed(M + N)
+        w = (torch.randn(N, k, device="cuda") * k ** -0.5).bfloat16()
+        lin, xs = ops.Linear(w), x[:, :k]
+        want = xs.float() @ w.float().t()
+        for forced in (None, dict(path=2, waves=8), dict(path=2, waves=4)):
+            got = ops.linear(xs, lin, **(forced or {}))
+            assert ((got.float() - want).abs() <= 2.0 ** -8 * want.abs() + 8.0 * k * 2.0 ** -24 + 1e-6).all(), (N, forced)
+        got = ops.linear(xs, lin, out_f32=True, row_idx=rows)
+        assert ((got - want[rows.long()]).abs() <= 8.0 * k * 2.0 ** -24 + 1e-6).all(), N
+
+
+@pytest.mark.parametrize("M", [40, 80])
+def test_head_of_more_than_2_gib(M):
+    """An LM head whose last columns lie past 2 GiB, of gathered rows."""
+    N, K = 131072, 8320
+    assert N * K * 2 > 1 << 31
+    torch.manual_seed(M)
+    w = torch.empty(N, K, device="cuda", dtype=torch.bfloat16).normal_(0.0, K ** -0.5)
+    lin = ops.Linear(w)
+    x = torch.randn(300, K, device="cuda").bfloat16()
+    rows = torch.randint(0, 300, (M,), device="cuda", dtype=torch.int32)
+    out = ops.linear(x, lin, out_f32=True, row_idx=rows)
+    for cols in (slice(0, 256), slice(N - 4096, N)):
+        want = x[rows.long()].float() @ w[cols].float().t()
+        assert ((out[:, cols] - want).abs() <= 8.0 * K * 2.0 ** -24 + 1e-6).all(), cols
