@@ -404,6 +404,7 @@ bool launch_gemm_sk(const GemmArgs& g, hipStream_t st) {
   if (g.M > 16 || g.row_idx != nullptr || g.norm_w != nullptr || g.ssp_out != nullptr || g.ssp_in != nullptr ||
       g.sk_pub == nullptr || g.K % 32 != 0)
     return false;
+  if (g.x_span >= (1ll << 31) || (int64_t)g.N * g.K * 2 >= (1ll << 31)) return false;  // (32-bit offsets within descriptors of 2 GiB)
   if (g.epi == EPI_QKV && (g.N / 16) % 2 != 0) return false;
   const int norm = g.rownorm ? 2 : 0;
   // instantiated pairs: plain / f32 without a norm, SiLU / QKV with the folded-gamma row scale

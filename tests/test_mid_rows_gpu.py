@@ -80,9 +80,9 @@ def test_rows_far_apart(M, stride):
         assert ((got - want[rows.long()]).abs() <= 8.0 * k * 2.0 ** -24 + 1e-6).all(), N
 
 
-@pytest.mark.parametrize("M", [40, 80])
+@pytest.mark.parametrize("M", [8, 40, 80])
 def test_head_of_more_than_2_gib(M):
-    """An LM head whose last columns lie past 2 GiB, of gathered rows."""
+    """An LM head whose last columns lie past 2 GiB, of gathered rows, and of rows in place also where stream-K is asked for."""
     N, K = 131072, 8320
     assert N * K * 2 > 1 << 31
     torch.manual_seed(M)
@@ -91,6 +91,8 @@ def test_head_of_more_than_2_gib(M):
     x = torch.randn(300, K, device="cuda").bfloat16()
     rows = torch.randint(0, 300, (M,), device="cuda", dtype=torch.int32)
     out = ops.linear(x, lin, out_f32=True, row_idx=rows)
+    plain = ops.linear(x[:M], lin, out_f32=True, path=3 if M <= 16 else 0)
     for cols in (slice(0, 256), slice(N - 4096, N)):
-        want = x[rows.long()].float() @ w[cols].float().t()
-        assert ((out[:, cols] - want).abs() <= 8.0 * K * 2.0 ** -24 + 1e-6).all(), cols
+        for got, rs in ((out, rows.long()), (plain, slice(0, M))):
+            want = x[rs].float() @ w[cols].float().t()
+            assert ((got[:, cols] - want).abs() <= 8.0 * K * 2.0 ** -24 + 1e-6).all(), cols
