@@ -39,29 +39,53 @@ static int cu_count_mid() {
   return n;
 }
 
-// Pieces of x for the 64-k tiles t0, t0 + dt, .. < nt of an image whose first k is the descriptor's: 8 rows each, the c-th of the 2 R in a
-// tile (16-row tile c / 2, half c & 1), at lds + (t 2 R + c) KiB. A wave keeps to one c, so that a piece is an addition to a scalar:
-// addresses worked out piece by piece took the small forms as long as their loads (1024 x 1024 at 24 rows 5.9 against 5.3 us).
+// An image of x from column x0 on, nt 64-k tiles of R 16-row tiles, by a block of nw waves. The lower 8 rows of all R tiles lie at lds + 2 t R KiB,
+// the upper ones behind them, a piece of 1 KiB each. (With addresses worked out piece by piece the small forms took as long as their loads:
+// 1024 x 1024 at 24 rows 5.9 us, 4.9 now.) 2 R waves or more keep to one piece of every tile each: a piece is then an addition to a
+// scalar. Fewer were uneven with that (1280 x 1280 at 17 rows, three waves, 5.5 us, 5.0 now; 8512 x 512 at 32 5.5, 5.1): halves of tiles are dealt
+// out to them one by one, R pieces off one setting of M0, whose instruction offsets count in memory too (the descriptor begins 4 KiB
+// below x0, and the i-th offset is i KiB less). Many waves take longer that way: 9904 x 1280 at 24 rows, nine of them, 8.0 -> 8.6.
 template <int R>
-__device__ __forceinline__ void stage_x(const GemmParams& p, u32x4 xrs, int row0, int kleft, int c, int t0, int dt, int nt, int lane,
-                                        uint32_t lds) {
-  const int col = x_piece_col(c & 1, lane);
-  const uint32_t vo = (uint32_t)x_piece_row(row0 + 16 * (c >> 1), c & 1, lane, p.M) * (uint32_t)p.lda * 2u + (uint32_t)col * 2u;
-  for (int t = t0; t < nt; t += dt) {
-    uint32_t v = vo;
-    if (64 * t + 64 > kleft && col >= 32) v -= 64;  // (K % 64 = 32: the second half of the last tile repeats the first and is not read)
-    blds16(xrs, v, (uint32_t)t * 128u, __builtin_amdgcn_readfirstlane(lds + (uint32_t)(t * 2 * R + c) * 1024u));
+__device__ __forceinline__ void stage_x(const GemmParams& p, const bf16_t* x0, int row0, int kleft, int nt, int wid, int nw, int lane, uint32_t lds) {
+  const u32x4 xrs = rsrc_words(x0 - 2048);
+  const uint32_t l0 = __builtin_amdgcn_readfirstlane(lds);
+  auto offset = [&](int i, int h) {
+    return ((uint32_t)x_piece_row(row0 + 16 * i, h, lane, p.M) * (uint32_t)p.lda + (uint32_t)x_piece_col(h, lane)) * 2u + 4096u;
+  };
+  // K % 64 = 32: the second half of the last tile's columns repeats the first and is not read
+  auto back = [&](int h) { return x_piece_col(h, lane) >= 32 ? 64u : 0u; };
+  const int whole = min(nt, kleft >> 6);
+  if (nw >= 2 * R) {
+    const int c = wid % (2 * R), h = c & 1, dt = (nw - c + 2 * R - 1) / (2 * R);
+    const uint32_t vo = offset(c >> 1, h), l = l0 + (uint32_t)(h * R + (c >> 1)) * 1024u;
+    for (int t = wid / (2 * R); t < nt; t += dt)
+      blds16(xrs, t < whole ? vo : vo - back(h), (uint32_t)t * 128u, l + (uint32_t)t * (R * 2048u));
+    return;
+  }
+  uint32_t vo[2][R];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < R; ++i) vo[h][i] = offset(i, h) - i * 1024u;
+  auto half = [&](int f) {
+    const uint32_t so = (uint32_t)(f >> 1) * 128u, l = l0 + (uint32_t)f * (R * 1024u);
+    if (f & 1) blds16_run<R>(xrs, vo[1], so, l);
+    else blds16_run<R>(xrs, vo[0], so, l);
+  };
+  int f = wid;
+  for (; f < 2 * whole; f += nw) half(f);
+  if (f < 2 * nt) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < R; ++i) vo[h][i] -= back(h);
+    for (; f < 2 * nt; f += nw) half(f);
   }
 }
-// the whole image by a block of nw waves
+// where a lane's fragment of k-step ks lies in a tile of such an image, that of the m-th 16-row tile m KiB on
 template <int R>
-__device__ __forceinline__ void stage_x_all(const GemmParams& p, u32x4 xrs, int row0, int kleft, int nt, int wid, int nw, int lane, uint32_t lds) {
-  if (nw >= 2 * R) {
-    const int c = wid % (2 * R);
-    stage_x<R>(p, xrs, row0, kleft, c, wid / (2 * R), (nw - c + 2 * R - 1) / (2 * R), nt, lane, lds);
-  } else {
-    for (int c = wid; c < 2 * R; c += nw) stage_x<R>(p, xrs, row0, kleft, c, 0, 1, nt, lane, lds);
-  }
+__device__ __forceinline__ int staged_frag(int ks, int lane) {
+  return x_frag_off(ks, lane) + ((lane & 15) >> 3) * (R - 1) * 1024;
 }
 
 template <int MT, int KS, int EPI, int NORM>
@@ -77,7 +101,7 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmParams p) {
   const int k0 = 2 * kt0, nks = min(2 * kt1, KT) - k0;  // nks <= KS (host-checked)
   const int nt = blockIdx.x * W + wid;
   // 1) x slice -> LDS
-  stage_x_all<MT>(p, rsrc_words(p.x + (size_t)kt0 * 64), 0, p.K - kt0 * 64, kt1 - kt0, wid, W, lane, lds_addr_of(smem));
+  stage_x<MT>(p, p.x + (size_t)kt0 * 64, 0, p.K - kt0 * 64, kt1 - kt0, wid, W, lane, lds_addr_of(smem));
   // 2) every weight fragment of this wave's tile slice (clamped past the slice: never consumed)
   uint4 w[KS];
   const uint4* wb = p.wp + ((size_t)nt * KT + k0) * 64 + lane;
@@ -93,14 +117,14 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmParams p) {
   float ss[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) ss[mt] = 0.f;
-  const int xo[2] = {x_frag_off(0, lane), x_frag_off(1, lane)};
+  const int xo[2] = {staged_frag<MT>(0, lane), staged_frag<MT>(1, lane)};
   const bool sums = S == 1 || (blockIdx.x == 0 && wid == 0);  // wave-uniform: who needs the rows' squares
 #pragma unroll
   for (int u = 0; u < KS; ++u) {
     if (u < nks) {  // wave-uniform
       uint4 xb[MT];
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) xb[mt] = *reinterpret_cast<const uint4*>(smem + ((u >> 1) * MT + mt) * 2048 + xo[u & 1]);
+      for (int mt = 0; mt < MT; ++mt) xb[mt] = *reinterpret_cast<const uint4*>(smem + (u >> 1) * (MT * 2048) + mt * 1024 + xo[u & 1]);
       if constexpr (NORM == 2) {
         if (sums) {
 #pragma unroll
@@ -166,7 +190,7 @@ __global__ __launch_bounds__(1024) void gemm_midw_kernel(GemmParams p) {
   const int nw = blockDim.x >> 6;
   const int KT = p.K >> 5, KP = (KT + 15) >> 4;
   const int ntiles = p.N >> 4, nb = gridDim.x, b = blockIdx.x;
-  const int t0 = (int)(((long long)ntiles * b) / nb), ntb = (int)(((long long)ntiles * (b + 1)) / nb) - t0;
+  const int t0 = (int)((uint32_t)(ntiles * b) / (uint32_t)nb), ntb = (int)((uint32_t)(ntiles * (b + 1)) / (uint32_t)nb) - t0;  // (16 tiles a block at most)
   const int my = wid / KP, part = wid - my * KP;
   const bool active = my < ntb;  // wave-uniform
   const int nt = t0 + (active ? my : 0);
@@ -176,8 +200,7 @@ __global__ __launch_bounds__(1024) void gemm_midw_kernel(GemmParams p) {
   const bool sums = my == 0 || KP == 1;
   uint4 w[16];
   const uint32_t lds0 = lds_addr_of(smem);
-  const u32x4 xrs = rsrc_words(p.x);
-  const int xo[2] = {x_frag_off(0, lane), x_frag_off(1, lane)};
+  const int xo[2] = {staged_frag<PH>(0, lane), staged_frag<PH>(1, lane)};
   f32x4 acc[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -187,7 +210,7 @@ __global__ __launch_bounds__(1024) void gemm_midw_kernel(GemmParams p) {
 #pragma unroll
   for (int ph = 0; ph < NPH; ++ph) {
     if (ph > 0) __builtin_amdgcn_s_barrier();  // every wave is done reading the previous phase's x
-    stage_x_all<PH>(p, xrs, PH * ph * 16, p.K, (KT + 1) >> 1, wid, nw, lane, lds0);
+    stage_x<PH>(p, p.x, PH * ph * 16, p.K, (KT + 1) >> 1, wid, nw, lane, lds0);
     if (ph == 0) {
       if (active) {
         const uint4* wb = p.wp + ((size_t)nt * KT + kb) * 64 + lane;
@@ -209,7 +232,7 @@ __global__ __launch_bounds__(1024) void gemm_midw_kernel(GemmParams p) {
 #pragma unroll
           for (int i = 0; i < PH; ++i) {
             if (PH * ph + i < MT) {
-              const uint4 xv = *reinterpret_cast<const uint4*>(smem + (((kb + u) >> 1) * PH + i) * 2048 + xo[u & 1]);  // (kb is even)
+              const uint4 xv = *reinterpret_cast<const uint4*>(smem + ((kb + u) >> 1) * (PH * 2048) + i * 1024 + xo[u & 1]);  // (kb is even)
               if constexpr (NORM == 2) {
                 if (sums) ss[PH * ph + i] = sumsq8(xv, ss[PH * ph + i]);
               }
@@ -358,7 +381,7 @@ bool launch_gemm_mid(const GemmArgs& g, hipStream_t st) {
   if ((g.M <= 16 && g.waves != 8) || g.M > 64 || g.row_idx != nullptr || g.norm_w != nullptr || g.N % 16 != 0 ||
       g.K % 32 != 0)
     return false;
-  if (g.x_span >= (1ll << 31)) return false;  // (stage_x: 32-bit offsets within a descriptor of 2 GiB)
+  if (g.x_span >= (1ll << 31) - 8192) return false;  // (stage_x: 32-bit offsets within a descriptor of 2 GiB)
   GemmParams p{};
   p.x = g.x; p.lda = g.lda; p.M = g.M; p.row_idx = nullptr;
   p.wp = reinterpret_cast<const uint4*>(g.wp); p.N = g.N; p.K = g.K;

@@ -32,9 +32,16 @@ __device__ __forceinline__ void blds16(u32x4 rsrc, uint32_t voff, uint32_t soff,
 // N of them off one setting of M0, the i-th 1 KiB i further in memory and in LDS (the instruction's offset counts in both)
 template <int N>
 __device__ __forceinline__ void blds16_run(u32x4 rsrc, const uint32_t (&voff)[N], uint32_t soff, uint32_t lds) {
-  static_assert(N == 2 || N == 4, "the offset has 12 bits");
+  static_assert(N >= 1 && N <= 4, "the offset has 12 bits");
   unsigned keep;
-  if constexpr (N == 2)
+  if constexpr (N == 1)
+    blds16(rsrc, voff[0], soff, lds);
+  else if constexpr (N == 3)
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %6\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %4, %5 offen lds\n\t"
+                 "buffer_load_dwordx4 %2, %4, %5 offen offset:1024 lds\n\tbuffer_load_dwordx4 %3, %4, %5 offen offset:2048 lds\n\t"
+                 "s_mov_b32 m0, %0"
+                 : "=&s"(keep) : "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "s"(rsrc), "s"(soff), "s"(lds) : "memory");
+  else if constexpr (N == 2)
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %5\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %3, %4 offen lds\n\t"
                  "buffer_load_dwordx4 %2, %3, %4 offen offset:1024 lds\n\ts_mov_b32 m0, %0"
                  : "=&s"(keep) : "v"(voff[0]), "v"(voff[1]), "s"(rsrc), "s"(soff), "s"(lds) : "memory");

@@ -30,6 +30,20 @@ def test_rows_of_a_mixed_step(M, N, K):
         assert close(got, torch.nn.functional.silu(y[:, : N // 2]) * y[:, N // 2:])
 
 
+@pytest.mark.parametrize("M", [17, 32, 41, 64])
+@pytest.mark.parametrize("N,K", [(512, 32), (512, 96), (544, 480), (5376, 224), (8512, 160), (8256, 544), (1296, 1312), (12352, 416), (20992, 96), (528, 2016)])
+def test_images_of_few_and_uneven_waves(M, N, K):
+    """One to eight waves stage an image of one to 32 tiles, the last of them whole or half: by halves of tiles dealt out to the waves, and
+    (two to a 16-row tile) by a piece of every tile each."""
+    torch.manual_seed(M + N + K)
+    w, x = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16(), torch.randn(M, K + 8, device="cuda").bfloat16()
+    x[:, K:] = float("nan")   # (nothing past K counts)
+    lin, want = ops.Linear(w), x[:, :K].float() @ w.float().t()
+    for forced in (None, dict(path=2, waves=8), dict(path=2, waves=1), dict(path=2, waves=2), dict(path=2, waves=4)):
+        got = ops.linear(x[:, :K], lin, out_f32=True, **(forced or {}))
+        assert ((got - want).abs() <= 8.0 * K * 2.0 ** -24 + 1e-6).all(), forced
+
+
 @pytest.mark.parametrize("M", [17, 25, 33, 64])
 @pytest.mark.parametrize("N,K", [(8192, 1024), (8256, 2560), (12352, 2112), (32000, 1536), (28672, 2176), (25600, 576)])
 def test_many_columns_of_a_mixed_step(M, N, K):
