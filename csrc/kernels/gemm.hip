@@ -145,6 +145,39 @@ static GemmParams to_params(const GemmArgs& g) {
   return p;
 }
 
+// What the medium kernel leaves of 17 .. 64 rows, long K of many columns and LM heads with a row gather, runs on the tiles of gemm_decode.h, which
+// hold one stage of weights ahead and stage x anew for each block's k-range, or on four-wave tiles, three to five stages in flight: 64 x
+// 64, two blocks to a CU, or 64 x 128. Whether: us, cold weights, tiles of gemm_decode.h -> four-wave tiles, at 17 / 64 rows.
+//   With a norm folded in: 8320 x 2304 22.3 -> 14.2 / 26.3 -> 15.6, 16384 x 4096 51.7 -> 27.6 / 58.1 -> 29.0, 32000 x 1536 25.4 -> 21.9 / 29.4 -> 24.0,
+//     151936 x 1536 96.2 -> 94.1 / 116 -> 114; behind at 65536 x 512 (19.9, 22.5 / 25.3, 27.4).
+//   Without one, up to 12288 columns from 25 rows on: 8320 x 4096 20.9, 21.2 / 28.9 -> 23.7. Wider, from K = 2048 on, by how well the other kernels fill the
+//     chip. Pairs and QKV, 64 columns to a block of theirs, lose more of it with more rows: 17408 x 3072 32.1 -> 26.4 / 44.2 -> 30.9; up to 24 rows of
+//     more than 28672 columns they are even or ahead (32000 x 6144 65.9, 72.6 / 87.9 -> 75.6). Others are 128 columns wide from 16384 on, one block to a
+//     CU: with the last round of them four fifths full or less 16384 x 3072 29.4 -> 20.1 / 35.1 -> 22.1, 25600 x 3072 32.1 -> 31.8 / 37.9 -> 35.3, 40960 x
+//     3072 59.3 -> 51.5 / 69.8 -> 58.4; fuller ones hold (32000 x 4096 48.7, 52.2 / 52.1, 54.4, 65536 x 2304 52.8, 58.7 / 65.7, 71.6, 128256 x 2304 104, 113 /
+//     129, 141), but for more than 32 rows in a single round nine tenths full (27648 x 2304 25.9, 26.9 / 30.8 -> 28.5). Columns that are no multiple
+//     of 128 run on the K-split kernels, which hold up to 24 rows (23360 x 3584 34.1, 37.4 / 60.7 -> 43.9).
+static bool four_wave_fits(const GemmArgs& g) {
+  if (g.norm_w != nullptr || g.N < 8192) return false;
+  if (g.rownorm) return true;
+  if (g.N <= 12288) return g.M > 24;
+  if (g.K <= 2048) return false;
+  const int cus = cu_count_gemm();
+  if (g.epi == EPI_SILU || g.epi == EPI_QKV) return g.M > 24 || g.N <= 112 * cus;
+  if (g.N % 128 != 0) return g.M > 24;
+  const int blocks = g.N / 128, slots = (blocks + cus - 1) / cus * cus;
+  return 10 * blocks <= 8 * slots || (g.M > 32 && 10 * blocks <= 9 * cus);
+}
+// 128 columns to a tile where the narrow ones come to more than one block per CU and these to one at most, and K is long enough for
+// their six stages (64 x 64 / 64 x 128, us with a norm folded in, at 17 / 64 rows: 16384 x 4096 (128 blocks of 128) 27.6, 33.6 / 29.0, 39.4; 17408 x 4096
+// 39.3 -> 34.8 / 46.4 -> 40.3; 24576 x 1024 13.9, 14.4 / 16.2, 16.2, x 1536 18.9 -> 18.7 / 22.1 -> 20.3, x 2304 26.4 -> 24.6 / 31.0 -> 27.0; 32000 x 1536 21.9,
+// 22.6 / 24.7 -> 24.0, x 2048 27.3, 28.9 / 30.7 -> 30.4, x 2304 30.6, 30.6 / 34.6 -> 32.3; 33792 x 2304 (264 blocks) 39.0, 46.4 / 43.8, 49.9): K of 2048 at most
+// and up to 32 rows want no more than three quarters of the CUs.
+static bool four_wave_wide(const GemmArgs& g) {
+  const int cus = cu_count_gemm(), blocks = g.N / 128;
+  return g.N % 128 == 0 && 2 * blocks > cus && blocks <= cus && g.K >= 1536 && (g.K > 2048 || g.M > 32 || 4 * blocks <= 3 * cus);
+}
+
 void launch_gemm(const GemmArgs& g, hipStream_t st) {
   if (g.M <= 0) return;
   // TP row-parallel decode GEMM with the all-reduce in the epilogue: the tile-per-block decode kernels
@@ -186,22 +219,14 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
     else if (g.N >= 4160) h.waves = 8;
     else if (g.K > 1024 && g.N <= 2048) h.waves = 4;
     if (h.waves != 0 && launch_gemm_mid(h, st)) return;
-    // What the mid kernel leaves, long K of many columns and LM heads with a row gather, went to the K-split kernels and the N-split tiles, which
-    // hold one stage of weights ahead and stage x anew for each block's k-range. The four-wave tiles keep three to five stages in flight:
-    // 64 x 64, two blocks to a CU, or 64 x 128 where those come to one block per CU. us with a norm folded in, before -> now, at 17 / 64 rows:
-    // 8256 x 2560 24.4 -> 17.2 / 28.7 -> 18.4, 12288 x 4096 37.1 -> 26.2 / 41.0 -> 29.9, 28672 x 4096 76.5 -> 38.2 / 80.8 -> 38.8, heads of 32000 x 1536
-    // 26.1 -> 22.3 / 29.8 -> 24.4, 8192 x 1024 11.9 -> 8.5 / 14.1 -> 9.0 (4096 x 1024 5.2, 8.1 / 8.9, 8.4: stays). Without one the old
-    // kernels hold up to 24 rows (10240 x 4096 24.5, 25.7 / 31.6 -> 28.7; 14336 x 6144 35.9 -> 28.8 / 48.3 -> 29.7) and short K of the widest (32000 x
-    // 512 10.1, 11.7 / 12.4, 14.2, 20480 x 1024 12.8, 12.7 / 15.6, 15.3). 64 x 64 / 64 x 128: 32000 x 1536 at 64 rows 25.6, 24.4, at 32 22.9, 23.3; 32000 x
-    // 4096 47.7, 44.0 / 43.5, 43.7; 32000 x 2048 30.8, 31.6 / 27.5, 29.7; 16384 x 4096 (128 blocks) 29.9, 45.2.
-    if (g.norm_w == nullptr && g.N >= 8192 && (g.rownorm || (g.N <= 12288 ? g.M > 24 : g.K > 2048))) {
-      const int wide = g.N % 128 == 0 ? g.N / 128 : 0;
+    if (four_wave_fits(g)) {
       h = g;
-      h.ntb = wide > 192 && wide <= 256 && (g.K > 2048 || (g.K >= 1536 && g.K < 2048 && g.M > 32)) ? 5240 : 5220;
+      h.ntb = four_wave_wide(g) ? 5240 : 5220;
       if (launch_gemm_prefill(h, st)) return;
     }
   }
-  // decode rows on the register-stationary kernel (path 4: a decode plan / forced; gemm_kx_bf16.hip)
+  // decode rows without a plan: half tiles or the register-stationary kernel where those are ahead (gemm_kx_bf16.hip); path 4, a decode plan or
+  // forced: the latter
   if (g.path == 0 && g.waves == 0 && g.splitk == 0 && g.ntb == 0 && (launch_kx_half(g, st) || (dense_kx_fits(g) && launch_dense_kx(g, st)))) return;
   if (g.path == 4) {
     GemmArgs h = g;
