@@ -40,9 +40,12 @@ bool launch_kx_half(const GemmArgs& g, hipStream_t st) {
 //     8 rows on: 10240 x 2048 10.3 -> 10.0 / 11.3 -> 10.2 / 13.6 -> 10.8, 6144 x 1792 6.7, 7.2 / 7.9 -> 7.4 / 9.1 -> 8.1, 4096 x 1792 5.3, 5.6 / 5.6, 6.0 / 6.3, 6.9
 //   fewer tiles than CUs: to K = 2048 for 4 rows at most (3072 x 1536 4.7 -> 4.5 / 4.8, 4.8 / 5.6, 5.5, 3584 x 1792 about even); above 8 rows
 //     slices of 16 k-quads at most (1024 x 4096 8.3 -> 7.2, 512 x 8192 9.1 -> 7.4, 2048 x 4096 8.6 -> 7.7; of 18, 24: 1536 x 4608 9.4, 9.6, 2048 x 6144 9.2, 10.6)
+//   but a norm's sums handed over that no wave can ask for ahead (K % 256, ss_pre_n4), for up to 4 rows of short K and a tile per CU: 1536 x 128 at 1 row
+//     3.7, 4.0, at 8 4.5 -> 4.1, 2080 x 640 4.2, 4.7 / 5.1 -> 4.8 (1152 x 896 4.5, 4.6 / 5.0 -> 4.9)
 bool dense_kx_fits(const GemmArgs& g) {
   if (g.M > 16 || g.N % 16 != 0 || g.K % 128 != 0 || g.epi == EPI_QKV) return false;
   const int tiles = g.N / 16, ncu = kx_cus(), KQ = g.K / 128, each = (tiles + ncu - 1) / ncu;
+  if (g.ssp_in != nullptr && g.M <= 4 && g.K % 256 != 0 && g.K <= 640 && tiles <= ncu) return false;
   if (g.K <= 1280) return true;
   if (tiles >= ncu) return each <= 5 && (g.K <= 1536 || (g.K <= 2048 && each >= 2 && each <= 4 && g.M >= 8));
   if (2 * tiles > ncu) return g.K <= 2048 && g.M <= 4;

@@ -98,3 +98,19 @@ def test_int4_blocks_with_fewer_waves_than_tiles(M, N, K):
     got, want = ops.linear(x, lin).float(), ref.linear_ref(x, w).float()
     assert (got - want).norm() / want.norm() < 2e-2   # (as every int4 product here: bf16 scales times zero points)
     assert bool(((got - want).abs().amax(0) < 0.1 * want.abs().max()).all())
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 16])
+@pytest.mark.parametrize("N,K", [(64, 128), (1536, 384), (4096, 640), (4128, 640), (1024, 896), (1024, 512)])
+def test_sums_of_16_columns_of_short_k(M, N, K):
+    """A norm's sums handed over where no wave can ask for them ahead (K % 256), on either side of the line below which the tile blocks take them."""
+    torch.manual_seed(M + N + K)
+    w, gamma, h = (_rand(N, K) * K ** -0.5).bfloat16(), (torch.rand(K, device="cuda") + 0.5).bfloat16(), _rand(M, K).bfloat16()
+    lin = ops.Linear(w.clone(), kind="silu")
+    assert lin.fold_norm(gamma)
+    ssp = h.float().pow(2).reshape(M, K // 16, 16).sum(-1).contiguous()
+    xn = h.float() * torch.rsqrt((h.float() ** 2).mean(-1, keepdim=True) + 1e-6)
+    y = xn @ (w.float() * gamma.float()).bfloat16().float().t()
+    want = torch.nn.functional.silu(y[:, : N // 2]) * y[:, N // 2:]
+    # fp32 sums in another order, one rounding to bf16
+    assert ((ops.linear(h, lin, prenorm=(ssp, 1e-6)).float() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()
