@@ -157,6 +157,18 @@ def test_stages_by_dma(M, N, K, out):
     assert bool((whole[M] == 7).all() and (whole[:, N:] == 7).all())
 
 
+@pytest.mark.parametrize("out", ["bf16", "odd", "gate", "fp32"])
+@pytest.mark.parametrize("M,N,K", [(4097, 2056, 256), (4097, 2056, 512), (4100, 2056, 576), (4100, 2184, 1024), (4100, 2184, 1088)])
+def test_many_tiles_of_short_k(M, N, K, out):
+    """More than two 128-row tiles per CU: by way of registers up to K = 512 (1024 with gates), by LDS-DMA beyond."""
+    test_stages_by_dma(M, N, K, out)
+
+
+@pytest.mark.parametrize("N,K", [(2560, 320), (2184, 640), (2184, 704)])
+def test_many_experts_of_short_k(N, K):
+    test_experts(N, K, [70, 0, 130, 33, 1] * 7)
+
+
 @pytest.mark.parametrize("sizes", [[300, 0, 129, 1, 600], [128] * 9 + [127, 0, 2], [700] * 6])
 @pytest.mark.parametrize("N,K", [(520, 256), (1024, 320)])
 def test_experts_by_dma(N, K, sizes):
