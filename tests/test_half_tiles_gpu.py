@@ -17,6 +17,11 @@ def _close(out, want, K):
     assert ((out.float() - want).abs() <= 2.0 ** -7 * want.abs() + 8.0 * K * 2.0 ** -24 + 2.0 ** -7).all()
 
 
+def _close_pair(out, want):
+    # one rounding to bf16 of a pair whose halves are off by some 2^-24 K^1/2 each, at most 5 of the other and its slope
+    assert ((out.float() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()
+
+
 @pytest.mark.parametrize("M", [1, 2, 4, 5, 8])
 @pytest.mark.parametrize("N,K", [(16, 128), (48, 384), (512, 2176), (1536, 1536), (2048, 6144), (1024, 6272), (256, 10240), (2048, 8960)])
 def test_half_tiles(M, N, K):
@@ -71,18 +76,18 @@ def test_register_stationary_choice(M, N, K):
     f32 = ops.linear(x, lin, out_f32=True)
     assert ((f32 - want).abs() <= 8.0 * K * 2.0 ** -24 + 1e-6).all()
     g, u = want[:, : N // 2], want[:, N // 2:]
-    _close(ops.linear(x, ops.Linear(w, kind="silu")), torch.nn.functional.silu(g) * u, 8 * K)
+    _close_pair(ops.linear(x, ops.Linear(w, kind="silu")), torch.nn.functional.silu(g) * u)
     gelu = ops.Linear(w, kind="silu")
     gelu.glu = (4, 0.0, 0.0)
-    _close(ops.linear(x, gelu), torch.nn.functional.gelu(g, approximate="tanh") * u, 8 * K)
+    _close_pair(ops.linear(x, gelu), torch.nn.functional.gelu(g, approximate="tanh") * u)
     gelu.glu = (2, 0.7, 1.702)
     gc, uc = g.clamp(max=0.7), u.clamp(-0.7, 0.7)
-    _close(ops.linear(x, gelu), gc * torch.sigmoid(1.702 * gc) * (uc + 1), 8 * K)
+    _close_pair(ops.linear(x, gelu), gc * torch.sigmoid(1.702 * gc) * (uc + 1))
     nl, gamma = ops.Linear(w.clone(), kind="silu"), (torch.rand(K, device="cuda") + 0.5).bfloat16()
     assert nl.fold_norm(gamma)
     xn = x.float() * torch.rsqrt((x.float() ** 2).mean(-1, keepdim=True) + 1e-6)
     y = xn @ (w.float() * gamma.float()).bfloat16().float().t()
-    _close(ops.linear(x, nl, norm=(gamma, 1e-6)), torch.nn.functional.silu(y[:, : N // 2]) * y[:, N // 2:], 8 * K)
+    _close_pair(ops.linear(x, nl, norm=(gamma, 1e-6)), torch.nn.functional.silu(y[:, : N // 2]) * y[:, N // 2:])
 
 
 @pytest.mark.parametrize("M", [1, 16])
@@ -112,5 +117,4 @@ def test_sums_of_16_columns_of_short_k(M, N, K):
     xn = h.float() * torch.rsqrt((h.float() ** 2).mean(-1, keepdim=True) + 1e-6)
     y = xn @ (w.float() * gamma.float()).bfloat16().float().t()
     want = torch.nn.functional.silu(y[:, : N // 2]) * y[:, N // 2:]
-    # fp32 sums in another order, one rounding to bf16
-    assert ((ops.linear(h, lin, prenorm=(ssp, 1e-6)).float() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()
+    _close_pair(ops.linear(h, lin, prenorm=(ssp, 1e-6)), want)
