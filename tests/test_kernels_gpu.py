@@ -698,7 +698,7 @@ def test_dense_kx_decode(M, N, K, w, sk, tb):
     C.gemm(x, lin.wp, N, K, out, 0, res=res, **kw)
     assert _rel_err(out, ref.linear_ref(x, wt, None, res)) < 1e-2
     tile = torch.empty_like(out)
-    C.gemm(x, lin.wp, N, K, tile, 0, res=res, ws=kw["ws"])
+    C.gemm(x, lin.wp, N, K, tile, 0, res=res, ws=kw["ws"], path=6)
     assert _rel_err(out, tile) < 5e-3
     h = res.clone()
     ssp_n = torch.empty(M, N // 16, dtype=torch.float32, device=DEV)
