@@ -85,6 +85,22 @@ def test_extreme_logits_and_the_ring(B, V):
                 assert ids[b] == few[b][lg[b, few[b]].argmax()], b
 
 
+@pytest.mark.parametrize("B", [1, 8, 200])
+def test_collective_words_in_the_ring(B):
+    """The three words of the own all-reduce behind the ids: a buffer that stands for its signal area, every word its own index."""
+    dev = "cuda"
+    area = torch.arange(1 << 16, dtype=torch.int32, device=dev)
+    ring = torch.full((2, B + 4), -7, dtype=torch.int32, pin_memory=True)
+    slot = torch.zeros(1, dtype=torch.int32, device=dev)
+    lg = torch.randn(B, 8192, device=dev)
+    for base in (0, area.data_ptr()):
+        out = ops.sample(lg, torch.zeros(B, device=dev), ring=(ring, slot, base))
+        torch.cuda.synchronize()
+        assert torch.equal(ring[0, :B], out.cpu()) and torch.all(ring[1] == -7)
+        error, ticks, calls, fault = ring[0, B:].tolist()
+        assert fault == -7 and ((error, ticks, calls) == (-7, -7, -7) if base == 0 else 0 < error == ticks - 1 == calls - 2)
+
+
 @pytest.mark.parametrize("T", [3.0e38, float("inf")])
 @pytest.mark.parametrize("B,V", [(1, 4096), (8, 32000), (300, 4096)])
 def test_infinite_temperature(B, V, T):
