@@ -628,13 +628,13 @@ void launch_attention(const AttnArgs& a, int dec_seqs, hipStream_t st) {
   if (fc.ct > 0) {
     AttnArgs f = a;
     f.num_tiles = tiles;
-    // the decode rows join this launch (grid rows past the tiles): no second attention launch
+    // the decode rows join this launch (blocks behind the tiles'): no second attention launch
     const int dec_rows = dec_seqs > 0 ? dec_seqs * a.num_parts : 0;
     // a 2-stage K/V ring with the lazy rescale (4 stages and eager rescale measured no faster:
     // profiles/r3_flash_split.log)
     constexpr int lazy = 1;
     const size_t lds = (size_t)2 * FL_STAGE + (size_t)a.max_blocks * 4;
-    // K split of the long causal ranges (zs parts per KV head, adjacent in grid.x) when the
+    // K split of the long causal ranges (zs parts per KV head, adjacent in the grid) when the
     // workspace holds every wave's partials: 2 parts while the step's working blocks fill less
     // than two waves of the chip's block slots (CT = 2 blocks hold a CU alone, CT = 1 two), 4
     // while 4 parts per block still fit in one wave (profiles/r3_flash_split.log: 4 parts won

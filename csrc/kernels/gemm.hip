@@ -193,16 +193,17 @@ void launch_gemm(const GemmArgs& g, hipStream_t st) {
   if (g.path == 2 && launch_gemm_mid(g, st)) return;
   if (g.path == 6) return launch_dispatch<false>(to_params(g), g, st);  // the kernels of gemm_decode.h (q4_prompt_form)
   // without a plan, 17 .. 64 rows: one block per CU owning whole tiles (wide) where K is short, K slices over narrow
-  // tiles where it is long. us at 32 rows, the K-split / tile kernels below -> now: 17920 x 1536 19 -> 14.5, 6464 x 1536
-  // 14.1 -> 9.0, 1536 x 8960 19.2 -> 13.1, 1024 x 4096 12.1 -> 8.4, 1536 x 1536 8.2 -> 6.6. Above 32 rows the wide form pays
-  // only once its tiles cover the CUs (N >= 4160; at 64 rows 6464 x 1536 17.7 -> 13.0, 1536 x 1536 10.5 -> 7.8 sliced). Long and wide stays
-  // with the kernels below (8192 x 3072 at 64 rows 23.6, sliced 29.3; 28672 x 4096 50), and so do up to 32 rows of 3072 to 4096 columns, which
-  // fill the chip without slices (4096 x 4096 at 24 rows 14.1, sliced 17.2, at 32 15.4, 17.3, at 48 21.0, 19.4; with longer K sooner:
-  // 3072 x 5120 at 32 18.8, 16.3), slices that come to little more than a workgroup per CU (2048 x 8960, 288 of them, at 24 rows 19.7, 20.9, at 64
-  // 29.3, 31.2; 6144 x 3072 at 17 17.2, 19.0) and the very shortest (1536 x 3072 at 17 rows 11.0, 12.1, at 32 13.1, 12.5; 1024 x 1024 at 48 9.5, 10.3).
+  // tiles where it is long. us at 32 rows, the K-split / tile kernels of gemm_decode.h -> now: 17920 x 1536 18.3 -> 13.2, 6464 x 1536
+  // 13.7 -> 7.2, 1536 x 8960 18.8 -> 12.8, 1024 x 4096 11.8 -> 7.9, 1536 x 1536 7.9 -> 5.1. Above 32 rows the wide form pays
+  // once its tiles cover the CUs (N >= 4160; at 64 rows 6464 x 1536 17.5 -> 10.0; 1536 x 1536 8.1, sliced 7.5, at 48 5.9, 6.9). Long and wide stays
+  // with the kernels below (8192 x 3072 at 64 rows 18.4, sliced 24.2), and so do up to 32 rows of 3072 to 4096 columns, which
+  // fill the chip without slices (4096 x 4096 at 24 rows 11.4, sliced 13.3, at 32 13.1, 13.8, at 48 18.8 -> 14.8; with longer K sooner:
+  // 3072 x 5120 at 32 16.4 -> 12.3), slices that come to little more than a workgroup per CU (2048 x 8960, 288 of them, at 17 rows 15.6, 15.8;
+  // 6144 x 3072 at 17 14.5, 15.1) and the very shortest (1536 x 3072 at 17 rows 8.1, 8.5, at 24 9.1 -> 8.8).
   // A folded norm costs the wide form more than the K-split kernels, which have more waves to sum squares: few columns of K up to 1024 and of
-  // 2048 stay with them (4096 x 1024 at 17 rows 8.4, wide 10.3, at 32 9.2, 10.5; 1024 x 2048 at 24 10.3, 11.4; 1024 x 1536 at 24 11.0, 10.2;
-  // 6144 x 4096 at 17 19.9, sliced 21.9, at 24 23.0, 22.2).
+  // 2048 stay with them (4096 x 1024 at 17 rows 5.3, wide 6.0, at 32 6.6, 6.4; 1024 x 2048 at 17 6.5, 6.6; 1024 x 1536 at 24 7.8 -> 6.1).
+  // The lines were drawn before the medium kernel brought x by whole lines, which some it does not take would now be ahead with: 2048 x 8960 at 24
+  // rows 17.3, sliced 15.9, at 64 27.0, 22.6; 3584 x 1792 at 48 12.0, wide 8.8; 1024 x 1024 at 48 6.6, wide 5.6; 1024 x 2048 with a norm at 32 8.5, 6.7.
   // (both stage rows of x by 16-B LDS-DMA: rows that are not 16-B aligned stay below)
   const bool rows16 = reinterpret_cast<uintptr_t>(g.x) % 16 == 0 && g.lda % 8 == 0;
   if (g.path == 0 && rows16 && g.M > 16 && g.M <= 64 && g.waves == 0 && g.splitk == 0 && g.ntb == 0 && g.N >= 512) {

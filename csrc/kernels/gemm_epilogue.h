@@ -289,7 +289,7 @@ __device__ __forceinline__ float prenorm_ss(const GemmParams& p, int m, int quar
 }
 
 // NORM 3 consumers: the producer's sums issued at launch, summed after the weight stream (prefetch
-// form: ssn <= 128 = K <= 2048, ssn % 16 == 0; else prenorm_ss after the stream)
+// form: K <= 2048, K % 256 == 0, so whole loads per lane: ssn % 16 == 0, of 8 columns ssn % 32 == 0; else prenorm_ss after the stream)
 constexpr int SS_PRE = 8;  // f32x4 loads per lane
 
 // The producer's per-tile sums of squares of row m, this lane's quarter, loaded at launch (NORM 3).

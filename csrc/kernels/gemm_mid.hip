@@ -11,8 +11,8 @@
 //
 // Here a block is W waves = W adjacent 16-column tiles (one per wave) over one K slice of at most
 // KS k-steps:
-//   1. the slice of x (MT m-tiles x KS k-steps, in 64-k tiles of two 1 KiB pieces of whole 128-B lines, lds_rows.h; rows past M
-//      repeat row M - 1) is DMA'd into LDS (global_load_lds_dwordx4), spread over the W waves;
+//   1. the slice of x (MT m-tiles x KS k-steps, in 64-k tiles of 1 KiB pieces, 8 rows of whole 128-B lines each, stage_x; rows past M
+//      repeat row M - 1) is DMA'd into LDS, spread over the W waves;
 //   2. every wave then issues ALL KS weight fragments of its tile (non-temporal 16-B loads into
 //      registers): the whole launch's weights are requested in the first microsecond;
 //   3. one counted vmcnt (the x pieces only) + barrier, then per k-step MT conflict-free
@@ -90,7 +90,7 @@ __device__ __forceinline__ int staged_frag(int ks, int lane) {
 
 template <int MT, int KS, int EPI, int NORM>
 __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmParams p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];  // [KS / 2][MT][2 KiB]
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // [KS / 2][2][MT][1 KiB]
   TLScope tl_scope(p.dbg_ts);
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -175,14 +175,14 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmParams p) {
 // fragments in registers (64 VGPRs, issued at launch: ~200 KB per CU in flight). us, cold weights, x staged by fragments and squared by
 // every wave -> by whole lines and once: 17920 x 1536 at 32 rows 14.1 -> 13.0, with a norm 17.7 -> 14.9, at 64 rows 19.1 -> 16.2 and 24.6 ->
 // 19.1 (96 x 128 four-wave tiles 20.9); sliced form 6144 x 4096 with a norm at 48 31.0 -> 26.0, at 64 36.0 -> 30.6. x is shared
-// through LDS, a PAIR of m-tiles (32 rows x full K, 2 KB per k-step) at a time: the weights stay
-// in registers while the second pair is DMA'd in. The parts of a tile meet in LDS (fixed part
+// through LDS, PH m-tiles (16 rows x full K, 1 KB per k-step each) at a time: the weights stay
+// in registers while the next ones are DMA'd in. The parts of a tile meet in LDS (fixed part
 // order: bit-reproducible) and the part-0 wave runs the epilogue.
 // PH: m-tiles of an image, two, or all three of 33 .. 48 rows where they fit (17920 x 1536 at 40 rows 15.5 -> 15.0, 6464 x 1536 9.3 -> 8.8. Of
 // four, the last one staged over the first during the MFMAs of the third: no faster, 17.4, 17.5, and slower with fewer tiles, 10.0 -> 10.6).
 template <int MT, int PH, int EPI, int NORM>
 __global__ __launch_bounds__(1024) void gemm_midw_kernel(GemmParams p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];  // x [(KT + 1) / 2][PH][2 KiB] | red, ssq
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // x [(KT + 1) / 2][2][PH][1 KiB] | red, ssq
   TLScope tl_scope(p.dbg_ts);
   constexpr int NPH = (MT + PH - 1) / PH;
   const int lane = threadIdx.x & 63;
@@ -345,7 +345,7 @@ static bool launch_mid_epi(const GemmParams& p, int force_w, int force_s, size_t
 }
 
 // the wide form (g.waves == 8 selects it): N of at least one tile per CU, (tiles per block) x
-// (16-k-step parts per tile) <= 16 waves, K <= 64 k-steps (the pair image fits 128 KiB of LDS)
+// (16-k-step parts per tile) <= 16 waves, K <= 64 k-steps (an image of two m-tiles takes 128 KiB of LDS, of three 160 KiB up to K = 1664)
 template <int EPI, int NORM>
 static bool launch_midw_epi(const GemmParams& p, hipStream_t st) {
   const int ntiles = p.N / 16, KT = p.K / 32, KP = (KT + 15) / 16;

@@ -1040,7 +1040,7 @@ template <int EPI, int NORM>
 bool launch_gemm_w4(const GemmParams& p, int code, int nz, hipStream_t st);
 
 // Returns false for shapes the kernels do not take (the caller keeps the N-split tile
-// kernels): K % 64, N % 64, a row gather, the gamma-in-registers RMSNorm mode. A forced form that N is no multiple of: false too, but an
+// kernels): K % 64, N % 64, a row gather but of fp32 outputs on four-wave tiles, the gamma-in-registers RMSNorm mode. A forced form that N is no multiple of: false too, but an
 // error for the four-wave tiles.
 template <int EPI, int NORM>
 static bool launch_prefill_epi(const GemmParams& p, int force_bn, int force_sk, size_t slab_bytes, int max_counters, int64_t span,

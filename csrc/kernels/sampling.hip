@@ -1,8 +1,8 @@
 // Per-row token sampling over the full vocabulary (V ~ 128k-152k) on gfx950:
 // temperature -> top-k -> top-p -> categorical, or argmax when temperature == 0.
 //
-// Parallel layout: each row is split into NSEG segments, one 256-thread block per
-// (segment, row), so a batch-8 step spreads its 8 x 600 KB of logits over 256 CUs
+// Parallel layout: each row is split into NSEG segments, one block of 512 threads (1024 where segments are long) per
+// (segment, row), so a batch-8 step spreads its 8 x 600 KB of logits over 192 CUs
 // instead of 8. After each pass the blocks of a row exchange tagged partials (sample_gran_kernel:
 // NSEG is chosen on the host so that B * NSEG <= 256 blocks, all co-resident, and every wait has a
 // give-up bound). With NSEG == 1 (large batches) a row is one block (sample_row_kernel).

@@ -454,12 +454,13 @@ void attention(const Tensor& q, int64_t q_stride, const Tensor& k_cache, const T
   vgate::launch_attention(a, a.S, cur_stream());
 }
 
-static void* device_view(const Tensor& t) {
+// a tensor's address for kernels: its own on the GPU, the mapped one of pinned host memory
+static void* device_view(const Tensor& t, const char* who) {
   if (t.is_cuda()) return t.data_ptr();
-  TORCH_CHECK(t.is_pinned(), "kernel_copy: host tensor must be pinned");
+  TORCH_CHECK(t.is_pinned(), who, ": host tensor must be pinned");
   void* d = nullptr;
   TORCH_CHECK(hipHostGetDevicePointer(&d, t.data_ptr(), 0) == hipSuccess && d != nullptr,
-              "kernel_copy: pinned host memory is not device-mapped");
+              who, ": pinned host memory is not device-mapped");
   return d;
 }
 
@@ -508,7 +509,7 @@ void sample(const Tensor& logits, const c10::optional<Tensor>& temperature,
     TORCH_CHECK(ring->dim() == 2 && ring->is_contiguous() && !ring->is_cuda(), "sample: ring = pinned int32 [slots, stride]");
     TORCH_CHECK(s.B <= ring->size(1) - 4, "sample: a ring slot holds the ids and four words");
     TORCH_CHECK(ring_slot.has_value() && ring_slot->defined() && ring_slot->numel() >= 1, "sample: the ring needs its slot");
-    s.ring = static_cast<int32_t*>(device_view(*ring));
+    s.ring = static_cast<int32_t*>(device_view(*ring, "sample: ring"));
     s.ring_slot = static_cast<const int32_t*>(fp(ring_slot, torch::kInt32));
     s.ring_stride = (int)ring->size(1);
     if (ar_base) s.ar = reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(ar_base) + vgate::ar_error_offset());
@@ -529,7 +530,7 @@ void kernel_copy(Tensor& dst, const Tensor& src, int64_t nbytes) {
   TORCH_CHECK(reinterpret_cast<uintptr_t>(dst.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(src.data_ptr()) % 16 == 0,
               "kernel_copy: 16-B aligned tensors");
   c10::DeviceGuard guard(dev.device());
-  vgate::launch_copy16(device_view(src), device_view(dst), (size_t)n, !dst.is_cuda(), cur_stream());
+  vgate::launch_copy16(device_view(src, "kernel_copy"), device_view(dst, "kernel_copy"), (size_t)n, !dst.is_cuda(), cur_stream());
 }
 
 void prefetch(const Tensor& t, int64_t blocks) {

@@ -537,8 +537,8 @@ _FAULT: dict = {}
 def fault_word(device) -> torch.Tensor:
     """Per-device sticky fault word of the in-launch hand-offs (bit 1: a flash K-split waiter gave
     up, 4: a stream-K partial poll, 8: a split-K granule poll, 16: a sampler row meeting, 32: a fused
-    QKV + attention granule poll, 64: a stream-K prefill ticket poll; bit 0 is reserved). Kernels only OR bits in; the step graph's last node
-    copies it to the host ring (ModelRunner.kernel_fault), and a non-zero word fails the engine."""
+    QKV + attention granule poll, 64: a stream-K prefill ticket poll; bit 0 is reserved). Kernels only OR bits in; the step's sampler
+    copies it to the host ring once it is set (ModelRunner.kernel_fault), and a non-zero word fails the engine."""
     key = _dev_key(device)
     t = _FAULT.get(key)
     if t is None:
@@ -548,10 +548,11 @@ def fault_word(device) -> torch.Tensor:
 
 def reset_handoffs(device) -> None:
     """Return every in-launch hand-off buffer of ``device`` to its zeroed start state after a fault
-    (the engine's recovery path; VERDICT r5 weak #9, ADVICE r5: a poll that gave up can leave a
+    (the engine's recovery path: a poll that gave up can leave a
     late producer granule behind, which a later sequence in the same row / position would accept).
     Waits for the device first, so no launch is still writing. The buffers keep their addresses:
-    captured graphs stay valid."""
+    captured graphs stay valid. Copies of the fault word in a runner's ring are its own to clear
+    (ModelRunner.reset_fault_ring)."""
     key = _dev_key(device)
     if torch.device(device).type == "cuda":
         torch.cuda.synchronize(device)

@@ -359,8 +359,10 @@ class ModelRunner:
         return toks
 
     def kernel_fault(self, k: int | None = None) -> int:
-        """The sticky fault word of the in-launch hand-offs (ops.fault_word) as the step graph's last
-        node copied it into ring slot ``k`` (default: the last collected step); 0 = healthy. No sync."""
+        """The sticky fault word of the in-launch hand-offs (ops.fault_word) as the step's sampler
+        copied it into ring slot ``k`` (default: the last collected step); 0 = healthy. No sync. The sampler
+        writes the word only where it is set, as the device's word is only ever added to: a copy stays until
+        :meth:`reset_fault_ring`, which therefore goes with every ops.reset_handoffs."""
         if not self.gpu:
             return 0
         if k is None:
