@@ -24,7 +24,7 @@ def main():
     ap.add_argument("--groups", type=int, default=200)
     ap.add_argument("--per-group", type=int, default=100)
     ap.add_argument("--vocab", type=int, default=151936)
-    ap.add_argument("--nseg", default="16,32,64,128", help="caps on segments per row to sweep")
+    ap.add_argument("--nseg", default="4,8,16,24", help="caps on segments per row to sweep")
     a = ap.parse_args()
     dev = torch.device("cuda:0")
     res = {}

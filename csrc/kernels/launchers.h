@@ -267,7 +267,7 @@ struct SampleArgs {
   const uint32_t* ar = nullptr;
 };
 // sampler workspace (int32 words): [0, SAMPLE_WS_GRAN) per-row epochs, then the granule regions
-constexpr int SAMPLE_GRAN_SEGS = 64;                        // max segments per row
+constexpr int SAMPLE_GRAN_SEGS = 24;                        // max segments per row (sample_segments)
 constexpr int SAMPLE_GRAN_ROWS = 128;                       // rows of the segmented mode (nseg >= 2)
 constexpr int SAMPLE_GRAN_ROW = 2 * SAMPLE_GRAN_SEGS * 2;   // uint4 per row: [parity][segment][2]
 constexpr int SAMPLE_WS_GRAN = 256;                         // int32 offset of the granules (16-B aligned)

@@ -414,7 +414,7 @@ int sample_segments(int B, int V) {
   const int V4 = V >> 2;
   int nseg = SAMPLE_MAX_BLOCKS / (B > 0 ? B : 1);
   if (nseg > g_sample_nseg) nseg = g_sample_nseg;
-  nseg = std::min(nseg, std::min(V4 / 256, std::max(8, std::min(24, V4 / 512))));
+  nseg = std::min(nseg, std::min(V4 / 256, std::max(8, std::min(SAMPLE_GRAN_SEGS, V4 / 512))));
   return nseg < 1 ? 1 : nseg;
 }
 
