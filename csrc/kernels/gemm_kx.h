@@ -482,8 +482,10 @@ static bool kx_launch_xp(GemmParams p, const GemmArgs& g, hipStream_t st) {
   if constexpr (EPI != EPI_QKV) {
     if (ntiles >= ncu && g.splitk <= 1 && g.ntb != -13 && g.ntb != -14) {
       const int nb = ncu, tneed = (ntiles + nb - 1) / nb;
-      const int nw = g.waves > 0 ? g.waves : std::min(16, KQ);
-      if (nw > 16 || tneed > nw) return false;  // (wave j finishes tile t0 + j)
+      // wave j finishes tile t0 + j, in int4 also a wave without a k-quad of its own (us, awq_gemm_kernel -> here, at 1 / 16 rows: 20480 x 512 7.4 -> 4.8 / 8.4 -> 5.2,
+      // 28672 x 256 5.7 -> 5.5 / 6.2 -> 6.0; in bf16 the tile blocks are ahead, 28672 x 512 8.1, 9.8 / 9.2, 10.2)
+      const int nw = g.waves > 0 ? g.waves : std::min(16, Q4 ? std::max(KQ, tneed) : KQ);
+      if (nw > 16 || tneed > nw) return false;
       const int kqw = (KQ + nw - 1) / nw;
       if (p.dbg_ts == nullptr) p.dbg_ts = tl_take(Q4 ? "awq_kx_wide" : "kx_wide", nb);
       p.splitk = 1;

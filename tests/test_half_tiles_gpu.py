@@ -91,7 +91,7 @@ def test_register_stationary_choice(M, N, K):
 
 
 @pytest.mark.parametrize("M", [1, 16])
-@pytest.mark.parametrize("N,K", [(20480, 512), (28672, 512), (16384, 384)])
+@pytest.mark.parametrize("N,K", [(20480, 512), (28672, 512), (16384, 384), (8192, 128), (12304, 256), (32768, 128), (32784, 640)])
 def test_int4_blocks_with_fewer_waves_than_tiles(M, N, K):
     from vgate.ops import reference as ref
     torch.manual_seed(M + N + K)
