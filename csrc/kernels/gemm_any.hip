@@ -880,17 +880,20 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st) {
       const bool f32 = g.out_f32 && !dual && g.gate == nullptr && g.N % 4 == 0 && g.ldo % 4 == 0 && g.o_bs % 4 == 0 && a16(g.out);
       // By LDS-DMA from four stages of k on (us, through registers -> by DMA: K = 64 of 3072 columns 9.5, 9.6; 12 products of 512 x 128 at 2048 rows
       // 12.9, 15.2, 16 of them 15.4, 18.8; 4096 x 256 at 1024 8.6 -> 8.3, 12 of 128 x 512 11.2, 11.3): two stages
-      // in LDS and two workgroups to a CU, or four stages where there is one at most, counting also those of groups without rows
+      // in LDS and two workgroups to a CU, or four stages where there is one at most
       // (two / four: 1024 x 4096 at 2048 rows, 128 workgroups, 47.6 -> 43.3 / 33.6; 8 experts of 1024 x 2048 with 150 rows each, 144, 28.5 -> 25.7 / 21.6,
-      // with 500, 320, 45.8 -> 33.2 / 42.2; pairs of 2048 x 1024 with 500, 64.8 -> 61.6 / 73.6; 64 uneven experts of 512 x 512 with 2300 rows, 332, some
-      // 256 of them with rows, 14.6 -> 12.5 / 16.9). Through registers a CU holds three workgroups: with more than two to a CU that wins over short K
+      // with 500, 320, 45.8 -> 33.2 / 42.2; pairs of 2048 x 1024 with 500, 64.8 -> 61.6 / 73.6). Workgroups past an expert's rows exit and do
+      // not count, but the host knows only about how many those are: in 110 drawn products four stages were ahead by 5 to 25 % wherever up to a
+      // workgroup per CU had rows (32 experts of 768 x 2944 with 46 rows each, 264, 192 of them with rows, registers 48.7, 52.3 / 39.3; 32 of 896 x 1600 with 38
+      // 30.7, 33.1 / 24.6; 8 of 1792 x 1024 with 178 19.7, 21.4 / 18.5) and behind by 10 to 25 % right above that (8 of 1344 x 2944 with 379, 264 with rows,
+      // 74.4, 58.4 / 73.5), so they are taken up to eleven twelfths of the CUs, where one estimate of the 110 was too low. Through registers a CU holds three workgroups: with more than two to a CU that wins over short K
       // (4224 x 256 with gates at 1985 rows, 528, 25.8, 32.7; 4536 x 320 28.5, 35.0; 5440 x 512 at 3324 51.0, 55.7; 5760 x 960 at 2124 51.1, 55.2; without
       // gates 2712 x 320 at 3958, fp32, 682, 20.5, 22.4, and even at 1024 x 512 of 12; 32 experts of 3072 x 576 with 38 rows each, 768, 24.7, 28.2, pairs of
       // 2176 x 640 with 51, 1088, 41.0, 45.7, of 3072 x 640 with 112 31.1, 34.0). What bounds the many is the operands' way through L2, 25 B a clock and CU.
       const int64_t blocks = (int64_t)grid2.x * grid2.y * grid2.z, cus = cu_count();
       const int64_t busy = g.group_off ? (int64_t)grid2.x * std::max(g.groups, mt128 - (g.groups + 1) / 2) : blocks;   // (experts: about so many have rows)
-      if (g.K % 64 == 0 && g.K >= 256 && (blocks <= cus || busy <= 2 * cus || g.K > (gated ? 1024 : g.group_off ? 640 : 512))) {
-        const bool few = blocks <= cus;
+      if (g.K % 64 == 0 && g.K >= 256 && (busy <= 2 * cus || g.K > (gated ? 1024 : g.group_off ? 640 : 512))) {
+        const bool few = blocks <= cus || (g.group_off && 12 * busy <= 11 * cus);
         auto by_dma = [&](auto du, auto out) {
           constexpr int DU = decltype(du)::value, O = decltype(out)::value;
           if (few) launch_any_dma<DU, 4, O>(v, grid2, st);

@@ -169,6 +169,13 @@ def test_many_experts_of_short_k(N, K):
     test_experts(N, K, [70, 0, 130, 33, 1] * 7)
 
 
+@pytest.mark.parametrize("sizes", [[70, 0, 46, 33, 1, 127, 40, 55] * 4, [33] * 31 + [1100], [128, 0, 129] * 7 + [2, 0, 0]])
+@pytest.mark.parametrize("N,K", [(768, 320), (520, 256), (896, 576)])
+def test_experts_on_a_workgroup_per_cu(N, K, sizes):
+    """More workgroups than CUs, of which some 0.7 to 1.8 per CU have rows: four stages in LDS below 11/12 of the CUs, two above."""
+    test_experts(N, K, sizes)
+
+
 @pytest.mark.parametrize("sizes", [[300, 0, 129, 1, 600], [128] * 9 + [127, 0, 2], [700] * 6])
 @pytest.mark.parametrize("N,K", [(520, 256), (1024, 320)])
 def test_experts_by_dma(N, K, sizes):
