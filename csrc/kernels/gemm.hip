@@ -149,7 +149,9 @@ static GemmParams to_params(const GemmArgs& g) {
 // hold one stage of weights ahead and stage x anew for each block's k-range, or on four-wave tiles, three to five stages in flight: 64 x
 // 64, two blocks to a CU, or 64 x 128. Whether: us, cold weights, tiles of gemm_decode.h -> four-wave tiles, at 17 / 64 rows.
 //   With a norm folded in: 8320 x 2304 22.3 -> 14.2 / 26.3 -> 15.6, 16384 x 4096 51.7 -> 27.6 / 58.1 -> 29.0, 32000 x 1536 25.4 -> 21.9 / 29.4 -> 24.0,
-//     151936 x 1536 96.2 -> 94.1 / 116 -> 114; behind at 65536 x 512 (19.9, 22.5 / 25.3, 27.4).
+//     151936 x 1536 96.2 -> 94.1 / 116 -> 114. But, not for pairs (131072 x 512 46 -> 40), K of one or two whole stages of the other kernels, 256 or 512, where their blocks of 128 columns fill
+//     whole rounds of CUs: 65536 x 512, fp32, 20.3, 22.8 / 24.8, 27.6, 98304 x 512 28.0, 30.2 / 33.4, 36.2, 128256 x 256 22.4, 23.1 / 29.5, 28.7 (49152 x 512, three halves
+//     of a round, 18.3 -> 16.6 / 21.2 -> 19.8, 151936 x 512 39.9 -> 38.8 / 49.1 -> 45.2; 65536 x 448 19.2 -> 17.3 / 23.5 -> 21.0, x 576 23.5 -> 20.0 / 28.3 -> 23.9).
 //   Without one, up to 12288 columns from 25 rows on: 8320 x 4096 20.9, 21.2 / 28.9 -> 23.7. Wider, from K = 2048 on, by how well the other kernels fill the
 //     chip. Pairs and QKV, 64 columns to a block of theirs, lose more of it with more rows: 17408 x 3072 32.1 -> 26.4 / 44.2 -> 30.9; up to 24 rows of
 //     more than 28672 columns they are even or ahead (32000 x 6144 65.9, 72.6 / 87.9 -> 75.6). Others are 128 columns wide from 16384 on, one block to a
@@ -159,10 +161,13 @@ static GemmParams to_params(const GemmArgs& g) {
 //     of 128 run on the K-split kernels, which hold up to 24 rows (23360 x 3584 34.1, 37.4 / 60.7 -> 43.9).
 static bool four_wave_fits(const GemmArgs& g) {
   if (g.norm_w != nullptr || g.N < 8192) return false;
-  if (g.rownorm) return true;
+  const int cus = cu_count_gemm();
+  if (g.rownorm) {
+    const int blocks = g.N / 128, slots = (blocks + cus - 1) / cus * cus;
+    return g.epi == EPI_SILU || g.epi == EPI_QKV || g.N % 128 != 0 || g.K > 512 || g.K % 256 != 0 || blocks <= cus || 20 * blocks <= 19 * slots;
+  }
   if (g.N <= 12288) return g.M > 24;
   if (g.K <= 2048) return false;
-  const int cus = cu_count_gemm();
   if (g.epi == EPI_SILU || g.epi == EPI_QKV) return g.M > 24 || g.N <= 112 * cus;
   if (g.N % 128 != 0) return g.M > 24;
   const int blocks = g.N / 128, slots = (blocks + cus - 1) / cus * cus;

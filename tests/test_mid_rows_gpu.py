@@ -72,6 +72,13 @@ def test_many_columns_of_a_mixed_step(M, N, K):
     assert ((got.float() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -7).all()
 
 
+@pytest.mark.parametrize("M", [17, 48])
+@pytest.mark.parametrize("N,K", [(32768, 256), (62208, 512), (62336, 512), (65536, 256), (65536, 320), (65600, 512), (98304, 512)])
+def test_heads_of_short_k_behind_a_norm(M, N, K):
+    """Blocks of 128 columns that fill whole rounds of CUs, and nearly, on either side of the lines to four-wave tiles."""
+    test_many_columns_of_a_mixed_step(M, N, K)
+
+
 @pytest.mark.parametrize("stride", [17_300_000, (1 << 25) + 8])
 @pytest.mark.parametrize("M", [17, 64])
 def test_rows_far_apart(M, stride):
