@@ -2,29 +2,34 @@
 // 4 bits and no bf16 copy is written and read back. Every fragment holds the very bf16 values of that copy ((v s - s z) gamma, rounded once),
 // and products and squares are summed in the order of the bf16 forms: the bits are theirs.
 //
-// As gemm_w4_kernel (gemm_prompt.h): four waves, one per SIMD, operands of a k-step read (here: and unpacked) during the MFMAs of the one
-// before, stages by LDS-DMA. The waves stand side by side over the columns, so that each fragment of W is unpacked by one wave of the block
-// only: unpacking is what bounds it (per fragment 23 VALU operations, 31 with gamma, against MT MFMAs of four cycles' issue and 16 cycles each),
-// hence the tiles of many rows and few columns. us, a bf16 copy and the bf16 kernels -> here (MI355X, cold weights): 256 rows, 17920 x 1536
-// with a norm 50.4 -> 39.0, 1536 x 8960 35.3 -> 27.3, 1536 x 1536 18.4 -> 14.7; 96 rows, 28672 x 4096 117 -> 52, 1536 x 8960 28.2 -> 17.8.
+// As gemm_w4_kernel (gemm_prompt.h): operands of a k-step are read (here: and unpacked) during the MFMAs of the one before, stages come by
+// LDS-DMA. The waves stand side by side over the columns, so that each fragment of W is unpacked by one wave of the block only.
+// What bounds it is the issue of vector instructions. One wave on a SIMD issues one every 5 to 6 cycles (a conversion every 8) whatever else
+// is ready; two or more take 4.3 each between MFMAs, which take 8 of issue and 16 of the matrix core. So two waves to a SIMD at least, eight
+// in a block or two to four blocks of four or eight on a CU (stages of 128 k, two or three of them as LDS allows); weights turn into floats
+// without conversions (unpack()); gamma is widened once per block and not once per wave and k-step. Per fragment 17 vector instructions, 25
+// with gamma, against MT MFMAs. LDS is next: an x fragment (8 cycles) serves NT MFMAs.
+// us, four waves with 23 and 31 instructions -> these (MI355X, cold weights, the same slices): 256 rows, 17920 x 1536 with a norm 35.1 -> 29.3,
+// 1536 x 8960 in 8 slices 27.3 -> 21.8, 1536 x 1536 11.4 -> 10.1; 448 rows, 17920 x 1536 55.9 -> 45.4, 1536 x 8960 31.6 -> 27.4; 96 rows 23.8 ->
+// 18.9 and 16.0 -> 15.5; a step of 256 rows through six layers of 1536 / 8960 694 -> 645.
 #include "gemm_prompt.h"
 
 namespace vgate {
 
-template <int MT, int NT>
-struct Q4 {  // geometry: four waves side by side, each 16 MT rows x 16 NT columns; stages of 128 k (one group)
-  static constexpr int BM = 16 * MT, BN = 64 * NT;
-  static constexpr int XB = BN * 64, SB = XB + BM * 256;  // W | x (two 64-k halves) | scales, zeros, gamma: 1 KiB each
-  static constexpr int STAGE = SB + 3072;
-  static constexpr int PPW = MT + NT + 1;  // DMA of a wave and stage
+template <int NW, int MT, int NT>
+struct Q4 {  // geometry: NW waves side by side, each 16 MT rows x 16 NT columns; stages of 128 k (one group)
+  static constexpr int BM = 16 * MT, BN = 16 * NW * NT;
+  static constexpr int XB = BN * 64, SB = XB + BM * 256;  // W | x (two 64-k halves) | scales, zeros: 1 KiB each
+  static constexpr int STAGE = SB + 2048;
+  static constexpr int XPW = 4 * MT / NW, PPW = XPW + NT + 1;  // x pieces and all DMA of a wave and stage
 };
 
-template <int MT, int NT, int NS, int EPI, bool NORM>
-__global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
-  using G = Q4<MT, NT>;
-  constexpr int PPW = G::PPW, STAGE = G::STAGE;
-  static_assert(NS * STAGE <= 160 * 1024, "LDS");
-  static_assert(NS >= 2 && (NS - 1) * PPW < 64 && (NT & (NT - 1)) == 0 && NT <= 8, "vmcnt; the block's scales repeat in 1 KiB");
+template <int NW, int MT, int NT, int NS, int EPI, bool NORM>
+__global__ __launch_bounds__(64 * NW, NW / 4) void gemm_q4_prompt_kernel(GemmParams p) {
+  using G = Q4<NW, MT, NT>;
+  constexpr int PPW = G::PPW, XPW = G::XPW, STAGE = G::STAGE;
+  static_assert(NS * STAGE <= 160 * 1024 && XPW * NW == 4 * MT, "LDS; x in equal shares");
+  static_assert(NS >= 2 && (NS - 1) * PPW < 64 && (G::BN & (G::BN - 1)) == 0 && G::BN <= 512, "vmcnt; the block's scales repeat in 1 KiB");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   TLScope tl_scope(p.dbg_ts);
   const int lane = threadIdx.x & 63, quad = lane >> 4;
@@ -41,16 +46,15 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
   const int n0 = (in / gm) * G::BN, nt0 = n0 / 16 + wid * NT;  // the wave's first column tile
   const u32x4 wrs = rsrc_words(p.wp + ((size_t)(n0 / 16) * KQ + q0) * 64);
   const u32x4 xrs = rsrc_words(p.x + (size_t)m0 * p.lda + q0 * 128);
-  // the wave's small piece: the group's scales, zeros (of the block's columns, asked for again until the 1 KiB is full) or gamma
-  const int kind = NORM ? min(wid, 2) : wid & 1;
-  const bf16_t* small = kind == 0 ? p.scales : kind == 1 ? p.zeros : p.norm_w;
-  const u32x4 srs = rsrc_words(small + (kind < 2 ? (size_t)q0 * p.N + n0 : (size_t)q0 * 128));
-  const uint32_t sstep = kind < 2 ? (uint32_t)p.N * 2u : 256u;
-  const uint32_t wvo = lane * 16, svo = (uint32_t)(lane * 16) & (kind < 2 ? 2u * G::BN - 1u : 255u);
-  uint32_t xvo[MT];  // pieces of 8 rows x 64 k: tile (piece >> 2), k half (piece >> 1) & 1, row half piece & 1
+  // the wave's small piece: the group's scales or zeros of the block's columns, asked for again until the 1 KiB is full
+  const int kind = wid & 1;
+  const u32x4 srs = rsrc_words((kind == 0 ? p.scales : p.zeros) + (size_t)q0 * p.N + n0);
+  const uint32_t sstep = (uint32_t)p.N * 2u;
+  const uint32_t wvo = lane * 16, svo = (uint32_t)(lane * 16) & (2u * G::BN - 1u);
+  uint32_t xvo[XPW];  // pieces of 8 rows x 64 k: tile (piece >> 2), k half (piece >> 1) & 1, row half piece & 1
 #pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    const int g = wid * MT + i;
+  for (int i = 0; i < XPW; ++i) {
+    const int g = wid * XPW + i;
     xvo[i] = (uint32_t)(x_piece_row(m0 + (g >> 2) * 16, g & 1, lane, p.M) - m0) * (uint32_t)p.lda * 2u + (uint32_t)x_piece_col(g & 1, lane) * 2u +
              (uint32_t)((g >> 1) & 1) * 128u;
   }
@@ -59,7 +63,7 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
   auto issue_piece = [&](int i, int st, int buf) {
     const uint32_t base = lds0 + buf * STAGE;
     if (i < NT) blds16(wrs, wvo, (uint32_t)(wid * NT + i) * wrow + (uint32_t)st * 1024u, base + (uint32_t)(wid * NT + i) * 1024u);
-    else if (i < NT + MT) blds16(xrs, xvo[i - NT], (uint32_t)st * 256u, base + G::XB + (uint32_t)(wid * MT + i - NT) * 1024u);
+    else if (i < NT + XPW) blds16(xrs, xvo[i - NT], (uint32_t)st * 256u, base + G::XB + (uint32_t)(wid * XPW + i - NT) * 1024u);
     else blds16(srs, svo, (uint32_t)st * sstep, base + G::SB + kind * 1024u);
   };
   f32x4 acc[NT][MT];
@@ -70,43 +74,54 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
       acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
       asm volatile("" : "+a"(acc[a][b]));  // (written here, well before the first mfma_acc)
     }
-  // wave w sums the squares of the row tiles w, w + 4, ...: a row in the order of K, as the bf16 forms do. It reads them again: which of the
+  // wave w sums the squares of the row tiles w, w + NW, ...: a row in the order of K, as the bf16 forms do. It reads them again: which of the
   // fragments in registers are its own would be a branch per k-step, around which the accumulators lose their place (5 to 7 times as long)
-  constexpr int SQ = NORM ? (MT + 3) / 4 : 1;
+  constexpr int SQ = NORM ? (MT + NW - 1) / NW : 1;
   float ss[SQ];
   int so[SQ];
 #pragma unroll
   for (int i = 0; i < SQ; ++i) {
     ss[i] = 0.f;
-    so[i] = min(wid + 4 * i, MT - 1) * 4096;
+    so[i] = min(wid + NW * i, MT - 1) * 4096;
   }
   uint4 wf[2][NT], xf[2][MT], wq[NT], sq[2][SQ];
-  float sc[NT], zs[NT], gam[8];
+  float sc[NT], sc4[NT], zs[NT];
+  float4 gam[2];
   const int xlo[2] = {G::XB + x_frag_off(0, lane), G::XB + x_frag_off(1, lane)};
   auto read_stage = [&](const char* sb) {  // the group's packed weights and scales
 #pragma unroll
     for (int a = 0; a < NT; ++a) {
       wq[a] = *reinterpret_cast<const uint4*>(sb + (wid * NT + a) * 1024 + lane * 16);
-      sc[a] = bf2f(*reinterpret_cast<const bf16_t*>(sb + G::SB + ((wid * NT + a) * 16 + (lane & 15)) * 2));
+      const float s = bf2f(*reinterpret_cast<const bf16_t*>(sb + G::SB + ((wid * NT + a) * 16 + (lane & 15)) * 2));
+      sc[a] = s * 0x1p24f;
+      sc4[a] = s * 0x1p20f;
       zs[a] = bf2f(*reinterpret_cast<const bf16_t*>(sb + G::SB + 1024 + ((wid * NT + a) * 16 + (lane & 15)) * 2));
     }
   };
-  auto read_gamma = [&](int u, const char* sb) {
-    if constexpr (NORM) unpack8(*reinterpret_cast<const uint4*>(sb + G::SB + 2048 + u * 64 + quad * 16), gam);
+  const char* gbase = smem + NS * STAGE + quad * 32;  // gamma of the slice, fp32
+  auto read_gamma = [&](int u, int t) {
+    if constexpr (NORM) {
+      gam[0] = *reinterpret_cast<const float4*>(gbase + t * 512 + u * 128);
+      gam[1] = *reinterpret_cast<const float4*>(gbase + t * 512 + u * 128 + 16);
+    }
   };
-  // half h of the wave's fragment of tile a at k-step u: the bf16 that the unpacked copy of the matrix would hold. (The low nibbles of a
-  // word's bytes are elements 0 4 1 5, the high ones 2 6 3 7; opaque once masked, so that each is one v_cvt_f32_ubyte away.)
+  // half h of the wave's fragment of tile a at k-step u: the bf16 that the unpacked copy of the matrix would hold. The low nibbles of a
+  // word's bytes are elements 0 4 1 5, the high ones 2 6 3 7: two of them, 16 bits apart, are a pair of f16 subnormals v 2^-24 (the high
+  // ones v 2^-20), exact, which v_fma_mix_f32 takes as they stand: v s - s z in one rounding without a conversion of v.
   auto unpack = [&](int a, int h, int u) {
     const uint32_t w = u == 0 ? wq[a].x : u == 1 ? wq[a].y : u == 2 ? wq[a].z : wq[a].w;
-    uint32_t m = (h ? w >> 4 : w) & 0x0F0F0F0Fu;
-    asm("" : "+v"(m));
-    float f[4] = {(float)(m & 0xFFu) * sc[a] - zs[a], (float)((m >> 16) & 0xFFu) * sc[a] - zs[a], (float)((m >> 8) & 0xFFu) * sc[a] - zs[a],
-                  (float)(m >> 24) * sc[a] - zs[a]};
+    const uint32_t lo = w & (h ? 0x00F000F0u : 0x000F000Fu), hi = (w >> 8) & (h ? 0x00F000F0u : 0x000F000Fu);
+    const float s = h ? sc4[a] : sc[a];
+    float f[4];
+    asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[1,0,0]" : "=v"(f[0]) : "v"(lo), "v"(s), "v"(zs[a]));
+    asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(f[1]) : "v"(lo), "v"(s), "v"(zs[a]));
+    asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[1,0,0]" : "=v"(f[2]) : "v"(hi), "v"(s), "v"(zs[a]));
+    asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(f[3]) : "v"(hi), "v"(s), "v"(zs[a]));
     if constexpr (NORM) {
-      f[0] *= gam[2 * h];
-      f[1] *= gam[2 * h + 1];
-      f[2] *= gam[2 * h + 4];
-      f[3] *= gam[2 * h + 5];
+      f[0] *= h ? gam[0].z : gam[0].x;
+      f[1] *= h ? gam[0].w : gam[0].y;
+      f[2] *= h ? gam[1].z : gam[1].x;
+      f[3] *= h ? gam[1].w : gam[1].y;
     }
     uint4& o = wf[u & 1][a];
     (h ? o.y : o.x) = pack_bf2(f[0], f[1]);
@@ -119,13 +134,13 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
   };
   // zeros in place of a stage's k half that belongs to the slice before or after (once in a slice at either end; no wave is reading it)
   auto clear = [&](char* sb, int half) {
-    for (int e = threadIdx.x; e < MT * 128; e += 256)
+    for (int e = threadIdx.x; e < MT * 128; e += 64 * NW)
       *reinterpret_cast<uint4*>(sb + G::XB + (e >> 7) * 4096 + half * 2048 + (e & 127) * 16) = make_uint4(0, 0, 0, 0);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   };
   constexpr int U = 2 * NT;  // halves of fragments of a k-step to unpack
   // the MFMAs of k-step u, a row tile at a time; between them the next k-step is read and unpacked and, at the last, the next stage asked for
-  auto phase = [&](auto uc, const char* sb, int st, int buf) {
+  auto phase = [&](auto uc, const char* sb, int t, int st, int buf) {
     constexpr int u = decltype(uc)::value, v = (u + 1) & 3;
     // (an MFMA reads what the VALU wrote two wait states before at the soonest, and the compiler does not see that mfma_acc() is one)
 #pragma unroll
@@ -135,7 +150,7 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
       wf[u & 1][a] = __builtin_bit_cast(uint4, f);
     }
     if constexpr (u == 3) read_stage(sb);
-    read_gamma(v, sb);
+    read_gamma(v, t);
 #pragma unroll
     for (int b = 0; b < MT; ++b) {
       if constexpr (NORM)
@@ -156,14 +171,32 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
   using C1 = std::integral_constant<int, 1>;
   using C2 = std::integral_constant<int, 2>;
   using C3 = std::integral_constant<int, 3>;
+  // gamma of the slice: bf16 by DMA into the second half of its place (asked for first: it has landed when the first stage has), widened there
+  if constexpr (NORM) {
+    u32x4 grs = rsrc_words(p.norm_w + (size_t)q0 * 128);
+    grs[2] = (uint32_t)nk * 256u;
+    for (int i = wid; i < (nk + 3) >> 2; i += NW) blds16(grs, wvo, (uint32_t)i * 1024u, lds0 + NS * STAGE + ((nk + 3) >> 2) * 1024 + i * 1024u);
+  }
 #pragma unroll
   for (int s0 = 0; s0 < NS; ++s0)
 #pragma unroll
     for (int i = 0; i < PPW; ++i) issue_piece(i, s0 < nk ? s0 : nk - 1, s0);
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * PPW) : "memory");
+  if constexpr (NORM) {
+    const bf16_t* raw = reinterpret_cast<const bf16_t*>(smem + NS * STAGE + ((nk + 3) >> 2) * 1024);
+    float* wide = reinterpret_cast<float*>(smem + NS * STAGE);
+    // (in place, from the front: a round of 64 NW elements is read by all before it is written, and lies behind what the next one reads)
+    for (int e0 = 0; e0 < nk * 128; e0 += 64 * NW) {
+      const int e = e0 + threadIdx.x;
+      const float g = e < nk * 128 ? bf2f(raw[e]) : 0.f;
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (e < nk * 128) wide[e] = g;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
   if (kt0 & 1) clear(smem, 0);
   read_stage(smem);
-  read_gamma(0, smem);
+  read_gamma(0, 0);
 #pragma unroll
   for (int b = 0; b < MT; ++b) read_x(b, 0, smem);
 #pragma unroll
@@ -173,12 +206,12 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
     char* sb = smem + buf * STAGE;
     const int nb = buf + 1 == NS ? 0 : buf + 1;
     if (t == nk - 1 && (kt1 & 1) != 0) clear(sb, 1);
-    phase(C0{}, sb, 0, 0);
-    phase(C1{}, sb, 0, 0);
-    phase(C2{}, sb, 0, 0);
+    phase(C0{}, sb, t, 0, 0);
+    phase(C1{}, sb, t, 0, 0);
+    phase(C2{}, sb, t, 0, 0);
     // this stage is read (its last k-step is in registers), the next one has landed: both for every wave
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * PPW) : "memory");
-    phase(C3{}, smem + nb * STAGE, t + NS < nk ? t + NS : nk - 1, buf);  // past the end: clamped duplicates, never used
+    phase(C3{}, smem + nb * STAGE, min(t + 1, nk - 1), t + NS < nk ? t + NS : nk - 1, buf);  // past the end: clamped duplicates, never used
     buf = nb;
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");  // the trailing duplicates
@@ -191,10 +224,10 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
     __syncthreads();
 #pragma unroll
     for (int b = 0; b < MT; ++b) {
-      float s2 = ss[b >> 2];
+      float s2 = ss[b / NW];
       s2 += xor16(s2);
       s2 += xor32(s2);
-      if (wid == (b & 3) && lane < 16) rows[b * 16 + lane] = s2;
+      if (wid == b % NW && lane < 16) rows[b * 16 + lane] = s2;
     }
     __syncthreads();
   }
@@ -226,22 +259,26 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_prompt_kernel(GemmParams p) {
   prompt_epilogue<NT, MT, EPI>(p, m0, nt0, lane, [&](int a, int b) { return NORM ? acc[a][b] * scale[b] : acc[a][b]; });
 }
 
+// LDS of a slice's gamma: fp32, whole KiB of its bf16 values twice over
+static int q4_gamma_lds(int K, int nz) { return (((K >> 6) + nz - 1) / nz + 2) / 2 * 512 + 2048; }
+
 template <int EPI, int NORM, int NTB>
 void launch_prefill_reduce(const GemmParams& p, int nz, hipStream_t st);
 
-template <int MT, int NT, int NS, int EPI, bool NORM>
+template <int NW, int MT, int NT, int NS, int EPI, bool NORM>
 static bool launch_q4_one(const GemmParams& p, int nz, hipStream_t st) {
-  using G = Q4<MT, NT>;
-  if (p.N % G::BN != 0) return false;
+  using G = Q4<NW, MT, NT>;
+  const int lds = NS * G::STAGE + (NORM ? q4_gamma_lds(p.K, nz) : 0);
+  if (p.N % G::BN != 0 || lds > 160 * 1024) return false;
   const int blocks = ((p.M + G::BM - 1) / G::BM) * (p.N / G::BN);
   GemmParams q = p;
   if (q.dbg_ts == nullptr) q.dbg_ts = tl_take("gemm_q4_prompt", blocks * nz);
-  auto kern = gemm_q4_prompt_kernel<MT, NT, NS, EPI, NORM>;
+  auto kern = gemm_q4_prompt_kernel<NW, MT, NT, NS, EPI, NORM>;
   static bool attr = [&] {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, NS * G::STAGE) == hipSuccess;
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
   }();
   (void)attr;
-  hipLaunchKernelGGL(kern, dim3(blocks, nz), dim3(256), NS * G::STAGE, st, q);
+  hipLaunchKernelGGL(kern, dim3(blocks, nz), dim3(64 * NW), lds, st, q);
   if (nz > 1) launch_prefill_reduce<EPI, NORM ? 2 : 0, 1>(p, nz, st);
   return true;
 }
@@ -249,39 +286,43 @@ static bool launch_q4_one(const GemmParams& p, int nz, hipStream_t st) {
 template <int EPI, bool NORM>
 static bool launch_q4_epi(const GemmParams& p, int code, int nz, hipStream_t st) {
   switch (code) {
-#define VG_Q4(MT, NT, NS) case 100 * MT + 10 * NT: return launch_q4_one<MT, NT, NS, EPI, NORM>(p, nz, st)
-    VG_Q4(4, 1, 3);  // two blocks to a CU
-    VG_Q4(6, 1, 3);
-    VG_Q4(6, 2, 4);
-    VG_Q4(8, 2, 3);
-    VG_Q4(10, 2, 3);
-    VG_Q4(16, 2, 2);
-    VG_Q4(6, 4, 3);
+#define VG_Q4(C, NW, MT, NT, NS) case C: return launch_q4_one<NW, MT, NT, NS, EPI, NORM>(p, nz, st)
+    VG_Q4(410, 4, 4, 1, 3);
+    VG_Q4(412, 4, 4, 1, 2);
+    VG_Q4(422, 8, 4, 1, 2);
+    VG_Q4(610, 4, 6, 1, 2);
+    VG_Q4(620, 8, 6, 1, 2);
+    VG_Q4(640, 8, 6, 2, 3);
+    VG_Q4(820, 8, 8, 1, 3);
+    VG_Q4(1020, 8, 10, 1, 3);
+    VG_Q4(1620, 4, 16, 2, 2);
 #undef VG_Q4
   }
   return false;
 }
 
 // Costs (us) as in choose_prefill_form() of gemm_prefill.hip, fitted to 15 shapes (N 512 .. 28672, K 1024 .. 14336) x 10 row counts 65 ..
-// 2048 on cold weights; K-tiles of 128. Unpacking is repeated by every row of blocks, so from some row count on a bf16 copy (2.2 us + 0.56
-// a million weights) and the bf16 kernels are ahead: 17920 x 1536 at 448 rows 60 against 64 us, at 1024 114 against 89; 1536 x 1536 at 1024 17
-// against 22. Free in its slices the choice took 1.019 of the best form's time, and 1 / 1.26 of the copy's (geometric means); with the cut of K
-// given, a step of 256 rows through six layers of 1536 / 8960 takes 737 us instead of 734 (947 with copies), one of 320 rows 795 instead of 745.
+// 2048 on cold weights; K-tiles of 128, rounds of as many blocks to a CU as their stages leave room for. Unpacking is repeated by every row
+// of blocks, so from some row count on a bf16 copy (2.2 us + 0.56 a million weights) and the bf16 kernels are ahead. Given the slices, the
+// choice takes 1.004 of the best tile's time (geometric mean). The copy's estimate is 1.15 times what it takes at 1000 rows and more (6144 x
+// 4096 with a norm at 2048 rows: 122 us, this kernel 140), hence the factor; of 21 shapes x 8 row counts the worst choice is 1.03 of the other.
 Q4Form q4_prompt_form(int M, int N, int K, bool norm, bool rows16, bool group128, size_t slab_bytes, int code, int sk) {
   struct Tile {
-    int code, bm, bn, per_cu;
+    int code, bm, bn, stages;
     struct {
-      float e, a, b, c, d, w, o;
+      float e, a, b, g, c, d, w, o;
     } cost[2];  // plain, with a norm in front
   };
   static constexpr Tile tiles[] = {
-      {410, 64, 64, 2, {{8.3f, 0.907f, 0.415f, 1.87f, 0.328f, 0.009f, 0.f}, {9.35f, 0.883f, 0.547f, 1.75f, 0.232f, 0.006f, 0.f}}},
-      {610, 96, 64, 1, {{5.99f, 2.07f, 0.594f, 2.46f, 0.434f, 0.f, 0.405f}, {6.74f, 2.86f, 0.81f, 2.26f, 0.299f, 0.f, 0.341f}}},
-      {620, 96, 128, 1, {{7.29f, 3.86f, 0.989f, 1.5f, 0.339f, 0.f, 0.087f}, {7.68f, 4.57f, 1.25f, 1.4f, 0.293f, 0.f, 0.113f}}},
-      {820, 128, 128, 1, {{7.92f, 3.83f, 1.15f, 1.06f, 0.358f, 0.f, 0.217f}, {8.51f, 5.2f, 1.41f, 0.477f, 0.298f, 0.f, 0.144f}}},
-      {1020, 160, 128, 1, {{8.98f, 4.86f, 1.31f, 0.152f, 0.336f, 0.f, 0.151f}, {9.24f, 6.01f, 1.59f, 0.f, 0.29f, 0.f, 0.154f}}},
-      {1620, 256, 128, 1, {{10.5f, 4.19f, 1.84f, 0.f, 0.347f, 0.f, 0.339f}, {10.9f, 5.22f, 2.17f, 0.f, 0.325f, 0.f, 0.426f}}},
-      {640, 96, 256, 1, {{8.39f, 5.55f, 1.74f, 0.353f, 0.343f, 0.f, 0.082f}, {8.99f, 6.65f, 2.09f, 0.f, 0.287f, 0.f, 0.079f}}}};
+      {410, 64, 64, 3, {{3.09f, 0.61f, 0.181f, 0.285f, 1.84f, 0.675f, 0.026f, 0.466f}, {3.43f, 0.809f, 0.288f, 0.371f, 2.8f, 0.515f, 0.031f, 0.467f}}},
+      {412, 64, 64, 2, {{2.65f, 0.f, 0.122f, 0.431f, 2.26f, 0.645f, 0.051f, 0.534f}, {3.79f, 0.f, 0.237f, 0.446f, 2.77f, 0.523f, 0.042f, 0.467f}}},
+      {422, 64, 128, 2, {{3.12f, 0.101f, 0.376f, 0.282f, 3.72f, 0.47f, 0.035f, 0.382f}, {4.15f, 0.511f, 0.591f, 0.264f, 3.55f, 0.447f, 0.018f, 0.322f}}},
+      {610, 96, 64, 2, {{2.88f, 0.042f, 0.154f, 0.473f, 2.29f, 0.652f, 0.042f, 0.553f}, {4.46f, 0.f, 0.323f, 0.481f, 2.67f, 0.524f, 0.031f, 0.513f}}},
+      {620, 96, 128, 2, {{3.67f, 0.442f, 0.513f, 0.251f, 3.35f, 0.511f, 0.025f, 0.413f}, {3.21f, 2.03f, 0.678f, 0.261f, 3.37f, 0.491f, 0.019f, 0.439f}}},
+      {640, 96, 256, 3, {{2.63f, 3.97f, 1.22f, 0.f, 3.06f, 0.409f, 0.012f, 0.298f}, {2.59f, 4.58f, 1.55f, 0.f, 3.65f, 0.371f, 0.008f, 0.27f}}},
+      {820, 128, 128, 3, {{2.16f, 2.88f, 0.848f, 0.f, 2.99f, 0.541f, 0.015f, 0.491f}, {2.19f, 3.49f, 1.08f, 0.f, 3.37f, 0.49f, 0.016f, 0.456f}}},
+      {1020, 160, 128, 3, {{1.6f, 3.67f, 1.f, 0.f, 3.23f, 0.499f, 0.021f, 0.47f}, {2.15f, 3.61f, 1.39f, 0.f, 3.92f, 0.43f, 0.016f, 0.412f}}},
+      {1620, 256, 128, 2, {{2.5f, 3.31f, 0.f, 1.64f, 3.07f, 0.497f, 0.013f, 0.481f}, {3.12f, 4.23f, 2.03f, 0.f, 3.22f, 0.436f, 0.004f, 0.427f}}}};
   // columns of the form's tiles; a width that N is no multiple of: launch_gemm() goes on to the kernels of gemm_decode.h
   const int width = code >= 5000 ? code / 10 % 10 * 32 : code == 1024 || code == 1025 || code == 512 ? 256 : code == 2560 ? 512 :
                     code == 2561 ? 320 : code == 256 || code == 768 || code == 769 || code == 1280 || code == 1281 ? 128 : 64;
@@ -299,14 +340,16 @@ Q4Form q4_prompt_form(int M, int N, int K, bool norm, bool rows16, bool group128
   const PrefillForm copy = prefill_form_cut(M, N, K, norm, rows16, slab_bytes, nz);
   Q4Form best = copy.us < 1e30f ? Q4Form{1, copy.code, nz} : Q4Form{code == 0 ? 6 : 1, code, sk};
   if (!group128 || !rows16 || K % 128 != 0) return best;
-  float least = 2.2f + 0.56f * weights + copy.us;
+  float least = 0.87f * (2.2f + 0.56f * weights + copy.us);
   auto over = [](int64_t x, int64_t y) { return (int)((x + y - 1) / y); };
   for (const Tile& t : tiles) {
+    const int kts = over(K / 128, nz), per_cu = 160 * 1024 / (t.stages * (t.bn * 64 + t.bm * 256 + 2048) + (norm ? q4_gamma_lds(K, nz) : 0));
+    if (N % t.bn != 0 || per_cu == 0) continue;
     const int64_t blocks = (int64_t)over(M, t.bm) * (N / t.bn) * nz;
-    if (N % t.bn != 0) continue;
     const auto& x = t.cost[norm ? 1 : 0];
-    const float us = x.e + x.a * over(blocks, (int64_t)cus * t.per_cu) + x.b * over(blocks, cus) * over(K / 128, nz) + x.w * 2.f * weights +
-                     x.o * omb + (nz > 1 ? x.c + x.d * 2.f * nz * omb : 0.f);
+    const int rounds = over(blocks, (int64_t)cus * min(per_cu, 4));
+    const float us = x.e + x.a * rounds + (x.b * over(blocks, cus) + x.g * rounds) * kts + x.w * 2.f * weights + x.o * omb +
+                     (nz > 1 ? x.c + x.d * 2.f * nz * omb : 0.f);
     if (us < least) {
       least = us;
       best = Q4Form{5, t.code, nz};

@@ -1329,6 +1329,34 @@ def test_awq_prompt_tiles(code, M, K, sk, norm):
     assert ((out.double() - want).norm() / want.norm()).item() < (K + 8) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("code", [412, 422])
+@pytest.mark.parametrize("M,K,sk", [(1, 128, 1), (65, 256, 1), (97, 640, 2), (577, 1536, 3)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_awq_prompt_two_stage_tiles(code, M, K, sk, norm):
+    test_awq_prompt_tiles(code, M, K, sk, norm)
+
+
+@pytest.mark.parametrize("code", [410, 412, 422, 610, 620, 640, 820, 1020, 1620])
+def test_awq_prompt_weights_are_those_of_the_copy(code):
+    """Every nibble, scales from 2^-130 (subnormal) to 2^100, zeros between the steps, gammas of both signs, an odd number of groups (an
+    incomplete KiB of gamma): the bits of the bf16 copy on a bf16 kernel, whose K is summed in the same order."""
+    C, N, K, M = ops.native(), 256, 640, 70
+    g = torch.Generator().manual_seed(code)
+    lin = ops.Linear(None, awq=dict(qint=(torch.arange(N * K, dtype=torch.int32) * 7 % 16).view(N, K), group=128, zeros=torch.zeros(K // 128, N, device=DEV),
+                                    scales=torch.ones(K // 128, N, dtype=torch.bfloat16, device=DEV)))
+    lin.scales.copy_((torch.rand(K // 128, N, generator=g) + 1.0) * 2.0 ** torch.randint(-130, 100, (K // 128, N), generator=g).float())
+    lin.zeros.copy_(lin.scales.float().cpu() * torch.rand(K // 128, N, generator=g) * 15)
+    gamma = torch.randn(K, generator=g).bfloat16().to(DEV)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    copy = torch.empty(N * K, dtype=torch.bfloat16, device=DEV)
+    C.awq_dequant(lin.wp, lin.scales, lin.zeros, N, K, 128, copy, gamma)
+    out, want = torch.empty(M, N, device=DEV), torch.empty(M, N, device=DEV)
+    C.gemm(x, lin.wp, N, K, out, 1, ws=ops.workspace(DEV), ntb=code, splitk=1, path=5, awq_scales=lin.scales, awq_zeros=lin.zeros, group=128,
+           norm_w=gamma, eps=1e-6)
+    C.gemm(x, copy, N, K, want, 1, ws=ops.workspace(DEV), path=1, ntb=641, splitk=1, rownorm=True, eps=1e-6)
+    assert torch.equal(out, want) and torch.isfinite(out).all()
+
+
 @pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("M,K,sk", [(65, 256, 1), (97, 640, 2), (130, 1152, 4), (300, 1536, 3), (577, 1664, 6)])
 def test_awq_prompt_tiles_give_the_bits_of_the_copied_matrix(M, K, sk, norm):
