@@ -43,6 +43,7 @@
 
 #include "lds_rows.h"
 #include "locate.h"
+#include "row_norm.h"
 #include "seq_launchers.h"
 
 namespace vgate {
@@ -68,35 +69,42 @@ __device__ __forceinline__ float turned(const LatentArgs& a, const void* x, int6
   return second ? (v * cs + u * sn) : (u * cs - v * sn);
 }
 
-__global__ __launch_bounds__(256) void latent_write_kernel(LatentArgs a, const void* __restrict__ kv, int64_t ldkv,
-                                                            const float* __restrict__ w, float eps,
-                                                            bf16_t* __restrict__ cache_t, int page) {
+// grid (token, 2 with the query's latent): the key's row and the query's norm read the same projection and nothing of each other, so
+// they share a launch (us, latents of 256 and 512, two launches -> one: 32 rows 4.7 + 3.9 -> 4.2, 2048 rows 8.4 + 5.9 -> 9.9). NI columns of the query's latent per thread in registers.
+template <int NI>
+__global__ __launch_bounds__(256) void latent_write_kernel(LatentArgs a, LatentWriteArgs b) {
   __shared__ float red[16];
   const int t = blockIdx.x;
+  if (blockIdx.y == 1) {  // (uniform)
+    const int64_t src = t * b.ldq, dst = (int64_t)t * b.qn;
+    float v[NI], w[NI];
+    load_row(b.qx, src, a.f32, b.qn, v);
+    load_row(b.qw, 0, 1, b.qn, w);
+    norm_row(v, b.qn, b.eps, 0, red, [&](int c) { return ldx(b.qx, src + c, a.f32); },
+             [&](int c, int i, float r) { stx(b.qy, dst + c, a.f32, r * (i >= 0 ? w[i] : b.qw[c])); });
+    return;
+  }
   const int slot = a.slots[t];
   if (slot < 0) return;  // uniform per block
-  const int64_t src = (int64_t)t * ldkv;
+  const int64_t src = t * b.ldkv;
   const int64_t dst = (int64_t)slot * (a.rank + a.rot);
-  float ss = 0.f;
-  for (int c = threadIdx.x; c < a.rank; c += blockDim.x) {
-    const float v = ldx(kv, src + c, a.f32);
-    ss = fmaf(v, v, ss);
-  }
-  ss = block_reduce_sum(ss, red);
-  const float inv = 1.f / sqrtf(ss / (float)a.rank + eps);
-  for (int c = threadIdx.x; c < a.rank; c += blockDim.x) {
-    const float v = ldx(kv, src + c, a.f32) * inv * w[c];
-    stx(a.cache, dst + c, a.f32, v);
+  bf16_t* cache_t = reinterpret_cast<bf16_t*>(b.cache_t);
+  float v[2], w[2];
+  load_row(b.kv, src, a.f32, a.rank, v);
+  load_row(b.w, 0, 1, a.rank, w);
+  norm_row(v, a.rank, b.eps, 0, red, [&](int c) { return ldx(b.kv, src + c, a.f32); }, [&](int c, int i, float r) {
+    r *= i >= 0 ? w[i] : b.w[c];
+    stx(a.cache, dst + c, a.f32, r);
     if (cache_t != nullptr)  // [page][column][key in page]
-      cache_t[((int64_t)(slot / page) * a.rank + c) * page + slot % page] = f2bf(v);
-  }
+      cache_t[((int64_t)(slot / b.page) * a.rank + c) * b.page + slot % b.page] = f2bf(r);
+  });
   const float pos = (float)a.positions[t];
   for (int i = threadIdx.x; i < a.rot; i += blockDim.x) {
     float o;
     if (i < a.rot_dims) {
-      o = turned(a, kv, src + a.rank, i, pos);
+      o = turned(a, b.kv, src + a.rank, i, pos);
     } else {
-      o = ldx(kv, src + a.rank + i, a.f32);
+      o = ldx(b.kv, src + a.rank + i, a.f32);
     }
     stx(a.cache, dst + a.rank + i, a.f32, o);
   }
@@ -973,11 +981,12 @@ bool mfma_takes(int rank, int rot, int f32, int page) {
 
 }  // namespace
 
-void launch_latent_write(const LatentArgs& a, const void* kv, int64_t ldkv, const float* w, float eps, void* cache_t,
-                         int page, hipStream_t st) {
+void launch_latent_write(const LatentArgs& a, const LatentWriteArgs& w, hipStream_t st) {
   if (a.T <= 0) return;
-  hipLaunchKernelGGL(latent_write_kernel, dim3(a.T), dim3(256), 0, st, a, kv, ldkv, w, eps,
-                     reinterpret_cast<bf16_t*>(cache_t), page);
+  const dim3 grid(a.T, w.qn > 0 ? 2 : 1);
+  if (w.qn <= 512) hipLaunchKernelGGL(latent_write_kernel<2>, grid, dim3(256), 0, st, a, w);
+  else if (w.qn <= 1024) hipLaunchKernelGGL(latent_write_kernel<4>, grid, dim3(256), 0, st, a, w);
+  else hipLaunchKernelGGL(latent_write_kernel<8>, grid, dim3(256), 0, st, a, w);
 }
 
 void launch_latent_qrope(const LatentArgs& a, const void* q, int H, int dim, void* qa, hipStream_t st) {

@@ -11,6 +11,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "row_norm.h"
 #include "seq_launchers.h"
 
 namespace vgate {
@@ -25,60 +26,76 @@ __device__ __forceinline__ void stx(void* p, int64_t i, int f32, float v) {
 }
 __device__ __forceinline__ float sigm(float x) { return 1.f / (1.f + expf(-x)); }
 
+// A row per workgroup, read once: what bounds a few rows is how often memory is waited for (once for each sum, for the result and for its
+// weights before: 32 rows of 1024 3.9 -> 3.6 us, of 1536 5.3 -> 5.0, launch included).
+template <int NI>
 __global__ __launch_bounds__(256) void norm_rows_kernel(const void* __restrict__ x, int64_t ldx_, int x_f32,
                                                          const int32_t* __restrict__ rows,
                                                          const float* __restrict__ w, int w_scalar, float eps, int center,
                                                          void* __restrict__ y, int64_t ldy, int y_f32, int n) {
   __shared__ float red[16];
   const int m = blockIdx.x;
-  const int64_t src = rows ? rows[m] : m;
-  const int64_t xo = src * ldx_;
-  float mean = 0.f;
-  if (center) {  // (uniform)
-    float s = 0.f;
-    for (int c = threadIdx.x; c < n; c += blockDim.x) s += ldx(x, xo + c, x_f32);
-    mean = block_reduce_sum(s, red) / (float)n;
+  const int64_t xo = (rows ? rows[m] : m) * ldx_, yo = m * ldy;
+  float v[NI], wv[NI];
+  load_row(x, xo, x_f32, n, v);
+  if (w_scalar) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) wv[i] = w[0];
+  } else {
+    load_row(w, 0, 1, n, wv);
   }
-  float ss = 0.f;
-  for (int c = threadIdx.x; c < n; c += blockDim.x) {
-    const float v = ldx(x, xo + c, x_f32) - mean;
-    ss = fmaf(v, v, ss);
-  }
-  ss = block_reduce_sum(ss, red);
-  const float inv = 1.f / sqrtf(ss / (float)n + eps);
-  const float ws = w_scalar ? w[0] : 1.f;
-  for (int c = threadIdx.x; c < n; c += blockDim.x) {
-    const float v = (ldx(x, xo + c, x_f32) - mean) * inv * (w_scalar ? ws : w[c]);
-    stx(y, (int64_t)m * ldy + c, y_f32, v);
-  }
+  norm_row(v, n, eps, center, red, [&](int c) { return ldx(x, xo + c, x_f32); },
+           [&](int c, int i, float r) { stx(y, yo + c, y_f32, r * (i >= 0 ? wv[i] : w[w_scalar ? 0 : c])); });
 }
 
-__global__ __launch_bounds__(256) void embed_rows_kernel(const int32_t* __restrict__ ids,
-                                                          const int32_t* __restrict__ prev,
-                                                          const void* __restrict__ table, int t_f32, float scale,
-                                                          float* __restrict__ x, int W, int vocab) {
-  const int t = blockIdx.x;
-  int tok = ids[t];
-  if (tok < 0 && prev != nullptr) tok = prev[-tok - 1];
-  const bool ok = tok >= 0 && tok < vocab;
-  for (int c = threadIdx.x; c < W; c += blockDim.x)
-    x[(int64_t)t * W + c] = ok ? ldx(table, (int64_t)tok * W + c, t_f32) * scale : 0.f;
+// A row per workgroup: the stream's row, and beside it what the first sublayers read of it (EmbedArgs), in place of a launch that reads
+// the row again (us, 1024 wide, two launches -> one: 32 rows 3.4 + 3.9 -> 5.1, 2048 rows 6.5 + 5.9 -> 9.1).
+template <int NI>
+__global__ __launch_bounds__(256) void embed_rows_kernel(EmbedArgs a) {
+  __shared__ float red[16];
+  const int t = blockIdx.x, W = a.W;
+  int tok = a.ids[t];
+  if (tok < 0 && a.prev != nullptr) tok = a.prev[-tok - 1];
+  const bool ok = tok >= 0 && tok < a.vocab;
+  const int64_t src = (int64_t)(ok ? tok : 0) * W, ro = (int64_t)t * W;
+  auto value = [&](int c) { return ok ? ldx(a.table, src + c, a.t_f32) * a.scale : 0.f; };
+  float v[NI], n1[NI], n2[NI];
+  load_row(a.table, src, a.t_f32, W, v);
+  if (a.n1 != nullptr && !a.scalar) load_row(a.n1, 0, 1, W, n1);
+  if (a.n2 != nullptr) load_row(a.n2, 0, 1, W, n2);
+#pragma unroll
+  for (int i = 0; i < NI; ++i) v[i] = ok ? v[i] * a.scale : 0.f;
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+    if ((int)threadIdx.x + 256 * i < W) a.x[ro + threadIdx.x + 256 * i] = v[i];
+  for (int c = threadIdx.x + 256 * NI; c < W; c += 256) a.x[ro + c] = value(c);
+  if (a.h1 == nullptr) return;  // (uniform)
+  if (a.n1 == nullptr) {        // a copy
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      if ((int)threadIdx.x + 256 * i < W) stx(a.h1, ro + threadIdx.x + 256 * i, a.h_f32, v[i]);
+    for (int c = threadIdx.x + 256 * NI; c < W; c += 256) stx(a.h1, ro + c, a.h_f32, value(c));
+    return;
+  }
+  norm_row(v, W, a.eps, a.center, red, value, [&](int c, int i, float r) {
+    stx(a.h1, ro + c, a.h_f32, r * (a.scalar ? a.n1[0] : i >= 0 ? n1[i] : a.n1[c]));
+    if (a.n2 != nullptr) stx(a.h2, ro + c, a.h_f32, r * (i >= 0 ? n2[i] : a.n2[c]));
+  });
 }
 
 // One workgroup per token. Every operand's loads of NI columns a thread stand together, outside of per-element conditions, so that
-// memory is waited for once per operand that may be missing instead of once per element (32 rows of 1024: 9.9 -> 4.6 us).
+// memory is waited for once per operand that may be missing instead of once per element (32 rows of 1024: 9.9 -> 4.6 us). With h the
+// new row's norm is made here too, in place of a launch that reads the row again (32 rows
+// 3.7 + 3.9 -> 5.8 us, 2048 rows 9.7 + 5.9 -> 13.0).
 template <int NI, bool F32>
-__global__ __launch_bounds__(256) void gated_residual_kernel(float* __restrict__ x, const void* __restrict__ y1,
-                                                              const void* __restrict__ g1, int64_t ldg1,
-                                                              const float* __restrict__ b1,
-                                                              const void* __restrict__ y2,
-                                                              const void* __restrict__ g2, int64_t ldg2,
-                                                              const float* __restrict__ b2, int W) {
-  const int t = blockIdx.x;
+__global__ __launch_bounds__(256) void gated_residual_kernel(GatedArgs a) {
+  __shared__ float red[16];
+  const int t = blockIdx.x, W = a.W;
   const int64_t ro = (int64_t)t * W;
-  for (int c0 = threadIdx.x; c0 < W; c0 += 256 * NI) {   // (columns past W: the last one's values, never stored)
+  float* __restrict__ x = a.x;
+  auto pass = [&](int c0, float (&xo)[NI]) {   // (columns past W: the last one's values, never stored)
     int c[NI];
-    float xo[NI], v[NI], u[NI], a1[NI], a2[NI], d1[NI], d2[NI];
+    float v[NI], u[NI], a1[NI], a2[NI], d1[NI], d2[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       c[i] = min(c0 + 256 * i, W - 1);
@@ -87,35 +104,41 @@ __global__ __launch_bounds__(256) void gated_residual_kernel(float* __restrict__
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       xo[i] = x[ro + c[i]];
-      v[i] = ldx(y1, ro + c[i], F32 ? 1 : 0);
+      v[i] = ldx(a.y1, ro + c[i], F32 ? 1 : 0);
     }
-    if (y2 != nullptr)
+    if (a.y2 != nullptr)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) u[i] = ldx(y2, ro + c[i], F32 ? 1 : 0);
-    if (g1 != nullptr)
+      for (int i = 0; i < NI; ++i) u[i] = ldx(a.y2, ro + c[i], F32 ? 1 : 0);
+    if (a.g1 != nullptr)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) a1[i] = ldx(g1, (int64_t)t * ldg1 + c[i], F32 ? 1 : 0);
-    if (g2 != nullptr)
+      for (int i = 0; i < NI; ++i) a1[i] = ldx(a.g1, (int64_t)t * a.ldg1 + c[i], F32 ? 1 : 0);
+    if (a.g2 != nullptr)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) a2[i] = ldx(g2, (int64_t)t * ldg2 + c[i], F32 ? 1 : 0);
-    if (g1 != nullptr && b1 != nullptr)
+      for (int i = 0; i < NI; ++i) a2[i] = ldx(a.g2, (int64_t)t * a.ldg2 + c[i], F32 ? 1 : 0);
+    if (a.g1 != nullptr && a.b1 != nullptr)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) d1[i] = b1[c[i]];
-    if (g2 != nullptr && b2 != nullptr)
+      for (int i = 0; i < NI; ++i) d1[i] = a.b1[c[i]];
+    if (a.g2 != nullptr && a.b2 != nullptr)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) d2[i] = b2[c[i]];
+      for (int i = 0; i < NI; ++i) d2[i] = a.b2[c[i]];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      if (g1 != nullptr) v[i] *= sigm(a1[i] + d1[i]);
-      if (g2 != nullptr) u[i] *= sigm(a2[i] + d2[i]);
-      if (c0 + 256 * i < W) x[ro + c[i]] = xo[i] + (v[i] + u[i]);
+      if (a.g1 != nullptr) v[i] *= sigm(a1[i] + d1[i]);
+      if (a.g2 != nullptr) u[i] *= sigm(a2[i] + d2[i]);
+      xo[i] += v[i] + u[i];
+      if (c0 + 256 * i < W) x[ro + c[i]] = xo[i];
     }
+  };
+  float keep[NI];
+  pass(threadIdx.x, keep);
+  for (int c0 = threadIdx.x + 256 * NI; c0 < W; c0 += 256 * NI) {
+    float more[NI];
+    pass(c0, more);
   }
-}
-
-__global__ __launch_bounds__(256) void cast_rows_kernel(const float* __restrict__ x, bf16_t* __restrict__ y, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) y[i] = f2bf(x[i]);
+  if (a.h == nullptr) return;  // (uniform)
+  const float w = a.norm[0];
+  norm_row(keep, W, a.eps, 0, red, [&](int c) { return x[ro + c]; },
+           [&](int c, int, float r) { stx(a.h, ro + c, F32 ? 1 : 0, r * w); });
 }
 
 // out[t][j] = act(gu[t][j]) * gu[t][n + j] for a stacked [gate; up] projection (bf16), 8 columns per thread
@@ -696,13 +719,6 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const void* __restrict
 
 }  // namespace
 
-void launch_cast_rows(const float* x, void* y, int T, int n, hipStream_t st) {
-  const int64_t tot = (int64_t)T * n;
-  if (tot <= 0) return;
-  hipLaunchKernelGGL(cast_rows_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, x,
-                     reinterpret_cast<bf16_t*>(y), tot);
-}
-
 void launch_glu_rows(const void* gu, int64_t ldg, void* out, int64_t ldo, int T, int n, int act, float limit, float alpha,
                      hipStream_t st) {
   const int64_t total = (int64_t)T * (n / 8);
@@ -799,27 +815,29 @@ void launch_post_norm_add(const PostNormArgs& a, hipStream_t st) {
 
 void launch_norm_rows(const void* x, int64_t ldx_, int x_f32, const int32_t* rows, const float* w, int w_scalar,
                       float eps, int center, void* y, int64_t ldy, int y_f32, int M, int n, hipStream_t st) {
-  if (M <= 0) return;
-  hipLaunchKernelGGL(norm_rows_kernel, dim3(M), dim3(256), 0, st, x, ldx_, x_f32, rows, w, w_scalar, eps, center, y, ldy,
-                     y_f32, n);
+  if (M <= 0 || n <= 0) return;
+  row_columns<8>((n + 255) / 256, [&](auto ni) {
+    hipLaunchKernelGGL(norm_rows_kernel<decltype(ni)::value>, dim3(M), dim3(256), 0, st, x, ldx_, x_f32, rows, w, w_scalar, eps, center,
+                       y, ldy, y_f32, n);
+  });
 }
 
-void launch_embed_rows(const int32_t* ids, const int32_t* prev, const void* table, int t_f32, float scale, float* x, int T,
-                       int W, int vocab, hipStream_t st) {
-  if (T <= 0) return;
-  hipLaunchKernelGGL(embed_rows_kernel, dim3(T), dim3(256), 0, st, ids, prev, table, t_f32, scale, x, W, vocab);
+void launch_embed_rows(const EmbedArgs& a, hipStream_t st) {
+  if (a.T <= 0 || a.W <= 0) return;
+  row_columns<8>((a.W + 255) / 256, [&](auto ni) {
+    hipLaunchKernelGGL(embed_rows_kernel<decltype(ni)::value>, dim3(a.T), dim3(256), 0, st, a);
+  });
 }
 
-void launch_gated_residual(float* x, const void* y1, const void* g1, int64_t ldg1, const float* b1, const void* y2,
-                           const void* g2, int64_t ldg2, const float* b2, int f32, int T, int W, hipStream_t st) {
-  if (T <= 0) return;
+void launch_gated_residual(const GatedArgs& a, hipStream_t st) {
+  if (a.T <= 0 || a.W <= 0) return;
   // the fewest columns per thread that take no more passes than four do (2048 rows, us with four / the fewest: 256 wide 6.5, 4.3, 1536
   // wide 13.2, 11.5)
-  const int passes = (W + 1023) / 1024;
-  row_columns<4>((W + 256 * passes - 1) / (256 * passes), [&](auto ni) {
+  const int passes = (a.W + 1023) / 1024;
+  row_columns<4>((a.W + 256 * passes - 1) / (256 * passes), [&](auto ni) {
     constexpr int NI = decltype(ni)::value;
-    auto kern = f32 ? gated_residual_kernel<NI, true> : gated_residual_kernel<NI, false>;
-    hipLaunchKernelGGL(kern, dim3(T), dim3(256), 0, st, x, y1, g1, ldg1, b1, y2, g2, ldg2, b2, W);
+    auto kern = a.f32 ? gated_residual_kernel<NI, true> : gated_residual_kernel<NI, false>;
+    hipLaunchKernelGGL(kern, dim3(a.T), dim3(256), 0, st, a);
   });
 }
 

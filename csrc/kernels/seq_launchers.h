@@ -37,15 +37,30 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st);
 // row's mean is taken off first (the variance is the mean of the squared deviations)
 void launch_norm_rows(const void* x, int64_t ldx, int x_f32, const int32_t* rows, const float* w, int w_scalar,
                       float eps, int center, void* y, int64_t ldy, int y_f32, int M, int n, hipStream_t st);
-// x[t][:] = table[id(t)][:] * scale as fp32; ids < 0 name the previous step's sample prev[-id - 1]
-void launch_embed_rows(const int32_t* ids, const int32_t* prev, const void* table, int t_f32, float scale, float* x, int T,
-                       int W, int vocab, hipStream_t st);
-// x += y1 * sigmoid(g1 + b1) [+ y2 * sigmoid(g2 + b2)]; null g: plain add
-void launch_gated_residual(float* x, const void* y1, const void* g1, int64_t ldg1, const float* b1, const void* y2,
-                           const void* g2, int64_t ldg2, const float* b2, int f32, int T, int W, hipStream_t st);
+// x[t][:] = table[id(t)][:] * scale as fp32; ids < 0 name the previous step's sample prev[-id - 1] (ids outside the table: zeros).
+// With h1 what the first sublayers read of the row: without n1 a copy, else norm(x[t]) * n1 (one number if `scalar`, else [W]; center: a
+// layer norm) and, with n2, h2[t] = norm(x[t]) * n2
+struct EmbedArgs {
+  const int32_t* ids = nullptr; const int32_t* prev = nullptr;
+  const void* table = nullptr; int t_f32 = 0; float scale = 1.f;
+  float* x = nullptr;
+  int T = 0, W = 0, vocab = 0;
+  const float* n1 = nullptr; const float* n2 = nullptr;
+  int scalar = 0, center = 0; float eps = 0.f;
+  void* h1 = nullptr; void* h2 = nullptr; int h_f32 = 0;
+};
+void launch_embed_rows(const EmbedArgs& a, hipStream_t st);
+// x += y1 * sigmoid(g1 + b1) [+ y2 * sigmoid(g2 + b2)]; null g: plain add. With h (of y1's dtype): h[t] = x[t] / sqrt(mean(x[t]^2) + eps)
+// * norm[0] from the new row
+struct GatedArgs {
+  float* x = nullptr;
+  const void* y1 = nullptr; const void* g1 = nullptr; int64_t ldg1 = 0; const float* b1 = nullptr;
+  const void* y2 = nullptr; const void* g2 = nullptr; int64_t ldg2 = 0; const float* b2 = nullptr;
+  int f32 = 0, T = 0, W = 0;
+  const float* norm = nullptr; float eps = 0.f; void* h = nullptr;
+};
+void launch_gated_residual(const GatedArgs& a, hipStream_t st);
 
-// y = x rounded to the activation dtype (bf16), rows of n
-void launch_cast_rows(const float* x, void* y, int T, int n, hipStream_t st);
 // out[t][j] = act(gu[t][j]) * gu[t][n + j], j < n (bf16 rows, n % 8 == 0, 16-B aligned); act 1 silu, 4 gelu_tanh,
 // 2 clamped: g' = min(g, limit), g' * sigmoid(alpha g') * (clamp(u, -limit, limit) + 1)
 void launch_glu_rows(const void* gu, int64_t ldg, void* out, int64_t ldo, int T, int n, int act, float limit, float alpha,
@@ -118,9 +133,15 @@ struct LatentArgs {
   int T = 0;
 };
 // cache[slot] = [rmsnorm(kv[:rank]) * w, rope(kv[rank:])]
-// (cache_t: optional second, transposed bf16 copy of the latent part, [page][column][key in page])
-void launch_latent_write(const LatentArgs& a, const void* kv, int64_t ldkv, const float* w, float eps, void* cache_t,
-                         int page, hipStream_t st);
+// (cache_t: optional second, transposed bf16 copy of the latent part, [page][column][key in page]); with qn > 0 also the norm of the
+// query's latent, qy[t] = qx[t] / sqrt(mean(qx[t]^2) + eps) * qw (rows of qn, in kv's dtype), of padding rows too
+struct LatentWriteArgs {
+  const void* kv = nullptr; int64_t ldkv = 0;
+  const float* w = nullptr; float eps = 0.f;
+  void* cache_t = nullptr; int page = 0;
+  const void* qx = nullptr; int64_t ldq = 0; const float* qw = nullptr; void* qy = nullptr; int qn = 0;
+};
+void launch_latent_write(const LatentArgs& a, const LatentWriteArgs& w, hipStream_t st);
 // qa[t][h][rank:] = rope(q[t][h][dim:]) for q laid out [T][H][dim + rot], qa [T][H][rank + rot]
 void launch_latent_qrope(const LatentArgs& a, const void* q, int H, int dim, void* qa, hipStream_t st);
 // ol[t][h][:rank] = softmax_j(scale * qa[t][h] . cache[j]) . cache[j][:rank] over the keys j with

@@ -111,27 +111,43 @@ void norm_rows(const Tensor& x, const Tensor& w, double eps, Tensor& y, const Op
                           y.stride(0), yf, (int)M, (int)n, cur_stream());
 }
 
-void embed_rows(const Tensor& ids, const Tensor& table, Tensor& x, const OptT& prev, double scale) {
-  const int tf = act_f32(table, "table");
+void embed_rows(const Tensor& ids, const Tensor& table, Tensor& x, const OptT& prev, double scale, const OptT& h, const OptT& norm,
+                double eps, bool scalar, bool center, const OptT& h2, const OptT& norm2) {
+  vgate::EmbedArgs a;
+  a.t_f32 = act_f32(table, "table");
   TORCH_CHECK(table.dim() == 2 && table.is_contiguous(), "embed_rows: table [vocab, W]");
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kFloat32 && x.is_contiguous() && x.dim() == 2 &&
               x.size(1) == table.size(1), "embed_rows: x fp32 [T, W]");
-  const int T = (int)x.size(0);
-  const int32_t* ip = i32p(ids, "ids", T);
-  const int32_t* pp = has(prev) ? i32p(*prev, "prev", 1) : nullptr;
+  a.T = (int)x.size(0); a.W = (int)x.size(1); a.vocab = (int)table.size(0);
+  a.ids = i32p(ids, "ids", a.T);
+  a.prev = has(prev) ? i32p(*prev, "prev", 1) : nullptr;
+  a.table = table.data_ptr(); a.scale = (float)scale; a.x = x.data_ptr<float>();
+  TORCH_CHECK(!has(norm) || has(h), "embed_rows: a norm without its output");
+  TORCH_CHECK(has(h2) == has(norm2) && (!has(h2) || (has(norm) && !scalar)), "embed_rows: a second output is a second norm, by a vector");
+  for (const OptT* t : {&h, &h2}) {
+    if (!has(*t)) continue;
+    const int f = act_f32(**t, "h");
+    TORCH_CHECK((*t)->sizes() == x.sizes() && (*t)->is_contiguous(), "embed_rows: h [T, W]");
+    if (t == &h) { a.h1 = (*t)->data_ptr(); a.h_f32 = f; }
+    else { a.h2 = (*t)->data_ptr(); TORCH_CHECK(f == a.h_f32, "embed_rows: h and h2 of one dtype"); }
+  }
+  a.n1 = f32p(norm, "norm", scalar ? 1 : a.W);
+  a.n2 = f32p(norm2, "norm2", a.W);
+  a.scalar = scalar ? 1 : 0; a.center = center ? 1 : 0; a.eps = (float)eps;
   c10::DeviceGuard guard(x.device());
-  vgate::launch_embed_rows(ip, pp, table.data_ptr(), tf, (float)scale, x.data_ptr<float>(), T, (int)x.size(1),
-                           (int)table.size(0), cur_stream());
+  vgate::launch_embed_rows(a, cur_stream());
 }
 
 void gated_residual(Tensor& x, const Tensor& y1, const OptT& g1, const OptT& b1, const OptT& y2, const OptT& g2,
-                    const OptT& b2) {
+                    const OptT& b2, const OptT& norm, double eps, const OptT& h) {
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kFloat32 && x.is_contiguous() && x.dim() == 2,
               "gated_residual: x fp32 [T, W]");
+  vgate::GatedArgs a;
   const int T = (int)x.size(0), W = (int)x.size(1);
-  const int f = act_f32(y1, "y1");
+  a.T = T; a.W = W;
+  a.f32 = act_f32(y1, "y1");
   auto chk = [&](const Tensor& t, const char* name, bool dense) {
-    TORCH_CHECK(act_f32(t, name) == f && t.dim() == 2 && t.size(0) >= T && t.size(1) == W, name, ": [T, W] of y1's dtype");
+    TORCH_CHECK(act_f32(t, name) == a.f32 && t.dim() == 2 && t.size(0) >= T && t.size(1) == W, name, ": [T, W] of y1's dtype");
     if (dense) TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
   };
   chk(y1, "y1", true);
@@ -139,11 +155,16 @@ void gated_residual(Tensor& x, const Tensor& y1, const OptT& g1, const OptT& b1,
   if (has(g1)) chk(*g1, "g1", false);
   if (has(g2)) chk(*g2, "g2", false);
   TORCH_CHECK(!has(g2) || has(y2), "gated_residual: g2 without y2");
+  TORCH_CHECK(has(norm) == has(h), "gated_residual: a norm weight and its output come together");
+  if (has(h)) chk(*h, "h", true);
+  a.x = x.data_ptr<float>(); a.y1 = y1.data_ptr();
+  if (has(g1)) { a.g1 = g1->data_ptr(); a.ldg1 = g1->stride(0); }
+  if (has(y2)) a.y2 = y2->data_ptr();
+  if (has(g2)) { a.g2 = g2->data_ptr(); a.ldg2 = g2->stride(0); }
+  a.b1 = f32p(b1, "b1", W); a.b2 = f32p(b2, "b2", W);
+  a.norm = f32p(norm, "norm", 1); a.eps = (float)eps; a.h = has(h) ? h->data_ptr() : nullptr;
   c10::DeviceGuard guard(x.device());
-  vgate::launch_gated_residual(x.data_ptr<float>(), y1.data_ptr(), has(g1) ? g1->data_ptr() : nullptr,
-                               has(g1) ? g1->stride(0) : 0, f32p(b1, "b1", W), has(y2) ? y2->data_ptr() : nullptr,
-                               has(g2) ? g2->data_ptr() : nullptr, has(g2) ? g2->stride(0) : 0, f32p(b2, "b2", W), f,
-                               T, W, cur_stream());
+  vgate::launch_gated_residual(a, cur_stream());
 }
 
 vgate::LatentArgs latent_common(const Tensor& positions, const Tensor& inv_freq, int64_t rot_dims, int64_t rank,
@@ -160,7 +181,7 @@ vgate::LatentArgs latent_common(const Tensor& positions, const Tensor& inv_freq,
 
 void latent_write(const Tensor& kv, const Tensor& w, double eps, const Tensor& positions, const Tensor& slots,
                   const Tensor& inv_freq, int64_t rot_dims, Tensor& cache, int64_t rank, const OptT& cache_t, bool rot_half,
-                  double rot_amp) {
+                  double rot_amp, const OptT& qx, const OptT& qw, const OptT& qy) {
   const int f = act_f32(kv, "kv");
   TORCH_CHECK(kv.dim() == 2 && cache.dim() == 3 && cache.is_contiguous() && act_f32(cache, "cache") == f,
               "latent_write: kv [T, rank + rot], cache [pages, page, rank + rot] of one dtype");
@@ -170,15 +191,21 @@ void latent_write(const Tensor& kv, const Tensor& w, double eps, const Tensor& p
   a.slots = i32p(slots, "slots", kv.size(0));  // values < pages * page: written by the step's block tables
   a.cache = cache.data_ptr(); a.f32 = f;
   OptT wo(w);
-  void* ct = nullptr;
+  vgate::LatentWriteArgs b;
+  b.kv = kv.data_ptr(); b.ldkv = kv.stride(0); b.w = f32p(wo, "w", rank); b.eps = (float)eps; b.page = (int)cache.size(1);
   if (has(cache_t)) {
     TORCH_CHECK(cache_t->is_cuda() && cache_t->scalar_type() == torch::kBFloat16 && cache_t->is_contiguous() &&
                 cache_t->numel() == cache.size(0) * cache.size(1) * rank, "latent_write: cache_t bf16 [pages, rank, page]");
-    ct = cache_t->data_ptr();
+    b.cache_t = cache_t->data_ptr();
+  }
+  TORCH_CHECK(has(qx) == has(qw) && has(qx) == has(qy), "latent_write: the query's rows, norm and output come together");
+  if (has(qx)) {
+    TORCH_CHECK(act_f32(*qx, "qx") == f && act_f32(*qy, "qy") == f && qx->dim() == 2 && qx->size(0) == kv.size(0) && qx->size(1) > 0 &&
+                qy->sizes() == qx->sizes() && qy->is_contiguous(), "latent_write: qx and qy [T, n] of kv's dtype");
+    b.qx = qx->data_ptr(); b.ldq = qx->stride(0); b.qn = (int)qx->size(1); b.qw = f32p(qw, "qw", b.qn); b.qy = qy->data_ptr();
   }
   c10::DeviceGuard guard(kv.device());
-  vgate::launch_latent_write(a, kv.data_ptr(), kv.stride(0), f32p(wo, "w", rank), (float)eps, ct, (int)cache.size(1),
-                             cur_stream());
+  vgate::launch_latent_write(a, b, cur_stream());
 }
 
 void latent_qrope(const Tensor& q, const Tensor& positions, const Tensor& inv_freq, int64_t rot_dims, Tensor& qa,
@@ -270,14 +297,6 @@ void delta_rule(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor&
   vgate::launch_delta_rule(p, (int)T, scratch.data_ptr<float>(), (size_t)scratch.numel(), cur_stream());
 }
 
-
-void cast_rows(const Tensor& x, Tensor& y) {
-  TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kFloat32 && x.is_contiguous() && x.dim() == 2, "cast_rows: x fp32 [T, n]");
-  TORCH_CHECK(y.is_cuda() && y.scalar_type() == torch::kBFloat16 && y.is_contiguous() && y.dim() == 2 &&
-              y.size(1) == x.size(1) && y.size(0) <= x.size(0), "cast_rows: y bf16 [<= T, n]");
-  c10::DeviceGuard guard(x.device());
-  vgate::launch_cast_rows(x.data_ptr<float>(), y.data_ptr(), (int)y.size(0), (int)y.size(1), cur_stream());
-}
 
 void glu_rows(const Tensor& gu, Tensor& out, int64_t act, double limit, double alpha) {
   TORCH_CHECK(gu.is_cuda() && gu.scalar_type() == torch::kBFloat16 && gu.dim() == 2 && gu.stride(1) == 1, "glu_rows: gu bf16 [T, 2 n]");
@@ -907,13 +926,15 @@ void bind_seq(pybind11::module& m) {
         py::arg("w"), py::arg("eps"), py::arg("y"), py::arg("rows") = py::none(), py::arg("scalar") = false,
         py::arg("center") = false);
   m.def("embed_rows", &embed_rows, "embedding gather into the fp32 residual stream", py::arg("ids"), py::arg("table"),
-        py::arg("x"), py::arg("prev") = py::none(), py::arg("scale") = 1.0);
+        py::arg("x"), py::arg("prev") = py::none(), py::arg("scale") = 1.0, py::arg("h") = py::none(), py::arg("norm") = py::none(),
+        py::arg("eps") = 0.0, py::arg("scalar") = false, py::arg("center") = false, py::arg("h2") = py::none(), py::arg("norm2") = py::none());
   m.def("gated_residual", &gated_residual, "x += y1 * sigmoid(g1 + b1) + y2 * sigmoid(g2 + b2)", py::arg("x"),
         py::arg("y1"), py::arg("g1") = py::none(), py::arg("b1") = py::none(), py::arg("y2") = py::none(),
-        py::arg("g2") = py::none(), py::arg("b2") = py::none());
+        py::arg("g2") = py::none(), py::arg("b2") = py::none(), py::arg("norm") = py::none(), py::arg("eps") = 0.0, py::arg("h") = py::none());
   m.def("latent_write", &latent_write, "latent norm + shared-key rotation + paged cache store", py::arg("kv"), py::arg("w"),
         py::arg("eps"), py::arg("positions"), py::arg("slots"), py::arg("inv_freq"), py::arg("rot_dims"), py::arg("cache"),
-        py::arg("rank"), py::arg("cache_t") = py::none(), py::arg("rot_half") = false, py::arg("rot_amp") = 1.0);
+        py::arg("rank"), py::arg("cache_t") = py::none(), py::arg("rot_half") = false, py::arg("rot_amp") = 1.0,
+        py::arg("qx") = py::none(), py::arg("qw") = py::none(), py::arg("qy") = py::none());
   m.def("latent_qrope", &latent_qrope, "rotate the rotated query part into the absorbed query buffer", py::arg("q"),
         py::arg("positions"), py::arg("inv_freq"), py::arg("rot_dims"), py::arg("qa"), py::arg("H"), py::arg("dim"),
         py::arg("rank"), py::arg("rot"), py::arg("rot_half") = false, py::arg("rot_amp") = 1.0);
@@ -939,7 +960,6 @@ void bind_seq(pybind11::module& m) {
     const auto p = vgate::delta_rule_plan((int)T, (int)S, (int)H, (int)D);
     return std::make_tuple(p.scan, (int64_t)p.lim, (int64_t)p.chunks);
   }, "(token scan, most tokens of a sequence that takes it or else the short form, chunks) of a delta_rule step of T rows and S sequences");
-  m.def("cast_rows", &cast_rows, "fp32 rows rounded to bf16");
   m.def("glu_rows", &glu_rows, "out = act(gate) * up over a stacked [gate; up] projection", py::arg("gu"), py::arg("out"),
         py::arg("act"), py::arg("limit") = 0.0, py::arg("alpha") = 1.702);
   m.def("act_rows", &act_rows, "out = act(x) over bf16 rows", py::arg("x"), py::arg("out"), py::arg("act"));

@@ -117,13 +117,14 @@ class GatedParallelLayer:
         return self.proj.nbytes() + self.mixer.nbytes() + (self.ff.nbytes() if self.ff else 0)
 
     def run(self, st, sv, cache) -> None:
-        x, h = st.x, st.h
-        seq.norm_rows(x, self.norm1, self.eps, h, scalar=True)
+        """st.x: the fp32 stream; st.h: this layer's normed input, made by the kernel before (the embedding's, or the residual
+        kernel of the layer before); st.next_layer: the layer that follows, or None."""
+        x, h, nxt = st.x, st.h, st.next_layer
         P = self.proj(h)
         y1 = self.mixer.forward(h, P, self.cols, sv, cache)
         y2 = self.ff.forward(h) if self.ff is not None else None
         seq.gated_residual(x, y1, self.cols(P, "rg1"), self.rg1_b, y2, self.cols(P, "rg2") if y2 is not None else None,
-                           self.rg2_b)
+                           self.rg2_b, **({} if nxt is None else dict(norm=nxt.norm1, eps=nxt.eps, h=h)))
 
 
 class PostNormLayer:
@@ -296,6 +297,10 @@ class PreNormLayer:
     def nbytes(self) -> int:
         return (self.proj.nbytes() if self.proj else 0) + self.mixer.nbytes() + (self.ff.nbytes() if self.ff else 0)
 
+    def first_input(self, st) -> dict:
+        """What the embedding kernel makes of the stream for this layer as the step's first."""
+        return dict(h=st.h, norm=self.norm1, eps=self.eps, center=self.center)
+
     def run(self, st, sv, cache) -> None:
         """st.x: the fp32 stream; st.h: the normed input in the activation dtype (``st.h_ready``: the kernel before
         has made this layer's already); st.next_norm: the norm weight of the layer that follows, or None."""
@@ -356,6 +361,10 @@ class ParallelNormLayer:
     def inputs(self, st) -> list:
         """What the kernel before this layer makes: its sublayers' normed inputs."""
         return [(self.norm1, st.h)] + ([(self.norm2, st.h2)] if self.ff is not None else [])
+
+    def first_input(self, st) -> dict:
+        second = dict(h2=st.h2, norm2=self.norm2) if self.ff is not None else {}
+        return dict(h=st.h, norm=self.norm1, eps=self.eps, **second)
 
     def run(self, st, sv, cache) -> None:
         """st.x: the fp32 stream; st.h, st.h2: the normed inputs in the activation dtype (``st.h_ready``: made by the kernel
@@ -420,6 +429,7 @@ class _Stream:
         self.h = self.x if self.f32 else torch.empty(T, W, dtype=act_dtype, device=device)
         self.mix = torch.empty(T, W, dtype=torch.float32, device=device) if depth_average else None
         self.result, self.layer, self.coef = self.x, 0, None
+        self.next_layer = None
 
     def begin(self, i: int, coef) -> None:
         self.layer, self.coef = i, coef
@@ -535,10 +545,14 @@ class HybridModel:
         dev, eps = self.device, self.arch.rms_eps
         st = _Stream(T, W, len(self.layers), self.act_dtype, dev, self.arch.depth_average,
                      normed_input=self.arch.arrangement != "post_norm")
-        seq.embed_rows(sv.ids, self.embed, st.x, prev=sv.prev_tokens)
-        if self.arch.arrangement == "post_norm" and not self.f32:
-            seq.cast_rows(st.x, st.h)   # (the gated_parallel arrangement makes h with its norm)
+        # h: a copy of the stream (post_norm, in bf16), or the first layer's normed input (gated_parallel)
+        if self.arch.arrangement == "post_norm":
+            first = {} if self.f32 else dict(h=st.h)
+        else:
+            first = dict(h=st.h, norm=self.layers[0].norm1, eps=self.layers[0].eps, scalar=True)
+        seq.embed_rows(sv.ids, self.embed, st.x, prev=sv.prev_tokens, **first)
         for li, L in enumerate(self.layers):
+            st.next_layer = self.layers[li + 1] if li + 1 < len(self.layers) else None
             st.begin(li, self.depth_coef[li] if self.depth_coef else None)
             L.run(st, sv, caches[li])
             st.end()
@@ -573,7 +587,11 @@ class HybridModel:
         returns the fp32 stream."""
         T, W = sv.T, self.arch.hidden_size
         st = _PreStream(T, W, self.act_dtype, self.device, second=self.side)
-        seq.embed_rows(sv.ids, self.embed, st.x, prev=sv.prev_tokens, scale=self.arch.embed_scale)
+        first = {}
+        if self.loop_in is None:   # (a looped model's first layer reads the loop's own projection)
+            first = self.layers[0].first_input(st)
+            st.h_ready = True
+        seq.embed_rows(sv.ids, self.embed, st.x, prev=sv.prev_tokens, scale=self.arch.embed_scale, **first)
         x0 = pair = None
         if self.loop_in is not None:
             x0 = st.x.clone()

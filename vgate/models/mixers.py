@@ -213,11 +213,10 @@ class LatentAttention:
         E = KR + R
         dt, dev = h.dtype, h.device
         cq = torch.empty(T, self.QR, dtype=dt, device=dev)
-        seq.norm_rows(cols(P, "dq"), self.dq_norm, self.eps, cq)
-        q = self.uq(cq)
         cache, cache_t = self._views(cache)
         seq.latent_write(cols(P, "dkv"), self.dkv_norm, self.eps, sv.positions, sv.slots, self.inv_freq,
-                         self.rot_dims, cache, KR, cache_t=cache_t, **self.rot)
+                         self.rot_dims, cache, KR, cache_t=cache_t, query=(cols(P, "dq"), self.dq_norm, cq), **self.rot)
+        q = self.uq(cq)
         qa = torch.empty(T, H, E, dtype=dt, device=dev)
         seq.gemm(q.view(T, H, D + R)[:, :, :D].permute(1, 0, 2), self.uk_t, qa[:, :, :KR].permute(1, 0, 2))
         if R:

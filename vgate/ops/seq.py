@@ -126,21 +126,27 @@ def norm_rows(x: torch.Tensor, w: torch.Tensor, eps: float, out: torch.Tensor, r
 
 
 def embed_rows(ids: torch.Tensor, table: torch.Tensor, out: torch.Tensor, prev: torch.Tensor | None = None,
-               scale: float = 1.0) -> torch.Tensor:
-    """fp32 rows of the embedding table times ``scale``; ids < 0 name the previous step's sample prev[-id - 1]."""
+               scale: float = 1.0, h: torch.Tensor | None = None, norm: torch.Tensor | None = None, eps: float = 0.0,
+               scalar: bool = False, center: bool = False, h2: torch.Tensor | None = None, norm2: torch.Tensor | None = None) -> torch.Tensor:
+    """fp32 rows of the embedding table times ``scale``; ids < 0 name the previous step's sample prev[-id - 1]. ``h``: what the first
+    sublayer reads of them, a copy in h's dtype or with ``norm`` what :func:`norm_rows` makes; ``h2``: the same by ``norm2``."""
     if table.is_cuda:
-        _C().embed_rows(ids, table, out, prev, scale)
+        _C().embed_rows(ids, table, out, prev, scale, h, norm, eps, scalar, center, h2, norm2)
         return out
     if prev is not None and bool((ids < 0).any()):
         ids = torch.where(ids < 0, prev.to(ids.device)[(-ids - 1).clamp(min=0).long()], ids)
     out.copy_(table[ids.long()].float() * scale)
+    for y, w in ((h, norm), (h2, norm2)):
+        if y is not None:
+            y.copy_(out) if w is None else norm_rows(out, w, eps, y, scalar=scalar, center=center)
     return out
 
 
-def gated_residual(x, y1, g1=None, b1=None, y2=None, g2=None, b2=None) -> None:
-    """x += y1 * sigmoid(g1 + b1) [+ y2 * sigmoid(g2 + b2)] in fp32 (g: strided column views)."""
+def gated_residual(x, y1, g1=None, b1=None, y2=None, g2=None, b2=None, norm=None, eps: float = 0.0, h=None) -> None:
+    """x += y1 * sigmoid(g1 + b1) [+ y2 * sigmoid(g2 + b2)] in fp32 (g: strided column views). ``h`` (y1's dtype): the new row's norm
+    times the one number ``norm``."""
     if x.is_cuda:
-        _C().gated_residual(x, y1, g1, b1, y2, g2, b2)
+        _C().gated_residual(x, y1, g1, b1, y2, g2, b2, norm, eps, h)
         return
     T = x.shape[0]
     v = y1.float()
@@ -152,6 +158,8 @@ def gated_residual(x, y1, g1=None, b1=None, y2=None, g2=None, b2=None) -> None:
             u = u * torch.sigmoid(g2[:T].float() + (b2 if b2 is not None else 0.0))
         v = v + u
     x += v
+    if h is not None:
+        norm_rows(x, norm, eps, h, scalar=True)
 
 
 def rope_inv_freq(dims: int, base: float, device, scaling: dict | None = None) -> torch.Tensor:
@@ -228,14 +236,18 @@ def _latent_turn(x, positions, inv_freq, rot_dims: int, rot_half: bool, rot_amp:
 
 
 def latent_write(kv, w, eps, positions, slots, inv_freq, rot_dims: int, cache, rank: int, cache_t=None,
-                 rot_half: bool = False, rot_amp: float = 1.0) -> None:
+                 rot_half: bool = False, rot_amp: float = 1.0, query=None) -> None:
     """cache[slot] = [rmsnorm(kv[:rank]) * w, rope(kv[rank:])] for every token with slot >= 0.
     ``cache_t`` (GPU, bf16): a second copy of the latent part laid out [page, column, key in page], the
     operand layout of the MFMA attention kernel's weighted sum. The rotation pairs entry 2i with 2i + 1, or with
-    ``rot_half`` entry i with i + rot_dims / 2; cos and sin are multiplied by ``rot_amp``."""
+    ``rot_half`` entry i with i + rot_dims / 2; cos and sin are multiplied by ``rot_amp``. ``query`` (x, w, y): in the same
+    launch y = x / sqrt(mean(x^2) + eps) * w of every row, padding too."""
     if kv.is_cuda:
-        _C().latent_write(kv, w, eps, positions, slots, inv_freq, rot_dims, cache, rank, cache_t, rot_half, rot_amp)
+        _C().latent_write(kv, w, eps, positions, slots, inv_freq, rot_dims, cache, rank, cache_t, rot_half, rot_amp,
+                          *(query or (None, None, None)))
         return
+    if query is not None:
+        norm_rows(query[0], query[1], eps, query[2])
     x = kv.float()
     c = x[:, :rank]
     c = c * (1.0 / torch.sqrt(c.pow(2).mean(-1, keepdim=True) + eps)) * w
@@ -387,15 +399,6 @@ def moe_combine(y, pos, wts, out, add=None) -> None:
 
 
 # ------------------------------------------------------------------ post-norm residual, depth average
-def cast_rows(x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
-    """out = x rounded to out's dtype (the copy of the fp32 stream a bf16 GEMM reads)."""
-    if x.is_cuda:
-        _C().cast_rows(x, out)
-        return out
-    out.copy_(x[: out.shape[0]])
-    return out
-
-
 def tanh_norm_rows(x: torch.Tensor, alpha: torch.Tensor, w: torch.Tensor, b: torch.Tensor, out: torch.Tensor,
                    rows: torch.Tensor | None = None) -> torch.Tensor:
     """out[m] = tanh(alpha * x[rows[m]]) * w + b: a norm without statistics (alpha one fp32 number, w / b
