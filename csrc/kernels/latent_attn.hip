@@ -41,6 +41,9 @@
 // DMA a step ahead and each wave carries 16 or 32 rows from scores to weighted latents in registers (latent_attn_staged_kernel).
 #include <stdlib.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "lds_rows.h"
 #include "locate.h"
 #include "row_norm.h"
@@ -70,7 +73,8 @@ __device__ __forceinline__ float turned(const LatentArgs& a, const void* x, int6
 }
 
 // grid (token, 2 with the query's latent): the key's row and the query's norm read the same projection and nothing of each other, so
-// they share a launch (us, latents of 256 and 512, two launches -> one: 32 rows 4.7 + 3.9 -> 4.2, 2048 rows 8.4 + 5.9 -> 9.9). NI columns of the query's latent per thread in registers.
+// they share a launch (us, latents of 256 and 512, two launches -> one: 32 rows 4.7 + 3.9 -> 4.2, 2048 rows 8.4 + 5.9 -> 9.9). NI
+// columns of the query's latent per thread in registers.
 template <int NI>
 __global__ __launch_bounds__(256) void latent_write_kernel(LatentArgs a, LatentWriteArgs b) {
   __shared__ float red[16];
@@ -276,13 +280,16 @@ __device__ __forceinline__ float group16_sum(float v) {
 }
 
 // NCT: 16-column tiles of the latent (rank <= 16 NCT); NQF: 32-wide fragments of a query row (E <= 32 NQF).
-// E % 8 == 0 (host-checked): every cache fragment is one unconditional 16-B load. Loads are issued in
-// groups (LG fragments, then their MFMAs) so a lone wave has several in flight; a fragment past the row's
+// E % 8 == 0 (host-checked): every cache fragment is one unconditional 16-B load; a fragment past the row's
 // end or the latent's last column is read from a clamped address: its partner (zero Q fragment) or its
 // output column (never stored) makes the value irrelevant, and cached values are always finite.
-constexpr int LG = 4;
-template <int NCT, int NQF>
-__global__ __launch_bounds__(256) void latent_attn_mfma_kernel(LatentArgs a, const bf16_t* __restrict__ qa, int H,
+// A decoded token's wave sees one or two key tiles, so what bounds it is how often it waits for memory: all of a tile's keys are asked
+// for together, all of its values while the softmax runs (by groups of 4 and 8 before, nine waits a tile), and the four waves' results meet
+// in LDS areas of their own, summed by all threads. us, 32 sequences: 12 heads, latent 512, some 700 keys 31.0 -> 22.7 and the merge 10.7 ->
+// 4.6; 8 heads, latent 256, 512 keys 16.2 -> 11.5 and 6.6 -> 4.6.
+// EXACT: rows of whole fragments and a latent of whole tiles (E = 32 NQF, rank = 16 NCT), nothing is clamped.
+template <int NCT, int NQF, bool EXACT>
+__global__ __launch_bounds__(256, NCT > 16 ? 1 : 2) void latent_attn_mfma_kernel(LatentArgs a, const bf16_t* __restrict__ qa, int H,
                                                                 float scale_log2e,
                                                                 const int32_t* __restrict__ block_tables,
                                                                 int max_blocks, int num_pages,
@@ -293,8 +300,9 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(LatentArgs a, con
                                                                 const float* __restrict__ sink, int parts,
                                                                 float* __restrict__ part_o, float* __restrict__ part_ml) {
   __shared__ __attribute__((aligned(16))) bf16_t pl[4][16][40];
-  __shared__ float mrg_m[4][16], mrg_l[4][16];
-  __shared__ float mrg_o[16][16 * NCT];  // split mode: the merged weighted latent of the 16 rows
+  __shared__ float mrg_m[4][16], mrg_l[4][16], row_l[16];
+  constexpr int OS = 16 * NCT + 4;        // row stride of the area (the four rows of an instruction in different banks)
+  extern __shared__ __attribute__((aligned(16))) float mrg_o[];  // split mode: the waves' weighted latents [4][16][OS]
   const int E = a.rank + a.rot, KR = a.rank;
   int tile;
   // (sequence, 64-row tile) of this workgroup
@@ -344,29 +352,42 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(LatentArgs a, con
   for (int j0 = kmin + (split ? 32 * (wv + 4 * part) : 0); j0 < kmax; j0 += split ? 128 * np : 32) {
     int pg0 = bt[j0 >> 4];
     int pg1 = (j0 + 16 < kmax) ? bt[(j0 >> 4) + 1] : pg0;
-    pg0 = min(max(pg0, 0), num_pages - 1);
-    pg1 = min(max(pg1, 0), num_pages - 1);
+    pg0 = __builtin_amdgcn_readfirstlane(min(max(pg0, 0), num_pages - 1));
+    pg1 = __builtin_amdgcn_readfirstlane(min(max(pg1, 0), num_pages - 1));
+    int kr = lr;
+    if (!EXACT) asm volatile("" : "+v"(kr));  // (opaque: clamped offsets are worked out here and not kept in registers over the loop)
     f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bf16_t* k0p = cache + ((int64_t)pg0 * 16 + lr) * E;
-    const bf16_t* k1p = cache + ((int64_t)pg1 * 16 + lr) * E;
+    const bf16_t* k0p = cache + (int64_t)pg0 * 16 * E;   // (the page is the wave's: a scalar base and 32-bit offsets)
+    const bf16_t* k1p = cache + (int64_t)pg1 * 16 * E;
+    // fragments asked for together, as registers allow without spilling (clamped addresses take one more each)
+    constexpr int KG = !EXACT ? 4 : (NCT > 16 ? NQF / 2 : NQF), VG = !EXACT ? 8 : (NCT > 16 ? NCT / 2 : NCT);
 #pragma unroll
-    for (int k0 = 0; k0 < NQF; k0 += LG) {
-      if (k0 < nqf) {  // wave-uniform
-        uint4 b0[LG], b1[LG];
+    for (int g = 0; g < NQF; g += KG) {
+      uint4 b0[KG], b1[KG];
 #pragma unroll
-        for (int u = 0; u < LG; ++u) {
-          const int off = min(32 * (k0 + u) + 8 * lg, E - 8);
+      for (int u = 0; u < KG; ++u)
+        if (g + u < NQF) {
+          const int off = kr * E + (EXACT ? 32 * (g + u) + 8 * lg : min(32 * (g + u) + 8 * lg, E - 8));
           b0[u] = ld16(k0p + off);
           b1[u] = ld16(k1p + off);
         }
 #pragma unroll
-        for (int u = 0; u < LG; ++u)
-          if (k0 + u < NQF) {
-            s0 = mfma16(qf[k0 + u], as_bf16x8(b0[u]), s0);
-            s1 = mfma16(qf[k0 + u], as_bf16x8(b1[u]), s1);
-          }
-      }
+      for (int u = 0; u < KG; ++u)
+        if (g + u < NQF) {
+          s0 = mfma16(qf[g + u], as_bf16x8(b0[u]), s0);
+          s1 = mfma16(qf[g + u], as_bf16x8(b1[u]), s1);
+        }
+      __builtin_amdgcn_sched_barrier(0);
     }
+    const bf16_t* tp = cache_t + ((int64_t)((lg >> 1) ? pg1 : pg0) * KR + kr) * 16 + 8 * (lg & 1);
+    uint4 vb[VG];
+    auto values = [&](int c0) {
+#pragma unroll
+      for (int u = 0; u < VG; ++u)
+        if (c0 + u < NCT) vb[u] = ld16(tp + (EXACT ? 256 * (c0 + u) : 16 * (min(16 * (c0 + u) + kr, KR - 1) - kr)));
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    values(0);  // (asked for here, ahead of the softmax)
     float al[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -387,29 +408,24 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(LatentArgs a, con
       for (int i = 0; i < 4; ++i) O[ct][i] *= al[i];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's P tile is written (LDS is in order per wave)
     const bf16x8 pf = as_bf16x8(*reinterpret_cast<const uint4*>(&pl[wv][lr][8 * lg]));
-    const int pgs = (lg >> 1) ? pg1 : pg0;
-    const bf16_t* tp = cache_t + (int64_t)pgs * KR * 16 + 8 * (lg & 1);
 #pragma unroll
-    for (int c0 = 0; c0 < NCT; c0 += 2 * LG) {
-      if (c0 < nct) {  // wave-uniform
-        uint4 b[2 * LG];
+    for (int c0 = 0; c0 < NCT; c0 += VG) {
+      if (c0 > 0) values(c0);
 #pragma unroll
-        for (int u = 0; u < 2 * LG; ++u) b[u] = ld16(tp + (int64_t)min(16 * (c0 + u) + lr, KR - 1) * 16);
-#pragma unroll
-        for (int u = 0; u < 2 * LG; ++u)
-          if (c0 + u < NCT) O[c0 + u] = mfma16(pf, as_bf16x8(b[u]), O[c0 + u]);
-      }
+      for (int u = 0; u < VG; ++u)
+        if (c0 + u < NCT) O[c0 + u] = mfma16(pf, as_bf16x8(vb[u]), O[c0 + u]);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // P tile read before the next tile overwrites it
   }
   if (split) {
-    float f[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float tot = group16_sum(lsum[i]);
       if (lr == 0) { mrg_m[wv][4 * lg + i] = m[i]; mrg_l[wv][4 * lg + i] = tot; }
     }
     __syncthreads();
+    const int64_t slot = (int64_t)part * gridDim.x + blockIdx.x;
+    float* area = mrg_o + wv * 16 * OS;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 4 * lg + i;
@@ -420,45 +436,41 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(LatentArgs a, con
       float L = 0.f;
 #pragma unroll
       for (int w = 0; w < 4; ++w) L += mrg_l[w][r] * exp2f(mrg_m[w][r] - Ms);  // a wave that saw no key: l = 0, exp2(-inf) = 0
-      f[i] = exp2f(m[i] - Ms);
-      lsum[i] = L;                // the merged row sum (the same in every lane of the row)
-      m[i] = M;
-    }
-    for (int w = 0; w < 4; ++w) {  // waves add their scaled partials in turn
-      if (wv == w) {
+      const float f = exp2f(m[i] - Ms);
 #pragma unroll
-        for (int ct = 0; ct < NCT; ++ct)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float* dst = &mrg_o[4 * lg + i][16 * ct + lr];
-            const float v = O[ct][i] * f[i];
-            *dst = (w == 0) ? v : *dst + v;
-          }
-      }
-      __syncthreads();
-    }
-    if (np > 1) {  // (workgroup-uniform) hand the partial result on: the merge kernel finishes the rows
-      const int64_t slot = (int64_t)part * gridDim.x + blockIdx.x;
-      float* po = part_o + slot * (16 * 16 * NCT);
-      for (int e = threadIdx.x; e < 16 * 16 * NCT; e += 256) po[e] = (&mrg_o[0][0])[e];
+      for (int ct = 0; ct < NCT; ++ct) area[r * OS + 16 * ct + lr] = O[ct][i] * f;
       if (wv == 0 && lr == 0) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          part_ml[(slot * 16 + 4 * lg + i) * 2] = m[i];
-          part_ml[(slot * 16 + 4 * lg + i) * 2 + 1] = lsum[i];
+        row_l[r] = L;
+        if (np > 1) {
+          part_ml[(slot * 16 + r) * 2] = M;
+          part_ml[(slot * 16 + r) * 2 + 1] = L;
         }
       }
-      return;
     }
-    if (wv != 0) return;
+    __syncthreads();
+    // four columns a thread and turn, the waves' parts added in wave order; np > 1 (workgroup-uniform): handed on, the merge kernel
+    // finishes the rows
+#pragma unroll 4
+    for (int e = threadIdx.x; e < 16 * 4 * NCT; e += 256) {
+      const int r = e / (4 * NCT), col = 4 * (e % (4 * NCT));
+      const float* o = mrg_o + r * OS + col;
+      const f32x4 y = ((*reinterpret_cast<const f32x4*>(o) + *reinterpret_cast<const f32x4*>(o + 16 * OS)) +
+                       *reinterpret_cast<const f32x4*>(o + 32 * OS)) + *reinterpret_cast<const f32x4*>(o + 48 * OS);
+      if (np > 1) {
+        *reinterpret_cast<f32x4*>(part_o + slot * (16 * 16 * NCT) + r * (16 * NCT) + col) = y;
+      } else if (r < nrows) {
+        const float inv = 1.f / row_l[r];
+        bf16_t* orow = ol + ((int64_t)(t0 + r / H) * H + r % H) * KR;
 #pragma unroll
-    for (int ct = 0; ct < NCT; ++ct)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) O[ct][i] = mrg_o[4 * lg + i][16 * ct + lr];
+        for (int j = 0; j < 4; ++j)
+          if (col + j < KR) orow[col + j] = f2bf(y[j] * inv);
+      }
+    }
+    return;
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const float tot = split ? lsum[i] : group16_sum(lsum[i]);
+    const float tot = group16_sum(lsum[i]);
     const float inv = 1.f / tot;
     const int r = row0 + 4 * lg + i;
     if (r < nrows) {
@@ -890,27 +902,36 @@ __global__ __launch_bounds__(256) void latent_attn_merge_kernel(int rank, int H,
   const int t0 = query_start[s], nrows = (query_start[s + 1] - t0) * H;
   if (nrows > 16) return;  // (not shared out: the attention kernel has stored its rows)
   constexpr int MAXP = 8;
-  // blockIdx.y: which four rows of the tile
-  for (int e = threadIdx.x; e < 4 * rank; e += blockDim.x) {
-    const int r = 4 * blockIdx.y + e / rank, col = e % rank;
+  // a thread's four columns of the blockIdx.y-th rows of the tile (a workgroup's threads take each column of its rows once at most: one
+  // wait for memory)
+  const int c4 = (rank + 3) / 4, per = 16 / gridDim.y;
+  for (int e = threadIdx.x; e < per * c4; e += blockDim.x) {
+    const int r = per * blockIdx.y + e / c4, col = 4 * (e % c4);   // (columns past the latent's last: within the row's stride, never stored)
     if (r >= nrows) continue;
-    float pm[MAXP], plv[MAXP], po[MAXP], M = -INFINITY;
+    float pm[MAXP], plv[MAXP], M = -INFINITY;
+    f32x4 po[MAXP];
 #pragma unroll
     for (int p = 0; p < MAXP; ++p) {  // all parts' loads asked for together
       const int64_t slot = (int64_t)min(p, parts - 1) * gridDim.x + blockIdx.x;
-      pm[p] = p < parts ? part_ml[(slot * 16 + r) * 2] : -INFINITY;
-      plv[p] = part_ml[(slot * 16 + r) * 2 + 1];
-      po[p] = part_o[slot * (16 * vs) + r * vs + col];
+      const float2 ml = *reinterpret_cast<const float2*>(part_ml + (slot * 16 + r) * 2);
+      pm[p] = p < parts ? ml.x : -INFINITY;
+      plv[p] = ml.y;
+      po[p] = *reinterpret_cast<const f32x4*>(part_o + slot * (16 * vs) + r * vs + col);
       M = fmaxf(M, pm[p]);
     }
-    float L = 0.f, y = 0.f;
+    float L = 0.f;
+    f32x4 y = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int p = 0; p < MAXP; ++p) {
       const float f = exp2f(pm[p] - M);  // a part that saw no key (or is none): max -inf, factor 0
       L = fmaf(plv[p], f, L);
-      y = fmaf(po[p], f, y);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = fmaf(po[p][j], f, y[j]);
     }
-    ol[((int64_t)(t0 + r / H) * H + r % H) * rank + col] = f2bf(y / L);
+    bf16_t* o = ol + ((int64_t)(t0 + r / H) * H + r % H) * rank + col;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (col + j < rank) o[j] = f2bf(y[j] / L);
   }
 }
 
@@ -956,12 +977,19 @@ void launch_mfma(const LatentArgs& a, const void* qa, int H, float scale, const 
   }
   float* part_o = scratch;
   float* part_ml = parts > 1 ? scratch + (size_t)parts * blocks * 16 * 16 * NCT : nullptr;
-  hipLaunchKernelGGL((latent_attn_mfma_kernel<NCT, NQF>), dim3(blocks, parts), dim3(256), 0, st, a,
-                     reinterpret_cast<const bf16_t*>(qa), H, scale * 1.4426950408889634f, block_tables, max_blocks,
-                     num_pages, context_lens, query_start, S, reinterpret_cast<const bf16_t*>(cache_t),
-                     reinterpret_cast<bf16_t*>(ol), window, sink, parts, part_o, part_ml);
+  auto decode = [&](auto nqf, auto exact) {
+    constexpr int LDS = 4 * 16 * (16 * NCT + 4) * 4;
+    auto kern = latent_attn_mfma_kernel<NCT, decltype(nqf)::value, decltype(exact)::value>;
+    static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS) == hipSuccess;
+    (void)attr;
+    hipLaunchKernelGGL(kern, dim3(blocks, parts), dim3(256), LDS, st, a, reinterpret_cast<const bf16_t*>(qa), H,
+                       scale * 1.4426950408889634f, block_tables, max_blocks, num_pages, context_lens, query_start, S,
+                       reinterpret_cast<const bf16_t*>(cache_t), reinterpret_cast<bf16_t*>(ol), window, sink, parts, part_o, part_ml);
+  };
+  if (a.rot == 64 && a.rank == 16 * NCT) decode(std::integral_constant<int, NCT / 2 + 2>{}, std::true_type{});
+  else decode(std::integral_constant<int, NQF>{}, std::false_type{});
   if (parts > 1)
-    hipLaunchKernelGGL(latent_attn_merge_kernel, dim3(blocks, 4), dim3(256), 0, st, a.rank, H, query_start, S, parts, 16 * NCT,
+    hipLaunchKernelGGL(latent_attn_merge_kernel, dim3(blocks, a.rank <= 256 ? 4 : 8), dim3(256), 0, st, a.rank, H, query_start, S, parts, 16 * NCT,
                        part_o, part_ml, reinterpret_cast<bf16_t*>(ol));
 }
 
@@ -1018,11 +1046,12 @@ void launch_latent_attn(const LatentArgs& a, const void* qa, int H, float scale,
 }
 
 // Decoded tokens on the MFMA kernel: how many workgroups share a sequence's key tiles (1: no split), chosen from the
-// step's shape so that the launch has about two workgroups per CU, and the scratch floats their partial results take.
+// step's shape so that the launch has about two workgroups per CU, or one where a latent of more than 256 takes a CU's registers
+// and LDS, and the scratch floats their partial results take.
 int latent_attn_parts(int T, int S, int H, int rank, int rot, int f32, int page) {
   if (!mfma_takes(rank, rot, f32, page) || (int64_t)T * H > 16 * (int64_t)S) return 1;
   const int wg = (T * H + 63) / 64 + S;
-  const int parts = 512 / (wg > 0 ? wg : 1);
+  const int parts = rank > 256 ? 256 / std::max(S, 1) : 512 / (wg > 0 ? wg : 1);
   return parts < 2 ? 1 : (parts > 8 ? 8 : parts);
 }
 size_t latent_attn_part_floats(int T, int S, int H, int rank, int rot, int parts) {
