@@ -274,13 +274,14 @@ __global__ __launch_bounds__(256) void gemm_any_mfma_kernel(AnyGemmArgs p) {
 // elements: whole 128-B lines of a weight row) in turn and meet in LDS; wave i finishes the i-th 16 rows. A tile's 64 rows go in passes of
 // 32. What bounds it is one trip to memory for the weights, 4 to 6 us a launch. UB pairs in flight per wave: one, and eight waves per SIMD
 // (with four the registers leave three, and K below 1024 is read in vain: 2048 x 512 with 8 rows each of 8 experts 7.3 us, 12.4); more for
-// up to 8 rows and long K, which are one chain of loads (a row of 2048 x 4096 11.9 -> 9.5 us).
-template <int DUAL, int UB>
+// up to 8 rows and long K, which are one chain of loads (a row of 2048 x 4096 11.9 -> 9.5 us), and for few workgroups.
+// ROWS: of a workgroup, 64, or 16 where workgroups are few (narrow outputs: their rows' chains then run side by side).
+template <int DUAL, int UB, int ROWS>
 __global__ __launch_bounds__(256) void gemm_any_rows_kernel(AnyGemmArgs p) {
   constexpr int NM = 1 + DUAL;
   __shared__ f32x4 red[4][2 * NM][64];
   int grp, r0, rend;
-  if (!locate_tile(p, blockIdx.y, grp, r0, rend)) return;
+  if (!locate_tile(p, blockIdx.y, grp, r0, rend, ROWS)) return;
   const int64_t b = blockIdx.z, wsel = p.group_off != nullptr ? grp : b;
   const int n0 = blockIdx.x * 16, K = p.K;
   const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = l & 15, lk = 8 * (l >> 4);
@@ -289,9 +290,9 @@ __global__ __launch_bounds__(256) void gemm_any_rows_kernel(AnyGemmArgs p) {
   const int64_t wo = wsel * p.w_bs + (int64_t)min(n, p.N - 1) * p.ldw;   // (columns past N: the last one's, never stored)
   const bf16_t* w = reinterpret_cast<const bf16_t*>(p.w) + wo;
   const bf16_t* w2 = DUAL ? reinterpret_cast<const bf16_t*>(p.w2) + wo : nullptr;
-  rend = min(rend, r0 + BM);
+  rend = min(rend, r0 + ROWS);
   for (; r0 < rend; r0 += 32) {
-    const bool two = rend - r0 > 16;   // (workgroup-uniform)
+    const bool two = ROWS > 16 && rend - r0 > 16;   // (workgroup-uniform)
     const bf16_t* ar[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {      // (rows past the end: the pass's first, never stored)
@@ -853,9 +854,19 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st) {
     const int64_t tiles = (int64_t)grid.x * mt * g.batch;
     if (al && (g.group_off ? g.M <= 512 && tiles < 768 : g.M <= 64 || tiles <= (!broad ? 128 : (g.M < 1024 ? 256 : 64)))) {
       const dim3 gr((g.N + 15) / 16, mt, g.batch);
+      // A workgroup of 16 rows where all of them together are no more than the CUs and a wave's k is a chain of several loads, which
+      // then are all under way (us, 64 rows / 16: 8 x 1024 at 32 rows 4.7, 3.6, at 2048 8.3, 3.8; 16 x 1536 at 512 11.4, 6.0; 128 x 768 at 300
+      // 7.8, 4.1; 1024 x 512 at 64, two passes in one, 6.4, 4.1). With one pass of K = 512 there is little to gain (128 x 512 at 32
+      // rows 3.9, 4.0, at 8 3.3, 3.7).
+      const dim3 gn(gr.x, (g.M + 15) / 16, g.batch);
+      if (!g.group_off && g.K > (g.M > 32 ? 256 : 512) && (int64_t)gn.x * gn.y * gn.z <= cu_count()) {
+        auto kern = dual ? gemm_any_rows_kernel<1, 2, 16> : (g.K > 512 ? gemm_any_rows_kernel<0, 4, 16> : gemm_any_rows_kernel<0, 2, 16>);
+        hipLaunchKernelGGL(kern, gn, block, 0, st, g);
+        return;
+      }
       const bool deep = g.M <= 8 && g.K > 512;
-      auto kern = dual ? (deep ? gemm_any_rows_kernel<1, 2> : gemm_any_rows_kernel<1, 1>)
-                       : (deep ? gemm_any_rows_kernel<0, 4> : gemm_any_rows_kernel<0, 1>);
+      auto kern = dual ? (deep ? gemm_any_rows_kernel<1, 2, BM> : gemm_any_rows_kernel<1, 1, BM>)
+                       : (deep ? gemm_any_rows_kernel<0, 4, BM> : gemm_any_rows_kernel<0, 1, BM>);
       hipLaunchKernelGGL(kern, gr, block, 0, st, g);
       return;
     }

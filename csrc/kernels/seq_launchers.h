@@ -325,12 +325,19 @@ void launch_selective_scan(const SelectiveScanArgs& a, int T, float* scratch, hi
 // idx, wts [T][top]: the `top` largest of s + corr with s by `score`: 0 sigmoid(z), 1 softmax(z) over all E;
 // wts = s of the chosen / (their sum + norm_eps) * scale. score 2: the `top` largest of z + corr, wts = softmax of z over
 // the chosen alone, times scale
-void launch_moe_route(const float* z, const float* corr, int T, int E, int top, float norm_eps, int score, float scale,
-                      int32_t* idx, float* wts, hipStream_t st);
+struct RouteArgs {
+  const float* z = nullptr; const float* corr = nullptr;   // [T][E], [E] (null: none)
+  int T = 0, E = 0, top = 0, score = 0;
+  float norm_eps = 0.f, scale = 1.f;
+  int32_t* idx = nullptr; float* wts = nullptr;
+};
+void launch_moe_route(const RouteArgs& a, hipStream_t st);
 // counting sort of the T * top (token, choice) pairs by expert: rows[p] = token, pos[t * top + c] = p,
 // off[E + 1] = group boundaries
 void launch_moe_sort(const int32_t* idx, int T, int E, int top, int32_t* rows, int32_t* pos, int32_t* off,
                      hipStream_t st);
+// both, in one launch where the step has few tokens
+void launch_moe_route_sort(const RouteArgs& a, int32_t* rows, int32_t* pos, int32_t* off, hipStream_t st);
 // out[t] = sum_c wts[t][c] * y[pos[t][c]] [+ add[t]] (add: out's dtype)
 void launch_moe_combine(const void* y, const int32_t* pos, const float* wts, int T, int W, int top, int y_f32,
                         const void* add, void* out, int out_f32, hipStream_t st);

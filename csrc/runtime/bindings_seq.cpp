@@ -819,29 +819,51 @@ void selective_scan(const Tensor& x, const Tensor& dt, const Tensor& B, const Te
   vgate::launch_selective_scan(p, (int)T, scratch.data_ptr<float>(), cur_stream());
 }
 
-void moe_route(const Tensor& z, const OptT& corr, int64_t top, double norm_eps, Tensor& idx, Tensor& wts, int64_t score,
-               double scale) {
+vgate::RouteArgs route_args(const Tensor& z, const OptT& corr, int64_t top, double norm_eps, Tensor& idx, Tensor& wts, int64_t score,
+                            double scale) {
   TORCH_CHECK(score >= 0 && score <= 2, "moe_route: score 0 (sigmoid), 1 (softmax) or 2 (softmax over the chosen)");
   TORCH_CHECK(z.is_cuda() && z.scalar_type() == torch::kFloat32 && z.is_contiguous() && z.dim() == 2, "moe_route: z fp32 [T, E]");
+  vgate::RouteArgs a;
   const int64_t T = z.size(0), E = z.size(1);
   TORCH_CHECK(top >= 1 && top <= E, "moe_route: top");
   TORCH_CHECK(idx.is_cuda() && idx.scalar_type() == torch::kInt32 && idx.is_contiguous() && idx.numel() == T * top, "moe_route: idx");
   TORCH_CHECK(wts.is_cuda() && wts.scalar_type() == torch::kFloat32 && wts.is_contiguous() && wts.numel() == T * top, "moe_route: wts");
+  a.z = z.data_ptr<float>(); a.corr = f32p(corr, "corr", E);
+  a.T = (int)T; a.E = (int)E; a.top = (int)top; a.score = (int)score;
+  a.norm_eps = (float)norm_eps; a.scale = (float)scale;
+  a.idx = idx.data_ptr<int32_t>(); a.wts = wts.data_ptr<float>();
+  return a;
+}
+
+void moe_route(const Tensor& z, const OptT& corr, int64_t top, double norm_eps, Tensor& idx, Tensor& wts, int64_t score,
+               double scale) {
+  const auto a = route_args(z, corr, top, norm_eps, idx, wts, score, scale);
   c10::DeviceGuard guard(z.device());
-  vgate::launch_moe_route(z.data_ptr<float>(), f32p(corr, "corr", E), (int)T, (int)E, (int)top, (float)norm_eps,
-                          (int)score, (float)scale, idx.data_ptr<int32_t>(), wts.data_ptr<float>(), cur_stream());
+  vgate::launch_moe_route(a, cur_stream());
+}
+
+void sort_outputs(int64_t T, int64_t E, int64_t top, Tensor& rows, Tensor& pos, Tensor& off) {
+  TORCH_CHECK(E >= 1 && E <= 4096, "moe_sort: experts 1..4096");
+  TORCH_CHECK(rows.numel() == T * top && pos.numel() == T * top && off.numel() == E + 1, "moe_sort: outputs");
+  i32p(rows, "rows", 0); i32p(pos, "pos", 0); i32p(off, "off", 0);
 }
 
 void moe_sort(const Tensor& idx, int64_t E, Tensor& rows, Tensor& pos, Tensor& off) {
   TORCH_CHECK(idx.dim() == 2, "moe_sort: idx [T, top]");
   const int64_t T = idx.size(0), top = idx.size(1);
-  TORCH_CHECK(E >= 1 && E <= 4096, "moe_sort: experts 1..4096");
   const int32_t* ip = i32p(idx, "idx", T * top);
-  TORCH_CHECK(rows.numel() == T * top && pos.numel() == T * top && off.numel() == E + 1, "moe_sort: outputs");
-  i32p(rows, "rows", 0); i32p(pos, "pos", 0); i32p(off, "off", 0);
+  sort_outputs(T, E, top, rows, pos, off);
   c10::DeviceGuard guard(idx.device());
   vgate::launch_moe_sort(ip, (int)T, (int)E, (int)top, rows.data_ptr<int32_t>(), pos.data_ptr<int32_t>(),
                          off.data_ptr<int32_t>(), cur_stream());
+}
+
+void moe_route_sort(const Tensor& z, const OptT& corr, int64_t top, double norm_eps, Tensor& idx, Tensor& wts, Tensor& rows, Tensor& pos,
+                    Tensor& off, int64_t score, double scale) {
+  const auto a = route_args(z, corr, top, norm_eps, idx, wts, score, scale);
+  sort_outputs(a.T, a.E, a.top, rows, pos, off);
+  c10::DeviceGuard guard(z.device());
+  vgate::launch_moe_route_sort(a, rows.data_ptr<int32_t>(), pos.data_ptr<int32_t>(), off.data_ptr<int32_t>(), cur_stream());
 }
 
 void moe_combine(const Tensor& y, const Tensor& pos, const Tensor& wts, Tensor& out, const OptT& add) {
@@ -1029,6 +1051,8 @@ void bind_seq(pybind11::module& m) {
   m.def("tanh_norm_rows", &tanh_norm_rows, "tanh(alpha x) * w + b over (gathered) rows");
   m.def("hyper_mix", &hyper_mix, "write of a sublayer to the stream's copies + the next sublayer's normed read + their sum");
   m.def("moe_sort", &moe_sort, "counting sort of (token, choice) pairs by expert");
+  m.def("moe_route_sort", &moe_route_sort, "moe_route and moe_sort", py::arg("z"), py::arg("corr"), py::arg("top"), py::arg("norm_eps"),
+        py::arg("idx"), py::arg("wts"), py::arg("rows"), py::arg("pos"), py::arg("off"), py::arg("score") = 0, py::arg("scale") = 1.0);
   m.def("moe_combine", &moe_combine, "weighted sum of a token's expert rows (+ a shared row)", py::arg("y"), py::arg("pos"),
         py::arg("wts"), py::arg("out"), py::arg("add") = py::none());
 }

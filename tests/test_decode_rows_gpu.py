@@ -1,5 +1,5 @@
-"""Decoded tokens of hybrid models: latent attention whose keys several workgroups share, against the CPU
-form."""
+"""Decoded tokens of hybrid models: latent attention whose keys several workgroups share, routing with its sort, and narrow products,
+against the ops' CPU forms."""
 import pytest
 import torch
 
@@ -32,3 +32,42 @@ def test_latent_attn_of_decoded_tokens(rank, rot, H, S):
                         window=window, sink=sink.cuda())
         seq.latent_attn(qa.float(), cache.float(), tables, ctx, start, want, scale, H, rank, rot, num_seqs=S, window=window, sink=sink)
         assert ((got.float().cpu() - want).abs() <= 4 * 2.0 ** -8 + 1e-4).all()
+
+
+@pytest.mark.parametrize("score", [seq.ROUTE_SIGMOID, seq.ROUTE_SOFTMAX, seq.ROUTE_TOP_SOFTMAX])
+@pytest.mark.parametrize("T,E,top", [(1, 1, 1), (7, 8, 2), (16, 64, 6), (16, 65, 4), (17, 60, 60), (65, 8, 2), (40, 65, 4), (33, 512, 8), (5, 600, 3)])
+def test_moe_route_sort(T, E, top, score):
+    """One launch and two, on either side of their line: the choice and weights of the CPU form, every pair in its expert's stretch once."""
+    g = torch.Generator().manual_seed(T + E)
+    z, corr = torch.randn(T, E, generator=g), 0.1 * torch.randn(E, generator=g)
+
+    def run(dev):
+        idx, wts = torch.empty(T, top, dtype=torch.int32, device=dev), torch.empty(T, top, device=dev)
+        rows, pos, off = (torch.full((n,), -1, dtype=torch.int32, device=dev) for n in (T * top, T * top, E + 1))
+        seq.moe_route_sort(z.to(dev), corr.to(dev), top, 1e-20, idx, wts, rows, pos, off, score=score, scale=1.5)
+        return [t.cpu() for t in (idx, wts, rows, pos, off)]
+
+    (idx, wts, rows, pos, off), want = run("cuda"), run("cpu")
+    assert torch.equal(idx, want[0]) and torch.allclose(wts, want[1], rtol=1e-5, atol=1e-7) and torch.equal(off, want[4])
+    assert sorted(pos.tolist()) == list(range(T * top))
+    token = torch.arange(T * top) // top
+    assert torch.equal(rows[pos.long()], token.int())
+    assert (off[idx.flatten().long()] <= pos).all() and (pos < off[idx.flatten().long() + 1]).all()
+
+
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 2047, 4096, 4097])
+@pytest.mark.parametrize("N,K", [(1, 264), (8, 1024), (16, 520), (72, 512), (17, 1000), (128, 2056)])
+def test_narrow_products(M, N, K):
+    """Workgroups of 16 rows and of 64, on either side of their line, ragged columns and k. fp32 sums of products of bf16: |error| below
+    K 2^-24 of the sum of the products' sizes."""
+    g = torch.Generator().manual_seed(M + N)
+    a, w, w2 = (torch.randn(r, K, generator=g).bfloat16().cuda() for r in (M, N, N))
+    bias = torch.randn(N, generator=g).cuda()
+    bound = (a.float().abs() @ w.float().abs().t()).max().item() * K * 2.0 ** -24 + 1e-6
+    out = torch.empty(M, N, device="cuda")
+    seq.gemm(a, w, out, bias=bias)
+    want = a.double() @ w.double().t() + bias
+    assert (out - want).abs().max().item() <= bound
+    seq.gemm(a, w, out, w2=w2, act=seq.ACT_SILU_MUL)
+    gate, up = a.double() @ w.double().t(), a.double() @ w2.double().t()
+    assert (out - torch.nn.functional.silu(gate) * up).abs().max().item() <= bound * (1.1 * up.abs().max().item() + gate.abs().max().item())

@@ -958,11 +958,10 @@ class MoEFF:
         z = self.router(h, out_f32=True)
         idx = torch.empty(T, self.top, dtype=torch.int32, device=dev)
         wts = torch.empty(T, self.top, dtype=torch.float32, device=dev)
-        seq.moe_route(z, self.corr, self.top, self.sum_eps, idx, wts, score=self.score, scale=self.scale)
         rows = torch.empty(T * self.top, dtype=torch.int32, device=dev)
         pos = torch.empty(T * self.top, dtype=torch.int32, device=dev)
         off = torch.empty(self.E + 1, dtype=torch.int32, device=dev)
-        seq.moe_sort(idx, self.E, rows, pos, off)
+        seq.moe_route_sort(z, self.corr, self.top, self.sum_eps, idx, wts, rows, pos, off, score=self.score, scale=self.scale)
         a1 = torch.empty(T * self.top, self.ff, dtype=dt, device=dev)
         if self.gated:
             seq.gemm(h, self.gate, a1, w2=self.up, a_rows=rows, group_off=off, act=self.act, limit=self.limit,

@@ -387,6 +387,15 @@ def moe_sort(idx, E: int, rows, pos, off) -> None:
     off.copy_(torch.cat([torch.zeros(1, dtype=torch.long), cnt.cumsum(0)]).int())
 
 
+def moe_route_sort(z, corr, top: int, norm_eps: float, idx, wts, rows, pos, off, score: int = ROUTE_SIGMOID, scale: float = 1.0) -> None:
+    """:func:`moe_route` and :func:`moe_sort` of its choice (one launch where the step has few tokens)."""
+    if z.is_cuda:
+        _C().moe_route_sort(z, corr, top, norm_eps, idx, wts, rows, pos, off, score, scale)
+        return
+    moe_route(z, corr, top, norm_eps, idx, wts, score=score, scale=scale)
+    moe_sort(idx, z.shape[1], rows, pos, off)
+
+
 def moe_combine(y, pos, wts, out, add=None) -> None:
     """out[t] = sum_c wts[t, c] * y[pos[t, c]] [+ add[t]] (fp32 sum; out bf16 or fp32)."""
     if y.is_cuda:
