@@ -82,6 +82,70 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ShortConvArgs p) {
   }
 }
 
+// R tokens a workgroup, 8 channels a thread (16-B pieces), at most four taps, bf16: rows, weights and the slot's rows are asked for together
+// and a row once per R tokens, where the kernel above waits for each tap of each token (3072 channels, us:
+// 32 tokens of 32 sequences 6.8 -> 3.3, 300 of 4 8.6 -> 4.6, 1024 of 8 25.8 -> 9.0, 2048 of 8 33.6 -> 13.7).
+template <int R>
+__global__ __launch_bounds__(256) void short_conv_run_kernel(ShortConvArgs p) {
+  const int total = p.query_start[p.S], last = min((int)(blockIdx.x + 1) * R, total);
+  const int c = (blockIdx.y * 256 + threadIdx.x) * 8, cc = min(c, p.C - 8);   // (channels past the last: its own, never stored)
+  const bf16_t* x = reinterpret_cast<const bf16_t*>(p.x);
+  f32x4 w[4][2], b[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};   // w[3]: the token's own row
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int i = m - (4 - p.taps);
+      w[m][q] = i >= 0 ? *reinterpret_cast<const f32x4*>(p.w + (int64_t)max(i, 0) * p.C + cc + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  if (p.b != nullptr) {
+    b[0] = *reinterpret_cast<const f32x4*>(p.b + cc);
+    b[1] = *reinterpret_cast<const f32x4*>(p.b + cc + 4);
+  }
+  for (int t = blockIdx.x * R; t < last;) {   // the run's sequences in turn (most runs have one)
+    uint4 v[R + 3];   // rows t - 3 ..
+#pragma unroll
+    for (int m = 0; m < R + 3; ++m) v[m] = ld16(x + (int64_t)min(max(t - 3 + m, 0), last - 1) * p.ldx + cc);
+    const int s = seq_of_row_wave(p.query_start, p.S, t);
+    const int slot = p.state_slots[s], t0 = p.query_start[s], t1 = p.query_start[s + 1], end = min(last, t1);
+    const int pos0 = p.context_lens[s] - (t1 - t0);
+    if (slot >= 0) {
+      f32x4 k[3][2];   // rows before the portion, from the slot
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        const int r = t - 3 + m - t0 + p.taps - 1;
+        const bool kept = t - 3 + m < t0 && r >= 0 && pos0 > 0;   // (uniform)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          k[m][q] = kept ? *reinterpret_cast<const f32x4*>(p.kept + ((int64_t)slot * (p.taps - 1) + r) * p.C + cc + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        if (t + u >= end) break;
+        float y[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = b[e >> 2][e & 3];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          if (m < 4 - p.taps) continue;
+          float f[8];
+          unpack8(v[u + m], f);
+          if (u + m < 3 && t - 3 + u + m < t0)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] = k[u + m < 3 ? u + m : 0][e >> 2][e & 3];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) y[e] = fmaf(w[m][e >> 2][e & 3], f[e], y[e]);
+        }
+        if (p.act)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) y[e] = silu_f(y[e]);
+        if (c < p.C) *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(p.out) + (int64_t)(t + u) * p.ldo + c) = pack8(y);
+      }
+    }
+    t = end;
+  }
+}
+
 enum { SCAN_WHOLE = 0, SCAN_LOCAL = 1, SCAN_OUTPUT = 2 };
 
 __device__ __forceinline__ bool locate_chunk(const SelectiveScanArgs& p, int CH, int bx, int& s, int& t0, int& t1) {
@@ -297,7 +361,14 @@ void launch_short_conv(const ShortConvArgs& a, hipStream_t st) {
   const int per = vec ? 256 * 8 : 256;
   int gy = (a.C + per - 1) / per;
   if (gy > 64) gy = 64;
-  if (vec) hipLaunchKernelGGL(short_conv_kernel<8>, dim3(a.T, gy), dim3(256), 0, st, a);
+  const uintptr_t rows = reinterpret_cast<uintptr_t>(a.w) | reinterpret_cast<uintptr_t>(a.b) | reinterpret_cast<uintptr_t>(a.kept);
+  if (vec && a.taps <= 4 && (rows & 15) == 0) {
+    // eight tokens a workgroup where a sequence has that many as a rule and the launch still fills the chip (2048 of 8
+    // 13.7 us, by workgroups of one token 18.6, 1024 of 8 9.0, 10.2)
+    const dim3 grid((unsigned)((a.T + 7) / 8), (a.C + per - 1) / per);
+    if (a.T >= 512 && a.T >= 8 * a.S) hipLaunchKernelGGL(short_conv_run_kernel<8>, grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(short_conv_run_kernel<1>, dim3(a.T, grid.y), dim3(256), 0, st, a);
+  } else if (vec) hipLaunchKernelGGL(short_conv_kernel<8>, dim3(a.T, gy), dim3(256), 0, st, a);
   else hipLaunchKernelGGL(short_conv_kernel<1>, dim3(a.T, gy), dim3(256), 0, st, a);
 }
 

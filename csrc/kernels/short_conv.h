@@ -80,6 +80,18 @@ __device__ __forceinline__ void short_conv_run8(const void* x, int64_t ld, int c
   }
 }
 
+// The sequence of row t (below) by a whole wave, a lane per sequence: one wait for memory where the halving above takes one a step.
+__device__ __forceinline__ int seq_of_row_wave(const int32_t* query_start, int S, int t) {
+  int s = 0;
+  for (int i0 = 0; i0 < S; i0 += 64) {
+    const int i = i0 + (threadIdx.x & 63);
+    const unsigned long long before = __ballot(i < S && query_start[min(i, S - 1) + 1] <= t);   // sequences that end at or before row t
+    s += __popcll(before);
+    if (before != ~0ull) break;
+  }
+  return min(s, S - 1);
+}
+
 __device__ __forceinline__ int seq_of_row(const int32_t* query_start, int S, int t) {
   int lo = 0, hi = S - 1;  // query_start[s] <= t < query_start[s + 1]
   while (lo < hi) {

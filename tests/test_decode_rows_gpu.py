@@ -71,3 +71,23 @@ def test_narrow_products(M, N, K):
     seq.gemm(a, w, out, w2=w2, act=seq.ACT_SILU_MUL)
     gate, up = a.double() @ w.double().t(), a.double() @ w2.double().t()
     assert (out - torch.nn.functional.silu(gate) * up).abs().max().item() <= bound * (1.1 * up.abs().max().item() + gate.abs().max().item())
+
+
+@pytest.mark.parametrize("C", [8, 2056])
+@pytest.mark.parametrize("taps", [1, 3, 4])
+@pytest.mark.parametrize("lens", [[1] * 70, [1] * 64 + [0, 3, 0], [5] * 110, [0, 700, 0, 9, 3], [1]])
+def test_short_conv_runs(C, taps, lens):
+    """Runs of one and of eight tokens across sequences of one to hundreds, some without a slot or without tokens, rows past the last
+    sequence: the bits of the kernel for rows that are not of whole pieces."""
+    g = torch.Generator().manual_seed(C + taps + len(lens))
+    T, S = sum(lens), len(lens)
+    x = torch.randn(T + 5, 2 * C, generator=g).bfloat16().cuda()[:, C:]
+    w, b, kept = (torch.randn(s, generator=g).cuda() for s in ((taps, C), (C,), (S, taps - 1, C)))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    slots = i32([-1 if s % 5 == 3 else S - 1 - s for s in range(S)])
+    ctx, start = i32([n + (13 if s % 2 else 0) for s, n in enumerate(lens)]), i32([sum(lens[:s]) for s in range(S + 1)])
+    a, o = torch.full((T + 5, C), 7.0, dtype=torch.bfloat16, device="cuda"), torch.full((T + 5, C + 1), 7.0, dtype=torch.bfloat16, device="cuda")[:, 1:]
+    for silu in (False, True):
+        seq.short_conv(x, w, b, kept, slots, ctx, start, a, silu=silu)
+        seq.short_conv(x, w, b, kept, slots, ctx, start, o, silu=silu)
+        assert torch.equal(a, o) and bool((a[T:] == 7.0).all())
