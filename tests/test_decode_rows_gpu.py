@@ -1,5 +1,5 @@
-"""Decoded tokens of hybrid models: latent attention whose keys several workgroups share, routing with its sort, and narrow products,
-against the ops' CPU forms."""
+"""Decoded tokens of hybrid models: latent attention whose keys several workgroups share, routing with its sort, narrow products and short
+convolutions, against the ops' other forms; linear attention's chunks against 64 bits."""
 import pytest
 import torch
 
@@ -91,3 +91,37 @@ def test_short_conv_runs(C, taps, lens):
         seq.short_conv(x, w, b, kept, slots, ctx, start, a, silu=silu)
         seq.short_conv(x, w, b, kept, slots, ctx, start, o, silu=silu)
         assert torch.equal(a, o) and bool((a[T:] == 7.0).all())
+
+
+@pytest.mark.parametrize("mode", ["gated", "head", "bonus"])
+@pytest.mark.parametrize("D,V", [(128, 128), (72, 24), (64, 64), (24, 40)])
+@pytest.mark.parametrize("n", [129, 144, 145, 176, 191, 192, 255, 300])
+def test_linear_attention_chunks(mode, D, V, n):
+    """Portions whose last chunk of 64 ends at and around each 16 tokens, fp32, a state before them, against the recurrence in 64 bits. An
+    output is sums of D and of 64 terms, rounded some (D + 64) times by 2^-24 at most."""
+    g = torch.Generator().manual_seed(n + D)
+    H, d = 2, "cuda"
+    q, k, v, z = (torch.randn(n, H * w, generator=g).to(d) for w in (D, D, V, D))
+    state = torch.randn(1, H, D, V, generator=g).to(d)
+    bonus = torch.randn(H, D, generator=g).to(d) if mode == "bonus" else None
+    fade = torch.tensor([0.5, 0.97], device=d) if mode == "head" else None
+    if mode == "head":
+        a, z = fade.double()[None, :, None].expand(n, H, D), None
+    elif mode == "bonus":
+        z = z - 2.0
+        a = torch.exp(-torch.exp(z.double())).view(n, H, D)
+    else:
+        a = torch.exp(torch.nn.functional.logsigmoid(z.double()) / 4.0).view(n, H, D)
+    S, want = state[0].double(), torch.empty(n, H, V, dtype=torch.float64, device=d)
+    for t in range(n):
+        kv = k[t].double().view(H, D, 1) * v[t].double().view(H, 1, V)
+        new = a[t][:, :, None] * S + kv
+        read = S + bonus.double()[:, :, None] * kv if mode == "bonus" else new
+        want[t], S = (read * q[t].double().view(H, D, 1)).sum(1), new
+    want = want / torch.sqrt((want * want).mean(-1, keepdim=True) + 1e-6)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=d)  # noqa: E731
+    out, gate = torch.empty(n, H * V, device=d), torch.full((n, H * V), 40.0, device=d)
+    seq.linear_attn(q, k, v, gate, z, fade, 4.0, 1.0, False, None, False, False, state, i32([0]), i32([n + 7]), i32([0, n]), out, 1e-6,
+                    decay_exp=mode == "bonus", bonus=bonus)
+    for got, exact in ((out.view(n, H, V), want), (state[0], S)):
+        assert ((got.double() - exact).norm() / exact.norm()).item() < (D + 64) * 2.0 ** -24
