@@ -300,7 +300,7 @@ __global__ __launch_bounds__(256, NCT > 16 ? 1 : 2) void latent_attn_mfma_kernel
                                                                 const float* __restrict__ sink, int parts,
                                                                 float* __restrict__ part_o, float* __restrict__ part_ml) {
   __shared__ __attribute__((aligned(16))) bf16_t pl[4][16][40];
-  __shared__ float mrg_m[4][16], mrg_l[4][16], row_l[16];
+  __shared__ float mrg_m[4][16], mrg_l[4][16], mrg_f[4][16], row_l[16];
   constexpr int OS = 16 * NCT + 4;        // row stride of the area (the four rows of an instruction in different banks)
   extern __shared__ __attribute__((aligned(16))) float mrg_o[];  // split mode: the waves' weighted latents [4][16][OS]
   const int E = a.rank + a.rot, KR = a.rank;
@@ -436,9 +436,9 @@ __global__ __launch_bounds__(256, NCT > 16 ? 1 : 2) void latent_attn_mfma_kernel
       float L = 0.f;
 #pragma unroll
       for (int w = 0; w < 4; ++w) L += mrg_l[w][r] * exp2f(mrg_m[w][r] - Ms);  // a wave that saw no key: l = 0, exp2(-inf) = 0
-      const float f = exp2f(m[i] - Ms);
 #pragma unroll
-      for (int ct = 0; ct < NCT; ++ct) area[r * OS + 16 * ct + lr] = O[ct][i] * f;
+      for (int ct = 0; ct < NCT; ++ct) area[r * OS + 16 * ct + lr] = O[ct][i];
+      if (lr == 0) mrg_f[wv][r] = exp2f(m[i] - Ms);
       if (wv == 0 && lr == 0) {
         row_l[r] = L;
         if (np > 1) {
@@ -448,14 +448,19 @@ __global__ __launch_bounds__(256, NCT > 16 ? 1 : 2) void latent_attn_mfma_kernel
       }
     }
     __syncthreads();
-    // four columns a thread and turn, the waves' parts added in wave order; np > 1 (workgroup-uniform): handed on, the merge kernel
-    // finishes the rows
+    // four columns a thread and turn, the waves' parts scaled and added in wave order, each by one fused step; np > 1 (workgroup-uniform):
+    // handed on, the merge kernel finishes the rows
 #pragma unroll 4
     for (int e = threadIdx.x; e < 16 * 4 * NCT; e += 256) {
       const int r = e / (4 * NCT), col = 4 * (e % (4 * NCT));
       const float* o = mrg_o + r * OS + col;
-      const f32x4 y = ((*reinterpret_cast<const f32x4*>(o) + *reinterpret_cast<const f32x4*>(o + 16 * OS)) +
-                       *reinterpret_cast<const f32x4*>(o + 32 * OS)) + *reinterpret_cast<const f32x4*>(o + 48 * OS);
+      f32x4 y = *reinterpret_cast<const f32x4*>(o) * mrg_f[0][r];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(o + 16 * w * OS);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) y[j] = fmaf(v[j], mrg_f[w][r], y[j]);
+      }
       if (np > 1) {
         *reinterpret_cast<f32x4*>(part_o + slot * (16 * 16 * NCT) + r * (16 * NCT) + col) = y;
       } else if (r < nrows) {

@@ -34,6 +34,26 @@ def test_latent_attn_of_decoded_tokens(rank, rot, H, S):
         assert ((got.float().cpu() - want).abs() <= 4 * 2.0 ** -8 + 1e-4).all()
 
 
+@pytest.mark.parametrize("rank,rot", [(128, 64), (256, 64), (512, 64), (264, 64), (96, 32)])
+def test_latent_attn_adds_its_waves_by_fused_steps(rank, rot, monkeypatch):
+    """Two waves whose sums are A and -A, a third with the row's maximum, so that both are scaled by the same inexact f: o0 f rounded, then
+    fma(o1, f, .) leaves the rounding of A f, at most 2^-24 of it and seldom none. (Both rounded ahead of the sum would leave zeros.)"""
+    monkeypatch.setattr(seq, "LATENT_SPLIT", False)   # (one workgroup: waves take tiles of 32 keys in turn)
+    H, E = 2, rank + rot
+    g = torch.Generator().manual_seed(rank)
+    A = torch.randn(rank, generator=g).bfloat16()
+    cache = torch.zeros(6, 16, E, dtype=torch.bfloat16)
+    cache[0, 0, :rank], cache[2, 0, :rank], cache[4, 0, rank] = A, -A, 1.3
+    qa = torch.zeros(1, H, E, dtype=torch.bfloat16)
+    qa[:, :, rank] = 1.0
+    out = torch.empty(1, H, rank, dtype=torch.bfloat16, device="cuda")
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    seq.latent_attn(qa.cuda(), cache.cuda(), i32([[0, 1, 2, 3, 4, 5]]), i32([96]), i32([0, 1]), out, 1.0, H, rank, rot,
+                    cache_t=cache[:, :, :rank].transpose(1, 2).contiguous().cuda())
+    out = out.float().cpu()
+    assert (out.abs() <= 2.0 ** -23 * A.float().abs()).all() and (out != 0).float().mean().item() > 0.8
+
+
 @pytest.mark.parametrize("score", [seq.ROUTE_SIGMOID, seq.ROUTE_SOFTMAX, seq.ROUTE_TOP_SOFTMAX])
 @pytest.mark.parametrize("T,E,top", [(1, 1, 1), (7, 8, 2), (16, 64, 6), (16, 65, 4), (17, 60, 60), (65, 8, 2), (40, 65, 4), (33, 512, 8), (5, 600, 3)])
 def test_moe_route_sort(T, E, top, score):
