@@ -35,9 +35,8 @@
 //            I' = g_(1..CT) I + sum_j g_(j+1..CT) k_j v_j^T
 //          (with a bonus the products stop at i - 1 and the term j = i is q_i . u k_i). Every product of decays is a product
 //          of factors <= 1 taken in order. local: the second sum, fp32 MFMA (16x16x4); carry as above; output: the
-//          triangle of weighted products (16 tokens at a time: a lane holds k_j g of four D / 32 channels and walks i; tiles below
-//          those with fp32 MFMA), then both products with fp32 MFMA, norm and gate. 2048 tokens, 8 heads of 128: 72 to 79 us, by the
-//          scan in chunks 162.
+//          triangle of weighted products (a lane holds k_j g of four D / 32 channels and walks i), then both products
+//          with fp32 MFMA, norm and gate. 2048 tokens, 8 heads of 128: 100 us, by the scan in chunks 162.
 #include <algorithm>
 
 #include "chunks.h"
@@ -676,11 +675,8 @@ __global__ __launch_bounds__(256) void linear_chunk_carry_kernel(LinearAttnArgs 
 }
 
 // grid (chunk, head), 512 threads: the outputs of a chunk from the state it starts from. Wave w owns the columns 16 w ..
-// Bound by chains through LDS with two waves per SIMD: a row's operands are asked for a row ahead, and the decays' products read their 16
-// tokens together (29 chunks of 8 heads of 128: 43.5 -> 37.0 us). Only the triangles of 16 tokens are walked row by row; the tiles below
-// them are products of 16 tokens' queries and keys on the matrix cores, each with the decays of its own 16 tokens (factors <= 1, nothing is
-// divided; those of whole 16s between them go onto the keys): 72 walked rows to a SIMD become 24 (gated 48.3 -> 39.2, constant decay 39.8 ->
-// 30.5; error against 64 bits 1.82e-7 -> 1.80e-7, 2.07e-7 -> 2.01e-7, with a bonus 1.61e-7 -> 1.60e-7).
+// Bound by chains through LDS with two waves per SIMD, the triangle's rows first: a row's operands are asked for a row ahead, and the decays'
+// products read their 16 tokens together (29 chunks of 8 heads of 128: 43.5 -> 37.0 us).
 template <int DP, bool F32, bool PRE>
 __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, int lim, const float* __restrict__ cstate,
                                                              float* __restrict__ oraw) {
@@ -690,7 +686,7 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
   float* lk = la + CT * DS;           // keys
   float* lq = lk + CT * DS;           // queries, then times the decays up to them
   float* tr = lq + CT * DS;           // [CT][CTP] the triangle
-  float* red = tr + CT * CTP;         // [8][CT] rows' sums of squares; before, [8][DP] decays of each 16 tokens and before them
+  float* red = tr + CT * CTP;         // [8][CT] rows' sums of squares; before, [4][DP] decays of 16 tokens
   int s, t0, t1;
   if (!locate_chunk<CT>(p.query_start, p.state_slots, p.S, lim, blockIdx.x, s, t0, t1)) return;
   const int h = blockIdx.y, D = p.D, V = p.V, tid = threadIdx.x;
@@ -732,9 +728,9 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
   }
   for (int e = tid; e < CT * CTP; e += 512) tr[e] = 0.f;
   __syncthreads();
-  {  // the triangles of 16 tokens on the diagonal: a wave owns eight columns j, lane = (channel group dg of eight, j). Waves w and w + 4,
-     // which share a SIMD, take one with 16 rows and one with 8
-    const int jb = w < 4 ? w : 11 - w, iend = (jb | 1) * 8 + 8;
+  {  // the triangle: a wave owns eight columns j, lane = (channel group dg of eight, j). A column has CT - j rows: waves w and
+     // w + 4, which share a SIMD, take stretches that add up alike
+    const int jb = w < 4 ? w : 11 - w;
     const int dg = l >> 3, j = 8 * jb + (l & 7);
     float x[4 * X], diag = 0.f;
 #pragma unroll
@@ -755,12 +751,12 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
       }
     };
     row(8 * jb);
-    for (int i = 8 * jb; i < iend; ++i) {
+    for (int i = 8 * jb; i < CT; ++i) {
       float r = 0.f;
       f32x4 a[X], q[X];
 #pragma unroll
       for (int m = 0; m < X; ++m) { a[m] = na[m]; q[m] = nq[m]; }
-      row(min(i + 1, iend - 1));
+      row(min(i + 1, CT - 1));
 #pragma unroll
       for (int m = 0; m < X; ++m)
 #pragma unroll
@@ -775,16 +771,14 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
     }
   }
   __syncthreads();
-  {  // within each 16 tokens, in place: queries times the decays up to them (with a bonus: before them), keys times the decays after
-     // them; red[m] = the decays of all 16. A channel and 16 tokens per thread
+  {  // q_i g_(1..i) (with a bonus g_(1..i-1)) in place: a channel and 16 tokens per thread
     const int d = tid & 127, part = tid >> 7;
+    float g = 1.f, a[16], q[16];   // (read together: a store between them would order the reads)
     if (d < DP) {
-      float g = 1.f, a[16], q[16], k[16];   // (read together: a store between them would order the reads)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         a[i] = la[(16 * part + i) * DS + d];
         q[i] = lq[(16 * part + i) * DS + d];
-        k[i] = lk[(16 * part + i) * DS + d];
       }
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
@@ -793,50 +787,17 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
         if (PRE) g *= a[i];
       }
       red[part * DP + d] = g;
-      g = 1.f;
-#pragma unroll
-      for (int i = 15; i >= 0; --i) {
-        k[i] *= g;
-        g *= a[i];
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        lq[(16 * part + i) * DS + d] = q[i];
-        lk[(16 * part + i) * DS + d] = k[i];
-      }
     }
-  }
-  __syncthreads();
-  // the six tiles below the diagonal, a wave each: q_i g_(I..i) . g_(between) k_j g_(j+1..J); the other two waves: the decays before each
-  // 16 tokens, red[4 + I]
-  if (w < 6) {
-    const int I = w < 1 ? 1 : (w < 3 ? 2 : 3), J = w - I * (I - 1) / 2;
-    f32x4 c[NT];   // (sums of 16 channels, then of those in pairs, as the walk above sums: long chains lose more)
+    __syncthreads();
+    if (d < DP) {
+      if (part > 0) {
+        float f = 1.f;
+        for (int m = 0; m < part; ++m) f *= red[m * DP + d];
 #pragma unroll
-    for (int m = 0; m < NT; ++m) c[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int n = 0; n < NT; ++n) {
-      const int at = 16 * n + 4 * kg;
-      const f32x4 A = ld4(&lq[(16 * I + lr) * DS + at]);
-      f32x4 K = ld4(&lk[(16 * J + lr) * DS + at]);
-      for (int m = J + 1; m < I; ++m) K *= ld4(&red[m * DP + at]);   // (uniform)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) c[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[e], K[e], c[n], 0, 0, 0);
-    }
-#pragma unroll
-    for (int o = NT / 2; o > 0; o /= 2)
-#pragma unroll
-      for (int m = 0; m < o; ++m) c[m] += c[m + o];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) tr[(16 * I + 4 * kg + i) * CTP + 16 * J + lr] = c[0][i];
-  } else {
-    for (int d = tid - 6 * 64; d < DP; d += 128) {
-      float f = 1.f;
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        red[(4 + m) * DP + d] = f;
-        f *= red[m * DP + d];
+        for (int i = 0; i < 16; ++i) q[i] *= f;
       }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) lq[(16 * part + i) * DS + d] = q[i];
     }
   }
   __syncthreads();
@@ -847,10 +808,7 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
   for (int n = 0; n < NT; ++n) {
     f32x4 A[CT / 16];
 #pragma unroll
-    for (int r = 0; r < CT / 16; ++r) {
-      A[r] = ld4(&lq[(16 * r + lr) * DS + 16 * n + 4 * kg]);
-      if (r > 0) A[r] *= ld4(&red[(4 + r) * DP + 16 * n + 4 * kg]);
-    }
+    for (int r = 0; r < CT / 16; ++r) A[r] = ld4(&lq[(16 * r + lr) * DS + 16 * n + 4 * kg]);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -890,7 +848,6 @@ __global__ __launch_bounds__(512) void linear_output_kernel(LinearAttnArgs p, in
       }
     return;
   }
-  __syncthreads();   // (the decays are read, the rows' sums come in their place)
   float wg[CT / 4];
   {
     int t[CT / 4], c[CT / 4];
@@ -965,7 +922,7 @@ void launch_small(const LinearAttnArgs& a, int T, const LinearPlan& plan, float*
     else hipLaunchKernelGGL((linear_short_kernel<128, F32, PRE>), grid, dim3(256), 0, st, a, lim, oraw);
   }
   if (chunks > 0) {
-    constexpr size_t bytes = ((size_t)3 * CT * (DP + 4) + CT * CTP + 8 * (DP > CT ? DP : CT)) * 4;
+    constexpr size_t bytes = ((size_t)3 * CT * (DP + 4) + CT * CTP + 8 * CT) * 4;
     auto out = linear_output_kernel<DP, F32, PRE>;
     static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(out), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                  (int)bytes) == hipSuccess;

@@ -145,3 +145,34 @@ def test_linear_attention_chunks(mode, D, V, n):
                     decay_exp=mode == "bonus", bonus=bonus)
     for got, exact in ((out.view(n, H, V), want), (state[0], S)):
         assert ((got.double() - exact).norm() / exact.norm()).item() < (D + 64) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("bonus", [False, True])
+@pytest.mark.parametrize("D,V", [(128, 128), (64, 64), (24, 64)])
+def test_linear_attention_weights_keys_token_by_token(D, V, bonus):
+    """What a token of the first chunk of 64 reads of each key: the key times the decays after it, one token at a time in fp32, then times the
+    query, whatever the tokens' distance. One channel is used, token j's value is 1 in column j, and eps is 2^60: nothing else rounds."""
+    n, fade, d = 200, torch.tensor([0.97], dtype=torch.float32), min(D - 1, 37)
+    g = torch.Generator().manual_seed(D + V)
+    q, k = torch.zeros(n, D), torch.zeros(n, D)
+    q[:, d], k[:, d] = torch.randn(n, generator=g), torch.randn(n, generator=g)
+    v = torch.zeros(n, V)
+    v[torch.arange(64), torch.arange(64)] = 1.0
+    u = torch.randn(1, D, generator=g)
+    want = torch.zeros(64, 64)
+    for j in range(64):
+        x = k[j, d]
+        want[j, j] = q[j, d] * x
+        if bonus:
+            want[j, j] = (q[j, d] * u[0, d]) * x
+        for i in range(j + 1, 64):
+            if bonus:
+                want[i, j] = q[i, d] * x
+            x = x * fade[0]
+            if not bonus:
+                want[i, j] = q[i, d] * x
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    out, state = torch.empty(n, V, device="cuda"), torch.zeros(1, 1, D, V, device="cuda")
+    seq.linear_attn(q.cuda(), k.cuda(), v.cuda(), torch.full((n, V), 40.0, device="cuda"), None, fade.cuda(), 1.0, 1.0, False, None, False, False,
+                    state, i32([0]), i32([n]), i32([0, n]), out, 2.0 ** 60, bonus=u.cuda() if bonus else None)
+    assert torch.equal(out[:64, :64].cpu() * 2.0 ** 30, want)
