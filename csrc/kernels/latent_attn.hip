@@ -41,7 +41,6 @@
 // DMA a step ahead and each wave carries 16 or 32 rows from scores to weighted latents in registers (latent_attn_staged_kernel).
 #include <stdlib.h>
 
-#include <algorithm>
 #include <type_traits>
 
 #include "lds_rows.h"
@@ -287,7 +286,10 @@ __device__ __forceinline__ float group16_sum(float v) {
 // for together, all of its values while the softmax runs (by groups of 4 and 8 before, nine waits a tile), and the four waves' results meet
 // in LDS areas of their own, summed by all threads. us, 32 sequences: 12 heads, latent 512, some 700 keys 31.0 -> 22.7 and the merge 10.7 ->
 // 4.6; 8 heads, latent 256, 512 keys 16.2 -> 11.5 and 6.6 -> 4.6.
-// EXACT: rows of whole fragments and a latent of whole tiles (E = 32 NQF, rank = 16 NCT), nothing is clamped.
+// EXACT: rows of whole fragments and a latent of whole tiles (E = 32 NQF, rank = 16 NCT), nothing is clamped. The others read and multiply
+// by what their rows do not have, too: leaving it out takes branches between the loads (us, 32 sequences, 12 heads, 700 keys, loads by groups of 4
+// and 8 -> now, and now with branches: latent 264 of 328 29.6 -> 20.6, 21.2; 384 of 448 32.0 -> 21.8, 22.8; 512 of 512 35.7 -> 22.9, 24.2; 200
+// of 224, 3 tokens beside 31 102 -> 78, 112).
 template <int NCT, int NQF, bool EXACT>
 __global__ __launch_bounds__(256, NCT > 16 ? 1 : 2) void latent_attn_mfma_kernel(LatentArgs a, const bf16_t* __restrict__ qa, int H,
                                                                 float scale_log2e,
@@ -1051,12 +1053,13 @@ void launch_latent_attn(const LatentArgs& a, const void* qa, int H, float scale,
 }
 
 // Decoded tokens on the MFMA kernel: how many workgroups share a sequence's key tiles (1: no split), chosen from the
-// step's shape so that the launch has about two workgroups per CU, or one where a latent of more than 256 takes a CU's registers
-// and LDS, and the scratch floats their partial results take.
+// step's shape so that the launch has about two workgroups per CU, and the scratch floats their partial results take. A latent of more than
+// 256 leaves room for one; fewer parts for it cost as much as they gain (us, latent 512, 12 heads, 700 keys, 512 / wg and 256 / S parts: 33
+// sequences in 64 slots 25.2 and 33.9, 48 45.5 and 35.8, 64 52.6 and 47.1, 80 in 128 51.6 and 65.9, 128 90.2 and 72.8).
 int latent_attn_parts(int T, int S, int H, int rank, int rot, int f32, int page) {
   if (!mfma_takes(rank, rot, f32, page) || (int64_t)T * H > 16 * (int64_t)S) return 1;
   const int wg = (T * H + 63) / 64 + S;
-  const int parts = rank > 256 ? 256 / std::max(S, 1) : 512 / (wg > 0 ? wg : 1);
+  const int parts = 512 / (wg > 0 ? wg : 1);
   return parts < 2 ? 1 : (parts > 8 ? 8 : parts);
 }
 size_t latent_attn_part_floats(int T, int S, int H, int rank, int rot, int parts) {

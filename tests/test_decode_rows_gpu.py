@@ -54,6 +54,14 @@ def test_latent_attn_adds_its_waves_by_fused_steps(rank, rot, monkeypatch):
     assert (out.abs() <= 2.0 ** -23 * A.float().abs()).all() and (out != 0).float().mean().item() > 0.8
 
 
+@pytest.mark.parametrize("rank", [128, 256, 264, 512])
+@pytest.mark.parametrize("T,S", [(1, 1), (32, 32), (48, 64), (64, 64), (96, 128), (128, 128), (256, 256), (300, 512)])
+def test_latent_attn_parts(T, S, rank):
+    """Two workgroups per CU in all, whatever the latent's size."""
+    H, wg = 12, (T * 12 + 63) // 64 + S
+    assert seq._C().latent_attn_split(T, S, H, rank, 64, False, 16)[0] == max(1, min(8, 512 // wg))
+
+
 @pytest.mark.parametrize("score", [seq.ROUTE_SIGMOID, seq.ROUTE_SOFTMAX, seq.ROUTE_TOP_SOFTMAX])
 @pytest.mark.parametrize("T,E,top", [(1, 1, 1), (7, 8, 2), (16, 64, 6), (16, 65, 4), (17, 60, 60), (65, 8, 2), (40, 65, 4), (33, 512, 8), (5, 600, 3)])
 def test_moe_route_sort(T, E, top, score):
