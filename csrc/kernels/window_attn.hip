@@ -790,8 +790,10 @@ __global__ __launch_bounds__(256) void window_attn_merge_kernel(WindowArgs a, in
       const int64_t slot = ((int64_t)min(p, a.parts - 1) * G + g) * gridDim.x + blockIdx.x;
       pm[p] = p < a.parts ? a.part_ml[(slot * 16 + rr) * 2] : -INFINITY;
       pl[p] = a.part_ml[(slot * 16 + rr) * 2 + 1];
-      po[p] = a.part_o[slot * (16 * vs) + rr * vs + col];
-      pq[p] = vrot > 0 ? a.part_o[slot * (16 * vs) + rr * vs + colo] : 0.f;   // (uniform)
+      const float o = a.part_o[slot * (16 * vs) + rr * vs + col];
+      const float q = vrot > 0 ? a.part_o[slot * (16 * vs) + rr * vs + colo] : 0.f;   // (uniform)
+      po[p] = p < a.parts ? o : 0.f;   // (nothing of the parts past the last: an infinity times their 0 would be NaN)
+      pq[p] = p < a.parts ? q : 0.f;
       M = fmaxf(M, pm[p]);
     }
     float L = 0.f, y = 0.f, yo = 0.f;
