@@ -107,7 +107,8 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_q4_prompt_kernel(GemmPar
   };
   // half h of the wave's fragment of tile a at k-step u: the bf16 that the unpacked copy of the matrix would hold. The low nibbles of a
   // word's bytes are elements 0 4 1 5, the high ones 2 6 3 7: two of them, 16 bits apart, are a pair of f16 subnormals v 2^-24 (the high
-  // ones v 2^-20), exact, which v_fma_mix_f32 takes as they stand: v s - s z in one rounding without a conversion of v.
+  // ones v 2^-20), exact, which v_fma_mix_f32 takes as they stand: v s - s z in one rounding without a conversion of v. (2^24 s has to be
+  // finite: a matrix with a scale of 2^104 or more goes by way of its copy, Linear.prompt_scales of vgate/ops.)
   auto unpack = [&](int a, int h, int u) {
     const uint32_t w = u == 0 ? wq[a].x : u == 1 ? wq[a].y : u == 2 ? wq[a].z : wq[a].w;
     const uint32_t lo = w & (h ? 0x00F000F0u : 0x000F000Fu), hi = (w >> 8) & (h ? 0x00F000F0u : 0x000F000Fu);

@@ -103,7 +103,7 @@ bool launch_dense_kx_out(const GemmArgs& g, hipStream_t st);  // fp32 outputs an
 // per CU owning whole tiles), g.splitk K slices; false for a shape / mode it does not take
 bool launch_awq_mid(const GemmArgs& g, hipStream_t st);
 // AWQ W4A16 prompt kernel (gemm_prompt_q4.hip, M > 64): g.ntb = a tile code, g.splitk = K slices, as q4_prompt_form() gives them; false
-// for a shape / mode it does not take.
+// for a shape / mode it does not take. Scales below 2^104, which the caller sees to.
 bool launch_q4_prompt(const GemmArgs& g, hipStream_t st);
 // How a step of more than 64 rows multiplies by int4 weights: path 5 that kernel; 1 a bf16 copy and a form of gemm_prefill.hip; 6 a bf16
 // copy and the kernels of gemm_decode.h. K is cut as form (code, sk), of q4_cut() or of a plan, cuts it: all of them give that form's bits.

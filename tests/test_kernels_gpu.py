@@ -1358,6 +1358,27 @@ def test_awq_prompt_weights_are_those_of_the_copy(code):
 
 
 @pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("power", [100, 103, 104, 112])
+def test_awq_prompts_with_huge_scales(power, norm):
+    """Rows of more than 64 by scales on either side of where 2^24 times them leaves fp32: K roundings of 2^-24 of exact bf16 products, one to
+    bf16."""
+    N, K, M = 1536, 1536, 256   # (the prompt kernel, without a norm in one slice of K and with one in four)
+    g = torch.Generator().manual_seed(power)
+    scales = (torch.rand(K // 128, N, generator=g) + 0.5).bfloat16() * 2.0 ** -6
+    scales[1, ::7] = 1.75 * 2.0 ** power
+    lin = ops.Linear(None, awq=dict(qint=torch.randint(0, 16, (N, K), generator=g, dtype=torch.int32), group=128, scales=scales.to(DEV),
+                                    zeros=torch.randint(0, 16, (K // 128, N), generator=g).float().to(DEV)))
+    x = (torch.randn(M, K, generator=g) * 2.0 ** -20).bfloat16().to(DEV)
+    kw = dict(norm=(torch.ones(K, dtype=torch.bfloat16, device=DEV), 1.0)) if norm else {}
+    got, want = ops.linear(x, lin, **kw), x.double() @ lin.dense_weight().double().t()
+    if norm:
+        want *= torch.rsqrt((x.double() ** 2).mean(1, keepdim=True) + 1.0)
+    assert torch.isfinite(got).all()
+    for c in range(7):   # (columns by themselves: the large ones would hide the others)
+        assert ((got.double() - want)[:, c::7].norm() / want[:, c::7].norm()).item() < 2.0 ** -8
+
+
+@pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("M,K,sk", [(65, 256, 1), (97, 640, 2), (130, 1152, 4), (300, 1536, 3), (577, 1664, 6)])
 def test_awq_prompt_tiles_give_the_bits_of_the_copied_matrix(M, K, sk, norm):
     """Every int4 tile against every bf16 form on the dequantised copy, K in as many slices, some of which begin or end inside a group of

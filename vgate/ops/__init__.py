@@ -198,6 +198,8 @@ class Linear:
                 self.scales = scales.to(torch.bfloat16).contiguous()
                 self.zeros = (scales.float() * zeros.float()).to(torch.bfloat16).contiguous()
                 self.szp = pack_awq_sz(self.scales, self.zeros) if self.group == 128 else None
+                # the int4 prompt kernel holds 2^24 times each scale in fp32 (false for NaN and infinities too)
+                self.prompt_scales = bool((self.scales.abs() < 2.0 ** 104).all())
                 self.w = None
             else:
                 self.w = ref.awq_dequant_ref(q, scales, zeros, self.group)
@@ -467,10 +469,10 @@ def _linear_awq_prompt(x, lin: "Linear", out, residual, norm, qkv, epi, M):
     gamma = norm[0] if norm is not None else None
     ws = workspace(x.device)
     rows16 = x.stride(0) % 8 == 0 and x.stride(0) < 1 << 20 and x.data_ptr() % 16 == 0 and lin.K < 1 << 20
-    aligned = not any(t is not None and t.data_ptr() % 16 for t in (gamma, lin.scales, lin.zeros))
+    takes = lin.group == 128 and lin.prompt_scales and not any(t is not None and t.data_ptr() % 16 for t in (gamma, lin.scales, lin.zeros))
     plan = lin.prefill_plan.get(_plan_bucket(lin.prefill_plan, M)) if lin.prefill_plan else None
     code, sk = _awq_cut(plan, M, lin.N, lin.K, gamma is not None, rows16, ws)
-    path, code, sk = C.q4_prompt_form(M, lin.N, lin.K, gamma is not None, rows16, lin.group == 128 and aligned, ws, code, sk)
+    path, code, sk = C.q4_prompt_form(M, lin.N, lin.K, gamma is not None, rows16, takes, ws, code, sk)
     if path != 5:
         return _linear_awq_dequant(x, lin, out, residual, norm, qkv, epi, M, dict(path=path, ntb=code, splitk=sk))
     kw = dict(bias=lin.bias, res=residual, ws=ws, ntb=code, splitk=sk, path=5, awq_scales=lin.scales, awq_zeros=lin.zeros,
