@@ -57,10 +57,12 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(EmbedArgs a) {
   int tok = a.ids[t];
   if (tok < 0 && a.prev != nullptr) tok = a.prev[-tok - 1];
   const bool ok = tok >= 0 && tok < a.vocab;
-  const int64_t src = (int64_t)(ok ? tok : 0) * W, ro = (int64_t)t * W;
+  const int64_t src = (int64_t)tok * W, ro = (int64_t)t * W;
   auto value = [&](int c) { return ok ? ldx(a.table, src + c, a.t_f32) * a.scale : 0.f; };
   float v[NI], n1[NI], n2[NI];
-  load_row(a.table, src, a.t_f32, W, v);
+#pragma unroll
+  for (int i = 0; i < NI; ++i) v[i] = 0.f;
+  if (ok) load_row(a.table, src, a.t_f32, W, v);   // (uniform; a table may have no row at all)
   if (a.n1 != nullptr && !a.scalar) load_row(a.n1, 0, 1, W, n1);
   if (a.n2 != nullptr) load_row(a.n2, 0, 1, W, n2);
 #pragma unroll

@@ -120,3 +120,13 @@ def test_latent_write_with_the_querys_norm(rank, n, dt):
     host = caches[2].cpu()
     seq.latent_write(kv.cpu(), w.cpu(), 1e-5, pos.cpu(), slots.cpu(), inv.cpu(), rot, host, rank)
     _round(caches[0], host, dt)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("W", [1, 300, 2500])
+def test_embedding_table_without_rows(W, dt):
+    """No id names a row of it: zeros, and nothing is read."""
+    table, ids = torch.empty(0, W, dtype=dt, device="cuda"), torch.tensor([0, 5, -3], dtype=torch.int32, device="cuda")
+    x, h = torch.full((3, W), 7.0, device="cuda"), torch.full((3, W), 7.0, dtype=dt, device="cuda")
+    seq.embed_rows(ids, table, x, h=h, norm=torch.ones(W, device="cuda"), eps=1e-3)
+    assert not x.any() and not h.any()
