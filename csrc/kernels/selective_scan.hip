@@ -82,13 +82,16 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ShortConvArgs p) {
   }
 }
 
-// R tokens a workgroup, 8 channels a thread (16-B pieces), at most four taps, bf16: rows, weights and the slot's rows are asked for together
-// and a row once per R tokens, where the kernel above waits for each tap of each token (3072 channels, us:
-// 32 tokens of 32 sequences 6.8 -> 3.3, 300 of 4 8.6 -> 4.6, 1024 of 8 25.8 -> 9.0, 2048 of 8 33.6 -> 13.7).
+// R tokens a workgroup, 8 channels a thread (16-B pieces), at most four taps, bf16: rows, weights and the slot's rows are asked for together,
+// where the kernel above waits for each tap of each token, and with R = 2 a row is read for two tokens. A workgroup's sequences come one after
+// another, some 1.6 us each, which is why R is no larger (a prompt's first tokens share theirs with decoded ones: 1024 tokens of
+// 57 sequences 11.7 us with R = 4). us, rows not in L2 (MI355X), the kernel above -> this, 3072 channels: 32 tokens of 32 sequences 7.0 ->
+// 3.5, 400 of 4 8.8 -> 6.2, 1024 of 8 13.9 -> 9.1, 2048 of 8 24.4 -> 15.8, five decoded and three prompts, 2048, 22.9 -> 14.2; 512 channels:
+// 32 of 32 4.5 -> 3.3, 2048 of 8 7.5 -> 5.4.
 template <int R>
 __global__ __launch_bounds__(256) void short_conv_run_kernel(ShortConvArgs p) {
   const int total = p.query_start[p.S], last = min((int)(blockIdx.x + 1) * R, total);
-  const int c = (blockIdx.y * 256 + threadIdx.x) * 8, cc = min(c, p.C - 8);   // (channels past the last: its own, never stored)
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 8, cc = min(c, p.C - 8);   // (channels past the last: its own, never stored)
   const bf16_t* x = reinterpret_cast<const bf16_t*>(p.x);
   f32x4 w[4][2], b[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};   // w[3]: the token's own row
 #pragma unroll
@@ -363,11 +366,13 @@ void launch_short_conv(const ShortConvArgs& a, hipStream_t st) {
   if (gy > 64) gy = 64;
   const uintptr_t rows = reinterpret_cast<uintptr_t>(a.w) | reinterpret_cast<uintptr_t>(a.b) | reinterpret_cast<uintptr_t>(a.kept);
   if (vec && a.taps <= 4 && (rows & 15) == 0) {
-    // eight tokens a workgroup where a sequence has that many as a rule and the launch still fills the chip (2048 of 8
-    // 13.7 us, by workgroups of one token 18.6, 1024 of 8 9.0, 10.2)
-    const dim3 grid((unsigned)((a.T + 7) / 8), (a.C + per - 1) / per);
-    if (a.T >= 512 && a.T >= 8 * a.S) hipLaunchKernelGGL(short_conv_run_kernel<8>, grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(short_conv_run_kernel<1>, dim3(a.T, grid.y), dim3(256), 0, st, a);
+    // as many waves as the channels take, in equal workgroups (512 channels in workgroups of four waves: 2048 tokens of 8 10.3 us and not
+    // 5.4). Two tokens a workgroup where the launch fills the chip without them and sequences have that many on average: one / two, 2048 x
+    // 3072 18.0, 15.8; 1024 x 2048 7.7, 7.3; 1024 x 1536 6.7, 6.8; 600 x 3072 7.6, 7.8; 1024 single tokens x 3072 16.1, 17.0.
+    const int gy1 = (a.C + 2047) / 2048, pieces = (a.C / 8 + gy1 - 1) / gy1;
+    const dim3 block((pieces + 63) / 64 * 64);
+    if ((int64_t)a.T * a.C >= 1 << 21 && a.T >= 2 * a.S) hipLaunchKernelGGL(short_conv_run_kernel<2>, dim3((a.T + 1) / 2, gy1), block, 0, st, a);
+    else hipLaunchKernelGGL(short_conv_run_kernel<1>, dim3(a.T, gy1), block, 0, st, a);
   } else if (vec) hipLaunchKernelGGL(short_conv_kernel<8>, dim3(a.T, gy), dim3(256), 0, st, a);
   else hipLaunchKernelGGL(short_conv_kernel<1>, dim3(a.T, gy), dim3(256), 0, st, a);
 }

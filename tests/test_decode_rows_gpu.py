@@ -121,6 +121,28 @@ def test_short_conv_runs(C, taps, lens):
         assert torch.equal(a, o) and bool((a[T:] == 7.0).all())
 
 
+@pytest.mark.parametrize("C", [1536, 4104])
+@pytest.mark.parametrize("taps", [1, 2, 3, 4])
+@pytest.mark.parametrize("lens", [[1, 1, 1, 1, 1, 700, 1, 2, 3, 701], [300, 1, 1, 2, 301, 0, 900], [1, 2] * 400 + [500], [1] * 9 + [0, 1500, 0, 1], [1] * 1400 + [9]])
+def test_short_conv_of_prompts_among_decodes(C, taps, lens):
+    """Two tokens a workgroup (all lists but the last, which has fewer than two tokens to a sequence): sequences that share one, those shorter
+    than the taps, kept rows read from either of its tokens, sequences without a slot: the bits of the kernel for rows that are not of whole
+    pieces."""
+    T, S = sum(lens), len(lens)
+    two = T * C >= 1 << 21 and T >= 2 * S   # the launcher's rule
+    assert two == (lens[0:10] != [1] * 10)
+    g = torch.Generator().manual_seed(C + taps + S)
+    x = torch.randn(T, C + 8, generator=g).bfloat16().cuda()[:, 8:]
+    w, b, kept = (torch.randn(s, generator=g).cuda() for s in ((taps, C), (C,), (S, taps - 1, C)))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    slots = i32([-1 if s % 7 == 4 else S - 1 - s for s in range(S)])
+    ctx, start = i32([n + (13 if s % 4 else 0) for s, n in enumerate(lens)]), i32([sum(lens[:s]) for s in range(S + 1)])
+    a, o = torch.full((T, C), 7.0, dtype=torch.bfloat16, device="cuda"), torch.full((T, C + 1), 7.0, dtype=torch.bfloat16, device="cuda")[:, 1:]
+    seq.short_conv(x, w, b, kept, slots, ctx, start, a, silu=True)
+    seq.short_conv(x, w, b, kept, slots, ctx, start, o, silu=True)
+    assert torch.equal(a, o)
+
+
 @pytest.mark.parametrize("mode", ["gated", "head", "bonus"])
 @pytest.mark.parametrize("D,V", [(128, 128), (72, 24), (64, 64), (24, 40)])
 @pytest.mark.parametrize("n", [129, 144, 145, 176, 191, 192, 255, 300])
