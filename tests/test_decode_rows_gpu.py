@@ -62,6 +62,35 @@ def test_latent_attn_parts(T, S, rank):
     assert seq._C().latent_attn_split(T, S, H, rank, 64, False, 16)[0] == max(1, min(8, 512 // wg))
 
 
+@pytest.mark.parametrize("rank,rot,H", [(256, 64, 8), (512, 64, 12), (264, 64, 12), (96, 32, 8)])
+@pytest.mark.parametrize("lens", [[1] * 8 + [3], [1, 1, 4, 1, 1, 1, 1, 0] + [1] * 20, [1] * 60 + [9, 1, 0, 7], [0] * 300 + [1, 5, 1, 3] + [0] * 300])
+def test_latent_attn_of_short_portions_among_decodes(rank, rot, H, lens):
+    """Steps that count as decoding (at most 16 rows to a slot) with portions of more than 16 rows, whose waves take rows and not keys, beside
+    sequences that several workgroups share (eight at first, one in the last list), and slots without tokens. Tolerance as above."""
+    g = torch.Generator().manual_seed(rank + len(lens))
+    S, T, E = len(lens), sum(lens), rank + rot
+    if T * H > 16 * S:
+        lens, S = lens + [0] * (T * H // 16 + 1 - S), T * H // 16 + 1
+    ctx = [n + (i * 131) % 700 if n else 0 for i, n in enumerate(lens)]
+    pages = [-(-c // 16) for c in ctx]
+    cache = torch.randn(sum(pages), 16, E, generator=g).clamp(-4, 4).bfloat16()
+    tables, at, start = torch.zeros(S, max(pages), dtype=torch.int32), 0, [0]
+    for i, n in enumerate(pages):
+        tables[i, :n] = torch.arange(at, at + n, dtype=torch.int32)
+        at += n
+        start.append(start[-1] + lens[i])
+    assert (seq._C().latent_attn_split(T, S, H, rank, rot, False, 16)[0] == 1) == (S > 500) and max(lens) * H > 16
+    qa, sink, scale = torch.randn(T, H, E, generator=g).bfloat16(), torch.randn(H, generator=g), E ** -0.5
+    ctx, start = torch.tensor(ctx, dtype=torch.int32), torch.tensor(start, dtype=torch.int32)
+    tr = cache[:, :, :rank].transpose(1, 2).contiguous()
+    for window in (seq.LATENT_FULL, 70):
+        got, want = torch.empty(T, H, rank, dtype=torch.bfloat16, device="cuda"), torch.empty(T, H, rank)
+        seq.latent_attn(qa.cuda(), cache.cuda(), tables.cuda(), ctx.cuda(), start.cuda(), got, scale, H, rank, rot, num_seqs=S, cache_t=tr.cuda(),
+                        window=window, sink=sink.cuda())
+        seq.latent_attn(qa.float(), cache.float(), tables, ctx, start, want, scale, H, rank, rot, num_seqs=S, window=window, sink=sink)
+        assert ((got.float().cpu() - want).abs() <= 4 * 2.0 ** -8 + 1e-4).all()
+
+
 @pytest.mark.parametrize("score", [seq.ROUTE_SIGMOID, seq.ROUTE_SOFTMAX, seq.ROUTE_TOP_SOFTMAX])
 @pytest.mark.parametrize("T,E,top", [(1, 1, 1), (7, 8, 2), (16, 64, 6), (16, 65, 4), (17, 60, 60), (65, 8, 2), (40, 65, 4), (33, 512, 8), (5, 600, 3)])
 def test_moe_route_sort(T, E, top, score):
