@@ -5,9 +5,11 @@
 // As gemm_w4_kernel (gemm_prompt.h): operands of a k-step are read (here: and unpacked) during the MFMAs of the one before, stages come by
 // LDS-DMA. The waves stand side by side over the columns, so that each fragment of W is unpacked by one wave of the block only.
 // What bounds it is the issue of vector instructions. One wave on a SIMD issues one every 5 to 6 cycles (a conversion every 8) whatever else
-// is ready; two or more take 4.3 each between MFMAs, which take 8 of issue and 16 of the matrix core. So two waves to a SIMD at least, eight
-// in a block or two to four blocks of four or eight on a CU (stages of 128 k, two or three of them as LDS allows); weights turn into floats
-// without conversions (unpack()); gamma is widened once per block and not once per wave and k-step. Per fragment 17 vector instructions, 25
+// is ready; two or more take 4.3 each between MFMAs, which take 8 of issue and 16 of the matrix core. So tiles are made for two waves to a SIMD
+// and more, eight in a block or two to four blocks of four or eight on a CU (stages of 128 k, two or three of them as LDS allows); one is left
+// where a launch has too few blocks of four waves, in tile 410 with a norm in front of slices of more than 2900 (their gamma takes the second
+// block's LDS) and in tile 1620. Weights turn into floats without conversions (unpack()); gamma is widened once per block and not once per
+// wave and k-step. Per fragment 17 vector instructions, 25
 // with gamma, against MT MFMAs. LDS is next: an x fragment (8 cycles) serves NT MFMAs.
 // us, four waves with 23 and 31 instructions -> these (MI355X, cold weights, the same slices): 256 rows, 17920 x 1536 with a norm 35.1 -> 29.3,
 // 1536 x 8960 in 8 slices 27.3 -> 21.8, 1536 x 1536 11.4 -> 10.1; 448 rows, 17920 x 1536 55.9 -> 45.4, 1536 x 8960 31.6 -> 27.4; 96 rows 23.8 ->
@@ -16,17 +18,19 @@
 
 namespace vgate {
 
-template <int NW, int MT, int NT>
+template <int NW, int MT, int NT, bool RING>
 struct Q4 {  // geometry: NW waves side by side, each 16 MT rows x 16 NT columns; stages of 128 k (one group)
   static constexpr int BM = 16 * MT, BN = 16 * NW * NT;
-  static constexpr int XB = BN * 64, SB = XB + BM * 256;  // W | x (two 64-k halves) | scales, zeros: 1 KiB each
-  static constexpr int STAGE = SB + 2048;
+  static constexpr int XB = BN * 64, SB = XB + BM * 256;  // W | x (two 64-k halves) | scales, zeros, RING: gamma: 1 KiB each
+  static constexpr int STAGE = SB + (RING ? 3072 : 2048);
   static constexpr int XPW = 4 * MT / NW, PPW = XPW + NT + 1;  // x pieces and all DMA of a wave and stage
 };
 
-template <int NW, int MT, int NT, int NS, int EPI, bool NORM>
+// RING: gamma comes with the stages, bf16, and is widened per wave and k-step; else the slice's stands in LDS as fp32.
+template <int NW, int MT, int NT, int NS, int EPI, bool NORM, bool RING>
 __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_q4_prompt_kernel(GemmParams p) {
-  using G = Q4<NW, MT, NT>;
+  using G = Q4<NW, MT, NT, RING>;
+  static_assert(!RING || (NORM && NW == 4), "two waves' small pieces are gamma");
   constexpr int PPW = G::PPW, XPW = G::XPW, STAGE = G::STAGE;
   static_assert(NS * STAGE <= 160 * 1024 && XPW * NW == 4 * MT, "LDS; x in equal shares");
   static_assert(NS >= 2 && (NS - 1) * PPW < 64 && (G::BN & (G::BN - 1)) == 0 && G::BN <= 512, "vmcnt; the block's scales repeat in 1 KiB");
@@ -46,11 +50,12 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_q4_prompt_kernel(GemmPar
   const int n0 = (in / gm) * G::BN, nt0 = n0 / 16 + wid * NT;  // the wave's first column tile
   const u32x4 wrs = rsrc_words(p.wp + ((size_t)(n0 / 16) * KQ + q0) * 64);
   const u32x4 xrs = rsrc_words(p.x + (size_t)m0 * p.lda + q0 * 128);
-  // the wave's small piece: the group's scales or zeros of the block's columns, asked for again until the 1 KiB is full
-  const int kind = wid & 1;
-  const u32x4 srs = rsrc_words((kind == 0 ? p.scales : p.zeros) + (size_t)q0 * p.N + n0);
-  const uint32_t sstep = (uint32_t)p.N * 2u;
-  const uint32_t wvo = lane * 16, svo = (uint32_t)(lane * 16) & (2u * G::BN - 1u);
+  // the wave's small piece: the group's scales or zeros of the block's columns or its gamma, asked for again until the 1 KiB is full
+  const int kind = RING ? min(wid, 2) : wid & 1;
+  const bf16_t* small = kind == 0 ? p.scales : kind == 1 ? p.zeros : p.norm_w;
+  const u32x4 srs = rsrc_words(small + (kind < 2 ? (size_t)q0 * p.N + n0 : (size_t)q0 * 128));
+  const uint32_t sstep = kind < 2 ? (uint32_t)p.N * 2u : 256u;
+  const uint32_t wvo = lane * 16, svo = (uint32_t)(lane * 16) & (kind < 2 ? 2u * G::BN - 1u : 255u);
   uint32_t xvo[XPW];  // pieces of 8 rows x 64 k: tile (piece >> 2), k half (piece >> 1) & 1, row half piece & 1
 #pragma unroll
   for (int i = 0; i < XPW; ++i) {
@@ -99,8 +104,13 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_q4_prompt_kernel(GemmPar
     }
   };
   const char* gbase = smem + NS * STAGE + quad * 32;  // gamma of the slice, fp32
-  auto read_gamma = [&](int u, int t) {
-    if constexpr (NORM) {
+  auto read_gamma = [&](int u, int t, const char* sb) {
+    if constexpr (RING) {
+      float g[8];
+      unpack8(*reinterpret_cast<const uint4*>(sb + G::SB + 2048 + u * 64 + quad * 16), g);
+      gam[0] = make_float4(g[0], g[1], g[2], g[3]);
+      gam[1] = make_float4(g[4], g[5], g[6], g[7]);
+    } else if constexpr (NORM) {
       gam[0] = *reinterpret_cast<const float4*>(gbase + t * 512 + u * 128);
       gam[1] = *reinterpret_cast<const float4*>(gbase + t * 512 + u * 128 + 16);
     }
@@ -151,7 +161,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_q4_prompt_kernel(GemmPar
       wf[u & 1][a] = __builtin_bit_cast(uint4, f);
     }
     if constexpr (u == 3) read_stage(sb);
-    read_gamma(v, t);
+    read_gamma(v, t, sb);
 #pragma unroll
     for (int b = 0; b < MT; ++b) {
       if constexpr (NORM)
@@ -173,7 +183,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_q4_prompt_kernel(GemmPar
   using C2 = std::integral_constant<int, 2>;
   using C3 = std::integral_constant<int, 3>;
   // gamma of the slice: bf16 by DMA into the second half of its place (asked for first: it has landed when the first stage has), widened there
-  if constexpr (NORM) {
+  if constexpr (NORM && !RING) {
     u32x4 grs = rsrc_words(p.norm_w + (size_t)q0 * 128);
     grs[2] = (uint32_t)nk * 256u;
     for (int i = wid; i < (nk + 3) >> 2; i += NW) blds16(grs, wvo, (uint32_t)i * 1024u, lds0 + NS * STAGE + ((nk + 3) >> 2) * 1024 + i * 1024u);
@@ -183,7 +193,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_q4_prompt_kernel(GemmPar
 #pragma unroll
     for (int i = 0; i < PPW; ++i) issue_piece(i, s0 < nk ? s0 : nk - 1, s0);
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * PPW) : "memory");
-  if constexpr (NORM) {
+  if constexpr (NORM && !RING) {
     const bf16_t* raw = reinterpret_cast<const bf16_t*>(smem + NS * STAGE + ((nk + 3) >> 2) * 1024);
     float* wide = reinterpret_cast<float*>(smem + NS * STAGE);
     // (in place, from the front: a round of 64 NW elements is read by all before it is written, and lies behind what the next one reads)
@@ -197,7 +207,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_q4_prompt_kernel(GemmPar
   }
   if (kt0 & 1) clear(smem, 0);
   read_stage(smem);
-  read_gamma(0, 0);
+  read_gamma(0, 0, smem);
 #pragma unroll
   for (int b = 0; b < MT; ++b) read_x(b, 0, smem);
 #pragma unroll
@@ -266,15 +276,15 @@ static int q4_gamma_lds(int K, int nz) { return (((K >> 6) + nz - 1) / nz + 2) /
 template <int EPI, int NORM, int NTB>
 void launch_prefill_reduce(const GemmParams& p, int nz, hipStream_t st);
 
-template <int NW, int MT, int NT, int NS, int EPI, bool NORM>
+template <int NW, int MT, int NT, int NS, int EPI, bool NORM, bool RING = false>
 static bool launch_q4_one(const GemmParams& p, int nz, hipStream_t st) {
-  using G = Q4<NW, MT, NT>;
-  const int lds = NS * G::STAGE + (NORM ? q4_gamma_lds(p.K, nz) : 0);
+  using G = Q4<NW, MT, NT, RING>;
+  const int lds = NS * G::STAGE + (NORM && !RING ? q4_gamma_lds(p.K, nz) : 0);
   if (p.N % G::BN != 0 || lds > 160 * 1024) return false;
   const int blocks = ((p.M + G::BM - 1) / G::BM) * (p.N / G::BN);
   GemmParams q = p;
   if (q.dbg_ts == nullptr) q.dbg_ts = tl_take("gemm_q4_prompt", blocks * nz);
-  auto kern = gemm_q4_prompt_kernel<NW, MT, NT, NS, EPI, NORM>;
+  auto kern = gemm_q4_prompt_kernel<NW, MT, NT, NS, EPI, NORM, RING>;
   static bool attr = [&] {
     return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
   }();
@@ -296,7 +306,10 @@ static bool launch_q4_epi(const GemmParams& p, int code, int nz, hipStream_t st)
     VG_Q4(640, 8, 6, 2, 3);
     VG_Q4(820, 8, 8, 1, 3);
     VG_Q4(1020, 8, 10, 1, 3);
-    VG_Q4(1620, 4, 16, 2, 2);
+    // four waves: eight would take a column tile each, and LDS 32 cycles of x fragments for 16 of the matrix cores. Long slices
+    // leave no room for their gamma, which then comes with the stages (28672 x 4096 at 256 rows 79 us, the next best tile 86; where both fit
+    // 0.5 % slower)
+    case 1620: return launch_q4_one<4, 16, 2, 2, EPI, NORM>(p, nz, st) || (NORM && launch_q4_one<4, 16, 2, 2, EPI, NORM, NORM>(p, nz, st));
 #undef VG_Q4
   }
   return false;
@@ -344,7 +357,8 @@ Q4Form q4_prompt_form(int M, int N, int K, bool norm, bool rows16, bool group128
   float least = 0.87f * (2.2f + 0.56f * weights + copy.us);
   auto over = [](int64_t x, int64_t y) { return (int)((x + y - 1) / y); };
   for (const Tile& t : tiles) {
-    const int kts = over(K / 128, nz), per_cu = 160 * 1024 / (t.stages * (t.bn * 64 + t.bm * 256 + 2048) + (norm ? q4_gamma_lds(K, nz) : 0));
+    const int kts = over(K / 128, nz), full = 160 * 1024 / (t.stages * (t.bn * 64 + t.bm * 256 + 2048) + (norm ? q4_gamma_lds(K, nz) : 0));
+    const int per_cu = t.code == 1620 ? 1 : full;   // (which fits whatever the slice)
     if (N % t.bn != 0 || per_cu == 0) continue;
     const int64_t blocks = (int64_t)over(M, t.bm) * (N / t.bn) * nz;
     const auto& x = t.cost[norm ? 1 : 0];

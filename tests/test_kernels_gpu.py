@@ -1357,6 +1357,22 @@ def test_awq_prompt_weights_are_those_of_the_copy(code):
     assert torch.equal(out, want) and torch.isfinite(out).all()
 
 
+@pytest.mark.parametrize("M,K,sk", [(1, 2560, 1), (70, 4096, 1), (300, 5120, 2), (257, 16384, 1)])
+def test_awq_prompt_tile_of_256_rows_behind_a_norm_and_long_slices(M, K, sk):
+    """Slices whose gamma does not fit beside the stages: the bits of the bf16 copy, summed in the same order."""
+    C, N = ops.native(), 256
+    lin = _awq(N, K, "plain", M + K)
+    x = torch.randn(M, K, device=DEV, generator=torch.Generator(DEV).manual_seed(K)).bfloat16()
+    gamma = (torch.rand(K, device=DEV) + 0.5).bfloat16()
+    copy = torch.empty(N * K, dtype=torch.bfloat16, device=DEV)
+    C.awq_dequant(lin.wp, lin.scales, lin.zeros, N, K, 128, copy, gamma)
+    out, want = torch.empty(M, N, device=DEV), torch.empty(M, N, device=DEV)
+    C.gemm(x, lin.wp, N, K, out, 1, ws=ops.workspace(DEV), ntb=1620, splitk=sk, path=5, awq_scales=lin.scales, awq_zeros=lin.zeros, group=128,
+           norm_w=gamma, eps=1e-6)
+    C.gemm(x, copy, N, K, want, 1, ws=ops.workspace(DEV), path=1, ntb=641, splitk=sk, rownorm=True, eps=1e-6)
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("power", [100, 103, 104, 112])
 def test_awq_prompts_with_huge_scales(power, norm):
