@@ -318,8 +318,11 @@ static bool launch_q4_epi(const GemmParams& p, int code, int nz, hipStream_t st)
 // Costs (us) as in choose_prefill_form() of gemm_prefill.hip, fitted to 15 shapes (N 512 .. 28672, K 1024 .. 14336) x 10 row counts 65 ..
 // 2048 on cold weights; K-tiles of 128, rounds of as many blocks to a CU as their stages leave room for. Unpacking is repeated by every row
 // of blocks, so from some row count on a bf16 copy (2.2 us + 0.56 a million weights) and the bf16 kernels are ahead. Given the slices, the
-// choice takes 1.004 of the best tile's time (geometric mean). The copy's estimate is 1.15 times what it takes at 1000 rows and more (6144 x
-// 4096 with a norm at 2048 rows: 122 us, this kernel 140), hence the factor; of 21 shapes x 8 row counts the worst choice is 1.03 of the other.
+// choice takes 1.004 of the best tile's time (geometric mean). The copy's estimate is taken at 0.87: measured over estimated, medians of 720
+// points (18 shapes x 20 row counts, with a norm and without), 0.80 to 0.93 by form, 0.95 for 256 x 256 tiles in several slices (0.87 there took the
+// copy where these tiles are 5 to 8 % ahead: 4096 x 14336 at 768 rows 126, 117); the four-wave forms in one slice at 0.82, since the tiles' own
+// estimates are up to 15 % short for many rounds (5120 x 13824 at 2048 rows 323, the copy 270). Over those points the choice takes 1.007 of the
+// best form's time.
 Q4Form q4_prompt_form(int M, int N, int K, bool norm, bool rows16, bool group128, size_t slab_bytes, int code, int sk) {
   struct Tile {
     int code, bm, bn, stages;
@@ -354,7 +357,8 @@ Q4Form q4_prompt_form(int M, int N, int K, bool norm, bool rows16, bool group128
   const PrefillForm copy = prefill_form_cut(M, N, K, norm, rows16, slab_bytes, nz);
   Q4Form best = copy.us < 1e30f ? Q4Form{1, copy.code, nz} : Q4Form{code == 0 ? 6 : 1, code, sk};
   if (!group128 || !rows16 || K % 128 != 0) return best;
-  float least = 0.87f * (2.2f + 0.56f * weights + copy.us);
+  const float part = copy.code == 1024 && nz > 2 ? 0.95f : copy.code >= 5000 && nz == 1 ? 0.82f : 0.87f;
+  float least = part * (2.2f + 0.56f * weights + copy.us);
   auto over = [](int64_t x, int64_t y) { return (int)((x + y - 1) / y); };
   for (const Tile& t : tiles) {
     const int kts = over(K / 128, nz), full = 160 * 1024 / (t.stages * (t.bn * 64 + t.bm * 256 + 2048) + (norm ? q4_gamma_lds(K, nz) : 0));
