@@ -857,10 +857,13 @@ void launch_gemm_any(const AnyGemmArgs& g, hipStream_t st) {
       // A workgroup of 16 rows where all of them together are no more than the CUs and a wave's k is a chain of several loads, which
       // then are all under way (us, 64 rows / 16: 8 x 1024 at 32 rows 4.7, 3.6, at 2048 8.3, 3.8; 16 x 1536 at 512 11.4, 6.0; 128 x 768 at 300
       // 7.8, 4.1; 1024 x 512 at 64, two passes in one, 6.4, 4.1). With one pass of K = 512 there is little to gain (128 x 512 at 32
-      // rows 3.9, 4.0, at 8 3.3, 3.7).
+      // rows 3.9, 4.0, at 8 3.3, 3.7). Half as many loads under way where their last round would lie past K by half (128 x 1536 at 16 rows
+      // by 64 5.5, by 16 with four 6.2).
       const dim3 gn(gr.x, (g.M + 15) / 16, g.batch);
       if (!g.group_off && g.K > (g.M > 32 ? 256 : 512) && (int64_t)gn.x * gn.y * gn.z <= cu_count()) {
-        auto kern = dual ? gemm_any_rows_kernel<1, 2, 16> : (g.K > 512 ? gemm_any_rows_kernel<0, 4, 16> : gemm_any_rows_kernel<0, 2, 16>);
+        auto even = [&](int k) { return (g.K + 2 * k - 1) / (2 * k) * 2 == (g.K + k - 1) / k; };   // rounds of 2 k: none of them half empty
+        auto kern = dual ? (even(256) ? gemm_any_rows_kernel<1, 2, 16> : gemm_any_rows_kernel<1, 1, 16>)
+                         : (even(512) ? gemm_any_rows_kernel<0, 4, 16> : gemm_any_rows_kernel<0, 2, 16>);
         hipLaunchKernelGGL(kern, gn, block, 0, st, g);
         return;
       }
