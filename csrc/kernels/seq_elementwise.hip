@@ -50,9 +50,9 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const void* __restrict__
 
 // A row per workgroup: the stream's row, and beside it what the first sublayers read of it (EmbedArgs), in place of a launch that reads
 // the row again (us, 1024 wide, two launches -> one: 32 rows 3.4 + 3.9 -> 5.1, 2048 rows 6.5 + 5.9 -> 9.1).
-template <int NI>
+// NEXT: with h1; without, the row is all there is to make (128 wide, 4096 rows: 3.0 us, 3.6 with the tests for it in the kernel).
+template <int NI, bool NEXT>
 __global__ __launch_bounds__(256) void embed_rows_kernel(EmbedArgs a) {
-  __shared__ float red[16];
   const int t = blockIdx.x, W = a.W;
   int tok = a.ids[t];
   if (tok < 0 && a.prev != nullptr) tok = a.prev[-tok - 1];
@@ -63,22 +63,23 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(EmbedArgs a) {
 #pragma unroll
   for (int i = 0; i < NI; ++i) v[i] = 0.f;
   if (ok) load_row(a.table, src, a.t_f32, W, v);   // (uniform; a table may have no row at all)
-  if (a.n1 != nullptr && !a.scalar) load_row(a.n1, 0, 1, W, n1);
-  if (a.n2 != nullptr) load_row(a.n2, 0, 1, W, n2);
+  if (NEXT && a.n1 != nullptr && !a.scalar) load_row(a.n1, 0, 1, W, n1);
+  if (NEXT && a.n2 != nullptr) load_row(a.n2, 0, 1, W, n2);
 #pragma unroll
   for (int i = 0; i < NI; ++i) v[i] = ok ? v[i] * a.scale : 0.f;
 #pragma unroll
   for (int i = 0; i < NI; ++i)
     if ((int)threadIdx.x + 256 * i < W) a.x[ro + threadIdx.x + 256 * i] = v[i];
   for (int c = threadIdx.x + 256 * NI; c < W; c += 256) a.x[ro + c] = value(c);
-  if (a.h1 == nullptr) return;  // (uniform)
-  if (a.n1 == nullptr) {        // a copy
+  if constexpr (!NEXT) return;
+  if (a.n1 == nullptr) {        // (uniform) a copy
 #pragma unroll
     for (int i = 0; i < NI; ++i)
       if ((int)threadIdx.x + 256 * i < W) stx(a.h1, ro + threadIdx.x + 256 * i, a.h_f32, v[i]);
     for (int c = threadIdx.x + 256 * NI; c < W; c += 256) stx(a.h1, ro + c, a.h_f32, value(c));
     return;
   }
+  __shared__ float red[16];
   norm_row(v, W, a.eps, a.center, red, value, [&](int c, int i, float r) {
     stx(a.h1, ro + c, a.h_f32, r * (a.scalar ? a.n1[0] : i >= 0 ? n1[i] : a.n1[c]));
     if (a.n2 != nullptr) stx(a.h2, ro + c, a.h_f32, r * (i >= 0 ? n2[i] : a.n2[c]));
@@ -89,15 +90,24 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(EmbedArgs a) {
 // memory is waited for once per operand that may be missing instead of once per element (32 rows of 1024: 9.9 -> 4.6 us). With h the
 // new row's norm is made here too, in place of a launch that reads the row again (32 rows
 // 3.7 + 3.9 -> 5.8 us, 2048 rows 9.7 + 5.9 -> 13.0).
-template <int NI, bool F32>
-__global__ __launch_bounds__(256) void gated_residual_kernel(GatedArgs a) {
-  __shared__ float red[16];
-  const int t = blockIdx.x, W = a.W;
+// NEXT: with h; else nothing of a row is kept past its sum, and threads past a narrow row's end do nothing (2048 rows of 8192: 44 us, 50
+// with the tests for h in the kernel; 4096 of 128 3.9, 4.6).
+template <int NI, bool F32, bool NEXT>
+__global__ __launch_bounds__(256) void gated_residual_kernel(float* __restrict__ x, const void* __restrict__ y1,
+                                                              const void* __restrict__ g1, int64_t ldg1,
+                                                              const float* __restrict__ b1,
+                                                              const void* __restrict__ y2,
+                                                              const void* __restrict__ g2, int64_t ldg2,
+                                                              const float* __restrict__ b2, int W,
+                                                              const float* __restrict__ norm, float eps, void* __restrict__ h) {
+  const int t = blockIdx.x;
   const int64_t ro = (int64_t)t * W;
-  float* __restrict__ x = a.x;
-  auto pass = [&](int c0, float (&xo)[NI]) {   // (columns past W: the last one's values, never stored)
+  float keep[NI];   // NEXT: the first pass's columns of the new row
+#pragma unroll
+  for (int i = 0; i < NI; ++i) keep[i] = 0.f;
+  for (int c0 = threadIdx.x; c0 < W; c0 += 256 * NI) {   // (columns past W: the last one's values, never stored)
     int c[NI];
-    float v[NI], u[NI], a1[NI], a2[NI], d1[NI], d2[NI];
+    float xo[NI], v[NI], u[NI], a1[NI], a2[NI], d1[NI], d2[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       c[i] = min(c0 + 256 * i, W - 1);
@@ -106,41 +116,36 @@ __global__ __launch_bounds__(256) void gated_residual_kernel(GatedArgs a) {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       xo[i] = x[ro + c[i]];
-      v[i] = ldx(a.y1, ro + c[i], F32 ? 1 : 0);
+      v[i] = ldx(y1, ro + c[i], F32 ? 1 : 0);
     }
-    if (a.y2 != nullptr)
+    if (y2 != nullptr)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) u[i] = ldx(a.y2, ro + c[i], F32 ? 1 : 0);
-    if (a.g1 != nullptr)
+      for (int i = 0; i < NI; ++i) u[i] = ldx(y2, ro + c[i], F32 ? 1 : 0);
+    if (g1 != nullptr)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) a1[i] = ldx(a.g1, (int64_t)t * a.ldg1 + c[i], F32 ? 1 : 0);
-    if (a.g2 != nullptr)
+      for (int i = 0; i < NI; ++i) a1[i] = ldx(g1, (int64_t)t * ldg1 + c[i], F32 ? 1 : 0);
+    if (g2 != nullptr)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) a2[i] = ldx(a.g2, (int64_t)t * a.ldg2 + c[i], F32 ? 1 : 0);
-    if (a.g1 != nullptr && a.b1 != nullptr)
+      for (int i = 0; i < NI; ++i) a2[i] = ldx(g2, (int64_t)t * ldg2 + c[i], F32 ? 1 : 0);
+    if (g1 != nullptr && b1 != nullptr)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) d1[i] = a.b1[c[i]];
-    if (a.g2 != nullptr && a.b2 != nullptr)
+      for (int i = 0; i < NI; ++i) d1[i] = b1[c[i]];
+    if (g2 != nullptr && b2 != nullptr)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) d2[i] = a.b2[c[i]];
+      for (int i = 0; i < NI; ++i) d2[i] = b2[c[i]];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      if (a.g1 != nullptr) v[i] *= sigm(a1[i] + d1[i]);
-      if (a.g2 != nullptr) u[i] *= sigm(a2[i] + d2[i]);
-      xo[i] += v[i] + u[i];
-      if (c0 + 256 * i < W) x[ro + c[i]] = xo[i];
+      if (g1 != nullptr) v[i] *= sigm(a1[i] + d1[i]);
+      if (g2 != nullptr) u[i] *= sigm(a2[i] + d2[i]);
+      if (c0 + 256 * i < W) x[ro + c[i]] = xo[i] + (v[i] + u[i]);
+      if (NEXT && c0 < 256) keep[i] = xo[i] + (v[i] + u[i]);
     }
-  };
-  float keep[NI];
-  pass(threadIdx.x, keep);
-  for (int c0 = threadIdx.x + 256 * NI; c0 < W; c0 += 256 * NI) {
-    float more[NI];
-    pass(c0, more);
   }
-  if (a.h == nullptr) return;  // (uniform)
-  const float w = a.norm[0];
-  norm_row(keep, W, a.eps, 0, red, [&](int c) { return x[ro + c]; },
-           [&](int c, int, float r) { stx(a.h, ro + c, F32 ? 1 : 0, r * w); });
+  if constexpr (!NEXT) return;
+  __shared__ float red[16];
+  const float w = norm[0];
+  norm_row(keep, W, eps, 0, red, [&](int c) { return x[ro + c]; },
+           [&](int c, int, float r) { stx(h, ro + c, F32 ? 1 : 0, r * w); });
 }
 
 // out[t][j] = act(gu[t][j]) * gu[t][n + j] for a stacked [gate; up] projection (bf16), 8 columns per thread
@@ -847,7 +852,9 @@ void launch_norm_rows(const void* x, int64_t ldx_, int x_f32, const int32_t* row
 void launch_embed_rows(const EmbedArgs& a, hipStream_t st) {
   if (a.T <= 0 || a.W <= 0) return;
   row_columns<8>((a.W + 255) / 256, [&](auto ni) {
-    hipLaunchKernelGGL(embed_rows_kernel<decltype(ni)::value>, dim3(a.T), dim3(256), 0, st, a);
+    constexpr int NI = decltype(ni)::value;
+    auto kern = a.h1 != nullptr ? embed_rows_kernel<NI, true> : embed_rows_kernel<NI, false>;
+    hipLaunchKernelGGL(kern, dim3(a.T), dim3(256), 0, st, a);
   });
 }
 
@@ -858,8 +865,9 @@ void launch_gated_residual(const GatedArgs& a, hipStream_t st) {
   const int passes = (a.W + 1023) / 1024;
   row_columns<4>((a.W + 256 * passes - 1) / (256 * passes), [&](auto ni) {
     constexpr int NI = decltype(ni)::value;
-    auto kern = a.f32 ? gated_residual_kernel<NI, true> : gated_residual_kernel<NI, false>;
-    hipLaunchKernelGGL(kern, dim3(a.T), dim3(256), 0, st, a);
+    auto kern = a.h != nullptr ? (a.f32 ? gated_residual_kernel<NI, true, true> : gated_residual_kernel<NI, false, true>)
+                               : (a.f32 ? gated_residual_kernel<NI, true, false> : gated_residual_kernel<NI, false, false>);
+    hipLaunchKernelGGL(kern, dim3(a.T), dim3(256), 0, st, a.x, a.y1, a.g1, a.ldg1, a.b1, a.y2, a.g2, a.ldg2, a.b2, a.W, a.norm, a.eps, a.h);
   });
 }
 
