@@ -882,13 +882,14 @@ void launch_moe_route(const RouteArgs& a, hipStream_t st) {
                      a.idx, a.wts);
 }
 
-// One launch for as many tokens as a workgroup has waves (us, two launches / one, 8 experts of which 2: 1 token 3.8, 3.1, 8 tokens 4.5, 3.4; with
-// two tokens a wave, 32, 4.5, 5.3). Where the lanes past E's power of two stay out, and a lane holds one score, two launches take 4.5 in
-// place of 6.1 at 32 tokens, 7.0 of 8.7 at 2048.
-constexpr int ROUTE_SORT_ROWS = 16;
+// One launch for as many tokens as a workgroup has waves, and few choices in all: its waves make them on one CU (us, two launches / one, 8
+// experts of which 2: 1 token 3.8, 3.1, 8 tokens 4.5, 3.4; with two tokens a wave, 32, 4.5, 5.3; 16 tokens, 8 of 64 12.3, 13.2, 32 of 64 32, 39).
+// Where the lanes past E's power of two stay out, and a lane holds one score, two launches take 4.5 in place of 6.1 at 32 tokens, 7.0 of 8.7
+// at 2048.
+constexpr int ROUTE_SORT_ROWS = 16, ROUTE_SORT_CHOICES = 64;
 void launch_moe_route_sort(const RouteArgs& a, int32_t* rows, int32_t* pos, int32_t* off, hipStream_t st) {
   if (a.T <= 0) return;
-  if (a.T > ROUTE_SORT_ROWS || a.E > 64 || a.top > 64) {
+  if (a.T > ROUTE_SORT_ROWS || a.E > 64 || a.T * a.top > ROUTE_SORT_CHOICES) {
     launch_moe_route(a, st);
     launch_moe_sort(a.idx, a.T, a.E, a.top, rows, pos, off, st);
     return;

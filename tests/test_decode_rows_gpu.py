@@ -92,7 +92,7 @@ def test_latent_attn_of_short_portions_among_decodes(rank, rot, H, lens):
 
 
 @pytest.mark.parametrize("score", [seq.ROUTE_SIGMOID, seq.ROUTE_SOFTMAX, seq.ROUTE_TOP_SOFTMAX])
-@pytest.mark.parametrize("T,E,top", [(1, 1, 1), (7, 8, 2), (16, 64, 6), (16, 65, 4), (17, 60, 60), (65, 8, 2), (40, 65, 4), (33, 512, 8), (5, 600, 3)])
+@pytest.mark.parametrize("T,E,top", [(1, 1, 1), (7, 8, 2), (16, 64, 6), (16, 65, 4), (17, 60, 60), (16, 64, 4), (16, 64, 5), (2, 64, 32), (1, 64, 64), (65, 8, 2), (40, 65, 4), (33, 512, 8), (5, 600, 3)])
 def test_moe_route_sort(T, E, top, score):
     """One launch and two, on either side of their line: the choice and weights of the CPU form, every pair in its expert's stretch once."""
     g = torch.Generator().manual_seed(T + E)
