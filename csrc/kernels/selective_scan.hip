@@ -86,8 +86,8 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ShortConvArgs p) {
 // where the kernel above waits for each tap of each token, and with R = 2 a row is read for two tokens. A workgroup's sequences come one after
 // another, some 1.6 us each, which is why R is no larger (a prompt's first tokens share theirs with decoded ones: 1024 tokens of
 // 57 sequences 11.7 us with R = 4). us, rows not in L2 (MI355X), the kernel above -> this, 3072 channels: 32 tokens of 32 sequences 7.0 ->
-// 3.5, 400 of 4 8.8 -> 6.2, 1024 of 8 13.9 -> 9.1, 2048 of 8 24.4 -> 15.8, five decoded and three prompts, 2048, 22.9 -> 14.2; 512 channels:
-// 32 of 32 4.5 -> 3.3, 2048 of 8 7.5 -> 5.4.
+// 3.5, 400 of 4 8.8 -> 6.2, 1024 of 8 13.9 -> 9.1, 2048 of 8 24.4 -> 15.8, five decoded and three prompts, 2048, 22.9 -> 14.2 (in a replayed
+// step 24.6 -> 14.8); 512 channels: 32 of 32 4.5 -> 3.3, 2048 of 8 7.5 -> 5.4.
 template <int R>
 __global__ __launch_bounds__(256) void short_conv_run_kernel(ShortConvArgs p) {
   const int total = p.query_start[p.S], last = min((int)(blockIdx.x + 1) * R, total);

@@ -134,8 +134,8 @@ def test_narrow_products(M, N, K):
 @pytest.mark.parametrize("taps", [1, 3, 4])
 @pytest.mark.parametrize("lens", [[1] * 70, [1] * 64 + [0, 3, 0], [5] * 110, [0, 700, 0, 9, 3], [1]])
 def test_short_conv_runs(C, taps, lens):
-    """Runs of one and of eight tokens across sequences of one to hundreds, some without a slot or without tokens, rows past the last
-    sequence: the bits of the kernel for rows that are not of whole pieces."""
+    """Workgroups of one token, one and several of channels, sequences of one token to hundreds, some without a slot or without tokens, rows
+    past the last sequence: the bits of the kernel for rows that are not of whole pieces."""
     g = torch.Generator().manual_seed(C + taps + len(lens))
     T, S = sum(lens), len(lens)
     x = torch.randn(T + 5, 2 * C, generator=g).bfloat16().cuda()[:, C:]

@@ -588,7 +588,7 @@ class HybridModel:
         T, W = sv.T, self.arch.hidden_size
         st = _PreStream(T, W, self.act_dtype, self.device, second=self.side)
         first = {}
-        if self.loop_in is None:   # (a looped model's first layer reads the loop's own projection)
+        if self.loop_in is None:   # (else a pass's start may rewrite the stream first)
             first = self.layers[0].first_input(st)
             st.h_ready = True
         seq.embed_rows(sv.ids, self.embed, st.x, prev=sv.prev_tokens, scale=self.arch.embed_scale, **first)
